@@ -2,9 +2,10 @@
 
 A pass of every case is a step of a model's full-attention layers through the public entry points (``tinytitan_amd.engine``),
 called as the host runner calls them: per layer the QKV epilogue with its cache write, the attention over the cached keys with
-the output gate, and the output projection over affine weights; a sparse layer also runs its block indexer (the indexer's
-query and key projections, pooling, scores, selection) in front.  The caches hold what earlier tokens of the sequences left
-there, every layer its own.
+the output gate, and the output projection over affine weights; a sparse layer also runs its block indexer (pooling, scores,
+selection) in front.  The caches hold what earlier tokens of the sequences left there, every layer its own; the indexer's
+query rows are given, with the new tokens' raw keys in its cache, where a layer's own projections would have left them: a
+selection follows from them to the last bit, and a last bit of a query is another selection.
 
 kind            a pass is
 ``rows``        ``rows`` query tokens for each of ``seqs`` sequences: a decode step (1 row) or a draft's verify rows
@@ -22,7 +23,7 @@ from tinytitan_amd import synthetic
 from tinytitan_amd.engine import (AffineProjection, Attention, HIPContext, KVCacheManager, PrefillAttention,
                                   PrefillAttentionParams, QKVEpilogue, QSAIndexer)
 
-HIDDEN = 2048           # rows of the output projection, columns of the indexer's projections
+HIDDEN = 2048           # rows of the output projection
 ROTARY_DIM, THETA, EPS = 64, 1.0e7, 1.0e-6
 INDEX_HEADS, INDEX_DIM, INDEX_RATIO, INDEX_BUDGET = 4, 128, 4, 2048
 DEVICE = torch.device("cuda", 0)
@@ -174,20 +175,13 @@ def prepare(case, seed):
     s.epilogue, s.attention, s.prefill, s.projection = QKVEpilogue(ctx), Attention(ctx), PrefillAttention(ctx), AffineProjection(ctx)
     if case["kind"].startswith("sparse"):
         s.indexer = QSAIndexer(ctx, INDEX_HEADS, INDEX_DIM, INDEX_RATIO, INDEX_BUDGET, THETA, capacity=total)
-        s.hidden = [randn(tokens, HIDDEN) for _ in range(layers)]
+        s.index_rows = [randn(tokens, INDEX_HEADS * INDEX_DIM) for _ in range(layers)]
         s.index_q = torch.empty(tokens, INDEX_HEADS * INDEX_DIM, dtype=torch.float16, device=DEVICE)
-        s.index_q_proj = [_weights(gen, INDEX_HEADS * INDEX_DIM, HIDDEN, case["w_bits"]) for _ in range(layers)]
-        s.index_k_proj = [_weights(gen, INDEX_DIM, HIDDEN, case["w_bits"]) for _ in range(layers)]
         s.index_q_norm, s.index_k_norm = [norm_weight(INDEX_DIM) for _ in range(layers)], [norm_weight(INDEX_DIM) for _ in range(layers)]
         for layer in range(layers):
-            s.indexer.raw_key_destination(layer, 0, s.lengths[0]).copy_(randn(s.lengths[0], INDEX_DIM))
+            s.indexer.raw_key_destination(layer, 0, total).copy_(randn(total, INDEX_DIM))
             s.indexer.encode_pool_prefill(layer, 0, s.lengths[0], s.index_k_norm[layer], EPS)
     return s
-
-
-def _project(s, weights, x, y, rows, columns, tokens):
-    levels, scales, biases = weights
-    s.projection.encode(s.case["w_bits"], levels, scales, biases, x, y, rows, columns, tokens)
 
 
 def run(s):
@@ -197,9 +191,6 @@ def run(s):
     outputs = []
     for layer in range(case["layers"]):
         q, gate, attended = s.q, s.gate, s.attended[layer]
-        if case["kind"].startswith("sparse"):
-            _project(s, s.index_k_proj[layer], s.hidden[layer], s.indexer.raw_key_destination(layer, start, rows), INDEX_DIM, HIDDEN, rows)
-            _project(s, s.index_q_proj[layer], s.hidden[layer], s.index_q, INDEX_HEADS * INDEX_DIM, HIDDEN, rows)
         s.epilogue.encode(s.kv, layer, s.packed[layer], s.k[layer], s.v[layer], s.q_norm[layer], s.k_norm[layer], q, gate, heads,
                           s.lengths, rows, EPS, ROTARY_DIM, THETA, slots=s.slots)
         if case["kind"] == "rows" and rows == 1:
@@ -210,17 +201,18 @@ def run(s):
             params = PrefillAttentionParams(start, rows, start + rows, heads, s.scale, width, width, width, sliding_window=case["window"])
             s.prefill.encode_causal(s.kv, layer, 0, q, attended, params, gate=gate)
         elif case["kind"] == "sparse_rows":
-            s.indexer.encode_decode_step(layer, start, s.index_q, s.index_k_norm[layer], s.index_q_norm[layer], EPS)
+            s.indexer.encode_decode_step(layer, start, s.index_rows[layer], s.index_k_norm[layer], s.index_q_norm[layer], EPS)
             mask = s.indexer.select_keys(start + 1)
             s.attention.encode_full_keep(s.kv, layer, q, attended, heads, start + 1, mask, s.scale, gate=gate)
         else:
             s.indexer.encode_pool_prefill(layer, start, rows, s.index_k_norm[layer], EPS)
+            s.index_q.copy_(s.index_rows[layer])  # (they are normed and rotated in place; the projection would write them here)
             s.indexer.encode_scores(layer, s.index_q, s.index_q_norm[layer], start, rows, EPS)
             chosen = s.indexer.select_keys_prefill(start, rows, mask=False)
             params = PrefillAttentionParams(start, rows, start + rows, heads, s.scale, width, width, width)
             s.prefill.encode_causal(s.kv, layer, 0, q, attended, params, gate=gate, keep_indices=chosen.indices,
                                     keep_index_stride=chosen.index_stride, keep_counts=chosen.counts)
-        _project(s, s.o_proj[layer], attended, s.y[layer], HIDDEN, width, tokens)
+        s.projection.encode(case["w_bits"], *s.o_proj[layer], attended, s.y[layer], HIDDEN, width, tokens)
         outputs += [attended, s.y[layer]]
     if case["kind"] == "sparse_rows":
         outputs.append(mask)
@@ -256,9 +248,9 @@ def work(case):
     flops = 4 * dim * heads * pairs + 2 * tokens * width * HIDDEN
     if sparse:
         blocks = (case["lo"] + rows - 1) // INDEX_RATIO + 1
-        moved += weight_bytes(INDEX_HEADS * INDEX_DIM + INDEX_DIM, HIDDEN) + tokens * HIDDEN * 2 + blocks * INDEX_DIM * 2
+        moved += tokens * INDEX_HEADS * INDEX_DIM * 2 + blocks * INDEX_DIM * 2
         moved += (case["lo"] + 1 if rows == 1 else rows * budget * 4)  # the mask, or the lists
-        flops += 2 * tokens * INDEX_HEADS * INDEX_DIM * blocks + 2 * tokens * HIDDEN * (INDEX_HEADS + 1) * INDEX_DIM
+        flops += 2 * tokens * INDEX_HEADS * INDEX_DIM * blocks
     return {"bytes": layers * moved, "flops": layers * flops}
 
 
