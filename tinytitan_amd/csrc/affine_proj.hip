@@ -10,19 +10,8 @@
 // Arithmetic, as there: per row and group  scale * sum(level * x) + bias * sum(x)  in fp32, the row
 // summed over its groups in fp32 and rounded to fp16 once.
 //
-// Mapping.  A wavefront owns 32 weight rows x a range of groups for a slab of 32 tokens.  One
-// v_mfma_f32_32x32x16_f16 contracts 16 columns: A = 32 tokens x 16 columns of x, B = 16 columns x 32
-// weight rows of levels (exact small integers in fp16), so a lane's 16 accumulators are 16 tokens
-// of ONE weight row and the group's scale and bias are one value per lane.  A second MFMA per step
-// against an all-ones B gives sum(x) of the same tokens in the same accumulator layout.  After the
-// four steps of a group: acc += scale * dot + bias * sum(x), 32 fp32 FMAs.  Products of an fp16 x and
-// an integer level are exact in the fp32 accumulator; only the order of the sums differs from the
-// reference's.
-// A lane reads one contiguous 16 bytes (4-bit) or 32 bytes (8-bit) of its weight row per group --
-// columns 32 h .. 32 h + 31 of the group for lane half h -- and the x fragments follow that order,
-// so weights go HBM -> registers -> MFMA operand with no shuffle and no LDS.
-// The waves of a workgroup split the row's groups between them and add their partial rows through
-// LDS in a fixed order (no atomics: the result does not depend on timing).
+// Three kernels by token count: a dot-product GEMV (1 to 4 tokens), tiles on the matrix cores (5 to 512), a GEMM over
+// half weights (513 and more).
 #include <cstdint>
 
 #include "internal.h"
@@ -37,12 +26,6 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 
 constexpr int kProjGroup = 64;      // Quantization.groupSize
-constexpr int kProjWaves = 8;       // wavefronts per workgroup, splitting the groups of a row
-constexpr int kProjHeld = 8;        // groups of x a wavefront keeps in registers
-constexpr int kProjTileRows = 32;   // weight rows per tile = MFMA N
-constexpr int kProjSlab = 32;       // tokens per slab = MFMA M
-constexpr int kStagePitch = 2 * kProjGroup + 8;  // halves per token of a wavefront's x patch in LDS: two groups + 16 B
-constexpr int kProjLdsBytes = kProjWaves * 16 * 64 * 4 + kProjWaves * kProjSlab * kStagePitch * 2;
 
 struct ProjArgs {
     const uint8_t *weights;
@@ -51,7 +34,6 @@ struct ProjArgs {
     _Float16 *y;
     long long x_stride, y_stride;
     int rows, columns, tokens;
-    int tiles_per_wg;  // consecutive 32-row tiles one workgroup walks with its x fragments kept
 };
 
 // Eight bytes -> eight halves holding 0..255 exactly: byte b under exponent byte 0x64 is 1024 + b.
@@ -118,133 +100,248 @@ __device__ __forceinline__ void load_params(unsigned (&dst)[N / 2], const uint16
     }
 }
 
-template <int BITS, bool ALIGNED>
-__global__ __launch_bounds__(kProjWaves * 64) void affine_proj_kernel(const ProjArgs a) {
-    extern __shared__ float partial[];  // [wave][accumulator][lane], then each wavefront's x patch
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = lane & 31, h = lane >> 5;
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+
+// ---------------------------------------------------------------------------
+// 5 to 512 tokens (a draft's rows of several sequences, a decode batch, the default prefill chunk): tiles of 16 MT tokens x
+// 16 NR weight rows.  A workgroup's eight wavefronts split the columns, a wavefront's groups in order; per group
+// v_mfma_f32_16x16x32_f16 twice with A = x (16 tokens x 32 columns) and B = the levels, so that a lane's accumulators are
+// four tokens of ONE row and the group's scale and bias are one value per lane, and twice against a constant for sum(x)
+// in the same layout: acc += scale * dot + bias * sum(x).  The wavefronts' partial tiles are added through LDS in
+// wavefront order: a token's bits depend neither on the tile's form nor on its neighbours.
+//
+// What bounds it is how its rows get into a CU.  Fragments straight from global memory put 16 lanes -- one token or row
+// each, strides of whole lines -- on the same 16 bytes of 16 lines, which the vector cache serves a line at a time: 16 tokens
+// (2048 x 4096, 4 bits) took 7.9 us a launch that way, and 6.0 with token strides 16 bytes off a multiple of a line.
+// So x and the levels go to LDS by LDS-direct loads in whole lines, their 16-byte pieces permuted by row on the way so
+// that the fragment reads hit every bank.
+// A 4-bit level is shifted into the mantissa of 16.0 (16 + level, exact; eight instructions for eight levels, whose pairs
+// (k, k + 4) x follows by a permute), and the constant of the sums is -16: a group's dot product starts from
+// -16 sum(x), exact as the rest of it.  (Levels as subnormal halves, n times 2^-24, would save those instructions' or and
+// the start, but the matrix cores lose low bits on them: 95.5 % of the outputs bit-equal to the oracle instead of 99.85.)
+// The rest is bytes per CU, 16 MT x 8 KiB of x + 16 NR x 2.25 KiB of levels, at 35-40 KB/us.  us a launch, before (tiles of
+// 32 x 32, x through registers and private patches of LDS) -> now:
+//   2048 x 4096, 4 bits:   5 tokens 6.6 -> 5.5, 16: 9.8 -> 5.6, 32: 10.0 -> 5.7, 64: 10.2 -> 7.4, 128: 10.5 -> 9.8,
+//                          256: 18.7 -> 14.9, 512: 29.2 -> 27.5
+//   2048 x 4096, 8 bits:   32: 10.9 -> 6.1, 128: 11.6 -> 9.7, 512: 32.9 -> 27.6
+//   2048 x 6144, 4 bits:   16: 14.6 -> 6.8, 128: 15.9 -> 11.6;  512 x 2048, 4 bits: 5: 4.8 -> 3.4, 128: 7.2 -> 3.8
+// ---------------------------------------------------------------------------
+constexpr int kTileWaves = 8;  // wavefronts that share a row's groups
+// A wavefront's part of LDS: x [token tile][group][16 tokens][128 B], then levels [16 NR rows][SPAN groups].
+constexpr int tile_x_bytes(int mt, int span) { return mt * span * 16 * 2 * kProjGroup; }
+constexpr int tile_w_bytes(int bits, bool aligned, int nr, int span) { return aligned ? nr * 16 * span * 8 * bits : 0; }
+constexpr int tile_lds_bytes(int bits, bool aligned, int mt, int nr, int span) {
+    const int sums = kTileWaves * 16 * mt * (16 * nr + 4) * 4;  // the partial tiles take the rows' place
+    const int staged = kTileWaves * (tile_x_bytes(mt, span) + tile_w_bytes(bits, aligned, nr, span));
+    return sums > staged ? sums : staged;
+}
+
+// Four registers of one 16-byte piece per lane group of 16 lanes -> register r of lane group k holds word k of lane group
+// r's piece.
+__device__ __forceinline__ void transpose_quarters(unsigned (&v)[4]) {
+    auto swap32 = [](unsigned &a, unsigned &b) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    };
+    auto swap16 = [](unsigned &a, unsigned &b) {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    };
+    swap32(v[0], v[2]);
+    swap32(v[1], v[3]);
+    swap16(v[0], v[1]);
+    swap16(v[2], v[3]);
+}
+
+template <int BITS, bool ALIGNED, int MT, int NR, int SPAN>
+__global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const ProjArgs a) {
+    constexpr int kTokens = 16 * MT, kRows = 16 * NR, kPitch = kRows + 4;
+    constexpr int kXBytes = tile_x_bytes(MT, SPAN), kWaveBytes = kXBytes + tile_w_bytes(BITS, ALIGNED, NR, SPAN);
+    constexpr int kRowPitch = SPAN * 8 * BITS, kRowPieces = kRowPitch / 16, kCopyRows = 64 / kRowPieces;  // of the levels in LDS
+    constexpr int kSwizzle = kRowPieces < 8 ? kRowPieces - 1 : 7;
+    extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int n = lane & 15, kq = lane >> 4;
+    const int row0 = blockIdx.x * kRows, token0 = blockIdx.y * kTokens;
     const int groups = a.columns / kProjGroup;
-    const int per_wave = (groups + kProjWaves - 1) / kProjWaves;
+    int per_wave = (groups + kTileWaves - 1) / kTileWaves;
+    if (groups >= 4 * kTileWaves) per_wave = (per_wave + 3) / 4 * 4;
     const int g_begin = min(groups, wave * per_wave), g_end = min(groups, g_begin + per_wave);
-    constexpr int kHalfGroupBytes = BITS * 4;
-    constexpr int kChunk = BITS == 4 ? 4 : 2;  // groups whose levels are in flight together
     const size_t row_bytes = (size_t)a.columns * BITS / 8;
 
-    // x fragments: lane (token c of the slab, half h) holds columns 64 g + 32 h + 8 t .. + 7 for step t.
-    const bool live = (int)blockIdx.y * kProjSlab + c < a.tokens;
-    // They come through LDS: straight from global memory a lane would read 16 bytes of its own token's row per
-    // instruction -- 32 cache lines touched for 1 KiB, each line touched again by three later instructions and by
-    // then evicted by the other wavefronts' rows.  Instead the wavefront reads two groups of all 32 tokens with
-    // whole lines (16 lanes = 256 contiguous bytes of a token), writes them to its own patch of LDS (rows padded
-    // by 16 B) and reads the fragments back; LDS serves a wavefront's accesses in order, so no barrier is needed.
-    h8 xa[kProjHeld][4];
-    _Float16 *const stage = reinterpret_cast<_Float16 *>(partial + kProjWaves * 16 * 64) + wave * (kProjSlab * kStagePitch);
-    auto load_x = [&](int g0) {
-        h8 raw[2][8];
-        auto fetch = [&](h8 (&dst)[8], int pair) {
-            const int g = min(g0 + 2 * pair + ((lane >> 3) & 1), groups - 1);  // a valid address always
+    // copies: lane -> 16 bytes of token lane / 8 (+ 8): piece (lane % 8) ^ (lane / 8) of a group's 128 bytes
+    const _Float16 *x_src[2 * MT];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int t = min((int)blockIdx.y * kProjSlab + 4 * i + (lane >> 4), a.tokens - 1);
-                dst[i] = *reinterpret_cast<const h8 *>(a.x + (long long)t * a.x_stride + kProjGroup * g + 8 * (lane & 7));
-            }
-        };
-        fetch(raw[0], 0);
+    for (int c = 0; c < 2 * MT; ++c)
+        x_src[c] = a.x + (long long)min(token0 + 8 * c + (lane >> 3), a.tokens - 1) * a.x_stride + 8 * ((lane & 7) ^ (lane >> 3));
+    unsigned char *const x_lds = tile_lds + wave * kWaveBytes, *const w_lds = x_lds + kXBytes;
+    const uint8_t *w_src[NR];
+    size_t p_at[NR];
 #pragma unroll
-        for (int pair = 0; pair < kProjHeld / 2; ++pair) {
-            if (pair + 1 < kProjHeld / 2) fetch(raw[(pair + 1) & 1], pair + 1);
+    for (int nr = 0; nr < NR; ++nr) {
+        const int row = min(row0 + 16 * nr + n, a.rows - 1);
+        w_src[nr] = a.weights + (size_t)row * row_bytes;
+        p_at[nr] = (size_t)row * groups;
+    }
+    const bool params_vector = groups % 4 == 0 && per_wave % 4 == 0 && (uintptr_t)a.scales % 8 == 0 && (uintptr_t)a.biases % 8 == 0;
+    const f4v zero = {0.f, 0.f, 0.f, 0.f};
+    f4v acc[MT][NR];
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                *reinterpret_cast<h8 *>(stage + (4 * i + (lane >> 4)) * kStagePitch + 8 * (lane & 15)) = raw[pair & 1][i];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int gi = 0; gi < 2; ++gi)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const h8 v = *reinterpret_cast<const h8 *>(stage + c * kStagePitch + kProjGroup * gi + 32 * h + 8 * t);
-                    xa[2 * pair + gi][t] = live ? v : (h8)(_Float16)0;
-                }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-    };
-    const bool x_held = g_end - g_begin <= kProjHeld;  // then loaded once, with the first tile
-    // a row's N scales (N * 2 bytes) in one load where every such run is aligned
-    const bool params_vector = groups % kChunk == 0 && per_wave % kChunk == 0 && (uintptr_t)a.scales % (2 * kChunk) == 0 &&
-                               (uintptr_t)a.biases % (2 * kChunk) == 0;
-    const h8 ones = (h8)(_Float16)1;
-    const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int nr = 0; nr < NR; ++nr) acc[mt][nr] = zero;
+    const h8 ones = (h8)(_Float16)(BITS == 4 ? -16 : 1);
 
-    for (int i = 0; i < a.tiles_per_wg; ++i) {
-        const int tile = blockIdx.x * a.tiles_per_wg + i;
-        if (tile * kProjTileRows >= a.rows) break;  // the whole workgroup
-        const int row = min(tile * kProjTileRows + c, a.rows - 1);
-        const uint8_t *w_row = a.weights + (size_t)row * row_bytes + h * kHalfGroupBytes;
-        const uint16_t *s_row = a.scales + (size_t)row * groups, *b_row = a.biases + (size_t)row * groups;
-        f16v acc = zero;
-        for (int g0 = g_begin; g0 < g_end; g0 += kProjHeld) {
+    for (int g0 = g_begin; g0 < g_end; g0 += 4) {
+        unsigned scales[NR][2], biases[NR][2];
 #pragma unroll
-            for (int sub = 0; sub < kProjHeld; sub += kChunk) {
-                if (g0 + sub >= g_end) break;  // the whole wavefront
-                unsigned w[kChunk][BITS];
-                unsigned scale_pairs[kChunk / 2], bias_pairs[kChunk / 2];
+        for (int sub = 0; sub < 4; sub += SPAN) {
+            if (g0 + sub >= g_end) break;
+            const int gs = g0 + sub;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last span's fragments have been read
 #pragma unroll
-                for (int gi = 0; gi < kChunk; ++gi) {
-                    const int g = min(g0 + sub + gi, groups - 1);  // a valid address always
-                    load_levels<BITS, ALIGNED>(w[gi], w_row + (size_t)g * (2 * kHalfGroupBytes));
+            for (int gi = 0; gi < SPAN; ++gi) {
+                if (gs + gi >= g_end) break;
+#pragma unroll
+                for (int c = 0; c < 2 * MT; ++c)
+                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(x_src[c] + kProjGroup * (gs + gi)),
+                                                     (__attribute__((address_space(3))) void *)(x_lds + gi * (2048 * MT) + c * 1024), 16, 0, 0);
+            }
+            if constexpr (ALIGNED) {
+#pragma unroll
+                for (int c = 0; c < kRows / kCopyRows; ++c) {
+                    const int local = kCopyRows * c + lane / kRowPieces, row = min(row0 + local, a.rows - 1);
+                    const size_t at = min((size_t)gs * (8 * BITS) + 16 * ((lane % kRowPieces) ^ (local & kSwizzle)), row_bytes - 16);
+                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(a.weights + (size_t)row * row_bytes + at),
+                                                     (__attribute__((address_space(3))) void *)(w_lds + c * 1024), 16, 0, 0);
                 }
-                load_params<kChunk>(scale_pairs, s_row, g0 + sub, groups, params_vector);
-                load_params<kChunk>(bias_pairs, b_row, g0 + sub, groups, params_vector);
-                // x (re)loaded while the levels are on their way
-                if (sub == 0 && (!x_held || i == 0)) load_x(g0);
-                // Every load of the chunk is issued before its first use: left to itself the scheduler
-                // sinks each group's loads to its MFMAs and the wavefront waits for memory once per group.
-                __builtin_amdgcn_sched_barrier(0);
+            }
+            unsigned w[NR][SPAN * BITS / 2];
 #pragma unroll
-                for (int gi = 0; gi < kChunk; ++gi) {
-                    if (g0 + sub + gi >= g_end) break;  // the whole wavefront
-                    f16v dot = zero, xsum = zero;
+            for (int nr = 0; nr < NR; ++nr) {
+                if constexpr (!ALIGNED) {
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        h8 levels;
-                        if constexpr (BITS == 4) levels = levels_of_nibbles(w[gi][t]);
-                        else levels = levels_of_bytes(w[gi][2 * t], w[gi][2 * t + 1]);
-                        dot = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[sub + gi][t], levels, dot, 0, 0, 0);
-                        xsum = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[sub + gi][t], ones, xsum, 0, 0, 0);
+                    for (int j = 0; j < SPAN * BITS / 8; ++j) {
+                        unsigned v[4];
+                        if constexpr (BITS == 4) load_levels<4, false>(v, w_src[nr] + (size_t)min(gs + 2 * j + (kq >> 1), groups - 1) * 32 + 16 * (kq & 1));
+                        else load_levels<4, false>(v, w_src[nr] + (size_t)min(gs + j, groups - 1) * 64 + 16 * kq);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) w[nr][4 * j + i] = v[i];
                     }
-                    // a bf16 is the upper half of the float
-                    const unsigned sp = scale_pairs[gi / 2], bp = bias_pairs[gi / 2];
-                    const float scale = __builtin_bit_cast(float, (gi & 1) ? (sp & 0xffff0000u) : (sp << 16));
-                    const float bias = __builtin_bit_cast(float, (gi & 1) ? (bp & 0xffff0000u) : (bp << 16));
+                }
+                if (sub == 0) {
+                    load_params<4>(scales[nr], a.scales + p_at[nr], g0, groups, params_vector);
+                    load_params<4>(biases[nr], a.biases + p_at[nr], g0, groups, params_vector);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wavefront's own copies: no barrier
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                    for (int j = 0; j < 16; ++j) acc[j] = fmaf(bias, xsum[j], fmaf(scale, dot[j], acc[j]));
+            for (int nr = 0; nr < NR; ++nr)
+#pragma unroll
+                for (int j = 0; j < SPAN * BITS / 8; ++j) {
+                    unsigned v[4] = {w[nr][4 * j], w[nr][4 * j + 1], w[nr][4 * j + 2], w[nr][4 * j + 3]};
+                    if constexpr (ALIGNED) {
+                        const u4v r = *reinterpret_cast<const u4v *>(w_lds + (16 * nr + n) * kRowPitch + (((4 * j + kq) ^ (n & kSwizzle)) << 4));
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = r[i];
+                    }
+                    if constexpr (BITS == 4) transpose_quarters(v);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) w[nr][4 * j + i] = v[i];
+                }
+#pragma unroll
+            for (int gi = 0; gi < SPAN; ++gi) {
+                if (gs + gi >= g_end) break;  // the whole wavefront
+                const int g4 = sub + gi;
+                h8 xf[MT][2];
+                f4v xsum[MT];
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const int piece = BITS == 4 ? 4 * i + kq : 2 * kq + i;
+                        const h8 v = *reinterpret_cast<const h8 *>(x_lds + gi * (2048 * MT) + (16 * mt + n) * 128 + ((piece ^ (n & 7)) << 4));
+                        if constexpr (BITS == 4) xf[mt][i] = h8{v[0], v[4], v[1], v[5], v[2], v[6], v[3], v[7]};
+                        else xf[mt][i] = v;
+                    }
+                    xsum[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[mt][0], ones, zero, 0, 0, 0);
+                    xsum[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[mt][1], ones, xsum[mt], 0, 0, 0);
+                }
+#pragma unroll
+                for (int nr = 0; nr < NR; ++nr) {
+                    const unsigned sp = scales[nr][g4 / 2], bp = biases[nr][g4 / 2];
+                    const float bias = __builtin_bit_cast(float, (g4 & 1) ? (bp & 0xffff0000u) : (bp << 16)) * (BITS == 4 ? -0.0625f : 1.0f);
+                    const float scale = __builtin_bit_cast(float, (g4 & 1) ? (sp & 0xffff0000u) : (sp << 16));
+                    h8 levels[2];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        u4v bits;  // 16 + level (4 bits), 1024 + level (8 bits)
+                        constexpr unsigned e = BITS == 4 ? 0x4c004c00u : 0x64646464u;
+                        if constexpr (BITS == 4) {
+                            const unsigned v = w[nr][2 * gi + i];
+                            bits = u4v{((v << 6) & 0x03c003c0u) | e, ((v << 2) & 0x03c003c0u) | e, ((v >> 2) & 0x03c003c0u) | e, ((v >> 6) & 0x03c003c0u) | e};
+                        } else {
+                            const unsigned w0 = w[nr][4 * gi + 2 * i], w1 = w[nr][4 * gi + 2 * i + 1];
+                            bits = u4v{__builtin_amdgcn_perm(e, w0, 0x04010400u), __builtin_amdgcn_perm(e, w0, 0x04030402u),
+                                       __builtin_amdgcn_perm(e, w1, 0x04010400u), __builtin_amdgcn_perm(e, w1, 0x04030402u)};
+                        }
+                        levels[i] = BITS == 4 ? __builtin_bit_cast(h8, bits) : __builtin_bit_cast(h8, bits) - (h8)(_Float16)1024;
+                    }
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) {
+                        f4v dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[mt][0], levels[0], BITS == 4 ? xsum[mt] : zero, 0, 0, 0);
+                        dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[mt][1], levels[1], dot, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[mt][nr][j] = fmaf(bias, xsum[mt][j], fmaf(scale, dot[j], acc[mt][nr][j]));
+                    }
                 }
             }
         }
-        // Add the waves' partial rows in wave order and write y: accumulator j of lane (c, h) is token
-        // 8 (j / 4) + 4 h + j % 4 of the slab, weight row c of the tile.
-        if (i > 0) __syncthreads();  // the previous tile's sums have been read
+    }
+    __syncthreads();
+    float *const sums = reinterpret_cast<float *>(tile_lds);  // [wavefront][token][kPitch]
 #pragma unroll
-        for (int j = 0; j < 16; ++j) partial[(wave * 16 + j) * 64 + lane] = acc[j];
-        __syncthreads();
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int j = wave; j < 16; j += kProjWaves) {
-            float sum = 0.0f;
+        for (int nr = 0; nr < NR; ++nr)
 #pragma unroll
-            for (int w2 = 0; w2 < kProjWaves; ++w2) sum += partial[(w2 * 16 + j) * 64 + lane];
-            const int out_token = blockIdx.y * kProjSlab + 8 * (j / 4) + 4 * h + (j % 4);
-            const int out_row = tile * kProjTileRows + c;
-            if (out_token < a.tokens && out_row < a.rows) a.y[(long long)out_token * a.y_stride + out_row] = (_Float16)sum;
-        }
+            for (int j = 0; j < 4; ++j) sums[(wave * kTokens + 16 * mt + 4 * kq + j) * kPitch + 16 * nr + n] = acc[mt][nr][j];
+    __syncthreads();
+    for (int at = threadIdx.x; at < kTokens * kRows; at += kTileWaves * 64) {
+        const int t = at / kRows, r = at % kRows;
+        float sum = 0.0f;
+#pragma unroll
+        for (int w2 = 0; w2 < kTileWaves; ++w2) sum += sums[(w2 * kTokens + t) * kPitch + r];
+        if (token0 + t < a.tokens && row0 + r < a.rows) a.y[(long long)(token0 + t) * a.y_stride + row0 + r] = (_Float16)sum;
     }
 }
 
+// The smallest tile whose workgroups find a CU each -- a wider tile reads less per output but takes longer: 32 tokens
+// 5.6 us in tiles of 16 x 16 (256 workgroups), 6.8 in 16 x 32, 9.1 in 32 x 32; 64 tokens 8.1 / 7.0 / 9.1; 128 tokens
+// 12.8 / 12.0 / 9.8 (10.2 with two groups instead of four in LDS at a time, which lets two workgroups share a CU) -- and
+// beyond that 32 x 32, two workgroups to a CU (256 tokens 14.9 us, with four groups in LDS 17.9), or over 8 bits, whose levels weigh twice as much, 32 x 64 (256 tokens 13.2 against 16.0 us).
+template <int BITS, bool ALIGNED>
+void launch_tile(tt_hip_ctx *ctx, const ProjArgs &a) {
+    auto tiles = [&](int mt, int nr) { return (long long)((a.rows + 16 * nr - 1) / (16 * nr)) * ((a.tokens + 16 * mt - 1) / (16 * mt)); };
+    auto launch = [&](auto kernel, int mt, int nr, int lds) {
+        const dim3 grid((unsigned)((a.rows + 16 * nr - 1) / (16 * nr)), (unsigned)((a.tokens + 16 * mt - 1) / (16 * mt)));
+        launch_profiled(ctx, kernel, grid, dim3(kTileWaves * 64), (unsigned)lds, a);
+    };
+    if (tiles(1, 1) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 1, 1, 4>, 1, 1, tile_lds_bytes(BITS, ALIGNED, 1, 1, 4));
+    else if (tiles(1, 2) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 1, 2, 4>, 1, 2, tile_lds_bytes(BITS, ALIGNED, 1, 2, 4));
+    else if (BITS == 4 && tiles(2, 2) <= ctx->n_cus) launch(affine_tile_kernel<4, ALIGNED, 2, 2, 4>, 2, 2, tile_lds_bytes(4, ALIGNED, 2, 2, 4));
+    else if (BITS == 4 || tiles(2, 2) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 2, 2, 2>, 2, 2, tile_lds_bytes(BITS, ALIGNED, 2, 2, 2));
+    else if constexpr (BITS == 8) launch(affine_tile_kernel<8, ALIGNED, 2, 4, 2>, 2, 4, tile_lds_bytes(8, ALIGNED, 2, 4, 2));
+}
+
 // ---------------------------------------------------------------------------
-// Up to nine tokens (a decode row, the two-row and four-row verify passes, a small decode batch): the matrix cores
-// have little to amortise, and 32-row tiles would leave three quarters of the chip idle at 2048 rows.
+// Up to four tokens (a decode row, the two-row and four-row verify passes): the matrix cores have little to amortise, and
+// tiles of 16 rows would leave half of the chip idle at 2048 rows.
 // Here a workgroup owns 8 weight rows and its eight wavefronts take the columns 512 at a time in
 // turn: a lane takes 8 consecutive columns of each row (one dword of nibbles or two of bytes,
 // coalesced; they lie in one group), widens them to fp16 levels and contracts them with its 8 x
@@ -252,10 +349,10 @@ __global__ __launch_bounds__(kProjWaves * 64) void affine_proj_kernel(const Proj
 // acc += scale * dot + bias * sum(x) as above.  All of a wavefront's loads for a 512-column chunk
 // are independent, so they are in flight together; lanes are added by DPP moves (six vector instructions a
 // sum; as six shuffles through LDS each, the 8 x TOK sums were most of the kernel: one token 5.5 -> 4.2 us a step,
-// four tokens 11.0 -> 6.3, which moved the hand-over to the MFMA kernel's flat 10.6 us from 5 tokens to 10),
+// four tokens 11.0 -> 6.3; from five on the tiles above are ahead, 5.4 us against 6.6),
 // wavefronts through LDS in a fixed order.  256 workgroups at 2048 rows.
 // ---------------------------------------------------------------------------
-constexpr int kGemvWaves = 8, kGemvRows = 8, kGemvMaxTokens = 9;
+constexpr int kGemvWaves = 8, kGemvRows = 8, kGemvMaxTokens = 4;
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float dot8(h8 a, h8 b) {
@@ -352,12 +449,7 @@ void launch_gemv(tt_hip_ctx *ctx, const ProjArgs &a) {
         case 1: launch_profiled(ctx, affine_gemv_kernel<BITS, 1, ALIGNED>, grid, block, 0u, a); break;
         case 2: launch_profiled(ctx, affine_gemv_kernel<BITS, 2, ALIGNED>, grid, block, 0u, a); break;
         case 3: launch_profiled(ctx, affine_gemv_kernel<BITS, 3, ALIGNED>, grid, block, 0u, a); break;
-        case 4: launch_profiled(ctx, affine_gemv_kernel<BITS, 4, ALIGNED>, grid, block, 0u, a); break;
-        case 5: launch_profiled(ctx, affine_gemv_kernel<BITS, 5, ALIGNED>, grid, block, 0u, a); break;
-        case 6: launch_profiled(ctx, affine_gemv_kernel<BITS, 6, ALIGNED>, grid, block, 0u, a); break;
-        case 7: launch_profiled(ctx, affine_gemv_kernel<BITS, 7, ALIGNED>, grid, block, 0u, a); break;
-        case 8: launch_profiled(ctx, affine_gemv_kernel<BITS, 8, ALIGNED>, grid, block, 0u, a); break;
-        default: launch_profiled(ctx, affine_gemv_kernel<BITS, 9, ALIGNED>, grid, block, 0u, a); break;
+        default: launch_profiled(ctx, affine_gemv_kernel<BITS, 4, ALIGNED>, grid, block, 0u, a); break;
     }
 }
 
@@ -381,9 +473,8 @@ void launch_gemv(tt_hip_ctx *ctx, const ProjArgs &a) {
 // group, in its middle.  The output tile leaves through LDS, [token][row], as 16-byte stores.
 // ---------------------------------------------------------------------------
 constexpr int kGemmTokens = 128, kGemmWaves = 4, kGemmRows = 32 * kGemmWaves;
-// From here on the GEMM is the faster of the two MFMA kernels at 2048 x 4096: 39-40 us up to 1024 tokens and 48 us
-// at 2048, where its grid fills the chip, against 33 us at 512 tokens and 45 us and more from 513 on for the factored
-// kernel, whose workgroups then come in a third round.
+// From here on the chunk is a GEMM: 39-40 us up to 1024 tokens and 48 us at 2048, where its grid fills the chip, against
+// 26 us at 512 tokens for the tiles above, whose time goes on growing by 25 us per 512 tokens.
 constexpr int kGemmMinTokens = 513;
 constexpr int kGemmThreads = kGemmWaves * 64;
 constexpr int kGemmPitch = kProjGroup + 8;                           // halves per token row of the x tile in LDS
@@ -646,17 +737,9 @@ int launch_gemm(tt_hip_ctx *ctx, const ProjArgs &a, dim3 grid) {
     return TT_HIP_OK;
 }
 
-// 100 KiB of LDS: above the 64 KiB a kernel gets without asking.
-template <int BITS, bool ALIGNED>
-int launch_proj(tt_hip_ctx *ctx, const ProjArgs &a, dim3 grid) {
-    auto kernel = affine_proj_kernel<BITS, ALIGNED>;  // its LDS limit was raised when the context was created
-    launch_profiled(ctx, kernel, grid, dim3(kProjWaves * 64), (unsigned)kProjLdsBytes, a);
-    return TT_HIP_OK;
-}
-
 }  // namespace
 
-// The two MFMA kernels' dynamic LDS limits, set once per device when a context is created on it.
+// The MFMA kernels' dynamic LDS limits, set once per device when a context is created on it.
 int configure_affine_kernels(tt_hip_ctx *ctx) {
     hipError_t e = hipSuccess;
 #define TT_CFG(KERNEL, BYTES) \
@@ -673,10 +756,22 @@ int configure_affine_kernels(tt_hip_ctx *ctx) {
     TT_CFG((affine_gemm_kernel<4, false, 2, true>), gemm_rs_lds_bytes())
     TT_CFG((affine_gemm_kernel<8, true, 2, true>), gemm_rs_lds_bytes())
     TT_CFG((affine_gemm_kernel<8, false, 2, true>), gemm_rs_lds_bytes())
-    TT_CFG((affine_proj_kernel<4, true>), kProjLdsBytes)
-    TT_CFG((affine_proj_kernel<4, false>), kProjLdsBytes)
-    TT_CFG((affine_proj_kernel<8, true>), kProjLdsBytes)
-    TT_CFG((affine_proj_kernel<8, false>), kProjLdsBytes)
+    TT_CFG((affine_tile_kernel<4, true, 1, 1, 4>), tile_lds_bytes(4, true, 1, 1, 4))
+    TT_CFG((affine_tile_kernel<4, true, 1, 2, 4>), tile_lds_bytes(4, true, 1, 2, 4))
+    TT_CFG((affine_tile_kernel<4, true, 2, 2, 4>), tile_lds_bytes(4, true, 2, 2, 4))
+    TT_CFG((affine_tile_kernel<4, true, 2, 2, 2>), tile_lds_bytes(4, true, 2, 2, 2))
+    TT_CFG((affine_tile_kernel<4, false, 1, 1, 4>), tile_lds_bytes(4, false, 1, 1, 4))
+    TT_CFG((affine_tile_kernel<4, false, 1, 2, 4>), tile_lds_bytes(4, false, 1, 2, 4))
+    TT_CFG((affine_tile_kernel<4, false, 2, 2, 4>), tile_lds_bytes(4, false, 2, 2, 4))
+    TT_CFG((affine_tile_kernel<4, false, 2, 2, 2>), tile_lds_bytes(4, false, 2, 2, 2))
+    TT_CFG((affine_tile_kernel<8, true, 1, 1, 4>), tile_lds_bytes(8, true, 1, 1, 4))
+    TT_CFG((affine_tile_kernel<8, true, 1, 2, 4>), tile_lds_bytes(8, true, 1, 2, 4))
+    TT_CFG((affine_tile_kernel<8, true, 2, 4, 2>), tile_lds_bytes(8, true, 2, 4, 2))
+    TT_CFG((affine_tile_kernel<8, true, 2, 2, 2>), tile_lds_bytes(8, true, 2, 2, 2))
+    TT_CFG((affine_tile_kernel<8, false, 1, 1, 4>), tile_lds_bytes(8, false, 1, 1, 4))
+    TT_CFG((affine_tile_kernel<8, false, 1, 2, 4>), tile_lds_bytes(8, false, 1, 2, 4))
+    TT_CFG((affine_tile_kernel<8, false, 2, 4, 2>), tile_lds_bytes(8, false, 2, 4, 2))
+    TT_CFG((affine_tile_kernel<8, false, 2, 2, 2>), tile_lds_bytes(8, false, 2, 2, 2))
 #undef TT_CFG
     return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "hipFuncSetAttribute(o_proj max dynamic LDS)");
 }
@@ -713,15 +808,7 @@ extern "C" int tt_hip_affine_projection(tt_hip_ctx *ctx, int weight_bits, const 
     a.rows = rows;
     a.columns = columns;
     a.tokens = token_count;
-    const int tiles = (rows + kProjTileRows - 1) / kProjTileRows;
-    const int slabs = (token_count + kProjSlab - 1) / kProjSlab;
-    // One tile per workgroup while that does not yet fill the chip twice; beyond that a workgroup
-    // keeps its x fragments and walks several tiles, which divides the reads of x.
-    a.tiles_per_wg = 1;
-    while (a.tiles_per_wg < 8 && (long long)((tiles + 2 * a.tiles_per_wg - 1) / (2 * a.tiles_per_wg)) * slabs >= 2LL * ctx->n_cus)
-        a.tiles_per_wg *= 2;
-    const dim3 grid((unsigned)((tiles + a.tiles_per_wg - 1) / a.tiles_per_wg), (unsigned)slabs);
-    if (slabs > 65535) return TT_HIP_ERR_SHAPE;
+    if (token_count > 32 * 65535) return TT_HIP_ERR_SHAPE;
     const bool aligned = (uintptr_t)weights % 16 == 0;
     if (token_count >= kGemmMinTokens) {
         const long long row_blocks = (rows + kGemmRows - 1) / kGemmRows, token_blocks = (token_count + kGemmTokens - 1) / kGemmTokens;
@@ -760,11 +847,15 @@ extern "C" int tt_hip_affine_projection(tt_hip_ctx *ctx, int weight_bits, const 
             else launch_gemv<8, false>(ctx, a);
         }
     } else {
-        int status;
-        if (weight_bits == 4) status = aligned ? launch_proj<4, true>(ctx, a, grid) : launch_proj<4, false>(ctx, a, grid);
-        else status = aligned ? launch_proj<8, true>(ctx, a, grid) : launch_proj<8, false>(ctx, a, grid);
-        if (status != TT_HIP_OK) return status;
+        // (aligned: rows of levels are then whole 16-byte pieces, too)
+        if (weight_bits == 4) {
+            if (aligned) launch_tile<4, true>(ctx, a);
+            else launch_tile<4, false>(ctx, a);
+        } else {
+            if (aligned) launch_tile<8, true>(ctx, a);
+            else launch_tile<8, false>(ctx, a);
+        }
     }
     const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "affine_proj_kernel launch");
+    return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "affine projection launch");
 }
