@@ -59,3 +59,37 @@ def test_rows_and_keys_on_both_sides_of_every_threshold(gpu_ctx, bits, rows, kv_
                                                    (4, 4, 128, 40, 20000), (16, 2, 256, 3, 33000)])
 def test_head_groups_the_chunk_kernel_does_not_take_and_few_rows(gpu_ctx, bits, H, KH, D, rows, kv_valid):
     _chunk(gpu_ctx, bits, H, KH, D, rows, kv_valid)
+
+
+@pytest.mark.parametrize("H,KH,D,rows,start,window,ring", [
+    (24, 2, 256, 777, 150, 500, 0),       # three head sets per KV head, ragged last tile, some windows clipped, some not
+    (32, 8, 128, 1029, 1237, 400, 1856),  # eight KV heads (one XCD each), over a ring
+    (16, 2, 256, 1030, 40, 0, 0),         # no window: the causal triangle, the longest tile first
+    (12, 1, 64, 2100, 3, 0, 0)])          # one KV head, 66 tiles of three head sets: a second round of workgroups
+def test_whole_chunks_in_single_tiles(gpu_ctx, H, KH, D, rows, start, window, ring):
+    import torch
+    from tinytitan_amd.engine import KVCacheManager, PrefillAttention, PrefillAttentionParams
+    total, scale = start + rows, float(D) ** -0.5
+    r = np.random.default_rng(rows + start)
+    k, v = (r.standard_normal((total, KH * D)).astype(np.float16) for _ in range(2))
+    q, g = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=1, max_context=total, initial_capacity=total, ring_capacity=ring)
+    first = max(0, start - window - 32) if ring else 0
+    at = first
+    while at < total:  # (a ring takes ranges that do not wrap)
+        n = min(total - at, ring - at % ring) if ring else total - at
+        kd, vd = _dev(k[at:at + n]), _dev(v[at:at + n])
+        torch.cuda.synchronize()
+        kv.append(0, 0, at, kd, vd)
+        gpu_ctx.synchronize()
+        at += n
+    qd, gd = _dev(q), _dev(g)
+    out = torch.full(qd.shape, float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, total, H, scale, H * D, H * D, H * D,
+                                                                                     sliding_window=window), gate=gd)
+    gpu_ctx.synchronize()
+    want = oracle.prefill_ref(q.astype(np.float32), k.astype(np.float32), v.astype(np.float32), H * D, KH * D, D, H, KH, start, rows,
+                              total, window, scale).reshape(rows, -1) / (1 + np.exp(-g.astype(np.float64)))
+    _check(out.float().cpu().numpy(), want, f"{rows} rows behind {start} keys, {H}q/{KH}kv/{D}, window {window}, ring {ring}")
+    kv.close()

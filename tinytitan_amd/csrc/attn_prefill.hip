@@ -55,7 +55,7 @@ struct PrefillArgs {
     int hsubs;     // group / 4
     int n_tiles;   // ceil(q_len / 32)
     int n_pairs;   // ceil(n_tiles / 2); with single_tiles: n_tiles
-    int single_tiles;  // 1: a workgroup takes ONE tile (tile = its pair index) instead of a long and a short one
+    int single_tiles;  // 1: a workgroup takes ONE tile instead of a long and a short one
     int per_kvh;   // hsubs * n_pairs
     int xs;        // XCDs per kv head (8 / n_kv_heads), 0: plain mapping
     int n_kv_heads;
@@ -194,8 +194,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
         r = wg - kvh * a.per_kvh;
     }
     if (r >= a.per_kvh || kvh >= a.n_kv_heads) return;
-    const int hsub = r / a.n_pairs;
-    const int pair = r - hsub * a.n_pairs;
+    // (whole tiles one by one: the head sets' longest tiles first, and so on down)
+    const bool longest_first = a.single_tiles && a.n_splits == 1;
+    const int hsub = longest_first ? r % a.hsubs : r / a.n_pairs;
+    const int pair = longest_first ? r / a.hsubs : r - hsub * a.n_pairs;
     const int head = kvh * a.group + hsub * 4 + w4;
     const _Float16 *kp = a.k_slot + (size_t)kvh * a.page_elems;
     const _Float16 *vp = a.v_slot + (size_t)kvh * a.page_elems;
@@ -257,12 +259,13 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
     float *const lsum_mine = reinterpret_cast<float *>(smem + LSUM_OFF) + w4 * 32 + li;
 
     // Tiles in pairs (tile i with tile n - 1 - i: every workgroup the same number of key blocks under a causal
-    // mask from position 0) -- or, where the keys are cut into ranges, one tile each: deep in a context the tiles
-    // are equally long anyway, and a workgroup with one tile leaves half the partial results of one with two.
+    // mask from position 0) -- or one tile each: where the keys are cut into ranges (deep in a context the tiles are equally
+    // long anyway, and a workgroup with one tile leaves half the partial results of one with two), and where pairs would
+    // leave CUs idle (estimate_chunk in context.hip), the longest tile first.
     const int n_passes = (a.single_tiles || pair == a.n_tiles - 1 - pair) ? 1 : 2;
     for (int pass = 0; pass < n_passes; ++pass) {
         // The long tile goes first: the short one then fills in behind it.
-        const int tile = a.single_tiles ? pair : (pass == 0 ? a.n_tiles - 1 - pair : pair);
+        const int tile = longest_first ? a.n_tiles - 1 - pair : a.single_tiles ? pair : (pass == 0 ? a.n_tiles - 1 - pair : pair);
         const int tok = tile * 32 + li;
         const bool valid = tok < a.q_len;
         const int lim = valid ? min(a.kv_valid, a.start + tok + 1) : 0;  // keys [lo, lim) are visible
@@ -277,7 +280,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
         const int mask_from = (a.start + tile * 32 + 1) >> 5;  // first block in which some row is masked by causality
         const int first_masked = min(mask_from, end >> 5);     // ... or cut by the valid length
         // This workgroup's share of them (all, without key splits); local step i is block jb + i.
-        jb = a.n_splits > 1 ? split * a.split_blocks : window_block;  // (key splits and windows are not combined)
+        jb = window_block + (a.n_splits > 1 ? split * a.split_blocks : 0);
         const int nb = (a.n_splits > 1 ? min(nb_tile, jb + a.split_blocks) : nb_tile) - jb;
         if (nb <= 0) continue;  // nothing of this tile in the range (the same for every wave)
 
@@ -500,9 +503,8 @@ static int launch_prefill_d(tt_hip_ctx *ctx, const PrefillArgs &args, unsigned g
 int launch_prefill(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot, int start, int q_len, int kv_valid,
                    int n_q_heads, const tt_half *q, long long q_stride, const tt_half *gate, long long g_stride,
                    float scale, tt_half *out, long long o_stride, int n_splits, int split_blocks, float *part_o,
-                   float *part_ml, const PageSource *pages, int window) {
+                   float *part_ml, const PageSource *pages, int window, bool single_tiles) {
     PrefillArgs a{};
-    if (window > 0 && n_splits > 1) return TT_HIP_ERR_INVALID_ARGUMENT;  // key ranges start at key 0
     a.window = window;
     if (!pages && kv->bits != 16) return TT_HIP_ERR_INVALID_ARGUMENT;  // this kernel reads fp16 pages only
     const size_t slot_off = (size_t)slot * kv->n_kv_heads * kv->page_elems();
@@ -519,7 +521,7 @@ int launch_prefill(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot, int star
     a.group = n_q_heads / kv->n_kv_heads;
     a.hsubs = a.group / 4;
     a.n_tiles = (q_len + 31) / 32;
-    a.single_tiles = n_splits > 1 ? 1 : 0;
+    a.single_tiles = n_splits > 1 || single_tiles ? 1 : 0;
     a.n_pairs = a.single_tiles ? a.n_tiles : (a.n_tiles + 1) / 2;
     a.per_kvh = a.hsubs * a.n_pairs;
     a.n_kv_heads = kv->n_kv_heads;

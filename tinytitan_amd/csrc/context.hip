@@ -433,7 +433,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         if (chunk_splits > 1) {
             st = launch_prefill(ctx, kv, layer, slots[base], starts[base], rows, totals[base], n_q_heads, q, q_tok_stride, gate,
                                 g_tok_stride, scale, out, o_tok_stride, chunk_splits, chunk_split_blocks, ctx->part_o,
-                                ctx->part_ml, pages);
+                                ctx->part_ml, pages, window);
             if (st == TT_HIP_OK) st = launch_combine(ctx, plan, D, n, a);
         } else {
             st = launch_splitk(ctx, plan, D, n, a, kv->bits);
@@ -441,6 +441,59 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         if (st != TT_HIP_OK) return st;
     }
     return TT_HIP_OK;
+}
+
+// What a chunk costs by the routes that serve it, in us, from timings at 16 q heads / 2 KV heads of 256, 8 / 2 of 256, 32 / 8 of
+// 128 and 16 / 4 of 64, 512 to 4096 rows behind 0 to 9000 keys, whole and through windows of 1024 and 4096 keys.  `first_blocks`
+// and `last_blocks`: the key blocks its first and its last tile of 32 rows walk.
+
+// One key block of the chunk kernel's step, by how much of the chip takes part (at D = 256 the card's clock follows it).
+static double chunk_step_us(int D, double fill) { return D == 256 ? 0.47 + 0.50 * fill : D == 128 ? 0.41 + 0.22 * fill : 0.45 + 0.05 * fill; }
+
+struct ChunkEstimate {
+    double us;
+    bool single_tiles;  // a workgroup per tile of 32 rows instead of one per pair of them
+};
+// The chunk kernel over all of a tile's keys.  Tiles in pairs (long with short) make workgroups of one length whatever the
+// triangle; a workgroup per tile, the longest first, uses twice the CUs where pairs leave some idle (1024 rows at position
+// 0 39.4 -> 33.5 us, behind 2000 keys 124 -> 77, 2048 rows behind 8000 keys 404 -> 298, 1024 rows of 32 / 8 heads of 128 behind
+// a window of 4096 keys 150 -> 80) and splits the rounds of several finer (2500 rows of 32 / 8 of 128 at position 0
+// 107 -> 80).  Where both need the same rounds pairs are ahead -- the second tile's first blocks ride in behind the first's
+// last: 4096 rows at position 0 138 against 148 us, 2500 rows behind 8000 keys 424 against 464 -- so single tiles have to
+// promise an eighth less.
+static ChunkEstimate estimate_chunk(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int first_blocks, int last_blocks) {
+    // a kv head's workgroups run on its own XCDs where it has whole ones
+    const int xs = (n_kv_heads <= 8 && 8 % n_kv_heads == 0) ? 8 / n_kv_heads : 0;
+    const int cus = xs > 0 ? xs * (ctx->n_cus / 8 > 0 ? ctx->n_cus / 8 : 1) : ctx->n_cus;
+    const int n_tiles = (q_len + 31) / 32, sets = (xs > 0 ? n_q_heads / n_kv_heads : n_q_heads) / 4;
+    const int singles = sets * n_tiles, pairs = sets * ((n_tiles + 1) / 2);
+    const double hi = first_blocks > last_blocks ? first_blocks : last_blocks, lo = first_blocks + last_blocks - hi;
+    // the longest first: no CU is done before its longest tile, before its share of all of them, or, with k rounds begun,
+    // before k + 1 tiles of the length the last of those rounds begins with
+    double by_tile = hi, share = singles * (hi + lo) / 2.0 / cus;
+    if (share > by_tile) by_tile = share;
+    for (int k = 1; k * cus < singles; ++k) {
+        const double round = (k + 1) * (hi - (hi - lo) * (double)(k * cus) / (singles - 1));
+        if (round > by_tile) by_tile = round;
+    }
+    const double by_pair = (double)((pairs + cus - 1) / cus) * (hi + lo);
+    ChunkEstimate e;
+    e.single_tiles = singles <= cus || by_tile < 0.88 * by_pair;
+    const int workgroups = e.single_tiles ? singles : pairs;
+    const double fill = workgroups < cus ? (double)workgroups / cus : 1.0;
+    e.us = (D == 256 ? 11.0 : D == 128 ? 7.0 : 5.0) + (e.single_tiles ? by_tile : by_pair) * chunk_step_us(D, fill);
+    return e;
+}
+
+// The split-K kernel's tiles of 32 packed rows: key blocks per wavefront, dearer while a tile walks few of them.
+static double estimate_splitk_chunk_us(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int first_blocks, int last_blocks) {
+    const int group = n_q_heads / n_kv_heads;
+    int gh = group;
+    while (gh > 32 || group % gh != 0) --gh;
+    const int tt = 32 / gh;
+    const double tiles = (double)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh), blocks = (first_blocks + last_blocks) / 2.0;
+    const double block_us = D == 256 ? 1.6 * (1.0 + 18.0 / blocks) : D == 128 ? 0.87 * (1.0 + 11.0 / blocks) : 0.46 * (1.0 + 8.0 / blocks);
+    return 5.0 + tiles * blocks / (4.0 * ctx->n_cus) * block_us;
 }
 
 }  // namespace tt
@@ -993,15 +1046,28 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
     // 25 us through the split-K tiles; behind a 1024-key window 62 us against 20 us.
     const long long pair_blocks = (2LL * start_pos + q_len) / 32 + 2;  // key blocks a workgroup's pair of tiles walks
     const bool filled = 2 * chunk_wgs >= ctx->n_cus || (window == 0 && 4 * chunk_wgs >= ctx->n_cus && pair_blocks <= 64);
+    // Key blocks that the chunk's tile of rows [32 t, 32 t + 32) walks.
+    auto tile_blocks = [&](int t) {
+        const long long end = std::min<long long>(kv_valid, (long long)start_pos + std::min(q_len, 32 * t + 32));
+        const long long first = window > 0 && start_pos + 32LL * t + 1 > window ? start_pos + 32LL * t + 1 - window : 0;
+        return (int)((end + 31) / 32 - first / 32);
+    };
+    const int first_blocks = tile_blocks(0), last_blocks = tile_blocks((q_len + 31) / 32 - 1);
+    const ChunkEstimate whole = estimate_chunk(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, first_blocks, last_blocks);
+    auto whole_tiles = [&](const PageSource *pages) {
+        if (hipSetDevice(ctx->device) != hipSuccess) return (int)TT_HIP_ERR_HIP;
+        return launch_prefill(ctx, kv, layer, slot, start_pos, q_len, kv_valid, n_q_heads, q, (long long)q_stride, gate,
+                              (long long)gate_stride, scale, out, (long long)o_stride, 1, 0, nullptr, nullptr, pages, window,
+                              whole.single_tiles);
+    };
+    const double splitk_us = estimate_splitk_chunk_us(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, first_blocks, last_blocks);
     if (window > 0) {
-        // The chunk kernel starts every tile at its window's first block; under-filled chunks over a
-        // long window, quantised pages and head groups it does not serve go through the split-K
-        // kernel (GQA-packed tiles, each walking only its rows' windows).
-        if (serves && filled && kv->bits == 16) {
-            if (hipSetDevice(ctx->device) != hipSuccess) return TT_HIP_ERR_HIP;
-            return launch_prefill(ctx, kv, layer, slot, start_pos, q_len, kv_valid, n_q_heads, q, (long long)q_stride, gate,
-                                  (long long)gate_stride, scale, out, (long long)o_stride, 1, 0, nullptr, nullptr, nullptr, window);
-        }
+        // The chunk kernel starts every tile at its window's first block.  It or the split-K kernel (GQA-packed tiles, each
+        // walking only its rows' windows), whichever is estimated faster; quantised pages and head groups the chunk
+        // kernel does not serve go through the latter.  32 / 8 heads of 128 behind a window of 4096 keys: 512 rows 65
+        // against 78 us, 777 rows 105 against 80; 16 / 2 of 256 behind 1024 keys: 512 rows 24 against 34, 777 rows 43
+        // against 34, 1024 rows 47 against 36.
+        if (serves && kv->bits == 16 && (filled || whole.us < splitk_us)) return whole_tiles(nullptr);
         return run_attention(ctx, kv, 0, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride,
                              gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride, 1, 0, nullptr, window);
     }
@@ -1052,6 +1118,7 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
         //    like a verify pass (64 rows at 16k keys 62 us against 89 us; 512 rows at 2k keys
         //    59 us against 104 us, where the partial results outweigh the keys).
         int n_splits = 1, split_blocks = 0;
+        double ranges_us = 0.0;
         if (!filled && q_len >= rows_from && kv_valid >= ranges_from) {
             const int nb_total = (kv_valid + 31) / 32;
             // With ranges a workgroup takes one 32-row tile of 4 heads (not a pair of tiles) over one range of key
@@ -1073,14 +1140,14 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
                     best_us = us;
                     split_blocks = blocks;
                     n_splits = (nb_total + blocks - 1) / blocks;
+                    ranges_us = (double)rounds * blocks * chunk_step_us(kv->head_dim, 1.0) + s * partial_us;
                 }
             }
         }
-        if (filled || (pages && n_splits < 2)) {
-            if (hipSetDevice(ctx->device) != hipSuccess) return TT_HIP_ERR_HIP;
-            return launch_prefill(ctx, kv, layer, slot, start_pos, q_len, kv_valid, n_q_heads, q, (long long)q_stride, gate,
-                                  (long long)gate_stride, scale, out, (long long)o_stride, 1, 0, nullptr, nullptr, pages);
-        }
+        // Unfilled chunks, too, where a workgroup per tile is estimated faster than the ranges (1536 rows behind 8000 keys
+        // 281 -> 237 us) or the split-K tiles (1024 rows behind 2000 keys 84 -> 77 us, 1536 rows 130 -> 92).
+        const bool whole_ahead = q_len >= 256 && whole.us < (n_splits >= 2 ? ranges_us : splitk_us);
+        if (filled || whole_ahead || (pages && n_splits < 2)) return whole_tiles(pages);
         if (n_splits >= 2)
             return run_attention(ctx, kv, 1, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0,
                                  (long long)q_stride, gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride,
