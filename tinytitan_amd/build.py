@@ -1,9 +1,10 @@
-"""Builds libctinytitan_hip.so for gfx950 with hipcc, in-tree."""
+"""Builds libctinytitan_hip.so for gfx950 with hipcc, and the Python module of its per-step calls with g++, in-tree."""
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
@@ -12,6 +13,9 @@ LIB_DIR = os.path.join(PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libctinytitan_hip.so")
 SOURCES = ["context.hip", "kv_cache.hip", "kv_quant.hip", "attn_splitk.hip", "attn_prefill.hip", "qkv_epilogue.hip",
            "affine_proj.hip", "qsa_indexer.hip"]
+
+CALLS_SOURCE = "py_calls.cpp"
+CALLS_PATH = os.path.join(LIB_DIR, "_tt_calls.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -36,11 +40,28 @@ def _compile(src: str, extra) -> str:
     return obj
 
 
+def _build_calls() -> None:
+    """The Python module (host code only): against the header, torch's tensor headers and the interpreter's."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wextra",
+           "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-I", sysconfig.get_paths()["include"], f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH, "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {CALLS_SOURCE}:\n{proc.stderr}")
+    if proc.stderr.strip():
+        sys.stderr.write(proc.stderr)
+
+
 def build(extra_flags=()) -> str:
-    """Compiles every HIP source and links the shared library.  Always recompiles."""
+    """Compiles every source and links the shared library and the Python module.  Always recompiles."""
     os.makedirs(LIB_DIR, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=4) as pool:
+    with ThreadPoolExecutor(max_workers=5) as pool:
+        calls = pool.submit(_build_calls)
         objs = list(pool.map(lambda s: _compile(s, list(extra_flags)), SOURCES))
+        calls.result()
     cmd = [HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB_PATH, *objs]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

@@ -7,12 +7,14 @@ computes needs a gfx950 device.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import re
 from typing import List
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("TT_HIP_LIBRARY", os.path.join(PKG, "lib", "libctinytitan_hip.so"))  # override: a differently built copy
+CALLS_PATH = os.path.join(PKG, "lib", "_tt_calls.so")
 HEADER_PATH = os.path.join(os.path.dirname(PKG), "include", "ctinytitan_hip.h")
 
 OK = 0
@@ -110,6 +112,7 @@ _SIGNATURES = {
 }
 
 _lib = None
+_calls = None
 
 
 class LibraryMissing(RuntimeError):
@@ -136,6 +139,22 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = L
     return _lib
+
+
+def calls():
+    """The module of the per-step calls (csrc/py_calls.cpp), bound to the library that ``lib`` has loaded."""
+    global _calls
+    if _calls is None:
+        lib()
+        if not os.path.exists(CALLS_PATH):
+            raise LibraryMissing(f"{CALLS_PATH} is not built; run `python -m tinytitan_amd.build`.")
+        import torch  # noqa: F401  (the module takes torch tensors: torch's libraries come first)
+        spec = importlib.util.spec_from_file_location("tinytitan_amd._tt_calls", CALLS_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.bind(LIB_PATH)
+        _calls = module
+    return _calls
 
 
 def strerror(status: int) -> str:

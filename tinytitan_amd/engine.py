@@ -12,7 +12,9 @@ Names and argument meaning follow the Swift types this path replaces:
 Tensors are torch fp16 CUDA(HIP) tensors; torch is only the owner of device
 memory here -- every computation happens inside libctinytitan_hip.so.  Swift
 ``throws`` / ``precondition`` failures surface as ``TinyTitanHIPError`` carrying
-the ABI status code.
+the ABI status code.  What a step calls per layer and token goes through
+``capi.calls()`` (tensors checked and the call made in native code), the rest
+through ctypes.
 """
 from __future__ import annotations
 
@@ -49,19 +51,13 @@ def _ptr_raw(t: torch.Tensor) -> int:
     return t.data_ptr()
 
 
-def _ptr16(t: torch.Tensor) -> int:
-    """Device tensor of 16-bit elements passed as raw bit patterns (bfloat16 weights)."""
-    if not t.is_cuda or t.element_size() != 2:
-        raise TypeError("expected a device tensor of 16-bit elements")
-    return t.data_ptr()
-
-
 class HIPContext:
     """Owns the HIP stream, split-K scratch and timing events (``tt_hip_ctx``)."""
 
     def __init__(self, device: int = 0):
         err = ctypes.c_int(0)
         self._lib = capi.lib()
+        self._calls = capi.calls()
         self.handle = self._lib.tt_hip_ctx_create(device, ctypes.byref(err))
         if not self.handle:
             raise TinyTitanHIPError(err.value, "tt_hip_ctx_create")
@@ -190,6 +186,7 @@ class KVCacheManager:
         """``ring_capacity`` > 0: a ring for sliding-window layers (row of position p at p % capacity)."""
         self.ctx = ctx
         self._lib = ctx._lib
+        self._calls = ctx._calls
         if initial_capacity is None:
             initial_capacity = min(max_context, 8192)  # KVCacheManager.swift:270-285
         err = ctypes.c_int(0)
@@ -251,8 +248,9 @@ class KVCacheManager:
             n_tokens = k.numel() // width
         if token_stride is None:
             token_stride = width
-        self.ctx._check(self._lib.tt_hip_kv_append(self.handle, layer, slot, position, n_tokens, _ptr(k), _ptr(v),
-                                                   token_stride), "tt_hip_kv_append")
+        status = self._calls.kv_append(self.handle, layer, slot, position, n_tokens, k, v, token_stride)
+        if status:
+            self.ctx._check(status, "tt_hip_kv_append")
 
     def export_rows(self, layer: int, slot: int, position: int, n_tokens: int):
         """K and V rows in the stored row format, ``[n_tokens][token_stride_bytes]`` uint8 each."""
@@ -343,68 +341,58 @@ class Attention:
 
     def __init__(self, ctx: HIPContext):
         self.ctx = ctx
-        self._lib = ctx._lib
+        self._calls = ctx._calls
 
     def encode_full(self, kv: KVCacheManager, layer: int, q: torch.Tensor, out: torch.Tensor, num_q_heads: int,
                     seq_len, scale: float, slot=0, gate: Optional[torch.Tensor] = None) -> None:
         """``seq_len`` is the exclusive key count (position + 1).  ``slot``/``seq_len`` may be
         lists for the batched form (one query token per sequence)."""
-        slots = list(slot) if isinstance(slot, (list, tuple)) else [slot]
-        lens = list(seq_len) if isinstance(seq_len, (list, tuple)) else [seq_len]
-        if len(slots) != len(lens):
-            raise TinyTitanHIPError(capi.ERR_INVALID_ARGUMENT, "Attention.encode_full")
-        self.ctx._check(self._lib.tt_hip_attn_decode(self.ctx.handle, kv.handle, layer, len(slots),
-                                                     capi.int_array(slots), capi.int_array(lens), num_q_heads,
-                                                     _ptr(q), _ptr(gate), scale, _ptr(out)), "tt_hip_attn_decode")
+        status = self._calls.attn_decode(self.ctx.handle, kv.handle, layer, slot, seq_len, num_q_heads, q, gate, scale, out)
+        if status:
+            self.ctx._check(status, "tt_hip_attn_decode")
 
     def encode_swa(self, kv: KVCacheManager, layer: int, q: torch.Tensor, out: torch.Tensor, num_q_heads: int,
                    seq_len, window: int, scale: float, slot=0, gate: Optional[torch.Tensor] = None) -> None:
         """``Attention.encodeSWA`` (Attention.swift:229-266): keys ``[max(0, seq_len - window), seq_len)``."""
-        slots = list(slot) if isinstance(slot, (list, tuple)) else [slot]
-        lens = list(seq_len) if isinstance(seq_len, (list, tuple)) else [seq_len]
-        if len(slots) != len(lens):
-            raise TinyTitanHIPError(capi.ERR_INVALID_ARGUMENT, "Attention.encode_swa")
-        self.ctx._check(self._lib.tt_hip_attn_decode_swa(self.ctx.handle, kv.handle, layer, len(slots),
-                                                         capi.int_array(slots), capi.int_array(lens), window, num_q_heads,
-                                                         _ptr(q), _ptr(gate), scale, _ptr(out)), "tt_hip_attn_decode_swa")
+        status = self._calls.attn_decode_swa(self.ctx.handle, kv.handle, layer, slot, seq_len, window, num_q_heads, q, gate, scale, out)
+        if status:
+            self.ctx._check(status, "tt_hip_attn_decode_swa")
 
     def encode_full_keep(self, kv: KVCacheManager, layer: int, q: torch.Tensor, out: torch.Tensor, num_q_heads: int,
                          seq_len, keep_mask: torch.Tensor, scale: float, slot=0, gate: Optional[torch.Tensor] = None,
                          keep_stride: Optional[int] = None) -> None:
         """``Attention.encodeFull(..., keepMask:)``: ``keep_mask`` is a uint8 device tensor, one byte per key
         position (0 drops the key); for several sequences their masks are ``keep_stride`` bytes apart."""
-        slots = list(slot) if isinstance(slot, (list, tuple)) else [slot]
-        lens = list(seq_len) if isinstance(seq_len, (list, tuple)) else [seq_len]
-        if len(slots) != len(lens) or keep_mask.dtype != torch.uint8:
+        if keep_mask.dtype != torch.uint8:
             raise TinyTitanHIPError(capi.ERR_INVALID_ARGUMENT, "Attention.encode_full_keep")
-        self.ctx._check(self._lib.tt_hip_attn_decode_keep(self.ctx.handle, kv.handle, layer, len(slots),
-                                                          capi.int_array(slots), capi.int_array(lens), _ptr_raw(keep_mask),
-                                                          keep_stride if keep_stride is not None else max(lens),
-                                                          num_q_heads, _ptr(q), _ptr(gate), scale, _ptr(out)),
-                        "tt_hip_attn_decode_keep")
+        if keep_stride is None:
+            keep_stride = max(seq_len) if isinstance(seq_len, (list, tuple)) else seq_len
+        status = self._calls.attn_decode_keep(self.ctx.handle, kv.handle, layer, slot, seq_len, keep_mask, keep_stride, num_q_heads, q,
+                                              gate, scale, out)
+        if status:
+            self.ctx._check(status, "tt_hip_attn_decode_keep")
 
     def encode_full_keep_indices(self, kv: KVCacheManager, layer: int, q: torch.Tensor, out: torch.Tensor, num_q_heads: int,
                                  seq_len, keep_indices: torch.Tensor, keep_counts: torch.Tensor, scale: float, slot=0,
                                  gate: Optional[torch.Tensor] = None, keep_index_stride: Optional[int] = None) -> None:
         """The same selection compacted (``DecodeKeySelection.indices`` / ``.count``): int32 device tensors, per
         sequence a list of key ids ``keep_index_stride`` entries apart and how many of them count."""
-        slots = list(slot) if isinstance(slot, (list, tuple)) else [slot]
-        lens = list(seq_len) if isinstance(seq_len, (list, tuple)) else [seq_len]
-        if len(slots) != len(lens) or keep_indices.dtype != torch.int32 or keep_counts.dtype != torch.int32:
+        if keep_indices.dtype != torch.int32 or keep_counts.dtype != torch.int32:
             raise TinyTitanHIPError(capi.ERR_INVALID_ARGUMENT, "Attention.encode_full_keep_indices")
-        self.ctx._check(self._lib.tt_hip_attn_decode_keep_indices(
-            self.ctx.handle, kv.handle, layer, len(slots), capi.int_array(slots), capi.int_array(lens), _ptr_raw(keep_indices),
-            keep_index_stride if keep_index_stride is not None else keep_indices.shape[-1], _ptr_raw(keep_counts), num_q_heads,
-            _ptr(q), _ptr(gate), scale, _ptr(out)), "tt_hip_attn_decode_keep_indices")
+        status = self._calls.attn_decode_keep_indices(
+            self.ctx.handle, kv.handle, layer, slot, seq_len, keep_indices,
+            keep_index_stride if keep_index_stride is not None else keep_indices.shape[-1], keep_counts, num_q_heads, q, gate, scale, out)
+        if status:
+            self.ctx._check(status, "tt_hip_attn_decode_keep_indices")
 
     def encode_verify_rows(self, kv: KVCacheManager, layer: int, q: torch.Tensor, out: torch.Tensor,
                            num_q_heads: int, start_positions: Sequence[int], rows: int, scale: float,
                            slots: Sequence[int], gate: Optional[torch.Tensor] = None, window: int = 0) -> None:
         """Row r of sequence i attends like a decode at ``start_positions[i] + r`` (over its last ``window`` keys)."""
-        self.ctx._check(self._lib.tt_hip_attn_verify_swa(self.ctx.handle, kv.handle, layer, len(slots),
-                                                         capi.int_array(slots), capi.int_array(start_positions), rows,
-                                                         window, num_q_heads, _ptr(q), _ptr(gate), scale, _ptr(out)),
-                        "tt_hip_attn_verify_swa")
+        status = self._calls.attn_verify_swa(self.ctx.handle, kv.handle, layer, slots, start_positions, rows, window, num_q_heads, q,
+                                             gate, scale, out)
+        if status:
+            self.ctx._check(status, "tt_hip_attn_verify_swa")
 
 
 @dataclass
@@ -424,7 +412,7 @@ class PrefillAttentionParams:
 class PrefillAttention:
     def __init__(self, ctx: HIPContext):
         self.ctx = ctx
-        self._lib = ctx._lib
+        self._calls = ctx._calls
 
     def encode_causal(self, kv: KVCacheManager, layer: int, slot: int, q: torch.Tensor, out: torch.Tensor,
                       params: PrefillAttentionParams, gate: Optional[torch.Tensor] = None,
@@ -436,35 +424,31 @@ class PrefillAttention:
         ``keep_index_stride`` / ``keep_counts``: the same selection compacted (int32 key ids per query and how
         many of them), as ``encodeCausal`` takes it for the tiled kernel."""
         p = params
+        gate_stride = p.gate_stride or p.q_stride
         if keep_indices is not None:
             if (keep_counts is None or keep_mask is not None or p.sliding_window or keep_indices.dtype != torch.int32
                     or keep_counts.dtype != torch.int32):
                 raise TinyTitanHIPError(capi.ERR_INVALID_ARGUMENT, "PrefillAttention.encode_causal")
-            self.ctx._check(self._lib.tt_hip_attn_prefill_keep_indices(
-                self.ctx.handle, kv.handle, layer, slot, p.start_position, p.query_count, p.kv_valid_count,
-                _ptr_raw(keep_indices), keep_index_stride or keep_indices.shape[-1], _ptr_raw(keep_counts), p.num_q_heads,
-                _ptr(q), p.q_stride, _ptr(gate), p.gate_stride or p.q_stride, p.scale, _ptr(out), p.o_stride),
-                "tt_hip_attn_prefill_keep_indices")
+            status = self._calls.attn_prefill_keep_indices(
+                self.ctx.handle, kv.handle, layer, slot, p.start_position, p.query_count, p.kv_valid_count, keep_indices,
+                keep_index_stride or keep_indices.shape[-1], keep_counts, p.num_q_heads, q, p.q_stride, gate, gate_stride, p.scale, out,
+                p.o_stride)
+            if status:
+                self.ctx._check(status, "tt_hip_attn_prefill_keep_indices")
             return
         if keep_mask is not None:
             if keep_mask.dtype != torch.uint8 or p.sliding_window:
                 raise TinyTitanHIPError(capi.ERR_INVALID_ARGUMENT, "PrefillAttention.encode_causal")
-            self.ctx._check(self._lib.tt_hip_attn_prefill_keep(
-                self.ctx.handle, kv.handle, layer, slot, p.start_position, p.query_count, p.kv_valid_count,
-                _ptr_raw(keep_mask), keep_stride or keep_mask.shape[-1], p.num_q_heads, _ptr(q), p.q_stride, _ptr(gate),
-                p.gate_stride or p.q_stride, p.scale, _ptr(out), p.o_stride), "tt_hip_attn_prefill_keep")
+            status = self._calls.attn_prefill_keep(
+                self.ctx.handle, kv.handle, layer, slot, p.start_position, p.query_count, p.kv_valid_count, keep_mask,
+                keep_stride or keep_mask.shape[-1], p.num_q_heads, q, p.q_stride, gate, gate_stride, p.scale, out, p.o_stride)
+            if status:
+                self.ctx._check(status, "tt_hip_attn_prefill_keep")
             return
-        if p.sliding_window:
-            self.ctx._check(self._lib.tt_hip_attn_prefill_swa(self.ctx.handle, kv.handle, layer, slot, p.start_position,
-                                                              p.query_count, p.kv_valid_count, p.sliding_window,
-                                                              p.num_q_heads, _ptr(q), p.q_stride, _ptr(gate),
-                                                              p.gate_stride or p.q_stride, p.scale, _ptr(out), p.o_stride),
-                            "tt_hip_attn_prefill_swa")
-            return
-        self.ctx._check(self._lib.tt_hip_attn_prefill(self.ctx.handle, kv.handle, layer, slot, p.start_position,
-                                                      p.query_count, p.kv_valid_count, p.num_q_heads, _ptr(q),
-                                                      p.q_stride, _ptr(gate), p.gate_stride or p.q_stride, p.scale,
-                                                      _ptr(out), p.o_stride), "tt_hip_attn_prefill")
+        status = self._calls.attn_prefill(self.ctx.handle, kv.handle, layer, slot, p.start_position, p.query_count, p.kv_valid_count,
+                                          p.sliding_window, p.num_q_heads, q, p.q_stride, gate, gate_stride, p.scale, out, p.o_stride)
+        if status:
+            self.ctx._check(status, "tt_hip_attn_prefill_swa" if p.sliding_window else "tt_hip_attn_prefill")
 
 
 class QKVEpilogue:
@@ -475,7 +459,7 @@ class QKVEpilogue:
 
     def __init__(self, ctx: HIPContext):
         self.ctx = ctx
-        self._lib = ctx._lib
+        self._calls = ctx._calls
 
     def encode(self, kv: KVCacheManager, layer: int, q_packed: torch.Tensor, k_proj: torch.Tensor,
                v_proj: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, q_out: torch.Tensor,
@@ -483,16 +467,13 @@ class QKVEpilogue:
                theta: float, slots=0, q_packed_stride: Optional[int] = None, kv_stride: Optional[int] = None,
                q_stride: Optional[int] = None, gate_stride: Optional[int] = None) -> None:
         """Token ``i * rows + r`` of sequence ``i`` sits at ``positions[i] + r`` of ``slots[i]``."""
-        slot_list = list(slots) if isinstance(slots, (list, tuple)) else [slots]
-        pos_list = list(positions) if isinstance(positions, (list, tuple)) else [positions]
-        if len(slot_list) != len(pos_list):
-            raise TinyTitanHIPError(capi.ERR_INVALID_ARGUMENT, "QKVEpilogue.encode")
         width = num_q_heads * kv.head_dim
-        self.ctx._check(self._lib.tt_hip_qkv_epilogue_append(
-            self.ctx.handle, kv.handle, layer, len(slot_list), capi.int_array(slot_list), capi.int_array(pos_list), rows,
-            num_q_heads, _ptr(q_packed), q_packed_stride or 2 * width, _ptr(k_proj), _ptr(v_proj),
-            kv_stride or kv.kv_heads * kv.head_dim, _ptr16(q_norm_weight), _ptr16(k_norm_weight), eps, rotary_dim, theta,
-            _ptr(q_out), q_stride or width, _ptr(gate_out), gate_stride or width), "tt_hip_qkv_epilogue_append")
+        status = self._calls.qkv_epilogue_append(
+            self.ctx.handle, kv.handle, layer, slots, positions, rows, num_q_heads, q_packed, q_packed_stride or 2 * width, k_proj, v_proj,
+            kv_stride or kv.kv_heads * kv.head_dim, q_norm_weight, k_norm_weight, eps, rotary_dim, theta, q_out, q_stride or width,
+            gate_out, gate_stride or width)
+        if status:
+            self.ctx._check(status, "tt_hip_qkv_epilogue_append")
 
 
 class AffineProjection:
@@ -505,16 +486,17 @@ class AffineProjection:
 
     def __init__(self, ctx: HIPContext):
         self.ctx = ctx
-        self._lib = ctx._lib
+        self._calls = ctx._calls
 
     def encode(self, weight_bits: int, weights: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                x: torch.Tensor, y: torch.Tensor, rows: int, columns: int, token_count: int,
                x_stride: Optional[int] = None, y_stride: Optional[int] = None, weights_offset: int = 0) -> None:
         """``weights_offset`` is a byte offset into ``weights`` (the reference binds tensors at offsets
         into one buffer)."""
-        self.ctx._check(self._lib.tt_hip_affine_projection(
-            self.ctx.handle, weight_bits, _ptr_raw(weights) + weights_offset, _ptr16(scales), _ptr16(biases), _ptr(x),
-            _ptr(y), rows, columns, token_count, x_stride or columns, y_stride or rows), "tt_hip_affine_projection")
+        status = self._calls.affine_projection(self.ctx.handle, weight_bits, weights, weights_offset, scales, biases, x, y, rows, columns,
+                                               token_count, x_stride or columns, y_stride or rows)
+        if status:
+            self.ctx._check(status, "tt_hip_affine_projection")
 
 
 @dataclass(frozen=True)
@@ -584,7 +566,7 @@ class QSAIndexer:
                  capacity: int):
         if capacity <= 0:
             raise ValueError("capacity must be positive")
-        self.ctx, self._lib = ctx, ctx._lib
+        self.ctx, self._calls = ctx, ctx._calls
         self.heads, self.head_dim, self.compress_ratio, self.budget = heads, head_dim, compress_ratio, budget
         self.rope_theta, self.capacity = rope_theta, capacity
         self.exactness = QSAExactness(budget, compress_ratio)
@@ -629,9 +611,10 @@ class QSAIndexer:
         raw, pooled = self.layer_buffers(layer)
         first_block = start_position // self.compress_ratio
         block_count = (end - 1) // self.compress_ratio - first_block + 1
-        self.ctx._check(self._lib.tt_hip_qsa_pool_blocks(
-            self.ctx.handle, _ptr(raw), _ptr(pooled), self.head_dim, first_block, block_count, self.compress_ratio, end,
-            _ptr16(key_norm), eps, self.rope_theta), "tt_hip_qsa_pool_blocks")
+        status = self._calls.qsa_pool_blocks(self.ctx.handle, raw, pooled, self.head_dim, first_block, block_count, self.compress_ratio,
+                                             end, key_norm, eps, self.rope_theta)
+        if status:
+            self.ctx._check(status, "tt_hip_qsa_pool_blocks")
 
     def encode_scores(self, layer: int, query_rows: torch.Tensor, query_norm: torch.Tensor, start_position: int,
                       tokens: int, eps: float) -> torch.Tensor:
@@ -639,15 +622,17 @@ class QSAIndexer:
         scores of every block up to the last query's (``encodeScores``, QSAIndexer.swift:271-330, for one token;
         ``encodeScoresPrefill``, :332-403, for a chunk).  Returns the scores ``[tokens][blocks]``."""
         _, pooled = self.layer_buffers(layer)
-        self.ctx._check(self._lib.tt_hip_qsa_norm_rope_rows(
-            self.ctx.handle, _ptr(query_rows), tokens, self.heads, self.head_dim, _ptr16(query_norm), eps,
-            self.rope_theta, start_position, 1), "tt_hip_qsa_norm_rope_rows")
+        status = self._calls.qsa_norm_rope_rows(self.ctx.handle, query_rows, tokens, self.heads, self.head_dim, query_norm, eps,
+                                                self.rope_theta, start_position, 1)
+        if status:
+            self.ctx._check(status, "tt_hip_qsa_norm_rope_rows")
         blocks = (start_position + tokens - 1) // self.compress_ratio + 1
         if self.scores_buf.numel() < blocks * tokens:
             self.scores_buf = torch.zeros(blocks * tokens, dtype=torch.float32, device=self.device)
-        self.ctx._check(self._lib.tt_hip_qsa_block_scores(
-            self.ctx.handle, _ptr(query_rows), _ptr(pooled), self.scores_buf.data_ptr(), blocks, self.head_dim,
-            self.heads, blocks, tokens), "tt_hip_qsa_block_scores")
+        status = self._calls.qsa_block_scores(self.ctx.handle, query_rows, pooled, self.scores_buf, blocks, self.head_dim, self.heads,
+                                              blocks, tokens)
+        if status:
+            self.ctx._check(status, "tt_hip_qsa_block_scores")
         self.scored_blocks_per_row = blocks
         return self.scores_buf[:blocks * tokens].view(tokens, blocks)
 
@@ -664,10 +649,10 @@ class QSAIndexer:
         blocks = position // self.compress_ratio + 1
         if self.scores_buf.numel() < blocks:
             self.scores_buf = torch.zeros(blocks, dtype=torch.float32, device=self.device)
-        self.ctx._check(self._lib.tt_hip_qsa_decode_scores(
-            self.ctx.handle, _ptr(raw), _ptr(pooled), self.head_dim, self.compress_ratio, position + 1, _ptr16(key_norm),
-            _ptr(query_rows), self.heads, _ptr16(query_norm), position, eps, self.rope_theta, self.scores_buf.data_ptr()),
-            "tt_hip_qsa_decode_scores")
+        status = self._calls.qsa_decode_scores(self.ctx.handle, raw, pooled, self.head_dim, self.compress_ratio, position + 1, key_norm,
+                                               query_rows, self.heads, query_norm, position, eps, self.rope_theta, self.scores_buf)
+        if status:
+            self.ctx._check(status, "tt_hip_qsa_decode_scores")
         self.scored_blocks_per_row = blocks
         return self.scores_buf[:blocks].view(1, blocks)
 
@@ -682,10 +667,11 @@ class QSAIndexer:
             self.keep_index_buf = torch.zeros(rows * width, dtype=torch.int32, device=self.device)
         if compact and (self.keep_count_buf is None or self.keep_count_buf.numel() < rows):
             self.keep_count_buf = torch.zeros(rows, dtype=torch.int32, device=self.device)
-        self.ctx._check(self._lib.tt_hip_qsa_select(
-            self.ctx.handle, self.scores_buf.data_ptr(), score_stride, rows, first_visible, self.compress_ratio, width,
-            self.keep_buf.data_ptr() if mask else None, keep_stride, self.keep_index_buf.data_ptr() if compact else None, width,
-            self.keep_count_buf.data_ptr() if compact else None), "tt_hip_qsa_select")
+        status = self._calls.qsa_select(self.ctx.handle, self.scores_buf, score_stride, rows, first_visible, self.compress_ratio, width,
+                                        self.keep_buf if mask else None, keep_stride, self.keep_index_buf if compact else None, width,
+                                        self.keep_count_buf if compact else None)
+        if status:
+            self.ctx._check(status, "tt_hip_qsa_select")
 
     def select_keys(self, visible_keys: int) -> Optional[torch.Tensor]:
         """The decode step's byte mask over ``visible_keys`` cells, or None when everything visible is kept
