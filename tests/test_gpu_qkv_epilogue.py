@@ -105,6 +105,14 @@ def test_verify_rows_of_several_sequences(gpu_ctx):
     kv.close()
 
 
+@pytest.mark.parametrize("H,KH,D,n_seq,rows", [(16, 2, 256, 1, 256), (16, 2, 256, 1, 257), (3, 3, 128, 5, 7), (9, 3, 256, 33, 1),
+                                               (6, 3, 64, 64, 3), (40, 5, 128, 3, 83)])
+def test_heads_per_wavefront_and_split_kv_rows(gpu_ctx, H, KH, D, n_seq, rows):
+    # one access per wavefront up to eight wavefronts a CU (256 tokens of 16 heads on 256 CUs), four beyond; K and V rows in
+    # wavefronts of their own, with KV heads and rows that do not fill a wavefront's lane groups
+    _run(gpu_ctx, H, KH, D, 32, n_seq, rows, [13 * s + 5 for s in range(n_seq)], list(range(n_seq)), seed=H + rows)
+
+
 def test_padded_strides_and_unaligned_buffers(gpu_ctx):
     # strides that are not multiples of 4 halves and buffers starting 1 half in: the scalar path
     kv = _run(gpu_ctx, 8, 2, 128, 32, 1, 70, [9], [0], seed=6, qp_pad=3, kv_pad=5, q_pad=7, g_pad=9, shift=1)

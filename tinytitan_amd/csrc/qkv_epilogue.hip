@@ -39,7 +39,8 @@ struct EpilogueArgs {
     _Float16 *k_layer, *v_layer;
     const unsigned short *q_weight, *k_weight;  // bf16
     long long qp_stride, kv_stride, q_stride, g_stride, page_elems;
-    int n_tokens, rows, n_q_heads, n_kv_heads;
+    int n_tokens, n_seq, rows, n_q_heads, n_kv_heads;
+    int q_runs;   // wavefronts per token of the query slices
     int kv_bits;  // 16: fp16 pages; 8 / 4: quantised pages (every K/V row then takes the row path)
     int rotary_half;
     float eps;
@@ -93,7 +94,8 @@ __device__ __forceinline__ Rotation rotation_for(int rotary_half, const float *f
         if (t * LPS < rotary_half) {  // wave-uniform
             const int i = t * LPS + j;
             const float angle = (float)position * freq[min(i, rotary_half - 1)];
-            const float ct = cosf(angle), st = sinf(angle);
+            float ct, st;
+            sincosf(angle, &st, &ct);  // one argument reduction for both
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 const float cc = __shfl(ct, my_lane + e), ss = __shfl(st, my_lane + e);
@@ -210,12 +212,13 @@ __device__ __forceinline__ void store_quantised(const EpilogueArgs &a, uint8_t *
 }  // namespace
 
 // ALIGNED: every caller pointer is a multiple of 16 bytes and every stride a multiple of 8 halves.
-template <int D, bool ALIGNED>
+// QI: accesses of D/8-lane slices per wavefront of the query part (SPW heads each).
+template <int D, bool ALIGNED, int QI>
 __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a) {
     constexpr int LPS = D / E;     // lanes per slice
     constexpr int SPW = 64 / LPS;  // slices a wavefront holds per access: 2, 4, 8 at D = 256, 128, 64
     extern __shared__ __attribute__((aligned(16))) _Float16 tile[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int sub = lane / LPS;          // which of the wavefront's slices
     const int d0 = (lane % LPS) * E;     // this lane's first dim
     const int wg = blockIdx.x;
@@ -264,41 +267,46 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
     }
 
     if (wg < a.block_wgs + a.row_wgs) {
-        // ---- ragged K/V rows: a lane group per (row, kv head); rows are the head_rows before the
-        // whole blocks and the tail_rows after them (every row of every sequence when there are none)
-        const long long item = ((long long)(wg - a.block_wgs) * 4 + wave) * SPW + sub;
-        const int per_seq = a.head_rows + a.tail_rows;
-        const int n_seq = a.n_tokens / a.rows;
-        const bool active = item < (long long)n_seq * per_seq * a.n_kv_heads;
-        const long long it = active ? item : 0;  // idle lane groups shadow item 0 (no stores)
-        const int rk = (int)(it / a.n_kv_heads), kvh = (int)(it - (long long)rk * a.n_kv_heads);
-        const int seq = rk / per_seq;
-        int row = rk - seq * per_seq;
+        // ---- ragged K/V rows: a lane group per (row, kv head); rows are the head_rows before the whole blocks and the
+        // tail_rows after them (every row of every sequence when there are none).  What a decode step's launch takes is
+        // the chain of one wavefront, so K rows and V rows have wavefronts of their own, the counts are divided in 32
+        // bits (every item is a row of at least 128 bytes of device memory, so they fit) and an angle's sine and
+        // cosine share one argument reduction: one token over 8 bits 4.44 -> 3.78 us, 7 over 4 bits 5.19 -> 4.32,
+        // 4 over 8 bits 4.82 -> 3.97, one over fp16 3.62 -> 3.49.
+        const unsigned item = ((unsigned)(wg - a.block_wgs) * 2 + (unsigned)(wave >> 1)) * SPW + (unsigned)sub;
+        const bool is_v = (wave & 1) != 0;  // wave-uniform
+        const unsigned per_seq = (unsigned)(a.head_rows + a.tail_rows), n_kv = (unsigned)a.n_kv_heads;
+        const bool active = item < (unsigned)a.n_seq * per_seq * n_kv;
+        const unsigned it = active ? item : 0;  // idle lane groups shadow item 0 (no stores)
+        const unsigned rk = it / n_kv, kvh = it - rk * n_kv;
+        const unsigned seq = per_seq == 1 ? rk : rk / per_seq;
+        int row = (int)(rk - seq * per_seq);
         if (row >= a.head_rows) row += a.n_blocks * kBlockTokens;  // skip what the block workgroups cover
-        const int token = seq * a.rows + row;
-        const int position = a.position[seq] + row;  // for the rotation
-        const int stored = a.row0[seq] + row;        // for the page
+        const int token = (int)seq * a.rows + row;
         const long long off = (long long)token * a.kv_stride + (long long)kvh * D + d0;
-        float k[E], v[E], w[E];
-        load_halves<ALIGNED>(k, a.k_proj + off);
-        load_halves<ALIGNED>(v, a.v_proj + off);
-        load_weight(w, a.k_weight, d0);
-        const Rotation rot = rotation_for<LPS>(a.rotary_half, a.freq, position, lane, d0);
-        norm_rope<D>(k, w, a.eps, rot);
-        if (a.kv_bits != 16) {  // wave-uniform
-            const size_t at = ((size_t)a.slot[seq] * a.n_kv_heads + kvh) * (size_t)a.page_elems * 2 +
-                              (size_t)(stored >> 5) * block_bytes(D, a.kv_bits);
-#pragma unroll
-            for (int e = 0; e < E; ++e) k[e] = (float)(_Float16)k[e];  // what the K row holds as fp16
-            store_quantised(a, reinterpret_cast<uint8_t *>(a.k_layer) + at, false, D, stored & 31, d0, k, lane, active);
-            store_quantised(a, reinterpret_cast<uint8_t *>(a.v_layer) + at, true, D, stored & 31, d0, v, lane, active);
-            return;
+        float x[E];
+        load_halves<ALIGNED>(x, (is_v ? a.v_proj : a.k_proj) + off);
+        const int stored = a.row0[seq] + row;  // for the page
+        const size_t page = (size_t)a.slot[seq] * a.n_kv_heads + kvh;
+        if (!is_v) {
+            float w[E];
+            load_weight(w, a.k_weight, d0);
+            const Rotation rot = rotation_for<LPS>(a.rotary_half, a.freq, a.position[seq] + row, lane, d0);
+            norm_rope<D>(x, w, a.eps, rot);
         }
-        if (active) {
-            const size_t page = ((size_t)a.slot[seq] * a.n_kv_heads + kvh) * (size_t)a.page_elems;
-            store_halves<true>(a.k_layer + page + k_offset(D, stored, d0), k);  // one whole 8-dim group
+        if (a.kv_bits != 16) {  // wave-uniform
+            const size_t at = page * (size_t)a.page_elems * 2 + (size_t)(stored >> 5) * block_bytes(D, a.kv_bits);
 #pragma unroll
-            for (int e = 0; e < E; ++e) a.v_layer[page + v_offset(D, stored, d0 + e)] = (_Float16)v[e];
+            for (int e = 0; e < E; ++e) x[e] = (float)(_Float16)x[e];  // what the row holds as fp16
+            store_quantised(a, reinterpret_cast<uint8_t *>(is_v ? a.v_layer : a.k_layer) + at, is_v, D, stored & 31, d0, x, lane, active);
+        } else if (active) {
+            const size_t first = page * (size_t)a.page_elems;
+            if (is_v) {
+#pragma unroll
+                for (int e = 0; e < E; ++e) a.v_layer[first + v_offset(D, stored, d0 + e)] = (_Float16)x[e];
+            } else {
+                store_halves<true>(a.k_layer + first + k_offset(D, stored, d0), x);  // one whole 8-dim group
+            }
         }
         return;
     }
@@ -306,13 +314,12 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
     // ---- query slices: one wavefront per (token, run of QI * SPW q heads); all of the run's loads
     // are in flight before the first is used, and every head shares the token's rotation
     {
-        constexpr int QI = 4;  // accesses per wavefront: 8 / 16 / 32 heads at D = 256 / 128 / 64
-        const int runs = (a.n_q_heads + QI * SPW - 1) / (QI * SPW);
-        const long long item = (long long)(wg - a.block_wgs - a.row_wgs) * 4 + wave;
-        if (item >= (long long)a.n_tokens * runs) return;
+        const unsigned runs = (unsigned)a.q_runs;
+        const unsigned item = (unsigned)(wg - a.block_wgs - a.row_wgs) * 4 + (unsigned)wave;
+        if (item >= (unsigned)a.n_tokens * runs) return;
         const int token = (int)(item / runs);
-        const int head_first = (int)(item - (long long)token * runs) * (QI * SPW);
-        const int seq = token / a.rows;
+        const int head_first = (int)(item - (unsigned)token * runs) * (QI * SPW);
+        const int seq = a.rows == 1 ? token : (int)((unsigned)token / (unsigned)a.rows);
         const int position = a.position[seq] + (token - seq * a.rows);
         float q[QI][E], g[QI][E], w[E];
 #pragma unroll
@@ -337,10 +344,12 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
 }
 
 template <int D>
-static int launch_epilogue_d(tt_hip_ctx *ctx, const EpilogueArgs &args, unsigned grid, bool aligned) {
+static int launch_epilogue_d(tt_hip_ctx *ctx, const EpilogueArgs &args, unsigned grid, bool aligned, int qi) {
     const size_t lds = args.block_wgs > 0 ? (size_t)2 * kBlockTokens * (D + kEpiloguePad) * sizeof(_Float16) : 0;
-    if (aligned) launch_profiled(ctx, qkv_epilogue_kernel<D, true>, dim3(grid), dim3(256), (unsigned)lds, args);
-    else launch_profiled(ctx, qkv_epilogue_kernel<D, false>, dim3(grid), dim3(256), (unsigned)lds, args);
+    if (aligned && qi == 1) launch_profiled(ctx, qkv_epilogue_kernel<D, true, 1>, dim3(grid), dim3(256), (unsigned)lds, args);
+    else if (aligned) launch_profiled(ctx, qkv_epilogue_kernel<D, true, 4>, dim3(grid), dim3(256), (unsigned)lds, args);
+    else if (qi == 1) launch_profiled(ctx, qkv_epilogue_kernel<D, false, 1>, dim3(grid), dim3(256), (unsigned)lds, args);
+    else launch_profiled(ctx, qkv_epilogue_kernel<D, false, 4>, dim3(grid), dim3(256), (unsigned)lds, args);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "qkv_epilogue_kernel launch");
 }
@@ -398,6 +407,7 @@ extern "C" int tt_hip_qkv_epilogue_append(tt_hip_ctx *ctx, tt_hip_kv *kv, int la
     a.g_stride = gate_stride;
     a.page_elems = (long long)kv->page_elems();
     a.n_tokens = n_seq * rows;
+    a.n_seq = n_seq;
     a.rows = rows;
     a.n_q_heads = n_q_heads;
     a.n_kv_heads = KH;
@@ -430,17 +440,25 @@ extern "C" int tt_hip_qkv_epilogue_append(tt_hip_ctx *ctx, tt_hip_kv *kv, int la
     a.block_wgs = a.n_blocks * KH;
     const int spw = 64 / (D / 8);  // slices per wavefront access
     const long long ragged = (long long)n_seq * (a.head_rows + a.tail_rows) * KH;
-    a.row_wgs = (int)((ragged + 4 * spw - 1) / (4 * spw));
-    const long long runs = (n_q_heads + 4 * spw - 1) / (4 * spw);
+    a.row_wgs = (int)((ragged + 2 * spw - 1) / (2 * spw));
+    // Query heads per wavefront: one access's worth while such wavefronts number no more than eight a CU -- what the launch
+    // takes is then one wavefront's chain, and four accesses' norms and rotations make it longer (16 heads of 256: 1 token
+    // 3.49 -> 3.12 us, 32 tokens 5.38 -> 4.69, 100 tokens 4.80 -> 4.09, 160 tokens 5.73 -> 5.28; 256 tokens, eight a CU,
+    // 6.08 -> 5.98) -- and four beyond, which work a token's angles out once for four times the heads (512 tokens 8.13
+    // against 8.33, 32 heads of 128: 1024 tokens 11.45 against 12.71).
+    const long long single = (long long)a.n_tokens * ((n_q_heads + spw - 1) / spw);
+    const int qi = single <= 8LL * ctx->n_cus ? 1 : 4;
+    const long long runs = (n_q_heads + qi * spw - 1) / (qi * spw);
+    a.q_runs = (int)runs;
     const long long q_wgs = ((long long)a.n_tokens * runs + 3) / 4;
     const long long grid = (long long)a.block_wgs + a.row_wgs + q_wgs;
     if (grid > 0x7fffffffLL) return TT_HIP_ERR_SHAPE;
     const bool aligned = (((uintptr_t)q_packed | (uintptr_t)k_proj | (uintptr_t)v_proj | (uintptr_t)q_out | (uintptr_t)gate_out) % 16) == 0 &&
                          (q_packed_stride | kv_stride | q_stride | gate_stride) % 8 == 0;
     switch (D) {
-        case 256: return launch_epilogue_d<256>(ctx, a, (unsigned)grid, aligned);
-        case 128: return launch_epilogue_d<128>(ctx, a, (unsigned)grid, aligned);
-        case 64: return launch_epilogue_d<64>(ctx, a, (unsigned)grid, aligned);
+        case 256: return launch_epilogue_d<256>(ctx, a, (unsigned)grid, aligned, qi);
+        case 128: return launch_epilogue_d<128>(ctx, a, (unsigned)grid, aligned, qi);
+        case 64: return launch_epilogue_d<64>(ctx, a, (unsigned)grid, aligned, qi);
         default: return TT_HIP_ERR_SHAPE;
     }
 }
