@@ -753,3 +753,57 @@ def test_word_path_keeps_the_tails_of_batched_sequences(gpu_ctx, T):
     kv.close()
     for i, (k, v) in enumerate(rows):
         _check(got[i, 0], _oracle_kept(q[i, 0], k, v, masks[i, :T], H, KH, D, 0.125), f"sequence {i} of {T} keys")
+
+
+@pytest.mark.parametrize("bits", [16, 8, 4])
+@pytest.mark.parametrize("D,H,KH", [(256, 16, 2), (256, 40, 2), (128, 8, 4), (64, 24, 2)])
+def test_a_block_s_loads_cover_exactly_the_kept_keys(gpu_ctx, bits, D, H, KH):
+    # A lane fetches its piece of a block only where the piece holds a kept key, so every place in a block is kept once
+    # on its own, in the first and in later blocks of the wavefronts, and a few together; tiles of 16 and of 32 rows,
+    # as a mask of a decode step and as a chunk's lists.  The dropped keys' values are large: one that slipped into a
+    # result would not stay inside the bar.
+    import torch
+    from tinytitan_amd.engine import PrefillAttention, PrefillAttentionParams
+    r = np.random.default_rng(bits + D + H)
+    rows, blocks = 7, 32 * 9
+    T = 32 * blocks + 5
+    groups = [[0, 31], [3, 4], [12, 13, 14, 15], [7, 8, 23, 24], [16], [15, 16], list(range(32)), [28, 29, 30]]
+    picks = np.zeros((2 * blocks, 32), bool)
+    for b in range(2 * blocks):
+        if b % 9 < 6:
+            picks[b, (b * 5 + b // 32) % 32] = True
+        elif b % 9 < 8:
+            picks[b, groups[b // 9 % len(groups)]] = True
+    keep1 = np.zeros(T, np.uint8)
+    keep1[:32 * blocks] = picks[:blocks].reshape(-1)
+    keep1[T - 1] = 1
+    start = T - rows
+    keep_rows = np.zeros((rows, ((T + 3) // 4) * 4), np.uint8)
+    for t in range(rows):
+        shifted = np.roll(picks, 3 * (t // 2), axis=0)[:blocks].reshape(-1)  # neighbours share a selection, or have one apart
+        keep_rows[t, :32 * blocks] = shifted
+        keep_rows[t, start + t] = 1
+        keep_rows[t, start + t + 1:] = 0
+    ever = keep1.astype(bool) | keep_rows[:, :T].any(axis=0)
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    v[~ever] += np.float16(40.0)
+    q = r.standard_normal((rows, H * D)).astype(np.float16)
+    kv = _cache(gpu_ctx, bits, KH, D, T)
+    _append(gpu_ctx, kv, 0, 0, 0, k, v)
+    ks, vs = (k, v) if bits == 16 else (_dequantised(k, bits), _dequantised(v, bits))
+    scale = D ** -0.5
+    got = _decode_keep(gpu_ctx, kv, q[:1].reshape(1, 1, H, D), [T], keep1, H, scale)
+    _check(got.reshape(H, D), _oracle_kept(q[0].reshape(H, D), ks, vs, keep1, H, KH, D, scale).reshape(H, D), f"decode D={D} {H}/{KH} bits {bits}")
+    stride = int(keep_rows.sum(axis=1).max())
+    lists, counts = np.zeros((rows, stride), np.int32), keep_rows.sum(axis=1).astype(np.int32)
+    for t in range(rows):
+        lists[t, :counts[t]] = np.flatnonzero(keep_rows[t])
+    qd, out = _dev(q), torch.full((rows, H * D), float("nan"), dtype=torch.float16, device="cuda")
+    lists_d, counts_d = _dev(lists), _dev(counts)
+    torch.cuda.synchronize()
+    PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, T, H, scale, H * D, H * D, H * D),
+                                            keep_indices=lists_d, keep_index_stride=stride, keep_counts=counts_d)
+    gpu_ctx.synchronize()
+    kv.close()
+    want = _oracle_rows_kept(q, ks, vs, start, keep_rows, H, KH, D, scale)
+    _check(out.float().cpu().numpy(), want, f"lists D={D} {H}/{KH} bits {bits}")

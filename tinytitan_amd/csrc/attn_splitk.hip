@@ -211,34 +211,63 @@ __device__ __forceinline__ h8 buf_load_h8(__amdgpu_buffer_rsrc_t rsrc, unsigned 
 // to memory -- the lane offset is what the hardware's range check is defined on.
 constexpr unsigned kVoidLoad = 0x7ff00000u;
 
+// What is added to a lane's offsets for the loads of one block: by the keys the lane's load holds, where a selection
+// names them.  A touched block of a sparse selection often holds one kept group of four keys: the lanes of K then
+// fetch those keys' 16-byte pieces instead of all 32, and a step of V whose sixteen keys are all dropped is not
+// fetched; a dropped key's elements read as zeros, under a score that the selection masks and a probability of 0.
+// (128 rows with a selection each behind 131k keys 189 -> 162 us, a decode step's row there 18.1 -> 16.4; loads of V lines
+// that hold one kept group remain.)
+template <int D, int NT>
+struct Voids {
+    unsigned all;   // the block as a whole (parameters of quantised pages)
+    unsigned k[2];  // 32 rows: [0]; 16 rows: tile a, tile b
+    unsigned v[2];  // 32 rows: key step t; 16 rows: [0]
+    __device__ __forceinline__ explicit Voids(unsigned void_bytes) : all(void_bytes), k{void_bytes, void_bytes}, v{void_bytes, void_bytes} {}
+    // `keys`: bit i set = key i of the block is kept by some row of the tile.
+    __device__ __forceinline__ Voids(unsigned void_bytes, unsigned keys, const Lane<D, NT> &ln) : all(void_bytes) {
+        auto unless = [&](unsigned mask) { return (keys & mask) ? void_bytes : kVoidLoad; };
+        if constexpr (NT == 32) {
+            k[0] = k[1] = unless(1u << ln.li);
+            v[0] = unless(0x0f0fu << (4 * ln.g));
+            v[1] = unless(0x0f0f0000u << (4 * ln.g));
+        } else {
+            const int ka = ln.li < 8 ? ln.li : ln.li + 8;
+            k[0] = unless(1u << ka);
+            k[1] = unless(256u << ka);
+            v[0] = v[1] = unless(0x0f0fu << (16 * (ln.g >> 1) + 4 * (ln.g & 1)));
+        }
+    }
+};
+
 template <int AUX, int D, int NT>
 __device__ __forceinline__ void load_k(KTile<D, NT> &t, __amdgpu_buffer_rsrc_t rk, unsigned block_bytes,
-                                       const Lane<D, NT> &ln, unsigned void_bytes = 0) {
-    const unsigned lane_bytes = (unsigned)ln.koff * 2u + void_bytes;
+                                       const Lane<D, NT> &ln, const Voids<D, NT> &vo) {
+    const unsigned lane_bytes = (unsigned)ln.koff * 2u;
     if constexpr (NT == 32) {
 #pragma unroll
-        for (int s = 0; s < D / 16; ++s) t.f[s] = buf_load_h8<AUX>(rk, lane_bytes, block_bytes + s * (2 * 32 * 16));
+        for (int s = 0; s < D / 16; ++s) t.f[s] = buf_load_h8<AUX>(rk, lane_bytes + vo.k[0], block_bytes + s * (2 * 32 * 16));
     } else {
 #pragma unroll
         for (int s = 0; s < D / 32; ++s) {
-            t.a[s] = buf_load_h8<AUX>(rk, lane_bytes, block_bytes + s * (4 * 32 * 16));
-            t.b[s] = buf_load_h8<AUX>(rk, lane_bytes, block_bytes + s * (4 * 32 * 16) + 128);
+            t.a[s] = buf_load_h8<AUX>(rk, lane_bytes + vo.k[0], block_bytes + s * (4 * 32 * 16));
+            t.b[s] = buf_load_h8<AUX>(rk, lane_bytes + vo.k[1], block_bytes + s * (4 * 32 * 16) + 128);
         }
     }
 }
 
 template <int AUX, int D, int NT>
 __device__ __forceinline__ void load_v(VTile<D, NT> &t, __amdgpu_buffer_rsrc_t rv, unsigned block_bytes,
-                                       const Lane<D, NT> &ln, unsigned void_bytes = 0) {
-    const unsigned lane_bytes = (unsigned)ln.voff * 2u + void_bytes;
+                                       const Lane<D, NT> &ln, const Voids<D, NT> &vo) {
+    const unsigned lane_bytes = (unsigned)ln.voff * 2u;
     if constexpr (NT == 32) {
 #pragma unroll
         for (int mt = 0; mt < D / 32; ++mt)
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) t.f[mt][tt] = buf_load_h8<AUX>(rv, lane_bytes, block_bytes + mt * (32 * 4 * 16) + tt * 32);
+            for (int tt = 0; tt < 2; ++tt)
+                t.f[mt][tt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[tt], block_bytes + mt * (32 * 4 * 16) + tt * 32);
     } else {
 #pragma unroll
-        for (int mt = 0; mt < D / 16; ++mt) t.f[mt] = buf_load_h8<AUX>(rv, lane_bytes, block_bytes + mt * (16 * 4 * 16));
+        for (int mt = 0; mt < D / 16; ++mt) t.f[mt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[0], block_bytes + mt * (16 * 4 * 16));
     }
 }
 
@@ -476,8 +505,8 @@ __device__ __forceinline__ void block_softmax_pv(RowState<D, NT> &st, Scores<D, 
 // behind a wait for every load, and nothing of the next block is in flight under the arithmetic of this one.
 template <int AUX, int D>
 __device__ __forceinline__ void block_scores_refill(Scores<D, 32> &sc, KTile<D, 32> &kt, const h8 *qf, __amdgpu_buffer_rsrc_t rk,
-                                                    unsigned next_bytes, const Lane<D, 32> &ln, unsigned void_bytes) {
-    const unsigned lane_bytes = (unsigned)ln.koff * 2u + void_bytes;
+                                                    unsigned next_bytes, const Lane<D, 32> &ln, const Voids<D, 32> &vo) {
+    const unsigned lane_bytes = (unsigned)ln.koff * 2u + vo.k[0];
     sc.s = (f16v)0.0f;
 #pragma unroll
     for (int t = 0; t < D / 16; ++t) {
@@ -490,11 +519,11 @@ __device__ __forceinline__ void block_scores_refill(Scores<D, 32> &sc, KTile<D, 
 template <int AUX, int D>
 __device__ __forceinline__ void block_softmax_pv_refill(RowState<D, 32> &st, Scores<D, 32> &sc, VTile<D, 32> &vt,
                                                         const Lane<D, 32> &ln, int kbase, int lo, int lim, float scale_log2e,
-                                                        __amdgpu_buffer_rsrc_t rv, unsigned next_bytes, unsigned void_bytes,
+                                                        __amdgpu_buffer_rsrc_t rv, unsigned next_bytes, const Voids<D, 32> &vo,
                                                         unsigned kept, const unsigned *row_keep, unsigned row_bits) {
     Probs<D, 32> pr;
     block_softmax<D, 32>(st, sc, pr, ln, kbase, lo, lim, scale_log2e, nullptr, kept, row_keep, row_bits);
-    const unsigned lane_bytes = (unsigned)ln.voff * 2u + void_bytes;
+    const unsigned lane_bytes[2] = {(unsigned)ln.voff * 2u + vo.v[0], (unsigned)ln.voff * 2u + vo.v[1]};
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int mt = 0; mt < D / 32; ++mt) {
@@ -502,7 +531,7 @@ __device__ __forceinline__ void block_softmax_pv_refill(RowState<D, 32> &st, Sco
         for (int t = 0; t < 2; ++t) st.o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vt.f[mt][t], pr.pf[t], st.o[mt], 0, 0, 0);
         asm volatile("" : "+a"(st.o[mt]));
 #pragma unroll
-        for (int t = 0; t < 2; ++t) vt.f[mt][t] = buf_load_h8<AUX>(rv, lane_bytes, next_bytes + mt * (32 * 4 * 16) + t * 32);
+        for (int t = 0; t < 2; ++t) vt.f[mt][t] = buf_load_h8<AUX>(rv, lane_bytes[t], next_bytes + mt * (32 * 4 * 16) + t * 32);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -648,38 +677,38 @@ struct QuantOffsets {
 
 template <int AUX, int D, int NT, int BITS>
 __device__ __forceinline__ void load_k(KTileQ<D, NT, BITS> &t, __amdgpu_buffer_rsrc_t rk, unsigned block_bytes,
-                                       const Lane<D, NT> &ln, unsigned void_bytes = 0) {
+                                       const Lane<D, NT> &ln, const Voids<D, NT> &vo) {
     typedef QuantOffsets<D, NT, BITS> O;
-    const unsigned lane_bytes = O::k_lane(ln) + void_bytes;
+    const unsigned lane_bytes = O::k_lane(ln);
     if constexpr (NT == 32) {
 #pragma unroll
-        for (int p = 0; p < D / 32; ++p) buf_load_words<AUX>(t.f[p], rk, lane_bytes, block_bytes + p * O::K_PAIR);
-        buf_load_words<AUX>(t.sb, rk, (unsigned)ln.li * O::GPH * 4 + void_bytes, block_bytes + O::LEVELS);
+        for (int p = 0; p < D / 32; ++p) buf_load_words<AUX>(t.f[p], rk, lane_bytes + vo.k[0], block_bytes + p * O::K_PAIR);
+        buf_load_words<AUX>(t.sb, rk, (unsigned)ln.li * O::GPH * 4 + vo.k[0], block_bytes + O::LEVELS);
     } else {
 #pragma unroll
         for (int p = 0; p < D / 64; ++p) {
-            buf_load_words<AUX>(t.a[p], rk, lane_bytes, block_bytes + p * O::K_PAIR);
-            buf_load_words<AUX>(t.b[p], rk, lane_bytes, block_bytes + p * O::K_PAIR + 8 * O::K_UNIT);
+            buf_load_words<AUX>(t.a[p], rk, lane_bytes + vo.k[0], block_bytes + p * O::K_PAIR);
+            buf_load_words<AUX>(t.b[p], rk, lane_bytes + vo.k[1], block_bytes + p * O::K_PAIR + 8 * O::K_UNIT);
         }
         const unsigned ka = ln.li < 8 ? ln.li : ln.li + 8;
-        buf_load_words<AUX>(t.sba, rk, ka * O::GPH * 4 + void_bytes, block_bytes + O::LEVELS);
-        buf_load_words<AUX>(t.sbb, rk, ka * O::GPH * 4 + void_bytes, block_bytes + O::LEVELS + 8 * O::GPH * 4);
+        buf_load_words<AUX>(t.sba, rk, ka * O::GPH * 4 + vo.k[0], block_bytes + O::LEVELS);
+        buf_load_words<AUX>(t.sbb, rk, ka * O::GPH * 4 + vo.k[1], block_bytes + O::LEVELS + 8 * O::GPH * 4);
     }
 }
 
 template <int AUX, int D, int NT, int BITS>
 __device__ __forceinline__ void load_v(VTileQ<D, NT, BITS> &t, __amdgpu_buffer_rsrc_t rv, unsigned block_bytes,
-                                       const Lane<D, NT> &ln, unsigned void_bytes = 0) {
+                                       const Lane<D, NT> &ln, const Voids<D, NT> &vo) {
     typedef QuantOffsets<D, NT, BITS> O;
-    const unsigned lane_bytes = O::v_lane(ln) + void_bytes;  // (row * 4 + chunk) runs
-    const unsigned param_lane = (unsigned)ln.g * 16 + void_bytes;
+    const unsigned lane_bytes = O::v_lane(ln);  // (row * 4 + chunk) runs
+    const unsigned param_lane = (unsigned)ln.g * 16 + vo.all;
     // Bias rows: lane rows 0 .. GPH-1 carry a group's biases, the others read zeros (void load).
-    const unsigned bias_lane = (unsigned)ln.li * 64 + (unsigned)ln.g * 16 + ((unsigned)ln.li < O::GPH ? void_bytes : kVoidLoad);
+    const unsigned bias_lane = (unsigned)ln.li * 64 + (unsigned)ln.g * 16 + ((unsigned)ln.li < O::GPH ? vo.all : kVoidLoad);
     if constexpr (NT == 32) {
 #pragma unroll
         for (int j = 0; j < D / 64; ++j)
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) buf_load_words<AUX>(t.f[j][tt], rv, lane_bytes, block_bytes + (j * 32 * 4 + tt * 2) * O::V_RUN);
+            for (int tt = 0; tt < 2; ++tt) buf_load_words<AUX>(t.f[j][tt], rv, lane_bytes + vo.v[tt], block_bytes + (j * 32 * 4 + tt * 2) * O::V_RUN);
 #pragma unroll
         for (int grp = 0; grp < (int)O::GPH; ++grp)
 #pragma unroll
@@ -688,7 +717,7 @@ __device__ __forceinline__ void load_v(VTileQ<D, NT, BITS> &t, __amdgpu_buffer_r
         for (int tt = 0; tt < 2; ++tt) buf_load_words<AUX>(t.bias[tt], rv, bias_lane, block_bytes + O::LEVELS + O::GPH * 64 + tt * 32);
     } else {
 #pragma unroll
-        for (int i = 0; i < D / 32; ++i) buf_load_words<AUX>(t.f[i], rv, lane_bytes, block_bytes + i * 16 * 4 * O::V_RUN);
+        for (int i = 0; i < D / 32; ++i) buf_load_words<AUX>(t.f[i], rv, lane_bytes + vo.v[0], block_bytes + i * 16 * 4 * O::V_RUN);
 #pragma unroll
         for (int grp = 0; grp < (int)O::GPH; ++grp) buf_load_words<AUX>(t.sc[grp], rv, param_lane, block_bytes + O::LEVELS + grp * 64);
         buf_load_words<AUX>(t.bias, rv, bias_lane, block_bytes + O::LEVELS + O::GPH * 64);
@@ -701,19 +730,19 @@ __device__ __forceinline__ void load_v(VTileQ<D, NT, BITS> &t, __amdgpu_buffer_r
 // has a whole block of work between issue and use -- a tile that was refilled in one piece
 // after the phase had only the other phase (levels are half the bytes of fp16 values, so half
 // as much was in flight), and the wave stood waiting for memory twice per block.  `next_bytes` /
-// `void_bytes` address the next block as in load_k; the scale/bias words of K are fetched into
+// `vo` address the next block as in load_k; the scale/bias words of K are fetched into
 // spare registers first and swapped in at the end.
 template <int AUX, int D, int NT, int BITS>
 __device__ __forceinline__ void block_scores(Scores<D, NT> &sc, KTileQ<D, NT, BITS> &kt, const h8 *qf, const h8 *qlds, int lane,
                                              __amdgpu_buffer_rsrc_t rk, unsigned next_bytes, const Lane<D, NT> &ln,
-                                             unsigned void_bytes) {
+                                             const Voids<D, NT> &vo) {
     typedef QuantOffsets<D, NT, BITS> O;
     constexpr int GPH = D / 64;
-    const unsigned lane_bytes = O::k_lane(ln) + void_bytes;
+    const unsigned lane_bytes = O::k_lane(ln);
     (void)qf;
     if constexpr (NT == 32) {
         unsigned sb_next[GPH];
-        buf_load_words<AUX>(sb_next, rk, (unsigned)ln.li * GPH * 4 + void_bytes, next_bytes + O::LEVELS);
+        buf_load_words<AUX>(sb_next, rk, (unsigned)ln.li * GPH * 4 + vo.k[0], next_bytes + O::LEVELS);
         sc.s = (f16v)0.0f;
         h8 q = qlds[lane];
 #pragma unroll
@@ -725,7 +754,7 @@ __device__ __forceinline__ void block_scores(Scores<D, NT> &sc, KTileQ<D, NT, BI
             sc.s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k0, q, sc.s, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             const h8 k1 = k_unit_operand<BITS>(kt.f[p], 1, kt.sb[p / 2]);
-            buf_load_words<AUX>(kt.f[p], rk, lane_bytes, next_bytes + p * O::K_PAIR);
+            buf_load_words<AUX>(kt.f[p], rk, lane_bytes + vo.k[0], next_bytes + p * O::K_PAIR);
             sc.s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k1, q1, sc.s, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             q = q_next;
@@ -735,8 +764,8 @@ __device__ __forceinline__ void block_scores(Scores<D, NT> &sc, KTileQ<D, NT, BI
     } else {
         unsigned sba_next[GPH], sbb_next[GPH];
         const unsigned ka = ln.li < 8 ? ln.li : ln.li + 8;
-        buf_load_words<AUX>(sba_next, rk, ka * GPH * 4 + void_bytes, next_bytes + O::LEVELS);
-        buf_load_words<AUX>(sbb_next, rk, ka * GPH * 4 + void_bytes, next_bytes + O::LEVELS + 8 * GPH * 4);
+        buf_load_words<AUX>(sba_next, rk, ka * GPH * 4 + vo.k[0], next_bytes + O::LEVELS);
+        buf_load_words<AUX>(sbb_next, rk, ka * GPH * 4 + vo.k[1], next_bytes + O::LEVELS + 8 * GPH * 4);
         sc.sa = (f4)0.0f;
         sc.sb = (f4)0.0f;
         h8 q = qlds[lane];
@@ -750,10 +779,10 @@ __device__ __forceinline__ void block_scores(Scores<D, NT> &sc, KTileQ<D, NT, BI
             sc.sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0, q, sc.sb, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             const h8 a1 = k_unit_operand<BITS>(kt.a[p], 1, kt.sba[p]);
-            buf_load_words<AUX>(kt.a[p], rk, lane_bytes, next_bytes + p * O::K_PAIR);
+            buf_load_words<AUX>(kt.a[p], rk, lane_bytes + vo.k[0], next_bytes + p * O::K_PAIR);
             sc.sa = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, q1, sc.sa, 0, 0, 0);
             const h8 b1 = k_unit_operand<BITS>(kt.b[p], 1, kt.sbb[p]);
-            buf_load_words<AUX>(kt.b[p], rk, lane_bytes, next_bytes + p * O::K_PAIR + 8 * O::K_UNIT);
+            buf_load_words<AUX>(kt.b[p], rk, lane_bytes + vo.k[1], next_bytes + p * O::K_PAIR + 8 * O::K_UNIT);
             sc.sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1, q1, sc.sb, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             q = q_next;
@@ -776,13 +805,13 @@ template <int AUX, int D, int NT, int BITS>
 __device__ __forceinline__ void block_softmax_pv(RowState<D, NT> &st, Scores<D, NT> &sc, VTileQ<D, NT, BITS> &vt,
                                                  const Lane<D, NT> &ln, int kbase, int lo, int lim, float scale_log2e,
                                                  typename RowState<D, NT>::acc_t &bias_acc, __amdgpu_buffer_rsrc_t rv,
-                                                 unsigned next_bytes, unsigned void_bytes, unsigned kept = ~0u,
+                                                 unsigned next_bytes, const Voids<D, NT> &vo, unsigned kept = ~0u,
                                                  const unsigned *row_keep = nullptr, unsigned row_bits = ~0u) {
     typedef QuantOffsets<D, NT, BITS> O;
     constexpr int GPH = D / 64;
-    const unsigned lane_bytes = O::v_lane(ln) + void_bytes;
-    const unsigned param_lane = (unsigned)ln.g * 16 + void_bytes;
-    const unsigned bias_lane = (unsigned)ln.li * 64 + (unsigned)ln.g * 16 + ((unsigned)ln.li < (unsigned)GPH ? void_bytes : kVoidLoad);
+    const unsigned lane_bytes = O::v_lane(ln);
+    const unsigned param_lane = (unsigned)ln.g * 16 + vo.all;
+    const unsigned bias_lane = (unsigned)ln.li * 64 + (unsigned)ln.g * 16 + ((unsigned)ln.li < (unsigned)GPH ? vo.all : kVoidLoad);
     Probs<D, NT> pr;
     block_softmax<D, NT>(st, sc, pr, ln, kbase, lo, lim, scale_log2e, &bias_acc, kept, row_keep, row_bits);
     if constexpr (NT == 32) {
@@ -805,7 +834,7 @@ __device__ __forceinline__ void block_softmax_pv(RowState<D, NT> &st, Scores<D, 
             for (int j = 0; j < D / 64; ++j) {  // dim tiles 2 j (dims 64 j + row) and 2 j + 1 (32 above), both of group j
                 h8 lo_op, hi_op;
                 v_run_operands<BITS>(vt.f[j][t], lo_op, hi_op);
-                buf_load_words<AUX>(vt.f[j][t], rv, lane_bytes, next_bytes + (j * 32 * 4 + t * 2) * O::V_RUN);
+                buf_load_words<AUX>(vt.f[j][t], rv, lane_bytes + vo.v[t], next_bytes + (j * 32 * 4 + t * 2) * O::V_RUN);
                 st.o[2 * j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo_op, ps[j][t], st.o[2 * j], 0, 0, 0);
                 st.o[2 * j + 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi_op, ps[j][t], st.o[2 * j + 1], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
@@ -828,7 +857,7 @@ __device__ __forceinline__ void block_softmax_pv(RowState<D, NT> &st, Scores<D, 
             const int j = i >> 1, rr = i & 1;
             h8 lo_op, hi_op;
             v_run_operands<BITS>(vt.f[i], lo_op, hi_op);
-            buf_load_words<AUX>(vt.f[i], rv, lane_bytes, next_bytes + i * 16 * 4 * O::V_RUN);
+            buf_load_words<AUX>(vt.f[i], rv, lane_bytes + vo.v[0], next_bytes + i * 16 * 4 * O::V_RUN);
             st.o[4 * j + rr] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo_op, ps[j], st.o[4 * j + rr], 0, 0, 0);
             st.o[4 * j + 2 + rr] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi_op, ps[j], st.o[4 * j + 2 + rr], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
@@ -1036,13 +1065,17 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     // of the entry after next and the row's bits of the next two entries are always on their way.
     const int *plan_blocks_tile = nullptr;
     const unsigned *plan_bits_tile = nullptr;
-    int e_at = 0, e_hi = 0, walked = 0, after_block = 0;
+    int e_at = 0, e_hi = 0, walked = 0;
+    typedef int i2 __attribute__((ext_vector_type(2)));
+    i2 after_entry = {0, 0};  // block, keys of it that any token keeps
+    unsigned first_keys = ~0u, nxt_keys = ~0u;
     unsigned bits_cur = ~0u, bits_next = ~0u, bits_after = ~0u;
     const int bits_col = valid ? t_local : 0;
-    auto plan_block = [&](int k) {  // block of the wavefront's k-th entry (a load; every lane the same word)
+    auto plan_entry = [&](int k) {  // the wavefront's k-th entry (a load; every lane the same words)
         const int e = e_at + k * WAVES;
-        const int got = plan_blocks_tile[e < e_hi ? e : 0];
-        return e < e_hi ? got : b_end;
+        const i2 got = *reinterpret_cast<const i2 *>(plan_blocks_tile + 2 * (size_t)(e < e_hi ? e : 0));
+        const i2 none = {b_end, 0};
+        return e < e_hi ? got : none;
     };
     auto plan_row_bits = [&](int k) {
         const int e = e_at + k * WAVES;
@@ -1053,18 +1086,21 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         const int *ranges = args.plan_ranges + (size_t)ti.tok_tile * (a.n_splits_max + 1) + split;
         e_at = __builtin_amdgcn_readfirstlane(ranges[0]) + wave;
         e_hi = __builtin_amdgcn_readfirstlane(ranges[1]);
-        plan_blocks_tile = args.plan_blocks + (size_t)ti.tok_tile * args.plan_cap;
+        plan_blocks_tile = args.plan_blocks + (size_t)ti.tok_tile * args.plan_cap * 2;
         plan_bits_tile = args.plan_bits + (size_t)ti.tok_tile * args.plan_cap * a.tt;
-        const int b0 = plan_block(0), b1 = plan_block(1);
-        after_block = plan_block(2);
+        const i2 e0 = plan_entry(0), e1 = plan_entry(1);
+        after_entry = plan_entry(2);
         bits_cur = plan_row_bits(0);
         bits_next = plan_row_bits(1);
-        b = __builtin_amdgcn_readfirstlane(b0);
-        nxt = __builtin_amdgcn_readfirstlane(b1);
+        b = __builtin_amdgcn_readfirstlane(e0[0]);
+        first_keys = (unsigned)__builtin_amdgcn_readfirstlane(e0[1]);
+        nxt = __builtin_amdgcn_readfirstlane(e1[0]);
+        nxt_keys = (unsigned)__builtin_amdgcn_readfirstlane(e1[1]);
     }
     const bool first_real = b < b_end;
     const unsigned first_bytes = first_real ? (unsigned)(a.ring_blocks ? b % a.ring_blocks : b) * BLK_BYTES : 0u;
-    const unsigned first_void = first_real ? 0u : kVoidLoad;
+    Voids<D, NT> first_void(first_real ? 0u : kVoidLoad);
+    if constexpr (KEEP == 3) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
     load_k<AUX>(kt, rk, first_bytes, ln, first_void);
     __builtin_amdgcn_sched_barrier(0);  // the first block's K loads are issued HERE, before the query is waited for
     if constexpr (KEEP == 1) {
@@ -1143,6 +1179,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         int nb = b + WAVES;
         unsigned kept = ~0u;
         bool next_kept = true;
+        unsigned next_keys = ~0u;  // the next block's keys that some row keeps
         const unsigned *row_keep = nullptr;
         if constexpr (KEEP == 1) {
             // the next block and the one after it, off the word of blocks still to do
@@ -1151,7 +1188,8 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
             const int after = todo ? b_first + (__ffsll((long long)todo) - 1) * WAVES : b_end;
             keep_after = __builtin_amdgcn_raw_buffer_load_b8(rkeep, (unsigned)after * 32u + (unsigned)(lane & 31), 0, 0);
             kept = (unsigned)__ballot(keep_cur != 0);  // lanes 32..63 repeat lanes 0..31
-            next_kept = __ballot(keep_next != 0) != 0ull;
+            next_keys = (unsigned)__ballot(keep_next != 0);
+            next_kept = next_keys != 0u;
         }
         if constexpr (KEEP == 2) {
             if (a.keep_words) {
@@ -1173,26 +1211,29 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         unsigned row_bits = ~0u;
         if constexpr (KEEP == 3) {
             nb = nxt;
-            nxt = __builtin_amdgcn_readfirstlane(after_block);
-            after_block = plan_block(walked + 3);
+            next_keys = nxt_keys;
+            nxt = __builtin_amdgcn_readfirstlane(after_entry[0]);
+            nxt_keys = (unsigned)__builtin_amdgcn_readfirstlane(after_entry[1]);
+            after_entry = plan_entry(walked + 3);
             bits_after = plan_row_bits(walked + 2);
             ++walked;
             row_bits = bits_cur;
         }
         const bool real = nb < b_end && next_kept;
         const unsigned next = real ? (unsigned)(a.ring_blocks ? nb % a.ring_blocks : nb) * BLK_BYTES : 0u;
-        const unsigned void_bytes = real ? 0u : kVoidLoad;
+        Voids<D, NT> vo(real ? 0u : kVoidLoad);
+        if constexpr (KEEP == 1 || KEEP == 3) vo = Voids<D, NT>(real ? 0u : kVoidLoad, next_keys, ln);
         if constexpr (BITS == 16 && NT == 32) {
-            block_scores_refill<AUX, D>(sc, kt, qf, rk, next, ln, void_bytes);
-            block_softmax_pv_refill<AUX, D>(st, sc, vt, ln, b << 5, lo, lim, a.scale_log2e, rv, next, void_bytes, kept, row_keep, row_bits);
+            block_scores_refill<AUX, D>(sc, kt, qf, rk, next, ln, vo);
+            block_softmax_pv_refill<AUX, D>(st, sc, vt, ln, b << 5, lo, lim, a.scale_log2e, rv, next, vo, kept, row_keep, row_bits);
         } else if constexpr (BITS == 16) {
             block_scores(sc, kt, qf, qlds, lane);
-            load_k<AUX>(kt, rk, next, ln, void_bytes);
+            load_k<AUX>(kt, rk, next, ln, vo);
             block_softmax_pv<D, NT>(st, sc, vt, ln, b << 5, lo, lim, a.scale_log2e, kept, row_keep, row_bits);
-            load_v<AUX>(vt, rv, next, ln, void_bytes);
+            load_v<AUX>(vt, rv, next, ln, vo);
         } else {  // the phases refill their tiles as they go
-            block_scores<AUX, D, NT, BITS>(sc, kt, qf, qlds, lane, rk, next, ln, void_bytes);
-            block_softmax_pv<AUX, D, NT, BITS>(st, sc, vt, ln, b << 5, lo, lim, a.scale_log2e, bias_acc, rv, next, void_bytes, kept,
+            block_scores<AUX, D, NT, BITS>(sc, kt, qf, qlds, lane, rk, next, ln, vo);
+            block_softmax_pv<AUX, D, NT, BITS>(st, sc, vt, ln, b << 5, lo, lim, a.scale_log2e, bias_acc, rv, next, vo, kept,
                                           row_keep, row_bits);
         }
         if constexpr (KEEP == 1) {

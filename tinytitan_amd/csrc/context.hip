@@ -113,7 +113,8 @@ __global__ __launch_bounds__(256) void keep_rows_from_indices_kernel(uint8_t *ro
 // them entry by entry, sources/TinyTitanCore/Metal/Prefill/prefill.metal:1069-1117) turned into what a tile of `tt`
 // tokens walks here: the ascending list of the 32-key blocks that hold a listed key some token of the tile can see
 // (key < min(kv_valid, start + row + 1), the reference's test of each entry), where every key range of `split_blocks`
-// blocks starts in that list, and per entry and token the listed keys of the block as 32 bits.  One workgroup per
+// blocks starts in that list, per entry the keys of the block that any token keeps, and per entry and token the
+// listed keys, as 32 bits each.  One workgroup per
 // token tile; its work is the tile's list entries plus one pass over a bitmap of the context's blocks in LDS (a bit
 // per block: 4 KiB per million keys) -- nothing of the order rows x context is written or read.  Entries may come in
 // any order and repeat: a bit is set once.
@@ -194,12 +195,12 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
     }
     __syncthreads();
     const int n_touched = (int)partial[T];  // at most min(ctx_blocks, listed entries) <= cap
-    int *my_blocks = blocks + (size_t)tile * cap;
+    int *my_blocks = blocks + (size_t)tile * cap * 2;
     for (int w = tid; w < W; w += T) {
         unsigned word = bitmap[w];
         int at = (int)prefix[w];
         while (word) {
-            my_blocks[at++] = w * 32 + (__ffs((int)word) - 1);
+            my_blocks[2 * at++] = w * 32 + (__ffs((int)word) - 1);
             word &= word - 1u;
         }
     }
@@ -227,6 +228,11 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
         });
         __syncthreads();
         for (int i = tid; i < here * tt; i += T) my_bits[(size_t)first * tt + i] = chunk[i];
+        for (int i = tid; i < here; i += T) {
+            unsigned any = 0u;
+            for (int r = 0; r < tt; ++r) any |= chunk[i * tt + r];
+            my_blocks[2 * (first + i) + 1] = (int)any;
+        }
     }
 }
 
@@ -401,17 +407,17 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             a.seq[i].first_split = first_split[i];
         }
         if (lists) {
-            // The lists' plan, in the context's selection store: [tile][n_splits + 1] range starts, [tile][cap] blocks,
-            // [tile][cap][tt] bits; a tile's list cannot be longer than the context's blocks or its tokens' entries.
+            // The lists' plan, in the context's selection store: [tile][n_splits + 1] range starts, [tile][cap] blocks with
+            // the keys any token keeps (pairs of words, on an even word), [tile][cap][tt] bits; a tile's list cannot be longer than the context's blocks or its tokens' entries.
             const int ctx_blocks = (totals[base] + 31) / 32;
             const long long entries = (long long)plan.tt * (long long)lists->stride;
             const int cap = (int)(entries < ctx_blocks ? entries : ctx_blocks) > 0 ? (int)(entries < ctx_blocks ? entries : ctx_blocks) : 1;
-            const size_t n_ranges = (size_t)plan.tok_tiles * (plan.n_splits_max + 1), n_blocks = (size_t)plan.tok_tiles * cap;
-            st = ensure_keep_rows(ctx, (n_ranges + n_blocks + n_blocks * plan.tt) * sizeof(int));
+            const size_t n_ranges = ((size_t)plan.tok_tiles * (plan.n_splits_max + 1) + 1) & ~(size_t)1, n_blocks = (size_t)plan.tok_tiles * cap;
+            st = ensure_keep_rows(ctx, (n_ranges + 2 * n_blocks + n_blocks * plan.tt) * sizeof(int));
             if (st != TT_HIP_OK) return st;
             int *ranges = reinterpret_cast<int *>(ctx->keep_rows);
             int *blocks = ranges + n_ranges;
-            unsigned *bits = reinterpret_cast<unsigned *>(blocks + n_blocks);
+            unsigned *bits = reinterpret_cast<unsigned *>(blocks + 2 * n_blocks);
             // LDS of the plan kernel: two words per 1,024 keys of context and the run of bits it gathers at a time, 32 KiB
             // of them or what the context's bitmap leaves of 64 KiB.
             const int words = (ctx_blocks + 31) / 32;
@@ -966,7 +972,7 @@ int tt_hip_attn_prefill_keep_indices(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, 
     const int tt = 32 / gh;  // tokens per tile of the 32-row tiles (the planner's own rule)
     const long long ctx_blocks = ((long long)kv_valid + 31) / 32, entries = (long long)tt * (long long)keep_index_stride;
     const long long cap = entries < ctx_blocks ? entries : ctx_blocks;
-    const long long per_tile = (cap * (1 + tt) + 260) * 4;
+    const long long per_tile = (cap * (2 + tt) + 260) * 4;
     long long tiles_per_call = (128ll << 20) / per_tile;
     if (tiles_per_call < 1) tiles_per_call = 1;
     const long long rows_per_call = tiles_per_call * tt;
