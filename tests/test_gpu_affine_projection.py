@@ -211,6 +211,23 @@ def test_gemm_with_the_columns_in_two_parts(gpu_ctx, bits, m, n, tokens, kw):
     assert np.array_equal(_project(gpu_ctx, bits, packed, scales, biases, x[perm], **kw), got[perm])
 
 
+@pytest.mark.parametrize("bits,m,n,tokens,kw", [(4, 2048, 1024, 1024, {}), (8, 2041, 1088, 961, {"x_stride": 1096, "y_stride": 2043}),
+                                                 (4, 2048, 1024, 1025, {}), (8, 2047, 1152, 1536, {"weights_offset": 2}),
+                                                 (4, 1920, 1024, 1537, {"y_stride": 1928}), (4, 2048, 1024, 1537, {})])
+def test_gemm_in_tiles_of_fewer_tokens(gpu_ctx, bits, m, n, tokens, kw):
+    # 16 blocks of 128 rows: tiles of 64 tokens up to 1024 tokens, of 96 up to 1536, of 128 from there (15 blocks: of 96 at 1537 too),
+    # full and ragged last tiles of each.  The bar is that of the tests around this one.
+    packed, scales, biases = _weights(m, n, bits, 105 + bits)
+    x = np.random.default_rng(106).standard_normal((tokens, n)).astype(np.float16)
+    got = _project(gpu_ctx, bits, packed, scales, biases, x, **kw)
+    pick = _sampled(tokens)
+    want = oracle.affine_projection(packed, scales, biases, x[pick].astype(np.float32), bits, half_weights=True)
+    _assert_parity(got[pick], want, _magnitude(packed, scales, biases, x[pick], bits), f"bits={bits} m={m} n={n} tokens={tokens} {kw}")
+    assert np.isfinite(got).all()
+    perm = np.random.default_rng(107).permutation(tokens)
+    assert np.array_equal(_project(gpu_ctx, bits, packed, scales, biases, x[perm], **kw), got[perm])
+
+
 @pytest.mark.parametrize("bits,m,n,tokens,kw", [(8, 2048, 512, 2176, {}), (4, 2000, 320, 2200, {"x_stride": 328, "y_stride": 2003}),
                                                  (4, 2000, 320, 2200, {"weights_offset": 2}), (4, 300, 4096, 16500, {})])
 def test_gemm_in_tiles_of_256_rows(gpu_ctx, bits, m, n, tokens, kw):

@@ -473,39 +473,45 @@ void launch_gemv(tt_hip_ctx *ctx, const ProjArgs &a) {
 // group, in its middle.  The output tile leaves through LDS, [token][row], as 16-byte stores.
 // ---------------------------------------------------------------------------
 constexpr int kGemmTokens = 128, kGemmWaves = 4, kGemmRows = 32 * kGemmWaves;
-// From here on the chunk is a GEMM: 39-40 us up to 1024 tokens and 48 us at 2048, where its grid fills the chip, against
+// From here on the chunk is a GEMM: 28-29 us up to 1024 tokens, 38 beyond and 43 at 2048, where its grid fills the chip, against
 // 26 us at 512 tokens for the tiles above, whose time goes on growing by 25 us per 512 tokens.
 constexpr int kGemmMinTokens = 513;
 constexpr int kGemmThreads = kGemmWaves * 64;
 constexpr int kGemmPitch = kProjGroup + 8;                           // halves per token row of the x tile in LDS
 constexpr int kGemmParamGroups = 64;                                 // groups whose scales and biases sit in LDS at a time
-constexpr int kGemmTileHalves = kGemmTokens * kGemmPitch;
+constexpr int gemm_tile_halves(int tokens) { return tokens * kGemmPitch; }
 constexpr int kGemmOutPitch = kGemmRows + 8;                         // halves per token of the output tile in LDS
-static_assert(kGemmTokens * kGemmOutPitch <= 2 * kGemmTileHalves, "the output tile takes the x tiles' space");
+static_assert(kGemmTokens * kGemmOutPitch <= 2 * gemm_tile_halves(kGemmTokens), "the output tile takes the x tiles' space");
 // KS = parts the columns are split into inside a workgroup (1 or 2): KS x 4 wavefronts, part p's four take the
 // groups [p x part_groups, (p + 1) x part_groups) with x tiles and a block of scales and biases of their own, and
 // the parts' accumulators are added through LDS at the end, in a fixed order.  For chunks whose tiles number no
 // more than the CUs: a workgroup's time is that of ONE wavefront's walk over the columns (44 us at 4096 columns,
 // whatever the number of tiles); in two parts it is 39-40 us, and 48-51 us instead of 56-57 at 2048 tokens, where
 // every CU has a workgroup.
-constexpr int gemm_lds_bytes(int ks) { return ks * 2 * kGemmTileHalves * (int)sizeof(_Float16) + kGemmParamGroups * kGemmRows * 4; }
-constexpr int gemm_rs_lds_bytes() { return 2 * kGemmTileHalves * (int)sizeof(_Float16) + kGemmParamGroups * 2 * kGemmRows * 4; }
+// Its time goes with the tokens of its tile more than with its columns' parts (a third and fourth part of a tile of 64
+// tokens: 31.3 us against 29.1 at 777 tokens, its registers halved), so a chunk that leaves CUs without a workgroup takes
+// tiles of 64 or 96 (TOKENS).
+constexpr int gemm_lds_bytes(int ks, int tokens = kGemmTokens) {
+    return ks * 2 * gemm_tile_halves(tokens) * (int)sizeof(_Float16) + kGemmParamGroups * kGemmRows * 4;
+}
+constexpr int gemm_rs_lds_bytes() { return 2 * gemm_tile_halves(kGemmTokens) * (int)sizeof(_Float16) + kGemmParamGroups * 2 * kGemmRows * 4; }
 
-template <int BITS, bool ALIGNED, int KS, bool RS = false>
+template <int BITS, bool ALIGNED, int KS, bool RS = false, int TOKENS = kGemmTokens>
 __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const ProjArgs a) {
     // RS (with KS = 2): the two parts split the ROWS instead of the columns -- a tile of 128 tokens x 256 rows, one x
     // tile for all eight wavefronts.
     constexpr int kThreads = kGemmThreads * KS, kPartParamGroups = RS ? kGemmParamGroups : kGemmParamGroups / KS;
     constexpr int kRows = RS ? kGemmRows * KS : kGemmRows;
-    constexpr int kStageThreads = RS ? kThreads : kGemmThreads, kStagePasses = kGemmTokens * 8 / kStageThreads;
-    static_assert(kGemmWaves * 64 * 64 * (int)sizeof(float) <= gemm_lds_bytes(2), "the parts' accumulators meet in the store");
-    // per part two x tiles of kGemmTokens x kGemmPitch halves, then per part [kPartParamGroups][kGemmRows] (scale, bias) pairs as fp16
+    constexpr int kStageThreads = RS ? kThreads : kGemmThreads, kStagePasses = TOKENS * 8 / kStageThreads;
+    constexpr int TT = TOKENS / 32;  // 32-token tiles: accumulators of a wavefront
+    static_assert(kGemmWaves * 64 * 16 * TT * (int)sizeof(float) <= gemm_lds_bytes(2, TOKENS), "the parts' accumulators meet in the store");
+    // per part two x tiles of TOKENS x kGemmPitch halves, then per part [kPartParamGroups][kGemmRows] (scale, bias) pairs as fp16
     extern __shared__ __attribute__((aligned(16))) _Float16 lds_store[];
     const int part = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kGemmThreads);
     const int tid = threadIdx.x % kGemmThreads, lane = tid & 63, wave = tid >> 6;  // tid, wave: inside the part
     const int stage_tid = RS ? (int)threadIdx.x : tid;
-    auto tile = [&](int which) { return lds_store + ((RS ? 0 : 2 * part) + which) * kGemmTileHalves; };
-    unsigned *const params = reinterpret_cast<unsigned *>(lds_store + (RS ? 1 : KS) * 2 * kGemmTileHalves) + (RS ? 0 : part * kPartParamGroups * kRows);
+    auto tile = [&](int which) { return lds_store + ((RS ? 0 : 2 * part) + which) * gemm_tile_halves(TOKENS); };
+    unsigned *const params = reinterpret_cast<unsigned *>(lds_store + (RS ? 1 : KS) * 2 * gemm_tile_halves(TOKENS)) + (RS ? 0 : part * kPartParamGroups * kRows);
     const int c = lane & 31, h = lane >> 5;
     // A wavefront owns 32 weight rows against all 128 tokens: every row's levels are widened by exactly one wavefront.
     // Workgroups are dealt to the 8 XCDs in turn, each with its own L2: the workgroups that share a token block
@@ -513,8 +519,8 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     const int row_blocks = (a.rows + kRows - 1) / kRows;
     const int id = blockIdx.x;
     const int token_block = (id & 7) + 8 * (id / (8 * row_blocks));
-    if (token_block * kGemmTokens >= a.tokens) return;  // the whole workgroup, before any barrier: padding of the grid
-    const int token0 = token_block * kGemmTokens, row0 = ((id >> 3) % row_blocks) * kRows;
+    if (token_block * TOKENS >= a.tokens) return;  // the whole workgroup, before any barrier: padding of the grid
+    const int token0 = token_block * TOKENS, row0 = ((id >> 3) % row_blocks) * kRows;
     const int groups = a.columns / kProjGroup;
     constexpr int kHalfGroupBytes = BITS * 4;
     // Levels are read kSpan groups at a time: a lane's 64 contiguous bytes of its row, so that a 128-byte line
@@ -564,7 +570,9 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
         }
     };
     const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    f16v acc[4] = {zero, zero, zero, zero};  // one per 32-token tile
+    f16v acc[TT];  // one per 32-token tile
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) acc[tt] = zero;
 
     // x rows are loaded two groups ahead of their use: slot g % 2 of x_ring holds group g's rows until they go
     // to LDS at the start of group g - 1 (the loop over a span is unrolled and spans are even, so the slot is a
@@ -617,11 +625,11 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     }
     // A fragments of contraction step t of a group: 32 tokens x 16 columns per token tile, af[t % 2]; a step's
     // fragments are read from LDS while the step before it multiplies.
-    h8 af[2][4];
-    auto read_fragments = [&](h8 (&dst)[4], int g, int t) {
+    h8 af[2][TT];
+    auto read_fragments = [&](h8 (&dst)[TT], int g, int t) {
         const _Float16 *xt = tile(g & 1);
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) dst[tt] = *reinterpret_cast<const h8 *>(xt + (32 * tt + c) * kGemmPitch + 32 * h + 8 * t);
+        for (int tt = 0; tt < TT; ++tt) dst[tt] = *reinterpret_cast<const h8 *>(xt + (32 * tt + c) * kGemmPitch + 32 * h + 8 * t);
     };
     read_fragments(af[0], 0, 0);
 
@@ -652,7 +660,7 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
                     read_fragments(af[(t + 1) & 1], g, t + 1);
                 }
 #pragma unroll
-                for (int tt = 0; tt < 4; ++tt)
+                for (int tt = 0; tt < TT; ++tt)
                     acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t & 1][tt], bw[k & 1][t], acc[tt], 0, 0, 0);
                 // a quarter of the next group's fragments per MFMA step (after the last group: made and not used).
                 // The empty statements tie the quarter to this step: without them all four are made in one run
@@ -663,10 +671,10 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
                 widen_scale(bw[(k + 1) & 1][t], w_of_next, t, scale_next, bias_next);
                 asm volatile("" : "+v"(bw[(k + 1) & 1][t]));
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = 0; i < TT; ++i) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
                     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one fragment read
-                    __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // a share of the widening
+                    __builtin_amdgcn_sched_group_barrier(0x002, 20 / TT, 0);  // a share of the widening
                 }
             }
             // The next block of scales and biases is first read one step before its first group is multiplied.
@@ -683,17 +691,17 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     __syncthreads();  // nobody reads an x tile any more
     if constexpr (KS == 2 && !RS) {
         // part 1's accumulators join part 0's: [wavefront][value][lane] floats, every lane its own words
-        float *const sums = reinterpret_cast<float *>(lds_store) + wave * 64 * 64 + lane;
+        float *const sums = reinterpret_cast<float *>(lds_store) + wave * 64 * 16 * TT + lane;
         if (part == 1) {
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
+            for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
                 for (int j = 0; j < 16; ++j) sums[(16 * tt + j) * 64] = acc[tt][j];
         }
         __syncthreads();
         if (part == 0) {
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
+            for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
                 for (int j = 0; j < 16; ++j) acc[tt][j] += sums[(16 * tt + j) * 64];
         }
@@ -713,7 +721,7 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     const int thread = threadIdx.x;
     constexpr int kPieces = kRows / 8;
 #pragma unroll
-    for (int i = 0; i < kGemmTokens * kPieces / kThreads; ++i) {
+    for (int i = 0; i < TOKENS * kPieces / kThreads; ++i) {
         const int at = thread + kThreads * i, local = at / kPieces, piece = at % kPieces;
         const int token = token0 + local, row = row0 + 8 * piece;
         if (token >= a.tokens || row >= a.rows) continue;
@@ -730,10 +738,10 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
 }
 
 // 68 KiB of LDS (104 KiB with two parts): above the 64 KiB a kernel gets without asking.
-template <int BITS, bool ALIGNED, int KS, bool RS = false>
+template <int BITS, bool ALIGNED, int KS, bool RS = false, int TOKENS = kGemmTokens>
 int launch_gemm(tt_hip_ctx *ctx, const ProjArgs &a, dim3 grid) {
-    auto kernel = affine_gemm_kernel<BITS, ALIGNED, KS, RS>;  // its LDS limit was raised when the context was created
-    launch_profiled(ctx, kernel, grid, dim3(kGemmThreads * KS), (unsigned)(RS ? gemm_rs_lds_bytes() : gemm_lds_bytes(KS)), a);
+    auto kernel = affine_gemm_kernel<BITS, ALIGNED, KS, RS, TOKENS>;  // its LDS limit was raised when the context was created
+    launch_profiled(ctx, kernel, grid, dim3(kGemmThreads * KS), (unsigned)(RS ? gemm_rs_lds_bytes() : gemm_lds_bytes(KS, TOKENS)), a);
     return TT_HIP_OK;
 }
 
@@ -752,6 +760,14 @@ int configure_affine_kernels(tt_hip_ctx *ctx) {
     TT_CFG((affine_gemm_kernel<4, false, 2>), gemm_lds_bytes(2))
     TT_CFG((affine_gemm_kernel<8, true, 2>), gemm_lds_bytes(2))
     TT_CFG((affine_gemm_kernel<8, false, 2>), gemm_lds_bytes(2))
+    TT_CFG((affine_gemm_kernel<4, true, 2, false, 64>), gemm_lds_bytes(2, 64))
+    TT_CFG((affine_gemm_kernel<4, true, 2, false, 96>), gemm_lds_bytes(2, 96))
+    TT_CFG((affine_gemm_kernel<4, false, 2, false, 64>), gemm_lds_bytes(2, 64))
+    TT_CFG((affine_gemm_kernel<4, false, 2, false, 96>), gemm_lds_bytes(2, 96))
+    TT_CFG((affine_gemm_kernel<8, true, 2, false, 64>), gemm_lds_bytes(2, 64))
+    TT_CFG((affine_gemm_kernel<8, true, 2, false, 96>), gemm_lds_bytes(2, 96))
+    TT_CFG((affine_gemm_kernel<8, false, 2, false, 64>), gemm_lds_bytes(2, 64))
+    TT_CFG((affine_gemm_kernel<8, false, 2, false, 96>), gemm_lds_bytes(2, 96))
     TT_CFG((affine_gemm_kernel<4, true, 2, true>), gemm_rs_lds_bytes())
     TT_CFG((affine_gemm_kernel<4, false, 2, true>), gemm_rs_lds_bytes())
     TT_CFG((affine_gemm_kernel<8, true, 2, true>), gemm_rs_lds_bytes())
@@ -815,7 +831,7 @@ extern "C" int tt_hip_affine_projection(tt_hip_ctx *ctx, int weight_bits, const 
         const long long padded = (token_blocks + 7) / 8 * 8 * row_blocks;  // token blocks in eights: see the kernel's id mapping
         if (padded > 0x7fffffffLL) return TT_HIP_ERR_SHAPE;
         const dim3 tiles_grid((unsigned)padded);
-        // Three forms of the kernel.  Tiles of 128 rows for no more than the CUs: the columns in two parts inside a
+        // Four forms of the kernel.  Tiles of 128 rows for no more than the CUs: the columns in two parts inside a
         // workgroup.  More than that: tiles of 256 rows, eight wavefronts, one workgroup per CU -- the x tile is then
         // fetched once for twice the rows, and what the card's power limit charges for is traffic (4096 tokens 94.5 ->
         // 87.7 us on one box, 92.7 -> 92.0 on another; 3072 tokens 82.1 -> 75.7; 8192 tokens 176 -> 167) -- unless their
@@ -823,8 +839,20 @@ extern "C" int tt_hip_affine_projection(tt_hip_ctx *ctx, int weight_bits, const 
         // of 128 rows, two workgroups per CU).
         const long long wide_blocks = (rows + 2 * kGemmRows - 1) / (2 * kGemmRows), wide_tiles = token_blocks * wide_blocks;
         const long long last_round = wide_tiles % ctx->n_cus;
+        const bool two_parts = columns / kProjGroup >= 16;
+        const auto tiles = [&](int tokens) { return (token_count + tokens - 1) / tokens * row_blocks; };
+        const auto grid_of = [&](int tokens) { return dim3((unsigned)(((token_count + tokens - 1) / tokens + 7) / 8 * 8 * row_blocks)); };
         int status;
-        if (token_blocks * row_blocks <= ctx->n_cus && columns / kProjGroup >= 16) {
+        if (two_parts && tiles(64) <= ctx->n_cus) {
+            // ... and with fewer tokens a tile while those tiles number no more than the CUs either: at 2048 rows x 4096 columns
+            // tiles of 64 38.0 -> 28.7 us up to 1024 tokens (8-bit levels 41.8 -> 30.5; at 1024 columns 14.4 -> 11.5; at
+            // 1100 tokens, a second workgroup on some CUs, 51.0 against 37.5 the other way), tiles of 96 41.3 -> 35.7 up to 1536.
+            if (weight_bits == 4) status = aligned ? launch_gemm<4, true, 2, false, 64>(ctx, a, grid_of(64)) : launch_gemm<4, false, 2, false, 64>(ctx, a, grid_of(64));
+            else status = aligned ? launch_gemm<8, true, 2, false, 64>(ctx, a, grid_of(64)) : launch_gemm<8, false, 2, false, 64>(ctx, a, grid_of(64));
+        } else if (two_parts && tiles(96) <= ctx->n_cus) {
+            if (weight_bits == 4) status = aligned ? launch_gemm<4, true, 2, false, 96>(ctx, a, grid_of(96)) : launch_gemm<4, false, 2, false, 96>(ctx, a, grid_of(96));
+            else status = aligned ? launch_gemm<8, true, 2, false, 96>(ctx, a, grid_of(96)) : launch_gemm<8, false, 2, false, 96>(ctx, a, grid_of(96));
+        } else if (two_parts && token_blocks * row_blocks <= ctx->n_cus) {
             if (weight_bits == 4) status = aligned ? launch_gemm<4, true, 2>(ctx, a, tiles_grid) : launch_gemm<4, false, 2>(ctx, a, tiles_grid);
             else status = aligned ? launch_gemm<8, true, 2>(ctx, a, tiles_grid) : launch_gemm<8, false, 2>(ctx, a, tiles_grid);
         } else if (wide_tiles <= ctx->n_cus || last_round == 0 || 10 * last_round > 6 * ctx->n_cus) {
