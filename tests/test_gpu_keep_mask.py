@@ -807,3 +807,53 @@ def test_a_block_s_loads_cover_exactly_the_kept_keys(gpu_ctx, bits, D, H, KH):
     kv.close()
     want = _oracle_rows_kept(q, ks, vs, start, keep_rows, H, KH, D, scale)
     _check(out.float().cpu().numpy(), want, f"lists D={D} {H}/{KH} bits {bits}")
+
+
+@pytest.mark.parametrize("split_tokens", [0, 512])
+@pytest.mark.parametrize("D,H,KH,T,rows", [(256, 16, 2, 6003, 38), (128, 32, 8, 9001, 21), (64, 16, 4, 12345, 50), (256, 40, 2, 2050, 5)])
+def test_lists_walked_by_groups_of_keys_equal_the_mask_form(gpu_ctx, D, H, KH, T, rows, split_tokens):
+    # Short lists over a long context are walked by eight groups of four keys at a time: list lengths off a multiple of
+    # eight, key ranges that hold none or a few of a tile's groups, a tile without a key, the context's last, partial
+    # group, and large values in every dropped key.  The oracle over each row's own keys, and the mask form's result.
+    import torch
+    from tinytitan_amd.engine import PrefillAttention, PrefillAttentionParams
+    r = np.random.default_rng(D + T)
+    start, scale = T - rows, D ** -0.5
+    group = H // KH
+    tt = 32 // max(g for g in range(1, 33) if group % g == 0)
+    stride = T // (2 * tt) - 1  # the widest lists that are walked by groups
+    keep = np.zeros((rows, ((T + 3) // 4) * 4), np.uint8)
+    for t in range(rows):
+        n = [1, 7, 8, 9, 40][t % 5]
+        at = r.choice((start + t) // 4, n, replace=False)
+        for g in at[:n]:
+            keep[t, 4 * g + r.integers(0, 4, size=r.integers(1, 5))] = 1
+        keep[t, start + t] = t % 3 != 0
+    keep[tt:2 * tt] = 0  # a whole tile of empty lists
+    lists, counts = r.integers(0, 2 ** 31 - 1, size=(rows, stride)).astype(np.int32), np.zeros(rows, np.int32)
+    for t in range(rows):
+        ids = np.flatnonzero(keep[t])
+        assert len(ids) <= stride
+        r.shuffle(ids)
+        lists[t, :len(ids)], counts[t] = ids, len(ids)
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    v[~keep[:, :T].any(axis=0)] += np.float16(40.0)
+    q, gate = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    kv = _cache(gpu_ctx, 16, KH, D, T)
+    _append(gpu_ctx, kv, 0, 0, 0, k, v)
+    by_mask = _prefill_keep(gpu_ctx, kv, q, start, T, keep, H, scale, gate=gate)
+    qd, gd, lists_d, counts_d = _dev(q), _dev(gate), _dev(lists), _dev(counts)
+    out = torch.full((rows, H * D), float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    gpu_ctx.set_split_tokens(split_tokens)
+    try:
+        PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, T, H, scale, H * D, H * D, H * D),
+                                                gate=gd, keep_indices=lists_d, keep_index_stride=stride, keep_counts=counts_d)
+    finally:
+        gpu_ctx.set_split_tokens(0)
+    gpu_ctx.synchronize()
+    got = out.float().cpu().numpy()
+    kv.close()
+    assert not got[tt:2 * tt].any()
+    assert np.abs(got - by_mask).max() <= 2e-3
+    _check(got, _oracle_rows_kept(q, k, v, start, keep, H, KH, D, scale, gate=gate), f"groups D={D} {H}/{KH}")

@@ -536,6 +536,77 @@ __device__ __forceinline__ void block_softmax_pv_refill(RowState<D, 32> &st, Sco
     }
 }
 
+// Eight listed groups of four keys taken as one block (KEEP = 4): every lane has offsets of its own.  K: a lane's key is one
+// of its group's four, 64 contiguous bytes per 8 dims.  V: the eight keys of a lane's operand are two groups, half a
+// chunk (8 bytes) of each.  A group that is not there has kVoidLoad for an offset.
+struct GroupOffsets {
+    unsigned k;
+    unsigned v[2][2];  // [key step][half of the operand]
+};
+template <int D>
+__device__ __forceinline__ GroupOffsets group_offsets(const int (&ids)[5], const Lane<D, 32> &ln) {
+    constexpr unsigned BLOCK = 32 * D * 2;
+    GroupOffsets o;
+    auto block_at = [&](int id) { return (unsigned)(id >> 3) * BLOCK; };
+    o.k = ids[0] < 0 ? kVoidLoad : block_at(ids[0]) + (unsigned)(ln.g * 32 + 4 * (ids[0] & 7) + (ln.li & 3)) * 16u;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int id = ids[1 + 2 * t + h], j = id & 7;  // keys 4 j .. 4 j + 3 of the block: half (j / 2) % 2 of chunk 2 (j / 4) + j % 2
+            o.v[t][h] = id < 0 ? kVoidLoad : block_at(id) + (unsigned)(ln.li * 64 + (2 * (j >> 2) + (j & 1)) * 16 + ((j >> 1) & 1) * 8);
+        }
+    return o;
+}
+typedef unsigned group_words __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ h8 load_group_pair(__amdgpu_buffer_rsrc_t rv, const unsigned (&at)[2], unsigned wave_bytes) {
+    const group_words lo = __builtin_bit_cast(group_words, __builtin_amdgcn_raw_buffer_load_b64(rv, at[0], wave_bytes, 0));
+    const group_words hi = __builtin_bit_cast(group_words, __builtin_amdgcn_raw_buffer_load_b64(rv, at[1], wave_bytes, 0));
+    const i4 both = {(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
+    return __builtin_bit_cast(h8, both);
+}
+template <int D>
+__device__ __forceinline__ void load_k_groups(KTile<D, 32> &kt, __amdgpu_buffer_rsrc_t rk, const GroupOffsets &o) {
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) kt.f[t] = buf_load_h8<0>(rk, o.k, t * (2 * 32 * 16));
+}
+template <int D>
+__device__ __forceinline__ void load_v_groups(VTile<D, 32> &vt, __amdgpu_buffer_rsrc_t rv, const GroupOffsets &o) {
+#pragma unroll
+    for (int mt = 0; mt < D / 32; ++mt)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) vt.f[mt][t] = load_group_pair(rv, o.v[t], mt * (32 * 4 * 16));
+}
+// The two phases with the next groups' loads between their MFMAs, as in block_scores_refill / block_softmax_pv_refill.
+template <int D>
+__device__ __forceinline__ void group_scores_refill(Scores<D, 32> &sc, KTile<D, 32> &kt, const h8 *qf, __amdgpu_buffer_rsrc_t rk, const GroupOffsets &next) {
+    sc.s = (f16v)0.0f;
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+        sc.s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kt.f[t], qf[t], sc.s, 0, 0, 0);
+        asm volatile("" : "+a"(sc.s));
+        kt.f[t] = buf_load_h8<0>(rk, next.k, t * (2 * 32 * 16));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <int D>
+__device__ __forceinline__ void group_softmax_pv_refill(RowState<D, 32> &st, Scores<D, 32> &sc, VTile<D, 32> &vt, const Lane<D, 32> &ln,
+                                                        float scale_log2e, __amdgpu_buffer_rsrc_t rv, const GroupOffsets &next, unsigned row_bits) {
+    Probs<D, 32> pr;
+    // (the bits say all: a listed key that the row cannot see is not among them)
+    block_softmax<D, 32>(st, sc, pr, ln, 0, 0, 32, scale_log2e, nullptr, ~0u, nullptr, row_bits);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < D / 32; ++mt) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) st.o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vt.f[mt][t], pr.pf[t], st.o[mt], 0, 0, 0);
+        asm volatile("" : "+a"(st.o[mt]));
+#pragma unroll
+        for (int t = 0; t < 2; ++t) vt.f[mt][t] = load_group_pair(rv, next.v[t], mt * (32 * 4 * 16));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Quantised pages (8 or 4 bits per value; layout in kv_layout.h).  A block's tiles hold the
 // levels as loaded plus this lane's scales and biases; levels become fp16 MFMA operands in
@@ -884,6 +955,8 @@ __device__ __forceinline__ void block_softmax_pv(RowState<D, NT> &st, Scores<D, 
 // KEEP = 3: the same selection as per-query index lists (keepIdx / keepCount, prefill.metal:1069-1117), served from the
 // plan keep_plan_kernel makes of them: per token tile the ascending list of key blocks its tokens keep a key of, and per
 // entry and token the kept keys as 32 bits -- the walk costs the selection, never the context.
+// KEEP = 4: the same, where few of a touched block's keys are listed (fp16 pages, tiles of 32): the plan lists groups of
+// four keys, and eight listed groups, wherever they lie, make a turn of the loop.
 // The hot arguments and this workgroup's sequence entry, by three scalar loads issued together (the compiler
 // would fetch each field where it is first used: five or six dependent trips to the kernarg segment before
 // the first K/V load can go out, about 0.15 us each).
@@ -1097,11 +1170,53 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         nxt = __builtin_amdgcn_readfirstlane(e1[0]);
         nxt_keys = (unsigned)__builtin_amdgcn_readfirstlane(e1[1]);
     }
+    // Groups: this wavefront takes runs of eight list positions v, v + WAVES, ... (aligned: a run may reach over the ends of the
+    // split's stretch [g_lo, g_hi), whose outside is void and masked).  A run's ids are asked for two turns ahead, its
+    // row bits one.
+    int run = 0, run_end = 0, g_lo = 0, g_hi = 0;
+    int ids_next[5];
+    GroupOffsets at_next;
+    auto group_ids = [&](int (&ids)[5], int v) {
+        const int place[5] = {li >> 2, g, g + 2, 4 + g, 6 + g};
+        const int base = 8 * min(v, run_end - 1);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            const int p = base + place[i], got = plan_blocks_tile[p];
+            ids[i] = v < run_end && p >= g_lo && p < g_hi ? got : -1;
+        }
+    };
+    auto run_bits = [&](int v) {
+        const unsigned got = plan_bits_tile[(size_t)min(v, run_end - 1) * a.tt + bits_col];
+        const int lo_cut = max(g_lo - 8 * v, 0), hi_cut = g_hi - 8 * v;  // positions of the run inside the stretch: [lo_cut, hi_cut)
+        const unsigned inside = (~0u << (4 * min(lo_cut, 7))) & (hi_cut >= 8 ? ~0u : (1u << (4 * max(hi_cut, 0))) - 1u);
+        return v < run_end && valid ? got & inside : 0u;
+    };
+    if constexpr (KEEP == 4) {
+        const int *ranges = args.plan_ranges + (size_t)ti.tok_tile * (a.n_splits_max + 1) + split;
+        g_lo = __builtin_amdgcn_readfirstlane(ranges[0]);
+        g_hi = __builtin_amdgcn_readfirstlane(ranges[1]);
+        run_end = g_hi > g_lo ? (g_hi + 7) >> 3 : 0;
+        run = (g_lo >> 3) + wave;
+        plan_blocks_tile = args.plan_blocks + (size_t)ti.tok_tile * args.plan_cap;
+        plan_bits_tile = args.plan_bits + (size_t)ti.tok_tile * (args.plan_cap >> 3) * a.tt;
+        b = b_end;  // (the walk over blocks finds nothing)
+    }
     const bool first_real = b < b_end;
     const unsigned first_bytes = first_real ? (unsigned)(a.ring_blocks ? b % a.ring_blocks : b) * BLK_BYTES : 0u;
     Voids<D, NT> first_void(first_real ? 0u : kVoidLoad);
     if constexpr (KEEP == 3) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
-    load_k<AUX>(kt, rk, first_bytes, ln, first_void);
+    if constexpr (KEEP == 4) {
+        if (run_end > 0) {
+            int ids_first[5];
+            group_ids(ids_first, run);
+            group_ids(ids_next, run + WAVES);
+            bits_cur = run_bits(run);
+            at_next = group_offsets<D>(ids_first, ln);
+            load_k_groups<D>(kt, rk, at_next);
+        }
+    } else {
+        load_k<AUX>(kt, rk, first_bytes, ln, first_void);
+    }
     __builtin_amdgcn_sched_barrier(0);  // the first block's K loads are issued HERE, before the query is waited for
     if constexpr (KEEP == 1) {
         const int mine = b_first < b_end ? (b_end - b_first + WAVES - 1) / WAVES : 0;  // this wavefront's blocks, at most 64
@@ -1165,16 +1280,31 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         if constexpr (Q_IN_LDS) qlds[s * 64 + lane] = qf[s];  // read back by this wave only: no barrier
     }
     __builtin_amdgcn_sched_barrier(0);
-    load_v<AUX>(vt, rv, first_bytes, ln, first_void);
+    if constexpr (KEEP == 4) {
+        if (run_end > 0) load_v_groups<D>(vt, rv, at_next);
+    } else {
+        load_v<AUX>(vt, rv, first_bytes, ln, first_void);
+    }
     __builtin_amdgcn_sched_barrier(0);
 
     RowState<D, NT> st;
     st.init();
     typename RowState<D, NT>::acc_t bias_acc = (typename RowState<D, NT>::acc_t)0.0f;  // quantised pages only
+    if constexpr (KEEP == 4) {
+        for (; run < run_end; run += WAVES) {
+            Scores<D, NT> sc;
+            at_next = group_offsets<D>(ids_next, ln);
+            group_ids(ids_next, run + 2 * WAVES);
+            bits_next = run_bits(run + WAVES);
+            group_scores_refill<D>(sc, kt, qf, rk, at_next);
+            group_softmax_pv_refill<D>(st, sc, vt, ln, a.scale_log2e, rv, at_next, bits_cur);
+            bits_cur = bits_next;
+        }
+    }
     // The next block's loads are issued UNCONDITIONALLY (void loads past the split's end).  A branch
     // around them would leave the compiler unable to count the loads in flight, and it would then
     // make the P.V step wait for the next block's K tile as well as for its own V tile.
-    while (b < b_end) {
+    while (KEEP != 4 && b < b_end) {
         Scores<D, NT> sc;
         int nb = b + WAVES;
         unsigned kept = ~0u;
@@ -1622,6 +1752,7 @@ static hipError_t configure_tile() {
     TT_CFG(16, 1) TT_CFG(8, 1) TT_CFG(4, 1)
     TT_CFG(16, 2) TT_CFG(8, 2) TT_CFG(4, 2)
     TT_CFG(16, 3) TT_CFG(8, 3) TT_CFG(4, 3)
+    if constexpr (NT == 32) { TT_CFG(16, 4) }
 #undef TT_CFG
     return e;
 }
@@ -1655,6 +1786,9 @@ int launch_splitk(tt_hip_ctx *ctx, const LaunchPlan &plan, int head_dim, int n_s
     if (plan.n_tiles > 65535 || n_seq > 65535) return TT_HIP_ERR_SHAPE;
 #define TT_CASE(DD, NN)                                                                              \
     if (head_dim == DD && plan.nt == NN) {                                                           \
+        if constexpr (NN == 32) {                                                                    \
+            if (args.plan_blocks && args.plan_groups) return launch_one<DD, NN, 4, 16, 4>(ctx, plan, n_seq, args); \
+        }                                                                                            \
         if (args.plan_blocks) {                                                                      \
             if (kv_bits == 16) return launch_one<DD, NN, 4, 16, 3>(ctx, plan, n_seq, args);          \
             if (kv_bits == 8) return launch_one<DD, NN, 4, 8, 3>(ctx, plan, n_seq, args);            \

@@ -118,16 +118,21 @@ __global__ __launch_bounds__(256) void keep_rows_from_indices_kernel(uint8_t *ro
 // token tile; its work is the tile's list entries plus one pass over a bitmap of the context's blocks in LDS (a bit
 // per block: 4 KiB per million keys) -- nothing of the order rows x context is written or read.  Entries may come in
 // any order and repeat: a bit is set once.
-// LDS: bitmap[W], prefix[W], partial[kPlanThreads + 1], chunk[chunk_entries * tt] words, W = ceil(ceil(kv_valid / 32) / 32).
+// GROUPS: the same with groups of four keys in the place of blocks: the ascending list of group ids, where the ranges start
+// in it, and per eight list positions and token one word, four bits a position.
+// LDS: bitmap[W], prefix[W], partial[kPlanThreads + 1], chunk[chunk_entries * tt] words, W = ceil(ceil(kv_valid / 32) / 32)
+// (GROUPS: ceil(ceil(kv_valid / 4) / 32), and an entry is eight positions).
 constexpr int kPlanThreads = 1024;  // sixteen wavefronts: the walks are chains of dependent scalar work that only other wavefronts hide
+constexpr int kPlanGroupKeys = 400000;  // keys whose groups' bitmap and prefix sums take 25 of the 64 KiB
+template <bool GROUPS>
 __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t *indices, unsigned index_stride, const uint32_t *counts,
                                                                  int start, int q_len, int kv_valid, int tt, int split_blocks,
                                                                  int n_splits, int cap, int chunk_entries, int *ranges, int *blocks,
                                                                  unsigned *bits) {
-    constexpr int T = kPlanThreads;
+    constexpr int T = kPlanThreads, kShift = GROUPS ? 2 : 5;  // keys of a unit: 1 << kShift
     extern __shared__ unsigned plan_lds[];
     const int tile = blockIdx.x, tid = threadIdx.x;
-    const int ctx_blocks = (kv_valid + 31) >> 5, W = (ctx_blocks + 31) >> 5;
+    const int ctx_blocks = (kv_valid + (1 << kShift) - 1) >> kShift, W = (ctx_blocks + 31) >> 5;
     unsigned *bitmap = plan_lds, *prefix = plan_lds + W, *partial = plan_lds + 2 * W;
     const int rows = min(tt, q_len - tile * tt);
     // The tile's lists as one run of rows * index_stride places, every thread a run of `per` neighbouring ones (so
@@ -170,7 +175,7 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
             for (unsigned j = 0; j < kBatch; ++j) place(base + j, keys[j]);
         }
     };
-    for_listed_keys([&](unsigned key, unsigned) { atomicOr(&bitmap[key >> 10], 1u << ((key >> 5) & 31u)); });
+    for_listed_keys([&](unsigned key, unsigned) { atomicOr(&bitmap[key >> (kShift + 5)], 1u << ((key >> kShift) & 31u)); });
     __syncthreads();  // (the scan takes the counts' words over: they are put back from my_count for the second walk)
     // exclusive prefix sums of the words' bit counts: a run of words per thread, a scan of the threads' runs inside
     // each wavefront by shuffles, the wavefronts' totals through LDS
@@ -195,17 +200,17 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
     }
     __syncthreads();
     const int n_touched = (int)partial[T];  // at most min(ctx_blocks, listed entries) <= cap
-    int *my_blocks = blocks + (size_t)tile * cap * 2;
+    int *my_blocks = blocks + (size_t)tile * cap * (GROUPS ? 1 : 2);
     for (int w = tid; w < W; w += T) {
         unsigned word = bitmap[w];
         int at = (int)prefix[w];
         while (word) {
-            my_blocks[2 * at++] = w * 32 + (__ffs((int)word) - 1);
+            my_blocks[(GROUPS ? 1 : 2) * at++] = w * 32 + (__ffs((int)word) - 1);
             word &= word - 1u;
         }
     }
     for (int s = tid; s <= n_splits; s += T) {
-        const long long first = (long long)s * split_blocks;
+        const long long first = (long long)s * split_blocks * (GROUPS ? 8 : 1);
         int at = n_touched;
         if (first < ctx_blocks) at = (int)(prefix[first >> 5] + __popc(bitmap[first >> 5] & ((1u << (first & 31)) - 1u)));
         ranges[(size_t)tile * (n_splits + 1) + s] = at;
@@ -213,21 +218,25 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
     // The bits, a run of `chunk_entries` list entries at a time: gathered in LDS (atomics there cost a few cycles; in
     // global memory every listed key would be a request of its own to L2, ~8 cycles each and 32 us for a tile's 8,000
     // keys), then written out side by side.
-    unsigned *my_bits = bits + (size_t)tile * cap * tt;
+    unsigned *my_bits = bits + (size_t)tile * (GROUPS ? cap >> 3 : cap) * tt;
+    const int n_entries = GROUPS ? (n_touched + 7) >> 3 : n_touched;
     unsigned *chunk = plan_lds + 2 * W + T + 1;  // chunk_entries * tt words
     if (tid < rows) row_counts[tid] = my_count;
-    for (int first = 0; first < n_touched; first += chunk_entries) {
-        const int here = min(chunk_entries, n_touched - first);
+    for (int first = 0; first < n_entries; first += chunk_entries) {
+        const int here = min(chunk_entries, n_entries - first);
         __syncthreads();  // (the counts are back in their words; the previous run has been written out)
         for (int i = tid; i < here * tt; i += T) chunk[i] = 0u;
         __syncthreads();
         for_listed_keys([&](unsigned key, unsigned r) {
-            const unsigned w = key >> 10, bit = (key >> 5) & 31u;
-            const int rank = (int)(prefix[w] + __popc(bitmap[w] & ((1u << bit) - 1u))) - first;
-            if (rank >= 0 && rank < here) atomicOr(&chunk[rank * tt + (int)r], 1u << (key & 31u));
+            const unsigned w = key >> (kShift + 5), bit = (key >> kShift) & 31u;
+            const int rank = (int)(prefix[w] + __popc(bitmap[w] & ((1u << bit) - 1u)));
+            const int entry = (GROUPS ? rank >> 3 : rank) - first;
+            const unsigned at = GROUPS ? 4u * ((unsigned)rank & 7u) + (key & 3u) : key & 31u;
+            if (entry >= 0 && entry < here) atomicOr(&chunk[entry * tt + (int)r], 1u << at);
         });
         __syncthreads();
         for (int i = tid; i < here * tt; i += T) my_bits[(size_t)first * tt + i] = chunk[i];
+        if constexpr (GROUPS) continue;
         for (int i = tid; i < here; i += T) {
             unsigned any = 0u;
             for (int r = 0; r < tt; ++r) any |= chunk[i * tt + r];
@@ -409,28 +418,44 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         if (lists) {
             // The lists' plan, in the context's selection store: [tile][n_splits + 1] range starts, [tile][cap] blocks with
             // the keys any token keeps (pairs of words, on an even word), [tile][cap][tt] bits; a tile's list cannot be longer than the context's blocks or its tokens' entries.
-            const int ctx_blocks = (totals[base] + 31) / 32;
+            // Groups of four keys instead of blocks of 32 (fp16 pages, tiles of 32 rows): a turn of the walk then takes eight
+            // listed groups instead of one touched block, of which a selection in blocks of four leaves 1.3 to 2 groups
+            // wanted at 32k keys and more (one row's list of 2,051 cells each): 128 rows of 16/2 heads of 256 behind 16k keys 74.0 ->
+            // 65.0 us, 32k 101.3 -> 74.2, 131k 163.0 -> 120.2, all rows sharing one selection 65.8 -> 47.8.
+            // Where the tile's lists could hold half of the keys most of a block is wanted, and a block's loads are the better ones
+            // (8k keys, 512 rows: 121.7 against 133.4 us).  Nor where many tiles walk wide heads: they share fetched lines in L2 only
+            // while they stay side by side, which the walk over blocks does better (512 rows behind 131k keys 536 against 708 us;
+            // with heads of 64 470 -> 208).  The group bitmap has to leave the plan kernel's LDS room for a run of bits.
             const long long entries = (long long)plan.tt * (long long)lists->stride;
-            const int cap = (int)(entries < ctx_blocks ? entries : ctx_blocks) > 0 ? (int)(entries < ctx_blocks ? entries : ctx_blocks) : 1;
-            const size_t n_ranges = ((size_t)plan.tok_tiles * (plan.n_splits_max + 1) + 1) & ~(size_t)1, n_blocks = (size_t)plan.tok_tiles * cap;
-            st = ensure_keep_rows(ctx, (n_ranges + 2 * n_blocks + n_blocks * plan.tt) * sizeof(int));
+            const bool groups = kv->bits == 16 && plan.nt == 32 && 2 * entries <= totals[base] &&
+                                (long long)plan.n_tiles * D <= 128ll * ctx->n_cus && totals[base] <= kPlanGroupKeys;
+            const int unit = groups ? 4 : 32;
+            const int ctx_units = (totals[base] + unit - 1) / unit;
+            int cap = (int)(entries < ctx_units ? entries : ctx_units);
+            if (cap < 1) cap = 1;
+            if (groups) cap = (cap + 7) & ~7;
+            const size_t n_ranges = ((size_t)plan.tok_tiles * (plan.n_splits_max + 1) + 1) & ~(size_t)1;
+            const size_t n_blocks = (size_t)plan.tok_tiles * cap * (groups ? 1 : 2), n_bits = (size_t)plan.tok_tiles * (groups ? cap >> 3 : cap) * plan.tt;
+            st = ensure_keep_rows(ctx, (n_ranges + n_blocks + n_bits) * sizeof(int));
             if (st != TT_HIP_OK) return st;
             int *ranges = reinterpret_cast<int *>(ctx->keep_rows);
             int *blocks = ranges + n_ranges;
-            unsigned *bits = reinterpret_cast<unsigned *>(blocks + 2 * n_blocks);
-            // LDS of the plan kernel: two words per 1,024 keys of context and the run of bits it gathers at a time, 32 KiB
+            unsigned *bits = reinterpret_cast<unsigned *>(blocks + n_blocks);
+            // LDS of the plan kernel: two words per 32 units of context and the run of bits it gathers at a time, 32 KiB
             // of them or what the context's bitmap leaves of 64 KiB.
-            const int words = (ctx_blocks + 31) / 32;
+            const int words = (ctx_units + 31) / 32;
             int chunk_words = (65536 / 4) - (2 * words + kPlanThreads + 1);
             if (chunk_words > 8192) chunk_words = 8192;
             const int chunk_entries = chunk_words / plan.tt;
             if (chunk_entries < 1) return TT_HIP_ERR_CAPACITY;
-            hipLaunchKernelGGL(keep_plan_kernel, dim3((unsigned)plan.tok_tiles), dim3(kPlanThreads),
+            const auto kernel = groups ? keep_plan_kernel<true> : keep_plan_kernel<false>;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)plan.tok_tiles), dim3(kPlanThreads),
                                (size_t)(2 * words + kPlanThreads + 1 + chunk_entries * plan.tt) * sizeof(unsigned), ctx->stream, lists->indices,
                                (unsigned)lists->stride, lists->counts, starts[base], rows, totals[base], plan.tt, plan.split_len / 32,
                                plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits);
             e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(ctx, e, "keep_plan_kernel launch");
+            a.plan_groups = groups;
             a.plan_ranges = ranges;
             a.plan_blocks = blocks;
             a.plan_bits = bits;
@@ -972,7 +997,9 @@ int tt_hip_attn_prefill_keep_indices(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, 
     const int tt = 32 / gh;  // tokens per tile of the 32-row tiles (the planner's own rule)
     const long long ctx_blocks = ((long long)kv_valid + 31) / 32, entries = (long long)tt * (long long)keep_index_stride;
     const long long cap = entries < ctx_blocks ? entries : ctx_blocks;
-    const long long per_tile = (cap * (2 + tt) + 260) * 4;
+    const long long group_cap = (entries < 8 * ctx_blocks ? entries : 8 * ctx_blocks) + 8;  // (a plan of groups, run_attention)
+    const long long block_words = cap * (2 + tt), group_words = group_cap + group_cap / 8 * tt;
+    const long long per_tile = ((block_words > group_words ? block_words : group_words) + 260) * 4;
     long long tiles_per_call = (128ll << 20) / per_tile;
     if (tiles_per_call < 1) tiles_per_call = 1;
     const long long rows_per_call = tiles_per_call * tt;

@@ -81,6 +81,8 @@ struct alignas(64) SplitKArgs {
     const int *plan_ranges;       // [token tile][n_splits_max + 1]: where each split's entries start in the tile's list
     const int *plan_blocks;       // [token tile][plan_cap][2]: the key blocks the tile's tokens keep a key of, ascending, and those keys (bits)
     const unsigned *plan_bits;    // [token tile][plan_cap][tt]: per entry and token, bit i = key 32 block + i is kept
+    int plan_groups;              // the plan lists groups of four keys: plan_blocks [token tile][plan_cap] group ids, plan_bits
+                                  // [token tile][plan_cap / 8][tt], four bits a list position
     int plan_cap;                 // entries a tile's list has room for
 };
 
