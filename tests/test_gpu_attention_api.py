@@ -803,3 +803,46 @@ def test_kernel_variant_switches_are_explicit_calls_and_change_no_result():
     ctx.graph_end().close()
     c.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("bits,D,H,KH,lengths,rows,window", [
+    (16, 256, 16, 2, [1, 20000, 37, 512, 385, 9001], 1, 0),                       # one round, short and long ones mixed
+    (16, 256, 16, 2, [700 + 311 * i for i in range(64)], 1, 0),                   # a table that is full
+    (8, 128, 8, 2, [5000 - 61 * i for i in range(66)], 1, 0),                     # two launches
+    (16, 64, 16, 4, [30, 12000, 4, 3000], 1, 0), (4, 128, 32, 8, [400, 8192, 6000], 1, 0),
+    (8, 256, 16, 2, [9000, 33, 4097], 4, 0),                                      # verify rows, one tile a KV head
+    (16, 256, 16, 2, [3000, 11, 7001], 8, 0),                                     # ... and two
+    (16, 128, 8, 4, [9000, 50, 2500, 1301], 1, 1000), (16, 64, 64, 32, [100 + 37 * i for i in range(40)], 1, 0),  # mostly last splits
+])
+def test_sequences_of_unlike_lengths_equal_their_own_calls(gpu_ctx, bits, D, H, KH, lengths, rows, window):
+    # A batch of unlike lengths has its split length counted out and its splits one behind the other in the grid; a sequence
+    # on its own takes neither.  The two differ in where the keys are cut only: the path's bar against the oracle holds both
+    # within 2e-3 of it, and one sequence's rows are checked against the oracle's other route by the tests above.
+    import torch
+    from tests.test_gpu_kv_quant import _append, _cache
+    from tinytitan_amd.engine import Attention
+    r = np.random.default_rng(len(lengths) + D + bits)
+    n, total = len(lengths), max(lengths) + rows
+    kv = _cache(gpu_ctx, bits, KH, D, total, slots=n)
+    for s, length in enumerate(lengths):
+        _append(gpu_ctx, kv, 0, s, 0, *(r.standard_normal((length + rows, KH, D)).astype(np.float16) for _ in range(2)))
+    q, gate = (_dev(r.standard_normal((n * rows, H * D)).astype(np.float16)) for _ in range(2))
+    att, scale = Attention(gpu_ctx), D ** -0.5
+
+    def attend(which):
+        rows_of = torch.cat([torch.arange(i * rows, (i + 1) * rows) for i in which]).cuda()
+        qs, gs = q[rows_of].contiguous(), gate[rows_of].contiguous()
+        out = torch.full(qs.shape, float("nan"), dtype=torch.float16, device="cuda")
+        torch.cuda.synchronize()
+        if rows == 1 and window == 0:
+            att.encode_full(kv, 0, qs, out, H, [lengths[i] + 1 for i in which], scale, slot=list(which), gate=gs)
+        else:
+            att.encode_verify_rows(kv, 0, qs, out, H, [lengths[i] for i in which], rows, scale, list(which), gate=gs, window=window)
+        gpu_ctx.synchronize()
+        return out.float().cpu().numpy()
+
+    together = attend(range(n))
+    alone = np.concatenate([attend([i]) for i in range(n)])
+    kv.close()
+    assert np.isfinite(together).all()
+    assert np.abs(together - alone).max() <= 2e-3

@@ -976,6 +976,11 @@ __device__ __forceinline__ void load_hot(SplitKHot &hot, SplitKSeq &sq, int seq)
     hot = __builtin_bit_cast(SplitKHot, w);
     sq = __builtin_bit_cast(SplitKSeq, e);
 }
+typedef __attribute__((address_space(4))) const i4 *seq_entries;  // SplitKSeq: [3] is first_split
+__device__ __forceinline__ seq_entries seq_table() {
+    return (seq_entries)((__attribute__((address_space(4))) const char *)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(SplitKArgs, seq));
+}
+static_assert(kMaxSeqPerLaunch == 64 && offsetof(SplitKSeq, first_split) == 12, "a lane per sequence");
 static_assert(offsetof(SplitKArgs, hot) == 0 && offsetof(SplitKArgs, seq) == 0x80, "load_hot's offsets");
 
 // STREAM: the launch reads every K/V byte once (see kStreamed).
@@ -1003,11 +1008,19 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: block pointers stay in SGPRs
     const Lane<D, NT> ln(lane);
     const int li = ln.li, g = ln.g;
-    const int seq = blockIdx.z;
+    int seq = blockIdx.z;
     SplitKHot a;
     SplitKSeq sq;
     load_hot(a, sq, seq);
     int split = blockIdx.x, tile = blockIdx.y;
+    if (a.flags & kHotPackedSplits) {
+        // Sequences of unlike lengths, their splits one behind the other in x: the entries of all of them in one load (those
+        // past the last start beyond every split), and this split's sequence is the last that starts no later.
+        const int first = seq_table()[lane][3];
+        seq = (int)__popcll(__ballot(first <= split)) - 1;
+        sq = __builtin_bit_cast(SplitKSeq, seq_table()[seq]);
+        split -= sq.first_split;
+    }
     if (a.flags & kHotXcdGrid) {  // many token tiles: the (split, tile) pairs are dealt out XCD by XCD, tile fastest
         const unsigned pairs = (unsigned)a.n_tiles * (unsigned)a.n_splits_max, per_xcd = (pairs + 7u) >> 3;
         const unsigned pair = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
@@ -1657,7 +1670,8 @@ int plan_launch(const tt_hip_ctx *ctx, int kind, int n_seq, int n_q_heads, int n
     p.waves = 4;
     const int min_split = 32 * p.waves;  // one key block per wave
     // Workgroup slots of the chip: the 16-row kernel fits two workgroups per CU, the 32-row one.
-    const long long slots = (long long)ctx->n_cus * (p.nt == 16 ? 2 : 1);
+    p.slots_per_cu = p.nt == 16 ? 2 : 1;
+    const long long slots = (long long)ctx->n_cus * p.slots_per_cu;
     int split_len;
     if (ctx->split_override > 0) {
         split_len = ((ctx->split_override + 31) / 32) * 32;
@@ -1669,6 +1683,9 @@ int plan_launch(const tt_hip_ctx *ctx, int kind, int n_seq, int n_q_heads, int n
         // for a CU and double the kernel's time.
         const long long pairs = (long long)n_seq * p.n_tiles;
         long long per_pair = ctx->n_cus / pairs;
+        // (two rounds, side by side on a CU, where a workgroup's loads are few bytes and its walk is long: 131k keys over 8
+        // bits with 16/4 heads of 64 23.4 -> 18.0 us, over 4 bits with 32/8 heads of 128 43.0 -> 35.6; with 16/2 of 256 27.4 -> 30.1)
+        if (head_dim * kv_bits <= 512 && pairs <= ctx->n_cus && max_keys >= 768 * per_pair) per_pair = 2 * ctx->n_cus / pairs;
         if (per_pair < 1) per_pair = 1;
         split_len = (int)((max_keys + per_pair - 1) / per_pair);
         split_len = ((split_len + min_split - 1) / min_split) * min_split;
@@ -1720,6 +1737,7 @@ template <int D, int NT, int WAVES, int BITS, int KEEP = 0, int STREAM = 0>
 static int launch_one(tt_hip_ctx *ctx, const LaunchPlan &plan, int n_seq, const SplitKArgs &args) {
     auto kernel = attn_splitk_kernel<D, NT, WAVES, BITS, KEEP, STREAM>;  // its LDS limit was raised when the context was created
     dim3 grid((unsigned)plan.n_splits_max, (unsigned)plan.n_tiles, (unsigned)n_seq);
+    if (plan.packed_splits > 0) grid = dim3((unsigned)plan.packed_splits, (unsigned)plan.n_tiles);
     if (plan.xcd_grid) grid = dim3((unsigned)(((long long)plan.n_splits_max * plan.n_tiles + 7) / 8 * 8), 1u, (unsigned)n_seq);
     launch_profiled(ctx, kernel, grid, dim3(WAVES * 64), (unsigned)(plan.lds_bytes + keep_list_bytes(KEEP, WAVES)), args);
     hipError_t e = hipGetLastError();

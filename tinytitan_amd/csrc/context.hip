@@ -1,4 +1,5 @@
 // Context, error reporting, timing and the three attention entry points of the C ABI.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -323,7 +324,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             if (walked(i) > max_keys) max_keys = walked(i);
             if (walked(i) < min_keys) min_keys = walked(i);
         }
-        LaunchPlan plan;
+        LaunchPlan plan{};
         const bool small_tiles_ok = kind == 0 && !keep && !lists && chunk_splits <= 1 && !pages;
         int st = plan_launch(ctx, kind, n, n_q_heads, kv->n_kv_heads, D, rows, total_keys, min_keys, max_keys, &plan, kv->bits,
                              small_tiles_ok);
@@ -331,6 +332,43 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         if (chunk_splits > 1) {  // the chunk kernel's geometry: 32-row one-head tiles, its own key ranges
             plan.split_len = chunk_split_blocks * 32;
             plan.n_splits_max = chunk_splits;
+        }
+        // Unlike lengths: the split length that makes the launch whole rounds of at most n_cus workgroups, counted with every
+        // sequence's short last split -- the planner's estimate does not know those, and a workgroup over a round waits for a
+        // whole one.  k workgroups a CU take len keys each at a k-th of the memory's rate, or at their own where k are too
+        // few to keep it busy (one workgroup of heads of 256, two of 128, four of 64), and 32,768 / D keys' worth of start,
+        // merge and partial results each.  32 decode rows of 16/2 heads of 256 behind 511 .. 16,383 keys 67.5 -> 49.6 us, 4
+        // verify rows x 6 sequences behind 5,000 .. 30,000 keys 58.6 -> 39.1, 20 decode rows over 8 bits 53.8 -> 47.8, 24 of
+        // 32/8 heads of 128 40.1 -> 37.8.  Never shorter splits than the planner's, whose partial results have a bound.
+        const bool ragged = kind == 0 && chunk_splits <= 1 && min_keys != max_keys && plan.n_splits_max > 1;
+        if (ragged && ctx->split_override <= 0) {
+            const long long sat = 256 / D, tails = (long long)n * plan.n_tiles;
+            long long best = 0;
+            int best_len = 0;
+            for (long long k = 1; k <= plan.slots_per_cu * 2; ++k) {
+                const long long most = k * ctx->n_cus;
+                // (mostly last splits: the planner's rule; 40 sequences behind 30 .. 3,000 keys, 32/8 heads of 128: 26.6 us against 29.3)
+                if (3 * tails > most) continue;
+                // (a last split is short by half on average)
+                long long len = ((total_keys * plan.n_tiles) / (most - tails / 2) + 127) / 128 * 128;
+                if (len < 128) len = 128;
+                auto workgroups = [&] {
+                    int w = 0;
+                    for (int i = 0; i < n; ++i) w += std::max((walked(i) + (int)len - 1) / (int)len, 1);
+                    return (long long)w * plan.n_tiles;
+                };
+                while (workgroups() > most) len += std::max(128ll, len / 16 / 128 * 128);
+                const long long cost = len * std::max(k, sat) + k * (32768 / D);
+                if (best_len == 0 || cost < best) {
+                    best = cost;
+                    best_len = (int)len;
+                }
+            }
+            if (best_len > plan.split_len) {
+                plan.split_len = best_len;
+                plan.n_splits_max = (max_keys + best_len - 1) / best_len;
+                plan.workgroups = (long long)plan.n_splits_max * plan.n_tiles * n;
+            }
         }
         // One selection per sequence: a wavefront keeps the blocks it still has to work on as one 64-bit word, at
         // most 64 per split.  One per query row: as a list, of at most kKeepWindows such words.
@@ -358,6 +396,10 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             const int mine = chunk_splits > 1 ? chunk_splits : (walked(i) + plan.split_len - 1) / plan.split_len;
             total_splits += (size_t)(mine < 1 ? 1 : mine);
         }
+        // Unlike lengths: a grid of (splits of the longest, tiles, sequences) would be full of workgroups that find nothing to
+        // do, and the others would not fall evenly on the XCDs (a split count of a multiple of eight sends split i of
+        // every sequence to XCD i mod 8).
+        plan.packed_splits = ragged && !plan.xcd_grid ? (int)total_splits : 0;
         if (plan.n_splits_max > 1) {
             const size_t part_rows = total_splits * plan.n_tiles * plan.nt;
             if (static_partials) {
@@ -398,7 +440,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         const bool aligned = aligned16(h.q) && aligned16(a.out) && (!a.gate || aligned16(a.gate)) && q_seq_stride % 8 == 0 &&
                              q_tok_stride % 8 == 0 && g_seq_stride % 8 == 0 && g_tok_stride % 8 == 0 && o_seq_stride % 8 == 0 &&
                              o_tok_stride % 8 == 0;
-        h.flags = (aligned ? kHotAligned : 0) | (plan.xcd_grid ? kHotXcdGrid : 0);
+        h.flags = (aligned ? kHotAligned : 0) | (plan.xcd_grid ? kHotXcdGrid : 0) | (plan.packed_splits > 0 ? kHotPackedSplits : 0);
         h.scale_log2e = scale * 1.4426950408889634f;
         h.window = window;
         h.ring_blocks = kv->ring_blocks();
@@ -415,6 +457,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             a.seq[i].total = totals[base + i];
             a.seq[i].first_split = first_split[i];
         }
+        for (int i = n; i < kMaxSeqPerLaunch; ++i) a.seq[i].first_split = 0x7fffffff;  // (behind every split: see kHotPackedSplits)
         if (lists) {
             // The lists' plan, in the context's selection store: [tile][n_splits + 1] range starts, [tile][cap] blocks with
             // the keys any token keeps (pairs of words, on an even word), [tile][cap][tt] bits; a tile's list cannot be longer than the context's blocks or its tokens' entries.
@@ -768,7 +811,7 @@ void tt_hip_graph_destroy(tt_hip_graph *graph) {
 int tt_hip_split_geometry(tt_hip_ctx *ctx, int n_seq, int n_q_heads, int n_kv_heads, int head_dim, int rows,
                           int seq_len, int *out_split_tokens, int *out_splits, int *out_workgroups) {
     if (!ctx || seq_len < 0) return TT_HIP_ERR_INVALID_ARGUMENT;
-    LaunchPlan plan;
+    LaunchPlan plan{};
     int st = plan_launch(ctx, 0, n_seq, n_q_heads, n_kv_heads, head_dim, rows, (long long)seq_len * n_seq, seq_len, seq_len, &plan, 16, true);
     if (st != TT_HIP_OK) return st;
     if (out_split_tokens) *out_split_tokens = plan.split_len;

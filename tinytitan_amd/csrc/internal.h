@@ -32,6 +32,8 @@ constexpr int kHotAligned = 1;  // q/gate/out rows are 16-byte aligned
 // workgroups that one XCD runs side by side are given consecutive (split, tile) pairs, tile fastest -- token
 // tiles of one KV head over one key range, whose K/V blocks they then share in that XCD's L2.
 constexpr int kHotXcdGrid = 2;
+// The grid is (splits of all sequences, tiles): split x belongs to the sequence whose first_split it falls behind.
+constexpr int kHotPackedSplits = 4;
 struct SplitKHot {                         // dword
     const _Float16 *k_layer;               //  0
     const _Float16 *v_layer;               //  2
@@ -51,7 +53,7 @@ struct SplitKHot {                         // dword
     float scale_log2e;                     // 22
     int n_splits_max;                      // 23
     int n_tiles;                           // 24  n_kv_heads * hsubs * tok_tiles
-    int flags;                             // 25  kHotAligned | kHotXcdGrid
+    int flags;                             // 25  kHotAligned | kHotXcdGrid | kHotPackedSplits
     int keep_words;   // 26  per-sequence masks start on 4-byte boundaries: a wavefront may read its blocks' bytes as words
     int gh_inv;       // 27  ceil(65536 / gh): (i * gh_inv) >> 16 == i / gh for 0 <= i < 64, gh <= 32
     float *part_o;    // 28  [first_split(seq) + split][tile][NT][D]
@@ -95,6 +97,8 @@ struct LaunchPlan {
     size_t lds_bytes;
     bool stream;  // every K/V byte is read once by the launch, and there are many of them: non-temporal loads
     bool xcd_grid;  // launch with kHotXcdGrid
+    int slots_per_cu;  // workgroups that the planner's rule for unlike lengths counts on
+    int packed_splits;  // > 0: launch with kHotPackedSplits over this many splits
 };
 
 }  // namespace tt
