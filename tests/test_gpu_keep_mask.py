@@ -857,3 +857,25 @@ def test_lists_walked_by_groups_of_keys_equal_the_mask_form(gpu_ctx, D, H, KH, T
     assert not got[tt:2 * tt].any()
     assert np.abs(got - by_mask).max() <= 2e-3
     _check(got, _oracle_rows_kept(q, k, v, start, keep, H, KH, D, scale, gate=gate), f"groups D={D} {H}/{KH}")
+
+
+@pytest.mark.parametrize("T", [8193, 20000, 40001, 70002])
+@pytest.mark.parametrize("bits,D,H,KH", [(16, 256, 16, 2), (8, 128, 16, 4), (4, 64, 24, 2)])
+def test_decode_reads_from_the_first_touched_block_on(gpu_ctx, bits, D, H, KH, T):
+    # One mask, any length: most wavefronts have no touched block, or only a late one, and bytes other than 1 keep a key too.
+    r = np.random.default_rng(T + D)
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    q = r.standard_normal((1, 1, H, D)).astype(np.float16)
+    keep = np.zeros(T, np.uint8)
+    at = r.choice(T, 60, replace=False)
+    keep[at] = r.choice(np.array([1, 2, 127, 128, 255], np.uint8), 60)
+    for tail in (0, 7):
+        keep[T - 3:] = [tail & 1, tail & 2, tail & 4]
+        v2 = v.copy()
+        v2[keep == 0] += np.float16(40.0)
+        kv = _cache(gpu_ctx, bits, KH, D, T)
+        _append(gpu_ctx, kv, 0, 0, 0, k, v2)
+        got = _decode_keep(gpu_ctx, kv, q, [T], keep, H, D ** -0.5)[0, 0]
+        kv.close()
+        ks, vs = (k, v2) if bits == 16 else (_dequantised(k, bits), _dequantised(v2, bits))
+        _check(got, _oracle_kept(q[0, 0], ks, vs, keep, H, KH, D, D ** -0.5), f"T={T} D={D} bits {bits} tail {tail}")

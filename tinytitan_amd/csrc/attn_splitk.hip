@@ -1078,24 +1078,54 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     // A block without a kept key is not read: its loads are void (no memory traffic), its turn works on zeros that
     // the selection masks anyway, so the HBM bytes of a selection are the blocks it touches, not the context.
     // (Skipping the turn's arithmetic too, with a branch around it, made the kernel slower: the compiler then
-    // waits for every load in flight at the join.)  The first block of a wavefront is read before its bytes
-    // are known -- waiting for them would put a round trip in front of it.
-    // Where the mask starts on a word boundary the wavefront also learns up front which of its blocks hold a kept
+    // waits for every load in flight at the join.)  Where the mask is tested block by block, the first block of a
+    // wavefront is read before its bytes are known -- waiting for them would put a round trip in front of it.
+    // Where the mask starts on a word boundary the wavefront learns up front which of its blocks hold a kept
     // key at all -- lane j reads the 32 bytes of its j-th block, one ballot makes a 64-bit word of them (the host
-    // keeps a split to 64 blocks per wavefront) -- and then walks only those: their arithmetic goes as well.
+    // keeps a split to 64 blocks per wavefront) -- and then walks only those, from the first: their arithmetic goes as
+    // well, and with a selection of one group in eight blocks most wavefronts read none or one (read before its bytes were
+    // known, every wavefront's first block was 33 MB a launch: 131k keys 20.7 -> 15.7 us with the step behind it).
     __amdgpu_buffer_rsrc_t rkeep;
     unsigned keep_cur = 1, keep_next = 1, keep_after = 1;
     const int b_first = b;
     unsigned long long todo = 0;  // bit j: block b_first + j * WAVES is still to be worked on
-    unsigned block_words = 0;
+    unsigned first_keys = ~0u;  // the first block's keys that some row keeps
     if constexpr (KEEP == 1) {
         rkeep = make_rsrc(args.keep + seq * args.keep_seq_stride, (unsigned)ti.total);
-        keep_cur = __builtin_amdgcn_raw_buffer_load_b8(rkeep, (unsigned)b * 32u + (unsigned)(lane & 31), 0, 0);
+        const int mine = b_first < b_end ? (b_end - b_first + WAVES - 1) / WAVES : 0;  // this wavefront's blocks, at most 64
+        todo = mine >= 64 ? ~0ull : ((1ull << mine) - 1ull);
         if (a.keep_words) {
+            unsigned words[8], block_keys = 0;  // bit i: key i of the lane's block is kept
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                block_words |= __builtin_amdgcn_raw_buffer_load_b32(rkeep, (unsigned)(b_first + lane * WAVES) * 32u + 4u * i, 0, 0);
+            for (int i = 0; i < 8; ++i) words[i] = __builtin_amdgcn_raw_buffer_load_b32(rkeep, (unsigned)(b_first + lane * WAVES) * 32u + 4u * i, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const unsigned set = (((words[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | words[i]) & 0x80808080u;  // a byte's top bit: the byte is not zero
+                block_keys |= ((set >> 7) * 0x10204080u >> 28) << (4 * i);
+            }
+            unsigned long long touched = __ballot(block_keys != 0);
+            // A mask is exactly `total` bytes: when that is not a multiple of 4 its last word straddles the end of
+            // the buffer's range and may read as zero whatever its bytes hold.  The block of the last key is
+            // therefore always walked and fetched whole; its keys are still tested byte by byte.
+            int tail_j = -1;
+            if (ti.total & 3) {
+                const int last_block = (ti.total - 1) >> 5, j = (last_block - b_first) / WAVES;
+                if (last_block >= b_first && (last_block - b_first) % WAVES == 0 && j < 64) {
+                    touched |= 1ull << j;
+                    tail_j = j;
+                }
+            }
+            todo &= touched;
+            const int j0 = todo ? __ffsll((long long)todo) - 1 : 0;
+            b = todo ? b_first + j0 * WAVES : b_end;
+            first_keys = j0 == tail_j ? ~0u : (unsigned)__builtin_amdgcn_readlane((int)block_keys, j0);
+            todo &= todo - 1;
+            keep_cur = __builtin_amdgcn_raw_buffer_load_b8(rkeep, (unsigned)b * 32u + (unsigned)(lane & 31), 0, 0);
+            const int nb0 = todo ? b_first + (__ffsll((long long)todo) - 1) * WAVES : b_end;
+            keep_next = __builtin_amdgcn_raw_buffer_load_b8(rkeep, (unsigned)nb0 * 32u + (unsigned)(lane & 31), 0, 0);
         } else {
+            todo &= ~1ull;  // the first block is in hand
+            keep_cur = __builtin_amdgcn_raw_buffer_load_b8(rkeep, (unsigned)b * 32u + (unsigned)(lane & 31), 0, 0);
             // block by block: the next block is the wavefront's second, and its bytes are asked for ahead of the
             // first block's data
             keep_next = __builtin_amdgcn_raw_buffer_load_b8(rkeep, (unsigned)(b + WAVES) * 32u + (unsigned)(lane & 31), 0, 0);
@@ -1154,7 +1184,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     int e_at = 0, e_hi = 0, walked = 0;
     typedef int i2 __attribute__((ext_vector_type(2)));
     i2 after_entry = {0, 0};  // block, keys of it that any token keeps
-    unsigned first_keys = ~0u, nxt_keys = ~0u;
+    unsigned nxt_keys = ~0u;
     unsigned bits_cur = ~0u, bits_next = ~0u, bits_after = ~0u;
     const int bits_col = valid ? t_local : 0;
     auto plan_entry = [&](int k) {  // the wavefront's k-th entry (a load; every lane the same words)
@@ -1217,7 +1247,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     const bool first_real = b < b_end;
     const unsigned first_bytes = first_real ? (unsigned)(a.ring_blocks ? b % a.ring_blocks : b) * BLK_BYTES : 0u;
     Voids<D, NT> first_void(first_real ? 0u : kVoidLoad);
-    if constexpr (KEEP == 3) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
+    if constexpr (KEEP == 1 || KEEP == 3) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
     if constexpr (KEEP == 4) {
         if (run_end > 0) {
             int ids_first[5];
@@ -1231,26 +1261,6 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         load_k<AUX>(kt, rk, first_bytes, ln, first_void);
     }
     __builtin_amdgcn_sched_barrier(0);  // the first block's K loads are issued HERE, before the query is waited for
-    if constexpr (KEEP == 1) {
-        const int mine = b_first < b_end ? (b_end - b_first + WAVES - 1) / WAVES : 0;  // this wavefront's blocks, at most 64
-        todo = mine >= 64 ? ~0ull : ((1ull << mine) - 1ull);
-        if (a.keep_words) {
-            unsigned long long touched = __ballot(block_words != 0);
-            // A mask is exactly `total` bytes: when that is not a multiple of 4 its last word straddles the end of
-            // the buffer's range and may read as zero whatever its bytes hold.  The block of the last key is
-            // therefore always walked; its keys are still tested byte by byte.
-            if (ti.total & 3) {
-                const int last_block = (ti.total - 1) >> 5, j = (last_block - b_first) / WAVES;
-                if (last_block >= b_first && (last_block - b_first) % WAVES == 0 && j < 64) touched |= 1ull << j;
-            }
-            todo &= touched;
-        }
-        todo &= ~1ull;  // the first block is in hand
-        if (a.keep_words) {
-            const int nb0 = todo ? b_first + (__ffsll((long long)todo) - 1) * WAVES : b_end;
-            keep_next = __builtin_amdgcn_raw_buffer_load_b8(rkeep, (unsigned)nb0 * 32u + (unsigned)(lane & 31), 0, 0);
-        }
-    }
     if constexpr (KEEP == 2) {
         if (a.keep_words) {
             // One list for the workgroup, its entries dealt out to the wavefronts in turn: every wavefront then walks

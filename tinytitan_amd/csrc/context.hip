@@ -450,10 +450,15 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         a.keep = keep ? keep + base * keep_seq_stride : nullptr;
         a.keep_seq_stride = keep_seq_stride;
         a.keep_row_stride = keep_row_stride;
-        // Finding a wavefront's touched blocks up front costs a round of loads in front of its first block: worth it
-        // from about eight blocks a wavefront on (below that the block-by-block test with void loads is faster).
-        // (Per-query rows are always word-aligned: the entry point requires it.)
-        h.keep_words = a.keep && (uintptr_t)a.keep % 4 == 0 && keep_seq_stride % 4 == 0 && plan.split_len >= 8 * plan.waves * 32;
+        // Finding a wavefront's touched blocks up front costs a round of loads in front of its first block.  A decode step gets
+        // back that no wavefront reads a block without a kept key, its first one included: worth it from two blocks a
+        // wavefront on (2,051 of 40,001 keys, 16/2 heads of 256: 14.9 -> 13.5 us, of 70,001 17.7 -> 14.0, of 131,070 22.3 -> 14.6,
+        // of 262,000 30.8 -> 14.9; with one block, at 8,000 keys, 10.3 against 10.7 the other way).  Per-query rows, whose
+        // walk reads every row's bytes first: from about eight.  (Those are always word-aligned: the entry point
+        // requires it; a single sequence's mask has no stride to mind.)
+        const int listed_blocks = keep_row_stride > 0 ? 8 : 2;
+        h.keep_words = a.keep && (uintptr_t)a.keep % 4 == 0 && (n == 1 || keep_seq_stride % 4 == 0) &&
+                       plan.split_len >= listed_blocks * plan.waves * 32;
         for (int i = 0; i < n; ++i) {
             a.seq[i].slot = slots[base + i];
             a.seq[i].start = starts[base + i];
