@@ -879,3 +879,41 @@ def test_decode_reads_from_the_first_touched_block_on(gpu_ctx, bits, D, H, KH, T
         kv.close()
         ks, vs = (k, v2) if bits == 16 else (_dequantised(k, bits), _dequantised(v2, bits))
         _check(got, _oracle_kept(q[0, 0], ks, vs, keep, H, KH, D, D ** -0.5), f"T={T} D={D} bits {bits} tail {tail}")
+
+
+@pytest.mark.parametrize("bits,D,H,KH,start,rows", [(8, 256, 16, 2, 6111, 130), (4, 128, 32, 8, 6500, 128), (8, 256, 24, 2, 20001, 128)])
+def test_lists_over_quantised_pages_that_are_dequantised_first(gpu_ctx, bits, D, H, KH, start, rows):
+    # Enough tiles that walk the context several times over: the visible blocks become fp16 pages once per call, of the second
+    # slot here.  The oracle over the dequantised rows, and the mask form, which walks the quantised pages.
+    import torch
+    from tinytitan_amd.engine import PrefillAttention, PrefillAttentionParams
+    r = np.random.default_rng(bits + start)
+    T, scale = start + rows, D ** -0.5
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    q, gate = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    stride = 2051 if start < 10000 else 1700  # (20,001 keys: groups of keys over the fp16 pages)
+    keep = np.zeros((rows, ((T + 3) // 4) * 4), np.uint8)
+    lists, counts = np.zeros((rows, stride), np.int32), np.zeros(rows, np.int32)
+    for t in range(rows):
+        groups = r.choice((start + t) // 4, 100 + t % 50, replace=False)
+        keep[t, (4 * groups[:, None] + np.arange(4)).reshape(-1)] = 1
+        keep[t, start + t] = 1
+        ids = np.flatnonzero(keep[t])
+        lists[t, :len(ids)], counts[t] = ids, len(ids)
+    kv = _cache(gpu_ctx, bits, KH, D, T, slots=2)
+    _append(gpu_ctx, kv, 0, 1, 0, k, v)
+    qd, gd, lists_d, counts_d = _dev(q), _dev(gate), _dev(lists), _dev(counts)
+    keep_d = _dev(keep)
+    att, params = PrefillAttention(gpu_ctx), PrefillAttentionParams(start, rows, T, H, scale, H * D, H * D, H * D)
+    outs = [torch.full((rows, H * D), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    att.encode_causal(kv, 0, 1, qd, outs[0], params, gate=gd, keep_indices=lists_d, keep_index_stride=stride, keep_counts=counts_d)
+    att.encode_causal(kv, 0, 1, qd, outs[1], params, gate=gd, keep_mask=keep_d, keep_stride=keep.shape[1])
+    gpu_ctx.synchronize()
+    by_list, by_mask = (o.float().cpu().numpy() for o in outs)
+    kv.close()
+    assert np.abs(by_list - by_mask).max() <= 2e-3
+    some = [0, 1, 63, rows - 1]
+    want = np.concatenate([_oracle_rows_kept(q[t:t + 1], _dequantised(k, bits), _dequantised(v, bits), start + t, keep[t:t + 1], H, KH, D, scale,
+                                             gate=gate[t:t + 1]) for t in some])
+    _check(by_list[some], want, f"dequantised pages D={D} {H}/{KH} bits {bits}")

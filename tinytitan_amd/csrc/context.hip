@@ -325,8 +325,11 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             if (walked(i) < min_keys) min_keys = walked(i);
         }
         LaunchPlan plan{};
+        // Lists over quantised pages that the caller has had dequantised: the split-K kernel walks those pages.
+        const bool walks_pages = lists && pages;
+        const int kv_bits = walks_pages ? 16 : kv->bits;
         const bool small_tiles_ok = kind == 0 && !keep && !lists && chunk_splits <= 1 && !pages;
-        int st = plan_launch(ctx, kind, n, n_q_heads, kv->n_kv_heads, D, rows, total_keys, min_keys, max_keys, &plan, kv->bits,
+        int st = plan_launch(ctx, kind, n, n_q_heads, kv->n_kv_heads, D, rows, total_keys, min_keys, max_keys, &plan, kv_bits,
                              small_tiles_ok);
         if (st != TT_HIP_OK) return st;
         if (chunk_splits > 1) {  // the chunk kernel's geometry: 32-row one-head tiles, its own key ranges
@@ -415,14 +418,14 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         SplitKArgs a;
         std::memset(&a, 0, sizeof(a));
         SplitKHot &h = a.hot;
-        h.k_layer = kv->k[layer];
-        h.v_layer = kv->v[layer];
+        h.k_layer = walks_pages ? pages->k : kv->k[layer];
+        h.v_layer = walks_pages ? pages->v : kv->v[layer];
         h.q = reinterpret_cast<const _Float16 *>(q) + base * q_seq_stride;
         a.gate = gate ? reinterpret_cast<const _Float16 *>(gate) + base * g_seq_stride : nullptr;
         a.out = reinterpret_cast<_Float16 *>(out) + base * o_seq_stride;
         h.part_o = static_partials ? ctx->static_scratch : ctx->part_o;
         h.part_ml = static_partials ? ctx->static_scratch + kStaticPartialRows * 256 : ctx->part_ml;
-        h.page_elems = (long long)kv->page_elems();
+        h.page_elems = walks_pages ? pages->page_elems : (long long)kv->page_elems();
         h.q_seq_stride = q_seq_stride;
         h.q_tok_stride = q_tok_stride;
         a.g_seq_stride = g_seq_stride;
@@ -446,7 +449,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         h.flags = (aligned ? kHotAligned : 0) | (plan.xcd_grid ? kHotXcdGrid : 0) | (plan.packed_splits > 0 ? kHotPackedSplits : 0);
         h.scale_log2e = scale * 1.4426950408889634f;
         h.window = window;
-        h.ring_blocks = kv->ring_blocks();
+        h.ring_blocks = walks_pages ? pages->ring_blocks : kv->ring_blocks();
         a.keep = keep ? keep + base * keep_seq_stride : nullptr;
         a.keep_seq_stride = keep_seq_stride;
         a.keep_row_stride = keep_row_stride;
@@ -460,7 +463,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         h.keep_words = a.keep && (uintptr_t)a.keep % 4 == 0 && (n == 1 || keep_seq_stride % 4 == 0) &&
                        plan.split_len >= listed_blocks * plan.waves * 32;
         for (int i = 0; i < n; ++i) {
-            a.seq[i].slot = slots[base + i];
+            a.seq[i].slot = walks_pages ? 0 : slots[base + i];
             a.seq[i].start = starts[base + i];
             a.seq[i].total = totals[base + i];
             a.seq[i].first_split = first_split[i];
@@ -478,7 +481,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             // while they stay side by side, which the walk over blocks does better (512 rows behind 131k keys 536 against 708 us;
             // with heads of 64 470 -> 208).  The group bitmap has to leave the plan kernel's LDS room for a run of bits.
             const long long entries = (long long)plan.tt * (long long)lists->stride;
-            const bool groups = kv->bits == 16 && plan.nt == 32 && 2 * entries <= totals[base] &&
+            const bool groups = kv_bits == 16 && plan.nt == 32 && 2 * entries <= totals[base] &&
                                 (long long)plan.n_tiles * D <= 128ll * ctx->n_cus && totals[base] <= kPlanGroupKeys;
             const int unit = groups ? 4 : 32;
             const int ctx_units = (totals[base] + unit - 1) / unit;
@@ -518,7 +521,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
                                 ctx->part_ml, pages, window);
             if (st == TT_HIP_OK) st = launch_combine(ctx, plan, D, n, a);
         } else {
-            st = launch_splitk(ctx, plan, D, n, a, kv->bits);
+            st = launch_splitk(ctx, plan, D, n, a, kv_bits);
         }
         if (st != TT_HIP_OK) return st;
     }
@@ -1054,13 +1057,33 @@ int tt_hip_attn_prefill_keep_indices(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, 
     long long tiles_per_call = (128ll << 20) / per_tile;
     if (tiles_per_call < 1) tiles_per_call = 1;
     const long long rows_per_call = tiles_per_call * tt;
+    PageSource staged{};
+    const PageSource *pages = nullptr;
+    // Quantised pages: a tile widens every block it walks, and blocks only, not groups of keys.  Where the tiles together walk
+    // the context several times over and there are enough of them to matter, the visible blocks are dequantised once per
+    // call instead, as for a dense chunk, and the fp16 kernels walk those (8 bits, 16/2 heads of 256, rows with a selection
+    // each / all with one: 128 rows behind 32k keys 142.1 -> 92.4 us / 84.9 -> 63.0, 256 behind 100k 391.6 -> 234.3 / 147.4 ->
+    // 122.9, 512 behind 16k 260.6 -> 198.2; walked about once, 128 rows behind 250k, 268.4 against 323.7 the other way, and
+    // behind 4,000 keys 54.6 against 56.4: another launch).
+    const long long tok_tiles = (q_len + tt - 1) / tt, tiles = tok_tiles * (group / gh) * kv->n_kv_heads;
+    const long long walked = tok_tiles * (entries < kv_valid ? entries : kv_valid);
+    if (kv->bits != 16 && !kv->ring && tiles * kv->head_dim >= 64 * 256 && kv_valid >= 6144 && walked >= 5ll * kv_valid) {
+        const int n_blocks = (kv_valid + 31) / 32;
+        const size_t page = (size_t)n_blocks * 32 * kv->head_dim;
+        if (ensure_stage(ctx, page * kv->n_kv_heads) == TT_HIP_OK) {  // (else, as inside a capture: the pages as they are)
+            const int st = launch_kvq_dequant_blocks(kv, layer, slot, n_blocks, ctx->stage_k, ctx->stage_v, page);
+            if (st != TT_HIP_OK) return st;
+            staged = PageSource{ctx->stage_k, ctx->stage_v, (long long)page, 0};
+            pages = &staged;
+        }
+    }
     for (long long r0 = 0; r0 < q_len; r0 += rows_per_call) {
         const int rows = (int)(q_len - r0 < rows_per_call ? q_len - r0 : rows_per_call);
         const int start = start_pos + (int)r0;
         const KeepLists lists{keep_indices + (size_t)r0 * keep_index_stride, keep_index_stride, keep_counts + r0};
         st = run_attention(ctx, kv, 0, layer, 1, &slot, &start, &kv_valid, rows, n_q_heads,
                            q + (size_t)r0 * q_stride, 0, (long long)q_stride, gate ? gate + (size_t)r0 * gate_stride : nullptr, 0,
-                           (long long)gate_stride, scale, out + (size_t)r0 * o_stride, 0, (long long)o_stride, 1, 0, nullptr, 0, nullptr,
+                           (long long)gate_stride, scale, out + (size_t)r0 * o_stride, 0, (long long)o_stride, 1, 0, pages, 0, nullptr,
                            0, 0, false, &lists);
         if (st != TT_HIP_OK) return st;
     }
