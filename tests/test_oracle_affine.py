@@ -117,7 +117,9 @@ def test_gemv_matches_the_reference_c_kernel_bit_for_bit(bits, rows, n):
     got = oracle.affine_gemv(packed, scales, biases, x, bits)
     reference = oracle.reference_affine_gemv(packed, scales, biases, x, bits)
     if reference is None:
-        assert not os.path.isdir("/root/reference"), "the reference checkout is here but oracle/_ref was not built"
+        # (a file that `make -C oracle ref` builds from: an empty folder of that name is no checkout)
+        assert not os.path.isfile("/root/reference/sources/TinyTitanKernelsC/int4_affine_gemv.c"), \
+            "the reference checkout is here but oracle/_ref was not built"
         pytest.skip("oracle/_ref is not built (no reference checkout on this machine)")
     assert np.array_equal(got, reference)
 
