@@ -55,6 +55,34 @@ def test_null_handles_are_errors_not_crashes(lib):
     assert err.value == capi.ERR_INVALID_ARGUMENT
 
 
+def test_per_step_calls_take_what_the_c_types_take(lib):
+    # The native module in front of the per-step calls: null handles, so that an accepted call ends in a status.
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    calls, bad = capi.calls(), capi.ERR_INVALID_ARGUMENT
+
+    def decode(slot, length, layer=0, heads=8, q=None, scale=1.0):
+        return calls.attn_decode(None, None, layer, slot, length, heads, q, None, scale, None)
+
+    for length in (5, [5], (5,), np.int64(5), [np.int64(5)], torch.tensor(5), np.array(5), 5.0, True, 1 << 70, [5] * 100):
+        assert decode([0] * 100 if isinstance(length, list) and len(length) == 100 else 0, length) == bad
+    assert decode([0, 1], [5]) == bad
+    for number in (5.0, np.int64(5), torch.tensor(5), "5", None):  # a count or an index that is no int
+        with pytest.raises(TypeError):
+            decode(0, 5, layer=number)
+        with pytest.raises(TypeError):
+            decode(0, 5, heads=number)
+    for length in ("five", None, object(), [None]):
+        with pytest.raises((TypeError, ValueError)):
+            decode(0, length)
+    with pytest.raises(TypeError):
+        decode(0, 5, q=torch.zeros(4, dtype=torch.float16))  # host memory
+    with FakeTensorMode():
+        device_rows = torch.empty(2, 4, dtype=torch.float16, device="cuda")
+        with pytest.raises(RuntimeError):  # a tensor without memory of its own: an exception, not the process's end
+            torch.vmap(lambda row: decode(0, 5, q=row))(device_rows)
+
+
 def test_context_create_without_a_device_reports_it(lib):
     import torch
     if torch.cuda.is_available():

@@ -10,6 +10,7 @@
 
 #include <dlfcn.h>
 
+#include <exception>
 #include <vector>
 
 #include "../../include/ctinytitan_hip.h"
@@ -61,9 +62,16 @@ struct Args {
         if (!p && PyErr_Occurred()) ok = false;
         return static_cast<T *>(p);
     }
-    long long integer() {
+    // a Python int, as ctypes takes one: no float or tensor is rounded to a count here, and bits beyond the C type's are dropped
+    unsigned long long integer() {
         PyObject *o = next();
-        return ok ? integer_of(o) : 0;
+        if (!ok) return 0;
+        if (!PyLong_Check(o)) {
+            ok = false;
+            PyErr_Format(PyExc_TypeError, "expected an int, got %s", Py_TYPE(o)->tp_name);
+            return 0;
+        }
+        return bits_of(o);
     }
     int i() { return (int)integer(); }
     size_t size() { return (size_t)integer(); }
@@ -79,23 +87,22 @@ struct Args {
         const at::Tensor *t = tensor();
         if (!t) return nullptr;
         if (!t->is_cuda() || t->scalar_type() != at::kHalf) return fail<tt_half>("expected an fp16 device tensor");
-        return static_cast<tt_half *>(t->data_ptr());
+        return static_cast<tt_half *>(address_of(*t));
     }
     // a device tensor of 16-bit elements, taken as bit patterns
     uint16_t *bits16() {
         const at::Tensor *t = tensor();
         if (!t) return nullptr;
         if (!t->is_cuda() || t->element_size() != 2) return fail<uint16_t>("expected a device tensor of 16-bit elements");
-        return static_cast<uint16_t *>(t->data_ptr());
+        return static_cast<uint16_t *>(address_of(*t));
     }
     // a contiguous device tensor of any type, or None
     void *raw() {
         const at::Tensor *t = tensor();
         if (!t) return nullptr;
-        if (!t->is_cuda() || !t->is_contiguous()) return fail<void>("expected a contiguous device tensor");
-        return t->data_ptr();
+        return address_of(*t, true);
     }
-    // whole numbers per sequence: a list, a tuple or any sequence of them, or one number
+    // whole numbers per sequence: a list, a tuple or any sequence of them, or one number (a tensor or array without a dimension too)
     template <int N>
     int ints(int (&inline_ints)[N], std::vector<int> &heap, const int **out) {
         PyObject *o = next();
@@ -106,7 +113,8 @@ struct Args {
             return 1;
         }
         const bool list = PyList_Check(o) || PyTuple_Check(o);
-        if (!list && !PySequence_Check(o)) {
+        if (!list && (!PySequence_Check(o) || PySequence_Size(o) < 0)) {
+            PyErr_Clear();  // (a sequence by its type that has no length)
             inline_ints[0] = (int)integer_of(o);
             return 1;
         }
@@ -136,21 +144,32 @@ private:
         PyErr_SetString(PyExc_TypeError, what);
         return nullptr;
     }
-    long long integer_of(PyObject *o) {
-        if (PyLong_Check(o)) {
-            const long long v = PyLong_AsLongLong(o);
-            if (v == -1 && PyErr_Occurred()) ok = false;
-            return v;
-        }
+    unsigned long long bits_of(PyObject *whole) {
+        const unsigned long long v = PyLong_AsUnsignedLongLongMask(whole);
+        if (v == ~0ull && PyErr_Occurred()) ok = false;
+        return v;
+    }
+    unsigned long long integer_of(PyObject *o) {
+        if (PyLong_Check(o)) return bits_of(o);
         PyObject *whole = PyNumber_Long(o);  // (what int() takes: a numpy integer, a tensor of one element)
         if (!whole) {
             ok = false;
             return 0;
         }
-        const long long v = PyLong_AsLongLong(whole);
+        const unsigned long long v = bits_of(whole);
         Py_DECREF(whole);
-        if (v == -1 && PyErr_Occurred()) ok = false;
         return v;
+    }
+    // Throws nothing: a tensor without memory of its own (a traced or fake one) is a Python exception.
+    void *address_of(const at::Tensor &t, bool raw = false) {
+        try {
+            if (raw && (!t.is_cuda() || !t.is_contiguous())) return fail<void>("expected a contiguous device tensor");
+            return t.data_ptr();
+        } catch (const std::exception &e) {
+            ok = false;
+            PyErr_SetString(PyExc_RuntimeError, e.what());
+            return nullptr;
+        }
     }
     const at::Tensor *tensor() {
         PyObject *o = next();
@@ -285,7 +304,7 @@ TT_CALL(attn_verify_swa) {
     const float scale = a.real();
     tt_half *out = a.half();
     return finish(a, [&] {
-        if (slots.count != starts.count) return (int)TT_HIP_ERR_INVALID_ARGUMENT;
+        if (slots.count > starts.count) return (int)TT_HIP_ERR_INVALID_ARGUMENT;  // (positions may be a longer table than the step's)
         return lib.tt_hip_attn_verify_swa(ctx, kv, layer, slots.count, slots.values, starts.values, rows, window, heads, q, gate, scale,
                                           out);
     });
