@@ -917,3 +917,62 @@ def test_lists_over_quantised_pages_that_are_dequantised_first(gpu_ctx, bits, D,
     want = np.concatenate([_oracle_rows_kept(q[t:t + 1], _dequantised(k, bits), _dequantised(v, bits), start + t, keep[t:t + 1], H, KH, D, scale,
                                              gate=gate[t:t + 1]) for t in some])
     _check(by_list[some], want, f"dequantised pages D={D} {H}/{KH} bits {bits}")
+
+
+@pytest.mark.parametrize("bits,D,H,KH,start,rows", [(16, 256, 16, 2, 9001, 300), (8, 256, 24, 2, 13092, 361), (16, 64, 16, 4, 7003, 297),
+                                                    (4, 128, 32, 8, 20011, 300)])
+def test_lists_whose_tiles_do_not_divide_the_chip_in_whole_rounds(bits, D, H, KH, start, rows):
+    # More splits a tile than one round of workgroups holds.  The oracle, one split a tile, and captures: where the partial
+    # results' store is too small the planner's own splits, else the eager call's.
+    import torch
+    from tinytitan_amd.engine import HIPContext, PrefillAttention, PrefillAttentionParams
+    ctx = HIPContext(0)
+    r = np.random.default_rng(rows)
+    T, scale, stride = start + rows, D ** -0.5, 1201
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    q, gate = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    keep = np.zeros((rows, T), np.uint8)
+    lists, counts = np.zeros((rows, stride), np.int32), np.zeros(rows, np.int32)
+    for t in range(rows):
+        groups = r.choice((start + t) // 4, 150 + t % 150, replace=False)
+        keep[t, (4 * groups[:, None] + np.arange(4)).reshape(-1)] = 1
+        keep[t, start + t] = 1
+        ids = np.flatnonzero(keep[t])
+        lists[t, :len(ids)], counts[t] = ids, len(ids)
+    kv = _cache(ctx, bits, KH, D, T)
+    _append(ctx, kv, 0, 0, 0, k, v)
+    qd, gd, lists_d, counts_d = _dev(q), _dev(gate), _dev(lists), _dev(counts)
+    att, params = PrefillAttention(ctx), PrefillAttentionParams(start, rows, T, H, scale, H * D, H * D, H * D)
+
+    def attend(replayed=False):
+        out = torch.full((rows, H * D), float("nan"), dtype=torch.float16, device="cuda")
+        torch.cuda.synchronize()
+        if replayed:
+            ctx.graph_begin()
+        att.encode_causal(kv, 0, 0, qd, out, params, gate=gd, keep_indices=lists_d, keep_index_stride=stride, keep_counts=counts_d)
+        if replayed:
+            graph = ctx.graph_end()
+            for _ in range(3):
+                out.fill_(float("nan"))
+                torch.cuda.synchronize()
+                graph.launch()
+                ctx.synchronize()
+            graph.close()
+        ctx.synchronize()
+        return out.float().cpu().numpy()
+
+    ctx.set_split_tokens(T + 32)
+    one_split = attend()
+    ctx.set_split_tokens(0)
+    first_capture = attend(replayed=True)
+    eager = attend()
+    second_capture = attend(replayed=True)
+    kv.close()
+    ctx.close()
+    assert np.array_equal(first_capture, one_split)
+    assert np.array_equal(second_capture, eager)
+    assert np.abs(eager - one_split).max() <= 2e-3
+    some = [0, 1, 63, rows - 1]
+    ks, vs = (k, v) if bits == 16 else (_dequantised(k, bits), _dequantised(v, bits))
+    want = np.concatenate([_oracle_rows_kept(q[t:t + 1], ks, vs, start + t, keep[t:t + 1], H, KH, D, scale, gate=gate[t:t + 1]) for t in some])
+    _check(eager[some], want, f"whole rounds D={D} {H}/{KH} bits {bits}")

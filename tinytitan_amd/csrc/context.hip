@@ -336,6 +336,62 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             plan.split_len = chunk_split_blocks * 32;
             plan.n_splits_max = chunk_splits;
         }
+        // The plan of a launch over lists (its layout: below).
+        bool groups = false;
+        int cap = 0, ctx_units = 0;
+        size_t n_blocks = 0, n_bits = 0;
+        if (lists) {
+            // Groups of four keys instead of blocks of 32 (fp16 pages, tiles of 32 rows): a turn of the walk then takes eight
+            // listed groups instead of one touched block, of which a selection in blocks of four leaves 1.3 to 2 groups
+            // wanted at 32k keys and more (one row's list of 2,051 cells each): 128 rows of 16/2 heads of 256 behind 16k keys 74.0 ->
+            // 65.0 us, 32k 101.3 -> 74.2, 131k 163.0 -> 120.2, all rows sharing one selection 65.8 -> 47.8.
+            // Where the tile's lists could hold half of the keys most of a block is wanted, and a block's loads are the better ones
+            // (8k keys, 512 rows: 121.7 against 133.4 us).  Nor where many tiles walk wide heads: they share fetched lines in L2 only
+            // while they stay side by side, which the walk over blocks does better (512 rows behind 131k keys 536 against 708 us;
+            // with heads of 64 470 -> 208).  The group bitmap has to leave the plan kernel's LDS room for a run of bits.
+            const long long entries = (long long)plan.tt * (long long)lists->stride;
+            groups = kv_bits == 16 && plan.nt == 32 && 2 * entries <= totals[base] &&
+                     (long long)plan.n_tiles * D <= 128ll * ctx->n_cus && totals[base] <= kPlanGroupKeys;
+            const int unit = groups ? 4 : 32;
+            ctx_units = (totals[base] + unit - 1) / unit;
+            cap = (int)(entries < ctx_units ? entries : ctx_units);
+            if (cap < 1) cap = 1;
+            if (groups) cap = (cap + 7) & ~7;
+            n_blocks = (size_t)plan.tok_tiles * cap * (groups ? 1 : 2);
+            n_bits = (size_t)plan.tok_tiles * (groups ? cap >> 3 : cap) * plan.tt;
+        }
+        auto list_ranges = [&](int splits) { return ((size_t)plan.tok_tiles * (splits + 1) + 1) & ~(size_t)1; };
+        auto list_plan_words = [&](int splits) { return list_ranges(splits) + n_blocks + n_bits; };
+        // Lists in tiles of 32 rows: a workgroup has a CU to itself, and the planner's splits -- as many per tile as one round of
+        // workgroups holds -- leave CUs idle where the tiles do not divide them: 362 tiles take two rounds, the second of them
+        // less than half full, 150 tiles one on 150 CUs.  More splits per tile, over whole rounds, are counted out in keys'
+        // worth of walking: a round costs a split's keys and its start and merge, 2 D; a split 13 ns (at D = 256) of partial results
+        // written and read, 1.3 keys; a combine that was not there 800.  Up to ten rounds (84 MB of partial results), and
+        // a sixteenth better than fewer splits.  16/2 heads of 256, 300 rows behind 30k keys (150 tiles, 1 split -> 3) 273 -> 208 us,
+        // over 8 bits 291 -> 224, 180 rows behind 100k (90 tiles, 2 -> 5) 182 -> 163; 24/2 heads, 361 rows behind 13k (362 tiles, 1 -> 2)
+        // 293 -> 253, 300 behind 40k (1 -> 3) 511 -> 375; 32/8 of 128, 300 behind 30k (304 tiles, 1 -> 3) 341 -> 245; 16/4 of 64, 300 behind
+        // 20k (152 tiles, 1 -> 5) 150 -> 77.  Left alone where it would lose: 400 rows behind 8k keys (200 tiles) 117 against 131 and more.
+        if (lists && plan.nt == 32 && ctx->split_override <= 0 && plan.n_splits_max >= 1 && max_keys > 384) {
+            auto rounds = [&](long long splits) { return (plan.n_tiles * splits + ctx->n_cus - 1) / ctx->n_cus; };
+            auto length = [&](int splits) { return ((max_keys + splits - 1) / splits + 127) / 128 * 128; };
+            auto cost = [&](int splits) {
+                const double merge = splits > 1 ? 800.0 + 1.3 * D / 256 * plan.n_tiles * splits : 0.0;
+                return (double)rounds(splits) * (length(splits) + 2 * D) + merge;
+            };
+            const int before = plan.n_splits_max;
+            int best = before;
+            for (int splits = before + 1; splits <= before + 8 && rounds(splits) <= 10; ++splits) {
+                const size_t part_rows = (size_t)plan.n_tiles * splits * plan.nt;
+                // (inside a capture nothing can grow: the planner's splits)
+                if (ctx->capturing && (part_rows > ctx->part_rows || list_plan_words(splits) * sizeof(int) > ctx->keep_rows_bytes)) break;
+                if (cost(splits) < cost(best) * (15.0 / 16.0)) best = splits;
+            }
+            if (best > before) {
+                plan.split_len = length(best);
+                plan.n_splits_max = (max_keys + plan.split_len - 1) / plan.split_len;
+                plan.workgroups = (long long)plan.n_splits_max * plan.n_tiles;
+            }
+        }
         // Unlike lengths: the split length that makes the launch whole rounds of at most n_cus workgroups, counted with every
         // sequence's short last split -- the planner's estimate does not know those, and a workgroup over a round waits for a
         // whole one.  k workgroups a CU take len keys each at a k-th of the memory's rate, or at their own where k are too
@@ -472,28 +528,10 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         if (lists) {
             // The lists' plan, in the context's selection store: [tile][n_splits + 1] range starts, [tile][cap] blocks with
             // the keys any token keeps (pairs of words, on an even word), [tile][cap][tt] bits; a tile's list cannot be longer than the context's blocks or its tokens' entries.
-            // Groups of four keys instead of blocks of 32 (fp16 pages, tiles of 32 rows): a turn of the walk then takes eight
-            // listed groups instead of one touched block, of which a selection in blocks of four leaves 1.3 to 2 groups
-            // wanted at 32k keys and more (one row's list of 2,051 cells each): 128 rows of 16/2 heads of 256 behind 16k keys 74.0 ->
-            // 65.0 us, 32k 101.3 -> 74.2, 131k 163.0 -> 120.2, all rows sharing one selection 65.8 -> 47.8.
-            // Where the tile's lists could hold half of the keys most of a block is wanted, and a block's loads are the better ones
-            // (8k keys, 512 rows: 121.7 against 133.4 us).  Nor where many tiles walk wide heads: they share fetched lines in L2 only
-            // while they stay side by side, which the walk over blocks does better (512 rows behind 131k keys 536 against 708 us;
-            // with heads of 64 470 -> 208).  The group bitmap has to leave the plan kernel's LDS room for a run of bits.
-            const long long entries = (long long)plan.tt * (long long)lists->stride;
-            const bool groups = kv_bits == 16 && plan.nt == 32 && 2 * entries <= totals[base] &&
-                                (long long)plan.n_tiles * D <= 128ll * ctx->n_cus && totals[base] <= kPlanGroupKeys;
-            const int unit = groups ? 4 : 32;
-            const int ctx_units = (totals[base] + unit - 1) / unit;
-            int cap = (int)(entries < ctx_units ? entries : ctx_units);
-            if (cap < 1) cap = 1;
-            if (groups) cap = (cap + 7) & ~7;
-            const size_t n_ranges = ((size_t)plan.tok_tiles * (plan.n_splits_max + 1) + 1) & ~(size_t)1;
-            const size_t n_blocks = (size_t)plan.tok_tiles * cap * (groups ? 1 : 2), n_bits = (size_t)plan.tok_tiles * (groups ? cap >> 3 : cap) * plan.tt;
-            st = ensure_keep_rows(ctx, (n_ranges + n_blocks + n_bits) * sizeof(int));
+            st = ensure_keep_rows(ctx, list_plan_words(plan.n_splits_max) * sizeof(int));
             if (st != TT_HIP_OK) return st;
             int *ranges = reinterpret_cast<int *>(ctx->keep_rows);
-            int *blocks = ranges + n_ranges;
+            int *blocks = ranges + list_ranges(plan.n_splits_max);
             unsigned *bits = reinterpret_cast<unsigned *>(blocks + n_blocks);
             // LDS of the plan kernel: two words per 32 units of context and the run of bits it gathers at a time, 32 KiB
             // of them or what the context's bitmap leaves of 64 KiB.
