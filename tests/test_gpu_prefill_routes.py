@@ -64,6 +64,9 @@ def test_head_groups_the_chunk_kernel_does_not_take_and_few_rows(gpu_ctx, bits, 
 @pytest.mark.parametrize("H,KH,D,rows,start,window,ring", [
     (24, 2, 256, 777, 150, 500, 0),       # three head sets per KV head, ragged last tile, some windows clipped, some not
     (32, 8, 128, 1029, 1237, 400, 1856),  # eight KV heads (one XCD each), over a ring
+    (24, 2, 256, 300, 5001, 3000, 0),     # a window cut into key ranges, its lower edge inside the first one's blocks
+    (32, 8, 128, 291, 4100, 3001, 3520),  # ... over a ring: 4,100 % 3,520 + 291 rows do not wrap
+    (16, 2, 256, 270, 1900, 4096, 0),     # ... and a window that no row fills
     (16, 2, 256, 1030, 40, 0, 0),         # no window: the causal triangle, the longest tile first
     (12, 1, 64, 2100, 3, 0, 0)])          # one KV head, 66 tiles of three head sets: a second round of workgroups
 def test_whole_chunks_in_single_tiles(gpu_ctx, H, KH, D, rows, start, window, ring):

@@ -608,6 +608,38 @@ static ChunkEstimate estimate_chunk(const tt_hip_ctx *ctx, int D, int n_q_heads,
     return e;
 }
 
+// The chunk kernel over ranges of the key blocks that a tile walks, at most `nb_total` of them.
+struct KeyRanges {
+    int n_splits = 1, split_blocks = 0;
+    double us = 0.0;
+};
+static KeyRanges plan_key_ranges(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int nb_total) {
+    // With ranges a workgroup takes one 32-row tile of 4 heads (not a pair of tiles) over one range of key
+    // blocks.  The number of ranges by a small model of the two costs: rounds of workgroups on the chip x the
+    // blocks of a range (0.8 us a block at D = 256), and the partial results -- rows x heads x D floats per range,
+    // written by the kernel and read by the combine pass (~3 TB/s for the pair).  At least 8 blocks a range.
+    KeyRanges r;
+    const long long range_wgs = (long long)((q_len + 31) / 32) * (n_q_heads / 4);
+    const double partial_us = (double)q_len * n_q_heads * D * 4.0 * 2.0 / 3.0e6;
+    double best_us = 0.0;
+    // (1, 2, 4 or 8 kv heads: a kv head's workgroups run on its 8 / n XCDs, an equal share each)
+    const int xs = (n_kv_heads <= 8 && 8 % n_kv_heads == 0) ? 8 / n_kv_heads : 0;
+    const long long xcd_cus = ctx->n_cus / 8 > 0 ? ctx->n_cus / 8 : 1;
+    for (int s = 2; s <= 32 && nb_total / s >= 8; ++s) {
+        const int blocks = (nb_total + s - 1) / s;
+        long long rounds = (range_wgs * s + ctx->n_cus - 1) / ctx->n_cus;
+        if (xs > 0) rounds = ((range_wgs / n_kv_heads * s + xs - 1) / xs + xcd_cus - 1) / xcd_cus;
+        const double us = (double)rounds * blocks * 0.8 * D / 256.0 + s * partial_us;
+        if (r.n_splits < 2 || us < best_us) {
+            best_us = us;
+            r.split_blocks = blocks;
+            r.n_splits = (nb_total + blocks - 1) / blocks;
+            r.us = (double)rounds * blocks * chunk_step_us(D, 1.0) + s * partial_us;
+        }
+    }
+    return r;
+}
+
 // The split-K kernel's tiles of 32 packed rows: key blocks per wavefront, dearer while a tile walks few of them.
 static double estimate_splitk_chunk_us(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int first_blocks, int last_blocks) {
     const int group = n_q_heads / n_kv_heads;
@@ -617,6 +649,18 @@ static double estimate_splitk_chunk_us(const tt_hip_ctx *ctx, int D, int n_q_hea
     const double tiles = (double)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh), blocks = (first_blocks + last_blocks) / 2.0;
     const double block_us = D == 256 ? 1.6 * (1.0 + 18.0 / blocks) : D == 128 ? 0.87 * (1.0 + 11.0 / blocks) : 0.46 * (1.0 + 8.0 / blocks);
     return 5.0 + tiles * blocks / (4.0 * ctx->n_cus) * block_us;
+}
+// Tiles of one length, as a window makes them, in the whole rounds that the planner's splits leave (from 64 blocks a tile
+// on; shorter walks start apart and even out).
+static double splitk_rounds_us(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int blocks, double even_us) {
+    const int group = n_q_heads / n_kv_heads;
+    int gh = group;
+    while (gh > 32 || group % gh != 0) --gh;
+    const int tt = 32 / gh;
+    const long long tiles = (long long)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh);
+    if (blocks < 64 || tiles <= 0) return even_us;
+    const long long splits = std::max<long long>(ctx->n_cus / tiles, 1), rounds = (tiles * splits + ctx->n_cus - 1) / ctx->n_cus;
+    return 5.0 + (even_us - 5.0) * ((double)rounds * ctx->n_cus / ((double)tiles * splits));
 }
 
 }  // namespace tt
@@ -1212,6 +1256,20 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
         // kernel does not serve go through the latter.  32 / 8 heads of 128 behind a window of 4096 keys: 512 rows 65
         // against 78 us, 777 rows 105 against 80; 16 / 2 of 256 behind 1024 keys: 512 rows 24 against 34, 777 rows 43
         // against 34, 1024 rows 47 against 36.
+        // Where the chunk does not fill the chip and the split-K tiles go in whole rounds with the last one part empty, the keys of a
+        // window cut into ranges, as behind a long context (300 rows behind 4096 keys: 24 / 2 heads of 256 113.6 -> 55.3 us, 32 / 8 of
+        // 128 56.7 -> 48.3; 16 / 2 of 256, 600 rows 115.7 -> 66.8, 270 behind 16,384 keys 188.6 -> 92.3), or the chunk kernel as it is.  16 us: the
+        // combine pass and both kernels' starts.  Inside a capture the partial results' store does not grow.
+        if (serves && kv->bits == 16 && !filled && q_len >= 256) {
+            const int longest = std::max(first_blocks, last_blocks);
+            const double tiles_us = splitk_rounds_us(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, longest, splitk_us);
+            const KeyRanges r = plan_key_ranges(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, longest);
+            const size_t part_rows = (size_t)r.n_splits * n_q_heads * ((q_len + 31) / 32) * 32;
+            if (r.n_splits >= 2 && r.us + 16.0 < 0.95 * std::min(whole.us, tiles_us) && (!ctx->capturing || part_rows <= ctx->part_rows))
+                return run_attention(ctx, kv, 1, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride, gate,
+                                     0, (long long)gate_stride, scale, out, 0, (long long)o_stride, r.n_splits, r.split_blocks, nullptr, window);
+            if (whole.us < 0.75 * tiles_us) return whole_tiles(nullptr);
+        }
         if (serves && kv->bits == 16 && (filled || whole.us < splitk_us)) return whole_tiles(nullptr);
         return run_attention(ctx, kv, 0, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride,
                              gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride, 1, 0, nullptr, window);
@@ -1265,29 +1323,10 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
         int n_splits = 1, split_blocks = 0;
         double ranges_us = 0.0;
         if (!filled && q_len >= rows_from && kv_valid >= ranges_from) {
-            const int nb_total = (kv_valid + 31) / 32;
-            // With ranges a workgroup takes one 32-row tile of 4 heads (not a pair of tiles) over one range of key
-            // blocks.  The number of ranges by a small model of the two costs: rounds of workgroups on the chip x the
-            // blocks of a range (0.8 us a block at D = 256), and the partial results -- rows x heads x D floats per range,
-            // written by the kernel and read by the combine pass (~3 TB/s for the pair).  At least 8 blocks a range.
-            const long long range_wgs = (long long)((q_len + 31) / 32) * (n_q_heads / 4);
-            const double partial_us = (double)q_len * n_q_heads * kv->head_dim * 4.0 * 2.0 / 3.0e6;
-            double best_us = 0.0;
-            // (1, 2, 4 or 8 kv heads: a kv head's workgroups run on its 8 / n XCDs, an equal share each)
-            const int xs = (kv->n_kv_heads <= 8 && 8 % kv->n_kv_heads == 0) ? 8 / kv->n_kv_heads : 0;
-            const long long xcd_cus = ctx->n_cus / 8 > 0 ? ctx->n_cus / 8 : 1;
-            for (int s = 2; s <= 32 && nb_total / s >= 8; ++s) {
-                const int blocks = (nb_total + s - 1) / s;
-                long long rounds = (range_wgs * s + ctx->n_cus - 1) / ctx->n_cus;
-                if (xs > 0) rounds = ((range_wgs / kv->n_kv_heads * s + xs - 1) / xs + xcd_cus - 1) / xcd_cus;
-                const double us = (double)rounds * blocks * 0.8 * kv->head_dim / 256.0 + s * partial_us;
-                if (n_splits < 2 || us < best_us) {
-                    best_us = us;
-                    split_blocks = blocks;
-                    n_splits = (nb_total + blocks - 1) / blocks;
-                    ranges_us = (double)rounds * blocks * chunk_step_us(kv->head_dim, 1.0) + s * partial_us;
-                }
-            }
+            const KeyRanges r = plan_key_ranges(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, (kv_valid + 31) / 32);
+            n_splits = r.n_splits;
+            split_blocks = r.split_blocks;
+            ranges_us = r.us;
         }
         // Unfilled chunks, too, where a workgroup per tile is estimated faster than the ranges (1536 rows behind 8000 keys
         // 281 -> 237 us) or the split-K tiles (1024 rows behind 2000 keys 84 -> 77 us, 1536 rows 130 -> 92).
