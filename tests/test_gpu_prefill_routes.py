@@ -66,7 +66,7 @@ def test_head_groups_the_chunk_kernel_does_not_take_and_few_rows(gpu_ctx, bits, 
     (32, 8, 128, 1029, 1237, 400, 1856),  # eight KV heads (one XCD each), over a ring
     (24, 2, 256, 300, 5001, 3000, 0),     # a window cut into key ranges, its lower edge inside the first one's blocks
     (32, 8, 128, 291, 4100, 3001, 3520),  # ... over a ring: 4,100 % 3,520 + 291 rows do not wrap
-    (16, 2, 256, 270, 1900, 4096, 0),     # ... and a window that no row fills
+    (16, 2, 256, 270, 1900, 4096, 0),     # a window that clips no row is none: the dense routes
     (16, 2, 256, 1030, 40, 0, 0),         # no window: the causal triangle, the longest tile first
     (12, 1, 64, 2100, 3, 0, 0)])          # one KV head, 66 tiles of three head sets: a second round of workgroups
 def test_whole_chunks_in_single_tiles(gpu_ctx, H, KH, D, rows, start, window, ring):
@@ -96,3 +96,34 @@ def test_whole_chunks_in_single_tiles(gpu_ctx, H, KH, D, rows, start, window, ri
                               total, window, scale).reshape(rows, -1) / (1 + np.exp(-g.astype(np.float64)))
     _check(out.float().cpu().numpy(), want, f"{rows} rows behind {start} keys, {H}q/{KH}kv/{D}, window {window}, ring {ring}")
     kv.close()
+
+
+@pytest.mark.parametrize("H,KH,D,rows,start,window", [(16, 2, 256, 650, 3980, 4096), (16, 2, 256, 513, 3617, 4096), (32, 8, 128, 257, 3873, 4096),
+                                                      (24, 2, 256, 577, 8159, 8192)])
+def test_key_ranges_of_a_window_that_begins_to_clip_inside_the_chunk(gpu_ctx, H, KH, D, rows, start, window):
+    # The first tile's window still reaches over key 0 and the last tile is ragged: the tiles between them walk a block more, and
+    # a tile's last row, whose own key lies in that block, shows whether it is walked.  The oracle on those rows.
+    import torch
+    from tinytitan_amd.engine import KVCacheManager, PrefillAttention, PrefillAttentionParams
+    total, scale = start + rows, float(D) ** -0.5
+    r = np.random.default_rng(rows + start)
+    k, v = (r.standard_normal((total, KH * D)).astype(np.float16) for _ in range(2))
+    q = r.standard_normal((rows, H * D)).astype(np.float16)
+    for head in range(KH):  # a row's own key along its group's first query head: a row without it is off by far more than the bar
+        k[start:, head * D:(head + 1) * D] = q[:, head * (H // KH) * D:][:, :D] * np.float16(0.5 * 16 * scale)
+    kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=1, max_context=total, initial_capacity=total)
+    kd, vd, qd = _dev(k), _dev(v), _dev(q)
+    out = torch.full(qd.shape, float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    kv.append(0, 0, 0, kd, vd)
+    PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, total, H, scale, H * D, H * D, H * D,
+                                                                                     sliding_window=window))
+    gpu_ctx.synchronize()
+    got = out.float().cpu().numpy()
+    kv.close()
+    assert np.isfinite(got).all()
+    k32, v32 = k.astype(np.float32), v.astype(np.float32)
+    for row in [0, *range(31, rows, 32), rows - 1]:
+        want = oracle.prefill_ref(q[row:row + 1].astype(np.float32), k32, v32, H * D, KH * D, D, H, KH, start + row, 1, start + row + 1,
+                                  window, scale).reshape(1, -1)
+        _check(got[row:row + 1], want, f"row {row} of {rows} behind {start} keys, {H}q/{KH}kv/{D}, window {window}")

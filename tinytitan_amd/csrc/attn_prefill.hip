@@ -261,7 +261,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
     // Tiles in pairs (tile i with tile n - 1 - i: every workgroup the same number of key blocks under a causal
     // mask from position 0) -- or one tile each: where the keys are cut into ranges (deep in a context the tiles are equally
     // long anyway, and a workgroup with one tile leaves half the partial results of one with two), and where pairs would
-    // leave CUs idle (estimate_chunk in context.hip), the longest tile first.
+    // leave CUs idle (estimate_chunk in chunk_plan.h), the longest tile first.
     const int n_passes = (a.single_tiles || pair == a.n_tiles - 1 - pair) ? 1 : 2;
     for (int pass = 0; pass < n_passes; ++pass) {
         // The long tile goes first: the short one then fills in behind it.

@@ -5,6 +5,7 @@
 #include <mutex>
 #include <new>
 
+#include "chunk_plan.h"
 #include "internal.h"
 
 // Split-K partials of tt_hip_attn_decode_noalloc, the entry point for callers that cannot allocate: a fixed
@@ -333,6 +334,9 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
                              small_tiles_ok);
         if (st != TT_HIP_OK) return st;
         if (chunk_splits > 1) {  // the chunk kernel's geometry: 32-row one-head tiles, its own key ranges
+            // (a tile that walked past the launched ranges would lose keys, and the combine pass would count a partial result more)
+            if (longest_tile_blocks(starts[base], rows, totals[base], window) > (long long)chunk_splits * chunk_split_blocks)
+                return TT_HIP_ERR_SHAPE;
             plan.split_len = chunk_split_blocks * 32;
             plan.n_splits_max = chunk_splits;
         }
@@ -564,103 +568,6 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         if (st != TT_HIP_OK) return st;
     }
     return TT_HIP_OK;
-}
-
-// What a chunk costs by the routes that serve it, in us, from timings at 16 q heads / 2 KV heads of 256, 8 / 2 of 256, 32 / 8 of
-// 128 and 16 / 4 of 64, 512 to 4096 rows behind 0 to 9000 keys, whole and through windows of 1024 and 4096 keys.  `first_blocks`
-// and `last_blocks`: the key blocks its first and its last tile of 32 rows walk.
-
-// One key block of the chunk kernel's step, by how much of the chip takes part (at D = 256 the card's clock follows it).
-static double chunk_step_us(int D, double fill) { return D == 256 ? 0.47 + 0.50 * fill : D == 128 ? 0.41 + 0.22 * fill : 0.45 + 0.05 * fill; }
-
-struct ChunkEstimate {
-    double us;
-    bool single_tiles;  // a workgroup per tile of 32 rows instead of one per pair of them
-};
-// The chunk kernel over all of a tile's keys.  Tiles in pairs (long with short) make workgroups of one length whatever the
-// triangle; a workgroup per tile, the longest first, uses twice the CUs where pairs leave some idle (1024 rows at position
-// 0 39.4 -> 33.5 us, behind 2000 keys 124 -> 77, 2048 rows behind 8000 keys 404 -> 298, 1024 rows of 32 / 8 heads of 128 behind
-// a window of 4096 keys 150 -> 80) and splits the rounds of several finer (2500 rows of 32 / 8 of 128 at position 0
-// 107 -> 80).  Where both need the same rounds pairs are ahead -- the second tile's first blocks ride in behind the first's
-// last: 4096 rows at position 0 138 against 148 us, 2500 rows behind 8000 keys 424 against 464 -- so single tiles have to
-// promise an eighth less.
-static ChunkEstimate estimate_chunk(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int first_blocks, int last_blocks) {
-    // a kv head's workgroups run on its own XCDs where it has whole ones
-    const int xs = (n_kv_heads <= 8 && 8 % n_kv_heads == 0) ? 8 / n_kv_heads : 0;
-    const int cus = xs > 0 ? xs * (ctx->n_cus / 8 > 0 ? ctx->n_cus / 8 : 1) : ctx->n_cus;
-    const int n_tiles = (q_len + 31) / 32, sets = (xs > 0 ? n_q_heads / n_kv_heads : n_q_heads) / 4;
-    const int singles = sets * n_tiles, pairs = sets * ((n_tiles + 1) / 2);
-    const double hi = first_blocks > last_blocks ? first_blocks : last_blocks, lo = first_blocks + last_blocks - hi;
-    // the longest first: no CU is done before its longest tile, before its share of all of them, or, with k rounds begun,
-    // before k + 1 tiles of the length the last of those rounds begins with
-    double by_tile = hi, share = singles * (hi + lo) / 2.0 / cus;
-    if (share > by_tile) by_tile = share;
-    for (int k = 1; k * cus < singles; ++k) {
-        const double round = (k + 1) * (hi - (hi - lo) * (double)(k * cus) / (singles - 1));
-        if (round > by_tile) by_tile = round;
-    }
-    const double by_pair = (double)((pairs + cus - 1) / cus) * (hi + lo);
-    ChunkEstimate e;
-    e.single_tiles = singles <= cus || by_tile < 0.88 * by_pair;
-    const int workgroups = e.single_tiles ? singles : pairs;
-    const double fill = workgroups < cus ? (double)workgroups / cus : 1.0;
-    e.us = (D == 256 ? 11.0 : D == 128 ? 7.0 : 5.0) + (e.single_tiles ? by_tile : by_pair) * chunk_step_us(D, fill);
-    return e;
-}
-
-// The chunk kernel over ranges of the key blocks that a tile walks, at most `nb_total` of them.
-struct KeyRanges {
-    int n_splits = 1, split_blocks = 0;
-    double us = 0.0;
-};
-static KeyRanges plan_key_ranges(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int nb_total) {
-    // With ranges a workgroup takes one 32-row tile of 4 heads (not a pair of tiles) over one range of key
-    // blocks.  The number of ranges by a small model of the two costs: rounds of workgroups on the chip x the
-    // blocks of a range (0.8 us a block at D = 256), and the partial results -- rows x heads x D floats per range,
-    // written by the kernel and read by the combine pass (~3 TB/s for the pair).  At least 8 blocks a range.
-    KeyRanges r;
-    const long long range_wgs = (long long)((q_len + 31) / 32) * (n_q_heads / 4);
-    const double partial_us = (double)q_len * n_q_heads * D * 4.0 * 2.0 / 3.0e6;
-    double best_us = 0.0;
-    // (1, 2, 4 or 8 kv heads: a kv head's workgroups run on its 8 / n XCDs, an equal share each)
-    const int xs = (n_kv_heads <= 8 && 8 % n_kv_heads == 0) ? 8 / n_kv_heads : 0;
-    const long long xcd_cus = ctx->n_cus / 8 > 0 ? ctx->n_cus / 8 : 1;
-    for (int s = 2; s <= 32 && nb_total / s >= 8; ++s) {
-        const int blocks = (nb_total + s - 1) / s;
-        long long rounds = (range_wgs * s + ctx->n_cus - 1) / ctx->n_cus;
-        if (xs > 0) rounds = ((range_wgs / n_kv_heads * s + xs - 1) / xs + xcd_cus - 1) / xcd_cus;
-        const double us = (double)rounds * blocks * 0.8 * D / 256.0 + s * partial_us;
-        if (r.n_splits < 2 || us < best_us) {
-            best_us = us;
-            r.split_blocks = blocks;
-            r.n_splits = (nb_total + blocks - 1) / blocks;
-            r.us = (double)rounds * blocks * chunk_step_us(D, 1.0) + s * partial_us;
-        }
-    }
-    return r;
-}
-
-// The split-K kernel's tiles of 32 packed rows: key blocks per wavefront, dearer while a tile walks few of them.
-static double estimate_splitk_chunk_us(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int first_blocks, int last_blocks) {
-    const int group = n_q_heads / n_kv_heads;
-    int gh = group;
-    while (gh > 32 || group % gh != 0) --gh;
-    const int tt = 32 / gh;
-    const double tiles = (double)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh), blocks = (first_blocks + last_blocks) / 2.0;
-    const double block_us = D == 256 ? 1.6 * (1.0 + 18.0 / blocks) : D == 128 ? 0.87 * (1.0 + 11.0 / blocks) : 0.46 * (1.0 + 8.0 / blocks);
-    return 5.0 + tiles * blocks / (4.0 * ctx->n_cus) * block_us;
-}
-// Tiles of one length, as a window makes them, in the whole rounds that the planner's splits leave (from 64 blocks a tile
-// on; shorter walks start apart and even out).
-static double splitk_rounds_us(const tt_hip_ctx *ctx, int D, int n_q_heads, int n_kv_heads, int q_len, int blocks, double even_us) {
-    const int group = n_q_heads / n_kv_heads;
-    int gh = group;
-    while (gh > 32 || group % gh != 0) --gh;
-    const int tt = 32 / gh;
-    const long long tiles = (long long)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh);
-    if (blocks < 64 || tiles <= 0) return even_us;
-    const long long splits = std::max<long long>(ctx->n_cus / tiles, 1), rounds = (tiles * splits + ctx->n_cus - 1) / ctx->n_cus;
-    return 5.0 + (even_us - 5.0) * ((double)rounds * ctx->n_cus / ((double)tiles * splits));
 }
 
 }  // namespace tt
@@ -1235,21 +1142,16 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
     // 25 us through the split-K tiles; behind a 1024-key window 62 us against 20 us.
     const long long pair_blocks = (2LL * start_pos + q_len) / 32 + 2;  // key blocks a workgroup's pair of tiles walks
     const bool filled = 2 * chunk_wgs >= ctx->n_cus || (window == 0 && 4 * chunk_wgs >= ctx->n_cus && pair_blocks <= 64);
-    // Key blocks that the chunk's tile of rows [32 t, 32 t + 32) walks.
-    auto tile_blocks = [&](int t) {
-        const long long end = std::min<long long>(kv_valid, (long long)start_pos + std::min(q_len, 32 * t + 32));
-        const long long first = window > 0 && start_pos + 32LL * t + 1 > window ? start_pos + 32LL * t + 1 - window : 0;
-        return (int)((end + 31) / 32 - first / 32);
-    };
-    const int first_blocks = tile_blocks(0), last_blocks = tile_blocks((q_len + 31) / 32 - 1);
-    const ChunkEstimate whole = estimate_chunk(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, first_blocks, last_blocks);
+    const int first_blocks = chunk_tile_blocks(start_pos, q_len, kv_valid, window, 0);
+    const int last_blocks = chunk_tile_blocks(start_pos, q_len, kv_valid, window, (q_len + 31) / 32 - 1);
+    const ChunkEstimate whole = estimate_chunk(ctx->n_cus, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, first_blocks, last_blocks);
     auto whole_tiles = [&](const PageSource *pages) {
         if (hipSetDevice(ctx->device) != hipSuccess) return (int)TT_HIP_ERR_HIP;
         return launch_prefill(ctx, kv, layer, slot, start_pos, q_len, kv_valid, n_q_heads, q, (long long)q_stride, gate,
                               (long long)gate_stride, scale, out, (long long)o_stride, 1, 0, nullptr, nullptr, pages, window,
                               whole.single_tiles);
     };
-    const double splitk_us = estimate_splitk_chunk_us(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, first_blocks, last_blocks);
+    const double splitk_us = estimate_splitk_chunk_us(ctx->n_cus, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, first_blocks, last_blocks);
     if (window > 0) {
         // The chunk kernel starts every tile at its window's first block.  It or the split-K kernel (GQA-packed tiles, each
         // walking only its rows' windows), whichever is estimated faster; quantised pages and head groups the chunk
@@ -1261,9 +1163,9 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
         // 128 56.7 -> 48.3; 16 / 2 of 256, 600 rows 115.7 -> 66.8, 270 behind 16,384 keys 188.6 -> 92.3), or the chunk kernel as it is.  16 us: the
         // combine pass and both kernels' starts.  Inside a capture the partial results' store does not grow.
         if (serves && kv->bits == 16 && !filled && q_len >= 256) {
-            const int longest = std::max(first_blocks, last_blocks);
-            const double tiles_us = splitk_rounds_us(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, longest, splitk_us);
-            const KeyRanges r = plan_key_ranges(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, longest);
+            const int longest = longest_tile_blocks(start_pos, q_len, kv_valid, window);
+            const double tiles_us = splitk_rounds_us(ctx->n_cus, n_q_heads, kv->n_kv_heads, q_len, longest, splitk_us);
+            const KeyRanges r = plan_window_ranges(ctx->n_cus, kv->head_dim, n_q_heads, kv->n_kv_heads, start_pos, q_len, kv_valid, window);
             const size_t part_rows = (size_t)r.n_splits * n_q_heads * ((q_len + 31) / 32) * 32;
             if (r.n_splits >= 2 && r.us + 16.0 < 0.95 * std::min(whole.us, tiles_us) && (!ctx->capturing || part_rows <= ctx->part_rows))
                 return run_attention(ctx, kv, 1, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride, gate,
@@ -1323,7 +1225,7 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
         int n_splits = 1, split_blocks = 0;
         double ranges_us = 0.0;
         if (!filled && q_len >= rows_from && kv_valid >= ranges_from) {
-            const KeyRanges r = plan_key_ranges(ctx, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, (kv_valid + 31) / 32);
+            const KeyRanges r = plan_key_ranges(ctx->n_cus, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, (kv_valid + 31) / 32);
             n_splits = r.n_splits;
             split_blocks = r.split_blocks;
             ranges_us = r.us;
