@@ -83,6 +83,29 @@ def test_per_step_calls_take_what_the_c_types_take(lib):
             torch.vmap(lambda row: decode(0, 5, q=row))(device_rows)
 
 
+def test_a_list_that_shrinks_while_its_items_are_converted(lib):
+    calls, freed = capi.calls(), []
+
+    class Item:
+        def __init__(self, table):
+            self.table = table
+
+        def __int__(self):
+            self.table.clear()
+            return 1
+
+        def __del__(self):
+            freed.append(self)
+
+    for n in (2, 64, 65, 200):
+        slots = []
+        slots += [Item(slots) for _ in range(n)]
+        lengths = [1] * n
+        converted = len(freed)
+        assert calls.attn_decode(None, None, 0, slots, lengths, 8, None, None, 1.0, None) == capi.ERR_INVALID_ARGUMENT
+        assert slots == [] and len(freed) == converted + n
+
+
 def test_context_create_without_a_device_reports_it(lib):
     import torch
     if torch.cuda.is_available():

@@ -112,27 +112,34 @@ struct Args {
             inline_ints[0] = (int)integer_of(o);
             return 1;
         }
-        const bool list = PyList_Check(o) || PyTuple_Check(o);
+        bool list = PyList_Check(o) || PyTuple_Check(o);
         if (!list && (!PySequence_Check(o) || PySequence_Size(o) < 0)) {
             PyErr_Clear();  // (a sequence by its type that has no length)
             inline_ints[0] = (int)integer_of(o);
             return 1;
         }
-        PyObject *fast = list ? nullptr : PySequence_Fast(o, "expected whole numbers, one per sequence");
-        if (!list && !fast) {
-            ok = false;
-            return 0;
+        // Items that are ints are read where they lie: no Python code runs meanwhile, so the caller's list stays as it is.  Any
+        // other item's conversion may run some that shortens the list, or hand the interpreter lock to a thread that
+        // does: those are converted from a copy.
+        PyObject *copy = nullptr;
+        Py_ssize_t n = list ? PySequence_Fast_GET_SIZE(o) : 0;
+        for (Py_ssize_t k = 0; k < n && list; ++k) list = PyLong_Check(PySequence_Fast_GET_ITEM(o, k));
+        if (!list) {
+            copy = PySequence_Tuple(o);
+            if (!copy) {
+                ok = false;
+                return 0;
+            }
+            n = PyTuple_GET_SIZE(copy);
         }
-        PyObject *seq = list ? o : fast;
-        const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
         int *to = inline_ints;
         if (n > N) {
             heap.resize((size_t)n);
             to = heap.data();
         }
-        for (Py_ssize_t k = 0; k < n && ok; ++k) to[k] = (int)integer_of(PySequence_Fast_GET_ITEM(seq, k));
+        for (Py_ssize_t k = 0; k < n && ok; ++k) to[k] = (int)integer_of(copy ? PyTuple_GET_ITEM(copy, k) : PySequence_Fast_GET_ITEM(o, k));
         *out = to;
-        Py_XDECREF(fast);
+        Py_XDECREF(copy);
         return (int)n;
     }
 
