@@ -67,7 +67,15 @@ def test_per_step_calls_take_what_the_c_types_take(lib):
     for length in (5, [5], (5,), np.int64(5), [np.int64(5)], torch.tensor(5), np.array(5), 5.0, True, 1 << 70, [5] * 100):
         assert decode([0] * 100 if isinstance(length, list) and len(length) == 100 else 0, length) == bad
     assert decode([0, 1], [5]) == bad
-    for number in (5.0, np.int64(5), torch.tensor(5), "5", None):  # a count or an index that is no int
+    direct = lib.tt_hip_attn_decode
+    one = (ctypes.c_int * 1)(5)
+    for number in (5, True, np.int64(5), np.uint8(5), np.array(5), torch.tensor(5), torch.tensor([5], dtype=torch.int32), 1 << 70):
+        assert direct(None, None, number, 1, one, one, number, None, None, 1.0, None) == bad
+        assert decode(0, 5, layer=number) == bad and decode(0, 5, heads=number) == bad
+        assert calls.attn_decode_keep(None, None, 0, 0, 5, None, number, 8, None, None, 1.0, None) == bad  # a stride: size_t
+    for number in (5.0, np.float32(5), torch.tensor(5.0), torch.tensor([5, 6]), "5", None):  # a count or an index that is no integer
+        with pytest.raises((TypeError, ctypes.ArgumentError)):
+            direct(None, None, number, 1, one, one, 8, None, None, 1.0, None)
         with pytest.raises(TypeError):
             decode(0, 5, layer=number)
         with pytest.raises(TypeError):

@@ -62,16 +62,13 @@ struct Args {
         if (!p && PyErr_Occurred()) ok = false;
         return static_cast<T *>(p);
     }
-    // a Python int, as ctypes takes one: no float or tensor is rounded to a count here, and bits beyond the C type's are dropped
+    // What ctypes takes for a C integer: an int, or what says of itself that it is one (__index__: a numpy integer, an integer
+    // tensor of one element).  No float is rounded to a count here, and bits beyond the C type's are dropped.
     unsigned long long integer() {
         PyObject *o = next();
         if (!ok) return 0;
-        if (!PyLong_Check(o)) {
-            ok = false;
-            PyErr_Format(PyExc_TypeError, "expected an int, got %s", Py_TYPE(o)->tp_name);
-            return 0;
-        }
-        return bits_of(o);
+        if (PyLong_Check(o)) return bits_of(o);
+        return bits_of_new(PyNumber_Index(o));
     }
     int i() { return (int)integer(); }
     size_t size() { return (size_t)integer(); }
@@ -158,7 +155,9 @@ private:
     }
     unsigned long long integer_of(PyObject *o) {
         if (PyLong_Check(o)) return bits_of(o);
-        PyObject *whole = PyNumber_Long(o);  // (what int() takes: a numpy integer, a tensor of one element)
+        return bits_of_new(PyNumber_Long(o));  // (what int() takes)
+    }
+    unsigned long long bits_of_new(PyObject *whole) {
         if (!whole) {
             ok = false;
             return 0;
