@@ -91,6 +91,31 @@ def test_per_step_calls_take_what_the_c_types_take(lib):
             torch.vmap(lambda row: decode(0, 5, q=row))(device_rows)
 
 
+def test_tables_are_what_they_were_before_the_native_calls(lib):
+    # A step's slots and lengths: a list or a tuple, or one number by int(); a verify pass's: whatever has a length.
+    import torch
+    calls, bad = capi.calls(), capi.ERR_INVALID_ARGUMENT
+
+    def decode(table):
+        return calls.attn_decode(None, None, 0, table, table, 8, None, None, 1.0, None)
+
+    def verify(table):
+        return calls.attn_verify_swa(None, None, 0, table, table, 1, 0, 8, None, None, 1.0, None)
+
+    several = [range(3), np.arange(3), torch.arange(3), {0: 1, 1: 2}, {0: 1, 1: 2}.values(), {0, 1}]
+    one = [3, np.int32(3), torch.tensor(3)]
+    for table in ([0, 1], (0, 1), [np.int64(0), torch.tensor(1)], *several):
+        assert verify(table) == bad
+    for table in ([0, 1], (0, 1), *one, torch.tensor([3]), 3.0, "3"):
+        assert decode(table) == bad
+    for table in several:
+        with pytest.raises((TypeError, ValueError)):
+            decode(table)
+    for table in (*one, 3.0, None, iter([0, 1]), ["x"], [None]):
+        with pytest.raises((TypeError, ValueError)):
+            verify(table)
+
+
 def test_a_list_that_shrinks_while_its_items_are_converted(lib):
     calls, freed = capi.calls(), []
 

@@ -99,21 +99,21 @@ struct Args {
         if (!t) return nullptr;
         return address_of(*t, true);
     }
-    // whole numbers per sequence: a list, a tuple or any sequence of them, or one number (a tensor or array without a dimension too)
+    // Whole numbers per sequence, each what int() takes.  As a step's own: a list or a tuple of them, or one number.  As a
+    // `table`: whatever has a length and can be gone through (an array, a tensor, a view of a dict), but no number.
     template <int N>
-    int ints(int (&inline_ints)[N], std::vector<int> &heap, const int **out) {
+    int ints(int (&inline_ints)[N], std::vector<int> &heap, const int **out, bool table) {
         PyObject *o = next();
         *out = inline_ints;
         if (!ok) return 0;
-        if (PyLong_Check(o)) {
+        bool list = PyList_Check(o) || PyTuple_Check(o);
+        if (!list && !table) {
             inline_ints[0] = (int)integer_of(o);
             return 1;
         }
-        bool list = PyList_Check(o) || PyTuple_Check(o);
-        if (!list && (!PySequence_Check(o) || PySequence_Size(o) < 0)) {
-            PyErr_Clear();  // (a sequence by its type that has no length)
-            inline_ints[0] = (int)integer_of(o);
-            return 1;
+        if (!list && PyObject_Size(o) < 0) {
+            ok = false;
+            return 0;
         }
         // Items that are ints are read where they lie: no Python code runs meanwhile, so the caller's list stays as it is.  Any
         // other item's conversion may run some that shortens the list, or hand the interpreter lock to a thread that
@@ -193,7 +193,7 @@ struct Ints {  // one per-sequence table of a call: on the stack for the batch s
     std::vector<int> heap;
     const int *values = on_stack;
     int count = 0;
-    void take(Args &a) { count = a.ints(on_stack, heap, &values); }
+    void take(Args &a, bool table = false) { count = a.ints(on_stack, heap, &values, table); }
 };
 
 template <typename Call>
@@ -303,8 +303,8 @@ TT_CALL(attn_verify_swa) {
     auto *kv = a.handle<tt_hip_kv>();
     const int layer = a.i();
     Ints slots, starts;
-    slots.take(a);
-    starts.take(a);
+    slots.take(a, true);
+    starts.take(a, true);
     const int rows = a.i(), window = a.i(), heads = a.i();
     const tt_half *q = a.half(), *gate = a.half();
     const float scale = a.real();
