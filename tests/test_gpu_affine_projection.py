@@ -142,6 +142,33 @@ def test_tiles_of_every_form_at_their_edges(gpu_ctx, bits, m, n, tokens, offset)
     _case(gpu_ctx, bits, m, n, tokens, 2000 + m + n + tokens, x_stride=n + 8, y_stride=m + 3, weights_offset=offset)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("tokens", [1, 5, 16, 40, 128, 300, 512])
+def test_infinities_and_levels_of_zero(gpu_ctx, bits, tokens):
+    # scale * sum(level * x) + bias * sum(x) as written: an infinite x leaves an infinity where its level is not zero and the
+    # bias does not pull the other way, a NaN elsewhere, and nothing in other tokens' rows; a row whose levels are all zero
+    # has no first sum at all, whatever the sizes of x (scale 1, so that what another order of the sums leaves would show).
+    rows, n = 200, 1152
+    packed, scales, biases = _weights(rows, n, bits, 77 + bits)
+    packed[:64], scales[:64], biases[:64] = 0, oracle.bf16_bits(1.0), 0
+    biases[64:132] = oracle.bf16_bits(0.03125)
+    r = np.random.default_rng(tokens)
+    x = r.uniform(-1.0, 1.0, (tokens, n)).astype(np.float16)
+    odd = np.arange(tokens) % 3 == 1 if tokens > 1 else np.ones(1, bool)
+    x[odd] = (x[odd].astype(np.float32) * 2.0 ** r.integers(-12, 15, x[odd].shape)).astype(np.float16)
+    finite = _project(gpu_ctx, bits, packed, scales, biases, x)
+    assert not finite[:, :64].any()
+    at = r.integers(0, n, tokens)
+    clipped = np.arange(tokens) % 4 == 0
+    x[clipped, at[clipped]] = np.where(at[clipped] % 2 == 0, np.inf, -np.inf).astype(np.float16)
+    got = _project(gpu_ctx, bits, packed, scales, biases, x)
+    with np.errstate(invalid="ignore"):
+        want = oracle.affine_projection(packed, scales, biases, x.astype(np.float32), bits)
+    assert np.isinf(want[clipped]).any() and np.isnan(want[clipped]).any()
+    assert np.array_equal(got[clipped], want[clipped], equal_nan=True)
+    assert np.array_equal(got[~clipped], finite[~clipped])
+
+
 GEMM_MIN_TOKENS = 513  # from here on a chunk takes the GEMM kernel, whose weights are rounded to fp16 like the reference's tensor-op tile
 
 

@@ -116,16 +116,17 @@ typedef unsigned u2v __attribute__((ext_vector_type(2)));
 // (2048 x 4096, 4 bits) took 7.9 us a launch that way, and 6.0 with token strides 16 bytes off a multiple of a line.
 // So x and the levels go to LDS by LDS-direct loads in whole lines, their 16-byte pieces permuted by row on the way so
 // that the fragment reads hit every bank.
-// A 4-bit level is shifted into the mantissa of 16.0 (16 + level, exact; eight instructions for eight levels, whose pairs
-// (k, k + 4) x follows by a permute), and the constant of the sums is -16: a group's dot product starts from
-// -16 sum(x), exact as the rest of it.  (Levels as subnormal halves, n times 2^-24, would save those instructions' or and
-// the start, but the matrix cores lose low bits on them: 95.5 % of the outputs bit-equal to the oracle instead of 99.85.)
+// A 4-bit level left where it lies in a half is a subnormal number; a multiplication makes it level / 512 (exact; nine
+// instructions for eight levels, whose pairs (k, k + 4) x follows by a permute), biases are taken by 512 less as well and
+// the tile's sums times 512 at the end.  (The matrix cores themselves lose low bits of subnormal halves: 95.5 % of the outputs
+// bit-equal to the oracle instead of 99.85.  Levels in the mantissa of 16.0, with a sum that starts from -16 sum(x), cost an
+// instruction less, but are rounded at up to three times their size, and an infinite x is a NaN in them.)
 // The rest is bytes per CU, 16 MT x 8 KiB of x + 16 NR x 2.25 KiB of levels, at 35-40 KB/us.  us a launch, before (tiles of
 // 32 x 32, x through registers and private patches of LDS) -> now:
-//   2048 x 4096, 4 bits:   5 tokens 6.6 -> 5.5, 16: 9.8 -> 5.6, 32: 10.0 -> 5.7, 64: 10.2 -> 7.4, 128: 10.5 -> 9.8,
-//                          256: 18.7 -> 14.9, 512: 29.2 -> 27.5
-//   2048 x 4096, 8 bits:   32: 10.9 -> 6.1, 128: 11.6 -> 9.7, 512: 32.9 -> 27.6
-//   2048 x 6144, 4 bits:   16: 14.6 -> 6.8, 128: 15.9 -> 11.6;  512 x 2048, 4 bits: 5: 4.8 -> 3.4, 128: 7.2 -> 3.8
+//   2048 x 4096, 4 bits:   5 tokens 6.2 -> 4.7, 16: 9.7 -> 4.8, 32: 9.8 -> 5.0, 64: 9.9 -> 7.0, 128: 10.1 -> 8.7,
+//                          256: 18.1 -> 14.7, 512: 29.5 -> 25.9
+//   2048 x 4096, 8 bits:   32: 10.8 -> 5.9, 128: 10.9 -> 9.4, 512: 33.0 -> 27.5
+//   4096 x 4096, 4 bits:   16: 9.9 -> 5.6, 128: 18.3 -> 15.1;  512 x 2048, 4 bits: 5: 4.8 -> 3.5, 128: 7.2 -> 3.8
 // ---------------------------------------------------------------------------
 constexpr int kTileWaves = 8;  // wavefronts that share a row's groups
 // A wavefront's part of LDS: x [token tile][group][16 tokens][128 B], then levels [16 NR rows][SPAN groups].
@@ -193,7 +194,9 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nr = 0; nr < NR; ++nr) acc[mt][nr] = zero;
-    const h8 ones = (h8)(_Float16)(BITS == 4 ? -16 : 1);
+    const h8 ones = (h8)(_Float16)1;
+    const h8 to_levels = {0x1p15f16, 0x1p15f16, 0x1p11f16, 0x1p11f16, 0x1p15f16, 0x1p15f16, 0x1p11f16, 0x1p11f16};
+    constexpr float kBiasUnit = BITS == 4 ? 0x1p-9f : 1.0f, kSumUnit = BITS == 4 ? 0x1p9f : 1.0f;
 
     for (int g0 = g_begin; g0 < g_end; g0 += 4) {
         unsigned scales[NR][2], biases[NR][2];
@@ -275,26 +278,22 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
 #pragma unroll
                 for (int nr = 0; nr < NR; ++nr) {
                     const unsigned sp = scales[nr][g4 / 2], bp = biases[nr][g4 / 2];
-                    const float bias = __builtin_bit_cast(float, (g4 & 1) ? (bp & 0xffff0000u) : (bp << 16)) * (BITS == 4 ? -0.0625f : 1.0f);
+                    const float bias = __builtin_bit_cast(float, (g4 & 1) ? (bp & 0xffff0000u) : (bp << 16)) * kBiasUnit;
                     const float scale = __builtin_bit_cast(float, (g4 & 1) ? (sp & 0xffff0000u) : (sp << 16));
                     h8 levels[2];
 #pragma unroll
                     for (int i = 0; i < 2; ++i) {
-                        u4v bits;  // 16 + level (4 bits), 1024 + level (8 bits)
-                        constexpr unsigned e = BITS == 4 ? 0x4c004c00u : 0x64646464u;
                         if constexpr (BITS == 4) {
-                            const unsigned v = w[nr][2 * gi + i];
-                            bits = u4v{((v << 6) & 0x03c003c0u) | e, ((v << 2) & 0x03c003c0u) | e, ((v >> 2) & 0x03c003c0u) | e, ((v >> 6) & 0x03c003c0u) | e};
+                            const unsigned v = w[nr][2 * gi + i], u = v >> 8;
+                            const u4v low = {v & 0x000f000fu, v & 0x00f000f0u, u & 0x000f000fu, u & 0x00f000f0u};  // level / 2^24, level / 2^20
+                            levels[i] = __builtin_bit_cast(h8, low) * to_levels;
                         } else {
-                            const unsigned w0 = w[nr][4 * gi + 2 * i], w1 = w[nr][4 * gi + 2 * i + 1];
-                            bits = u4v{__builtin_amdgcn_perm(e, w0, 0x04010400u), __builtin_amdgcn_perm(e, w0, 0x04030402u),
-                                       __builtin_amdgcn_perm(e, w1, 0x04010400u), __builtin_amdgcn_perm(e, w1, 0x04030402u)};
+                            levels[i] = levels_of_bytes(w[nr][4 * gi + 2 * i], w[nr][4 * gi + 2 * i + 1]);
                         }
-                        levels[i] = BITS == 4 ? __builtin_bit_cast(h8, bits) : __builtin_bit_cast(h8, bits) - (h8)(_Float16)1024;
                     }
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) {
-                        f4v dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[mt][0], levels[0], BITS == 4 ? xsum[mt] : zero, 0, 0, 0);
+                        f4v dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[mt][0], levels[0], zero, 0, 0, 0);
                         dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[mt][1], levels[1], dot, 0, 0, 0);
 #pragma unroll
                         for (int j = 0; j < 4; ++j) acc[mt][nr][j] = fmaf(bias, xsum[mt][j], fmaf(scale, dot[j], acc[mt][nr][j]));
@@ -317,7 +316,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
         float sum = 0.0f;
 #pragma unroll
         for (int w2 = 0; w2 < kTileWaves; ++w2) sum += sums[(w2 * kTokens + t) * kPitch + r];
-        if (token0 + t < a.tokens && row0 + r < a.rows) a.y[(long long)(token0 + t) * a.y_stride + row0 + r] = (_Float16)sum;
+        if (token0 + t < a.tokens && row0 + r < a.rows) a.y[(long long)(token0 + t) * a.y_stride + row0 + r] = (_Float16)(sum * kSumUnit);
     }
 }
 
