@@ -137,7 +137,8 @@ def test_rows_are_independent_of_their_neighbours(gpu_ctx):
     (4, 17, 64, 5), (4, 2047, 704, 16), (8, 15, 2112, 17),      # 16 x 16; one group, 11 and 33 groups (parts of 2, of 8 and an odd one)
     (4, 2041, 320, 33), (8, 1030, 2304, 64),                    # 16 tokens x 32 rows
     (4, 1999, 1088, 97), (8, 2047, 192, 128), (4, 63, 4160, 512),  # 32 x 32
-    (8, 2017, 320, 300)])                                       # 32 x 64, 8 bits
+    (8, 2017, 320, 300),                                        # 32 x 64, 8 bits
+    (4, 8191, 64, 300), (4, 8192, 64, 512), (4, 8197, 128, 290), (8, 8255, 64, 45), (4, 12300, 64, 33), (8, 8200, 64, 6)])  # many rows, in passes
 def test_tiles_of_every_form_at_their_edges(gpu_ctx, bits, m, n, tokens, offset):
     _case(gpu_ctx, bits, m, n, tokens, 2000 + m + n + tokens, x_stride=n + 8, y_stride=m + 3, weights_offset=offset)
 

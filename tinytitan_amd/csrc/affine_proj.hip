@@ -34,6 +34,7 @@ struct ProjArgs {
     _Float16 *y;
     long long x_stride, y_stride;
     int rows, columns, tokens;
+    int pass_tiles, pass_rows;  // > 0: the grid is one-dimensional, passes over the rows (affine_tile_kernel)
 };
 
 // Eight bytes -> eight halves holding 0..255 exactly: byte b under exponent byte 0x64 is 1024 + b.
@@ -126,7 +127,7 @@ typedef unsigned u2v __attribute__((ext_vector_type(2)));
 //   2048 x 4096, 4 bits:   5 tokens 6.2 -> 4.7, 16: 9.7 -> 4.8, 32: 9.8 -> 5.0, 64: 9.9 -> 7.0, 128: 10.1 -> 8.7,
 //                          256: 18.1 -> 14.7, 512: 29.5 -> 25.9
 //   2048 x 4096, 8 bits:   32: 10.8 -> 5.9, 128: 10.9 -> 9.4, 512: 33.0 -> 27.5
-//   4096 x 4096, 4 bits:   16: 9.9 -> 5.6, 128: 18.3 -> 15.1;  512 x 2048, 4 bits: 5: 4.8 -> 3.5, 128: 7.2 -> 3.8
+//   2048 x 6144, 4 bits:   16: 13.7 -> 6.3, 128: 14.6 -> 11.0;  512 x 2048, 4 bits: 5: 4.8 -> 3.5, 128: 7.2 -> 3.8
 // ---------------------------------------------------------------------------
 constexpr int kTileWaves = 8;  // wavefronts that share a row's groups
 // A wavefront's part of LDS: x [token tile][group][16 tokens][128 B], then levels [16 NR rows][SPAN groups].
@@ -166,7 +167,16 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int n = lane & 15, kq = lane >> 4;
-    const int row0 = blockIdx.x * kRows, token0 = blockIdx.y * kTokens;
+    int row_tile = blockIdx.x, token_tile = blockIdx.y;
+    if (a.pass_tiles > 0) {
+        // A pass is `pass_tiles` token tiles over all rows; an XCD takes every eighth row tile, with all of a pass's token
+        // tiles one after the other.
+        const int at = (int)(blockIdx.x >> 3), pass = at / (a.pass_tiles * a.pass_rows), in_pass = at - pass * (a.pass_tiles * a.pass_rows);
+        token_tile = pass * a.pass_tiles + in_pass % a.pass_tiles;
+        row_tile = 8 * (in_pass / a.pass_tiles) + (int)(blockIdx.x & 7);
+        if (row_tile * kRows >= a.rows || token_tile * kTokens >= a.tokens) return;  // the whole workgroup: padding of the grid
+    }
+    const int row0 = row_tile * kRows, token0 = token_tile * kTokens;
     const int groups = a.columns / kProjGroup;
     int per_wave = (groups + kTileWaves - 1) / kTileWaves;
     if (groups >= 4 * kTileWaves) per_wave = (per_wave + 3) / 4 * 4;
@@ -321,15 +331,28 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
 }
 
 // The smallest tile whose workgroups find a CU each -- a wider tile reads less per output but takes longer: 32 tokens
-// 5.6 us in tiles of 16 x 16 (256 workgroups), 6.8 in 16 x 32, 9.1 in 32 x 32; 64 tokens 8.1 / 7.0 / 9.1; 128 tokens
-// 12.8 / 12.0 / 9.8 (10.2 with two groups instead of four in LDS at a time, which lets two workgroups share a CU) -- and
-// beyond that 32 x 32, two workgroups to a CU (256 tokens 14.9 us, with four groups in LDS 17.9), or over 8 bits, whose levels weigh twice as much, 32 x 64 (256 tokens 13.2 against 16.0 us).
+// 5.1 us in tiles of 16 x 16 (256 workgroups), 7.0 in 16 x 32, 8.7 in 32 x 32; 64 tokens 7.4 / 7.0 / 8.7; 128 tokens
+// 12.2 / 12.3 / 8.8 (9.8 with two groups instead of four in LDS at a time, which lets two workgroups share a CU) -- and
+// beyond that 32 x 32, two workgroups to a CU (256 tokens 14.7 us, with four groups in LDS 16.1), or over 8 bits, whose levels weigh twice as much, 32 x 64 (256 tokens 13.2 against 16.0 us).
 template <int BITS, bool ALIGNED>
 void launch_tile(tt_hip_ctx *ctx, const ProjArgs &a) {
     auto tiles = [&](int mt, int nr) { return (long long)((a.rows + 16 * nr - 1) / (16 * nr)) * ((a.tokens + 16 * mt - 1) / (16 * mt)); };
     auto launch = [&](auto kernel, int mt, int nr, int lds) {
-        const dim3 grid((unsigned)((a.rows + 16 * nr - 1) / (16 * nr)), (unsigned)((a.tokens + 16 * mt - 1) / (16 * mt)));
-        launch_profiled(ctx, kernel, grid, dim3(kTileWaves * 64), (unsigned)lds, a);
+        dim3 grid((unsigned)((a.rows + 16 * nr - 1) / (16 * nr)), (unsigned)((a.tokens + 16 * mt - 1) / (16 * mt)));
+        // Many rows: their weights outlast no L2 from one token tile to the next, so the token tiles of some rows follow each
+        // other on one XCD, eight at a time (the x of 256 tokens and the weights in flight still fit its L2).  4 bits, 4096
+        // columns: 8192 rows x 256 tokens 50.8 -> 47.9 us, 512 98.3 -> 93.2, 16,384 x 128 52.2 -> 47.9, 512 195.1 -> 181.5; 8
+        // bits 16,384 x 256 111.7 -> 106.8.  Fewer rows stay in the L2s as they are: 2048 x 64 7.15 against 7.36, 512 25.8 against 26.4.
+        ProjArgs b = a;
+        if (a.rows >= 8192 && grid.y > 1) {
+            const unsigned pass = grid.y < 8 ? grid.y : 8, passes = (grid.y + pass - 1) / pass, per_xcd = (grid.x + 7) / 8;
+            if ((unsigned long long)per_xcd * 8 * pass * passes <= 1u << 22) {  // (a grid of 2^31 threads)
+                b.pass_tiles = (int)pass;
+                b.pass_rows = (int)per_xcd;
+                grid = dim3(per_xcd * 8 * pass * passes);
+            }
+        }
+        launch_profiled(ctx, kernel, grid, dim3(kTileWaves * 64), (unsigned)lds, b);
     };
     if (tiles(1, 1) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 1, 1, 4>, 1, 1, tile_lds_bytes(BITS, ALIGNED, 1, 1, 4));
     else if (tiles(1, 2) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 1, 2, 4>, 1, 2, tile_lds_bytes(BITS, ALIGNED, 1, 2, 4));
