@@ -502,8 +502,6 @@ constexpr int kGemmThreads = kGemmWaves * 64;
 constexpr int kGemmPitch = kProjGroup + 8;                           // halves per token row of the x tile in LDS
 constexpr int kGemmParamGroups = 64;                                 // groups whose scales and biases sit in LDS at a time
 constexpr int gemm_tile_halves(int tokens) { return tokens * kGemmPitch; }
-constexpr int kGemmOutPitch = kGemmRows + 8;                         // halves per token of the output tile in LDS
-static_assert(kGemmTokens * kGemmOutPitch <= 2 * gemm_tile_halves(kGemmTokens), "the output tile takes the x tiles' space");
 // KS = parts the columns are split into inside a workgroup (1 or 2): KS x 4 wavefronts, part p's four take the
 // groups [p x part_groups, (p + 1) x part_groups) with x tiles and a block of scales and biases of their own, and
 // the parts' accumulators are added through LDS at the end, in a fixed order.  For chunks whose tiles number no
@@ -731,9 +729,10 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     }
     _Float16 *const out_tile = lds_store;
     constexpr int kOutPitch = kRows + 8;
+    static_assert(TOKENS * kOutPitch * (int)sizeof(_Float16) <= (RS ? gemm_rs_lds_bytes() : gemm_lds_bytes(KS, TOKENS)), "the output tile takes the store's space");
     if (part == 0 || RS) {
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int j = 0; j < 16; ++j)
                 out_tile[(32 * tt + 8 * (j / 4) + 4 * h + (j % 4)) * kOutPitch + param_at] = (_Float16)acc[tt][j];
