@@ -144,6 +144,30 @@ def test_tiles_of_every_form_at_their_edges(gpu_ctx, bits, m, n, tokens, offset)
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("groups", [2, 6, 14, 16, 18, 30, 34, 1, 15, 20])  # by pairs: two groups a wavefront, four with an even count; not by pairs
+@pytest.mark.parametrize("shift", [0, 1, 2])  # scales and biases 2 and 4 bytes off a multiple of 8
+def test_scales_and_biases_in_fours_pairs_and_one_by_one(gpu_ctx, bits, groups, shift):
+    import torch
+    from tinytitan_amd.engine import AffineProjection
+    rows, n, tokens = 39, 64 * groups, 21
+    packed, scales, biases = _weights(rows, n, bits, groups + bits)
+    x = np.random.default_rng(groups).uniform(-1.0, 1.0, (tokens, n)).astype(np.float16)
+
+    def shifted(values):  # (NaN bit patterns in front of the values)
+        raw = np.full(values.size + shift, 0x7fff, np.uint16)
+        raw[shift:] = values.reshape(-1)
+        return _dev(raw.view(np.int16))[shift:]
+
+    wd, xd, sd, bd = _dev(packed.reshape(-1)), _dev(x), shifted(scales), shifted(biases)
+    yd = torch.full((tokens, rows), float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    AffineProjection(gpu_ctx).encode(bits, wd, sd, bd, xd, yd, rows, n, tokens)
+    gpu_ctx.synchronize()
+    want = oracle.affine_projection(packed, scales, biases, x.astype(np.float32), bits)
+    _assert_parity(yd.cpu().numpy().astype(np.float32), want, _magnitude(packed, scales, biases, x, bits), f"bits={bits} groups={groups} shift={shift}")
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("tokens", [1, 5, 16, 40, 128, 300, 512])
 def test_infinities_and_levels_of_zero(gpu_ctx, bits, tokens):
     # scale * sum(level * x) + bias * sum(x) as written: an infinite x leaves an infinity where its level is not zero and the

@@ -197,7 +197,15 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
         w_src[nr] = a.weights + (size_t)row * row_bytes;
         p_at[nr] = (size_t)row * groups;
     }
-    const bool params_vector = groups % 4 == 0 && per_wave % 4 == 0 && (uintptr_t)a.scales % 8 == 0 && (uintptr_t)a.biases % 8 == 0;
+    // A row's next four scales (or biases) in one load where every such run is aligned, in pairs where those are (1024
+    // columns, whose 16 groups are two a wavefront: 300 tokens over 8 bits 22.3 -> 15.4 us, over 4 bits 16.4 -> 10.8).
+    const bool by_fours = groups % 4 == 0 && per_wave % 4 == 0 && (uintptr_t)a.scales % 8 == 0 && (uintptr_t)a.biases % 8 == 0;
+    const bool by_twos = groups % 2 == 0 && per_wave % 2 == 0 && (uintptr_t)a.scales % 4 == 0 && (uintptr_t)a.biases % 4 == 0;
+    auto next_params = [&](unsigned (&dst)[2], const uint16_t *row, int g0) {
+        if (by_fours || !by_twos) return load_params<4>(dst, row, g0, groups, by_fours);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dst[i] = *reinterpret_cast<const unsigned *>(row + min(g0 + 2 * i, groups - 2));
+    };
     const f4v zero = {0.f, 0.f, 0.f, 0.f};
     f4v acc[MT][NR];
 #pragma unroll
@@ -246,8 +254,8 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
                     }
                 }
                 if (sub == 0) {
-                    load_params<4>(scales[nr], a.scales + p_at[nr], g0, groups, params_vector);
-                    load_params<4>(biases[nr], a.biases + p_at[nr], g0, groups, params_vector);
+                    next_params(scales[nr], a.scales + p_at[nr], g0);
+                    next_params(biases[nr], a.biases + p_at[nr], g0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
