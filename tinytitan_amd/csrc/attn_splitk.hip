@@ -1247,7 +1247,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     const bool first_real = b < b_end;
     const unsigned first_bytes = first_real ? (unsigned)(a.ring_blocks ? b % a.ring_blocks : b) * BLK_BYTES : 0u;
     Voids<D, NT> first_void(first_real ? 0u : kVoidLoad);
-    if constexpr (KEEP == 1 || KEEP == 3) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
+    if constexpr (KEEP == 1 || (KEEP == 3 && BITS == 16)) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
     if constexpr (KEEP == 4) {
         if (run_end > 0) {
             int ids_first[5];
@@ -1375,7 +1375,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         const bool real = nb < b_end && next_kept;
         const unsigned next = real ? (unsigned)(a.ring_blocks ? nb % a.ring_blocks : nb) * BLK_BYTES : 0u;
         Voids<D, NT> vo(real ? 0u : kVoidLoad);
-        if constexpr (KEEP == 1 || KEEP == 3) vo = Voids<D, NT>(real ? 0u : kVoidLoad, next_keys, ln);
+        if constexpr (KEEP == 1 || (KEEP == 3 && BITS == 16)) vo = Voids<D, NT>(real ? 0u : kVoidLoad, next_keys, ln);
         if constexpr (BITS == 16 && NT == 32) {
             block_scores_refill<AUX, D>(sc, kt, qf, rk, next, ln, vo);
             block_softmax_pv_refill<AUX, D>(st, sc, vt, ln, b << 5, lo, lim, a.scale_log2e, rv, next, vo, kept, row_keep, row_bits);

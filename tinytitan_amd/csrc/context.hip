@@ -115,8 +115,8 @@ __global__ __launch_bounds__(256) void keep_rows_from_indices_kernel(uint8_t *ro
 // them entry by entry, sources/TinyTitanCore/Metal/Prefill/prefill.metal:1069-1117) turned into what a tile of `tt`
 // tokens walks here: the ascending list of the 32-key blocks that hold a listed key some token of the tile can see
 // (key < min(kv_valid, start + row + 1), the reference's test of each entry), where every key range of `split_blocks`
-// blocks starts in that list, per entry the keys of the block that any token keeps, and per entry and token the
-// listed keys, as 32 bits each.  One workgroup per
+// blocks starts in that list, per entry the keys of the block that any token keeps (`any_keys`), and per entry and token
+// the listed keys, as 32 bits each.  One workgroup per
 // token tile; its work is the tile's list entries plus one pass over a bitmap of the context's blocks in LDS (a bit
 // per block: 4 KiB per million keys) -- nothing of the order rows x context is written or read.  Entries may come in
 // any order and repeat: a bit is set once.
@@ -130,7 +130,7 @@ template <bool GROUPS>
 __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t *indices, unsigned index_stride, const uint32_t *counts,
                                                                  int start, int q_len, int kv_valid, int tt, int split_blocks,
                                                                  int n_splits, int cap, int chunk_entries, int *ranges, int *blocks,
-                                                                 unsigned *bits) {
+                                                                 unsigned *bits, bool any_keys) {
     constexpr int T = kPlanThreads, kShift = GROUPS ? 2 : 5;  // keys of a unit: 1 << kShift
     extern __shared__ unsigned plan_lds[];
     const int tile = blockIdx.x, tid = threadIdx.x;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
         });
         __syncthreads();
         for (int i = tid; i < here * tt; i += T) my_bits[(size_t)first * tt + i] = chunk[i];
-        if constexpr (GROUPS) continue;
+        if (GROUPS || !any_keys) continue;
         for (int i = tid; i < here; i += T) {
             unsigned any = 0u;
             for (int r = 0; r < tt; ++r) any |= chunk[i * tt + r];
@@ -548,7 +548,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             hipLaunchKernelGGL(kernel, dim3((unsigned)plan.tok_tiles), dim3(kPlanThreads),
                                (size_t)(2 * words + kPlanThreads + 1 + chunk_entries * plan.tt) * sizeof(unsigned), ctx->stream, lists->indices,
                                (unsigned)lists->stride, lists->counts, starts[base], rows, totals[base], plan.tt, plan.split_len / 32,
-                               plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits);
+                               plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits, kv_bits == 16);
             e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(ctx, e, "keep_plan_kernel launch");
             a.plan_groups = groups;
