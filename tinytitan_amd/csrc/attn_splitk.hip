@@ -216,7 +216,7 @@ constexpr unsigned kVoidLoad = 0x7ff00000u;
 // fetch those keys' 16-byte pieces instead of all 32, and a step of V whose sixteen keys are all dropped is not
 // fetched; a dropped key's elements read as zeros, under a score that the selection masks and a probability of 0.
 // (128 rows with a selection each behind 131k keys 189 -> 162 us, a decode step's row there 18.1 -> 16.4; loads of V lines
-// that hold one kept group remain.)
+// that hold one kept group remain.  Where a chunk's lists fetch whole blocks: lists_fetch_by_key.)
 template <int D, int NT>
 struct Voids {
     unsigned all;   // the block as a whole (parameters of quantised pages)
@@ -1182,6 +1182,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     const int *plan_blocks_tile = nullptr;
     const unsigned *plan_bits_tile = nullptr;
     int e_at = 0, e_hi = 0, walked = 0;
+    constexpr bool BY_KEY = KEEP == 1 || (KEEP == 3 && lists_fetch_by_key(D, BITS));  // see Voids
     typedef int i2 __attribute__((ext_vector_type(2)));
     i2 after_entry = {0, 0};  // block, keys of it that any token keeps
     unsigned nxt_keys = ~0u;
@@ -1189,7 +1190,10 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     const int bits_col = valid ? t_local : 0;
     auto plan_entry = [&](int k) {  // the wavefront's k-th entry (a load; every lane the same words)
         const int e = e_at + k * WAVES;
-        const i2 got = *reinterpret_cast<const i2 *>(plan_blocks_tile + 2 * (size_t)(e < e_hi ? e : 0));
+        const int *at = plan_blocks_tile + 2 * (size_t)(e < e_hi ? e : 0);
+        i2 got = {0, 0};
+        if constexpr (BY_KEY) got = *reinterpret_cast<const i2 *>(at);
+        else got[0] = at[0];  // (the register of a second word that nothing uses is given to something else, which then waits for the load)
         const i2 none = {b_end, 0};
         return e < e_hi ? got : none;
     };
@@ -1247,7 +1251,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     const bool first_real = b < b_end;
     const unsigned first_bytes = first_real ? (unsigned)(a.ring_blocks ? b % a.ring_blocks : b) * BLK_BYTES : 0u;
     Voids<D, NT> first_void(first_real ? 0u : kVoidLoad);
-    if constexpr (KEEP == 1 || (KEEP == 3 && BITS == 16)) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
+    if constexpr (BY_KEY) first_void = Voids<D, NT>(first_real ? 0u : kVoidLoad, first_keys, ln);
     if constexpr (KEEP == 4) {
         if (run_end > 0) {
             int ids_first[5];
@@ -1375,7 +1379,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         const bool real = nb < b_end && next_kept;
         const unsigned next = real ? (unsigned)(a.ring_blocks ? nb % a.ring_blocks : nb) * BLK_BYTES : 0u;
         Voids<D, NT> vo(real ? 0u : kVoidLoad);
-        if constexpr (KEEP == 1 || (KEEP == 3 && BITS == 16)) vo = Voids<D, NT>(real ? 0u : kVoidLoad, next_keys, ln);
+        if constexpr (BY_KEY) vo = Voids<D, NT>(real ? 0u : kVoidLoad, next_keys, ln);
         if constexpr (BITS == 16 && NT == 32) {
             block_scores_refill<AUX, D>(sc, kt, qf, rk, next, ln, vo);
             block_softmax_pv_refill<AUX, D>(st, sc, vt, ln, b << 5, lo, lim, a.scale_log2e, rv, next, vo, kept, row_keep, row_bits);

@@ -548,7 +548,7 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             hipLaunchKernelGGL(kernel, dim3((unsigned)plan.tok_tiles), dim3(kPlanThreads),
                                (size_t)(2 * words + kPlanThreads + 1 + chunk_entries * plan.tt) * sizeof(unsigned), ctx->stream, lists->indices,
                                (unsigned)lists->stride, lists->counts, starts[base], rows, totals[base], plan.tt, plan.split_len / 32,
-                               plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits, kv_bits == 16);
+                               plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits, lists_fetch_by_key(D, kv_bits));
             e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(ctx, e, "keep_plan_kernel launch");
             a.plan_groups = groups;

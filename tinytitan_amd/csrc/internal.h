@@ -88,6 +88,12 @@ struct alignas(64) SplitKArgs {
     int plan_cap;                 // entries a tile's list has room for
 };
 
+// Whether a chunk's lists, walked block by block, fetch a touched block's kept keys only (Voids in attn_splitk.hip), or the
+// block whole: the offsets by key cost a block's turn the same whatever its bytes.  By key / whole: 16/2 heads of 256, 128 rows
+// behind 131k keys 162 / 189 us; 32/8 of 128, 512 rows behind 25,000 310 / 331, 200 behind 4,500 61.1 / 60.1; 16/4 of 64, 300
+// behind 25,000 88.5 / 85.2; 8 bits, 8/2 of 256, 489 rows behind 257,507 789 / 755.
+constexpr bool lists_fetch_by_key(int head_dim, int kv_bits) { return head_dim >= 128 && kv_bits == 16; }
+
 struct LaunchPlan {
     int nt;  // 16 or 32 query rows per tile
     int gh, tt, hsubs, tok_tiles, n_tiles;
