@@ -18,6 +18,7 @@
 // (sources/TinyTitanCore/Metal/Prefill/prefill.metal:1172-1313).
 #include <type_traits>
 
+#include "chunk_plan.h"
 #include "internal.h"
 #include "wave_ops.h"
 
@@ -1650,8 +1651,7 @@ int plan_launch(const tt_hip_ctx *ctx, int kind, int n_seq, int n_q_heads, int n
         p.gh = 1;
     } else {
         // GQA-packed rows: all q heads of a KV head (times the tile's tokens) share one pass over K/V.
-        p.gh = group;
-        while (p.gh > 32 || group % p.gh != 0) --p.gh;  // largest divisor of group that fits a tile
+        p.gh = packed_heads(group);
         p.nt = (rows * p.gh <= 16) ? 16 : 32;
         // Tiles of 16 rows although the rows would fill tiles of 32, while the launch reads little: the 32-row
         // kernel's fixed costs (one workgroup per CU, 32 rows x D floats per wavefront merged through LDS and left as

@@ -6,6 +6,13 @@
 
 namespace tt {
 
+// Query heads that the split-K kernel packs into a tile of at most 32 rows: the largest divisor of a KV head's group.
+inline int packed_heads(int group) {
+    int gh = group;
+    while (gh > 32 || group % gh != 0) --gh;
+    return gh;
+}
+
 // Key blocks of 32 that the chunk's tile of rows [32 t, 32 t + 32) walks: from the block of the first key its first row sees (a
 // window: the last `window` keys up to the row's own) to the block of its last row's own key.
 inline int chunk_tile_blocks(int start, int q_len, int kv_valid, int window, int t) {
@@ -102,10 +109,7 @@ inline KeyRanges plan_window_ranges(int n_cus, int D, int n_q_heads, int n_kv_he
 
 // The split-K kernel's tiles of 32 packed rows: key blocks per wavefront, dearer while a tile walks few of them.
 inline double estimate_splitk_chunk_us(int n_cus, int D, int n_q_heads, int n_kv_heads, int q_len, int first_blocks, int last_blocks) {
-    const int group = n_q_heads / n_kv_heads;
-    int gh = group;
-    while (gh > 32 || group % gh != 0) --gh;
-    const int tt = 32 / gh;
+    const int group = n_q_heads / n_kv_heads, gh = packed_heads(group), tt = 32 / gh;
     const double tiles = (double)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh), blocks = (first_blocks + last_blocks) / 2.0;
     const double block_us = D == 256 ? 1.6 * (1.0 + 18.0 / blocks) : D == 128 ? 0.87 * (1.0 + 11.0 / blocks) : 0.46 * (1.0 + 8.0 / blocks);
     return 5.0 + tiles * blocks / (4.0 * n_cus) * block_us;
@@ -113,10 +117,7 @@ inline double estimate_splitk_chunk_us(int n_cus, int D, int n_q_heads, int n_kv
 // Tiles of one length, as a window makes them, in the whole rounds that the planner's splits leave (from 64 blocks a tile
 // on; shorter walks start apart and even out).
 inline double splitk_rounds_us(int n_cus, int n_q_heads, int n_kv_heads, int q_len, int blocks, double even_us) {
-    const int group = n_q_heads / n_kv_heads;
-    int gh = group;
-    while (gh > 32 || group % gh != 0) --gh;
-    const int tt = 32 / gh;
+    const int group = n_q_heads / n_kv_heads, gh = packed_heads(group), tt = 32 / gh;
     const long long tiles = (long long)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh);
     if (blocks < 64 || tiles <= 0) return even_us;
     const long long splits = std::max<long long>(n_cus / tiles, 1), rounds = (tiles * splits + n_cus - 1) / n_cus;

@@ -1034,10 +1034,8 @@ int tt_hip_attn_prefill_keep_indices(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, 
     // The lists are served as they are: a launch turns them into each token tile's list of touched key blocks and
     // per-token key bits (keep_plan_kernel), which the attention kernel then walks -- work and memory of the order of
     // the selection.  Long chunks go in pieces of rows, so that the plan of one piece stays below 128 MiB.
-    const int group = n_q_heads / kv->n_kv_heads;
-    int gh = group;
-    while (gh > 32 || group % gh != 0) --gh;
-    const int tt = 32 / gh;  // tokens per tile of the 32-row tiles (the planner's own rule)
+    const int group = n_q_heads / kv->n_kv_heads, gh = packed_heads(group);
+    const int tt = 32 / gh;  // tokens per tile of the 32-row tiles
     const long long ctx_blocks = ((long long)kv_valid + 31) / 32, entries = (long long)tt * (long long)keep_index_stride;
     const long long cap = entries < ctx_blocks ? entries : ctx_blocks;
     const long long group_cap = (entries < 8 * ctx_blocks ? entries : 8 * ctx_blocks) + 8;  // (a plan of groups, run_attention)
