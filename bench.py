@@ -57,8 +57,8 @@ def indexer_bytes(context: int, tokens: int) -> int:
 # attn_splitk_c1_c3_c5_trace_and_traffic.md, attn_splitk_kv8_quantised.md, affine_proj_o1_o5_o4.md; "C2/8" is C2
 # over an 8-bit cache).  None: not measured
 # for that workload.
-MEASURED_TRAFFIC_BYTES = {"C1": 4477212, "C2": 69383103, "C3": 598966317, "C4": 113935667, "C5": 1114007952,
-                          "E4": 151546501, "C2/8": 37988966, "O1": 4868151, "O5": 7137478, "O4": 96536529}
+MEASURED_TRAFFIC_BYTES = {"C1": 4477212, "C2": 69383103, "C3": 592486288, "C4": 113935667, "C5": 1114007952,
+                          "E4": 151546501, "C2/8": 37988966, "O1": 4868151, "O5": 7021814, "O4": 96536529}
 
 
 def _load_engine():

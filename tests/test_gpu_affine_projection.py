@@ -116,7 +116,7 @@ def test_other_shapes_and_padded_strides(gpu_ctx, bits, m, n, tokens):
 
 def test_rows_are_independent_of_their_neighbours(gpu_ctx):
     # a token's row does not depend on where it sits in the batch: permuting x permutes y bit for bit, and a
-    # sub-batch gives the same bits as the full one (up to 9 tokens take a different kernel with another order
+    # sub-batch gives the same bits as the full one (up to 4 tokens take a different kernel with another order
     # of the fp32 sums: there the same row agrees to the rounding of that order)
     bits, rows, n, tokens = 4, 512, 1024, 70
     packed, scales, biases = _weights(rows, n, bits, 5)
