@@ -414,3 +414,32 @@ def test_row_maxima_that_keep_growing_rescale_the_accumulators(gpu_ctx, bits, D,
     want = oracle.decode(q[W - 1].astype(np.float32), kq.reshape(T, -1), vq.reshape(T, -1), H, KH, D, scale)
     _check(dec[0], want, f"{bits}-bit decode under rising scores")
     kv.close()
+
+
+@pytest.mark.parametrize("bits,D,H,KH,n,rows,keys", [
+    (8, 64, 16, 4, 16, 1, 4095), (8, 64, 16, 4, 16, 1, 4096),      # tiles of 16 rows, four workgroups a tile: eight from 1024 keys each
+    (4, 128, 16, 8, 8, 1, 5119), (4, 128, 16, 8, 8, 1, 5120),      # 16 rows of 128: from 1280
+    (4, 128, 32, 4, 4, 8, 12287), (4, 128, 32, 4, 4, 8, 12289),    # 32 of 128: from 1536
+    (4, 64, 8, 4, 64, 1, 4095), (4, 64, 8, 4, 64, 1, 4097)])       # one workgroup a tile, no combine: from 4096
+def test_equal_lengths_on_both_sides_of_two_rounds(gpu_ctx, bits, D, H, KH, n, rows, keys):
+    import torch
+    from tinytitan_amd.engine import Attention
+    r = np.random.default_rng(keys + n)
+    kv, start, scale = _cache(gpu_ctx, bits, KH, D, keys, slots=n), keys - rows, D ** -0.5
+    k, v = _rows(keys, KH, D, seed=keys, spread=False)
+    for s in range(n):  # (a sequence of its own each, out of the same rows)
+        _append(gpu_ctx, kv, 0, s, 0, np.roll(k, 7 * s, axis=0), np.roll(v, 7 * s, axis=0))
+    q = r.standard_normal((n * rows, H * D)).astype(np.float16)
+    qd = _dev(q)
+    out = torch.full(qd.shape, float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    Attention(gpu_ctx).encode_verify_rows(kv, 0, qd, out, H, [start] * n, rows, scale, list(range(n)))
+    gpu_ctx.synchronize()
+    got = out.float().cpu().numpy()
+    kv.close()
+    kq, vq = _dequantised(k, bits), _dequantised(v, bits)
+    for s in (0, n // 2, n - 1):
+        want = oracle.attention_batch(q[s * rows:(s + 1) * rows].astype(np.float32), np.roll(kq, 7 * s, axis=0).reshape(keys, -1),
+                                      np.roll(vq, 7 * s, axis=0).reshape(keys, -1), rows, start, H, KH, D, scale, threads=4)
+        _check(got[s * rows:(s + 1) * rows], want.reshape(rows, -1), f"sequence {s} of {n}, {keys} keys")
+    assert np.isfinite(got).all()

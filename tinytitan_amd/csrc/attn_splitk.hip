@@ -1697,9 +1697,14 @@ int plan_launch(const tt_hip_ctx *ctx, int kind, int n_seq, int n_q_heads, int n
         // for a CU and double the kernel's time.
         const long long pairs = (long long)n_seq * p.n_tiles;
         long long per_pair = ctx->n_cus / pairs;
-        // (two rounds, side by side on a CU, where a workgroup's loads are few bytes and its walk is long: 131k keys over 8
-        // bits with 16/4 heads of 64 23.4 -> 18.0 us, over 4 bits with 32/8 heads of 128 43.0 -> 35.6; with 16/2 of 256 27.4 -> 30.1)
-        if (head_dim * kv_bits <= 512 && pairs <= ctx->n_cus && max_keys >= 768 * per_pair) per_pair = 2 * ctx->n_cus / pairs;
+        // Two rounds, side by side on a CU, where a workgroup's loads are few bytes and its walk is long (131k keys over 8 bits
+        // with 16/4 heads of 64 23.4 -> 18.0 us, over 4 bits with 32/8 heads of 128 43.0 -> 35.6; with 16/2 of 256 27.4 -> 30.1).
+        // Twice the partial results have to be worth it, which is a walk the longer the more rows and dims they have (before the
+        // line / at it: 16 rows of 64, 920 keys a workgroup 12.8 -> 13.0 us, 1080 15.2 -> 13.0; 16 of 128 or 32 of 64, 860 keys
+        // 14.9 -> 15.8, 1300 19.0 -> 16.2; 32 of 128, 1400 keys 26.3 -> 28.3, 1730 39.2 -> 30.3), and where there was one
+        // workgroup a tile, and no combine, a longer one still (1613 keys 21.0 -> 27.0, 3416 25.9 -> 29.2, 8486 87 -> 61).
+        const long long walk = per_pair <= 1 ? 4096 : p.nt * head_dim <= 1024 ? 1024 : p.nt * head_dim <= 2048 ? 1280 : 1536;
+        if (head_dim * kv_bits <= 512 && pairs <= ctx->n_cus && max_keys >= walk * per_pair) per_pair = 2 * ctx->n_cus / pairs;
         if (per_pair < 1) per_pair = 1;
         split_len = (int)((max_keys + per_pair - 1) / per_pair);
         split_len = ((split_len + min_split - 1) / min_split) * min_split;
