@@ -67,6 +67,9 @@ def test_head_groups_the_chunk_kernel_does_not_take_and_few_rows(gpu_ctx, bits, 
     (24, 2, 256, 300, 5001, 3000, 0),     # a window cut into key ranges, its lower edge inside the first one's blocks
     (32, 8, 128, 291, 4100, 3001, 3520),  # ... over a ring: 4,100 % 3,520 + 291 rows do not wrap
     (16, 2, 256, 270, 1900, 4096, 0),     # a window that clips no row is none: the dense routes
+    (24, 2, 256, 256, 300, 33, 0),        # a short window: the split-K tiles all at work at once
+    (24, 2, 256, 257, 300, 33, 0),        # ... and two tiles more
+    (32, 8, 128, 512, 600, 128, 0), (32, 8, 128, 513, 600, 128, 0),
     (16, 2, 256, 1030, 40, 0, 0),         # no window: the causal triangle, the longest tile first
     (12, 1, 64, 2100, 3, 0, 0)])          # one KV head, 66 tiles of three head sets: a second round of workgroups
 def test_whole_chunks_in_single_tiles(gpu_ctx, H, KH, D, rows, start, window, ring):

@@ -107,18 +107,23 @@ inline KeyRanges plan_window_ranges(int n_cus, int D, int n_q_heads, int n_kv_he
     return plan_key_ranges(n_cus, D, n_q_heads, n_kv_heads, q_len, longest_tile_blocks(start, q_len, kv_valid, window));
 }
 
+// Tiles of 32 packed rows that the split-K kernel makes of a chunk, and how many of them run at once.
+inline long long splitk_tiles(int n_q_heads, int n_kv_heads, int q_len) {
+    const int group = n_q_heads / n_kv_heads, gh = packed_heads(group), tt = 32 / gh;
+    return (long long)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh);
+}
+inline long long splitk_tiles_at_once(int n_cus, int D) { return (long long)n_cus * (D == 256 ? 1 : D == 128 ? 2 : 3); }
+
 // The split-K kernel's tiles of 32 packed rows: key blocks per wavefront, dearer while a tile walks few of them.
 inline double estimate_splitk_chunk_us(int n_cus, int D, int n_q_heads, int n_kv_heads, int q_len, int first_blocks, int last_blocks) {
-    const int group = n_q_heads / n_kv_heads, gh = packed_heads(group), tt = 32 / gh;
-    const double tiles = (double)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh), blocks = (first_blocks + last_blocks) / 2.0;
+    const double tiles = (double)splitk_tiles(n_q_heads, n_kv_heads, q_len), blocks = (first_blocks + last_blocks) / 2.0;
     const double block_us = D == 256 ? 1.6 * (1.0 + 18.0 / blocks) : D == 128 ? 0.87 * (1.0 + 11.0 / blocks) : 0.46 * (1.0 + 8.0 / blocks);
     return 5.0 + tiles * blocks / (4.0 * n_cus) * block_us;
 }
 // Tiles of one length, as a window makes them, in the whole rounds that the planner's splits leave (from 64 blocks a tile
 // on; shorter walks start apart and even out).
 inline double splitk_rounds_us(int n_cus, int n_q_heads, int n_kv_heads, int q_len, int blocks, double even_us) {
-    const int group = n_q_heads / n_kv_heads, gh = packed_heads(group), tt = 32 / gh;
-    const long long tiles = (long long)((q_len + tt - 1) / tt) * n_kv_heads * (group / gh);
+    const long long tiles = splitk_tiles(n_q_heads, n_kv_heads, q_len);
     if (blocks < 64 || tiles <= 0) return even_us;
     const long long splits = std::max<long long>(n_cus / tiles, 1), rounds = (tiles * splits + n_cus - 1) / n_cus;
     return 5.0 + (even_us - 5.0) * ((double)rounds * n_cus / ((double)tiles * splits));

@@ -1170,7 +1170,11 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
                                      0, (long long)gate_stride, scale, out, 0, (long long)o_stride, r.n_splits, r.split_blocks, nullptr, window);
             if (whole.us < 0.75 * tiles_us) return whole_tiles(nullptr);
         }
-        if (serves && kv->bits == 16 && (filled || whole.us < splitk_us)) return whole_tiles(nullptr);
+        // The estimates do not hold where the split-K tiles are all at work at once, as a few hundred rows of a short window are: 64 / 8
+        // heads of 64, 226 rows behind 96 keys 7.0 us against 10.1, 32 / 8 of 128, 428 behind 128 12.9 / 14.6, 24 / 2 of 256, 247 behind
+        // 33 12.6 / 19.1; one more round the other way (279 rows there 22.5 / 19.1, 560 of 32 / 8 19.1 / 13.8).
+        const bool more_rounds = splitk_tiles(n_q_heads, kv->n_kv_heads, q_len) > splitk_tiles_at_once(ctx->n_cus, kv->head_dim);
+        if (serves && kv->bits == 16 && (filled || (more_rounds && whole.us < splitk_us))) return whole_tiles(nullptr);
         return run_attention(ctx, kv, 0, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride,
                              gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride, 1, 0, nullptr, window);
     }
