@@ -196,8 +196,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
     if (r >= a.per_kvh || kvh >= a.n_kv_heads) return;
     // (whole tiles one by one: the head sets' longest tiles first, and so on down)
     const bool longest_first = a.single_tiles && a.n_splits == 1;
-    const int hsub = longest_first ? r % a.hsubs : r / a.n_pairs;
-    const int pair = longest_first ? r / a.hsubs : r - hsub * a.n_pairs;
+    // (one division: each is a chain in front of the first load)
+    const int per = longest_first ? a.hsubs : a.n_pairs, quotient = r / per, rest = r - quotient * per;
+    const int hsub = longest_first ? rest : quotient;
+    const int pair = longest_first ? quotient : rest;
     const int head = kvh * a.group + hsub * 4 + w4;
     const _Float16 *kp = a.k_slot + (size_t)kvh * a.page_elems;
     const _Float16 *vp = a.v_slot + (size_t)kvh * a.page_elems;
