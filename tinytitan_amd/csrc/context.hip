@@ -241,7 +241,9 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
         if (GROUPS || !any_keys) continue;
         for (int i = tid; i < here; i += T) {
             unsigned any = 0u;
-            for (int r = 0; r < tt; ++r) any |= chunk[i * tt + r];
+            // (each from a place of its own on: all from the first, 32 tokens' words are one bank's, and 30 rows of 8/8 heads of 128
+            // behind 48,000 keys took 177 us instead of 166)
+            for (int r = 0, at = i % tt; r < tt; ++r, at = at + 1 < tt ? at + 1 : 0) any |= chunk[i * tt + at];
             my_blocks[2 * (first + i) + 1] = (int)any;
         }
     }
