@@ -275,7 +275,9 @@ def test_prefill_chunk_of_many_tiles_in_few_splits_merges_by_half_tiles(gpu_ctx,
 
 @pytest.mark.parametrize("bits,D,H,KH,start,rows", [(16, 256, 16, 2, 20000, 37), (8, 128, 8, 2, 3000, 70), (16, 64, 4, 4, 100, 9),
                                                     # a tile's tokens: 32, and 6 (the plan's walk over a block's rows begins anywhere)
-                                                    (16, 128, 8, 8, 2000, 70), (16, 128, 40, 8, 2000, 45)])
+                                                    (16, 128, 8, 8, 2000, 70), (16, 128, 40, 8, 2000, 45),
+                                                    # 264 tiles: only the listed keys are fetched
+                                                    (16, 128, 32, 8, 2500, 264)])
 def test_prefill_chunk_over_index_lists_equals_the_mask_form(gpu_ctx, bits, D, H, KH, start, rows):
     # The compacted form of a chunk's selection (keepIndices / keepIndexStride / keepCounts, prefill.metal:1069-1117):
     # per row a list of key ids -- here unsorted, with a repeat, with ids the row cannot see yet and one past the

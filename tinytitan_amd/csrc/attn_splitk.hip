@@ -958,6 +958,7 @@ __device__ __forceinline__ void block_softmax_pv(RowState<D, NT> &st, Scores<D, 
 // entry and token the kept keys as 32 bits -- the walk costs the selection, never the context.
 // KEEP = 4: the same, where few of a touched block's keys are listed (fp16 pages, tiles of 32): the plan lists groups of
 // four keys, and eight listed groups, wherever they lie, make a turn of the loop.
+// KEEP = 5: KEEP = 3 whose blocks' loads cover the listed keys only (lists_fetch_by_key).
 // The hot arguments and this workgroup's sequence entry, by three scalar loads issued together (the compiler
 // would fetch each field where it is first used: five or six dependent trips to the kernarg segment before
 // the first K/V load can go out, about 0.15 us each).
@@ -1183,7 +1184,8 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     const int *plan_blocks_tile = nullptr;
     const unsigned *plan_bits_tile = nullptr;
     int e_at = 0, e_hi = 0, walked = 0;
-    constexpr bool BY_KEY = KEEP == 1 || (KEEP == 3 && lists_fetch_by_key(D, BITS));  // see Voids
+    constexpr bool LISTS = KEEP == 3 || KEEP == 5;
+    constexpr bool BY_KEY = KEEP == 1 || KEEP == 5;  // see Voids
     typedef int i2 __attribute__((ext_vector_type(2)));
     i2 after_entry = {0, 0};  // block, keys of it that any token keeps
     unsigned nxt_keys = ~0u;
@@ -1203,7 +1205,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         const unsigned got = plan_bits_tile[(size_t)(e < e_hi ? e : 0) * a.tt + bits_col];
         return e < e_hi ? got : 0u;
     };
-    if constexpr (KEEP == 3) {
+    if constexpr (LISTS) {
         const int *ranges = args.plan_ranges + (size_t)ti.tok_tile * (a.n_splits_max + 1) + split;
         e_at = __builtin_amdgcn_readfirstlane(ranges[0]) + wave;
         e_hi = __builtin_amdgcn_readfirstlane(ranges[1]);
@@ -1367,7 +1369,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
             row_keep = row_cur;
         }
         unsigned row_bits = ~0u;
-        if constexpr (KEEP == 3) {
+        if constexpr (LISTS) {
             nb = nxt;
             next_keys = nxt_keys;
             nxt = __builtin_amdgcn_readfirstlane(after_entry[0]);
@@ -1405,7 +1407,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
                 row_next[i] = row_after[i];
             }
         }
-        if constexpr (KEEP == 3) {
+        if constexpr (LISTS) {
             bits_cur = bits_next;
             bits_next = bits_after;
         }
@@ -1788,8 +1790,10 @@ static hipError_t configure_tile() {
     TT_CFG(16, 0) TT_CFG(8, 0) TT_CFG(4, 0)
     TT_CFG(16, 1) TT_CFG(8, 1) TT_CFG(4, 1)
     TT_CFG(16, 2) TT_CFG(8, 2) TT_CFG(4, 2)
-    TT_CFG(16, 3) TT_CFG(8, 3) TT_CFG(4, 3)
+    if constexpr (D != 256) { TT_CFG(16, 3) }  // (heads of 256: by key always)
+    TT_CFG(8, 3) TT_CFG(4, 3)
     if constexpr (NT == 32) { TT_CFG(16, 4) }
+    if constexpr (lists_fetch_by_key(D, 16)) { TT_CFG(16, 5) }
 #undef TT_CFG
     return e;
 }
@@ -1826,8 +1830,13 @@ int launch_splitk(tt_hip_ctx *ctx, const LaunchPlan &plan, int head_dim, int n_s
         if constexpr (NN == 32) {                                                                    \
             if (args.plan_blocks && args.plan_groups) return launch_one<DD, NN, 4, 16, 4>(ctx, plan, n_seq, args); \
         }                                                                                            \
+        if constexpr (lists_fetch_by_key(DD, 16)) {                                                  \
+            if (args.plan_blocks && args.plan_by_key) return launch_one<DD, NN, 4, 16, 5>(ctx, plan, n_seq, args); \
+        }                                                                                            \
         if (args.plan_blocks) {                                                                      \
-            if (kv_bits == 16) return launch_one<DD, NN, 4, 16, 3>(ctx, plan, n_seq, args);          \
+            if constexpr (DD != 256) {                                                               \
+                if (kv_bits == 16) return launch_one<DD, NN, 4, 16, 3>(ctx, plan, n_seq, args);      \
+            }                                                                                        \
             if (kv_bits == 8) return launch_one<DD, NN, 4, 8, 3>(ctx, plan, n_seq, args);            \
             if (kv_bits == 4) return launch_one<DD, NN, 4, 4, 3>(ctx, plan, n_seq, args);            \
         }                                                                                            \

@@ -546,14 +546,17 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             if (chunk_words > 8192) chunk_words = 8192;
             const int chunk_entries = chunk_words / plan.tt;
             if (chunk_entries < 1) return TT_HIP_ERR_CAPACITY;
+            const bool by_key = !groups && launch_fetches_by_key(D, kv_bits, plan.n_tiles, (long long)plan.tt * (long long)lists->stride,
+                                                                 totals[base], ctx->n_cus);
             const auto kernel = groups ? keep_plan_kernel<true> : keep_plan_kernel<false>;
             hipLaunchKernelGGL(kernel, dim3((unsigned)plan.tok_tiles), dim3(kPlanThreads),
                                (size_t)(2 * words + kPlanThreads + 1 + chunk_entries * plan.tt) * sizeof(unsigned), ctx->stream, lists->indices,
                                (unsigned)lists->stride, lists->counts, starts[base], rows, totals[base], plan.tt, plan.split_len / 32,
-                               plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits, lists_fetch_by_key(D, kv_bits));
+                               plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits, by_key);
             e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(ctx, e, "keep_plan_kernel launch");
             a.plan_groups = groups;
+            a.plan_by_key = by_key;
             a.plan_ranges = ranges;
             a.plan_blocks = blocks;
             a.plan_bits = bits;

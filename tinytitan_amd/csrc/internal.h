@@ -83,16 +83,24 @@ struct alignas(64) SplitKArgs {
     const int *plan_ranges;       // [token tile][n_splits_max + 1]: where each split's entries start in the tile's list
     const int *plan_blocks;       // [token tile][plan_cap][2]: the key blocks the tile's tokens keep a key of, ascending, and those keys (bits)
     const unsigned *plan_bits;    // [token tile][plan_cap][tt]: per entry and token, bit i = key 32 block + i is kept
+    int plan_by_key;              // plan_blocks' second words are there, and the launch fetches those keys only
     int plan_groups;              // the plan lists groups of four keys: plan_blocks [token tile][plan_cap] group ids, plan_bits
                                   // [token tile][plan_cap / 8][tt], four bits a list position
     int plan_cap;                 // entries a tile's list has room for
 };
 
-// Whether a chunk's lists, walked block by block, fetch a touched block's kept keys only (Voids in attn_splitk.hip), or the
-// block whole: the offsets by key cost a block's turn the same whatever its bytes.  By key / whole: 16/2 heads of 256, 128 rows
-// behind 131k keys 162 / 189 us; 32/8 of 128, 512 rows behind 25,000 310 / 331, 200 behind 4,500 61.1 / 60.1; 16/4 of 64, 300
-// behind 25,000 88.5 / 85.2; 8 bits, 8/2 of 256, 489 rows behind 257,507 789 / 755.
+// Whether a chunk's lists, walked block by block, may fetch a touched block's kept keys only (Voids in attn_splitk.hip), or
+// always the block whole: the offsets by key cost a block's turn the same whatever its bytes.  By key / whole: 16/4 of 64, 300
+// rows behind 25,000 88.5 / 85.2 us; 8 bits, 8/2 of 256, 489 rows behind 257,507 789 / 755.
 constexpr bool lists_fetch_by_key(int head_dim, int kv_bits) { return head_dim >= 128 && kv_bits == 16; }
+// ... and whether this launch does.  Heads of 256: 16/2, 128 rows behind 131k keys 162 / 189 us.  Heads of 128 where the fetches
+// are what the launch waits for -- tiles for most of the chip -- and a tile's lists leave out enough keys, as they do with
+// no more entries than there are keys: 32/8 heads, 200 rows behind 24,168 146 / 151, 500 behind 18,596 244 / 252, behind 101k
+// 1035 / 1784; else the offsets are in the way: 128 rows behind 24,168 103.4 / 100.6, 500 behind 4,508 91.5 / 89.6, 8/8 heads
+// (32 tokens' lists a tile), 500 rows behind 48,001 344 / 329.
+inline bool launch_fetches_by_key(int head_dim, int kv_bits, long long n_tiles, long long entries, int keys, int n_cus) {
+    return lists_fetch_by_key(head_dim, kv_bits) && (head_dim == 256 || (4 * n_tiles >= 3ll * n_cus && entries < keys));
+}
 
 struct LaunchPlan {
     int nt;  // 16 or 32 query rows per tile
