@@ -814,6 +814,7 @@ def test_kernel_variant_switches_are_explicit_calls_and_change_no_result():
     (16, 256, 16, 2, [3000, 11, 7001], 8, 0),                                     # ... and two
     (16, 256, 16, 2, [300 + 450 * i for i in range(9)], 3, 0), (8, 256, 24, 2, [5000, 301, 40, 7777, 2100], 5, 0),
     (16, 128, 8, 4, [9000, 50, 2500, 1301], 1, 1000), (16, 64, 64, 32, [100 + 37 * i for i in range(40)], 1, 0),  # mostly last splits
+    (8, 64, 16, 4, [81, 439, 483, 91, 432], 1, 0), (16, 256, 24, 2, [600, 301], 5, 0),  # a CU for every workgroup, idle ones included
 ])
 def test_sequences_of_unlike_lengths_equal_their_own_calls(gpu_ctx, bits, D, H, KH, lengths, rows, window):
     # A batch of unlike lengths has its split length counted out and its splits one behind the other in the grid; a sequence

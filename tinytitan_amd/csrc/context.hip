@@ -470,7 +470,10 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         // every sequence to XCD i mod 8).
         // A KV head's token tiles read the same keys: rounded up to a multiple of eight, their workgroups of one split meet on
         // one XCD (20 sequences x 3 verify rows in tiles of 16, 300 .. 9,000 keys: 45.2 -> 21.0 us; 8 rows 59.2 -> 26.7).
-        plan.packed_splits = ragged ? (int)total_splits : 0;
+        // Not where the workgroups of one token tile find a CU each, the idle ones included: finding the sequence is a load more
+        // in front of the first key (5 decode rows of 16/4 heads of 64 behind 81 .. 491 keys over 8 bits 6.54 us, packed 6.78; 24 rows
+        // of 16/2 of 256 behind 336 .. 433 10.39 / 11.00; two tiles, 3 rows x 2 sequences of 24/2 of 256, 11.94 against 11.32).
+        plan.packed_splits = ragged && (plan.workgroups > ctx->n_cus || plan.tok_tiles > 1) ? (int)total_splits : 0;
         if (plan.packed_splits > 0 && plan.tok_tiles > 1) plan.packed_splits = (plan.packed_splits + 7) & ~7;
         if (plan.n_splits_max > 1) {
             const size_t part_rows = total_splits * plan.n_tiles * plan.nt;
