@@ -527,10 +527,12 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         // is worth it from two blocks a wavefront on (2,051 of 40,001 keys, 16/2 heads: 14.9 -> 13.5 us, of 70,001 17.7 -> 14.0, of
         // 131,070 22.3 -> 14.6, of 262,000 30.8 -> 14.9; with one block, at 8,000 keys, 10.3 against 10.7 the other way), over
         // narrower heads and quantised pages, whose blocks are fewer bytes, from about six (block by block / up front: 16/4 of
-        // 64 behind 8,428 keys 7.76 / 8.13, 40/8 of 128 over 8 bits behind 20,002, five blocks, 13.4 / 13.9, behind 25,003, seven, 15.6 / 14.6).
+        // 64 behind 8,428 keys 7.76 / 8.13, 40/8 of 128 over 8 bits behind 20,002, five blocks, 13.5 / 13.8, behind 25,003, seven, 15.9 / 14.9).
+        // From 50,000 keys on, of which a selection of two thousand in groups of four touches about one block in four, from four (24/2
+        // of 256 over 4 bits behind 55,000 18.6 / 17.4, 16/4 of 64 over 8 bits behind 72,327, five blocks, 14.1 / 12.8).
         // Per-query rows, whose walk reads every row's bytes first: from about eight.  (Those are always word-aligned: the
         // entry point requires it; a single sequence's mask has no stride to mind.)
-        const int listed_blocks = keep_row_stride > 0 ? 8 : D == 256 && kv_bits == 16 ? 2 : 6;
+        const int listed_blocks = keep_row_stride > 0 ? 8 : D == 256 && kv_bits == 16 ? 2 : max_keys >= 50000 ? 4 : 6;
         h.keep_words = a.keep && (uintptr_t)a.keep % 4 == 0 && (n == 1 || keep_seq_stride % 4 == 0) &&
                        plan.split_len >= listed_blocks * plan.waves * 32;
         for (int i = 0; i < n; ++i) {
