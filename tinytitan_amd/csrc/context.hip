@@ -377,10 +377,10 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
         // over 8 bits 291 -> 224, 180 rows behind 100k (90 tiles, 2 -> 5) 182 -> 163; 24/2 heads, 361 rows behind 13k (362 tiles, 1 -> 2)
         // 293 -> 253, 300 behind 40k (1 -> 3) 511 -> 375; 32/8 of 128, 300 behind 30k (304 tiles, 1 -> 3) 341 -> 245; 16/4 of 64, 300 behind
         // 20k (152 tiles, 1 -> 5) 150 -> 77.  Left alone where it would lose: 400 rows behind 8k keys (200 tiles) 117 against 131 and more;
-        // and where there are more tiles than CUs and a tile walks less than 8192 keys of 64 dims: a CU has several of those at work at
-        // once, so that rounds are not waited for (64/8 of 64, 640 tiles: 319 rows behind 4,508 keys 72.9 us -> 79.8 in two
-        // splits, behind 6,064 88.9 -> 92.5, behind 9,001 119.4 -> 118.0).
-        const bool several_at_work = plan.n_tiles > ctx->n_cus && (long long)max_keys * D < 8192 * 64;
+        // and where there are more than two tiles a CU and a tile walks less than 8192 keys of 64 dims: a CU has several of those at
+        // work at once, so that rounds are not waited for (64/8 of 64, 640 tiles: 319 rows behind 4,508 keys 72.9 us -> 79.8 in
+        // two splits, behind 6,064 88.9 -> 92.5, behind 9,001 119.4 -> 118.0; 320 tiles: 158 rows behind 5,324 66.3 -> 59.5).
+        const bool several_at_work = plan.n_tiles > 2 * ctx->n_cus && (long long)max_keys * D < 8192 * 64;
         if (lists && plan.nt == 32 && ctx->split_override <= 0 && plan.n_splits_max >= 1 && max_keys > 384 && !several_at_work) {
             auto rounds = [&](long long splits) { return (plan.n_tiles * splits + ctx->n_cus - 1) / ctx->n_cus; };
             auto length = [&](int splits) { return ((max_keys + splits - 1) / splits + 127) / 128 * 128; };
