@@ -796,8 +796,11 @@ def test_a_block_s_loads_cover_exactly_the_kept_keys(gpu_ctx, bits, D, H, KH):
     _append(gpu_ctx, kv, 0, 0, 0, k, v)
     ks, vs = (k, v) if bits == 16 else (_dequantised(k, bits), _dequantised(v, bits))
     scale = D ** -0.5
-    got = _decode_keep(gpu_ctx, kv, q[:1].reshape(1, 1, H, D), [T], keep1, H, scale)
-    _check(got.reshape(H, D), _oracle_kept(q[0].reshape(H, D), ks, vs, keep1, H, KH, D, scale).reshape(H, D), f"decode D={D} {H}/{KH} bits {bits}")
+    for split_tokens in (0, 1024):  # a wavefront's blocks tested one by one, and (eight of them) found up front
+        gpu_ctx.set_split_tokens(split_tokens)
+        got = _decode_keep(gpu_ctx, kv, q[:1].reshape(1, 1, H, D), [T], keep1, H, scale)
+        gpu_ctx.set_split_tokens(0)
+        _check(got.reshape(H, D), _oracle_kept(q[0].reshape(H, D), ks, vs, keep1, H, KH, D, scale).reshape(H, D), f"decode D={D} {H}/{KH} bits {bits} splits {split_tokens}")
     stride = int(keep_rows.sum(axis=1).max())
     lists, counts = np.zeros((rows, stride), np.int32), keep_rows.sum(axis=1).astype(np.int32)
     for t in range(rows):
@@ -864,7 +867,7 @@ def test_lists_walked_by_groups_of_keys_equal_the_mask_form(gpu_ctx, D, H, KH, T
 
 
 @pytest.mark.parametrize("T", [8193, 20000, 40001, 70002])
-@pytest.mark.parametrize("bits,D,H,KH", [(16, 256, 16, 2), (8, 128, 16, 4), (4, 64, 24, 2)])
+@pytest.mark.parametrize("bits,D,H,KH", [(16, 256, 16, 2), (8, 128, 16, 4), (4, 64, 24, 2), (8, 256, 16, 2)])
 def test_decode_reads_from_the_first_touched_block_on(gpu_ctx, bits, D, H, KH, T):
     # One mask, any length: most wavefronts have no touched block, or only a late one, and bytes other than 1 keep a key too.
     r = np.random.default_rng(T + D)
