@@ -188,3 +188,14 @@ def test_v_layout_matches_the_score_register_order(lib):
         keys = [first + i for i in range(4)] + [first + 8 + i for i in range(4)]
         offs = [lib.tt_hip_kv_v_offset(D, key, 9) for key in keys]
         assert offs == [(9 * 4 + g4) * 8 + j for j in range(8)]
+
+
+def test_v_layout_of_wide_heads_keeps_a_chunk_of_sixteen_dims_together(lib):
+    # Heads of 256: [d / 16][chunk][d % 16][8 keys], a chunk's keys in the score registers' order as above.
+    D = 256
+    for d in (0, 7, 8, 15, 16, 100, 255):
+        for t in range(2):
+            for g in range(2):
+                keys = [8 * ((8 * t + j) // 4) + 4 * g + (8 * t + j) % 4 for j in range(8)]
+                offs = [lib.tt_hip_kv_v_offset(D, 64 + key, d) for key in keys]
+                assert offs == [2 * 32 * D + ((d // 16 * 4 + 2 * t + g) * 16 + d % 16) * 8 + j for j in range(8)]

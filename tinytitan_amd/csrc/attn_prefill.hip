@@ -210,7 +210,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
     // the same number of copies in flight and one constant vmcnt tracks them.
     const unsigned smem_base = (unsigned)(size_t)(lds_ptr_t)smem;
     const unsigned k_lane_offset = (unsigned)lane * 16u;
-    const unsigned v_lane_offset = (unsigned)((li * 4 + g) * 16);  // this lane's 16 bytes inside a V chunk gather
+    const unsigned v_lane_offset = (unsigned)v_piece(D, li, g) * 2u;  // this lane's 16 bytes inside a V chunk gather
     int jb = 0;  // first key block of this workgroup's range in the current tile
     // Block b of the tile in hand lives in slot (b + slot_off) % kBuffers.  When a second tile follows (carry_nb > 0:
     // it has that many blocks, from block 0), the copies past the end of the first fetch ITS first blocks -- K 0..3 and
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
 #pragma unroll
     for (int c = 0; c < CPW; ++c) {
         const int chunk = w4 * CPW + c, mt = chunk >> 1, t = chunk & 1;
-        v_src_off[c] = (unsigned)((32 * mt * 4 + 2 * t) * 16);
+        v_src_off[c] = (unsigned)v_piece(D, 32 * mt, 2 * t) * 2u;
     }
     auto step_copies = [&](int i, int nb) {  // of step i; nb blocks in the range
         StepCopies sc;

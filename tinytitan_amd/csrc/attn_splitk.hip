@@ -166,6 +166,23 @@ struct VTile<D, 16> {
     h8 f[D / 16];
 };
 
+// The dims of a 32-row tile's V operands over fp16 pages of heads of 256.  A 128-byte line there holds eight dims of a chunk; two
+// operand tiles in a row share the lines of the same 64 dims, the first one's rows the lower four dims of each line, the
+// second one's the upper four.  So the first of their loads asks for all of those lines -- as it does over narrower heads' [d][chunk],
+// whose lines hold every chunk -- and the second finds them on their way: with one wavefront a SIMD more of them are under way
+// (8 sequences x 4 rows behind 64k keys 181.2 -> 175.2 us).  Tiles of 16 rows, two wavefronts a SIMD, read their contiguous
+// 1 KiB a load (in pairs 32 sequences of 511 .. 16,383 keys 61.3 -> 67.4 us).
+// Row 4 q + i of operand tile mt is dim v_tile_dim(mt) + v_row_dim(4 q + i): four consecutive dims for four consecutive i.
+constexpr bool paired_v_tiles(int head_dim, int nt) { return head_dim == 256 && nt == 32; }
+template <int D, int NT>
+__device__ __forceinline__ constexpr int v_tile_dim(int mt, bool paired = paired_v_tiles(D, NT)) {
+    return paired ? 2 * NT * (mt >> 1) + 4 * (mt & 1) : NT * mt;
+}
+template <int D, int NT>
+__device__ __forceinline__ constexpr int v_row_dim(int row, bool paired = paired_v_tiles(D, NT)) {
+    return paired ? 8 * (row >> 2) + (row & 3) : row;
+}
+
 template <int D, int NT>
 struct Lane {
     static constexpr int LN = NT;
@@ -176,11 +193,11 @@ struct Lane {
         g = lane / LN;
         if constexpr (NT == 32) {
             koff = (g * 32 + li) * 8;
-            voff = (li * 4 + g) * 8;
+            voff = v_piece(D, v_row_dim<D, NT>(li), g);
         } else {
             const int ka = li < 8 ? li : li + 8;
             koff = (g * 32 + ka) * 8;
-            voff = (li * 4 + g) * 8;
+            voff = v_piece(D, v_row_dim<D, NT>(li), g);
         }
     }
 };
@@ -265,10 +282,10 @@ __device__ __forceinline__ void load_v(VTile<D, NT> &t, __amdgpu_buffer_rsrc_t r
         for (int mt = 0; mt < D / 32; ++mt)
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
-                t.f[mt][tt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[tt], block_bytes + mt * (32 * 4 * 16) + tt * 32);
+                t.f[mt][tt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[tt], block_bytes + 2 * v_piece(D, v_tile_dim<D, NT>(mt), 2 * tt));
     } else {
 #pragma unroll
-        for (int mt = 0; mt < D / 16; ++mt) t.f[mt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[0], block_bytes + mt * (16 * 4 * 16));
+        for (int mt = 0; mt < D / 16; ++mt) t.f[mt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[0], block_bytes + 2 * v_piece(D, 16 * mt, 0));
     }
 }
 
@@ -532,14 +549,16 @@ __device__ __forceinline__ void block_softmax_pv_refill(RowState<D, 32> &st, Sco
         for (int t = 0; t < 2; ++t) st.o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vt.f[mt][t], pr.pf[t], st.o[mt], 0, 0, 0);
         asm volatile("" : "+a"(st.o[mt]));
 #pragma unroll
-        for (int t = 0; t < 2; ++t) vt.f[mt][t] = buf_load_h8<AUX>(rv, lane_bytes[t], next_bytes + mt * (32 * 4 * 16) + t * 32);
+        for (int t = 0; t < 2; ++t) vt.f[mt][t] = buf_load_h8<AUX>(rv, lane_bytes[t], next_bytes + 2 * v_piece(D, v_tile_dim<D, 32>(mt), 2 * t));
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
 // Eight listed groups of four keys taken as one block (KEEP = 4): every lane has offsets of its own.  K: a lane's key is one
 // of its group's four, 64 contiguous bytes per 8 dims.  V: the eight keys of a lane's operand are two groups, half a
-// chunk (8 bytes) of each.  A group that is not there has kVoidLoad for an offset.
+// chunk (8 bytes) of each, over heads of 256 in 256 contiguous bytes per 16 dims.  (While those lay in all of the block's lines their
+// passage through the vector cache was the kernel: 128 rows of 16/2 heads with a selection each behind 131k keys, 64 requests
+// a load instead of 16, 114 -> 74.8 us.)  A group that is not there has kVoidLoad for an offset.
 struct GroupOffsets {
     unsigned k;
     unsigned v[2][2];  // [key step][half of the operand]
@@ -555,7 +574,7 @@ __device__ __forceinline__ GroupOffsets group_offsets(const int (&ids)[5], const
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int id = ids[1 + 2 * t + h], j = id & 7;  // keys 4 j .. 4 j + 3 of the block: half (j / 2) % 2 of chunk 2 (j / 4) + j % 2
-            o.v[t][h] = id < 0 ? kVoidLoad : block_at(id) + (unsigned)(ln.li * 64 + (2 * (j >> 2) + (j & 1)) * 16 + ((j >> 1) & 1) * 8);
+            o.v[t][h] = id < 0 ? kVoidLoad : block_at(id) + 2u * (unsigned)(v_piece(D, ln.li, 2 * (j >> 2) + (j & 1)) + ((j >> 1) & 1) * 4);
         }
     return o;
 }
@@ -576,7 +595,7 @@ __device__ __forceinline__ void load_v_groups(VTile<D, 32> &vt, __amdgpu_buffer_
 #pragma unroll
     for (int mt = 0; mt < D / 32; ++mt)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) vt.f[mt][t] = load_group_pair(rv, o.v[t], mt * (32 * 4 * 16));
+        for (int t = 0; t < 2; ++t) vt.f[mt][t] = load_group_pair(rv, o.v[t], 2 * v_piece(D, 32 * mt, 0));
 }
 // The two phases with the next groups' loads between their MFMAs, as in block_scores_refill / block_softmax_pv_refill.
 template <int D>
@@ -603,7 +622,7 @@ __device__ __forceinline__ void group_softmax_pv_refill(RowState<D, 32> &st, Sco
         for (int t = 0; t < 2; ++t) st.o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vt.f[mt][t], pr.pf[t], st.o[mt], 0, 0, 0);
         asm volatile("" : "+a"(st.o[mt]));
 #pragma unroll
-        for (int t = 0; t < 2; ++t) vt.f[mt][t] = load_group_pair(rv, next.v[t], mt * (32 * 4 * 16));
+        for (int t = 0; t < 2; ++t) vt.f[mt][t] = load_group_pair(rv, next.v[t], 2 * v_piece(D, 32 * mt, 0));
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -744,7 +763,7 @@ struct QuantOffsets {
     static constexpr unsigned K_PAIR = (NT == 32 ? 2u : 4u) * 32u * K_UNIT;  // bytes between step pairs
     static constexpr unsigned V_RUN = 8u * BITS / 4;                   // bytes of one (dim pair, chunk) run
     __device__ __forceinline__ static unsigned k_lane(const Lane<D, NT> &ln) { return (unsigned)ln.koff / 8u * K_UNIT; }
-    __device__ __forceinline__ static unsigned v_lane(const Lane<D, NT> &ln) { return (unsigned)ln.voff / 8u * V_RUN; }
+    __device__ __forceinline__ static unsigned v_lane(const Lane<D, NT> &ln) { return (unsigned)(ln.li * 4 + ln.g) * V_RUN; }
 };
 
 template <int AUX, int D, int NT, int BITS>
@@ -1001,6 +1020,7 @@ __device__ __forceinline__ void load_row_words(unsigned (&dst)[8], __amdgpu_buff
 template <int D, int NT, int WAVES, int BITS, int KEEP = 0, int STREAM = 0>
 __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void attn_splitk_kernel(const SplitKArgs args) {
     constexpr int AUX = STREAM ? kStreamed : 0;
+    constexpr bool PAIRED = paired_v_tiles(D, NT) && BITS == 16 && KEEP != 4;  // (groups of keys and quantised pages: dims as they come)
     extern __shared__ float lds[];
     constexpr int ROW = D + kLdsPad;  // staged O row stride in floats
     constexpr int REGION = NT * ROW + NT * 2;
@@ -1438,7 +1458,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
 #pragma unroll
             for (int vq = 0; vq < 4; ++vq) {
                 f4 x = {st.o[mt][4 * vq], st.o[mt][4 * vq + 1], st.o[mt][4 * vq + 2], st.o[mt][4 * vq + 3]};
-                *reinterpret_cast<f4 *>(region + li * ROW + 32 * mt + 8 * vq + 4 * g) = x;
+                *reinterpret_cast<f4 *>(region + li * ROW + v_tile_dim<D, NT>(mt, PAIRED) + v_row_dim<D, NT>(8 * vq + 4 * g, PAIRED)) = x;
             }
     } else {
 #pragma unroll

@@ -60,9 +60,9 @@ __global__ __launch_bounds__(256) void kv_read_kernel(const _Float16 *__restrict
 
 // Whole 32-token blocks: one workgroup per (block, kv head).  The 32 source rows are read
 // coalesced (16 bytes per thread along a row) into LDS, then written out in the swizzled order,
-// 16 bytes per thread and contiguous across the workgroup: K as [d / 8][key][8], V as
-// [d][chunk][8] with each chunk's eight keys gathered from LDS.  HBM sees each byte once, as
-// full lines, in both directions.
+// 16 bytes per thread: K as [d / 8][key][8], V as
+// [d][chunk][8] (see v_piece) with each chunk's eight keys gathered from LDS.  HBM sees each
+// byte once, as full lines, in both directions.
 constexpr int kAppendPad = 8;  // halves of padding per LDS row: rows 16 bytes off a bank-aligned stride
 
 __global__ __launch_bounds__(256) void kv_append_blocks_kernel(_Float16 *__restrict__ k_layer, _Float16 *__restrict__ v_layer,
@@ -91,12 +91,11 @@ __global__ __launch_bounds__(256) void kv_append_blocks_kernel(_Float16 *__restr
         // K piece p = (d / 8, key)
         const int d8 = p >> 5, key = p & 31;
         *reinterpret_cast<h8 *>(k_layer + dst0 + (size_t)p * 8) = *reinterpret_cast<const h8 *>(kt + key * row_halves + d8 * 8);
-        // V piece p = (d, chunk)
-        const int d = p >> 2, c = p & 3;
+        const int d = p >> 2, c = p & 3;  // V piece (d, chunk)
         h8 x;
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = vt[v_key_at(c, i) * row_halves + d];
-        *reinterpret_cast<h8 *>(v_layer + dst0 + (size_t)p * 8) = x;
+        *reinterpret_cast<h8 *>(v_layer + dst0 + v_piece(head_dim, d, c)) = x;
     }
 }
 
@@ -164,7 +163,7 @@ __global__ __launch_bounds__(256) void kv_read_blocks_kernel(const _Float16 *__r
         const int d8 = p >> 5, key = p & 31;  // K piece (d / 8, key)
         *reinterpret_cast<h8 *>(kt + key * row_halves + d8 * 8) = *reinterpret_cast<const h8 *>(k_layer + src0 + (size_t)p * 8);
         const int d = p >> 2, c = p & 3;  // V piece (d, chunk)
-        const h8 x = *reinterpret_cast<const h8 *>(v_layer + src0 + (size_t)p * 8);
+        const h8 x = *reinterpret_cast<const h8 *>(v_layer + src0 + v_piece(head_dim, d, c));
 #pragma unroll
         for (int i = 0; i < 8; ++i) vt[v_key_at(c, i) * row_halves + d] = x[i];
     }

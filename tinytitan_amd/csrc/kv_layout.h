@@ -10,11 +10,16 @@
 //       g = l / 32) holds d = 16 s + 8 g + j  ->  1 KiB contiguous per step.
 //       v_mfma_f32_16x16x32_f16 reads the same block as 128-byte runs.
 //
-//   V block  [d 0..D-1][chunk 0..3][8 halves]
+//   V block  [d 0..D-1][chunk 0..3][8 halves]; at D = 256 [d / 16][chunk 0..3][d % 16][8 halves]
 //       chunk c = 2 t + g holds keys {16 t + 4 g + (0..3), 16 t + 8 + 4 g + (0..3)}:
 //       exactly the keys whose probabilities one lane owns after the S^T MFMA
 //       (C layout: lane (n, g), register v -> key 8 (v / 4) + 4 g + v % 4), so
 //       P needs no cross-lane movement between the two contractions.
+//       By chunk inside 16 dims, the keys of a selection lie together: four kept keys are halves of
+//       the 16-byte pieces of one chunk, 4 KiB of whole lines instead of a part of every line of the
+//       block's 16 KiB, and a 16-dim operand of all 32 keys is still 1 KiB in one piece.  (By chunk
+//       over all 256 dims a dense read's four runs lie 4 KiB apart, on the same channel of the L2:
+//       decode behind 32k keys 102.5 -> 104.9 us for four layers, 8 x 4 rows behind 64k 175 -> 179.5.)
 //
 // Quantised pages (8 or 4 bits per value, one fp16 scale and bias per token and group of 64
 // consecutive dims -- the reference's row format, sources/TinyTitan/Runtime/KVCache/
@@ -58,11 +63,17 @@ TT_HD int v_index_of_key(int key) { return 4 * ((key >> 3) & 1) + (key & 3); }
 // Inverse: the key stored at (chunk, index).
 TT_HD int v_key_at(int chunk, int index) { return 16 * (chunk >> 1) + 8 * (index >> 2) + 4 * (chunk & 1) + (index & 3); }
 
+// Offset in halves of a V block's piece (d, chunk): eight keys of one dim.  Sixteen dims further on it is 512 more.
+TT_HD constexpr int v_piece(int head_dim, int d, int chunk) {
+    return head_dim == 256 ? ((d >> 4) * 4 + chunk) * 128 + (d & 15) * 8 : (d * 4 + chunk) * 8;
+}
+
 // Offset in halves of V element (position, d) within its page.
 TT_HD size_t v_offset(int head_dim, int position, int d) {
     const size_t block = (size_t)(position / kBlockTokens);
     const int key = position % kBlockTokens;
-    return block * (size_t)(kBlockTokens * head_dim) + (size_t)((d * 4 + v_chunk_of_key(key)) * 8 + v_index_of_key(key));
+    return block * (size_t)(kBlockTokens * head_dim) +
+           (size_t)(v_piece(head_dim, d, v_chunk_of_key(key)) + v_index_of_key(key));
 }
 
 constexpr int kQuantGroup = 64;  // KVCacheManager.quantizationGroupSize

@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) void kvq_dequant_blocks_kernel(const QuantArgs
             h8 o;
 #pragma unroll
             for (int i = 0; i < 8; ++i) o[i] = (_Float16)((float)lv[i] * (float)scale[i] + (float)bias[i]);
-            *reinterpret_cast<h8 *>(v_dst + dst + (size_t)p * 8) = o;
+            *reinterpret_cast<h8 *>(v_dst + dst + v_piece(D, d, chunk)) = o;
         }
     }
 }

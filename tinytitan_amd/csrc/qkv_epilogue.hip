@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
             h8 x;
 #pragma unroll
             for (int i = 0; i < 8; ++i) x[i] = vt[v_key_at(c, i) * ROW + d];
-            *reinterpret_cast<h8 *>(a.v_layer + dst0 + (size_t)p * 8) = x;
+            *reinterpret_cast<h8 *>(a.v_layer + dst0 + v_piece(D, d, c)) = x;
         }
         return;
     }
