@@ -983,3 +983,42 @@ def test_lists_whose_tiles_do_not_divide_the_chip_in_whole_rounds(bits, D, H, KH
     ks, vs = (k, v) if bits == 16 else (_dequantised(k, bits), _dequantised(v, bits))
     want = np.concatenate([_oracle_rows_kept(q[t:t + 1], ks, vs, start + t, keep[t:t + 1], H, KH, D, scale, gate=gate[t:t + 1]) for t in some])
     _check(eager[some], want, f"whole rounds D={D} {H}/{KH} bits {bits}")
+
+
+@pytest.mark.parametrize("H,KH,T,rows,past", [(16, 2, 3199, 33, 0), (16, 2, 3200, 33, 0), (16, 2, 3203, 33, 1), (24, 2, 4611, 301, 0), (40, 2, 3300, 260, 0)])
+def test_wide_lists_and_many_tiles_of_wide_heads_equal_the_mask_form(gpu_ctx, H, KH, T, rows, past):
+    # Heads of 256 on both sides of the line between groups of keys and blocks: the shortest contexts that are walked by groups,
+    # the widest lists (`past`: one entry wider), and more tiles than half of the CUs.
+    import torch
+    from tinytitan_amd.engine import PrefillAttention, PrefillAttentionParams
+    D = 256
+    r = np.random.default_rng(T + H)
+    start, scale = T - rows, D ** -0.5
+    tt = 32 // (H // KH)
+    stride = 8 * T // (9 * tt) + past
+    keep = np.zeros((rows, ((T + 3) // 4) * 4), np.uint8)
+    for t in range(rows):
+        for g in r.choice((start + t) // 4, [stride // 4 - 1, 3, 200][t % 3], replace=False):
+            keep[t, 4 * g:4 * g + (4 if t % 2 else r.integers(1, 5))] = 1
+        keep[t, start + t] = 1
+    lists, counts = np.zeros((rows, stride), np.int32), np.zeros(rows, np.int32)
+    for t in range(rows):
+        ids = np.flatnonzero(keep[t])
+        lists[t, :len(ids)], counts[t] = ids, len(ids)
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    q, gate = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    kv = _cache(gpu_ctx, 16, KH, D, T)
+    _append(gpu_ctx, kv, 0, 0, 0, k, v)
+    by_mask = _prefill_keep(gpu_ctx, kv, q, start, T, keep, H, scale, gate=gate)
+    qd, gd, lists_d, counts_d = _dev(q), _dev(gate), _dev(lists), _dev(counts)
+    out = torch.full((rows, H * D), float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, T, H, scale, H * D, H * D, H * D),
+                                            gate=gd, keep_indices=lists_d, keep_index_stride=stride, keep_counts=counts_d)
+    gpu_ctx.synchronize()
+    got = out.float().cpu().numpy()
+    kv.close()
+    assert np.abs(got - by_mask).max() <= 2e-3
+    some = [0, 1, 2, tt, rows - 1]
+    want = np.concatenate([_oracle_rows_kept(q[t:t + 1], k, v, start + t, keep[t:t + 1], H, KH, D, scale, gate=gate[t:t + 1]) for t in some])
+    _check(got[some], want, f"wide lists {H}/{KH} T={T}")

@@ -350,14 +350,18 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             // Groups of four keys instead of blocks of 32 (fp16 pages, tiles of 32 rows): a turn of the walk then takes eight
             // listed groups instead of one touched block, of which a selection in blocks of four leaves 1.3 to 2 groups
             // wanted at 32k keys and more (one row's list of 2,051 cells each): 128 rows of 16/2 heads of 256 behind 16k keys 74.0 ->
-            // 65.0 us, 32k 101.3 -> 74.2, 131k 163.0 -> 120.2, all rows sharing one selection 65.8 -> 47.8.
-            // Where the tile's lists could hold half of the keys most of a block is wanted, and a block's loads are the better ones
-            // (8k keys, 512 rows: 121.7 against 133.4 us).  Nor where many tiles walk wide heads: they share fetched lines in L2 only
-            // while they stay side by side, which the walk over blocks does better (512 rows behind 131k keys 536 against 708 us;
-            // with heads of 64 470 -> 208).  The group bitmap has to leave the plan kernel's LDS room for a run of bits.
+            // 55 us, 32k 101.3 -> 59.6, 131k 163.0 -> 80.7.
+            // Where the tile's lists could hold most of the keys, most of a block is wanted and its loads are the better ones.
+            // Heads of 256, whose groups lie in lines of their own (kv_layout.h): as long as the lists hold no more than eight
+            // ninths of the keys, from 3,200 keys on (by blocks / by groups: 24/2 heads, 300 rows behind 4,500 keys 130 / 126 us, 512
+            // behind 9,000 226 / 150, behind 64,000 593 / 212, 40/2 heads, 512 behind 3,500 209 / 185, behind 2,500 171 / 182).
+            // Narrower heads: half of the keys (8k keys, 512 rows: 121.7 against 133.4 us), and a bound on the tiles: many share
+            // fetched lines in L2 only while they stay side by side, which the walk over blocks does better (inside the bound 512 rows of
+            // heads of 64 behind 131k keys 470 -> 208 us).  The group bitmap has to leave the plan kernel's LDS room for a run of bits.
             const long long entries = (long long)plan.tt * (long long)lists->stride;
-            groups = kv_bits == 16 && plan.nt == 32 && 2 * entries <= totals[base] &&
-                     (long long)plan.n_tiles * D <= 128ll * ctx->n_cus && totals[base] <= kPlanGroupKeys;
+            groups = kv_bits == 16 && plan.nt == 32 && totals[base] <= kPlanGroupKeys &&
+                     (D == 256 ? 9 * entries <= 8ll * totals[base] && totals[base] >= 3200
+                               : 2 * entries <= totals[base] && (long long)plan.n_tiles * D <= 128ll * ctx->n_cus);
             const int unit = groups ? 4 : 32;
             ctx_units = (totals[base] + unit - 1) / unit;
             cap = (int)(entries < ctx_units ? entries : ctx_units);
