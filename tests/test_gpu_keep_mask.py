@@ -998,7 +998,7 @@ def test_wide_lists_and_many_tiles_of_wide_heads_equal_the_mask_form(gpu_ctx, H,
     stride = 8 * T // (9 * tt) + past
     keep = np.zeros((rows, ((T + 3) // 4) * 4), np.uint8)
     for t in range(rows):
-        for g in r.choice((start + t) // 4, [stride // 4 - 1, 3, 200][t % 3], replace=False):
+        for g in r.choice((start + t) // 4, [stride // 4 - 1, 3, stride // 8][t % 3], replace=False):
             keep[t, 4 * g:4 * g + (4 if t % 2 else r.integers(1, 5))] = 1
         keep[t, start + t] = 1
     lists, counts = np.zeros((rows, stride), np.int32), np.zeros(rows, np.int32)
