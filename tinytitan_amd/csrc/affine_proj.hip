@@ -377,9 +377,9 @@ void launch_tile(tt_hip_ctx *ctx, const ProjArgs &a) {
 // coalesced; they lie in one group), widens them to fp16 levels and contracts them with its 8 x
 // values by v_dot2_f32_f16 (products exact, fp32 accumulation), then
 // acc += scale * dot + bias * sum(x) as above.  All of a wavefront's loads for a 512-column chunk
-// are independent, so they are in flight together; lanes are added by DPP moves (six vector instructions a
-// sum; as six shuffles through LDS each, the 8 x TOK sums were most of the kernel: one token 5.5 -> 4.2 us a step,
-// four tokens 11.0 -> 6.3; from five on the tiles above are ahead, 5.4 us against 6.6),
+// are independent, so they are in flight together; the lanes' 8 x TOK sums are added by moves between lanes that pack two values
+// into one at every step (wave_sums; a chain of six DPP moves for each was most of a launch of four tokens: 2048 x 4096 over 4
+// bits, launch to launch, one token 3.60 -> 3.33 us, two 4.23 -> 3.72, four 5.62 -> 4.59, where five take the tiles above 4.91),
 // wavefronts through LDS in a fixed order.  256 workgroups at 2048 rows.
 // ---------------------------------------------------------------------------
 constexpr int kGemvWaves = 8, kGemvRows = 8, kGemvMaxTokens = 4;
@@ -454,13 +454,12 @@ __global__ __launch_bounds__(kGemvWaves * 64) void affine_gemv_kernel(const Proj
             for (int t = 0; t < TOK; ++t) acc[r][t] = fmaf(bias, xsum[t], fmaf(scale, dot8(xv[t], levels), acc[r][t]));
         }
     }
+    float v[kGemvRows * TOK];
 #pragma unroll
-    for (int r = 0; r < kGemvRows; ++r)
-#pragma unroll
-        for (int t = 0; t < TOK; ++t) {
-            const float v = wave_sum_in_lane63(acc[r][t]);
-            if (lane == 63) partial[wave][r * TOK + t] = v;
-        }
+    for (int i = 0; i < kGemvRows * TOK; ++i) v[i] = acc[i / TOK][i % TOK];
+    int mine;  // the sum that this lane ends up with
+    const float sum = wave_sums<kGemvRows * TOK>(v, lane, mine);
+    if (mine >= 0) partial[wave][mine] = sum;
     __syncthreads();
     if (threadIdx.x < kGemvRows * TOK) {
         const int r = threadIdx.x / TOK, t = threadIdx.x % TOK;

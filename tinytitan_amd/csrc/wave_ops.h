@@ -84,6 +84,60 @@ __device__ __forceinline__ float wave_sum_in_lane63(float x) {
     return x;
 }
 
+// The sums of the 64 lanes of N <= 32 values, each value's in a lane of its own: `mine` is the value whose sum the lane gets, -1
+// in the lanes that are left over.  Six steps, every one of which adds two lanes and, while there are several values, packs two
+// of them into one register on the way -- by v_permlane32_swap, v_permlane16_swap, then by picks and DPP moves inside a
+// row -- so that the work halves from step to step: 71 instructions for 32 values, where six a value are 192.  A value's
+// additions are the same ones whatever N is.
+template <int CTRL>
+__device__ __forceinline__ float sums_moved(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+template <int N>
+__device__ __forceinline__ float wave_sums(float (&v)[N], int lane, int &mine) {
+    static_assert(N >= 1 && N <= 32, "a lane bit tells two values apart, and one is left for the last step");
+    auto pairs = [&](int count, auto join) {  // the values 2 i and 2 i + 1 become value i; an odd last one stands for both
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (2 * i < count) v[i] = join(v[2 * i], v[2 * i + 1 < count ? 2 * i + 1 : 2 * i]);
+        return (count + 1) / 2;
+    };
+    // lanes l and l ^ 32, then l and l ^ 16: the lower ones keep a's sum, the upper ones b's
+    int count = pairs(N, [](float a, float b) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+        return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+    });
+    count = pairs(count, [](float a, float b) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+        return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+    });
+    // inside a row of 16: row_ror:8, row_half_mirror, quad_perm [2,3,0,1]
+    const auto step = [&](int bit, auto ctrl) {
+        const bool upper = (lane & bit) != 0;
+        if (count == 1) {
+            v[0] += sums_moved<decltype(ctrl)::value>(v[0]);
+            return;
+        }
+        count = pairs(count, [&](float a, float b) { return (upper ? b : a) + sums_moved<decltype(ctrl)::value>(upper ? a : b); });
+    };
+    step(8, std::integral_constant<int, 0x128>{});
+    step(4, std::integral_constant<int, 0x141>{});
+    step(2, std::integral_constant<int, 0x4E>{});
+    v[0] += sums_moved<0xB1>(v[0]);
+    mine = (lane >> 5) + ((lane >> 4) & 1) * 2 + ((lane >> 3) & 1) * 4;
+    int unused = 7;
+    if constexpr (N > 8) {
+        mine += ((lane >> 2) & 1) * 8;
+        unused = 3;
+    }
+    if constexpr (N > 16) {
+        mine += ((lane >> 1) & 1) * 16;
+        unused = 1;
+    }
+    if (mine >= N || (lane & unused)) mine = -1;
+    return v[0];
+}
+
 // Sums, minima and maxima over aligned groups of 8, 16 or 32 lanes, every lane of a group getting the result, by DPP
 // moves: quad_perm [1,0,3,2] and [2,3,0,1] inside a quad; then row_half_mirror (lane i <-> 7 - i: the other quad,
 // whose lanes all hold that quad's value by now) and row_mirror (i <-> 15 - i: the other eight); the other row of 16 by
