@@ -130,3 +130,34 @@ def test_key_ranges_of_a_window_that_begins_to_clip_inside_the_chunk(gpu_ctx, H,
         want = oracle.prefill_ref(q[row:row + 1].astype(np.float32), k32, v32, H * D, KH * D, D, H, KH, start + row, 1, start + row + 1,
                                   window, scale).reshape(1, -1)
         _check(got[row:row + 1], want, f"row {row} of {rows} behind {start} keys, {H}q/{KH}kv/{D}, window {window}")
+
+
+@pytest.mark.parametrize("H,KH,rows,start,window", [(16, 2, 3989, 0, 0), (16, 2, 4000, 33, 0), (16, 2, 4031, 0, 0), (8, 2, 70, 20003, 0), (32, 8, 777, 5003, 4096)])
+def test_heads_of_128_in_steps_of_two_blocks(gpu_ctx, H, KH, rows, start, window):
+    # Two key blocks a step: tiles, pairs of tiles (the second one's first blocks copied in behind the first one's last) and key ranges of odd and
+    # even numbers of blocks.  Rows on both sides of the tiles' edges, against the oracle over each row's own keys.
+    import torch
+    from tinytitan_amd.engine import KVCacheManager, PrefillAttention, PrefillAttentionParams
+    D = 128
+    total, scale = start + rows, float(D) ** -0.5
+    r = np.random.default_rng(rows + start)
+    k, v = (r.standard_normal((total, KH * D)).astype(np.float16) for _ in range(2))
+    q, g = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=1, max_context=total, initial_capacity=total)
+    kd, vd, qd, gd = _dev(k), _dev(v), _dev(q), _dev(g)
+    out = torch.full(qd.shape, float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    kv.append(0, 0, 0, kd, vd)
+    PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, total, H, scale, H * D, H * D, H * D,
+                                                                                     sliding_window=window), gate=gd)
+    gpu_ctx.synchronize()
+    got = out.float().cpu().numpy()
+    kv.close()
+    assert np.isfinite(got).all()
+    k32, v32 = k.astype(np.float32), v.astype(np.float32)
+    edges = {e + o for e in range(0, rows, 32) for o in (-1, 0)}
+    some = sorted(e for e in edges | {rows - 1} if 0 <= e < rows)
+    for row in some[::max(1, len(some) // 60)] + [rows - 1]:
+        want = oracle.prefill_ref(q[row:row + 1].astype(np.float32), k32, v32, H * D, KH * D, D, H, KH, start + row, 1, start + row + 1,
+                                  window, scale).reshape(1, -1) / (1 + np.exp(-g[row:row + 1].astype(np.float64)))
+        _check(got[row:row + 1], want, f"row {row} of {rows} behind {start} keys, {H}q/{KH}kv/{D}, window {window}")

@@ -22,8 +22,8 @@
 // waves per CU also issue LDS reads about 1.6x faster than four can (the per-wave issue rate
 // is what limits a 4-wave design).  One workgroup barrier per key block separates the steps.
 //
-// K/V blocks stream L2 -> LDS with direct-to-LDS 128-bit loads (no registers), four stages
-// deep, issued two steps ahead of their first use; the K fragment layout in HBM is the MFMA
+// K/V blocks stream L2 -> LDS with direct-to-LDS 128-bit loads (no registers), three or four stages
+// deep, issued one or two steps ahead of their first use; the K fragment layout in HBM is the MFMA
 // operand layout, V is permuted into it by the copy.
 //
 // The online softmax rescales lazily: a row's reference max only moves when its block max
@@ -76,7 +76,18 @@ namespace {
 
 constexpr float kNegBig = -1.0e30f;
 constexpr float kRescaleThreshold = 8.0f;
-constexpr int kBuffers = 4;  // LDS stages (K block + V block each): 128 KiB at D = 256
+// Key blocks of 32 that a step takes, and how many steps' K and V the rings in LDS hold.  Heads of 128 take two: a step's MFMAs are then
+// as many as at 256, its two score chains have no link that waits for the one before it, and there is one barrier, one row
+// maximum and one rescale test for 64 keys (32/8 heads, 777 rows behind 5,003 keys 107.5 -> 95.4 us, 4096 behind 8,000
+// 770 -> 710; V's ring holds three so that all of it stays within 160 KiB).  Two workgroups of one block a step on a CU (rings
+// of three, 128 registers) came to 721 where the chip is full and lost 5 % where it is not.
+constexpr int step_blocks(int D) { return D == 128 ? 2 : 1; }
+constexpr int k_ring(int) { return 4; }
+constexpr int v_ring(int D) { return D == 128 ? 3 : 4; }
+template <int RING>
+__device__ __forceinline__ int in_ring(int j) {  // j >= -RING
+    return RING == 4 ? j & 3 : (int)((unsigned)(j + RING) % (unsigned)RING);
+}
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -112,24 +123,25 @@ __device__ __forceinline__ void copy16_global_to_lds(const void *base, unsigned 
 // probabilities (B operand of the two P.V k-steps) against the reference.  The row sum is taken
 // over the ROUNDED probabilities (dot2 against ones), i.e. over exactly the weights the P.V MFMAs
 // see.  Returns the factor the row's accumulators must be scaled by before this block is added.
-__device__ __forceinline__ float softmax_step(const f16v &s_raw, bool mask, int kbase, int lo, int lim, int g,
-                                              float scale_log2e, float &m, float &l, h8 (&pf)[2]) {
+template <int NB>
+__device__ __forceinline__ float softmax_step(const f16v (&s_raw)[NB], bool mask, int kbase, int lo, int lim, int g,
+                                              float scale_log2e, float &m, float &l, h8 (&pf)[2 * NB]) {
     const h2 ones = {(_Float16)1.0f, (_Float16)1.0f};
     // The maximum is taken over the raw scores and scaled once (the host sends only chunks with scale > 0 here), and a
     // probability is one fused multiply-add and one exp2 off its raw score.
-    float t[16];
+    float t[16 * NB];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) t[v] = s_raw[v];
+    for (int v = 0; v < 16 * NB; ++v) t[v] = s_raw[v >> 4][v & 15];
     if (mask) {  // wave-uniform: only the blocks on or past the tile's diagonal, or at its window's lower edge
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
+        for (int v = 0; v < 16 * NB; ++v) {
             const int key = kbase + 8 * (v >> 2) + 4 * g + (v & 3);
             if (key >= lim || key < lo) t[v] = -INFINITY;
         }
     }
     float mx = fmaxf(t[0], t[1]);
 #pragma unroll
-    for (int v = 2; v < 16; v += 2) mx = fmaxf(fmaxf(t[v], t[v + 1]), mx);
+    for (int v = 2; v < 16 * NB; v += 2) mx = fmaxf(fmaxf(t[v], t[v + 1]), mx);
     mx = max_across_halves(mx) * scale_log2e;
     const bool move = mx > m + kRescaleThreshold;  // a row's first visible block always moves
     const float m_new = move ? mx : m;
@@ -137,7 +149,7 @@ __device__ __forceinline__ float softmax_step(const f16v &s_raw, bool mask, int 
     l *= alpha;
     m = m_new;
 #pragma unroll
-    for (int v = 0; v < 16; v += 2) {
+    for (int v = 0; v < 16 * NB; v += 2) {
         const h2 p = {(_Float16)fast_exp2(__builtin_fmaf(t[v], scale_log2e, -m)), (_Float16)fast_exp2(__builtin_fmaf(t[v + 1], scale_log2e, -m))};
         l = __builtin_amdgcn_fdot2(p, ones, l, false);
         pf[v >> 3][v & 7] = p[0];
@@ -149,15 +161,20 @@ __device__ __forceinline__ float softmax_step(const f16v &s_raw, bool mask, int 
 }  // namespace
 
 template <int D>
-__global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs a) {
+__global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(const PrefillArgs a) {
     constexpr int KS = D / 16;  // k-steps of S^T
     constexpr int MT = D / 32;  // 32-dim tiles of O^T
     constexpr int BLOCK_BYTES = 32 * D * 2;
+    constexpr int NB = step_blocks(D);            // key blocks per step
+    constexpr int KR = k_ring(D), VR = v_ring(D);
+    constexpr int SLOT_BYTES = NB * BLOCK_BYTES;
     constexpr int CHUNKS = BLOCK_BYTES / 1024;    // 1 KiB chunks per block (= KS = 2 MT)
-    constexpr int CPW = CHUNKS / 4;               // copies one wave issues per step (a K and a V block over 8 waves)
-    constexpr int V_OFF = kBuffers * BLOCK_BYTES;    // K ring, then V ring, kBuffers blocks each
-    constexpr int P_OFF = 2 * kBuffers * BLOCK_BYTES;  // P^T: [2 steps][4 heads][2 k-steps][64 lanes][16 B]
-    constexpr int ALPHA_OFF = P_OFF + 2 * 4 * 2048;    // rescale factors: [2 steps][4 heads][32 rows] floats
+    constexpr int CPW = NB * CHUNKS / 4;          // copies one wave issues per step (K and V of a step's blocks over 8 waves)
+    static_assert(CHUNKS % CPW == 0, "a wave's copies of a step are of one block");
+    constexpr int V_OFF = KR * SLOT_BYTES;             // K ring, then V ring
+    constexpr int P_OFF = (KR + VR) * SLOT_BYTES;      // P^T: [2 steps][4 heads][2 NB k-steps][64 lanes][16 B]
+    constexpr int P_STEP = 4 * NB * 2048;
+    constexpr int ALPHA_OFF = P_OFF + 2 * P_STEP;      // rescale factors: [2 steps][4 heads][32 rows] floats
     constexpr int LSUM_OFF = ALPHA_OFF + 2 * 4 * 128;  // row sums: [4 heads][32 rows] floats
     constexpr int STAGE_OFF = LSUM_OFF + 4 * 128;      // output rows on their way out: [4 heads][32 rows][32 dims + 16 B]
     constexpr int STAGE_PITCH = 64 + 16;
@@ -204,27 +221,30 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
     const _Float16 *kp = a.k_slot + (size_t)kvh * a.page_elems;
     const _Float16 *vp = a.v_slot + (size_t)kvh * a.page_elems;
 
-    // Copies of step i: K block i + 4 and V block i + 2, 2 CHUNKS one-KiB chunks of which this wave
-    // issues CPW.  Block b lives in slot b % kBuffers of its ring.  Past the end of the tile the
+    // Copies of step i: K of step i + KR and V of step i + VR - 2, of which this wave issues CPW one-KiB chunks.  Step
+    // j's blocks live in slot j % KR (% VR) of their ring.  Past the end of the tile the
     // last block is copied again (into a slot nobody reads any more), so that every step puts
     // the same number of copies in flight and one constant vmcnt tracks them.
     const unsigned smem_base = (unsigned)(size_t)(lds_ptr_t)smem;
     const unsigned k_lane_offset = (unsigned)lane * 16u;
     const unsigned v_lane_offset = (unsigned)v_piece(D, li, g) * 2u;  // this lane's 16 bytes inside a V chunk gather
     int jb = 0;  // first key block of this workgroup's range in the current tile
-    // Block b of the tile in hand lives in slot (b + slot_off) % kBuffers.  When a second tile follows (carry_nb > 0:
-    // it has that many blocks, from block 0), the copies past the end of the first fetch ITS first blocks -- K 0..3 and
-    // V 0..3 are in LDS when the first tile's last step ends, in the slots that follow on, and the second tile starts
-    // without waiting for memory.
+    // Step j of the tile in hand lives in slot (j + slot_off) % ring.  When a second tile follows (carry_nb > 0:
+    // it has that many blocks, from block 0), the copies past the end of the first fetch ITS first blocks -- a ring of K
+    // and one of V are in LDS when the first tile's last step ends, in the slots that follow on, and the second tile starts
+    // without waiting for memory.  (A wave copies and reads K or V, so the offset is that of its own ring.)
     int slot_off = 0, carry_nb = 0;
     auto page_block = [&](int block) { return a.ring_blocks ? block % a.ring_blocks : block; };
+    auto role_ring = [&](int j) { return value_wave ? in_ring<VR>(j) : in_ring<KR>(j); };
+    const int my_block = NB == 1 ? 0 : w4 * CPW / CHUNKS;  // which of a step's blocks this wave copies from
+    const int my_chunk = w4 * CPW - my_block * CHUNKS;
     auto source_block = [&](int j, int nb) {  // the block that step-relative index j stands for
-        if (j < nb || carry_nb == 0) return jb + max(min(j, nb - 1), 0);
-        return min((j - nb) & (kBuffers - 1), carry_nb - 1);  // (a slot's block again once the four are in: the same bytes)
+        const int steps = (nb + NB - 1) / NB;
+        if (j < steps || carry_nb == 0) return jb + max(min(NB * j + my_block, nb - 1), 0);
+        return min(NB * role_ring(j - steps) + my_block, carry_nb - 1);  // (a slot's blocks again once the ring is full: the same bytes)
     };
-    // A step's copies: this wave's CPW one-KiB chunks of ONE block -- K block i + 4 for the score waves (chunk
-    // wave * CPW + c; the LDS layout is the HBM layout, fragment s is chunk s), V block i + 2 for the value waves
-    // (gathered so that LDS holds fragment (mt, t) as [lane][8 halves]).  Where the block lies in the page and in the
+    // A step's copies: this wave's CPW one-KiB chunks of ONE block -- of K for the score waves (the LDS layout is the HBM
+    // layout, fragment s is chunk s), of V for the value waves (gathered so that LDS holds fragment (mt, t) as [lane][8 halves]).  Where the block lies in the page and in the
     // ring is worked out ONCE per step (step_copies); a copy then costs two scalar adds on top of its load -- worked
     // out per copy it was 30 scalar instructions each, 120 to 145 a step in the instruction stream of a wave whose
     // matrix instructions wait behind them.
@@ -235,15 +255,15 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
     unsigned v_src_off[CPW];  // source offsets of this value wave's chunks inside a V block
 #pragma unroll
     for (int c = 0; c < CPW; ++c) {
-        const int chunk = w4 * CPW + c, mt = chunk >> 1, t = chunk & 1;
+        const int chunk = my_chunk + c, mt = chunk >> 1, t = chunk & 1;
         v_src_off[c] = (unsigned)v_piece(D, 32 * mt, 2 * t) * 2u;
     }
     auto step_copies = [&](int i, int nb) {  // of step i; nb blocks in the range
         StepCopies sc;
-        const int j = value_wave ? i + 2 : i + 4;
+        const int j = value_wave ? i + VR - 2 : i + KR;
         const _Float16 *page = value_wave ? vp : kp;
-        sc.src = reinterpret_cast<const char *>(page + (size_t)page_block(source_block(j, nb)) * (32 * D)) + (value_wave ? 0 : w4 * CPW * 1024);
-        sc.dst = smem_base + (unsigned)((value_wave ? V_OFF : 0) + ((j + slot_off) & (kBuffers - 1)) * BLOCK_BYTES + w4 * CPW * 1024);
+        sc.src = reinterpret_cast<const char *>(page + (size_t)page_block(source_block(j, nb)) * (32 * D)) + (value_wave ? 0 : my_chunk * 1024);
+        sc.dst = smem_base + (unsigned)((value_wave ? V_OFF : 0) + role_ring(j + slot_off) * SLOT_BYTES + w4 * CPW * 1024);
         return sc;
     };
     auto issue_copy = [&](const StepCopies &sc, int c) {  // copy c (0 .. CPW-1)
@@ -256,7 +276,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
         for (int c = 0; c < CPW; ++c) issue_copy(sc, c);
     };
 
-    char *const p_mine = smem + P_OFF + w4 * 2048 + lane * 16;           // + step parity * 8192, + k-step * 1024
+    char *const p_mine = smem + P_OFF + w4 * (NB * 2048) + lane * 16;  // + step parity * P_STEP, + k-step * 1024
     float *const alpha_mine = reinterpret_cast<float *>(smem + ALPHA_OFF) + w4 * 32 + li;  // + step parity * 128
     float *const lsum_mine = reinterpret_cast<float *>(smem + LSUM_OFF) + w4 * 32 + li;
 
@@ -280,11 +300,17 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
         const int end = min(a.kv_valid, a.start + min(a.q_len, tile * 32 + 32));
         const int nb_tile = (end + 31) >> 5;                   // key blocks this tile needs
         const int mask_from = (a.start + tile * 32 + 1) >> 5;  // first block in which some row is masked by causality
-        const int first_masked = min(mask_from, end >> 5);     // ... or cut by the valid length
-        // This workgroup's share of them (all, without key splits); local step i is block jb + i.
+        // This workgroup's share of them (all, without key splits); local step i is blocks jb + NB i ..
         jb = window_block + (a.n_splits > 1 ? split * a.split_blocks : 0);
         const int nb = (a.n_splits > 1 ? min(nb_tile, jb + a.split_blocks) : nb_tile) - jb;
         if (nb <= 0) continue;  // nothing of this tile in the range (the same for every wave)
+        const int steps = (nb + NB - 1) / NB;
+        int first_masked = min(mask_from, end >> 5);  // ... or cut by the valid length
+        int hi = lim;                                 // keys [lo, hi) count here
+        if constexpr (NB > 1) {  // (the range may end inside the last step)
+            first_masked = __builtin_amdgcn_readfirstlane(min(first_masked, jb + nb));
+            hi = min(lim, (jb + nb) * 32);
+        }
 
         if (pass > 0) __syncthreads();  // every wave is done with the previous pass's LDS
         const bool carried = carry_nb > 0;  // this tile's first blocks came in behind the previous tile's last
@@ -296,19 +322,21 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
         }
         if (!carried) {
 #pragma unroll
-            for (int i = -4; i < 0; ++i) issue_step(i, nb);  // K blocks 0..3, V blocks 0..1
+            for (int i = -KR; i < 0; ++i) issue_step(i, nb);  // K of steps 0 .. KR - 1, V of steps 0 .. VR - 3
         }
 
-        // End of step i.  K(i+2) and V(i+1) -- copies of step i-2 -- must have landed: the next
-        // step reads them from LDS.  The copies of steps i-1 and i may still fly.  Then the
+        // End of step i.  What the next step reads from LDS, K(i+2) and V(i+1), was copied KR - 2 and VR - 2 steps before
+        // and must have landed; the copies of the steps since may still fly.  Then the
         // barrier that publishes them and this step's P^T.
-        auto end_step = [&]() {
-            TT_WAIT_VMCNT(2 * CPW);
+        auto end_step = [&](auto ring) {
+            TT_WAIT_VMCNT((decltype(ring)::value - 2) * CPW);
             __syncthreads();
         };
+        constexpr std::integral_constant<int, KR> k_landed{};
+        constexpr std::integral_constant<int, VR> v_landed{};
 
-        // Step i (0 .. nb + 1): the score waves run the MFMAs of block i, the value waves those of
-        // block i - 2; both fetch the NEXT step's fragments from LDS into the registers the
+        // Step i (0 .. steps + 1): the score waves run the MFMAs of step i's blocks, the value waves those of
+        // step i - 2's; both fetch the NEXT step's fragments from LDS into the registers the
         // MFMAs have just read, so that after the barrier the matrix pipe starts at once.
         // The two roles run separate loops (their register sets are disjoint that way) that
         // meet at the same barriers.
@@ -324,38 +352,43 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
             float m = kNegBig, l = 0.0f;
             TT_WAIT_VMCNT(0);  // the first stages and the query rows
             __syncthreads();
-            h8 kf[KS];
+            h8 kf[NB * KS];
 #pragma unroll
-            for (int t = 0; t < KS; ++t)
-                kf[t] = *reinterpret_cast<const h8 *>(smem + (slot_off & (kBuffers - 1)) * BLOCK_BYTES + lane * 16 + t * 1024);
-            __syncthreads();  // every score wave holds K block 0: step 0 may refill its slot
+            for (int t = 0; t < NB * KS; ++t)
+                kf[t] = *reinterpret_cast<const h8 *>(smem + slot_off * SLOT_BYTES + lane * 16 + t * 1024);
+            __syncthreads();  // every score wave holds K of step 0: step 0 may refill its slot
 #pragma nounroll
-            for (int i = 0; i < nb; ++i) {
-                const char *next = smem + ((i + 1 + slot_off) & (kBuffers - 1)) * BLOCK_BYTES + lane * 16;
+            for (int i = 0; i < steps; ++i) {
+                const char *next = smem + in_ring<KR>(i + 1 + slot_off) * SLOT_BYTES + lane * 16;
                 const StepCopies sc = step_copies(i, nb);
-                f16v s = (f16v)0.0f;
+                f16v s[NB];
 #pragma unroll
-                for (int t = 0; t < KS; ++t) {
-                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[t], qf[t], s, 0, 0, 0);
-                    kf[t] = *reinterpret_cast<const h8 *>(next + t * 1024);
+                for (int b = 0; b < NB; ++b) s[b] = (f16v)0.0f;
+                // (a step of two blocks: their chains of MFMAs in turn)
+#pragma unroll
+                for (int u = 0; u < NB * KS; ++u) {
+                    const int b = u % NB, t = u / NB, f = b * KS + t;
+                    s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[f], qf[t], s[b], 0, 0, 0);
+                    kf[f] = *reinterpret_cast<const h8 *>(next + f * 1024);
                     // this step's copies, one at a time between MFMAs: a burst would stall the wave
                     // on the CU's vector memory path (64 B/clk for all eight waves)
-                    if (t % (KS / CPW) == 0) issue_copy(sc, t / (KS / CPW));
+                    if (u % (NB * KS / CPW) == 0) issue_copy(sc, u / (NB * KS / CPW));
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                h8 pf[2];
-                const float alpha = softmax_step(s, jb + i >= first_masked || jb + i <= last_lo_block, (jb + i) << 5, lo, lim, g,
-                                                 a.scale_log2e, m, l, pf);
-                char *pdst = p_mine + (i & 1) * 8192;
-                *reinterpret_cast<h8 *>(pdst) = pf[0];
-                *reinterpret_cast<h8 *>(pdst + 1024) = pf[1];
+                h8 pf[2 * NB];
+                const int block = jb + NB * i;
+                const float alpha = softmax_step<NB>(s, block + NB - 1 >= first_masked || block <= last_lo_block, block << 5, lo, hi, g,
+                                                     a.scale_log2e, m, l, pf);
+                char *pdst = p_mine + (i & 1) * P_STEP;
+#pragma unroll
+                for (int t = 0; t < 2 * NB; ++t) *reinterpret_cast<h8 *>(pdst + t * 1024) = pf[t];
                 if (g == 0) alpha_mine[(i & 1) * 128] = alpha;
-                end_step();
+                end_step(k_landed);
             }
-            issue_step(nb, nb);
-            end_step();  // the value waves' last two steps
-            issue_step(nb + 1, nb);
-            end_step();
+            issue_step(steps, nb);
+            end_step(k_landed);  // the value waves' last two steps
+            issue_step(steps + 1, nb);
+            end_step(k_landed);
             const float lt = sum_across_halves(l);
             if (g == 0) {
                 if (a.n_splits > 1) {  // partial: the row's reference max (log2 domain) and sum over this key range
@@ -374,47 +407,59 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
             for (int mt = 0; mt < MT; ++mt) o[mt] = (f16v)0.0f;
             TT_WAIT_VMCNT(0);
             __syncthreads();
-            __syncthreads();  // (the score waves fetch K block 0 between these two)
-            // Two steps behind the score wave: block j's P^T (written in step j) and V fragments are
+            __syncthreads();  // (the score waves fetch K of step 0 between these two)
+            // Two steps behind the score wave: step j's P^T (written in step j) and V fragments are
             // fetched from LDS into registers during step j + 1 and consumed in step j + 2, so
             // that the MFMAs of a step start right after its barrier.
             issue_step(0, nb);
-            end_step();  // step 0: the score waves' first
+            end_step(v_landed);  // step 0: the score waves' first
             issue_step(1, nb);
-            h8 vf[2 * MT], pf[2];
+            h8 vf[NB * 2 * MT], pf[2 * NB];
 #pragma unroll
-            for (int c = 0; c < 2 * MT; ++c)
-                vf[c] = *reinterpret_cast<const h8 *>(smem + V_OFF + (slot_off & (kBuffers - 1)) * BLOCK_BYTES + lane * 16 + c * 1024);
-            pf[0] = *reinterpret_cast<const h8 *>(p_mine);
-            pf[1] = *reinterpret_cast<const h8 *>(p_mine + 1024);
+            for (int c = 0; c < NB * 2 * MT; ++c)
+                vf[c] = *reinterpret_cast<const h8 *>(smem + V_OFF + slot_off * SLOT_BYTES + lane * 16 + c * 1024);
+#pragma unroll
+            for (int t = 0; t < 2 * NB; ++t) pf[t] = *reinterpret_cast<const h8 *>(p_mine + t * 1024);
             float alpha = alpha_mine[0];
-            end_step();  // step 1
+            end_step(v_landed);  // step 1
 #pragma nounroll
-            for (int i = 2; i <= nb + 1; ++i) {
-                const int jn = i - 1;  // the block fetched in this step (past the last one: stale but harmless data)
-                const char *next = smem + V_OFF + ((jn + slot_off) & (kBuffers - 1)) * BLOCK_BYTES + lane * 16;
-                const char *psrc = p_mine + (jn & 1) * 8192;
+            for (int i = 2; i <= steps + 1; ++i) {
+                const int jn = i - 1;  // the step fetched in this one (past the last one: stale but harmless data)
+                const char *next = smem + V_OFF + in_ring<VR>(jn + slot_off) * SLOT_BYTES + lane * 16;
+                const char *psrc = p_mine + (jn & 1) * P_STEP;
                 const StepCopies sc = step_copies(i, nb);
                 if (__any(alpha != 1.0f)) {
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) o[mt] *= alpha;
                 }
-                h8 pn[2];
-                pn[0] = *reinterpret_cast<const h8 *>(psrc);
-                pn[1] = *reinterpret_cast<const h8 *>(psrc + 1024);
                 alpha = alpha_mine[(jn & 1) * 128];
-                // Both k-steps of a 32-dim tile back to back: consecutive MFMAs on one accumulator
-                // forward it inside the matrix pipe instead of going through the register file.
-#pragma unroll
-                for (int c = 0; c < 2 * MT; ++c) {
-                    o[c >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[c], pf[c & 1], o[c >> 1], 0, 0, 0);
+                auto multiply = [&](int u, int mt, int t) {  // the u-th: k-step t (block t / 2, its k-step t % 2) of 32-dim tile mt
+                    const int c = (t >> 1) * 2 * MT + 2 * mt + (t & 1);  // the fragment's place in the slot
+                    o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[c], pf[t], o[mt], 0, 0, 0);
                     vf[c] = *reinterpret_cast<const h8 *>(next + c * 1024);
-                    if (c % (KS / CPW) == 0) issue_copy(sc, c / (KS / CPW));
+                    if (u % (NB * KS / CPW) == 0) issue_copy(sc, u / (NB * KS / CPW));
                     __builtin_amdgcn_sched_barrier(0);
+                };
+                if constexpr (D == 256) {
+                    // All k-steps of a 32-dim tile back to back: consecutive MFMAs on one accumulator
+                    // forward it inside the matrix pipe instead of going through the register file.
+                    h8 pn[2 * NB];
+#pragma unroll
+                    for (int t = 0; t < 2 * NB; ++t) pn[t] = *reinterpret_cast<const h8 *>(psrc + t * 1024);
+#pragma unroll
+                    for (int u = 0; u < NB * 2 * MT; ++u) multiply(u, u / (2 * NB), u % (2 * NB));
+#pragma unroll
+                    for (int t = 0; t < 2 * NB; ++t) pf[t] = pn[t];
+                } else {
+                    // One k-step after the other: its P^T is read into the registers that its MFMAs are done with.
+#pragma unroll
+                    for (int t = 0; t < 2 * NB; ++t) {
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) multiply(t * MT + mt, mt, t);
+                        pf[t] = *reinterpret_cast<const h8 *>(psrc + t * 1024);
+                    }
                 }
-                pf[0] = pn[0];
-                pf[1] = pn[1];
-                end_step();
+                end_step(v_landed);
             }
             TT_WAIT_VMCNT(0);
             __syncthreads();  // the row sums are in LDS
@@ -466,7 +511,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(const PrefillArgs 
                 }
             }
         }
-        if (carry_nb > 0) slot_off = (slot_off + nb) & (kBuffers - 1);  // where the next tile's block 0 sits
+        if (carry_nb > 0) slot_off = role_ring(slot_off + steps);  // where the next tile's first step sits
     }
 }
 
@@ -478,8 +523,11 @@ bool prefill_kernel_serves(int n_q_heads, int n_kv_heads, int head_dim, bool ali
     return aligned && group % 4 == 0 && (head_dim == 256 || head_dim == 128 || head_dim == 64);
 }
 
-// four K+V stages (128 KiB at D = 256) + P^T hand-over (16 KiB) + rescale factors and row sums + the output rows' staging (10 KiB)
-static constexpr int prefill_lds_bytes(int D) { return kBuffers * 2 * 32 * D * 2 + 2 * 4 * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80; }
+// the rings of K and V (128 KiB at D = 256, 112 at 128) + P^T hand-over (16, 32 KiB) + rescale factors and row sums + the output rows' staging (10 KiB)
+static constexpr int prefill_lds_bytes(int D) {
+    return (k_ring(D) + v_ring(D)) * step_blocks(D) * 32 * D * 2 + 2 * 4 * step_blocks(D) * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80;
+}
+static_assert(prefill_lds_bytes(256) <= 160 * 1024 && prefill_lds_bytes(128) <= 160 * 1024, "a CU's LDS");
 
 int configure_prefill_kernels(tt_hip_ctx *ctx) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_kernel<256>),

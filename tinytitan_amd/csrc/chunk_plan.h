@@ -33,8 +33,8 @@ inline int longest_tile_blocks(int start, int q_len, int kv_valid, int window) {
 // 128 and 16 / 4 of 64, 512 to 4096 rows behind 0 to 9000 keys, whole and through windows of 1024 and 4096 keys.  `first_blocks`
 // and `last_blocks`: the key blocks its first and its last tile of 32 rows walk.
 
-// One key block of the chunk kernel's step, by how much of the chip takes part (at D = 256 the card's clock follows it).
-inline double chunk_step_us(int D, double fill) { return D == 256 ? 0.47 + 0.50 * fill : D == 128 ? 0.41 + 0.22 * fill : 0.45 + 0.05 * fill; }
+// One key block of the chunk kernel's step, by how much of the chip takes part (at D = 256 the card's clock follows it; at 128 half a step of two).
+inline double chunk_step_us(int D, double fill) { return D == 256 ? 0.47 + 0.50 * fill : D == 128 ? 0.38 + 0.20 * fill : 0.45 + 0.05 * fill; }
 
 struct ChunkEstimate {
     double us;
