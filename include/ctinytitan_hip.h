@@ -129,7 +129,7 @@ TT_HIP_API int tt_hip_calibrate_read(tt_hip_ctx *ctx, const void *src, size_t by
  * (a decode step at another length is another graph).  Its kernels address the
  * context's scratch and the caches' stores directly; once any of them has been
  * reallocated or freed since the capture (a later eager call that grew the
- * split scratch, the staging pages or the selection workspace,
+ * split scratch or the staging pages,
  * tt_hip_kv_reserve growth, tt_hip_kv_destroy), tt_hip_graph_launch returns
  * TT_HIP_ERR_STALE instead of replaying: capture again.  The
  * reference's analogue is encoding a whole layer into one MTLCommandBuffer
@@ -616,9 +616,10 @@ TT_HIP_API int tt_hip_qsa_decode_scores(tt_hip_ctx *ctx, const tt_half *raw_keys
  * Replaces qsa_select_decode (qsa.metal:156-226), QSAIndexer.selectKeys / selectKeysCompact /
  * encodeSelectKeys (QSAIndexer+Scratch.swift:191-284) and the host loop of selectKeysPrefill
  * (QSAIndexer.swift:414-497).  Scores must not be NaN (the reference's comparison has no order for
- * them either).  Up to 7 rows of more than 16,384 blocks each, or 8 of more than 32,768 (a decode or verify step at a long
- * context) are spread over many workgroups through a workspace the context allocates on first use:
- * that first call is refused with TT_HIP_ERR_BUSY while a graph is being captured.
+ * them either).  Rows of more than 16,384 blocks, up to a quarter of the CUs in number, and rows of more than 65,536 are
+ * spread over many workgroups through a workspace of 64 MiB that the context allocates on first use.  While a graph is
+ * being captured nothing is allocated: up to 7 such rows, or 8 of more than 32,768 blocks (a decode or verify step at a
+ * long context), are refused with TT_HIP_ERR_BUSY until a call outside has, and more rows are recorded as a workgroup each.
  * TT_HIP_ERR_SHAPE: keep_stride below the last row's visible keys, score_stride below its complete
  * blocks, index_stride below width. */
 TT_HIP_API int tt_hip_qsa_select(tt_hip_ctx *ctx, const float *scores, size_t score_stride, int rows, int first_visible,

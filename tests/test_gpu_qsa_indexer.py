@@ -669,3 +669,74 @@ def test_indexer_snapshot_payload(gpu_ctx):
         restored.restore_snapshot_payload(bytes(payload), 4, position + 4)   # other blocks than the position implies
     with pytest.raises(ValueError):
         restored.restore_snapshot_payload(bytes(payload[:-10]), 4, position)  # truncated
+
+
+@pytest.mark.parametrize("blocks,rows,kind,width", [(16385, 1, "half", 2051), (18432, 3, "half", 7), (18433, 64, "half", 2051), (40000, 64, "half", 2050),
+                                                    (131072, 2, "half", 2051), (131073, 2, "half", 2051), (33000, 2, "ties", 2051), (66000, 5, "ties", 2049),
+                                                    (70000, 2, "uniform", 2051), (140000, 1, "uniform", 9003), (20000, 2, "few", 2051), (20000, 2, "signed", 2052)])
+def test_spread_rows_sort_their_chunks(gpu_ctx, blocks, rows, kind, width):
+    # Chunks of 2,048 and 4,096 blocks, the last one whole, of one block or missing from the rows that see less; candidates of the
+    # rank's bin that fit LDS, that do not, and that share one score with a few others among them; a width that cuts a block and one of a
+    # single block.
+    rng = np.random.default_rng(blocks + rows)
+    ratio = 4
+    first = blocks * ratio - 1
+    n = (first + rows - 1) // ratio + 1
+    if kind == "uniform":
+        scores = rng.random((rows, n))
+    elif kind == "ties":
+        scores = np.where(rng.random((rows, n)) < 0.005, rng.random((rows, n)), np.where(rng.random((rows, n)) < 0.3, 1e-38, 0.0))
+    elif kind == "few":  # one score everywhere but for a few blocks of its bin
+        scores = np.where(rng.random((rows, n)) < 0.001, 1.01, 1.0)
+    elif kind == "signed":
+        scores = -np.abs(rng.standard_normal((rows, n)))
+        scores[:, ::3] = -0.0
+    else:
+        scores = np.maximum(rng.standard_normal((rows, n)), 0.0)
+    scores = scores.astype(np.float32)
+    both = _select(gpu_ctx, scores, rows, first, ratio, width)
+    _check_rows(both, scores, rows, first, ratio, width)
+    _, idx, cnt = _select(gpu_ctx, scores, rows, first, ratio, width, mask=False)
+    assert np.array_equal(cnt, both[2]) and all(np.array_equal(idx[r, :cnt[r]], both[1][r, :cnt[r]]) for r in range(rows))
+
+
+def test_long_rows_in_a_capture_without_the_workspace(gpu_ctx):
+    # Nothing is allocated inside a capture: a step's few rows are refused until an eager call has made the workspace, and more rows,
+    # which an eager call spreads, are recorded as a workgroup each, with the same results.
+    import torch
+    from tinytitan_amd import capi
+    from tinytitan_amd.engine import HIPContext
+    ctx = HIPContext(gpu_ctx.device)
+    rows, ratio, width, first = 9, 4, 131, 4 * 16500
+    last = first + rows - 1
+    n = last // ratio
+    scores = np.maximum(np.random.default_rng(3).standard_normal((rows, n)), 0).astype(np.float32)
+    sd = torch.from_numpy(scores).cuda()
+    idx = torch.full((rows, width), -1, dtype=torch.int32, device="cuda")
+    cnt = torch.full((rows,), -1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+
+    def call(k):
+        return _lib(ctx).tt_hip_qsa_select(ctx.handle, sd.data_ptr(), n, k, first, ratio, width, None, 0, idx.data_ptr(), width, cnt.data_ptr())
+
+    ctx.graph_begin()
+    assert call(7) == capi.ERR_BUSY
+    assert call(rows) == 0
+    graph = ctx.graph_end()
+    for _ in range(2):
+        idx.fill_(-1)
+        cnt.fill_(-1)
+        torch.cuda.synchronize()
+        graph.launch()
+        ctx.synchronize()
+        replayed, counts = idx.cpu().numpy(), cnt.cpu().numpy()
+        for r in range(rows):
+            _, _, want = oracle.qsa_select_keys(scores[r], first + r, ratio, width)
+            assert counts[r] == len(want) and np.array_equal(replayed[r, :counts[r]], want), r
+        idx.fill_(-1)
+        torch.cuda.synchronize()
+        assert call(7) == 0  # eager, spread
+        ctx.synchronize()
+        assert np.array_equal(idx.cpu().numpy()[:7], replayed[:7])
+    graph.close()
+    ctx.close()

@@ -130,8 +130,7 @@ struct tt_hip_ctx {
     size_t part_rows = 0;  // capacity in (seq, tile, split, n) rows
     _Float16 *stage_k = nullptr, *stage_v = nullptr;  // fp16 pages of one slot, dequantised for a prefill chunk
     size_t stage_elems = 0;                           // halves in each
-    void *select_ws = nullptr;  // histograms, bitmaps and candidate lists of the multi-workgroup key selection; zero between calls
-    size_t select_ws_bytes = 0;
+    void *select_ws = nullptr;  // the multi-workgroup key selection's sorted chunks and their tables
     uint8_t *keep_rows = nullptr;  // selection bytes written out from a chunk's index lists (tt_hip_attn_prefill_keep_indices)
     size_t keep_rows_bytes = 0;
     int split_override = 0;

@@ -22,6 +22,7 @@
 // one wavefront, eight-bit passes where that does not settle it: one workgroup per query row with
 // the row's scores in registers, or, for a few rows of very many blocks, many workgroups per row in
 // two launches.
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
@@ -1000,271 +1001,376 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
     if (a.counts && tid == 0) a.counts[row] = min(total + tail, width);
 }
 
-// ---- One query row over many workgroups: a decode step at a long context.
-// A single workgroup is one CU's arithmetic, and at 64 Ki blocks the passes above are some
-// hundred microseconds of it.  Here a row is cut into chunks of kChunkBlocks blocks, one
-// workgroup each, in two launches:
-//   1. every chunk adds its blocks to a histogram over the upper 12 bits of the orderable score;
-//   2. every chunk finds, from that histogram, the bin the block at rank B falls into (each for
-//      itself: 4096 counters), then settles its own blocks: a higher bin is a whole block, a
-//      lower one is dropped (mask bytes written, one bit per whole block into a bitmap), blocks
-//      of that bin go to a candidate list.  The chunk that finishes last (a counter; nobody
-//      waits) copies the bitmap to LDS, resolves the candidates with the radix select over their
-//      remaining bits -- they are the few blocks that share 12 bits with the answer, unless many
-//      scores tie -- writes their mask bytes, sets their bits, and reads the index list off the copy.
-// The workspace (histogram, counters) is zero between calls: the last chunk leaves it so.
+// ---- Query rows over many workgroups each.
+// A single workgroup is one CU's arithmetic, some fifty instructions a block.  Here a row is cut into chunks of up to 4,096
+// blocks, one workgroup each, in two launches that exchange nothing inside themselves:
+//   1. every chunk sorts its blocks by the upper 12 bits of the orderable score (a counting sort: counters in LDS, an exclusive
+//      sum over them) and leaves the sorted blocks -- the score's other 20 bits and the place in the chunk, one word each --
+//      with the table of where each of the 4,096 bins starts;
+//   2. every chunk adds the chunks' tables up -- at every 64th bin, then at the 64 bins behind the one it finds -- to the bin the
+//      row's block at rank B falls into, reads that bin's blocks of all chunks (a few hundred), finds the block at the
+//      rank among them, and settles its own blocks: mask bytes, and their places in the index list behind what the chunks
+//      before it keep.
+// No counter, flag or fence between workgroups: a histogram added up by atomics, candidate lists appended to and the last
+// workgroup to finish resolving them were 16.8 us for a row of 32,768 blocks, most of it such trips through memory (256
+// where most scores are equal); this is 11.3 (27).
 constexpr int kChunkThreads = 256;
-constexpr int kChunkKeys = 8;                                // per thread
-constexpr int kChunkBlocks = kChunkThreads * kChunkKeys;     // 2048
-constexpr int kBinBits = 12, kBins = 1 << kBinBits;
-constexpr int kMultiRows = 8;                                // rows a call may spread this way
-constexpr int kMaxSpreadBlocks = 262144;                     // blocks of a row whose bitmap the last chunk holds in LDS (32 KiB)
+constexpr int kBinBits = 12, kBins = 1 << kBinBits, kLowBits = 32 - kBinBits;
+constexpr int kMaxChunks = 64;            // of a row: a lane each
+constexpr unsigned kMaxChunkBlocks = 4096;  // places in a chunk have 12 bits
+constexpr int kMaxSpreadBlocks = kMaxChunks * (int)kMaxChunkBlocks;
+constexpr unsigned kHeldCandidates = 8192;  // in LDS
 
-struct MultiArgs {
+struct SpreadArgs {
     SelectArgs s;
-    unsigned *hist;                 // [rows][kBins]
-    unsigned long long *counters;   // [rows][2]: one word, candidates appended (low half) and chunks done (high half)
-    unsigned long long *bitmap;     // [rows][bitmap_words]: bit b of word w = block 64 w + b is kept whole
-    unsigned long long *candidates; // [rows][cand_stride] keys
-    long long bitmap_words, cand_stride;
+    int chunks;            // of the row that sees most
+    unsigned short *coarse;  // [rows][chunks][64]: blocks of the chunk in bins above (from the top) bin 64 l
+    unsigned short *starts;  // [rows][chunks][kBins]: ... above bin d
+    unsigned *sorted;        // [rows][chunks][chunk blocks]
 };
 
-__device__ __forceinline__ void chunk_keys(unsigned (&ok)[kChunkKeys], const float *scores, unsigned base, unsigned blocks, unsigned tid) {
+struct SpreadRow {
+    unsigned visible, complete, tail, blocks, B, partial;
+    // the host sends rows here only with visible > width >= ratio, so that B < blocks
+    __device__ __forceinline__ SpreadRow(const SelectArgs &s, unsigned row) {
+        visible = (unsigned)s.first_visible + row;
+        blocks = visible / (unsigned)s.ratio;
+        complete = blocks * (unsigned)s.ratio;
+        tail = visible - complete;
+        const unsigned remaining = (unsigned)s.width - tail;
+        B = remaining / (unsigned)s.ratio;
+        partial = remaining - B * (unsigned)s.ratio;
+    }
+};
+
+__device__ __forceinline__ unsigned bin_of(unsigned ok) { return (unsigned)kBins - 1u - (ok >> kLowBits); }  // counted from the top
+
+template <int KPT, int THREADS>
+__device__ __forceinline__ void chunk_keys(unsigned (&ok)[KPT], const float *scores, unsigned base, unsigned blocks, unsigned tid) {
 #pragma unroll
-    for (int j = 0; j < kChunkKeys; ++j) {
-        const unsigned i = base + (unsigned)j * kChunkThreads + tid;
+    for (int j = 0; j < KPT; ++j) {
+        const unsigned i = base + (unsigned)j * THREADS + tid;
         ok[j] = i < blocks ? orderable(scores[i]) : 0u;
     }
 }
 
-__global__ __launch_bounds__(kChunkThreads) void qsa_select_histogram_kernel(const MultiArgs a) {
-    __shared__ unsigned hist[kBins];
-    const unsigned tid = threadIdx.x, lane = tid & 63;
-    const long long row = blockIdx.y;
-    const unsigned visible = (unsigned)a.s.first_visible + (unsigned)row;
-    const unsigned blocks = visible / (unsigned)a.s.ratio;
-    const unsigned base = blockIdx.x * kChunkBlocks;
-    if (base >= blocks) return;
-    unsigned ok[kChunkKeys];
-    chunk_keys(ok, a.s.scores + row * a.s.score_stride, base, blocks, tid);
-    for (unsigned b = tid; b < kBins; b += kChunkThreads) hist[b] = 0;
+template <int CHUNK, int THREADS>
+__global__ __launch_bounds__(THREADS) void qsa_sort_chunks_kernel(const SpreadArgs a) {
+    constexpr int KPT = CHUNK / THREADS;
+    constexpr unsigned kOwn = kBins / THREADS, kWords = kOwn * (THREADS + 1);
+    static_assert(CHUNK <= (int)kMaxChunkBlocks && KPT * THREADS == CHUNK && (kOwn == 4 || kOwn == 16), "12 bits a place; a thread's bins leave in whole words");
+    // A thread owns neighbouring bins; neither their reads nor additions to neighbouring bins meet in a bank.
+    __shared__ unsigned counts[kWords];
+    __shared__ unsigned wave_totals[THREADS / 64];
+    auto slot = [](unsigned d) { return (d % kOwn) * (THREADS + 1u) + d / kOwn; };
+    const unsigned tid = threadIdx.x, row = blockIdx.y;
+    const SpreadRow r(a.s, row);
+    const unsigned base = blockIdx.x * (unsigned)CHUNK;
+    if (base >= r.blocks) return;
+    unsigned ok[KPT], place[KPT];
+    chunk_keys<KPT, THREADS>(ok, a.s.scores + (long long)row * a.s.score_stride, base, r.blocks, tid);
+#pragma unroll
+    for (unsigned u = 0; u <= kOwn; ++u)
+        if (u * THREADS + tid < kWords) counts[u * THREADS + tid] = 0u;
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kChunkKeys; ++j)
-        histogram_add(hist, ok[j] >> (32 - kBinBits), base + (unsigned)j * kChunkThreads + tid < blocks, lane);
+    for (int j = 0; j < KPT; ++j) {
+        place[j] = 0u;
+        if (base + (unsigned)j * THREADS + tid < r.blocks) place[j] = atomicAdd(&counts[slot(bin_of(ok[j]))], 1u);
+    }
     __syncthreads();
-    unsigned *out = a.hist + row * kBins;
-    for (unsigned b = tid; b < kBins; b += kChunkThreads) {
-        const unsigned n = hist[b];
-        if (n) atomicAdd(&out[b], n);
+    unsigned own[kOwn], sum = 0u, all;
+#pragma unroll
+    for (unsigned u = 0; u < kOwn; ++u) {
+        own[u] = counts[u * (THREADS + 1u) + tid];
+        sum += own[u];
+    }
+    unsigned before = workgroup_exclusive_sum<THREADS>(sum, wave_totals, all);
+    const size_t chunk = (size_t)row * (unsigned)a.chunks + blockIdx.x;
+    if ((tid * kOwn) % 64u == 0u) a.coarse[chunk * 64 + tid * kOwn / 64u] = (unsigned short)before;
+    unsigned packed[kOwn / 2];
+#pragma unroll
+    for (unsigned u = 0; u < kOwn; ++u) {
+        counts[u * (THREADS + 1u) + tid] = before;
+        packed[u / 2] = (u & 1u) ? packed[u / 2] | (before << 16) : before;
+        before += own[u];
+    }
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    u2 *const table = reinterpret_cast<u2 *>(a.starts + chunk * kBins + kOwn * tid);
+#pragma unroll
+    for (unsigned u = 0; u < kOwn / 4; ++u) table[u] = u2{packed[2 * u], packed[2 * u + 1]};
+    __syncthreads();
+    // (blocks behind the first B + 1 of their own chunk are nobody's candidates)
+    unsigned *const out = a.sorted + chunk * CHUNK;
+#pragma unroll
+    for (int j = 0; j < KPT; ++j) {
+        const unsigned local = (unsigned)j * THREADS + tid;
+        if (base + local >= r.blocks) continue;
+        const unsigned first = counts[slot(bin_of(ok[j]))];
+        if (first <= r.B) out[first + place[j]] = (ok[j] << kBinBits) | (kMaxChunkBlocks - 1u - local);
     }
 }
 
-__global__ __launch_bounds__(kChunkThreads) void qsa_select_settle_kernel(const MultiArgs a) {
+template <int KPT>
+__global__ __launch_bounds__(kChunkThreads) void qsa_settle_chunks_kernel(const SpreadArgs a) {
+    constexpr unsigned kChunk = KPT * kChunkThreads, kWaves = kChunkThreads / 64;
     __shared__ unsigned hist[256];
-    __shared__ unsigned wave_totals[kChunkThreads / 64];
-    __shared__ unsigned bin_sh, rank_sh, ticket_sh, n_cand_sh, candidates_sh, partial_block_sh;
-    __shared__ unsigned long long prefix_sh;
-    __shared__ unsigned long long bitmap_sh[kMaxSpreadBlocks / 64];  // the last chunk's copy of the row's bitmap
-    const unsigned tid = threadIdx.x, lane = tid & 63;
-    const long long row = blockIdx.y;
-    const unsigned ratio = (unsigned)a.s.ratio, width = (unsigned)a.s.width;
-    const unsigned visible = (unsigned)a.s.first_visible + (unsigned)row;
-    const unsigned complete = (visible / ratio) * ratio, tail = visible - complete, blocks = complete / ratio;
-    // the host sends a row here only with visible > width, width > tail and B < blocks
-    const unsigned remaining = width - tail, B = remaining / ratio, partial = remaining - B * ratio;
-    const float *scores = a.s.scores + row * a.s.score_stride;
-    uint8_t *keep = a.s.keep ? a.s.keep + row * a.s.keep_stride : nullptr;  // no mask asked for: the list alone
-    unsigned *g_hist = a.hist + row * kBins;
-    unsigned long long *counter = a.counters + row * 2;
-    unsigned long long *bitmap = a.bitmap + row * a.bitmap_words;
-    unsigned long long *cand = a.candidates + row * a.cand_stride;
-    const unsigned base = blockIdx.x * kChunkBlocks;
-    const unsigned n_chunks = (blocks + kChunkBlocks - 1) / kChunkBlocks;
-    if (blockIdx.x >= n_chunks) return;
-
-    unsigned ok[kChunkKeys];
-    chunk_keys(ok, scores, base, blocks, tid);  // in flight while the histogram is read
-    // The bin of the block at rank B: thread t owns the 16 bins below 4096 - 16 t, highest first.
-    constexpr int kOwn = kBins / kChunkThreads;
-    unsigned own[kOwn], own_sum = 0;
+    __shared__ unsigned wave_totals[kWaves];
+    __shared__ unsigned chunk_first[kMaxChunks], chunk_at[kMaxChunks];  // a chunk's first candidate among its sorted blocks, and in the row's list
+    __shared__ unsigned bin_sh, rank_sh, count_sh, n_listed_sh, prefix_sh, tie_chunk_sh, least_sh, most_sh;
+    __shared__ unsigned long long key_sh, listed[64];
+    __shared__ unsigned offsets[KPT * kWaves], words_sh[kHeldCandidates];
+    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, row = blockIdx.y, mine = blockIdx.x;
+    const SpreadRow r(a.s, row);
+    const unsigned base = mine * kChunk, ratio = (unsigned)a.s.ratio;
+    if (base >= r.blocks) return;
+    const unsigned n_chunks = (r.blocks + kChunk - 1u) / kChunk;
+    const size_t chunk0 = (size_t)row * (unsigned)a.chunks;
+    unsigned ok[KPT];
+    chunk_keys<KPT, kChunkThreads>(ok, a.s.scores + (long long)row * a.s.score_stride, base, r.blocks, tid);  // in flight while the tables are read
+    if (wave == 0) {
+        // The last bin with at most B blocks above it holds the block at rank B.
+        const unsigned short *coarse = a.coarse + chunk0 * 64 + lane, *starts = a.starts + chunk0 * kBins;
+        auto added_up = [&](const unsigned short *entry, unsigned stride) {  // the chunks' entries, sixteen on their way at a time
+            unsigned sum = 0u;
+            for (unsigned c0 = 0; c0 < n_chunks; c0 += 16u) {
+                unsigned got[16];
 #pragma unroll
-    for (int u = 0; u < kOwn; ++u) {
-        own[u] = g_hist[kBins - 1 - ((int)tid * kOwn + u)];
-        own_sum += own[u];
-    }
-    unsigned all;
-    unsigned above = workgroup_exclusive_sum<kChunkThreads>(own_sum, wave_totals, all);
-    if (above <= B && B < above + own_sum) {
+                for (unsigned u = 0; u < 16u; ++u) got[u] = entry[min(c0 + u, n_chunks - 1u) * stride];
 #pragma unroll
-        for (int u = 0; u < kOwn; ++u) {
-            if (above <= B && B < above + own[u]) {
-                bin_sh = kBins - 1 - ((int)tid * kOwn + u);
-                rank_sh = B - above;
+                for (unsigned u = 0; u < 16u; ++u) sum += c0 + u < n_chunks ? got[u] : 0u;
             }
-            above += own[u];
+            return sum;
+        };
+        const unsigned first = 64u * ((unsigned)__popcll(__ballot(added_up(coarse, 64u) <= r.B)) - 1u);
+        const unsigned above = added_up(starts + first + lane, (unsigned)kBins);
+        const unsigned last = (unsigned)__popcll(__ballot(above <= r.B)) - 1u, bin = first + last;
+        const unsigned rank = r.B - (unsigned)__builtin_amdgcn_readlane((int)above, (int)last);
+        unsigned begin = 0u, end = 0u;
+        if (lane < n_chunks) {
+            begin = starts[lane * (unsigned)kBins + bin];
+            end = bin + 1u < (unsigned)kBins ? (unsigned)starts[lane * (unsigned)kBins + bin + 1u] : min(kChunk, r.blocks - lane * kChunk);
+        }
+        const unsigned upto = wave_inclusive_sum(end - begin, lane);
+        chunk_first[lane] = begin;
+        chunk_at[lane] = upto - (end - begin);
+        if (lane == 63u) {
+            bin_sh = bin;
+            rank_sh = rank;
+            count_sh = upto;
+            n_listed_sh = 0u;
+            prefix_sh = 0u;
+            least_sh = ~0u;
+            most_sh = 0u;
         }
     }
     __syncthreads();
-    const unsigned bin = bin_sh;
-
-    const bool words = ratio == 4 && ((uintptr_t)keep & 3) == 0;
-    // a wavefront's candidates take one update of the list's counter (a trip to memory and back)
-    unsigned wave_candidates = 0;
+    // A candidate: its score's 20 low bits, then its inverted index -- larger is better, and no two are alike.
+    const unsigned n_candidates = (unsigned)__builtin_amdgcn_readfirstlane((int)count_sh);
+    auto key_of = [&](unsigned c, unsigned word) {  // of chunk c
+        return ((unsigned long long)(word >> kBinBits) << 32) | (unsigned long long)~(c * kChunk + (kMaxChunkBlocks - 1u - (word & (kMaxChunkBlocks - 1u))));
+    };
+    auto chunk_of = [&](unsigned n) {  // the last chunk whose candidates start no later than the n-th of all
+        unsigned c = 0u;
 #pragma unroll
-    for (int j = 0; j < kChunkKeys; ++j) {
-        const unsigned i = base + (unsigned)j * kChunkThreads + tid;
-        wave_candidates += (unsigned)__popcll(__ballot(i < blocks && (ok[j] >> (32 - kBinBits)) == bin));
-    }
-    unsigned at = 0;
-    if (wave_candidates) {
-        if (lane == 0) at = (unsigned)atomicAdd(counter, (unsigned long long)wave_candidates);
-        at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
-    }
-#pragma unroll
-    for (int j = 0; j < kChunkKeys; ++j) {
-        const unsigned i = base + (unsigned)j * kChunkThreads + tid;
-        const bool valid = i < blocks;
-        const unsigned key_bin = ok[j] >> (32 - kBinBits);
-        const bool whole = valid && key_bin > bin, candidate = valid && key_bin == bin;
-        const unsigned long long whole_mask = __ballot(whole), cand_mask = __ballot(candidate);
-        if (lane == 0 && (i >> 6) < a.bitmap_words) bitmap[i >> 6] = whole_mask;  // i is a multiple of 64 here
-        if (candidate) cand[at + (unsigned)__popcll(cand_mask & ((1ull << lane) - 1ull))] = ((unsigned long long)ok[j] << 32) | (unsigned long long)~i;
-        at += (unsigned)__popcll(cand_mask);
-        if (valid && !candidate && keep) {
-            if (words) *reinterpret_cast<unsigned *>(keep + 4ull * i) = whole ? 0x01010101u : 0u;
-            else for (unsigned c = 0; c < ratio; ++c) keep[(unsigned long long)i * ratio + c] = whole ? 1 : 0;
-        }
-    }
-    if (blockIdx.x == 0 && keep) {
-        for (unsigned c = complete + tid; c < visible; c += kChunkThreads) keep[c] = 1;
-        for (long long c = visible + tid; c < a.s.keep_stride; c += kChunkThreads) keep[c] = 0;
-    }
-    // Who finishes last goes on; everything written above is visible to it.  The counter's high half
-    // counts the chunks done; what its low half holds when the last chunk draws its number is the
-    // final count of candidates (every other chunk appended before it drew).
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) {
-        const unsigned long long drawn = atomicAdd(counter, 1ull << 32);
-        ticket_sh = (unsigned)(drawn >> 32);
-        n_cand_sh = (unsigned)drawn;
-    }
-    __syncthreads();
-    if (ticket_sh != n_chunks - 1) return;
-    __threadfence();
-
-    // The whole-block bits of every chunk, into LDS: the candidates kept whole join them there, and
-    // the index list is read off it.
-    const unsigned n_words = (blocks + 63) / 64;
-    for (unsigned w = tid; w < n_words; w += kChunkThreads)
-        bitmap_sh[w] = __hip_atomic_load(&bitmap[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // Radix select of the candidate at rank_sh over the bits below the bin: 4 bits, then 8 at a time.
-    const unsigned n_cand = n_cand_sh;
-    // Up to kChunkBlocks candidates are read once and stay in registers; more (many scores tie) are
-    // re-read in every pass.
-    const bool held = n_cand <= kChunkBlocks;
-    unsigned long long held_keys[kChunkKeys];
+        for (unsigned step = kMaxChunks / 2; step > 0u; step >>= 1)
+            if (c + step < n_chunks && chunk_at[c + step] <= n) c += step;
+        return c;
+    };
+    auto size = [&](unsigned c) { return (c + 1u < n_chunks ? chunk_at[c + 1u] : n_candidates) - chunk_at[c]; };
+    // Their words wait in LDS, one chunk's behind the other's; more than fit there (many scores are alike) are read again in
+    // every pass, a chunk's all at once and the next chunk's behind them.
+    const bool held = n_candidates <= kHeldCandidates;
     if (held) {
-#pragma unroll
-        for (int j = 0; j < kChunkKeys; ++j) {
-            const unsigned n = (unsigned)j * kChunkThreads + tid;
-            held_keys[j] = n < n_cand ? cand[n] : 0ull;
+#pragma unroll 2
+        for (unsigned n = tid; n < n_candidates; n += kChunkThreads) {
+            const unsigned c = chunk_of(n);
+            words_sh[n] = a.sorted[(chunk0 + c) * kChunk + chunk_first[c] + (n - chunk_at[c])];
         }
     }
-    auto for_each_candidate = [&](auto &&visit) {
-        if (held) {
+    auto for_each_candidate = [&](auto &&visit) {  // visit(score's low bits, of a chunk before this one, its key)
+        if (held) {  // (a thread reads the words it wrote)
+            const unsigned n_before = chunk_at[mine];
+            for (unsigned n = tid; n < n_candidates; n += kChunkThreads) {
+                const unsigned word = words_sh[n];
+                visit(word >> kBinBits, n < n_before, [&] { return key_of(chunk_of(n), word); });
+            }
+            return;
+        }
+        unsigned next[KPT];
+        auto load = [&](unsigned c) {
+            const unsigned n = size(c), *src = a.sorted + (chunk0 + c) * kChunk + chunk_first[c];
 #pragma unroll
-            for (int j = 0; j < kChunkKeys; ++j)
-                if ((unsigned)j * kChunkThreads + tid < n_cand) visit(held_keys[j]);
-        } else {
-            for (unsigned n = tid; n < n_cand; n += kChunkThreads) visit(cand[n]);
+            for (int j = 0; j < KPT; ++j) {
+                const unsigned at = (unsigned)j * kChunkThreads + tid;
+                next[j] = at < n ? src[at] : 0u;
+            }
+        };
+        load(0u);
+        for (unsigned c = 0; c < n_chunks; ++c) {
+            unsigned now[KPT];
+#pragma unroll
+            for (int j = 0; j < KPT; ++j) now[j] = next[j];
+            load(min(c + 1u, n_chunks - 1u));
+            const unsigned n = size(c);
+#pragma unroll
+            for (int j = 0; j < KPT; ++j)
+                if ((unsigned)j * kChunkThreads + tid < n) visit(now[j] >> kBinBits, c < mine, [&] { return key_of(c, now[j]); });
         }
     };
-    if (tid == 0) {
-        prefix_sh = (unsigned long long)bin << (64 - kBinBits);
-        candidates_sh = n_cand;
-        partial_block_sh = ~0u;
-    }
-    int pass = 6;
-    for (; pass >= 0; --pass) {
-        hist[tid] = 0;
+    // (so many are mostly one score, as where fewer blocks than the budget are above zero: one pass sees that there is nothing to tell apart)
+    bool one_score = false;
+    if (!held) {
+        unsigned least = ~0u, most = 0u;
+        for_each_candidate([&](unsigned score, bool, auto &&) {
+            least = min(least, score);
+            most = max(most, score);
+        });
+        most = wave_max(most, lane);
+        least = ~wave_max(~least, lane);
+        if (lane == 0) {
+            atomicMin(&least_sh, least);
+            atomicMax(&most_sh, most);
+        }
         __syncthreads();
-        const unsigned long long prefix = prefix_sh;
-        const unsigned rank = rank_sh;
-        if (candidates_sh == 1) break;
-        const unsigned shift = pass == 6 ? 48u : (unsigned)pass * 8u;
-        const unsigned digits = pass == 6 ? 0xFu : 0xFFu;
-        const unsigned long long fixed = pass == 6 ? (~0ull << (64 - kBinBits)) : (~0ull << (shift + 8u));
-        for_each_candidate([&](unsigned long long k) {
-            if ((k & fixed) == prefix) atomicAdd(&hist[(unsigned)(k >> shift) & digits], 1u);
+        one_score = least_sh == most_sh;
+        if (one_score && tid == 0) prefix_sh = least_sh;
+        __syncthreads();
+    }
+    // Radix passes over the score's 20 bits, eight at a time from the top, until a wavefront's worth of candidates share the rank's ...
+    unsigned shift = one_score ? 0u : (unsigned)kLowBits, fixed = one_score ? ~0u : 0u;
+    while (count_sh > 64u && shift > 0u) {
+        const unsigned bits = shift == 4u ? 4u : 8u;
+        shift -= bits;
+        hist[tid] = 0u;
+        __syncthreads();
+        const unsigned prefix = prefix_sh, rank = rank_sh;
+        for_each_candidate([&](unsigned score, bool, auto &&) {
+            histogram_add(hist, (score >> shift) & ((1u << bits) - 1u), (score & fixed) == prefix, lane);
         });
         __syncthreads();
-        if (tid < 64) {
+        if (wave == 0) {
             unsigned digit, rank_within, count;
             if (choose_digit(hist, rank, lane, digit, rank_within, count)) {
                 rank_sh = rank_within;
-                prefix_sh = prefix | ((unsigned long long)digit << shift);
-                candidates_sh = count;
+                prefix_sh = prefix | (digit << shift);
+                count_sh = count;
             }
         }
+        fixed = ~0u << shift;
         __syncthreads();
     }
-    if (pass >= 0) {
-        const unsigned long long prefix = prefix_sh;
-        const unsigned long long fixed = pass == 6 ? (~0ull << (64 - kBinBits)) : (~0ull << ((unsigned)pass * 8u + 8u));
-        __syncthreads();
-        for_each_candidate([&](unsigned long long k) {
-            if ((k & fixed) == prefix) prefix_sh = k;
+    const unsigned prefix = prefix_sh;
+    if (count_sh <= 64u) {
+        // ... which one wavefront then ranks: the lane whose key has `rank` larger ones holds the answer.
+        for_each_candidate([&](unsigned score, bool, auto &&key) {
+            if ((score & fixed) == prefix) listed[atomicAdd(&n_listed_sh, 1u)] = key();
         });
         __syncthreads();
-    }
-    const unsigned long long key = prefix_sh;
-    for_each_candidate([&](unsigned long long k) {
-        const unsigned i = ~(unsigned)k;
-        const bool whole = k > key, at_rank = k == key;
-        if (whole) atomicOr(reinterpret_cast<unsigned *>(bitmap_sh) + (i >> 5), 1u << (i & 31));  // little endian: bit i of the 64-bit words
-        if (at_rank) partial_block_sh = i;
-        if (!keep) return;
-        if (words) *reinterpret_cast<unsigned *>(keep + 4ull * i) = whole ? 0x01010101u : (at_rank ? (0x01010101u & ((1u << (8u * partial)) - 1u)) : 0u);
-        else for (unsigned c = 0; c < ratio; ++c) keep[(unsigned long long)i * ratio + c] = (whole || (at_rank && c < partial)) ? 1 : 0;
-    });
-    // leave the workspace zero for the next call
-    for (unsigned b = tid; b < kBins; b += kChunkThreads) g_hist[b] = 0;
-    if (tid == 0) *counter = 0ull;
-    unsigned *indices = a.s.indices ? a.s.indices + row * a.s.index_stride : nullptr;
-    if (!indices && !a.s.counts) return;
-    __syncthreads();
-    // The index list off the bitmap: a thread takes a run of words, counts its bits, and writes
-    // its blocks' cells behind those of the threads before it.
-    const unsigned per_thread = (n_words + kChunkThreads - 1) / kChunkThreads;
-    const unsigned first = min(n_words, tid * per_thread), last = min(n_words, first + per_thread);
-    unsigned bits = 0;
-    for (unsigned w = first; w < last; ++w) bits += (unsigned)__popcll(bitmap_sh[w]);
-    unsigned whole_blocks;
-    unsigned before = workgroup_exclusive_sum<kChunkThreads>(bits, wave_totals, whole_blocks);
-    const unsigned partial_block = partial_block_sh;
-    const unsigned total = whole_blocks * ratio + (partial_block != ~0u ? partial : 0u);
-    if (indices) {
-        for (unsigned w = first; w < last; ++w) {
-            unsigned long long m = bitmap_sh[w];
-            if (partial_block != ~0u && (partial_block >> 6) == w) {
-                // the cut block sits behind the whole blocks before it: those of earlier words, and the lower bits of this one
-                const unsigned rank = before + (unsigned)__popcll(m & ((1ull << (partial_block & 63)) - 1ull));
-                for (unsigned c = 0; c < partial; ++c) indices[rank * ratio + c] = partial_block * ratio + c;
-            }
-            while (m) {
-                const unsigned i = w * 64 + (unsigned)__ffsll((long long)m) - 1u;
-                m &= m - 1;
-                const unsigned at = before * ratio + ((partial_block != ~0u && i > partial_block) ? partial : 0u);
-                for (unsigned c = 0; c < ratio; ++c) indices[at + c] = i * ratio + c;
-                ++before;
+        if (wave == 0) {
+            const unsigned n = count_sh, rank = rank_sh;
+            const unsigned long long k = lane < n ? listed[lane] : 0ull;
+            unsigned larger = 0u;
+            for (unsigned m = 0; m < n; ++m) larger += listed[m] > k ? 1u : 0u;
+            if (lane < n && larger == rank) key_sh = k;
+        }
+        __syncthreads();
+    } else {
+        // More blocks than that with one score: the earliest are the best.  Each chunk's number of them says in which chunk the rank
+        // falls, and that chunk's scores, in order, which block it is.
+        hist[tid] = one_score && tid < n_chunks ? size(tid) : 0u;
+        __syncthreads();
+        if (!one_score) for_each_candidate([&](unsigned score, bool, auto &&key) {
+            if (score == prefix) atomicAdd(&hist[~(unsigned)key() / kChunk], 1u);
+        });
+        __syncthreads();
+        if (wave == 0) {
+            const unsigned rank = rank_sh, alike = hist[lane], upto = wave_inclusive_sum(alike, lane), at = upto - alike;
+            if (at <= rank && rank < upto) {
+                tie_chunk_sh = lane;
+                rank_sh = rank - at;
             }
         }
-        for (unsigned c = tid; c < tail; c += kChunkThreads)
-            if (total + c < width) indices[total + c] = complete + c;
+        __syncthreads();
+        const unsigned tied = (((unsigned)kBins - 1u - bin_sh) << kLowBits) | prefix, first = tie_chunk_sh * kChunk, rank = rank_sh;
+        unsigned other[KPT];
+        chunk_keys<KPT, kChunkThreads>(other, a.s.scores + (long long)row * a.s.score_stride, first, r.blocks, tid);
+        unsigned long long alike[KPT];
+#pragma unroll
+        for (int j = 0; j < KPT; ++j) {
+            alike[j] = __ballot(first + (unsigned)j * kChunkThreads + tid < r.blocks && other[j] == tied);
+            if (lane == 0) offsets[j * kWaves + wave] = (unsigned)__popcll(alike[j]);
+        }
+        __syncthreads();
+        unsigned all;
+        const unsigned word_at = workgroup_exclusive_sum<kChunkThreads>(tid < KPT * kWaves ? offsets[tid] : 0u, wave_totals, all);
+        if (tid < KPT * kWaves) offsets[tid] = word_at;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KPT; ++j)
+            if (((alike[j] >> lane) & 1ull) && offsets[j * kWaves + wave] + (unsigned)__popcll(alike[j] & ((1ull << lane) - 1ull)) == rank)
+                key_sh = ((unsigned long long)prefix << 32) | (unsigned long long)~(first + (unsigned)j * kChunkThreads + tid);
+        __syncthreads();
     }
-    if (a.s.counts && tid == 0) a.s.counts[row] = min(total + tail, width);
+    const unsigned long long key = key_sh;
+    const unsigned rank_block = ~(unsigned)key;
+    const unsigned rank_ok = (((unsigned)kBins - 1u - bin_sh) << kLowBits) | (unsigned)(key >> 32);
+
+    uint8_t *keep = a.s.keep ? a.s.keep + (long long)row * a.s.keep_stride : nullptr;  // no mask asked for: the list alone
+    unsigned *indices = a.s.indices ? a.s.indices + (long long)row * a.s.index_stride : nullptr;
+    const bool words = ratio == 4 && ((uintptr_t)keep & 3) == 0;
+    unsigned long long kept[KPT];  // of the wavefront's 64 blocks of every j: those kept whole
+#pragma unroll
+    for (int j = 0; j < KPT; ++j) {
+        const unsigned i = base + (unsigned)j * kChunkThreads + tid;
+        const bool valid = i < r.blocks, whole = valid && (ok[j] > rank_ok || (ok[j] == rank_ok && i < rank_block));
+        kept[j] = __ballot(whole);
+        if (valid && keep) {
+            const unsigned cells = whole ? ratio : i == rank_block ? r.partial : 0u;
+            if (words) *reinterpret_cast<unsigned *>(keep + 4ull * i) = cells == 4u ? 0x01010101u : 0x01010101u & ((1u << (8u * cells)) - 1u);
+            else for (unsigned c = 0; c < ratio; ++c) keep[(unsigned long long)i * ratio + c] = c < cells ? 1 : 0;
+        }
+    }
+    if (mine == 0) {
+        if (keep) {
+            for (unsigned c = r.complete + tid; c < r.visible; c += kChunkThreads) keep[c] = 1;
+            for (long long c = (long long)r.visible + tid; c < a.s.keep_stride; c += kChunkThreads) keep[c] = 0;
+        }
+        // exactly B blocks are larger than the one at rank B
+        if (indices)
+            for (unsigned c = tid; c < r.tail; c += kChunkThreads) indices[r.B * ratio + r.partial + c] = r.complete + c;
+        if (a.s.counts && tid == 0) a.s.counts[row] = (unsigned)a.s.width;
+    }
+    if (!indices) return;
+    // Whole blocks of the chunks before this one: what they hold above the bin, and their candidates above the rank.
+    unsigned earlier = tid < mine ? chunk_first[tid] : 0u, before;
+    if (one_score) {  // the blocks before the rank's
+        if (tid == 0) earlier += mine <= tie_chunk_sh ? chunk_at[mine] : chunk_at[tie_chunk_sh] + rank_sh;
+    } else {
+        const unsigned score = (unsigned)(key >> 32);
+        for_each_candidate([&](unsigned s, bool before_mine, auto &&its_key) {
+            if (before_mine && s >= score) earlier += s > score || its_key() > key ? 1u : 0u;
+        });
+    }
+    (void)workgroup_exclusive_sum<kChunkThreads>(earlier, wave_totals, before);
+    if (lane == 0)
+#pragma unroll
+        for (int j = 0; j < KPT; ++j) offsets[j * kWaves + wave] = (unsigned)__popcll(kept[j]);
+    __syncthreads();
+    const unsigned word_blocks = tid < KPT * kWaves ? offsets[tid] : 0u;
+    unsigned all;
+    const unsigned word_at = before + workgroup_exclusive_sum<kChunkThreads>(word_blocks, wave_totals, all);
+    if (tid < KPT * kWaves) offsets[tid] = word_at;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < KPT; ++j) {
+        const unsigned i = base + (unsigned)j * kChunkThreads + tid;
+        const bool whole = (kept[j] >> lane) & 1ull;
+        if (!whole && i != rank_block) continue;
+        const unsigned rank = offsets[j * kWaves + wave] + (unsigned)__popcll(kept[j] & ((1ull << lane) - 1ull));
+        const unsigned at = rank * ratio + (i > rank_block ? r.partial : 0u), cells = whole ? ratio : r.partial;
+        for (unsigned c = 0; c < cells; ++c) indices[at + c] = i * ratio + c;
+    }
 }
 
 void fill_frequencies(RowsArgs &a, int head_dim, float theta) {
@@ -1465,23 +1571,27 @@ extern "C" int tt_hip_qsa_block_scores(tt_hip_ctx *ctx, const tt_half *query, co
     return timed.finish("qsa_scores_kernel launch");
 }
 
-// Workspace of the multi-workgroup selection, zeroed when allocated and left zero by every call.
-static int ensure_select_workspace(tt_hip_ctx *ctx, size_t bytes) {
-    if (bytes <= ctx->select_ws_bytes) return TT_HIP_OK;
-    if (ctx->capturing) return TT_HIP_ERR_BUSY;  // allocating would synchronise inside a capture
-    hipError_t e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
-    if (ctx->select_ws) (void)hipFree(ctx->select_ws);
-    ctx->select_ws = nullptr;
-    ctx->select_ws_bytes = 0;
-    ++ctx->generation;
-    e = hipMalloc(&ctx->select_ws, bytes);
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc(selection workspace)");
-    // on the stream the selection kernels run on (created non-blocking: the null stream orders nothing with it)
-    e = hipMemsetAsync(ctx->select_ws, 0, bytes, ctx->stream);
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMemsetAsync(selection workspace)");
-    ctx->select_ws_bytes = bytes;
+// Workspace of the multi-workgroup selection, of one size for the context's life (its rows go as many at a time as fit: 340 of
+// 32,768 blocks): every call writes what it reads.
+constexpr size_t kSelectWorkspace = (size_t)64 << 20;
+constexpr int kFewRows = 8;  // rows of a decode or verify step, which are not selected without it
+static int ensure_select_workspace(tt_hip_ctx *ctx) {
+    if (ctx->select_ws) return TT_HIP_OK;
+    if (ctx->capturing) return TT_HIP_ERR_BUSY;  // no allocation inside a capture
+    const hipError_t e = hipMalloc(&ctx->select_ws, kSelectWorkspace);
+    if (e != hipSuccess) {
+        ctx->select_ws = nullptr;
+        return hip_fail(ctx, e, "hipMalloc(selection workspace)");
+    }
     return TT_HIP_OK;
+}
+
+template <int KPT>
+static void launch_spread(tt_hip_ctx *ctx, const SpreadArgs &m, unsigned chunks, unsigned rows) {
+    // (a chunk per CU: as many wavefronts as it takes; several a CU: fewer barriers)
+    if ((long long)chunks * rows <= ctx->n_cus) hipLaunchKernelGGL((qsa_sort_chunks_kernel<KPT * kChunkThreads, 1024>), dim3(chunks, rows), dim3(1024), 0, ctx->stream, m);
+    else hipLaunchKernelGGL((qsa_sort_chunks_kernel<KPT * kChunkThreads, kChunkThreads>), dim3(chunks, rows), dim3(kChunkThreads), 0, ctx->stream, m);
+    hipLaunchKernelGGL(qsa_settle_chunks_kernel<KPT>, dim3(chunks, rows), dim3(kChunkThreads), 0, ctx->stream, m);
 }
 
 extern "C" int tt_hip_qsa_select(tt_hip_ctx *ctx, const float *scores, size_t score_stride, int rows, int first_visible,
@@ -1514,38 +1624,48 @@ extern "C" int tt_hip_qsa_select(tt_hip_ctx *ctx, const float *scores, size_t sc
     // blocks of the row that sees most; a thread of the register form holds 1, 4, 16, 32 or 64 of them
     const long long max_blocks = last_visible / ratio;
     const dim3 grid((unsigned)rows), wg(kSelectThreads);
-    // A few rows with many blocks each (a decode or verify step at a long context) spread over many
-    // workgroups, provided every row has a real selection to make (B < blocks, see the kernel).  The
-    // two launches and their trips through memory cost about what one workgroup needs for 16 Ki blocks.
-    // (more rows run side by side as workgroups of their own: 8 rows of 32,768 blocks 43.3 us that way, 47.1 us spread;
-    // 4 rows of 17,500 blocks the same either way)
-    bool spread = rows <= kMultiRows && max_blocks > 16LL * kSelectThreads * (rows >= 8 ? 2 : 1) && max_blocks <= kMaxSpreadBlocks;
-    for (int r = 0; r < rows && spread; ++r) {
-        const long long visible = (long long)first_visible + r, complete = visible / ratio * ratio, tail = visible - complete;
-        spread = visible > width && width > tail && (width - tail) / ratio < complete / ratio;
-    }
+    // Rows with many blocks each spread over many workgroups, provided every row has a real selection to make (B < blocks).
+    // A workgroup per row is its CU's arithmetic (16,385 to 32,768 blocks 19.5 us, up to 65,536 34, whatever the rows, while
+    // they find a CU each); spread, every block is handled twice and the launch's work goes over all CUs: 1 row of 32,768
+    // blocks 16.8 -> 11.3 us, 4 rows 24.7 -> 13.9, 64 rows 22.0 -> 19.8, 64 rows of 50,000 33.8 -> 25.1; 128 rows of 20,000 19.6
+    // against 23.7, of 32,768 35.0 against 36.9.  Beyond 65,536 blocks a row's scores do not fit its workgroup's registers (128
+    // rows of 100,000 520 -> 119 us).
+    const long long all_blocks = (long long)rows * max_blocks;
+    const bool pays = max_blocks > 64ll * kSelectThreads || (max_blocks > 16ll * kSelectThreads && 4 * rows <= ctx->n_cus);
+    const bool spread = pays && max_blocks <= kMaxSpreadBlocks && first_visible > width && width >= ratio;
     if (spread) {
-        const long long chunks = (max_blocks + kChunkBlocks - 1) / kChunkBlocks;
-        MultiArgs m{};
-        m.s = a;
-        m.bitmap_words = chunks * (kChunkBlocks / 64);
-        m.cand_stride = chunks * kChunkBlocks;
-        const size_t hist_bytes = (size_t)kMultiRows * kBins * 4, counter_bytes = (size_t)kMultiRows * 16;
-        const size_t bitmap_bytes = (size_t)rows * m.bitmap_words * 8, cand_bytes = (size_t)rows * m.cand_stride * 8;
-        const int st = ensure_select_workspace(ctx, hist_bytes + counter_bytes + bitmap_bytes + cand_bytes);
-        if (st != TT_HIP_OK) return st;
-        // The histograms and counters must be zero when a call starts, so they sit first, at offsets that
-        // do not depend on the call; bitmap and candidates behind them are written before they are read.
-        uint8_t *ws = static_cast<uint8_t *>(ctx->select_ws);
-        m.hist = reinterpret_cast<unsigned *>(ws);
-        m.counters = reinterpret_cast<unsigned long long *>(ws + hist_bytes);
-        m.bitmap = reinterpret_cast<unsigned long long *>(ws + hist_bytes + counter_bytes);
-        m.candidates = reinterpret_cast<unsigned long long *>(ws + hist_bytes + counter_bytes + bitmap_bytes);
-        const dim3 chunk_grid((unsigned)chunks, (unsigned)rows), chunk_wg(kChunkThreads);
-        Timed timed(ctx);
-        hipLaunchKernelGGL(qsa_select_histogram_kernel, chunk_grid, chunk_wg, 0, ctx->stream, m);
-        hipLaunchKernelGGL(qsa_select_settle_kernel, chunk_grid, chunk_wg, 0, ctx->stream, m);
-        return timed.finish("qsa_select_settle_kernel launch");
+        // (chunks of 2,048 while their workgroups are few: 16 rows of 20,000 blocks 14.0 us against 19.0 in chunks of 4,096, 64 rows of
+        // 65,536 31.4 against 25.9; a row has at most 64 chunks)
+        const int kpt = max_blocks > kMaxChunks * 8ll * kChunkThreads || all_blocks > 2ll << 20 ? 16 : 8;
+        const long long chunk = (long long)kpt * kChunkThreads, chunks = (max_blocks + chunk - 1) / chunk;
+        const size_t per_row = (size_t)chunks * (kBins * 2 + 64 * 2 + (size_t)chunk * 4);
+        static_assert(kMaxChunks * (kBins * 2 + 64 * 2 + (size_t)kMaxChunkBlocks * 4) <= kSelectWorkspace, "a row fits");
+        const int rows_at_once = (int)std::min<size_t>((size_t)rows, kSelectWorkspace / per_row);
+        const int st = ensure_select_workspace(ctx);
+        if (st == TT_HIP_OK) {
+            Timed timed(ctx);
+            for (int r0 = 0; r0 < rows; r0 += rows_at_once) {
+                const int n = std::min(rows_at_once, rows - r0);
+                SpreadArgs m{};
+                m.s = a;
+                m.s.scores += (long long)r0 * a.score_stride;
+                if (keep) m.s.keep += (long long)r0 * a.keep_stride;
+                if (indices) m.s.indices += (long long)r0 * a.index_stride;
+                if (counts) m.s.counts += r0;
+                m.s.first_visible += r0;
+                m.chunks = (int)chunks;
+                uint8_t *ws = static_cast<uint8_t *>(ctx->select_ws);
+                m.starts = reinterpret_cast<unsigned short *>(ws);
+                m.coarse = m.starts + (size_t)n * chunks * kBins;
+                m.sorted = reinterpret_cast<unsigned *>(m.coarse + (size_t)n * chunks * 64);
+                if (kpt == 8) launch_spread<8>(ctx, m, (unsigned)chunks, (unsigned)n);
+                else launch_spread<16>(ctx, m, (unsigned)chunks, (unsigned)n);
+            }
+            return timed.finish("qsa_settle_chunks_kernel launch");
+        }
+        // Without the workspace (a capture before any eager call, no memory): a decode or verify step's few rows are refused, as the
+        // header says, rather than recorded as a workgroup each for every replay; all others take the forms below.
+        if (rows <= kFewRows && max_blocks > (rows == kFewRows ? 32ll : 16ll) * kSelectThreads) return st;
     }
     Timed timed(ctx);
     // Many rows (a long chunk) fill the chip by themselves: workgroups of 256 threads spend less of their time in
