@@ -740,3 +740,33 @@ def test_long_rows_in_a_capture_without_the_workspace(gpu_ctx):
         assert np.array_equal(idx.cpu().numpy()[:7], replayed[:7])
     graph.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("blocks,width,kind", [(16384, 2051, "normal"), (16385, 2051, "normal"), (32769, 2050, "normal"), (65536, 7, "normal"),
+                                               (20000, 2560, "normal"), (20000, 2564, "normal"), (9000, 2049, "half"), (30000, 2051, "lanes"),
+                                               (40000, 2051, "last"), (30000, 2051, "ties"), (30000, 2051, "inf")])
+def test_long_rows_thinned_to_a_block_a_thread(gpu_ctx, blocks, width, kind):
+    # A workgroup per row whose blocks are cut down by the threads' largest ones first: at the edges of 16, 32 and 64 blocks a thread,
+    # at the largest selection that is (640 blocks) and one beyond; rows that go on whole because their largest blocks belong to few
+    # threads, because too many are alike, or because the best are one score.
+    rng = np.random.default_rng(blocks + width)
+    ratio, rows = 4, 67
+    first = blocks * ratio - rows + 2
+    n = blocks + 1
+    scores = rng.standard_normal((rows, n))
+    if kind == "half":
+        scores = np.maximum(scores, 0.0)
+    elif kind == "lanes":  # (thread t holds blocks t, t + 1024, ...)
+        scores[:, np.arange(n) % 1024 < 20] += 10.0
+    elif kind == "last":
+        scores[:, -3:] += 10.0
+    elif kind == "ties":
+        scores = np.where(rng.random((rows, n)) < 0.01, 2.0, 1.0)
+    elif kind == "inf":
+        scores = np.where(rng.random((rows, n)) < 0.001, np.inf, scores)
+        scores[:, ::7] = -np.inf
+    scores = scores.astype(np.float32)
+    both = _select(gpu_ctx, scores, rows, first, ratio, width)
+    _check_rows(both, scores, rows, first, ratio, width)
+    _, idx, cnt = _select(gpu_ctx, scores, rows, first, ratio, width, mask=False)
+    assert np.array_equal(cnt, both[2]) and all(np.array_equal(idx[r, :cnt[r]], both[1][r, :cnt[r]]) for r in range(rows))

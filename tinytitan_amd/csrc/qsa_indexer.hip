@@ -445,6 +445,18 @@ __device__ __forceinline__ unsigned opaque(unsigned x) {
     return x;
 }
 
+// The orderable scores of blocks base + tid, base + THREADS + tid, ...; 0 past the last of `blocks` (there is one).  Every place is
+// loaded, past the end the last block again: loads under a condition each were waited for one by one, a trip to memory
+// for every 1,024 blocks of a row (128 rows of 32,000 blocks 27.4 -> 21.0 us).
+template <int KPT, int THREADS>
+__device__ __forceinline__ void load_keys(unsigned (&ok)[KPT], const float *scores, unsigned base, unsigned blocks, unsigned tid) {
+    float x[KPT];
+#pragma unroll
+    for (int j = 0; j < KPT; ++j) x[j] = scores[min(base + (unsigned)j * THREADS + tid, blocks - 1u)];
+#pragma unroll
+    for (int j = 0; j < KPT; ++j) ok[j] = base + (unsigned)j * THREADS + tid < blocks ? orderable(x[j]) : 0u;
+}
+
 // Exclusive prefix sum of one value per thread over a workgroup of THREADS threads; `total`
 // receives the sum.  Two barriers.
 // The largest value of the 64 lanes, in every lane: the same moves as the sum below, then lane 63's.
@@ -747,51 +759,50 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
     const unsigned complete = (visible / ratio) * ratio;
     const unsigned tail = visible - complete;
     const unsigned blocks = complete / ratio;
-    unsigned ok[KPT];
-#pragma unroll
-    for (int j = 0; j < KPT; ++j) {
-        const unsigned i = (unsigned)j * THREADS + tid;
-        ok[j] = i < blocks ? orderable(scores[i]) : 0u;
-    }
+    unsigned ok[KPT] = {};
+    if (blocks > 0u) load_keys<KPT, THREADS>(ok, scores, 0u, blocks, tid);
     if (keep)
         for (unsigned c = complete + tid; c < visible; c += THREADS) keep[c] = 1;
     const unsigned remaining = width > tail ? width - tail : 0;
     const unsigned B = remaining / ratio;
     unsigned partial = remaining - B * ratio;
-    // (key_hi, key_lo): the key of the block at rank B; larger keys are whole blocks.  rank_block: that block, or none
-    unsigned key_hi, key_lo, rank_block = ~0u;
-    if (remaining == 0) {
-        key_hi = key_lo = ~0u;
-    } else if (B >= blocks) {
-        key_hi = key_lo = 0u;  // every key is larger: its low word, the inverted index, is never 0
-        partial = 0;
-    } else {
+    // The upper 16 bits of the workgroup's largest value (one barrier; wave_totals is free again behind the next one).
+    auto upper_bits_of_largest = [&](unsigned x) {
+        x = wave_max(x >> 16, lane);
+        if (lane == 0) wave_totals[wave] = x;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < THREADS / 64; ++w) x = max(x, wave_totals[w]);
+        return x;
+    };
+    auto largest_of = [](const auto &keys) {
+        unsigned x = 0u;
+        for (const unsigned key : keys) x = max(x, key);  // (a place without a block holds 0)
+        return x;
+    };
+    // (prefix_hi_sh, prefix_lo_sh): the key at rank B of n_keys, which a thread holds the upper words of; block_of(j, thread) is
+    // keys[j]'s block, or no block at all.  top16: the largest one's upper 16 bits where they are known.
+    auto search = [&](const auto &keys, auto &&block_of, unsigned n_keys, unsigned top16) {
+        constexpr int N = (int)(sizeof(keys) / sizeof(unsigned));
         if (tid == 0) {
             prefix_hi_sh = 0u;
             prefix_lo_sh = 0u;
             rank_sh = B;
-            candidates_sh = blocks;
+            candidates_sh = n_keys;
             wide_found_sh = 0u;
             n_listed_sh = 0u;
         }
         // The score's two upper bytes at once (see choose_wide); the 8-bit passes go on from the third byte, or from
         // the first when the rank lies below the window.
-        unsigned top16 = 0u;
-#pragma unroll
-        for (int j = 0; j < KPT; ++j)
-            if ((unsigned)j * THREADS + tid < blocks) top16 = max(top16, ok[j] >> 16);
-        top16 = wave_max(top16, lane);
-        if (lane == 0) wave_totals[wave] = top16;
+        if (top16 == 0u) top16 = upper_bits_of_largest(largest_of(keys));
         for (unsigned b = tid; b < kWideBins; b += THREADS) wide[b] = 0u;
         __syncthreads();
-#pragma unroll
-        for (int w = 0; w < THREADS / 64; ++w) top16 = max(top16, wave_totals[w]);
         {
             const unsigned tid = opaque(threadIdx.x);
 #pragma unroll
-            for (int j = 0; j < KPT; ++j) {
-                const unsigned r = top16 - (ok[j] >> 16);
-                if ((unsigned)j * THREADS + tid < blocks && r < kWideBins) atomicAdd(&wide[wide_slot(r)], 1u);
+            for (int j = 0; j < N; ++j) {
+                const unsigned r = top16 - (keys[j] >> 16);
+                if (block_of(j, tid) < blocks && r < kWideBins) atomicAdd(&wide[wide_slot(r)], 1u);
             }
         }
         __syncthreads();
@@ -814,9 +825,9 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
             const unsigned prefix16 = prefix_hi_sh >> 16;
             const unsigned tid = opaque(threadIdx.x);
 #pragma unroll
-            for (int j = 0; j < KPT; ++j) {
-                const unsigned i = (unsigned)j * THREADS + tid;
-                const bool match = i < blocks && (ok[j] >> 16) == prefix16;
+            for (int j = 0; j < N; ++j) {
+                const unsigned i = block_of(j, tid);
+                const bool match = i < blocks && (keys[j] >> 16) == prefix16;
                 const unsigned long long m = __ballot(match);
                 if (m != 0ull) {
                     const int lead = __ffsll((long long)m) - 1;
@@ -824,7 +835,7 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
                     if (lane == (unsigned)lead) at = atomicAdd(&n_listed_sh, (unsigned)__popcll(m));
                     at = (unsigned)__builtin_amdgcn_readlane((int)at, lead) + (unsigned)__popcll(m & ((1ull << lane) - 1ull));
                     if (match) {
-                        listed_hi[at] = ok[j];
+                        listed_hi[at] = keys[j];
                         listed_lo[at] = ~i;
                     }
                 }
@@ -857,10 +868,10 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
             const unsigned shift = (unsigned)(pass & 3) * 8u;
             const unsigned fixed = (pass & 3) == 3 ? 0u : (~0u << (shift + 8u));  // digits of this word already chosen
 #pragma unroll
-            for (int j = 0; j < KPT; ++j) {
-                const unsigned i = (unsigned)j * THREADS + tid;
-                const unsigned word = high ? ok[j] : ~i;
-                const bool match = i < blocks && (high ? (word & fixed) == prefix_hi : (ok[j] == prefix_hi && (word & fixed) == prefix_lo));
+            for (int j = 0; j < N; ++j) {
+                const unsigned i = block_of(j, tid);
+                const unsigned word = high ? keys[j] : ~i;
+                const bool match = i < blocks && (high ? (word & fixed) == prefix_hi : (keys[j] == prefix_hi && (word & fixed) == prefix_lo));
                 histogram_add(hist, (word >> shift) & 0xFFu, match, lane);
             }
             __syncthreads();
@@ -883,15 +894,69 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
             __syncthreads();
             const unsigned tid = opaque(threadIdx.x);
 #pragma unroll
-            for (int j = 0; j < KPT; ++j) {
-                const unsigned i = (unsigned)j * THREADS + tid;
-                if (i < blocks && (ok[j] & fixed_hi) == prefix_hi && (~i & fixed_lo) == prefix_lo) {
-                    prefix_hi_sh = ok[j];
+            for (int j = 0; j < N; ++j) {
+                const unsigned i = block_of(j, tid);
+                if (i < blocks && (keys[j] & fixed_hi) == prefix_hi && (~i & fixed_lo) == prefix_lo) {
+                    prefix_hi_sh = keys[j];
                     prefix_lo_sh = ~i;
                 }
             }
             __syncthreads();
         }
+    };
+    // Rows of many blocks are thinned first: B < THREADS blocks are wanted, and the largest block of B + 1 threads is no smaller
+    // than the threads' B-th largest, so nothing below that is: seven hundred blocks are left of 8,192 or of 65,536 for the usual 512
+    // of 1,024 threads, a thread takes one of them, and what was a pass over all of the row's blocks is one over these: 128 rows
+    // of 16,000 / 32,000 / 60,000 blocks 14.0 -> 13.4, 21.0 -> 16.2, 34.9 -> 23.0 us; with a mask, which is a pass over all blocks again, 15.7
+    // -> 16.0, 23.6 -> 20.9, 39.6 -> 31.3, and 8,000 blocks 11.5 -> 12.4.  (More than a thread each, as where most scores are alike:
+    // the row goes on whole.)
+    constexpr bool kThins = THREADS == kSelectThreads && KPT >= 16;
+    constexpr unsigned kThinnedRanks = THREADS * 5 / 8;  // (expected to leave no more than 990)
+    bool thinned = false;
+    unsigned top16 = 0u, candidate = ~0u, candidate_key[1] = {0u}, n_candidates = 0u;
+    auto thin = [&] {
+        const unsigned largest = largest_of(ok);
+        if (tid == 0) wide_found_sh = 0u;
+        for (unsigned b = tid; b < kWideBins; b += THREADS) wide[b] = 0u;
+        top16 = upper_bits_of_largest(largest);
+        const unsigned r = top16 - (largest >> 16);
+        if (r < kWideBins) atomicAdd(&wide[wide_slot(r)], 1u);
+        __syncthreads();
+        if (wave == 0) {
+            unsigned bin, rank_within, count;
+            if (choose_wide(wide, B, lane, bin, rank_within, count)) wide_found_sh = (top16 - bin) << 16;
+        }
+        __syncthreads();
+        const unsigned least = wide_found_sh;
+        if (least == 0u) return false;
+        unsigned long long mine = 0ull;
+#pragma unroll
+        for (int j = 0; j < KPT; ++j) mine |= ok[j] >= least ? 1ull << j : 0ull;
+        unsigned at = workgroup_exclusive_sum<THREADS>((unsigned)__popcll(mine), wave_totals, n_candidates);
+        if (n_candidates > (unsigned)THREADS) return false;
+        for (; mine != 0ull; mine &= mine - 1ull) wide[at++] = (unsigned)(__ffsll((long long)mine) - 1) * THREADS + tid;
+        for (unsigned w = tid; w < 2u * KPT * (THREADS / 64); w += THREADS) reinterpret_cast<unsigned *>(bitmap_sh)[w] = 0u;
+        __syncthreads();
+        if (tid < n_candidates) {
+            candidate = wide[tid];
+            candidate_key[0] = orderable(scores[candidate]);
+        }
+        __syncthreads();
+        return true;
+    };
+    // (key_hi, key_lo): the key of the block at rank B; larger keys are whole blocks.  rank_block: that block, or none
+    unsigned key_hi, key_lo, rank_block = ~0u;
+    if (remaining == 0) {
+        key_hi = key_lo = ~0u;
+    } else if (B >= blocks) {
+        key_hi = key_lo = 0u;  // every key is larger: its low word, the inverted index, is never 0
+        partial = 0;
+    } else {
+        if constexpr (kThins) {
+            if (B <= kThinnedRanks && (KPT >= 32 || !keep)) thinned = thin();
+        }
+        if (thinned) search(candidate_key, [&](int, unsigned) { return candidate; }, n_candidates, top16);
+        else search(ok, [&](int j, unsigned thread) { return (unsigned)j * THREADS + thread; }, blocks, top16);
         key_hi = prefix_hi_sh;
         key_lo = prefix_lo_sh;
         rank_block = ~key_lo;  // the key is a block's: its low word is that block's inverted index
@@ -904,14 +969,10 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
     if (tid == 0) partial_block_sh = rank_block;
     __syncthreads();
     const unsigned tid_mask = opaque(threadIdx.x);
-    unsigned ballots_lo = 0u, ballots_hi = 0u;
-#pragma unroll
-    for (int j = 0; j < KPT; ++j) {
-        const unsigned i = (unsigned)j * THREADS + tid_mask;
-        const bool valid = i < blocks;
-        const bool whole = valid && (ok[j] > key_hi || (ok[j] == key_hi && ~i > key_lo));
+    auto larger = [&](unsigned key, unsigned i) { return i < blocks && (key > key_hi || (key == key_hi && ~i > key_lo)); };
+    auto write_cells = [&](unsigned i, bool whole) {
         const bool at_rank = i == rank_block;
-        if (valid && keep) {
+        if (i < blocks && keep) {
             if (words) {
                 const unsigned cells = whole ? 0x01010101u : (at_rank ? (0x01010101u & ((1u << (8u * partial)) - 1u)) : 0u);
                 *reinterpret_cast<unsigned *>(keep + 4ull * i) = cells;
@@ -919,15 +980,31 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
                 for (unsigned c = 0; c < ratio; ++c) keep[(unsigned long long)i * ratio + c] = (whole || (at_rank && c < partial)) ? 1 : 0;
             }
         }
-        if (listing) {
-            const unsigned long long m = __ballot(whole);
-            ballots_lo = lane == (unsigned)j ? (unsigned)m : ballots_lo;
-            ballots_hi = lane == (unsigned)j ? (unsigned)(m >> 32) : ballots_hi;
+    };
+    if (thinned) {  // (no other block is larger; the bitmap was cleared)
+        unsigned *const bits = reinterpret_cast<unsigned *>(bitmap_sh);
+        if (larger(candidate_key[0], candidate)) atomicOr(&bits[candidate / 32u], 1u << (candidate % 32u));
+        __syncthreads();
+        if (keep)
+            for (unsigned i = tid_mask; i < blocks; i += THREADS) write_cells(i, ((bits[i / 32u] >> (i % 32u)) & 1u) != 0u);
+        if (!listing) return;
+    } else {
+        unsigned ballots_lo = 0u, ballots_hi = 0u;
+#pragma unroll
+        for (int j = 0; j < KPT; ++j) {
+            const unsigned i = (unsigned)j * THREADS + tid_mask;
+            const bool whole = larger(ok[j], i);
+            write_cells(i, whole);
+            if (listing) {
+                const unsigned long long m = __ballot(whole);
+                ballots_lo = lane == (unsigned)j ? (unsigned)m : ballots_lo;
+                ballots_hi = lane == (unsigned)j ? (unsigned)(m >> 32) : ballots_hi;
+            }
         }
+        if (!listing) return;
+        if (lane < (unsigned)KPT) bitmap_sh[lane * (THREADS / 64) + wave] = ((unsigned long long)ballots_hi << 32) | ballots_lo;
+        __syncthreads();
     }
-    if (!listing) return;
-    if (lane < (unsigned)KPT) bitmap_sh[lane * (THREADS / 64) + wave] = ((unsigned long long)ballots_hi << 32) | ballots_lo;
-    __syncthreads();
     // The kept cells ascending: word (j, wavefront) covers blocks j THREADS + 64 wavefront ..., so the words
     // in storage order are the blocks in order.  One word per thread: count, exclusive sum, then the set bits.
     constexpr unsigned kWords = KPT * (THREADS / 64);
@@ -1045,15 +1122,6 @@ struct SpreadRow {
 
 __device__ __forceinline__ unsigned bin_of(unsigned ok) { return (unsigned)kBins - 1u - (ok >> kLowBits); }  // counted from the top
 
-template <int KPT, int THREADS>
-__device__ __forceinline__ void chunk_keys(unsigned (&ok)[KPT], const float *scores, unsigned base, unsigned blocks, unsigned tid) {
-#pragma unroll
-    for (int j = 0; j < KPT; ++j) {
-        const unsigned i = base + (unsigned)j * THREADS + tid;
-        ok[j] = i < blocks ? orderable(scores[i]) : 0u;
-    }
-}
-
 template <int CHUNK, int THREADS>
 __global__ __launch_bounds__(THREADS) void qsa_sort_chunks_kernel(const SpreadArgs a) {
     constexpr int KPT = CHUNK / THREADS;
@@ -1068,7 +1136,7 @@ __global__ __launch_bounds__(THREADS) void qsa_sort_chunks_kernel(const SpreadAr
     const unsigned base = blockIdx.x * (unsigned)CHUNK;
     if (base >= r.blocks) return;
     unsigned ok[KPT], place[KPT];
-    chunk_keys<KPT, THREADS>(ok, a.s.scores + (long long)row * a.s.score_stride, base, r.blocks, tid);
+    load_keys<KPT, THREADS>(ok, a.s.scores + (long long)row * a.s.score_stride, base, r.blocks, tid);
 #pragma unroll
     for (unsigned u = 0; u <= kOwn; ++u)
         if (u * THREADS + tid < kWords) counts[u * THREADS + tid] = 0u;
@@ -1127,7 +1195,7 @@ __global__ __launch_bounds__(kChunkThreads) void qsa_settle_chunks_kernel(const 
     const unsigned n_chunks = (r.blocks + kChunk - 1u) / kChunk;
     const size_t chunk0 = (size_t)row * (unsigned)a.chunks;
     unsigned ok[KPT];
-    chunk_keys<KPT, kChunkThreads>(ok, a.s.scores + (long long)row * a.s.score_stride, base, r.blocks, tid);  // in flight while the tables are read
+    load_keys<KPT, kChunkThreads>(ok, a.s.scores + (long long)row * a.s.score_stride, base, r.blocks, tid);  // in flight while the tables are read
     if (wave == 0) {
         // The last bin with at most B blocks above it holds the block at rank B.
         const unsigned short *coarse = a.coarse + chunk0 * 64 + lane, *starts = a.starts + chunk0 * kBins;
@@ -1294,7 +1362,7 @@ __global__ __launch_bounds__(kChunkThreads) void qsa_settle_chunks_kernel(const 
         __syncthreads();
         const unsigned tied = (((unsigned)kBins - 1u - bin_sh) << kLowBits) | prefix, first = tie_chunk_sh * kChunk, rank = rank_sh;
         unsigned other[KPT];
-        chunk_keys<KPT, kChunkThreads>(other, a.s.scores + (long long)row * a.s.score_stride, first, r.blocks, tid);
+        load_keys<KPT, kChunkThreads>(other, a.s.scores + (long long)row * a.s.score_stride, first, r.blocks, tid);
         unsigned long long alike[KPT];
 #pragma unroll
         for (int j = 0; j < KPT; ++j) {
@@ -1625,13 +1693,13 @@ extern "C" int tt_hip_qsa_select(tt_hip_ctx *ctx, const float *scores, size_t sc
     const long long max_blocks = last_visible / ratio;
     const dim3 grid((unsigned)rows), wg(kSelectThreads);
     // Rows with many blocks each spread over many workgroups, provided every row has a real selection to make (B < blocks).
-    // A workgroup per row is its CU's arithmetic (16,385 to 32,768 blocks 19.5 us, up to 65,536 34, whatever the rows, while
-    // they find a CU each); spread, every block is handled twice and the launch's work goes over all CUs: 1 row of 32,768
-    // blocks 16.8 -> 11.3 us, 4 rows 24.7 -> 13.9, 64 rows 22.0 -> 19.8, 64 rows of 50,000 33.8 -> 25.1; 128 rows of 20,000 19.6
-    // against 23.7, of 32,768 35.0 against 36.9.  Beyond 65,536 blocks a row's scores do not fit its workgroup's registers (128
-    // rows of 100,000 520 -> 119 us).
+    // A workgroup per row takes a CU 15 us for 17,000 to 32,768 blocks and 20 up to 65,536, whatever the rows while they find a CU
+    // each, and with a mask to write 17 to 20 and 23 to 30; spread, every block is handled twice and the launch's work goes over all
+    // CUs: 1 row of 32,000 blocks 14.2 -> 11.9 us, 32 rows 15.3 -> 14.3, 48 rows 15.3 against 16.1, 64 rows 15.3 against 18.0; with a
+    // mask 32 rows 18.9 -> 15.0, 64 rows of 24,000 18.2 -> 17.5, of 65,000 29.9 -> 27.1.  Beyond 65,536 blocks a row's scores do not
+    // fit its workgroup's registers (128 rows of 100,000 520 -> 119 us).
     const long long all_blocks = (long long)rows * max_blocks;
-    const bool pays = max_blocks > 64ll * kSelectThreads || (max_blocks > 16ll * kSelectThreads && 4 * rows <= ctx->n_cus);
+    const bool pays = max_blocks > 64ll * kSelectThreads || (max_blocks > 16ll * kSelectThreads && (keep ? 4 : 6) * rows <= ctx->n_cus);
     const bool spread = pays && max_blocks <= kMaxSpreadBlocks && first_visible > width && width >= ratio;
     if (spread) {
         // (chunks of 2,048 while their workgroups are few: 16 rows of 20,000 blocks 14.0 us against 19.0 in chunks of 4,096, 64 rows of
