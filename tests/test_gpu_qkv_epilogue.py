@@ -100,6 +100,13 @@ def test_chunk_whole_blocks_and_ragged_edges(gpu_ctx, position, rows):
     kv.close()
 
 
+@pytest.mark.parametrize("H,KH,D,rot,rows", [(16, 4, 64, 64, 643), (16, 4, 64, 64, 644), (8, 1, 64, 32, 700), (16, 2, 256, 256, 391), (32, 8, 128, 64, 385)])
+def test_chunks_on_both_sides_of_the_block_rule(gpu_ctx, H, KH, D, rot, rows):
+    # narrow heads go on by rows until those are more than 160 workgroups; whole blocks with every slot of angles in use
+    kv = _run(gpu_ctx, H, KH, D, rot, 1, rows, [39], [0], seed=rows)
+    kv.close()
+
+
 def test_verify_rows_of_several_sequences(gpu_ctx):
     kv = _run(gpu_ctx, 16, 2, 256, 64, 3, 4, [100, 65, 30], [0, 2, 1], seed=5, capacity=256)
     kv.close()

@@ -33,7 +33,7 @@ constexpr int kMaxEpilogueSeq = 64;
 constexpr int kMaxRotaryHalf = 128;
 constexpr int kEpiloguePad = 8;  // halves of padding per LDS row
 
-struct EpilogueArgs {
+struct EpilogueHead {
     const _Float16 *q_packed, *k_proj, *v_proj;
     _Float16 *q_out, *gate_out;
     _Float16 *k_layer, *v_layer;
@@ -49,6 +49,8 @@ struct EpilogueArgs {
     int block_wgs, row_wgs;
     int first_block, n_blocks;  // whole blocks (single-sequence calls only)
     int head_rows, tail_rows;   // ragged rows before / after the whole blocks (per sequence: rows when no blocks)
+};
+struct EpilogueArgs : EpilogueHead {
     int slot[kMaxEpilogueSeq], position[kMaxEpilogueSeq];
     int row0[kMaxEpilogueSeq];  // where position[s] is stored: the same, or position % capacity on a ring
     float freq[kMaxRotaryHalf];  // theta^(-2i / rotary_dim), computed on the host with the C library's powf
@@ -59,6 +61,34 @@ namespace {
 constexpr int E = 8;  // dims per lane: one 16-byte access
 
 __device__ __forceinline__ float bf16_to_float(unsigned short w) { return __builtin_bit_cast(float, (unsigned)w << 16); }
+
+// The launch's arguments in one trip: left to the compiler each is read where it is first used, five scalar trips one behind the
+// other before a ragged row's first load goes out.
+typedef int head_words __attribute__((ext_vector_type(16)));
+struct HeadWords {
+    head_words lo, mid, hi;
+};
+static_assert(sizeof(EpilogueHead) == 176 && sizeof(EpilogueArgs) >= sizeof(HeadWords), "three pieces of 64 bytes hold the head");
+__device__ __forceinline__ void load_head(EpilogueHead &head) {
+    const unsigned long long base = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+    HeadWords w;
+    asm volatile("s_load_dwordx16 %0, %3, 0x0\n\ts_load_dwordx16 %1, %3, 0x40\n\ts_load_dwordx16 %2, %3, 0x80\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(w.lo), "=&s"(w.mid), "=&s"(w.hi)
+                 : "s"(base)
+                 : "memory");
+    __builtin_memcpy(&head, &w, sizeof(head));
+    // (what comes out of an asm block is a pointer to anywhere: these are to global memory)
+    auto global = [](auto *&p) { p = (decltype(p + 0))(__attribute__((address_space(1))) char *)(unsigned long long)p; };
+    global(head.q_packed);
+    global(head.k_proj);
+    global(head.v_proj);
+    global(head.q_out);
+    global(head.gate_out);
+    global(head.k_layer);
+    global(head.v_layer);
+    global(head.q_weight);
+    global(head.k_weight);
+}
 
 // A head slice (D dims) is held by D / 8 consecutive lanes, 8 dims each, so a wavefront works on
 // 64 / (D / 8) slices at once.  Rotation pairs are (i, i + rotary_half): the partner lane is
@@ -74,8 +104,21 @@ struct Rotation {
 // others idling), so the work is spread instead: lane j of a slice's group of LPS lanes
 // evaluates angle indices j, j + LPS, ... (at most 4), and every lane then collects the 8 it
 // needs with cross-lane reads.
+// (Their frequencies are loaded in front of a slice's rows, and held where they are -- pin -- behind the rows' loads: each would
+// else be loaded where its angle is worked out, a trip to memory in the middle of the chain.)
+struct Frequencies {
+    float of[4];
+    __device__ __forceinline__ void pin() { asm volatile("" : "+v"(of[0]), "+v"(of[1]), "+v"(of[2]), "+v"(of[3])); }
+};
 template <int LPS>
-__device__ __forceinline__ Rotation rotation_for(int rotary_half, const float *freq, int position, int lane, int d0) {
+__device__ __forceinline__ Frequencies load_frequencies(int rotary_half, const float *freq, int lane) {
+    Frequencies f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) f.of[t] = freq[min(t * LPS + lane % LPS, max(rotary_half - 1, 0))];
+    return f;
+}
+template <int LPS>
+__device__ __forceinline__ Rotation rotation_for(int rotary_half, const Frequencies &freq, int position, int lane, int d0) {
     Rotation r;
     const int shift = rotary_half / E;
     r.low = d0 < rotary_half;
@@ -92,8 +135,7 @@ __device__ __forceinline__ Rotation rotation_for(int rotary_half, const float *f
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         if (t * LPS < rotary_half) {  // wave-uniform
-            const int i = t * LPS + j;
-            const float angle = (float)position * freq[min(i, rotary_half - 1)];
+            const float angle = (float)position * freq.of[t];
             float ct, st;
             sincosf(angle, &st, &ct);  // one argument reduction for both
 #pragma unroll
@@ -127,23 +169,35 @@ __device__ __forceinline__ void norm_rope(float (&x)[E], const float (&w)[E], fl
     }
 }
 
-__device__ __forceinline__ void load_weight(float (&w)[E], const unsigned short *weight, int d0) {
+// A lane's loads stay as they come until all of a slice's are on their way: converted where they are issued, they were waited
+// for in front of the branches behind them, and the next loads went out a trip to memory later.
+struct WeightBits {
+    unsigned short of[E];
+};
+__device__ __forceinline__ WeightBits load_weight(const unsigned short *weight, int d0) {
+    WeightBits w;
 #pragma unroll
-    for (int e = 0; e < E; ++e) w[e] = bf16_to_float(weight[d0 + e]);
+    for (int e = 0; e < E; ++e) w.of[e] = weight[d0 + e];
+    return w;
+}
+__device__ __forceinline__ void to_floats(float (&x)[E], const WeightBits &w) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = bf16_to_float(w.of[e]);
 }
 
 // 8 consecutive halves <-> fp32.  VEC: the address is a multiple of 16 bytes (one load/store).
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 template <bool VEC>
-__device__ __forceinline__ void load_halves(float (&x)[E], const _Float16 *p) {
-    if constexpr (VEC) {
-        const h8 v = *reinterpret_cast<const h8 *>(p);
+__device__ __forceinline__ h8 load_halves(const _Float16 *p) {
+    if constexpr (VEC) return *reinterpret_cast<const h8 *>(p);
+    h8 v;
 #pragma unroll
-        for (int e = 0; e < E; ++e) x[e] = (float)v[e];
-    } else {
+    for (int e = 0; e < E; ++e) v[e] = p[e];
+    return v;
+}
+__device__ __forceinline__ void to_floats(float (&x)[E], h8 v) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) x[e] = (float)p[e];
-    }
+    for (int e = 0; e < E; ++e) x[e] = (float)v[e];
 }
 template <bool VEC>
 __device__ __forceinline__ void store_halves(_Float16 *p, const float (&x)[E]) {
@@ -164,7 +218,7 @@ __device__ __forceinline__ void store_halves(_Float16 *p, const float (&x)[E]) {
 // hold a group of 64 dims find its minimum and maximum with three exchanges.  `x` holds the fp16
 // values the quantiser's source row would hold.  Every lane runs the exchanges; `active` gates
 // the stores.
-__device__ __forceinline__ void store_quantised(const EpilogueArgs &a, uint8_t *block, bool is_v, int head_dim, int key,
+__device__ __forceinline__ void store_quantised(const EpilogueHead &a, uint8_t *block, bool is_v, int head_dim, int key,
                                                 int d0, const float (&x)[E], int lane, bool active) {
     const int bits = a.kv_bits;
     float lo = x[0], hi = x[0];
@@ -214,7 +268,9 @@ __device__ __forceinline__ void store_quantised(const EpilogueArgs &a, uint8_t *
 // ALIGNED: every caller pointer is a multiple of 16 bytes and every stride a multiple of 8 halves.
 // QI: accesses of D/8-lane slices per wavefront of the query part (SPW heads each).
 template <int D, bool ALIGNED, int QI>
-__global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a) {
+__global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs tables) {
+    EpilogueHead a;
+    load_head(a);
     constexpr int LPS = D / E;     // lanes per slice
     constexpr int SPW = 64 / LPS;  // slices a wavefront holds per access: 2, 4, 8 at D = 256, 128, 64
     extern __shared__ __attribute__((aligned(16))) _Float16 tile[];
@@ -232,26 +288,32 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
         constexpr int NI = RPW / SPW;          // accesses per wavefront, SPW rows each
         _Float16 *kt = tile, *vt = tile + kBlockTokens * ROW;
         const int token0 = a.head_rows + blk * kBlockTokens;
-        const int position0 = a.position[0] + token0;
-        float k[NI][E], v[NI][E], w[E];
+        const int position0 = tables.position[0] + token0;
+        h8 k[NI], v[NI];
 #pragma unroll
         for (int i = 0; i < NI; ++i) {  // all of the wavefront's rows in flight at once
             const int row = wave * RPW + i * SPW + sub;
             const long long off = (long long)(token0 + row) * a.kv_stride + (long long)kvh * D + d0;
-            load_halves<ALIGNED>(k[i], a.k_proj + off);
-            load_halves<ALIGNED>(v[i], a.v_proj + off);
+            k[i] = load_halves<ALIGNED>(a.k_proj + off);
+            v[i] = load_halves<ALIGNED>(a.v_proj + off);
         }
-        load_weight(w, a.k_weight, d0);
+        Frequencies freq = load_frequencies<LPS>(a.rotary_half, tables.freq, lane);
+        const WeightBits weight = load_weight(a.k_weight, d0);
+        freq.pin();
+        float w[E];
+        to_floats(w, weight);
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int row = wave * RPW + i * SPW + sub;
-            const Rotation rot = rotation_for<LPS>(a.rotary_half, a.freq, position0 + row, lane, d0);
-            norm_rope<D>(k[i], w, a.eps, rot);
-            store_halves<true>(kt + row * ROW + d0, k[i]);
-            store_halves<true>(vt + row * ROW + d0, v[i]);
+            const Rotation rot = rotation_for<LPS>(a.rotary_half, freq, position0 + row, lane, d0);
+            float x[E];
+            to_floats(x, k[i]);
+            norm_rope<D>(x, w, a.eps, rot);
+            store_halves<true>(kt + row * ROW + d0, x);
+            *reinterpret_cast<h8 *>(vt + row * ROW + d0) = v[i];
         }
         __syncthreads();
-        const size_t dst0 = ((size_t)a.slot[0] * a.n_kv_heads + kvh) * (size_t)a.page_elems +
+        const size_t dst0 = ((size_t)tables.slot[0] * a.n_kv_heads + kvh) * (size_t)a.page_elems +
                             (size_t)(a.first_block + blk) * (size_t)(kBlockTokens * D);
         constexpr int PIECES = kBlockTokens * D / 8;
         for (int p = threadIdx.x; p < PIECES; p += 256) {
@@ -272,7 +334,9 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
         // the chain of one wavefront, so K rows and V rows have wavefronts of their own, the counts are divided in 32
         // bits (every item is a row of at least 128 bytes of device memory, so they fit) and an angle's sine and
         // cosine share one argument reduction: one token over 8 bits 4.44 -> 3.78 us, 7 over 4 bits 5.19 -> 4.32,
-        // 4 over 8 bits 4.82 -> 3.97, one over fp16 3.62 -> 3.49.
+        // 4 over 8 bits 4.82 -> 3.97, one over fp16 3.62 -> 3.49.  And everything a lane loads is asked for at once, in one trip behind
+        // the arguments' (16/2 heads of 256, launches in a row: one token 3.02 -> 2.75 us, over 8 bits 3.71 -> 3.38; 32/8 of 128 3.51 ->
+        // 3.08; the whole chunk of 777 rows 9.7 -> 7.8, of 4096 rows 29.5 -> 27.6).
         const unsigned item = ((unsigned)(wg - a.block_wgs) * 2 + (unsigned)(wave >> 1)) * SPW + (unsigned)sub;
         const bool is_v = (wave & 1) != 0;  // wave-uniform
         const unsigned per_seq = (unsigned)(a.head_rows + a.tail_rows), n_kv = (unsigned)a.n_kv_heads;
@@ -284,16 +348,25 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
         if (row >= a.head_rows) row += a.n_blocks * kBlockTokens;  // skip what the block workgroups cover
         const int token = (int)seq * a.rows + row;
         const long long off = (long long)token * a.kv_stride + (long long)kvh * D + d0;
+        // (a V row's wavefront asks for what a K row's needs, too: a branch would come between the loads)
+        Frequencies freq = load_frequencies<LPS>(a.rotary_half, tables.freq, lane);
+        int position = tables.position[seq], row0 = tables.row0[seq], slot = tables.slot[seq];
+        const h8 halves = load_halves<ALIGNED>((is_v ? a.v_proj : a.k_proj) + off);
+        const WeightBits weight = load_weight(a.k_weight, d0);
+        freq.pin();
+        asm volatile("" : "+v"(position), "+v"(row0), "+v"(slot));
         float x[E];
-        load_halves<ALIGNED>(x, (is_v ? a.v_proj : a.k_proj) + off);
-        const int stored = a.row0[seq] + row;  // for the page
-        const size_t page = (size_t)a.slot[seq] * a.n_kv_heads + kvh;
         if (!is_v) {
+            const Rotation rot = rotation_for<LPS>(a.rotary_half, freq, position + row, lane, d0);
             float w[E];
-            load_weight(w, a.k_weight, d0);
-            const Rotation rot = rotation_for<LPS>(a.rotary_half, a.freq, a.position[seq] + row, lane, d0);
+            to_floats(w, weight);
+            to_floats(x, halves);
             norm_rope<D>(x, w, a.eps, rot);
+        } else {
+            to_floats(x, halves);
         }
+        const int stored = row0 + row;  // for the page
+        const size_t page = (size_t)slot * a.n_kv_heads + kvh;
         if (a.kv_bits != 16) {  // wave-uniform
             const size_t at = page * (size_t)a.page_elems * 2 + (size_t)(stored >> 5) * block_bytes(D, a.kv_bits);
 #pragma unroll
@@ -320,24 +393,31 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs a)
         const int token = (int)(item / runs);
         const int head_first = (int)(item - (unsigned)token * runs) * (QI * SPW);
         const int seq = a.rows == 1 ? token : (int)((unsigned)token / (unsigned)a.rows);
-        const int position = a.position[seq] + (token - seq * a.rows);
-        float q[QI][E], g[QI][E], w[E];
+        const int position = tables.position[seq] + (token - seq * a.rows);
+        Frequencies freq = load_frequencies<LPS>(a.rotary_half, tables.freq, lane);
+        h8 q[QI], g[QI];
 #pragma unroll
         for (int i = 0; i < QI; ++i) {
             const int head = min(head_first + i * SPW + sub, a.n_q_heads - 1);  // past the last head: shadow it
             const _Float16 *src = a.q_packed + token * a.qp_stride + (long long)head * 2 * D + d0;
-            load_halves<ALIGNED>(q[i], src);
-            load_halves<ALIGNED>(g[i], src + D);
+            q[i] = load_halves<ALIGNED>(src);
+            g[i] = load_halves<ALIGNED>(src + D);
         }
-        load_weight(w, a.q_weight, d0);
-        const Rotation rot = rotation_for<LPS>(a.rotary_half, a.freq, position, lane, d0);
+        const WeightBits weight = load_weight(a.q_weight, d0);
+        freq.pin();
+        const Rotation rot = rotation_for<LPS>(a.rotary_half, freq, position, lane, d0);
+        float w[E];
+        to_floats(w, weight);
 #pragma unroll
         for (int i = 0; i < QI; ++i) {
             const int head = head_first + i * SPW + sub;
-            norm_rope<D>(q[i], w, a.eps, rot);
+            float x[E], gate[E];
+            to_floats(x, q[i]);
+            to_floats(gate, g[i]);
+            norm_rope<D>(x, w, a.eps, rot);
             if (head < a.n_q_heads) {
-                store_halves<ALIGNED>(a.q_out + token * a.q_stride + (long long)head * D + d0, q[i]);
-                store_halves<ALIGNED>(a.gate_out + token * a.g_stride + (long long)head * D + d0, g[i]);
+                store_halves<ALIGNED>(a.q_out + token * a.q_stride + (long long)head * D + d0, x);
+                store_halves<ALIGNED>(a.gate_out + token * a.g_stride + (long long)head * D + d0, gate);
             }
         }
     }
@@ -420,9 +500,11 @@ extern "C" int tt_hip_qkv_epilogue_append(tt_hip_ctx *ctx, tt_hip_kv *kv, int la
     int first_full = 0, last_full_end = 0;
     const int row0 = a.row0[0];  // whole blocks are blocks of the page: counted from where the rows are stored
     // (quantised pages: every row through the row path, which quantises.  Short chunks too: a block's workgroup writes
-    // its 32 tokens one after the other, and with a handful of blocks those few workgroups are the whole launch's time
-    // -- 128 tokens 6.6 us by blocks, 5.0 us by rows; 256 tokens 7.0 / 5.6; 512 tokens 7.9 / 8.2.)
-    if (n_seq == 1 && kv->bits == 16 && rows >= 384) {
+    // its 32 tokens one after the other, and with a handful of blocks those few workgroups are the whole launch's time:
+    // 16/2 heads of 256, 384 tokens 6.8 us by blocks, 6.2 by rows, 512 tokens 7.2 / 7.5; 32/8 of 128, 384 tokens 6.0 / 8.0; 16/4
+    // of 64, 512 tokens 5.4 / 5.1, 777 tokens 5.4 / 5.8.)
+    const long long row_path_wgs = (long long)rows * KH / (2 * (64 / (D / 8)));
+    if (n_seq == 1 && kv->bits == 16 && rows >= 384 && row_path_wgs > 160) {
         first_full = ((row0 + kBlockTokens - 1) / kBlockTokens) * kBlockTokens;
         last_full_end = ((row0 + rows) / kBlockTokens) * kBlockTokens;
     }
