@@ -565,6 +565,33 @@ def test_split_geometry_reports_dispatch_shape(gpu_ctx):
     gpu_ctx.set_split_tokens(0)
 
 
+@pytest.mark.parametrize("D,gated,splits", [
+    (256, True, (2, 32)), (256, True, (33,)), (128, False, (128,)), (64, True, (129,)), (256, True, (193,)),  # a workgroup per 64 dims
+    (256, True, (1, 4, 2, 3, 4, 1, 4, 4)), (128, True, (5, 16, 17, 1, 32, 4, 31, 2)), (64, False, (16, 3, 32, 8, 15, 17, 5, 4))])
+def test_combine_at_the_edges_of_its_batches(gpu_ctx, D, gated, splits):
+    # One block of 32 keys a split, so that the partial results a combine pass merges are counted out: up to 32 and more, whole
+    # batches of 128 and one past them, a second batch of 64 maxima; four, a turn of 16, and two over a batch of eight.
+    H, KH = 8, 2
+    lens = [32 * n - (i % 3) for i, n in enumerate(splits)]
+    r = np.random.default_rng(sum(lens) + D)
+    k, v = (r.standard_normal((max(lens), KH, D)).astype(np.float16) for _ in range(2))
+    q = r.standard_normal((len(lens), H * D)).astype(np.float16)
+    gate = r.standard_normal(q.shape).astype(np.float16) if gated else None
+    c = Cache(gpu_ctx, k, v, slots=len(lens))
+    for slot in range(1, len(lens)):
+        c.put(0, slot, 0, k[:lens[slot]], v[:lens[slot]])
+    gpu_ctx.set_split_tokens(32)
+    try:
+        got = _decode(gpu_ctx, c.kv, q, lens, H, D ** -0.5, gate=gate)
+    finally:
+        gpu_ctx.set_split_tokens(0)
+    for i, n in enumerate(lens):
+        want = oracle.decode(q[i].astype(np.float32), c.k32[:n], c.v32[:n], H, KH, D, D ** -0.5,
+                             gate=None if gate is None else gate[i].astype(np.float32))
+        _check(got[i].reshape(-1), np.asarray(want).reshape(-1), f"{splits[i]} splits of one block, head size {D}")
+    c.close()
+
+
 def test_graph_replay_matches_eager(gpu_ctx):
     import torch
     from tinytitan_amd import capi

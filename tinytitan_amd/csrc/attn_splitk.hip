@@ -82,31 +82,35 @@ __device__ __forceinline__ TileInfo tile_info(const SplitKHot &a, const SplitKSe
 }
 
 // The gate's four values of one output item, asked for ahead of the arithmetic they end up multiplying (a combine pass
-// that fetches them only when its sums are done waits for memory once more with nothing else to do).
-__device__ __forceinline__ void load_gate4(const SplitKArgs &a, int seq, int tok, int head, int d, int D, bool aligned, float (&g)[4]) {
-    g[0] = g[1] = g[2] = g[3] = 0.0f;
-    if (!a.gate) return;
-    const _Float16 *gp = a.gate + seq * a.g_seq_stride + tok * a.g_tok_stride + (long long)head * D + d;
-    if (aligned) {
-        const h4 gv = *reinterpret_cast<const h4 *>(gp);
+// that fetches them only when its sums are done waits for memory once more with nothing else to do), and kept as they come:
+// converted in the branch that loads them, they were waited for there, in front of the partial results' loads.
+template <typename Args>
+__device__ __forceinline__ h4 load_gate4(const Args &a, int seq, int tok, int head, int d, int D, bool aligned) {
+    h4 g = (h4)(_Float16)0.0f;
+    if (a.gate) {
+        const global_halves gp = (global_halves)(a.gate + seq * a.g_seq_stride + tok * a.g_tok_stride + (long long)head * D + d);
+        if (aligned) {
+            g = *(const __attribute__((address_space(1))) h4 *)gp;
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) g[i] = (float)gv[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) g[i] = (float)gp[i];
+            for (int i = 0; i < 4; ++i) g[i] = gp[i];
+        }
     }
+    return g;
 }
 // Final value of one output element with the gate's values in hand: normalise, gate in fp32, round once.
-__device__ __forceinline__ void store_out4_gated(const SplitKArgs &a, int seq, int tok, int head, int d, int D, f4 o, float inv_l,
-                                                 bool aligned, const float (&g)[4]) {
+template <typename Args>
+__device__ __forceinline__ void store_out4_gated(const Args &a, int seq, int tok, int head, int d, int D, f4 o, float inv_l,
+                                                 bool aligned, h4 g) {
     f4 r = o * inv_l;
     if (a.gate) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] *= 1.0f / (1.0f + __expf(-g[i]));
+        for (int i = 0; i < 4; ++i) r[i] *= 1.0f / (1.0f + __expf(-(float)g[i]));
     }
-    _Float16 *op = a.out + seq * a.o_seq_stride + tok * a.o_tok_stride + (long long)head * D + d;
+    typedef __attribute__((address_space(1))) _Float16 *global_out;
+    const global_out op = (global_out)(a.out + seq * a.o_seq_stride + tok * a.o_tok_stride + (long long)head * D + d);
     if (aligned) {
-        *reinterpret_cast<h4 *>(op) = h4{(_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3]};
+        *(__attribute__((address_space(1))) h4 *)op = h4{(_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3]};
     } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) op[i] = (_Float16)r[i];
@@ -997,6 +1001,36 @@ __device__ __forceinline__ void load_hot(SplitKHot &hot, SplitKSeq &sq, int seq)
     hot = __builtin_bit_cast(SplitKHot, w);
     sq = __builtin_bit_cast(SplitKSeq, e);
 }
+// ... and for a combine pass, whose first request is the gate's, where the rows go and their gate beside them.
+struct SplitKOut {
+    const _Float16 *gate;
+    _Float16 *out;
+    long long g_seq_stride, g_tok_stride, o_seq_stride, o_tok_stride;
+};
+static_assert(offsetof(SplitKArgs, gate) == 0x480 && offsetof(SplitKArgs, o_tok_stride) == 0x480 + offsetof(SplitKOut, o_tok_stride) &&
+                  offsetof(SplitKArgs, out) == 0x480 + offsetof(SplitKOut, out) && sizeof(SplitKOut) == 48,
+              "load_combine's offsets");
+__device__ __forceinline__ void load_combine(SplitKHot &hot, SplitKSeq &sq, SplitKOut &out, int seq) {
+    typedef int i8v __attribute__((ext_vector_type(8)));
+    struct OutWords {
+        i8v lo;
+        i4 hi;
+    };
+    const unsigned long long base = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+    const unsigned long long entry = base + (unsigned)seq * (unsigned)sizeof(SplitKSeq);
+    HotWords w;
+    i4 e, t_hi;
+    i8v t_lo;
+    asm volatile("s_load_dwordx16 %0, %5, 0x0\n\ts_load_dwordx16 %1, %5, 0x40\n\ts_load_dwordx4 %2, %6, 0x80\n\t"
+                 "s_load_dwordx8 %3, %5, 0x480\n\ts_load_dwordx4 %4, %5, 0x4a0\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(w.lo), "=&s"(w.hi), "=&s"(e), "=&s"(t_lo), "=&s"(t_hi)
+                 : "s"(base), "s"(entry)
+                 : "memory");
+    hot = __builtin_bit_cast(SplitKHot, w);
+    sq = __builtin_bit_cast(SplitKSeq, e);
+    const OutWords t = {t_lo, t_hi};
+    __builtin_memcpy(&out, &t, sizeof(out));
+}
 typedef __attribute__((address_space(4))) const i4 *seq_entries;  // SplitKSeq: [3] is first_split
 __device__ __forceinline__ seq_entries seq_table() {
     return (seq_entries)((__attribute__((address_space(4))) const char *)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(SplitKArgs, seq));
@@ -1516,6 +1550,19 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
 // groups add up through two shuffles and LDS.  All-empty input yields zeros
 // (sources/TinyTitanCore/Metal/Attention/attention.metal:418-427).
 // ---------------------------------------------------------------------------
+// What such a pass takes is its chain of trips to memory, and it is two: the arguments, then the gate, the
+// maxima and the partial rows together -- with the gate converted where it was loaded, its arguments read in a trip of
+// their own and the second 64 maxima behind the first they were five.  A decode step's launch 0.2 us less (two layers of 7
+// sequences of 300 .. 9,000 keys over 4 bits 40.8 -> 40.0 us, four of one of 20,010 over 8 bits 78.2 -> 77.4), the rows kernel
+// behind a chunk of 128 rows over key ranges 2.2 (two layers behind 32,640 keys 240.5 -> 236.1).
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(1))) f2 *global_pairs;  // part_ml: a partial row's (max, sum)
+typedef const __attribute__((address_space(1))) char *global_bytes;
+
+__device__ __forceinline__ int splits_of(const TileInfo &ti, int split_len) {
+    return (int)((unsigned)(max(ti.tile_end - ti.k0, 1) + split_len - 1) / (unsigned)split_len);  // (an empty range has one, of zeros)
+}
+
 template <int D, int NT>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const SplitKArgs args) {
     constexpr int DCH = D / 64;
@@ -1524,55 +1571,65 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const SplitKArgs args
     const int tile = blockIdx.y, seq = blockIdx.z;
     SplitKHot a;
     SplitKSeq sq;
-    load_hot(a, sq, seq);
+    SplitKOut out;
+    load_combine(a, sq, out, seq);
     const TileInfo ti = tile_info(a, sq, tile);
     if (n >= ti.tile_rows * a.gh) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int n_splits = (ti.tile_end - ti.k0 + a.split_len - 1) / a.split_len;
-    if (n_splits < 1) n_splits = 1;
+    const int n_splits = splits_of(ti, a.split_len);
     // partial rows of split s: ((first_split + s) * n_tiles + tile) * NT + n
-    const size_t tfirst = (size_t)sq.first_split;
     const size_t tstride = (size_t)a.n_tiles * NT;
-    const size_t toff = (size_t)tile * NT + n;
+    const size_t first_row = (size_t)sq.first_split * tstride + (size_t)tile * NT + n;
     const int d = dchunk * 64 + (lane & 15) * 4;
-    // the gate's values of the item this thread stores at the end (threads 0-15), first of all requests
-    const int tl = n / a.gh;
+    const global_pairs ml = (global_pairs)a.part_ml + first_row;
+    const global_bytes rows = (global_bytes)a.part_o + (first_row * D + d) * sizeof(float);
+    auto partial_row = [&](int s) { return *(const __attribute__((address_space(1))) f4 *)(rows + s * tstride * (D * sizeof(float))); };
+    // the gate's values of the item that threads 0-15 store at the end, first of all requests
+    const int tl = (n * a.gh_inv) >> 16;
     const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
     const bool aligned = (a.flags & kHotAligned) != 0;
-    float gate4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (threadIdx.x < 16) load_gate4(args, seq, ti.t0 + tl, hh, d, D, aligned, gate4);
-    // This thread's first kBatch splits are requested BEFORE the global max is known: their
-    // addresses do not depend on it, so the max's loads and these share one trip to memory.
-    constexpr int kBatch = 8;
+    const h4 gate4 = load_gate4(out, seq, ti.t0 + tl, hh, d, D, aligned);
     const int s0 = wave * 4 + (lane >> 4);
-    f4 po[kBatch];
-    float pm[kBatch], pl[kBatch];
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-        const int s = s0 + 16 * i;
-        const size_t row = (tfirst + (s < n_splits ? s : 0)) * tstride + toff;
-        pm[i] = s < n_splits ? a.part_ml[row * 2] : kNegBig;
-        pl[i] = a.part_ml[row * 2 + 1];
-        po[i] = *reinterpret_cast<const f4 *>(a.part_o + row * D + d);
-    }
-    float mg = kNegBig;
-    for (int s = lane; s < n_splits; s += 64) mg = fmaxf(mg, a.part_ml[((tfirst + s) * tstride + toff) * 2]);
-    mg = wave_max_f32(mg, lane);
     f4 acc = (f4)0.0f;
     float l = 0.0f;
+    // This thread's first BATCH splits are requested BEFORE the global max is known: their
+    // addresses do not depend on it, so the max's loads and these share one trip to memory.
+    auto sum_splits = [&](auto batch) {
+        constexpr int BATCH = decltype(batch)::value, MAXIMA = (BATCH * 16 + 63) / 64;
+        f4 po[BATCH];
+        f2 pml[BATCH];
+        float maxima[MAXIMA];
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-        const float f = s0 + 16 * i < n_splits ? fast_exp2(pm[i] - mg) : 0.0f;
-        l += f * pl[i];
-        acc += f * po[i];
-    }
+        for (int i = 0; i < MAXIMA; ++i) maxima[i] = ml[min(lane + 64 * i, n_splits - 1) * tstride][0];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int s = s0 + 16 * i < n_splits ? s0 + 16 * i : 0;
+            pml[i] = ml[s * tstride];
+            po[i] = partial_row(s);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (the maximum's wait is not to come in front of the rest of the requests)
+        float mg = maxima[0];
+#pragma unroll
+        for (int i = 1; i < MAXIMA; ++i) mg = fmaxf(mg, maxima[i]);
+        for (int s = lane + 64 * MAXIMA; s < n_splits; s += 64) mg = fmaxf(mg, ml[s * tstride][0]);
+        mg = wave_max_f32(mg, lane);
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const float f = s0 + 16 * i < n_splits ? fast_exp2(pml[i][0] - mg) : 0.0f;
+            l += f * pml[i][1];
+            acc += f * po[i];
+        }
 #pragma unroll 4
-    for (int s = s0 + 16 * kBatch; s < n_splits; s += 16) {
-        const size_t row = (tfirst + s) * tstride + toff;
-        const float f = fast_exp2(a.part_ml[row * 2] - mg);
-        l += f * a.part_ml[row * 2 + 1];
-        acc += f * *reinterpret_cast<const f4 *>(a.part_o + row * D + d);
-    }
+        for (int s = s0 + 16 * BATCH; s < n_splits; s += 16) {
+            const f2 p = ml[s * tstride];
+            const float f = fast_exp2(p[0] - mg);
+            l += f * p[1];
+            acc += f * partial_row(s);
+        }
+    };
+    // (few splits: requests for the places of more would each pass through the CU's vector memory path)
+    if (n_splits <= 32) sum_splits(std::integral_constant<int, 2>{});
+    else sum_splits(std::integral_constant<int, 8>{});
     // (lanes l, l ^ 16, l ^ 32, l ^ 48, added in that order: v_permlane16_swap / v_permlane32_swap, no trip through LDS)
     l = sum_across_quarters(l);
 #pragma unroll
@@ -1588,14 +1645,14 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const SplitKArgs args
             lsum += sm[w][64];
             o += *reinterpret_cast<const f4 *>(&sm[w][lane * 4]);
         }
-        store_out4_gated(args, seq, ti.t0 + tl, hh, d, D, o, lsum > 0.0f ? 1.0f / lsum : 0.0f, aligned, gate4);
+        store_out4_gated(out, seq, ti.t0 + tl, hh, d, D, o, lsum > 0.0f ? 1.0f / lsum : 0.0f, aligned, gate4);
     }
 }
 
 // Pass 2 for launches of many tiles with few splits each (a chunk through the split-K tiles, or through the chunk
 // kernel over key ranges): one workgroup per four rows of a tile instead of one per (row, 64 dims) -- the many tiny
 // workgroups of attn_combine_kernel cost more to dispatch than these take to run.  A thread owns one (row, 4 dims)
-// item and all of its splits, kCombineRowsSplits at a time: their loads are requested together, so a thread makes
+// item and all of its splits, up to kCombineRowsSplits at a time: their loads are requested together, so a thread makes
 // one trip to memory per turn, not one per split (the host sends more than two turns' worth to the other kernel).
 // grid = (NT / 4, tile, sequence), 256 threads.
 constexpr int kCombineRowsSplits = 16;
@@ -1603,50 +1660,56 @@ constexpr int kCombineRowsSplits = 16;
 template <int D, int NT>
 __global__ __launch_bounds__(256) void attn_combine_rows_kernel(const SplitKArgs args) {
     constexpr int D4 = D / 4, ROWS = 4;
+    static_assert(ROWS * D4 <= 256, "an item a thread");
     const int tile = blockIdx.y, seq = blockIdx.z;
     SplitKHot a;
     SplitKSeq sq;
-    load_hot(a, sq, seq);
+    SplitKOut out;
+    load_combine(a, sq, out, seq);
     const TileInfo ti = tile_info(a, sq, tile);
-    int n_splits = (ti.tile_end - ti.k0 + a.split_len - 1) / a.split_len;
-    if (n_splits < 1) n_splits = 1;
-    const size_t tfirst = (size_t)sq.first_split, tstride = (size_t)a.n_tiles * NT;
-    const int n_valid = ti.tile_rows * a.gh;
-    for (int item = threadIdx.x; item < ROWS * D4; item += 256) {
-        const int n = blockIdx.x * ROWS + item / D4, d = (item % D4) * 4;
-        if (n >= n_valid) break;
-        const size_t toff = (size_t)tile * NT + n;
-        float mg = kNegBig, l = 0.0f;
-        f4 acc = (f4)0.0f;
-        for (int first = 0; first < n_splits; first += kCombineRowsSplits) {  // (one turn up to kCombineRowsSplits splits)
-            float pm[kCombineRowsSplits], pl[kCombineRowsSplits];
-            f4 po[kCombineRowsSplits];
+    const int n = blockIdx.x * ROWS + (int)threadIdx.x / D4, d = ((int)threadIdx.x % D4) * 4;
+    if ((int)threadIdx.x >= ROWS * D4 || n >= ti.tile_rows * a.gh) return;
+    const int n_splits = splits_of(ti, a.split_len);
+    const size_t tstride = (size_t)a.n_tiles * NT;
+    const size_t first_row = (size_t)sq.first_split * tstride + (size_t)tile * NT + n;
+    const global_pairs ml = (global_pairs)a.part_ml + first_row;
+    const global_bytes rows = (global_bytes)a.part_o + (first_row * D + d) * sizeof(float);
+    const int tl = (n * a.gh_inv) >> 16;
+    const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
+    const bool aligned = (a.flags & kHotAligned) != 0;
+    const h4 gate4 = load_gate4(out, seq, ti.t0 + tl, hh, d, D, aligned);
+    float mg = kNegBig, l = 0.0f;
+    f4 acc = (f4)0.0f;
+    auto turn = [&](auto splits, int first) {
+        constexpr int SPLITS = decltype(splits)::value;
+        f2 pml[SPLITS];
+        f4 po[SPLITS];
 #pragma unroll
-            for (int i = 0; i < kCombineRowsSplits; ++i) {
-                const int s = first + i;
-                const size_t row = (tfirst + (s < n_splits ? s : 0)) * tstride + toff;
-                pm[i] = s < n_splits ? a.part_ml[row * 2] : kNegBig;
-                pl[i] = a.part_ml[row * 2 + 1];
-                po[i] = *reinterpret_cast<const f4 *>(a.part_o + row * D + d);
-            }
-            float m_new = mg;
-#pragma unroll
-            for (int i = 0; i < kCombineRowsSplits; ++i) m_new = fmaxf(m_new, pm[i]);
-            const float keep = fast_exp2(mg - m_new);  // (first turn: what is kept is zero anyway)
-            l *= keep;
-            acc *= keep;
-            mg = m_new;
-#pragma unroll
-            for (int i = 0; i < kCombineRowsSplits; ++i) {
-                const float f = first + i < n_splits ? fast_exp2(pm[i] - mg) : 0.0f;
-                l += f * pl[i];
-                acc += f * po[i];
-            }
+        for (int i = 0; i < SPLITS; ++i) {
+            const int s = first + i < n_splits ? first + i : 0;
+            pml[i] = ml[s * tstride];
+            po[i] = *(const __attribute__((address_space(1))) f4 *)(rows + s * tstride * (D * sizeof(float)));
         }
-        const int tl = n / a.gh;
-        const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
-        store_out4(args, seq, ti.t0 + tl, hh, d, D, acc, l > 0.0f ? 1.0f / l : 0.0f, (a.flags & kHotAligned) != 0);
-    }
+        __builtin_amdgcn_sched_barrier(0);  // (left alone, a request goes out when a row before it has come: fewer registers)
+        float m_new = mg;
+#pragma unroll
+        for (int i = 0; i < SPLITS; ++i) m_new = fmaxf(m_new, first + i < n_splits ? pml[i][0] : kNegBig);
+        const float keep = fast_exp2(mg - m_new);  // (first turn: what is kept is zero anyway)
+        l *= keep;
+        acc *= keep;
+        mg = m_new;
+#pragma unroll
+        for (int i = 0; i < SPLITS; ++i) {
+            const float f = first + i < n_splits ? fast_exp2(pml[i][0] - mg) : 0.0f;
+            l += f * pml[i][1];
+            acc += f * po[i];
+        }
+    };
+    // (one turn up to kCombineRowsSplits splits, of four places where there are no more)
+    if (n_splits <= 4) turn(std::integral_constant<int, 4>{}, 0);
+    else
+        for (int first = 0; first < n_splits; first += kCombineRowsSplits) turn(std::integral_constant<int, kCombineRowsSplits>{}, first);
+    store_out4_gated(out, seq, ti.t0 + tl, hh, d, D, acc, l > 0.0f ? 1.0f / l : 0.0f, aligned, gate4);
 }
 
 // ---------------------------------------------------------------------------
