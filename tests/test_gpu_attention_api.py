@@ -566,7 +566,7 @@ def test_split_geometry_reports_dispatch_shape(gpu_ctx):
 
 
 @pytest.mark.parametrize("D,gated,splits", [
-    (256, True, (2, 32)), (256, True, (33,)), (128, False, (128,)), (64, True, (129,)), (256, True, (193,)),  # a workgroup per 64 dims
+    (256, True, (2, 32)), (256, True, (33,)), (128, True, (64,)), (64, False, (65,)), (128, False, (128,)), (64, True, (129,)), (256, True, (193,)),  # a workgroup per 64 dims
     (256, True, (1, 4, 2, 3, 4, 1, 4, 4)), (128, True, (5, 16, 17, 1, 32, 4, 31, 2)), (64, False, (16, 3, 32, 8, 15, 17, 5, 4))])
 def test_combine_at_the_edges_of_its_batches(gpu_ctx, D, gated, splits):
     # One block of 32 keys a split, so that the partial results a combine pass merges are counted out: up to 32 and more, whole
