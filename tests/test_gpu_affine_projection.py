@@ -280,6 +280,21 @@ def test_gemm_in_tiles_of_fewer_tokens(gpu_ctx, bits, m, n, tokens, kw):
     assert np.array_equal(_project(gpu_ctx, bits, packed, scales, biases, x[perm], **kw), got[perm])
 
 
+@pytest.mark.parametrize("bits,m,n,tokens,kw", [(4, 200, 1536, 600, {}), (8, 200, 1536, 600, {"x_stride": 1544, "y_stride": 203}),
+                                                 (4, 300, 2560, 513, {"weights_offset": 2}), (8, 136, 7680, 530, {}),
+                                                 (4, 2048, 3584, 1300, {}), (8, 2041, 4608, 2000, {"y_stride": 2043})])
+def test_gemm_whose_second_part_starts_between_eights(gpu_ctx, bits, m, n, tokens, kw):
+    # 24, 40, 56, 72 and 120 groups: whole eights, but the second part's first group, 12, 20, 28, 36 or 60, is 4 modulo 8, and the
+    # last eight that a thread stages from there reaches over the matrix's last group.  Tiles of 64, 96 and 128 tokens.
+    packed, scales, biases = _weights(m, n, bits, 115 + bits)
+    x = np.random.default_rng(116).standard_normal((tokens, n)).astype(np.float16)
+    got = _project(gpu_ctx, bits, packed, scales, biases, x, **kw)
+    pick = _sampled(tokens)
+    want = oracle.affine_projection(packed, scales, biases, x[pick].astype(np.float32), bits, half_weights=True)
+    _assert_parity(got[pick], want, _magnitude(packed, scales, biases, x[pick], bits), f"bits={bits} m={m} n={n} tokens={tokens} {kw}")
+    assert np.isfinite(got).all()
+
+
 @pytest.mark.parametrize("bits,m,n,tokens,kw", [(8, 2048, 512, 2176, {}), (4, 2000, 320, 2200, {"x_stride": 328, "y_stride": 2003}),
                                                  (4, 2000, 320, 2200, {"weights_offset": 2}), (4, 300, 4096, 16500, {})])
 def test_gemm_in_tiles_of_256_rows(gpu_ctx, bits, m, n, tokens, kw):

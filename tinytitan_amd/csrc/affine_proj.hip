@@ -600,7 +600,9 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
                 load_params<8>(bias_bits[i], a.biases + at, at_group, groups, vector);
             }
         };
-        if (params_vector) load(min(g, groups - 8), true);  // (eight groups past the matrix's last are not read back)
+        // (Eight groups that are all past the matrix's last are not read back.  Eight that reach over it, where a second part starts
+        // between eights -- 24 groups: at the 12th -- are, in part, and are loaded one by one.)
+        if (params_vector && (g >= groups || g + 8 <= groups)) load(min(g, groups - 8), true);
         else load(g, false);
 #pragma unroll
         for (int i = 0; i < kPasses; ++i) {
