@@ -53,11 +53,88 @@ int main() {
 }
 '''
 
+# The chunk kernel's copies into its rings, in the order one wavefront issues them.  A copy in flight lands at any time up to the wait
+# that covers it, in any order, so until then its place may hold either block: no other copy may be on its way there unless it
+# brings the same block, and what a step reads has landed and is not being overwritten.
+COPIES = r'''
+#include <algorithm>
+#include <cstdio>
+#include <map>
+#include <vector>
+#include "chunk_plan.h"
 
-@pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
-def test_ranges_cover_every_tile(tmp_path):
+struct Ring {
+    int step, ring, ahead, which;
+    std::map<int, int> landed;                 // slot -> block
+    std::vector<std::vector<std::pair<int, int>>> flying;  // by turn: (slot, block)
+    int slot_off = 0, bad = 0;
+    void copy(int i, int first, int nb, int carry) {
+        const int j = i + ahead, slot = tt::in_ring(ring, j + slot_off), block = tt::copied_block(step, ring, j, which, first, nb, carry);
+        for (const auto &turn : flying)
+            for (const auto &c : turn) bad += c.first == slot && c.second != block;
+        flying.push_back({{slot, block}});
+    }
+    void wait(size_t turns) {
+        for (; flying.size() > turns; flying.erase(flying.begin()))
+            for (const auto &c : flying.front()) landed[c.first] = c.second;
+    }
+    void read(int j, int first, int nb) {  // step j's blocks, while this step's copies fly
+        const int slot = tt::in_ring(ring, j + slot_off), want = first + std::min(step * j + which, nb - 1);
+        bad += landed.count(slot) == 0 || landed[slot] != want;
+        for (const auto &turn : flying)
+            for (const auto &c : turn) bad += c.first == slot && c.second != want;
+    }
+};
+
+static int run(int D, bool of_v, int which, int first, int nb, int carry) {
+    const int step = tt::step_blocks(D), ring = of_v ? tt::v_ring(D) : tt::k_ring(D);
+    Ring r{step, ring, tt::copies_ahead(ring, of_v), which, {}, {}};
+    for (int tile = 0; tile < (carry > 0 ? 2 : 1); ++tile) {
+        const int jb = tile ? 0 : first, n = tile ? carry : nb, next = tile ? 0 : carry, steps = (n + step - 1) / step;
+        if (tile == 0)
+            for (int i = -r.ahead; i < 0; ++i) r.copy(i, jb, n, next);
+        r.wait(0);
+        if (!of_v) r.read(0, jb, n);
+        for (int i = 0; i <= steps + 1; ++i) {
+            r.copy(i, jb, n, next);
+            if (!of_v && i + 1 < steps) r.read(i + 1, jb, n);
+            if (of_v && i >= 1 && i - 1 < steps) r.read(i - 1, jb, n);
+            r.wait(ring - 2);
+        }
+        r.wait(0);
+        r.slot_off = tt::in_ring(ring, r.slot_off + steps);
+    }
+    if (r.bad) std::printf("heads of %d, %s, block %d of a step, %d blocks, then %d: %d\n", D, of_v ? "V" : "K", which, nb, carry, r.bad);
+    return r.bad != 0;
+}
+
+int main() {
+    int bad = 0;
+    for (int D : {64, 128, 256})
+        for (int of_v = 0; of_v < 2; ++of_v)
+            for (int which = 0; which < tt::step_blocks(D); ++which)
+                for (int nb = 1; nb < 24; ++nb) {
+                    for (int carry = 0; carry < 24; ++carry) bad += run(D, of_v != 0, which, 0, nb, carry);
+                    bad += run(D, of_v != 0, which, 5, nb, 0);
+                }
+    return bad != 0;
+}
+'''
+
+
+def _runs(tmp_path, text):
     source, program = tmp_path / "plan.cpp", tmp_path / "plan"
-    source.write_text(PROGRAM)
+    source.write_text(text)
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wextra", "-Werror", "-I", CSRC, str(source), "-o", str(program)], check=True)
     ran = subprocess.run([str(program)], capture_output=True, text=True)
     assert ran.returncode == 0, ran.stdout[-4000:]
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
+def test_ranges_cover_every_tile(tmp_path):
+    _runs(tmp_path, PROGRAM)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
+def test_copies_into_the_rings_meet_nowhere(tmp_path):
+    _runs(tmp_path, COPIES)

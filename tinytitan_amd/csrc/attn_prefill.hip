@@ -20,7 +20,7 @@
 // Neither needs more than half of the register file, so two waves fit per SIMD, and the
 // hardware overlaps one wave's MFMAs with the other's softmax VALU work and LDS reads; eight
 // waves per CU also issue LDS reads about 1.6x faster than four can (the per-wave issue rate
-// is what limits a 4-wave design).  One workgroup barrier per key block separates the steps.
+// is what limits a 4-wave design).  One workgroup barrier separates the steps, of one key block (heads of 128: two).
 //
 // K/V blocks stream L2 -> LDS with direct-to-LDS 128-bit loads (no registers), three or four stages
 // deep, issued one or two steps ahead of their first use; the K fragment layout in HBM is the MFMA
@@ -33,6 +33,7 @@
 // Replaces attention_prefill_causal_q8 / attention_prefill_causal_tiled
 // (sources/TinyTitanCore/Metal/Prefill/prefill.metal:1056-1313) dispatched by
 // PrefillAttention.encodeCausal (sources/TinyTitan/Kernels/Attention/PrefillAttention.swift:165-258).
+#include "chunk_plan.h"
 #include "internal.h"
 #include "wave_ops.h"
 
@@ -76,19 +77,6 @@ namespace {
 
 constexpr float kNegBig = -1.0e30f;
 constexpr float kRescaleThreshold = 8.0f;
-// Key blocks of 32 that a step takes, and how many steps' K and V the rings in LDS hold.  Heads of 128 take two: a step's MFMAs are then
-// as many as at 256, its two score chains have no link that waits for the one before it, and there is one barrier, one row
-// maximum and one rescale test for 64 keys (32/8 heads, 777 rows behind 5,003 keys 107.5 -> 95.4 us, 4096 behind 8,000
-// 770 -> 710; V's ring holds three so that all of it stays within 160 KiB).  Two workgroups of one block a step on a CU (rings
-// of three, 128 registers) came to 721 where the chip is full and lost 5 % where it is not.
-constexpr int step_blocks(int D) { return D == 128 ? 2 : 1; }
-constexpr int k_ring(int) { return 4; }
-constexpr int v_ring(int D) { return D == 128 ? 3 : 4; }
-template <int RING>
-__device__ __forceinline__ int in_ring(int j) {  // j >= -RING
-    return RING == 4 ? j & 3 : (int)((unsigned)(j + RING) % (unsigned)RING);
-}
-
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
@@ -221,8 +209,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     const _Float16 *kp = a.k_slot + (size_t)kvh * a.page_elems;
     const _Float16 *vp = a.v_slot + (size_t)kvh * a.page_elems;
 
-    // Copies of step i: K of step i + KR and V of step i + VR - 2, of which this wave issues CPW one-KiB chunks.  Step
-    // j's blocks live in slot j % KR (% VR) of their ring.  Past the end of the tile the
+    // Copies of step i: K of step i + KR and V of step i + VR - 2 (copies_ahead), of which this wave issues CPW one-KiB chunks.
+    // Step j's blocks live in slot j % KR (% VR) of their ring.  Past the end of the tile the
     // last block is copied again (into a slot nobody reads any more), so that every step puts
     // the same number of copies in flight and one constant vmcnt tracks them.
     const unsigned smem_base = (unsigned)(size_t)(lds_ptr_t)smem;
@@ -235,13 +223,11 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     // without waiting for memory.  (A wave copies and reads K or V, so the offset is that of its own ring.)
     int slot_off = 0, carry_nb = 0;
     auto page_block = [&](int block) { return a.ring_blocks ? block % a.ring_blocks : block; };
-    auto role_ring = [&](int j) { return value_wave ? in_ring<VR>(j) : in_ring<KR>(j); };
+    auto role_ring = [&](int j) { return value_wave ? in_ring(VR, j) : in_ring(KR, j); };
     const int my_block = NB == 1 ? 0 : w4 * CPW / CHUNKS;  // which of a step's blocks this wave copies from
     const int my_chunk = w4 * CPW - my_block * CHUNKS;
     auto source_block = [&](int j, int nb) {  // the block that step-relative index j stands for
-        const int steps = (nb + NB - 1) / NB;
-        if (j < steps || carry_nb == 0) return jb + max(min(NB * j + my_block, nb - 1), 0);
-        return min(NB * role_ring(j - steps) + my_block, carry_nb - 1);  // (a slot's blocks again once the ring is full: the same bytes)
+        return value_wave ? copied_block(NB, VR, j, my_block, jb, nb, carry_nb) : copied_block(NB, KR, j, my_block, jb, nb, carry_nb);
     };
     // A step's copies: this wave's CPW one-KiB chunks of ONE block -- of K for the score waves (the LDS layout is the HBM
     // layout, fragment s is chunk s), of V for the value waves (gathered so that LDS holds fragment (mt, t) as [lane][8 halves]).  Where the block lies in the page and in the
@@ -260,7 +246,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     }
     auto step_copies = [&](int i, int nb) {  // of step i; nb blocks in the range
         StepCopies sc;
-        const int j = value_wave ? i + VR - 2 : i + KR;
+        const int j = i + (value_wave ? copies_ahead(VR, true) : copies_ahead(KR, false));
         const _Float16 *page = value_wave ? vp : kp;
         sc.src = reinterpret_cast<const char *>(page + (size_t)page_block(source_block(j, nb)) * (32 * D)) + (value_wave ? 0 : my_chunk * 1024);
         sc.dst = smem_base + (unsigned)((value_wave ? V_OFF : 0) + role_ring(j + slot_off) * SLOT_BYTES + w4 * CPW * 1024);
@@ -321,12 +307,15 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             carry_nb = max((end2 + 31) >> 5, 0);
         }
         if (!carried) {
+            // K of steps 0 .. KR - 1, V of steps 0 .. VR - 3, each to a place of its own: nothing orders two copies in flight.  (The value
+            // waves once took the score waves' KR turns: with a ring of three, two different blocks on their way to one place.)
 #pragma unroll
-            for (int i = -KR; i < 0; ++i) issue_step(i, nb);  // K of steps 0 .. KR - 1, V of steps 0 .. VR - 3
+            for (int i = -copies_ahead(KR, false); i < 0; ++i)
+                if (!value_wave || i >= -copies_ahead(VR, true)) issue_step(i, nb);
         }
 
-        // End of step i.  What the next step reads from LDS, K(i+2) and V(i+1), was copied KR - 2 and VR - 2 steps before
-        // and must have landed; the copies of the steps since may still fly.  Then the
+        // End of step i.  What the next step reads from LDS, K(i+2) and V(i), was copied in steps i + 2 - KR and i + 2 - VR
+        // and must have landed; the copies of the KR - 2 and VR - 2 steps since may still fly.  Then the
         // barrier that publishes them and this step's P^T.
         auto end_step = [&](auto ring) {
             TT_WAIT_VMCNT((decltype(ring)::value - 2) * CPW);
@@ -359,7 +348,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             __syncthreads();  // every score wave holds K of step 0: step 0 may refill its slot
 #pragma nounroll
             for (int i = 0; i < steps; ++i) {
-                const char *next = smem + in_ring<KR>(i + 1 + slot_off) * SLOT_BYTES + lane * 16;
+                const char *next = smem + in_ring(KR, i + 1 + slot_off) * SLOT_BYTES + lane * 16;
                 const StepCopies sc = step_copies(i, nb);
                 f16v s[NB];
 #pragma unroll
@@ -425,7 +414,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
 #pragma nounroll
             for (int i = 2; i <= steps + 1; ++i) {
                 const int jn = i - 1;  // the step fetched in this one (past the last one: stale but harmless data)
-                const char *next = smem + V_OFF + in_ring<VR>(jn + slot_off) * SLOT_BYTES + lane * 16;
+                const char *next = smem + V_OFF + in_ring(VR, jn + slot_off) * SLOT_BYTES + lane * 16;
                 const char *psrc = p_mine + (jn & 1) * P_STEP;
                 const StepCopies sc = step_copies(i, nb);
                 if (__any(alpha != 1.0f)) {

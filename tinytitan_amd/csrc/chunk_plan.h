@@ -29,6 +29,28 @@ inline int longest_tile_blocks(int start, int q_len, int kv_valid, int window) {
     return longest;
 }
 
+// ---- The chunk kernel's steps and the rings in LDS that its copies fill (attn_prefill.hip).
+
+// Key blocks of 32 that a step takes, and how many steps' K and V the rings in LDS hold.  Heads of 128 take two: a step's MFMAs are then
+// as many as at 256, its two score chains have no link that waits for the one before it, and there is one barrier, one row
+// maximum and one rescale test for 64 keys (32/8 heads, 777 rows behind 5,003 keys 107.5 -> 95.4 us, 4096 behind 8,000
+// 770 -> 710; V's ring holds three so that all of it stays within 160 KiB).  Two workgroups of one block a step on a CU (rings
+// of three, 128 registers) came to 721 where the chip is full and lost 5 % where it is not.
+constexpr int step_blocks(int D) { return D == 128 ? 2 : 1; }
+constexpr int k_ring(int) { return 4; }
+constexpr int v_ring(int D) { return D == 128 ? 3 : 4; }
+constexpr int in_ring(int ring, int j) { return (int)((unsigned)j % (unsigned)ring); }  // j >= 0
+// Step i, and in front of step 0 a turn for each i below it down to -copies_ahead, issues the copies of step i + copies_ahead.
+constexpr int copies_ahead(int ring, bool of_v) { return of_v ? ring - 2 : ring; }
+// What is copied for step j of a range of `nb` blocks from block `first` on: the `which`-th of the step's blocks.  Past the range's last the
+// last again, or, when a second tile follows (of `carry` blocks, from block 0), that tile's first, a ring of them; then
+// a slot's blocks again: the same bytes.
+constexpr int copied_block(int step, int ring, int j, int which, int first, int nb, int carry) {
+    const int steps = (nb + step - 1) / step;
+    const int at = j < steps || carry == 0 ? step * j + which : step * in_ring(ring, j - steps) + which;
+    return j < steps || carry == 0 ? first + (at < nb ? at : nb - 1) : (at < carry ? at : carry - 1);
+}
+
 // What a chunk costs by the routes that serve it, in us, from timings at 16 q heads / 2 KV heads of 256, 8 / 2 of 256, 32 / 8 of
 // 128 and 16 / 4 of 64, 512 to 4096 rows behind 0 to 9000 keys, whole and through windows of 1024 and 4096 keys.  `first_blocks`
 // and `last_blocks`: the key blocks its first and its last tile of 32 rows walk.
