@@ -161,3 +161,36 @@ def test_heads_of_128_in_steps_of_two_blocks(gpu_ctx, H, KH, rows, start, window
         want = oracle.prefill_ref(q[row:row + 1].astype(np.float32), k32, v32, H * D, KH * D, D, H, KH, start + row, 1, start + row + 1,
                                   window, scale).reshape(1, -1) / (1 + np.exp(-g[row:row + 1].astype(np.float64)))
         _check(got[row:row + 1], want, f"row {row} of {rows} behind {start} keys, {H}q/{KH}kv/{D}, window {window}")
+
+
+@pytest.mark.parametrize("rows,kv_valid,first", [(128, 6200, 24), (128, 6300, 24), (160, 6400, 24), (160, 7300, 24), (545, 545, 0), (545, 577, 0)])
+def test_infinite_values_reach_the_output_as_they_are(gpu_ctx, rows, kv_valid, first):
+    # Key ranges of 13, 11, 17 and 18 blocks, and a whole tile of one row and 18 or 19 blocks: an infinite value in a visible key's
+    # dim makes that dim infinite, whichever block it lies in -- the step that has one block left must not add it again with
+    # probabilities of zero.  Every block from `first` on that all of the checked rows see has an infinity, in one of the dims
+    # 0 .. 95 each; the other dims against the oracle.
+    import torch
+    from tinytitan_amd.engine import KVCacheManager
+    H, KH, D = 8, 2, 128
+    start, scale = kv_valid - rows, float(D) ** -0.5
+    r = np.random.default_rng(kv_valid + rows)
+    k, v = (r.standard_normal((kv_valid, KH, D)).astype(np.float16) for _ in range(2))
+    q = (0.05 * r.standard_normal((rows, H * D))).astype(np.float16)
+    checked = slice(rows - 1, rows) if rows > 512 else slice(0, rows)  # (a last tile of one row)
+    seen = start + checked.start + 1
+    infinite = v.copy()
+    dims = np.zeros(D, bool)
+    for block in range(first, (seen + 31) // 32 if rows > 512 else seen // 32):
+        infinite[min(32 * block + 31, seen - 1), :, block % 96] = np.inf
+        dims[block % 96] = True
+    kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=1, max_context=kv_valid, initial_capacity=kv_valid)
+    kd, vd = _dev(k), _dev(infinite)
+    torch.cuda.synchronize()
+    kv.append(0, 0, 0, kd, vd)
+    gpu_ctx.synchronize()
+    got = _prefill(gpu_ctx, kv, q, start, rows, kv_valid, H, scale)[checked].reshape(-1, H, D)
+    kv.close()
+    assert (got[:, :, dims] == np.inf).all(), f"dims {sorted(set(np.argwhere(dims[None, None] & (got != np.inf))[:, 2].tolist()))}"
+    want = oracle.attention_batch(q.astype(np.float32), k.reshape(kv_valid, -1).astype(np.float32), v.reshape(kv_valid, -1).astype(np.float32),
+                                  rows, start, H, KH, D, scale, threads=4).reshape(rows, H, D)[checked]
+    _check(got[:, :, ~dims], want[:, :, ~dims], f"{rows} rows, {kv_valid} keys")

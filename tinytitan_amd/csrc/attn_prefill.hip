@@ -153,7 +153,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     constexpr int KS = D / 16;  // k-steps of S^T
     constexpr int MT = D / 32;  // 32-dim tiles of O^T
     constexpr int BLOCK_BYTES = 32 * D * 2;
-    constexpr int NB = step_blocks(D);            // key blocks per step
+    constexpr int NB = step_blocks(D);            // key blocks per step: one or two
+    static_assert(NB <= 2);
     constexpr int KR = k_ring(D), VR = v_ring(D);
     constexpr int SLOT_BYTES = NB * BLOCK_BYTES;
     constexpr int CHUNKS = BLOCK_BYTES / 1024;    // 1 KiB chunks per block (= KS = 2 MT)
@@ -412,7 +413,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             float alpha = alpha_mine[0];
             end_step(v_landed);  // step 1
 #pragma nounroll
-            for (int i = 2; i <= steps + 1; ++i) {
+            for (int i = 2; i <= nb / NB + 1; ++i) {
                 const int jn = i - 1;  // the step fetched in this one (past the last one: stale but harmless data)
                 const char *next = smem + V_OFF + in_ring(VR, jn + slot_off) * SLOT_BYTES + lane * 16;
                 const char *psrc = p_mine + (jn & 1) * P_STEP;
@@ -449,6 +450,22 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
                     }
                 }
                 end_step(v_landed);
+            }
+            if constexpr (NB > 1) {
+                // An odd range's last block, without the copy of it that lies in the second one's place: its probabilities are zero, but
+                // zero times an infinite value is not.
+                if (nb % NB != 0) {
+                    issue_step(steps + 1, nb);
+                    if (__any(alpha != 1.0f)) {
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) o[mt] *= alpha;
+                    }
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[2 * mt + t], pf[t], o[mt], 0, 0, 0);
+                    end_step(v_landed);
+                }
             }
             TT_WAIT_VMCNT(0);
             __syncthreads();  // the row sums are in LDS
