@@ -148,14 +148,12 @@ __device__ __forceinline__ float softmax_step(const f16v (&s_raw)[NB], bool mask
 
 }  // namespace
 
-template <int D>
+template <int D, int NB>  // NB: key blocks per step, one or two
 __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(const PrefillArgs a) {
     constexpr int KS = D / 16;  // k-steps of S^T
     constexpr int MT = D / 32;  // 32-dim tiles of O^T
     constexpr int BLOCK_BYTES = 32 * D * 2;
-    constexpr int NB = step_blocks(D);            // key blocks per step: one or two
-    static_assert(NB <= 2);
-    constexpr int KR = k_ring(D), VR = v_ring(D);
+    constexpr int KR = k_ring(NB), VR = v_ring(NB);
     constexpr int SLOT_BYTES = NB * BLOCK_BYTES;
     constexpr int CHUNKS = BLOCK_BYTES / 1024;    // 1 KiB chunks per block (= KS = 2 MT)
     constexpr int CPW = NB * CHUNKS / 4;          // copies one wave issues per step (K and V of a step's blocks over 8 waves)
@@ -530,27 +528,28 @@ bool prefill_kernel_serves(int n_q_heads, int n_kv_heads, int head_dim, bool ali
 }
 
 // the rings of K and V (128 KiB at D = 256, 112 at 128) + P^T hand-over (16, 32 KiB) + rescale factors and row sums + the output rows' staging (10 KiB)
-static constexpr int prefill_lds_bytes(int D) {
-    return (k_ring(D) + v_ring(D)) * step_blocks(D) * 32 * D * 2 + 2 * 4 * step_blocks(D) * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80;
+static constexpr int prefill_lds_bytes(int D, int NB) {
+    return (k_ring(NB) + v_ring(NB)) * NB * 32 * D * 2 + 2 * 4 * NB * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80;
 }
-static_assert(prefill_lds_bytes(256) <= 160 * 1024 && prefill_lds_bytes(128) <= 160 * 1024, "a CU's LDS");
+static_assert(prefill_lds_bytes(256, 1) <= 160 * 1024 && prefill_lds_bytes(128, 2) <= 160 * 1024, "a CU's LDS");
 
+template <int D, int NB>
+static hipError_t configure_prefill() {
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_kernel<D, NB>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               prefill_lds_bytes(D, NB));
+}
 int configure_prefill_kernels(tt_hip_ctx *ctx) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_kernel<256>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, prefill_lds_bytes(256));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_kernel<128>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, prefill_lds_bytes(128));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_kernel<64>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, prefill_lds_bytes(64));
+    hipError_t e = configure_prefill<256, 1>();
+    if (e == hipSuccess) e = configure_prefill<128, 1>();
+    if (e == hipSuccess) e = configure_prefill<128, 2>();
+    if (e == hipSuccess) e = configure_prefill<64, 1>();
     return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "hipFuncSetAttribute(chunk kernel max dynamic LDS)");
 }
 
-template <int D>
+template <int D, int NB>
 static int launch_prefill_d(tt_hip_ctx *ctx, const PrefillArgs &args, unsigned grid) {
-    constexpr int lds = prefill_lds_bytes(D);
-    auto kernel = attn_prefill_kernel<D>;  // (its LDS limit was raised when the first context on this device was created)
+    constexpr int lds = prefill_lds_bytes(D, NB);
+    auto kernel = attn_prefill_kernel<D, NB>;  // (its LDS limit was raised when the first context on this device was created)
     launch_profiled(ctx, kernel, dim3(grid), dim3(512), (unsigned)lds, args);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "attn_prefill_kernel launch");
@@ -601,10 +600,12 @@ int launch_prefill(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot, int star
         a.xcd_chunk = (a.per_kvh * a.n_splits + a.xs - 1) / a.xs;
         grid = 8u * (unsigned)a.xcd_chunk;
     }
+    const int walk = a.n_splits > 1 ? std::min(split_blocks, most_tile_blocks(start, q_len, kv_valid, window))
+                                    : most_tile_blocks(start, q_len, kv_valid, window);
     switch (kv->head_dim) {
-        case 256: return launch_prefill_d<256>(ctx, a, grid);
-        case 128: return launch_prefill_d<128>(ctx, a, grid);
-        case 64: return launch_prefill_d<64>(ctx, a, grid);
+        case 256: return launch_prefill_d<256, 1>(ctx, a, grid);
+        case 128: return step_blocks(128, walk) == 2 ? launch_prefill_d<128, 2>(ctx, a, grid) : launch_prefill_d<128, 1>(ctx, a, grid);
+        case 64: return launch_prefill_d<64, 1>(ctx, a, grid);
         default: return TT_HIP_ERR_SHAPE;
     }
 }

@@ -31,14 +31,17 @@ inline int longest_tile_blocks(int start, int q_len, int kv_valid, int window) {
 
 // ---- The chunk kernel's steps and the rings in LDS that its copies fill (attn_prefill.hip).
 
-// Key blocks of 32 that a step takes, and how many steps' K and V the rings in LDS hold.  Heads of 128 take two: a step's MFMAs are then
-// as many as at 256, its two score chains have no link that waits for the one before it, and there is one barrier, one row
-// maximum and one rescale test for 64 keys (32/8 heads, 777 rows behind 5,003 keys 107.5 -> 95.4 us, 4096 behind 8,000
-// 770 -> 710; V's ring holds three so that all of it stays within 160 KiB).  Two workgroups of one block a step on a CU (rings
-// of three, 128 registers) came to 721 where the chip is full and lost 5 % where it is not.
-constexpr int step_blocks(int D) { return D == 128 ? 2 : 1; }
+// Key blocks of 32 that a step takes.  Heads of 128 take two: a step's MFMAs are then as many as at 256, its two score chains have no
+// link that waits for the one before it, and there is one barrier, one row maximum and one rescale test for 64 keys
+// (32/8 heads, 777 rows behind 5,003 keys 107.5 -> 95.4 us, 4096 behind 8,000 770 -> 710).  Two workgroups of one block a step on
+// a CU (rings of three, 128 registers) came to 721 where the chip is full and lost 5 % where it is not.  Not where a tile
+// walks so few that the steps in front of the first product and a half empty last step weigh more (one at a time / two, 64/8 heads,
+// 2,048 rows behind windows of 33 and 96 keys, three and five blocks: 46.0 / 49.1 us, 50.3 / 53.6; over three head counts and 256 to 4,096
+// rows seven blocks are 2 % slower in twos, six and eight 1 % faster).
+constexpr int step_blocks(int D, int walk) { return D == 128 && (walk == 6 || walk > 7) ? 2 : 1; }
+// How many steps' K and V the rings in LDS hold: with two blocks a step three of V, so that all of it stays within 160 KiB.
 constexpr int k_ring(int) { return 4; }
-constexpr int v_ring(int D) { return D == 128 ? 3 : 4; }
+constexpr int v_ring(int step) { return step == 2 ? 3 : 4; }
 constexpr int in_ring(int ring, int j) { return (int)((unsigned)j % (unsigned)ring); }  // j >= 0
 // Step i, and in front of step 0 a turn for each i below it down to -copies_ahead, issues the copies of step i + copies_ahead.
 constexpr int copies_ahead(int ring, bool of_v) { return of_v ? ring - 2 : ring; }
@@ -49,6 +52,12 @@ constexpr int copied_block(int step, int ring, int j, int which, int first, int 
     const int steps = (nb + step - 1) / step;
     const int at = j < steps || carry == 0 ? step * j + which : step * in_ring(ring, j - steps) + which;
     return j < steps || carry == 0 ? first + (at < nb ? at : nb - 1) : (at < carry ? at : carry - 1);
+}
+
+// At most this many blocks a tile walks: of all keys up to its last row's, those that the windows of 32 rows can touch.
+inline int most_tile_blocks(int start, int q_len, int kv_valid, int window) {
+    const int all = (int)((std::min<long long>(kv_valid, (long long)start + q_len) + 31) / 32);
+    return window > 0 ? (int)std::min<long long>(all, ((long long)window + 61) / 32 + 1) : all;
 }
 
 // What a chunk costs by the routes that serve it, in us, from timings at 16 q heads / 2 KV heads of 256, 8 / 2 of 256, 32 / 8 of
