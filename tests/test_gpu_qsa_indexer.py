@@ -770,3 +770,20 @@ def test_long_rows_thinned_to_a_block_a_thread(gpu_ctx, blocks, width, kind):
     _check_rows(both, scores, rows, first, ratio, width)
     _, idx, cnt = _select(gpu_ctx, scores, rows, first, ratio, width, mask=False)
     assert np.array_equal(cnt, both[2]) and all(np.array_equal(idx[r, :cnt[r]], both[1][r, :cnt[r]]) for r in range(rows))
+
+
+@pytest.mark.parametrize("rows,blocks", [(257, 8193), (257, 16384), (1024, 8200), (1025, 16000), (1024, 8192)])
+@pytest.mark.parametrize("mask", [True, False])
+def test_rows_of_a_chunk_on_both_sides_of_the_forms(gpu_ctx, rows, blocks, mask):
+    # More rows than the card has CUs: rows of 8,193 to 16,384 blocks two workgroups a CU, also from 1,024 rows on, where shorter rows
+    # go to small workgroups.  Scores of few values tie; the last row sees all blocks and one cell.
+    rng = np.random.default_rng(rows + blocks)
+    scores = rng.standard_normal((rows, blocks)).astype(np.float32)
+    scores[1::3] = np.round(scores[1::3], 1)
+    visible = blocks * RATIO + 1 - (rows - 1)
+    keep, idx, cnt = _select(gpu_ctx, scores, rows, visible, RATIO, 2051, mask=mask)
+    for r in {0, 1, 2, 255, 256, rows // 2, rows - 2, rows - 1}:
+        _, want, want_idx = oracle.qsa_select_keys(scores[r], visible + r, RATIO, 2051)
+        assert cnt[r] == len(want_idx) and np.array_equal(idx[r, :cnt[r]].astype(np.uint32), want_idx), r
+        if mask:
+            assert np.array_equal(keep[r, :visible + r], want) and not keep[r, visible + r:].any(), r

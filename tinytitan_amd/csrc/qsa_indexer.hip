@@ -771,8 +771,10 @@ __global__ __launch_bounds__(kSelectThreads) void qsa_select_stream_kernel(const
 // consecutive blocks, so a ballot is 64 blocks' worth of a bitmap; the words, in block order, get
 // one thread each: an exclusive sum of their bit counts over the workgroup, then the set bits.
 // At most one block (the one at the rank) gives `partial` cells; whole blocks behind it shift by that.
-template <int KPT, int THREADS>
-__global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a) {
+// WAVES: the wavefronts a SIMD shall have room for -- eight are two workgroups of 1,024 threads a CU, which 16 scores a thread do
+// not come to by themselves (90 scalar registers are held in vector lanes then).
+template <int KPT, int THREADS, int WAVES = 1>
+__global__ __launch_bounds__(THREADS, WAVES) void qsa_select_kernel(const SelectArgs a) {
     __shared__ unsigned hist[256];
     __shared__ unsigned wave_totals[THREADS / 64];
     __shared__ unsigned long long bitmap_sh[KPT * (THREADS / 64)];  // bit l of word (j, wavefront): that lane's block j is kept whole
@@ -836,9 +838,9 @@ __global__ __launch_bounds__(THREADS) void qsa_select_kernel(const SelectArgs a)
         }
         // The score's two upper bytes at once (see choose_wide); the 8-bit passes go on from the third byte, or from
         // the first when the rank lies below the window.
-        if (top16 == 0u) top16 = upper_bits_of_largest(largest_of(keys));
         for (unsigned b = tid; b < kWideBins; b += THREADS) wide[b] = 0u;
-        __syncthreads();
+        if (top16 == 0u) top16 = upper_bits_of_largest(largest_of(keys));  // (with a barrier)
+        else __syncthreads();
         {
             const unsigned tid = opaque(threadIdx.x);
 #pragma unroll
@@ -1782,9 +1784,11 @@ extern "C" int tt_hip_qsa_select(tt_hip_ctx *ctx, const float *scores, size_t sc
     // barriers and more of them fit a CU.  Fewer rows want their latency short: 1024 threads each.
     constexpr int kSmall = 256;
     const dim3 small_wg(kSmall);
-    // (from 1024 rows on: 128 rows behind 32k keys take 53.0 us a step with the small workgroups and 35.8 us with the
-    // large ones, 256 rows behind 16k keys 47.7 / 35.4, 512 rows behind 2k keys 28.3 / 26.4, 1024 rows behind 8k keys
-    // 58.4 / 57.6, 2048 rows behind 16k keys 116.6 / 121.3, 4096 rows from position 0 64.2 / 78.7)
+    // (from 1024 rows on and up to 8,192 blocks: 128 rows behind 32k keys take 53.0 us a step with the small workgroups and 35.8
+    // us with the large ones, 256 rows behind 16k keys 47.7 / 35.4, 512 rows behind 2k keys 28.3 / 26.4, 1024 rows of 5,000 blocks
+    // 20.4 where 1,023 take 25.2 in large ones, of 8,100 22.1 / 25.9.  With 64 scores a thread a CU holds three small ones,
+    // three wavefronts a SIMD, or two large ones, eight: 1024 rows of 9,000 blocks 45.4 / 31.9 us, 1500 51.9 / 45.9, 2048 69.4 / 59.4, of
+    // 16,000 49.1 / 34.8, 56.7 / 48.6, 75.9 / 63.2.)
     constexpr int small_from = 1024;
     // scores per thread: the smallest of 1, 2, 4, 8, 16, 32, 64 that holds the row (every unused one is a turn of
     // each unrolled loop all the same)
@@ -1792,11 +1796,13 @@ extern "C" int tt_hip_qsa_select(tt_hip_ctx *ctx, const float *scores, size_t sc
     else if (rows >= small_from && max_blocks <= 8LL * kSmall) hipLaunchKernelGGL((qsa_select_kernel<8, kSmall>), grid, small_wg, 0, ctx->stream, a);
     else if (rows >= small_from && max_blocks <= 16LL * kSmall) hipLaunchKernelGGL((qsa_select_kernel<16, kSmall>), grid, small_wg, 0, ctx->stream, a);
     else if (rows >= small_from && max_blocks <= 32LL * kSmall) hipLaunchKernelGGL((qsa_select_kernel<32, kSmall>), grid, small_wg, 0, ctx->stream, a);
-    else if (rows >= small_from && max_blocks <= 64LL * kSmall) hipLaunchKernelGGL((qsa_select_kernel<64, kSmall>), grid, small_wg, 0, ctx->stream, a);
     else if (max_blocks <= 1LL * kSelectThreads) hipLaunchKernelGGL((qsa_select_kernel<1, kSelectThreads>), grid, wg, 0, ctx->stream, a);
     else if (max_blocks <= 2LL * kSelectThreads) hipLaunchKernelGGL((qsa_select_kernel<2, kSelectThreads>), grid, wg, 0, ctx->stream, a);
     else if (max_blocks <= 4LL * kSelectThreads) hipLaunchKernelGGL((qsa_select_kernel<4, kSelectThreads>), grid, wg, 0, ctx->stream, a);
     else if (max_blocks <= 8LL * kSelectThreads) hipLaunchKernelGGL((qsa_select_kernel<8, kSelectThreads>), grid, wg, 0, ctx->stream, a);
+    // (two workgroups a CU, once there are more rows than CUs: 257 rows of 9,000 blocks 23.0 -> 16.7 us, 1023 47.0 -> 31.9; up to 256 13.2, where
+    // the form that leaves a second one room takes 13.6)
+    else if (max_blocks <= 16LL * kSelectThreads && rows > ctx->n_cus) hipLaunchKernelGGL((qsa_select_kernel<16, kSelectThreads, 8>), grid, wg, 0, ctx->stream, a);
     else if (max_blocks <= 16LL * kSelectThreads) hipLaunchKernelGGL((qsa_select_kernel<16, kSelectThreads>), grid, wg, 0, ctx->stream, a);
     else if (max_blocks <= 32LL * kSelectThreads) hipLaunchKernelGGL((qsa_select_kernel<32, kSelectThreads>), grid, wg, 0, ctx->stream, a);
     else if (max_blocks <= 64LL * kSelectThreads) hipLaunchKernelGGL((qsa_select_kernel<64, kSelectThreads>), grid, wg, 0, ctx->stream, a);
