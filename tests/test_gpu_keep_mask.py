@@ -985,17 +985,13 @@ def test_lists_whose_tiles_do_not_divide_the_chip_in_whole_rounds(bits, D, H, KH
     _check(eager[some], want, f"whole rounds D={D} {H}/{KH} bits {bits}")
 
 
-@pytest.mark.parametrize("H,KH,T,rows,past", [(16, 2, 3199, 33, 0), (16, 2, 3200, 33, 0), (16, 2, 3203, 33, 1), (24, 2, 4611, 301, 0), (40, 2, 3300, 260, 0)])
-def test_wide_lists_and_many_tiles_of_wide_heads_equal_the_mask_form(gpu_ctx, H, KH, T, rows, past):
-    # Heads of 256 on both sides of the line between groups of keys and blocks: the shortest contexts that are walked by groups,
-    # the widest lists (`past`: one entry wider), and more tiles than half of the CUs.
+def _lists_equal_the_mask_form(gpu_ctx, H, KH, T, rows, stride):
     import torch
     from tinytitan_amd.engine import PrefillAttention, PrefillAttentionParams
     D = 256
     r = np.random.default_rng(T + H)
     start, scale = T - rows, D ** -0.5
     tt = 32 // (H // KH)
-    stride = 8 * T // (9 * tt) + past
     keep = np.zeros((rows, ((T + 3) // 4) * 4), np.uint8)
     for t in range(rows):
         for g in r.choice((start + t) // 4, [stride // 4 - 1, 3, stride // 8][t % 3], replace=False):
@@ -1021,4 +1017,18 @@ def test_wide_lists_and_many_tiles_of_wide_heads_equal_the_mask_form(gpu_ctx, H,
     assert np.abs(got - by_mask).max() <= 2e-3
     some = [0, 1, 2, tt, rows - 1]
     want = np.concatenate([_oracle_rows_kept(q[t:t + 1], k, v, start + t, keep[t:t + 1], H, KH, D, scale, gate=gate[t:t + 1]) for t in some])
-    _check(got[some], want, f"wide lists {H}/{KH} T={T}")
+    _check(got[some], want, f"lists of {stride} {H}/{KH} T={T}")
+
+
+@pytest.mark.parametrize("H,KH,T,rows,past", [(16, 2, 3199, 33, 0), (16, 2, 3200, 33, 0), (16, 2, 3203, 33, 1), (24, 2, 4611, 301, 0), (40, 2, 3300, 260, 0)])
+def test_wide_lists_and_many_tiles_of_wide_heads_equal_the_mask_form(gpu_ctx, H, KH, T, rows, past):
+    # Heads of 256 on both sides of the line between groups of keys and blocks: the shortest contexts that are walked by groups,
+    # the widest lists (`past`: one entry wider), and more tiles than half of the CUs.
+    _lists_equal_the_mask_form(gpu_ctx, H, KH, T, rows, 8 * T // (9 * (32 // (H // KH))) + past)
+
+
+@pytest.mark.parametrize("H,KH,T,rows,past", [(16, 2, 3100, 40, 0), (16, 2, 3100, 40, 1), (24, 2, 2999, 300, 0), (8, 2, 600, 520, 0), (8, 2, 600, 520, 1),
+                                              (40, 2, 1025, 130, 0)])
+def test_lists_of_half_the_keys_of_wide_heads_equal_the_mask_form(gpu_ctx, H, KH, T, rows, past):
+    # Heads of 256 behind few keys: groups of keys up to lists of half of them, blocks with an entry more; few tiles and many.
+    _lists_equal_the_mask_form(gpu_ctx, H, KH, T, rows, T // (2 * (32 // (H // KH))) + past)

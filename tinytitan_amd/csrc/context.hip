@@ -354,13 +354,16 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             // Where the tile's lists could hold most of the keys, most of a block is wanted and its loads are the better ones.
             // Heads of 256, whose groups lie in lines of their own (kv_layout.h): as long as the lists hold no more than eight
             // ninths of the keys, from 3,200 keys on (by blocks / by groups: 24/2 heads, 300 rows behind 4,500 keys 130 / 126 us, 512
-            // behind 9,000 226 / 150, behind 64,000 593 / 212, 40/2 heads, 512 behind 3,500 209 / 185, behind 2,500 171 / 182).
+            // behind 9,000 226 / 150, behind 64,000 593 / 212, 40/2 heads, 512 behind 3,500 209 / 185, behind 2,500 171 / 182).  With fewer
+            // keys as long as they hold no more than half of them (lists of 256 keys, 24/2 heads, 300 rows behind 2,700 keys 78.7 / 49.1,
+            // 128 rows 39.5 / 30.0; of 32 keys, 8/2 heads, 512 rows behind 1,800 38.5 / 28.8; all rows with one list of 64, 16/2 heads, 64
+            // rows behind 2,700 26.1 / 27.3).
             // Narrower heads: half of the keys (8k keys, 512 rows: 121.7 against 133.4 us), and a bound on the tiles: many share
             // fetched lines in L2 only while they stay side by side, which the walk over blocks does better (inside the bound 512 rows of
             // heads of 64 behind 131k keys 470 -> 208 us).  The group bitmap has to leave the plan kernel's LDS room for a run of bits.
             const long long entries = (long long)plan.tt * (long long)lists->stride;
             groups = kv_bits == 16 && plan.nt == 32 && totals[base] <= kPlanGroupKeys &&
-                     (D == 256 ? 9 * entries <= 8ll * totals[base] && totals[base] >= 3200
+                     (D == 256 ? 2 * entries <= totals[base] || (9 * entries <= 8ll * totals[base] && totals[base] >= 3200)
                                : 2 * entries <= totals[base] && (long long)plan.n_tiles * D <= 128ll * ctx->n_cus);
             const int unit = groups ? 4 : 32;
             ctx_units = (totals[base] + unit - 1) / unit;
