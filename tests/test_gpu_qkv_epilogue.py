@@ -102,8 +102,17 @@ def test_chunk_whole_blocks_and_ragged_edges(gpu_ctx, position, rows):
 
 @pytest.mark.parametrize("H,KH,D,rot,rows", [(16, 4, 64, 64, 643), (16, 4, 64, 64, 644), (8, 1, 64, 32, 700), (16, 2, 256, 256, 391), (32, 8, 128, 64, 385)])
 def test_chunks_on_both_sides_of_the_block_rule(gpu_ctx, H, KH, D, rot, rows):
-    # narrow heads go on by rows until those are more than 160 workgroups; whole blocks with every slot of angles in use
+    # chunks of several head counts by blocks and by rows; whole blocks with every slot of angles in use
     kv = _run(gpu_ctx, H, KH, D, rot, 1, rows, [39], [0], seed=rows)
+    kv.close()
+
+
+@pytest.mark.parametrize("position", [0, 5])
+@pytest.mark.parametrize("H,KH,D,rows", [(16, 4, 64, 256), (16, 4, 64, 260), (16, 16, 64, 127), (16, 16, 64, 128), (16, 2, 256, 513), (16, 2, 256, 514),
+                                         (24, 2, 256, 408), (24, 2, 256, 412), (8, 8, 256, 128), (8, 8, 256, 129), (32, 8, 128, 257), (16, 2, 256, 576)])
+def test_chunks_on_both_sides_of_a_workgroup_for_every_cu(gpu_ctx, H, KH, D, rows, position):
+    # whole blocks from where the rows' workgroups outnumber the CUs (heads of 64: a quarter of them; many query heads: earlier)
+    kv = _run(gpu_ctx, H, KH, D, 64, 1, rows, [position], [0], seed=rows)
     kv.close()
 
 

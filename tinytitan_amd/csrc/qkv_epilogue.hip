@@ -289,6 +289,8 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs ta
         _Float16 *kt = tile, *vt = tile + kBlockTokens * ROW;
         const int token0 = a.head_rows + blk * kBlockTokens;
         const int position0 = tables.position[0] + token0;
+        Frequencies freq;
+        if constexpr (NI == 1) freq = load_frequencies<LPS>(a.rotary_half, tables.freq, lane);
         h8 k[NI], v[NI];
 #pragma unroll
         for (int i = 0; i < NI; ++i) {  // all of the wavefront's rows in flight at once
@@ -297,15 +299,20 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(const EpilogueArgs ta
             k[i] = load_halves<ALIGNED>(a.k_proj + off);
             v[i] = load_halves<ALIGNED>(a.v_proj + off);
         }
-        Frequencies freq = load_frequencies<LPS>(a.rotary_half, tables.freq, lane);
+        if constexpr (NI > 1) freq = load_frequencies<LPS>(a.rotary_half, tables.freq, lane);
         const WeightBits weight = load_weight(a.k_weight, d0);
         freq.pin();
+        Rotation rot;
+        if constexpr (NI == 1) {  // (D = 64, one access a wavefront: its angles while the rows are on their way; 16/16 heads, 512 tokens 5.6 -> 5.0 us)
+            rot = rotation_for<LPS>(a.rotary_half, freq, position0 + wave * RPW + sub, lane, d0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         float w[E];
         to_floats(w, weight);
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int row = wave * RPW + i * SPW + sub;
-            const Rotation rot = rotation_for<LPS>(a.rotary_half, freq, position0 + row, lane, d0);
+            if constexpr (NI > 1) rot = rotation_for<LPS>(a.rotary_half, freq, position0 + row, lane, d0);
             float x[E];
             to_floats(x, k[i]);
             norm_rope<D>(x, w, a.eps, rot);
@@ -499,12 +506,17 @@ extern "C" int tt_hip_qkv_epilogue_append(tt_hip_ctx *ctx, tt_hip_kv *kv, int la
     // Whole blocks only for one sequence (a prefill chunk); decode and verify rows are few.
     int first_full = 0, last_full_end = 0;
     const int row0 = a.row0[0];  // whole blocks are blocks of the page: counted from where the rows are stored
-    // (quantised pages: every row through the row path, which quantises.  Short chunks too: a block's workgroup writes
-    // its 32 tokens one after the other, and with a handful of blocks those few workgroups are the whole launch's time:
-    // 16/2 heads of 256, 384 tokens 6.8 us by blocks, 6.2 by rows, 512 tokens 7.2 / 7.5; 32/8 of 128, 384 tokens 6.0 / 8.0; 16/4
-    // of 64, 512 tokens 5.4 / 5.1, 777 tokens 5.4 / 5.8.)
+    // (quantised pages: every row through the row path, which quantises.  And chunks whose rows find a CU for each of their
+    // workgroups, of four wavefronts and 2 x 64 / (D / 8) rows of K and V: a block's workgroup writes its 32 tokens one after the other,
+    // 6 us however few there are.  By rows / by blocks: 16/2 heads of 256, 512 tokens (256 workgroups) 6.3 / 7.0 us, 576 7.8 / 7.2; 8/2,
+    // 640 (320) 6.0 / 6.7, 700 7.5 / 6.8; 8/8, 256 (512) 6.8 / 6.4; 32/8 of 128, 256 (256) 5.6 / 5.5, 384 8.0 / 5.9.  With more query
+    // heads the launch is full before: 24/2 of 256, 384 (192, and 288 for the queries) 6.2 / 7.1, 448 7.6 / 7.3.  Blocks of 64 dims are
+    // one access a wavefront: 8/2 heads, 512 (64) 4.3 / 4.3, 777 4.7 / 4.4; 16/4, 384 (96) 5.0 / 4.3, 777 5.9 / 5.0.)
     const long long row_path_wgs = (long long)rows * KH / (2 * (64 / (D / 8)));
-    if (n_seq == 1 && kv->bits == 16 && rows >= 384 && row_path_wgs > 160) {
+    const long long query_wgs = (long long)rows * ((n_q_heads + 4 * (64 / (D / 8)) - 1) / (4 * (64 / (D / 8)))) / 4;
+    const bool by_blocks = D == 64 ? 4 * row_path_wgs > ctx->n_cus
+                                   : row_path_wgs > ctx->n_cus || (4 * row_path_wgs > 3LL * ctx->n_cus && row_path_wgs + query_wgs > 2LL * ctx->n_cus);
+    if (n_seq == 1 && kv->bits == 16 && rows >= 4 * kBlockTokens && by_blocks) {
         first_full = ((row0 + kBlockTokens - 1) / kBlockTokens) * kBlockTokens;
         last_full_end = ((row0 + rows) / kBlockTokens) * kBlockTokens;
     }
