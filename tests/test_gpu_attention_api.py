@@ -875,3 +875,34 @@ def test_sequences_of_unlike_lengths_equal_their_own_calls(gpu_ctx, bits, D, H, 
     kv.close()
     assert np.isfinite(together).all()
     assert np.abs(together - alone).max() <= 2e-3
+
+
+@pytest.mark.parametrize("n,rows", [(40956, 4), (40900, 4), (41003, 3)])
+def test_verify_rows_over_more_pages_than_the_caches_hold(gpu_ctx, n, rows):
+    # 8 sequences of 16/2 heads of 256, a workgroup for every CU: from 640 MiB of pages on (40,960 keys each) the V operands of the
+    # 32-row tiles are paired, below they are not.  The oracle on two of the sequences.
+    import torch
+    from tinytitan_amd.engine import Attention, KVCacheManager
+    H, KH, D, seqs = 16, 2, 256, 8
+    total, scale = n + rows, D ** -0.5
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    k, v = (torch.randn(total, KH * D, generator=gen, device="cuda", dtype=torch.float16) for _ in range(2))
+    q, gate = (torch.randn(seqs, rows, H * D, generator=gen, device="cuda", dtype=torch.float16) for _ in range(2))
+    kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=seqs, max_context=total, initial_capacity=total)
+    torch.cuda.synchronize()
+    for s in range(seqs):  # a sequence's keys: the same rows, turned by its number
+        ks, vs = torch.roll(k, s, 0), torch.roll(v, s, 0)
+        torch.cuda.synchronize()
+        kv.append(0, s, 0, ks, vs)
+        gpu_ctx.synchronize()
+    out = torch.full((seqs, rows, H * D), float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    Attention(gpu_ctx).encode_verify_rows(kv, 0, q, out, H, [n] * seqs, rows, scale, list(range(seqs)), gate=gate)
+    gpu_ctx.synchronize()
+    got = out.float().cpu().numpy()
+    kv.close()
+    for s in (1, 6):
+        ks, vs = (torch.roll(t, s, 0).float().cpu().numpy() for t in (k, v))
+        want = oracle.attention_batch(q[s].float().cpu().numpy(), ks, vs, rows, n, H, KH, D, scale, threads=8).reshape(rows, -1)
+        _check(got[s], want / (1 + np.exp(-gate[s].double().cpu().numpy())), f"sequence {s} of {seqs} behind {n} keys")

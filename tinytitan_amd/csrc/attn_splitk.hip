@@ -170,38 +170,28 @@ struct VTile<D, 16> {
     h8 f[D / 16];
 };
 
-// The dims of a 32-row tile's V operands over fp16 pages of heads of 256.  A 128-byte line there holds eight dims of a chunk; two
-// operand tiles in a row share the lines of the same 64 dims, the first one's rows the lower four dims of each line, the
-// second one's the upper four.  So the first of their loads asks for all of those lines -- as it does over narrower heads' [d][chunk],
-// whose lines hold every chunk -- and the second finds them on their way: with one wavefront a SIMD more of them are under way
-// (8 sequences x 4 rows behind 64k keys 181.2 -> 175.2 us).  Tiles of 16 rows, two wavefronts a SIMD, read their contiguous
-// 1 KiB a load (in pairs 32 sequences of 511 .. 16,383 keys 61.3 -> 67.4 us).
-// Row 4 q + i of operand tile mt is dim v_tile_dim(mt) + v_row_dim(4 q + i): four consecutive dims for four consecutive i.
-constexpr bool paired_v_tiles(int head_dim, int nt) { return head_dim == 256 && nt == 32; }
-template <int D, int NT>
-__device__ __forceinline__ constexpr int v_tile_dim(int mt, bool paired = paired_v_tiles(D, NT)) {
-    return paired ? 2 * NT * (mt >> 1) + 4 * (mt & 1) : NT * mt;
-}
-template <int D, int NT>
-__device__ __forceinline__ constexpr int v_row_dim(int row, bool paired = paired_v_tiles(D, NT)) {
-    return paired ? 8 * (row >> 2) + (row & 3) : row;
-}
+// The dims of a 32-row tile's V operands over fp16 pages of heads of 256, where they are paired.  A 128-byte line there holds eight dims of
+// a chunk; two operand tiles in a row then share the lines of the same 64 dims, the first one's rows the lower four dims of
+// each line, the second one's the upper four, so that the first of their loads asks for all of those lines and the second
+// finds them on their way.  Row 4 q + i of operand tile mt is dim v_tile_dim(mt) + v_row_dim(4 q + i).
+__device__ __forceinline__ constexpr int v_tile_dim(int mt, bool paired) { return paired ? 64 * (mt >> 1) + 4 * (mt & 1) : 32 * mt; }
+__device__ __forceinline__ constexpr int v_row_dim(int row, bool paired) { return paired ? 8 * (row >> 2) + (row & 3) : row; }
 
 template <int D, int NT>
 struct Lane {
     static constexpr int LN = NT;
     int li, g;       // position inside the lane group, lane group
     int koff, voff;  // this lane's element offset inside a K / V block
-    __device__ __forceinline__ explicit Lane(int lane) {
+    __device__ __forceinline__ explicit Lane(int lane, bool paired = false) {
         li = lane & (LN - 1);
         g = lane / LN;
         if constexpr (NT == 32) {
             koff = (g * 32 + li) * 8;
-            voff = v_piece(D, v_row_dim<D, NT>(li), g);
+            voff = v_piece(D, v_row_dim(li, paired), g);
         } else {
             const int ka = li < 8 ? li : li + 8;
             koff = (g * 32 + ka) * 8;
-            voff = v_piece(D, v_row_dim<D, NT>(li), g);
+            voff = v_piece(D, li, g);
         }
     }
 };
@@ -220,10 +210,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, un
 // verify pass of a few rows).  Those loads are marked non-temporal: the data is not kept in L2 or in the
 // memory-side cache ahead of lines that will be used again (the split partials, the next layer's weights), and
 // a pass over 64 MiB of pages runs 7 % faster for it (13.5 -> 12.5 us), the step behind it 10 %.
+// With kPaired its V operands are paired (v_tile_dim).
 constexpr int kStreamed = 2;  // the nt bit of a gfx950 buffer load
+constexpr int kPaired = 256;
 template <int AUX>
 __device__ __forceinline__ h8 buf_load_h8(__amdgpu_buffer_rsrc_t rsrc, unsigned lane_bytes, unsigned wave_bytes) {
-    i4 r = __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_bytes, wave_bytes, AUX);
+    i4 r = __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_bytes, wave_bytes, AUX & ~kPaired);
     return __builtin_bit_cast(h8, r);
 }
 
@@ -286,7 +278,7 @@ __device__ __forceinline__ void load_v(VTile<D, NT> &t, __amdgpu_buffer_rsrc_t r
         for (int mt = 0; mt < D / 32; ++mt)
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
-                t.f[mt][tt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[tt], block_bytes + 2 * v_piece(D, v_tile_dim<D, NT>(mt), 2 * tt));
+                t.f[mt][tt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[tt], block_bytes + 2 * v_piece(D, v_tile_dim(mt, AUX & kPaired), 2 * tt));
     } else {
 #pragma unroll
         for (int mt = 0; mt < D / 16; ++mt) t.f[mt] = buf_load_h8<AUX>(rv, lane_bytes + vo.v[0], block_bytes + 2 * v_piece(D, 16 * mt, 0));
@@ -553,7 +545,7 @@ __device__ __forceinline__ void block_softmax_pv_refill(RowState<D, 32> &st, Sco
         for (int t = 0; t < 2; ++t) st.o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vt.f[mt][t], pr.pf[t], st.o[mt], 0, 0, 0);
         asm volatile("" : "+a"(st.o[mt]));
 #pragma unroll
-        for (int t = 0; t < 2; ++t) vt.f[mt][t] = buf_load_h8<AUX>(rv, lane_bytes[t], next_bytes + 2 * v_piece(D, v_tile_dim<D, 32>(mt), 2 * t));
+        for (int t = 0; t < 2; ++t) vt.f[mt][t] = buf_load_h8<AUX>(rv, lane_bytes[t], next_bytes + 2 * v_piece(D, v_tile_dim(mt, AUX & kPaired), 2 * t));
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -1038,7 +1030,7 @@ __device__ __forceinline__ seq_entries seq_table() {
 static_assert(kMaxSeqPerLaunch == 64 && offsetof(SplitKSeq, first_split) == 12, "a lane per sequence");
 static_assert(offsetof(SplitKArgs, hot) == 0 && offsetof(SplitKArgs, seq) == 0x80, "load_hot's offsets");
 
-// STREAM: the launch reads every K/V byte once (see kStreamed).
+// STREAM: the launch reads every K/V byte once (see kStreamed); 2: and its V operands are paired (see v_tile_dim).
 // A row's 32 selection bytes of one key block, as 8 words in two loads (the row stride is a multiple of 4 bytes, which is
 // all a buffer load of four dwords asks for; dwords past the buffer's range read as zero one by one).
 __device__ __forceinline__ void load_row_words(unsigned (&dst)[8], __amdgpu_buffer_rsrc_t rsrc, unsigned bytes) {
@@ -1053,8 +1045,9 @@ __device__ __forceinline__ void load_row_words(unsigned (&dst)[8], __amdgpu_buff
 
 template <int D, int NT, int WAVES, int BITS, int KEEP = 0, int STREAM = 0>
 __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void attn_splitk_kernel(const SplitKArgs args) {
-    constexpr int AUX = STREAM ? kStreamed : 0;
-    constexpr bool PAIRED = paired_v_tiles(D, NT) && BITS == 16 && KEEP != 4;  // (groups of keys and quantised pages: dims as they come)
+    constexpr bool PAIRED = STREAM == 2;
+    static_assert(!PAIRED || (D == 256 && NT == 32 && BITS == 16 && KEEP == 0));
+    constexpr int AUX = (STREAM ? kStreamed : 0) | (PAIRED ? kPaired : 0);
     extern __shared__ float lds[];
     constexpr int ROW = D + kLdsPad;  // staged O row stride in floats
     constexpr int REGION = NT * ROW + NT * 2;
@@ -1062,7 +1055,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     constexpr unsigned BLK_BYTES = BITS == 16 ? 32 * D * 2 : 32 * D * BITS / 8 + 32 * (D / 64) * 4;  // bytes per block
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: block pointers stay in SGPRs
-    const Lane<D, NT> ln(lane);
+    const Lane<D, NT> ln(lane, PAIRED);
     const int li = ln.li, g = ln.g;
     int seq = blockIdx.z;
     SplitKHot a;
@@ -1492,7 +1485,7 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
 #pragma unroll
             for (int vq = 0; vq < 4; ++vq) {
                 f4 x = {st.o[mt][4 * vq], st.o[mt][4 * vq + 1], st.o[mt][4 * vq + 2], st.o[mt][4 * vq + 3]};
-                *reinterpret_cast<f4 *>(region + li * ROW + v_tile_dim<D, NT>(mt, PAIRED) + v_row_dim<D, NT>(8 * vq + 4 * g, PAIRED)) = x;
+                *reinterpret_cast<f4 *>(region + li * ROW + v_tile_dim(mt, PAIRED) + v_row_dim(8 * vq + 4 * g, PAIRED)) = x;
             }
     } else {
 #pragma unroll
@@ -1860,6 +1853,11 @@ template <int D, int NT, int BITS, int KEEP>
 static hipError_t configure_one() {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_splitk_kernel<D, NT, 4, BITS, KEEP, 0>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(lds_bytes_for(D, NT, 4) + keep_list_bytes(KEEP, 4)));
+    if constexpr (D == 256 && NT == 32 && BITS == 16 && KEEP == 0) {
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_splitk_kernel<D, NT, 4, BITS, KEEP, 2>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes_for(D, NT, 4));
+    }
     if constexpr (KEEP < 2) {  // (a chunk's per-query selections come with many token tiles: never streamed)
         if (e == hipSuccess)
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_splitk_kernel<D, NT, 4, BITS, KEEP, 1>),
@@ -1941,6 +1939,9 @@ int launch_splitk(tt_hip_ctx *ctx, const LaunchPlan &plan, int head_dim, int n_s
             if (kv_bits == 4) return launch_one<DD, NN, 4, 4, 1>(ctx, plan, n_seq, args);            \
         }                                                                                            \
         if (plan.stream) {                                                                           \
+            if constexpr (DD == 256 && NN == 32) {                                                   \
+                if (kv_bits == 16 && plan.paired) return launch_one<DD, NN, 4, 16, 0, 2>(ctx, plan, n_seq, args); \
+            }                                                                                        \
             if (kv_bits == 16) return launch_one<DD, NN, 4, 16, 0, 1>(ctx, plan, n_seq, args);       \
             if (kv_bits == 8) return launch_one<DD, NN, 4, 8, 0, 1>(ctx, plan, n_seq, args);         \
             if (kv_bits == 4) return launch_one<DD, NN, 4, 4, 0, 1>(ctx, plan, n_seq, args);         \

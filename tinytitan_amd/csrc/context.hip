@@ -463,6 +463,12 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             const long long kv_bytes = total_keys * (long long)kv->n_kv_heads * (long long)(kv->block_bytes() / kBlockTokens) * 2;
             plan.stream = plan.tok_tiles == 1 && plan.hsubs == 1 && chunk_splits <= 1 && keep_row_stride == 0 &&
                           (ctx->stream_override < 0 ? kv_bytes >= (16ll << 20) : ctx->stream_override != 0);
+            // V operands in pairs where every CU has a workgroup of its own for the whole of a long launch, which is then what the memory
+            // gives (8 sequences x 4 rows of 16/2 heads behind 64k keys, 1 GiB, 179.0 -> 173.8 us a step; behind 45,678, 0.7 GiB,
+            // 121.2 -> 119.7): there the lines asked for early are worth it.  They are not with less to read (one sequence behind 65,540
+            // keys plain / paired 32.5 / 35.5 us, 3 behind 100,003 100.9 / 101.7) nor with idle CUs (20 behind 20,010, 240
+            // workgroups, 130.1 / 132.7), and least of all where several tiles walk the same keys (8 rows, 5 behind 65,540 132.2 / 141.3).
+            plan.paired = plan.stream && plan.workgroups % ctx->n_cus == 0 && kv_bytes >= (640ll << 20);
         }
         // A sequence's splits: what its own keys need (at least one), packed one sequence after the other.
         int first_split[kMaxSeqPerLaunch];

@@ -110,6 +110,7 @@ struct LaunchPlan {
     long long workgroups;
     size_t lds_bytes;
     bool stream;  // every K/V byte is read once by the launch, and there are many of them: non-temporal loads
+    bool paired;  // ... and V operands in pairs, over heads of 256 in tiles of 32 rows
     bool xcd_grid;  // launch with kHotXcdGrid
     int slots_per_cu;  // workgroups that the planner's rule for unlike lengths counts on
     int packed_splits;  // > 0: launch with kHotPackedSplits over this many splits
