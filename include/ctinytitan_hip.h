@@ -617,7 +617,8 @@ TT_HIP_API int tt_hip_qsa_decode_scores(tt_hip_ctx *ctx, const tt_half *raw_keys
  * encodeSelectKeys (QSAIndexer+Scratch.swift:191-284) and the host loop of selectKeysPrefill
  * (QSAIndexer.swift:414-497).  Scores must not be NaN (the reference's comparison has no order for
  * them either).  Rows of more than 16,384 blocks, up to a sixth of the CUs in number (with a mask a quarter), and rows of more than 65,536 are
- * spread over many workgroups through a workspace of 64 MiB that the context allocates on first use.  While a graph is
+ * spread over many workgroups through a workspace of 64 MiB that the context allocates on first use (a workgroup each where it cannot
+ * be had).  While a graph is
  * being captured nothing is allocated: up to 7 such rows, or 8 of more than 32,768 blocks (a decode or verify step at a
  * long context), are refused with TT_HIP_ERR_BUSY until a call outside has, and more rows are recorded as a workgroup each.
  * TT_HIP_ERR_SHAPE: keep_stride below the last row's visible keys, score_stride below its complete

@@ -1683,8 +1683,8 @@ extern "C" int tt_hip_qsa_block_scores(tt_hip_ctx *ctx, const tt_half *query, co
     return timed.finish("qsa_scores_kernel launch");
 }
 
-// Workspace of the multi-workgroup selection, of one size for the context's life (its rows go as many at a time as fit: 340 of
-// 32,768 blocks): every call writes what it reads.
+// Workspace of the multi-workgroup selection, of one size for the context's life: every call writes what it reads.  Rows of up to 65,536
+// blocks that are spread fit at once, of 66,000 blocks 159; more go in turns.
 constexpr size_t kSelectWorkspace = (size_t)64 << 20;
 constexpr int kFewRows = 8;  // rows of a decode or verify step, which are not selected without it
 static int ensure_select_workspace(tt_hip_ctx *ctx) {
@@ -1775,9 +1775,10 @@ extern "C" int tt_hip_qsa_select(tt_hip_ctx *ctx, const float *scores, size_t sc
             }
             return timed.finish("qsa_settle_chunks_kernel launch");
         }
-        // Without the workspace (a capture before any eager call, no memory): a decode or verify step's few rows are refused, as the
-        // header says, rather than recorded as a workgroup each for every replay; all others take the forms below.
-        if (rows <= kFewRows && max_blocks > (rows == kFewRows ? 32ll : 16ll) * kSelectThreads) return st;
+        // Without the workspace: a decode or verify step's few rows in a capture before any eager call are refused, as the
+        // header says, rather than recorded as a workgroup each for every replay; all others, and all where there is no
+        // memory for it, take the forms below.
+        if (st == TT_HIP_ERR_BUSY && rows <= kFewRows && max_blocks > (rows == kFewRows ? 32ll : 16ll) * kSelectThreads) return st;
     }
     Timed timed(ctx);
     // Many rows (a long chunk) fill the chip by themselves: workgroups of 256 threads spend less of their time in
