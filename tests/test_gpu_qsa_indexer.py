@@ -787,3 +787,19 @@ def test_rows_of_a_chunk_on_both_sides_of_the_forms(gpu_ctx, rows, blocks, mask)
         assert cnt[r] == len(want_idx) and np.array_equal(idx[r, :cnt[r]].astype(np.uint32), want_idx), r
         if mask:
             assert np.array_equal(keep[r, :visible + r], want) and not keep[r, visible + r:].any(), r
+
+
+@pytest.mark.parametrize("mask", [True, False])
+def test_more_spread_rows_than_the_workspace_holds_at_once(gpu_ctx, mask):
+    # 165 rows of 66,000 blocks: 159 in the first turn, the others in a second one over the same workspace.
+    rng = np.random.default_rng(165)
+    rows, blocks, width = 165, 66000, 2051
+    first = blocks * RATIO - 1
+    scores = np.maximum(rng.standard_normal((rows, (first + rows - 1) // RATIO + 1), dtype=np.float32), 0.0)
+    keep, idx, cnt = _select(gpu_ctx, scores, rows, first, RATIO, width, mask=mask)
+    assert (cnt == width).all()
+    for r in (0, 80, 157, 158, 159, 160, 164):
+        _, want, want_idx = oracle.qsa_select_keys(scores[r], first + r, RATIO, width)
+        assert np.array_equal(idx[r].astype(np.uint32), want_idx), r
+        if mask:
+            assert np.array_equal(keep[r, :first + r], want) and not keep[r, first + r:].any(), r
