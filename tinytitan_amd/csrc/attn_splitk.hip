@@ -1557,7 +1557,7 @@ __device__ __forceinline__ int splits_of(const TileInfo &ti, int split_len) {
 }
 
 template <int D, int NT>
-__global__ __launch_bounds__(256) void attn_combine_kernel(const SplitKArgs args) {
+__global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] const SplitKArgs args) {  // (load_combine reads them)
     constexpr int DCH = D / 64;
     __shared__ float sm[4][68];
     const int n = blockIdx.x / DCH, dchunk = blockIdx.x - n * DCH;
@@ -1653,7 +1653,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const SplitKArgs args
 constexpr int kCombineRowsSplits = 16;
 
 template <int D, int NT>
-__global__ __launch_bounds__(256) void attn_combine_rows_kernel(const SplitKArgs args) {
+__global__ __launch_bounds__(256) void attn_combine_rows_kernel([[maybe_unused]] const SplitKArgs args) {  // (load_combine reads them)
     constexpr int D4 = D / 4, ROWS = 4;
     static_assert(ROWS * D4 <= 256, "an item a thread");
     const int tile = blockIdx.y, seq = blockIdx.z;
