@@ -1738,15 +1738,15 @@ int plan_launch(const tt_hip_ctx *ctx, int kind, int n_seq, int n_q_heads, int n
         // the partial result) then outweigh reading the cache once per tile of 16.  "Little" is counted in keys walked
         // by tiles of 16 over the whole launch, keys x tiles of 16 x KV heads (figures for 2 KV heads of 256, fp16):
         //  * A few verify rows (up to four tiles of 16 per KV head, whose reads all come from HBM): 4 rows at 8k keys
-        //    17.8 -> 13.1 us, at 2k keys 14.4 -> 10.9, 4 sequences x 4 rows at 4k keys 22.6 -> 16.2, 8 rows at 8k keys
-        //    18.3 -> 15.1; at 64k keys 36.3 against 37.2 the other way.  Over quantised pages the 32-row tile is dearer
-        //    still (4 rows at 64k keys over 8 bits 29.2 -> 25.0 us).
+        //    16.4 -> 13.8 us, at 2k keys 13.5 -> 9.8, 4 sequences x 4 rows at 4k keys 19.5 -> 16.7, 8 rows at 8k keys
+        //    18.6 -> 16.0; at 36k keys 24.1 against 24.3, at 64k keys 32.6 against 35.5 the other way.  Over quantised
+        //    pages the 32-row tile is dearer still (4 rows at 64k keys over 8 bits 28.6 -> 24.6 us).
         //  * A short chunk behind a short context (more tiles, which re-read the same keys from L2), as long as the
         //    tiles are one round of workgroups: 32 rows from position 0 11.0 -> 6.5 us, 128 rows behind 1024 keys
-        //    20.9 -> 17.6, 256 rows behind 1024 keys 26.0 -> 20.7; 128 rows behind 3072 keys 28.2 against 29.6 and 512
-        //    rows from position 0 17.0 against 19.7 the other way.
+        //    18.7 -> 15.0, 256 rows behind 1024 keys 22.8 -> 17.4; 128 rows behind 3072 keys 26.4 against 29.2 the
+        //    other way, and 512 rows from position 0 were 17.0 against 19.7.
         // With 8 KV heads of 128 the same counts hold per KV head four times earlier (4 sequences x 16 rows at 4k keys:
-        // 24.4 us in tiles of 32, 30.0 in tiles of 16; 8 rows at 8k keys 16.7 against 13.4), with 4 of 64 twice.
+        // 22.2 us in tiles of 32, 27.2 in tiles of 16; 8 rows at 8k keys 15.1 against 13.9), with 4 of 64 twice.
         if (small_tiles_ok && p.nt == 32 && p.gh <= 16) {
             const long long tiles16 = (rows + 16 / p.gh - 1) / (16 / p.gh);
             const long long launch_tiles16 = tiles16 * n_kv_heads * (group / p.gh);  // per sequence
