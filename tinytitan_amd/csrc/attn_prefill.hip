@@ -109,12 +109,14 @@ __device__ __forceinline__ void copy16_global_to_lds(const void *base, unsigned 
 // One online-softmax step of the score wave on a block's scores: mask, move the row's reference
 // max where the block max exceeds it by more than the threshold, and produce the
 // probabilities (B operand of the two P.V k-steps) against the reference.  The row sum is taken
-// over the ROUNDED probabilities (dot2 against ones), i.e. over exactly the weights the P.V MFMAs
-// see.  Returns the factor the row's accumulators must be scaled by before this block is added.
+// over the ROUNDED probabilities, i.e. over exactly the weights the P.V MFMAs see, by v_fma_mix_f32: a half of either side
+// joins an fp32 sum in one instruction that runs beside a matrix instruction of the SIMD's other wavefront.  (v_dot2_f32_f16, half as many,
+// waits until the matrix pipe is free: 64 of them beside another wavefront's MFMAs take as long as those do, 64 of any other instruction
+// here 1.25 times their own time.  64/8 heads of 64, 2,048 rows behind 4,000 keys 252.0 -> 235.3 us; 32/8 of 128, 4,096 behind 8,000
+// 729 -> 719; heads of 256, whose softmax is a smaller part, the same.)  Returns the factor the row's accumulators must be scaled by before this block is added.
 template <int NB>
 __device__ __forceinline__ float softmax_step(const f16v (&s_raw)[NB], bool mask, int kbase, int lo, int lim, int g,
                                               float scale_log2e, float &m, float &l, h8 (&pf)[2 * NB]) {
-    const h2 ones = {(_Float16)1.0f, (_Float16)1.0f};
     // The maximum is taken over the raw scores and scaled once (the host sends only chunks with scale > 0 here), and a
     // probability is one fused multiply-add and one exp2 off its raw score.
     float t[16 * NB];
@@ -136,13 +138,16 @@ __device__ __forceinline__ float softmax_step(const f16v (&s_raw)[NB], bool mask
     const float alpha = move ? fast_exp2(m - m_new) : 1.0f;
     l *= alpha;
     m = m_new;
+    float l_odd = 0.0f;  // (two sums: neither waits for the other's last addition)
 #pragma unroll
     for (int v = 0; v < 16 * NB; v += 2) {
         const h2 p = {(_Float16)fast_exp2(__builtin_fmaf(t[v], scale_log2e, -m)), (_Float16)fast_exp2(__builtin_fmaf(t[v + 1], scale_log2e, -m))};
-        l = __builtin_amdgcn_fdot2(p, ones, l, false);
+        asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(l) : "v"(p));
+        asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(l_odd) : "v"(p));
         pf[v >> 3][v & 7] = p[0];
         pf[v >> 3][(v & 7) + 1] = p[1];
     }
+    l += l_odd;
     return alpha;
 }
 
