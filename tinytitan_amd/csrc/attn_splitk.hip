@@ -105,7 +105,7 @@ __device__ __forceinline__ void store_out4_gated(const Args &a, int seq, int tok
     f4 r = o * inv_l;
     if (a.gate) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] *= 1.0f / (1.0f + __expf(-(float)g[i]));
+        for (int i = 0; i < 4; ++i) r[i] *= sigmoid((float)g[i]);
     }
     typedef __attribute__((address_space(1))) _Float16 *global_out;
     const global_out op = (global_out)(a.out + seq * a.o_seq_stride + tok * a.o_tok_stride + (long long)head * D + d);
@@ -130,10 +130,10 @@ __device__ __forceinline__ void store_out4(const SplitKArgs &a, int seq, int tok
         } else {
             g0 = (float)gp[0]; g1 = (float)gp[1]; g2 = (float)gp[2]; g3 = (float)gp[3];
         }
-        r[0] *= 1.0f / (1.0f + __expf(-g0));
-        r[1] *= 1.0f / (1.0f + __expf(-g1));
-        r[2] *= 1.0f / (1.0f + __expf(-g2));
-        r[3] *= 1.0f / (1.0f + __expf(-g3));
+        r[0] *= sigmoid(g0);
+        r[1] *= sigmoid(g1);
+        r[2] *= sigmoid(g2);
+        r[3] *= sigmoid(g3);
     }
     _Float16 *op = a.out + seq * a.o_seq_stride + tok * a.o_tok_stride + (long long)head * D + d;
     if (aligned) {
