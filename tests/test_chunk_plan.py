@@ -121,6 +121,78 @@ int main() {
 }
 '''
 
+# The same of the kernel over halves of the keys: in step i its wavefronts read step i (K and V) and step i + 1 (K), then hand their results over in the
+# place that the copies of the step behind a tile's last three would have taken.
+HALVES = r'''
+#include <algorithm>
+#include <cstdio>
+#include <map>
+#include <vector>
+#include "chunk_plan.h"
+
+struct Half {
+    int half = 0, off = 0, bad = 0;
+    std::map<int, int> landed;
+    std::vector<std::vector<std::pair<int, int>>> flying;
+    int slot(int step) const { return (step + off) % tt::kHalvesRing; }
+    void copy(int step, int first, int nb, int next_first, int next_nb) {
+        const int block = tt::halves_block(step, half, first, nb, next_first, next_nb);
+        for (const auto &turn : flying)
+            for (const auto &c : turn) bad += c.first == slot(step) && c.second != block;
+        flying.push_back({{slot(step), block}});
+    }
+    void wait(size_t turns) {
+        for (; flying.size() > turns; flying.erase(flying.begin()))
+            for (const auto &c : flying.front()) landed[c.first] = c.second;
+    }
+    void read(int step, int first, int nb) {
+        if (2 * step + half >= nb) return;  // (past the half's last block: whatever is there, it is not used)
+        bad += landed.count(slot(step)) == 0 || landed[slot(step)] != first + 2 * step + half;
+        for (const auto &turn : flying)
+            for (const auto &c : turn) bad += c.first == slot(step);
+    }
+};
+
+static int run(int half, int first, int nb, int next_first, int next_nb) {
+    Half h;
+    h.half = half;
+    for (int tile = 0; tile < (next_nb > 0 ? 2 : 1); ++tile) {
+        const int jb = tile ? next_first : first, n = tile ? next_nb : nb, steps = (n + 1) / 2, nf = tile ? 0 : next_first, nn = tile ? 0 : next_nb;
+        if (tile == 0) {
+            for (int i = 0; i + 1 < tt::kHalvesAhead; ++i) h.copy(i, jb, n, nf, nn);
+            h.wait(0);
+            h.copy(tt::kHalvesAhead - 1, jb, n, nf, nn);
+        }
+        h.read(0, jb, n);
+        for (int i = 0; i < steps; ++i) {
+            h.read(i, jb, n);
+            h.read(i + 1, jb, n);
+            h.copy(i + tt::kHalvesAhead, jb, n, nf, nn);
+            h.read(i, jb, n);
+            h.read(i + 1, jb, n);
+            h.wait(1);
+        }
+        h.wait(0);
+        // where the results meet no later step's block lies
+        const int meet = h.slot(steps + tt::kHalvesRing - 1);
+        for (int i = 0; i < tt::kHalvesAhead; ++i) h.bad += h.slot(steps + i) == meet;
+        h.landed.erase(meet);
+        h.off = (h.off + steps) % tt::kHalvesRing;
+    }
+    if (h.bad) std::printf("half %d, %d blocks, then %d: %d\n", half, nb, next_nb, h.bad);
+    return h.bad != 0;
+}
+
+int main() {
+    int bad = 0;
+    for (int half : {0, 1})
+        for (int nb = 1; nb < 24; ++nb)
+            for (int next = 0; next < 24; ++next)
+                for (int next_first : {0, 3}) bad += run(half, next ? 0 : 5, nb, next_first, next);
+    return bad != 0;
+}
+'''
+
 
 def _runs(tmp_path, text):
     source, program = tmp_path / "plan.cpp", tmp_path / "plan"
@@ -138,3 +210,8 @@ def test_ranges_cover_every_tile(tmp_path):
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
 def test_copies_into_the_rings_meet_nowhere(tmp_path):
     _runs(tmp_path, COPIES)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
+def test_copies_of_the_halves_meet_nowhere(tmp_path):
+    _runs(tmp_path, HALVES)

@@ -194,3 +194,44 @@ def test_infinite_values_reach_the_output_as_they_are(gpu_ctx, rows, kv_valid, f
     want = oracle.attention_batch(q.astype(np.float32), k.reshape(kv_valid, -1).astype(np.float32), v.reshape(kv_valid, -1).astype(np.float32),
                                   rows, start, H, KH, D, scale, threads=4).reshape(rows, H, D)[checked]
     _check(got[:, :, ~dims], want[:, :, ~dims], f"{rows} rows, {kv_valid} keys")
+
+
+@pytest.mark.parametrize("H,KH,rows,start,window,ring", [
+    (64, 8, 2048, 5000, 33, 0), (64, 8, 2048, 5000, 64, 0), (64, 8, 2048, 5000, 99, 0),  # three, four and five blocks a tile, tiles in pairs
+    (64, 8, 2047, 3001, 130, 2400),                                                       # pairs over a ring that wraps inside a tile's range
+    (8, 2, 4096, 50, 256, 0), (8, 2, 4096, 50, 288, 0),                                   # ten and eleven, in one round
+    (8, 2, 33, 40000, 0, 0)])                                                             # key ranges of one full tile and one of one row
+def test_heads_of_128_by_halves_of_the_keys(gpu_ctx, H, KH, rows, start, window, ring):
+    # On both sides of the lines between the two kernels over heads of 128, rows at the tiles' edges against the oracle over each row's keys.
+    import torch
+    from tinytitan_amd.engine import KVCacheManager, PrefillAttention, PrefillAttentionParams
+    D = 128
+    total, scale = start + rows, float(D) ** -0.5
+    r = np.random.default_rng(rows + start + window)
+    k, v = (r.standard_normal((total, KH * D)).astype(np.float16) for _ in range(2))
+    q, g = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=1, max_context=total, initial_capacity=total, ring_capacity=ring)
+    at = max(0, start - window - 32) if ring else 0
+    while at < total:  # (a ring takes ranges that do not wrap)
+        n = min(total - at, ring - at % ring) if ring else total - at
+        kd, vd = _dev(k[at:at + n]), _dev(v[at:at + n])
+        torch.cuda.synchronize()
+        kv.append(0, 0, at, kd, vd)
+        gpu_ctx.synchronize()
+        at += n
+    qd, gd = _dev(q), _dev(g)
+    out = torch.full(qd.shape, float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, total, H, scale, H * D, H * D, H * D,
+                                                                                     sliding_window=window), gate=gd)
+    gpu_ctx.synchronize()
+    got = out.float().cpu().numpy()
+    kv.close()
+    assert np.isfinite(got).all()
+    edges = sorted(e + o for e in range(0, rows, 32) for o in (-1, 0) if 0 <= e + o < rows)
+    for row in sorted({*edges[::max(1, len(edges) // 40)], rows - 1}):
+        last = start + row + 1
+        lo = max(0, last - window) if window else 0
+        want = oracle.prefill_ref(q[row:row + 1].astype(np.float32), k[lo:last].astype(np.float32), v[lo:last].astype(np.float32), H * D, KH * D, D,
+                                  H, KH, last - lo - 1, 1, last - lo, 0, scale).reshape(1, -1) / (1 + np.exp(-g[row:row + 1].astype(np.float64)))
+        _check(got[row:row + 1], want, f"row {row} of {rows} behind {start} keys, {H}q/{KH}kv, window {window}, ring {ring}")

@@ -20,7 +20,10 @@
 // Neither needs more than half of the register file, so two waves fit per SIMD, and the
 // hardware overlaps one wave's MFMAs with the other's softmax VALU work and LDS reads; eight
 // waves per CU also issue LDS reads about 1.6x faster than four can (the per-wave issue rate
-// is what limits a 4-wave design).  One workgroup barrier separates the steps, of one key block (heads of 128: two).
+// is what limits a 4-wave design).  One workgroup barrier separates the steps, of one key block.
+//
+// Heads of 128 have half the matrix instructions for the same softmax, and a score wave is then most of a step: their two wavefronts a
+// SIMD share the KEYS instead (attn_prefill_halves_kernel).
 //
 // K/V blocks stream L2 -> LDS with direct-to-LDS 128-bit loads (no registers), three or four stages
 // deep, issued one or two steps ahead of their first use; the K fragment layout in HBM is the MFMA
@@ -103,6 +106,38 @@ __device__ __forceinline__ void copy16_global_to_lds(const void *base, unsigned 
                  : "memory");
 }
 
+// N pieces of 1 KiB that lie one behind the other in both places (an instruction's offset counts for both).
+template <int N>
+__device__ __forceinline__ void copies_global_to_lds(const void *base, unsigned first, unsigned second, unsigned lds_addr) {
+    static_assert(N == 2, "two copies");
+    const unsigned long long b = (unsigned long long)base;
+    const unsigned b_hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+    const unsigned b_lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+    base = (const void *)(((unsigned long long)b_hi << 32) | (unsigned long long)b_lo);
+    lds_addr = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
+    unsigned saved_m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %1\n\tglobal_load_lds_dwordx4 %4, %1 offset:1024\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved_m0)
+                 : "s"(base), "v"(first), "s"(lds_addr), "v"(second)
+                 : "memory");
+}
+
+// o *= alpha in place (written out the compiler moves all of o around in every step for the few that rescale).  Ahead of it the block's
+// softmax, behind it two wait states before a matrix instruction reads.
+__device__ __forceinline__ void rescale_tile(f16v &o, float alpha) {
+#pragma unroll
+    for (int j = 0; j < 16; j += 4) {
+        float a0 = o[j], a1 = o[j + 1], a2 = o[j + 2], a3 = o[j + 3];
+        asm volatile("v_mul_f32 %0, %4, %0\n\tv_mul_f32 %1, %4, %1\n\tv_mul_f32 %2, %4, %2\n\tv_mul_f32 %3, %4, %3\n\ts_nop 4"
+                     : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)
+                     : "v"(alpha));
+        o[j] = a0;
+        o[j + 1] = a1;
+        o[j + 2] = a2;
+        o[j + 3] = a3;
+    }
+}
+
 // vmcnt(n) only: leaves the LDS/scalar and export counters alone.
 #define TT_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
@@ -114,24 +149,23 @@ __device__ __forceinline__ void copy16_global_to_lds(const void *base, unsigned 
 // waits until the matrix pipe is free: 64 of them beside another wavefront's MFMAs take as long as those do, 64 of any other instruction
 // here 1.25 times their own time.  64/8 heads of 64, 2,048 rows behind 4,000 keys 252.0 -> 235.3 us; 32/8 of 128, 4,096 behind 8,000
 // 729 -> 719; heads of 256, whose softmax is a smaller part, the same.)  Returns the factor the row's accumulators must be scaled by before this block is added.
-template <int NB>
-__device__ __forceinline__ float softmax_step(const f16v (&s_raw)[NB], bool mask, int kbase, int lo, int lim, int g,
-                                              float scale_log2e, float &m, float &l, h8 (&pf)[2 * NB]) {
+__device__ __forceinline__ float softmax_step(const f16v &s_raw, bool mask, int kbase, int lo, int lim, int g, float scale_log2e, float &m,
+                                              float &l, h8 (&pf)[2]) {
     // The maximum is taken over the raw scores and scaled once (the host sends only chunks with scale > 0 here), and a
     // probability is one fused multiply-add and one exp2 off its raw score.
-    float t[16 * NB];
+    float t[16];
 #pragma unroll
-    for (int v = 0; v < 16 * NB; ++v) t[v] = s_raw[v >> 4][v & 15];
+    for (int v = 0; v < 16; ++v) t[v] = s_raw[v];
     if (mask) {  // wave-uniform: only the blocks on or past the tile's diagonal, or at its window's lower edge
 #pragma unroll
-        for (int v = 0; v < 16 * NB; ++v) {
+        for (int v = 0; v < 16; ++v) {
             const int key = kbase + 8 * (v >> 2) + 4 * g + (v & 3);
             if (key >= lim || key < lo) t[v] = -INFINITY;
         }
     }
     float mx = fmaxf(t[0], t[1]);
 #pragma unroll
-    for (int v = 2; v < 16 * NB; v += 2) mx = fmaxf(fmaxf(t[v], t[v + 1]), mx);
+    for (int v = 2; v < 16; v += 2) mx = fmaxf(fmaxf(t[v], t[v + 1]), mx);
     mx = max_across_halves(mx) * scale_log2e;
     const bool move = mx > m + kRescaleThreshold;  // a row's first visible block always moves
     const float m_new = move ? mx : m;
@@ -140,7 +174,7 @@ __device__ __forceinline__ float softmax_step(const f16v (&s_raw)[NB], bool mask
     m = m_new;
     float l_odd = 0.0f;  // (two sums: neither waits for the other's last addition)
 #pragma unroll
-    for (int v = 0; v < 16 * NB; v += 2) {
+    for (int v = 0; v < 16; v += 2) {
         const h2 p = {(_Float16)fast_exp2(__builtin_fmaf(t[v], scale_log2e, -m)), (_Float16)fast_exp2(__builtin_fmaf(t[v + 1], scale_log2e, -m))};
         asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(l) : "v"(p));
         asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(l_odd) : "v"(p));
@@ -151,21 +185,61 @@ __device__ __forceinline__ float softmax_step(const f16v (&s_raw)[NB], bool mask
     return alpha;
 }
 
+// Workgroup -> (kv head, head sub-group, tile pair); kv heads are spread over XCDs so
+// that each XCD's L2 holds one kv head's K/V.
+struct ChunkItem {
+    int kvh, hsub, pair, split;
+    bool longest_first;
+};
+__device__ __forceinline__ bool chunk_item(const PrefillArgs &a, ChunkItem &item) {
+    int split = blockIdx.x / a.base_grid;
+    const int wg = blockIdx.x - split * a.base_grid;  // base_grid is a multiple of 8: wg & 7 is still the XCD
+    int kvh, r;
+    if (a.xcd_chunk > 0) {
+        // Key ranges: the (range, tile, head set) items of a kv head, range-major, are cut into as many runs as the kv
+        // head has XCDs (workgroup b runs on XCD b % 8).  Every XCD gets the same number of workgroups whatever the
+        // number of tiles -- dealt out tile by tile, 3 or 5 tiles per head set leave some XCDs with twice the work of
+        // others -- and a range's K/V blocks are fetched into one L2, or two, instead of all of the kv head's.
+        const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
+        kvh = x / a.xs;
+        const int w = (x - kvh * a.xs) * a.xcd_chunk + j;
+        if (w >= a.per_kvh * a.n_splits) return false;
+        split = w / a.per_kvh;
+        r = w - split * a.per_kvh;
+    } else if (a.xs > 0) {
+        const int x = wg & 7, y = wg >> 3;
+        kvh = x / a.xs;
+        r = y * a.xs + (x - kvh * a.xs);
+    } else {
+        kvh = wg / a.per_kvh;
+        r = wg - kvh * a.per_kvh;
+    }
+    if (r >= a.per_kvh || kvh >= a.n_kv_heads) return false;
+    // (whole tiles one by one: the head sets' longest tiles first, and so on down)
+    item.longest_first = a.single_tiles && a.n_splits == 1;
+    // (one division: each is a chain in front of the first load)
+    const int per = item.longest_first ? a.hsubs : a.n_pairs, quotient = r / per, rest = r - quotient * per;
+    item.kvh = kvh;
+    item.hsub = item.longest_first ? rest : quotient;
+    item.pair = item.longest_first ? quotient : rest;
+    item.split = split;
+    return true;
+}
+
 }  // namespace
 
-template <int D, int NB>  // NB: key blocks per step, one or two
+template <int D>
 __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(const PrefillArgs a) {
     constexpr int KS = D / 16;  // k-steps of S^T
     constexpr int MT = D / 32;  // 32-dim tiles of O^T
     constexpr int BLOCK_BYTES = 32 * D * 2;
-    constexpr int KR = k_ring(NB), VR = v_ring(NB);
-    constexpr int SLOT_BYTES = NB * BLOCK_BYTES;
+    constexpr int KR = k_ring(1), VR = v_ring(1);
+    constexpr int SLOT_BYTES = BLOCK_BYTES;
     constexpr int CHUNKS = BLOCK_BYTES / 1024;    // 1 KiB chunks per block (= KS = 2 MT)
-    constexpr int CPW = NB * CHUNKS / 4;          // copies one wave issues per step (K and V of a step's blocks over 8 waves)
-    static_assert(CHUNKS % CPW == 0, "a wave's copies of a step are of one block");
+    constexpr int CPW = CHUNKS / 4;               // copies one wave issues per step (K and V of a block over 8 waves)
     constexpr int V_OFF = KR * SLOT_BYTES;             // K ring, then V ring
-    constexpr int P_OFF = (KR + VR) * SLOT_BYTES;      // P^T: [2 steps][4 heads][2 NB k-steps][64 lanes][16 B]
-    constexpr int P_STEP = 4 * NB * 2048;
+    constexpr int P_OFF = (KR + VR) * SLOT_BYTES;      // P^T: [2 steps][4 heads][2 k-steps][64 lanes][16 B]
+    constexpr int P_STEP = 4 * 2048;
     constexpr int ALPHA_OFF = P_OFF + 2 * P_STEP;      // rescale factors: [2 steps][4 heads][32 rows] floats
     constexpr int LSUM_OFF = ALPHA_OFF + 2 * 4 * 128;  // row sums: [4 heads][32 rows] floats
     constexpr int STAGE_OFF = LSUM_OFF + 4 * 128;      // output rows on their way out: [4 heads][32 rows][32 dims + 16 B]
@@ -178,37 +252,10 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     const int w4 = wave & 3;
     const int li = lane & 31, g = lane >> 5;
 
-    // Workgroup -> (kv head, head sub-group, tile pair); kv heads are spread over XCDs so
-    // that each XCD's L2 holds one kv head's K/V.
-    int split = blockIdx.x / a.base_grid;
-    const int wg = blockIdx.x - split * a.base_grid;  // base_grid is a multiple of 8: wg & 7 is still the XCD
-    int kvh, r;
-    if (a.xcd_chunk > 0) {
-        // Key ranges: the (range, tile, head set) items of a kv head, range-major, are cut into as many runs as the kv
-        // head has XCDs (workgroup b runs on XCD b % 8).  Every XCD gets the same number of workgroups whatever the
-        // number of tiles -- dealt out tile by tile, 3 or 5 tiles per head set leave some XCDs with twice the work of
-        // others -- and a range's K/V blocks are fetched into one L2, or two, instead of all of the kv head's.
-        const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-        kvh = x / a.xs;
-        const int w = (x - kvh * a.xs) * a.xcd_chunk + j;
-        if (w >= a.per_kvh * a.n_splits) return;
-        split = w / a.per_kvh;
-        r = w - split * a.per_kvh;
-    } else if (a.xs > 0) {
-        const int x = wg & 7, y = wg >> 3;
-        kvh = x / a.xs;
-        r = y * a.xs + (x - kvh * a.xs);
-    } else {
-        kvh = wg / a.per_kvh;
-        r = wg - kvh * a.per_kvh;
-    }
-    if (r >= a.per_kvh || kvh >= a.n_kv_heads) return;
-    // (whole tiles one by one: the head sets' longest tiles first, and so on down)
-    const bool longest_first = a.single_tiles && a.n_splits == 1;
-    // (one division: each is a chain in front of the first load)
-    const int per = longest_first ? a.hsubs : a.n_pairs, quotient = r / per, rest = r - quotient * per;
-    const int hsub = longest_first ? rest : quotient;
-    const int pair = longest_first ? quotient : rest;
+    ChunkItem item;
+    if (!chunk_item(a, item)) return;
+    const int kvh = item.kvh, hsub = item.hsub, pair = item.pair, split = item.split;
+    const bool longest_first = item.longest_first;
     const int head = kvh * a.group + hsub * 4 + w4;
     const _Float16 *kp = a.k_slot + (size_t)kvh * a.page_elems;
     const _Float16 *vp = a.v_slot + (size_t)kvh * a.page_elems;
@@ -228,10 +275,9 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     int slot_off = 0, carry_nb = 0;
     auto page_block = [&](int block) { return a.ring_blocks ? block % a.ring_blocks : block; };
     auto role_ring = [&](int j) { return value_wave ? in_ring(VR, j) : in_ring(KR, j); };
-    const int my_block = NB == 1 ? 0 : w4 * CPW / CHUNKS;  // which of a step's blocks this wave copies from
-    const int my_chunk = w4 * CPW - my_block * CHUNKS;
+    const int my_chunk = w4 * CPW;
     auto source_block = [&](int j, int nb) {  // the block that step-relative index j stands for
-        return value_wave ? copied_block(NB, VR, j, my_block, jb, nb, carry_nb) : copied_block(NB, KR, j, my_block, jb, nb, carry_nb);
+        return value_wave ? copied_block(1, VR, j, 0, jb, nb, carry_nb) : copied_block(1, KR, j, 0, jb, nb, carry_nb);
     };
     // A step's copies: this wave's CPW one-KiB chunks of ONE block -- of K for the score waves (the LDS layout is the HBM
     // layout, fragment s is chunk s), of V for the value waves (gathered so that LDS holds fragment (mt, t) as [lane][8 halves]).  Where the block lies in the page and in the
@@ -266,7 +312,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
         for (int c = 0; c < CPW; ++c) issue_copy(sc, c);
     };
 
-    char *const p_mine = smem + P_OFF + w4 * (NB * 2048) + lane * 16;  // + step parity * P_STEP, + k-step * 1024
+    char *const p_mine = smem + P_OFF + w4 * 2048 + lane * 16;  // + step parity * P_STEP, + k-step * 1024
     float *const alpha_mine = reinterpret_cast<float *>(smem + ALPHA_OFF) + w4 * 32 + li;  // + step parity * 128
     float *const lsum_mine = reinterpret_cast<float *>(smem + LSUM_OFF) + w4 * 32 + li;
 
@@ -290,17 +336,11 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
         const int end = min(a.kv_valid, a.start + min(a.q_len, tile * 32 + 32));
         const int nb_tile = (end + 31) >> 5;                   // key blocks this tile needs
         const int mask_from = (a.start + tile * 32 + 1) >> 5;  // first block in which some row is masked by causality
-        // This workgroup's share of them (all, without key splits); local step i is blocks jb + NB i ..
+        // This workgroup's share of them (all, without key splits); local step i is block jb + i
         jb = window_block + (a.n_splits > 1 ? split * a.split_blocks : 0);
         const int nb = (a.n_splits > 1 ? min(nb_tile, jb + a.split_blocks) : nb_tile) - jb;
         if (nb <= 0) continue;  // nothing of this tile in the range (the same for every wave)
-        const int steps = (nb + NB - 1) / NB;
-        int first_masked = min(mask_from, end >> 5);  // ... or cut by the valid length
-        int hi = lim;                                 // keys [lo, hi) count here
-        if constexpr (NB > 1) {  // (the range may end inside the last step)
-            first_masked = __builtin_amdgcn_readfirstlane(min(first_masked, jb + nb));
-            hi = min(lim, (jb + nb) * 32);
-        }
+        const int first_masked = min(mask_from, end >> 5);  // ... or cut by the valid length
 
         if (pass > 0) __syncthreads();  // every wave is done with the previous pass's LDS
         const bool carried = carry_nb > 0;  // this tile's first blocks came in behind the previous tile's last
@@ -345,42 +385,37 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             float m = kNegBig, l = 0.0f;
             TT_WAIT_VMCNT(0);  // the first stages and the query rows
             __syncthreads();
-            h8 kf[NB * KS];
+            h8 kf[KS];
 #pragma unroll
-            for (int t = 0; t < NB * KS; ++t)
+            for (int t = 0; t < KS; ++t)
                 kf[t] = *reinterpret_cast<const h8 *>(smem + slot_off * SLOT_BYTES + lane * 16 + t * 1024);
             __syncthreads();  // every score wave holds K of step 0: step 0 may refill its slot
 #pragma nounroll
-            for (int i = 0; i < steps; ++i) {
+            for (int i = 0; i < nb; ++i) {
                 const char *next = smem + in_ring(KR, i + 1 + slot_off) * SLOT_BYTES + lane * 16;
                 const StepCopies sc = step_copies(i, nb);
-                f16v s[NB];
+                f16v s = (f16v)0.0f;
 #pragma unroll
-                for (int b = 0; b < NB; ++b) s[b] = (f16v)0.0f;
-                // (a step of two blocks: their chains of MFMAs in turn)
-#pragma unroll
-                for (int u = 0; u < NB * KS; ++u) {
-                    const int b = u % NB, t = u / NB, f = b * KS + t;
-                    s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[f], qf[t], s[b], 0, 0, 0);
-                    kf[f] = *reinterpret_cast<const h8 *>(next + f * 1024);
+                for (int t = 0; t < KS; ++t) {
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[t], qf[t], s, 0, 0, 0);
+                    kf[t] = *reinterpret_cast<const h8 *>(next + t * 1024);
                     // this step's copies, one at a time between MFMAs: a burst would stall the wave
                     // on the CU's vector memory path (64 B/clk for all eight waves)
-                    if (u % (NB * KS / CPW) == 0) issue_copy(sc, u / (NB * KS / CPW));
+                    if (t % (KS / CPW) == 0) issue_copy(sc, t / (KS / CPW));
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                h8 pf[2 * NB];
-                const int block = jb + NB * i;
-                const float alpha = softmax_step<NB>(s, block + NB - 1 >= first_masked || block <= last_lo_block, block << 5, lo, hi, g,
-                                                     a.scale_log2e, m, l, pf);
+                h8 pf[2];
+                const int block = jb + i;
+                const float alpha = softmax_step(s, block >= first_masked || block <= last_lo_block, block << 5, lo, lim, g, a.scale_log2e, m, l, pf);
                 char *pdst = p_mine + (i & 1) * P_STEP;
 #pragma unroll
-                for (int t = 0; t < 2 * NB; ++t) *reinterpret_cast<h8 *>(pdst + t * 1024) = pf[t];
+                for (int t = 0; t < 2; ++t) *reinterpret_cast<h8 *>(pdst + t * 1024) = pf[t];
                 if (g == 0) alpha_mine[(i & 1) * 128] = alpha;
                 end_step(k_landed);
             }
-            issue_step(steps, nb);
+            issue_step(nb, nb);
             end_step(k_landed);  // the value waves' last two steps
-            issue_step(steps + 1, nb);
+            issue_step(nb + 1, nb);
             end_step(k_landed);
             const float lt = sum_across_halves(l);
             if (g == 0) {
@@ -407,16 +442,16 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             issue_step(0, nb);
             end_step(v_landed);  // step 0: the score waves' first
             issue_step(1, nb);
-            h8 vf[NB * 2 * MT], pf[2 * NB];
+            h8 vf[2 * MT], pf[2];
 #pragma unroll
-            for (int c = 0; c < NB * 2 * MT; ++c)
+            for (int c = 0; c < 2 * MT; ++c)
                 vf[c] = *reinterpret_cast<const h8 *>(smem + V_OFF + slot_off * SLOT_BYTES + lane * 16 + c * 1024);
 #pragma unroll
-            for (int t = 0; t < 2 * NB; ++t) pf[t] = *reinterpret_cast<const h8 *>(p_mine + t * 1024);
+            for (int t = 0; t < 2; ++t) pf[t] = *reinterpret_cast<const h8 *>(p_mine + t * 1024);
             float alpha = alpha_mine[0];
             end_step(v_landed);  // step 1
 #pragma nounroll
-            for (int i = 2; i <= nb / NB + 1; ++i) {
+            for (int i = 2; i <= nb + 1; ++i) {
                 const int jn = i - 1;  // the step fetched in this one (past the last one: stale but harmless data)
                 const char *next = smem + V_OFF + in_ring(VR, jn + slot_off) * SLOT_BYTES + lane * 16;
                 const char *psrc = p_mine + (jn & 1) * P_STEP;
@@ -426,49 +461,33 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
                     for (int mt = 0; mt < MT; ++mt) o[mt] *= alpha;
                 }
                 alpha = alpha_mine[(jn & 1) * 128];
-                auto multiply = [&](int u, int mt, int t) {  // the u-th: k-step t (block t / 2, its k-step t % 2) of 32-dim tile mt
-                    const int c = (t >> 1) * 2 * MT + 2 * mt + (t & 1);  // the fragment's place in the slot
+                auto multiply = [&](int u, int mt, int t) {  // the u-th: k-step t of 32-dim tile mt
+                    const int c = 2 * mt + t;  // the fragment's place in the slot
                     o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[c], pf[t], o[mt], 0, 0, 0);
                     vf[c] = *reinterpret_cast<const h8 *>(next + c * 1024);
-                    if (u % (NB * KS / CPW) == 0) issue_copy(sc, u / (NB * KS / CPW));
+                    if (u % (KS / CPW) == 0) issue_copy(sc, u / (KS / CPW));
                     __builtin_amdgcn_sched_barrier(0);
                 };
                 if constexpr (D == 256) {
                     // All k-steps of a 32-dim tile back to back: consecutive MFMAs on one accumulator
                     // forward it inside the matrix pipe instead of going through the register file.
-                    h8 pn[2 * NB];
+                    h8 pn[2];
 #pragma unroll
-                    for (int t = 0; t < 2 * NB; ++t) pn[t] = *reinterpret_cast<const h8 *>(psrc + t * 1024);
+                    for (int t = 0; t < 2; ++t) pn[t] = *reinterpret_cast<const h8 *>(psrc + t * 1024);
 #pragma unroll
-                    for (int u = 0; u < NB * 2 * MT; ++u) multiply(u, u / (2 * NB), u % (2 * NB));
+                    for (int u = 0; u < 2 * MT; ++u) multiply(u, u / 2, u % 2);
 #pragma unroll
-                    for (int t = 0; t < 2 * NB; ++t) pf[t] = pn[t];
+                    for (int t = 0; t < 2; ++t) pf[t] = pn[t];
                 } else {
                     // One k-step after the other: its P^T is read into the registers that its MFMAs are done with.
 #pragma unroll
-                    for (int t = 0; t < 2 * NB; ++t) {
+                    for (int t = 0; t < 2; ++t) {
 #pragma unroll
                         for (int mt = 0; mt < MT; ++mt) multiply(t * MT + mt, mt, t);
                         pf[t] = *reinterpret_cast<const h8 *>(psrc + t * 1024);
                     }
                 }
                 end_step(v_landed);
-            }
-            if constexpr (NB > 1) {
-                // An odd range's last block, without the copy of it that lies in the second one's place: its probabilities are zero, but
-                // zero times an infinite value is not.
-                if (nb % NB != 0) {
-                    issue_step(steps + 1, nb);
-                    if (__any(alpha != 1.0f)) {
-#pragma unroll
-                        for (int mt = 0; mt < MT; ++mt) o[mt] *= alpha;
-                    }
-#pragma unroll
-                    for (int t = 0; t < 2; ++t)
-#pragma unroll
-                        for (int mt = 0; mt < MT; ++mt) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[2 * mt + t], pf[t], o[mt], 0, 0, 0);
-                    end_step(v_landed);
-                }
             }
             TT_WAIT_VMCNT(0);
             __syncthreads();  // the row sums are in LDS
@@ -532,7 +551,314 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
                 }
             }
         }
-        if (carry_nb > 0) slot_off = role_ring(slot_off + steps);  // where the next tile's first step sits
+        if (carry_nb > 0) slot_off = role_ring(slot_off + nb);  // where the next tile's first step sits
+    }
+}
+
+
+// Heads of 128: the two wavefronts of a SIMD share a (head, tile) by KEYS -- of a step's two blocks wavefront w4 takes the first,
+// w4 + 4 the second -- and each does all of its block's work: scores, softmax, values.  P^T stays in its registers, and a block's 16 matrix instructions
+// stand against one softmax in either wavefront, where a score wave had 16 and two softmaxes a step and its value wave 16 and none.
+//
+// What bounds a step is what two instruction streams issue on one SIMD (16 matrix instructions of 33 cycles and about 130 others each,
+// and the issue goes to the older wavefront first), so they are kept half a step apart: between two barriers the first half goes softmax,
+// values, next scores and the second values, scores, softmax, a softmax beside the other's matrix instructions, which also have the
+// higher priority.  The loop keeps its places as running sums (`look` works one out anew where a page's ring or the range ends): 75 scalar
+// instructions a step, with each place from the step's number, were 7 %.  The halves meet at the tile's end, each writing out half of the dims.
+// 32/8 heads, 777 rows behind a window of 4,096 keys 79.5 -> 70 us (a step of 0.96 -> 0.86 us; its matrix instructions and barrier alone 0.64),
+// 4,096 rows behind 8,000 keys 729 -> 659 (0.93 -> 1.02 PFLOP/s), from position 0 179 -> 161, 128 rows behind 32,000
+// 97.6 -> 88.  Measured and dropped: both halves in step (2,144 instead of 1,640 cycles by the issue model; 84 us), copies five steps ahead (the same),
+// all of a step's copies in one run or in other places (the same to 1 %), the higher priority for the softmax or for the younger half (0 to -4 %).
+template <int D>
+__global__ __launch_bounds__(512, 2) void attn_prefill_halves_kernel(const PrefillArgs a) {
+    constexpr int KS = D / 16, MT = D / 32;
+    constexpr int BLOCK_BYTES = 32 * D * 2, CHUNKS = BLOCK_BYTES / 1024;
+    constexpr int CPW = CHUNKS / 4;  // copies of K, and of V, that one wave issues per step: a quarter of its own block
+    constexpr int RING = kHalvesRing, SLOT_BYTES = 2 * BLOCK_BYTES, RING_BYTES = RING * SLOT_BYTES;
+    static_assert((RING_BYTES & (RING_BYTES - 1)) == 0, "places go round by a mask");
+    constexpr int V_OFF = RING_BYTES, X_OFF = 2 * RING_BYTES;  // X: what the halves hand each other, then rows on their way out
+    constexpr int STAGE_PITCH = 64 + 16;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = wave >> 2, w4 = wave & 3;
+    const int li = lane & 31, g = lane >> 5;
+
+    ChunkItem item;
+    if (!chunk_item(a, item)) return;
+    const int pair = item.pair, split = item.split;
+    const int head = item.kvh * a.group + item.hsub * 4 + w4;
+    const _Float16 *kp = a.k_slot + (size_t)item.kvh * a.page_elems;
+    const _Float16 *vp = a.v_slot + (size_t)item.kvh * a.page_elems;
+
+    // Copies of a step: this wavefront's quarter of its half's block, of K and of V.  K lies in HBM as in LDS; of V a
+    // 16-byte piece per lane, gathered so that LDS holds fragment (mt, t) as [lane][8 halves].
+    const unsigned smem_base = (unsigned)(size_t)(lds_ptr_t)smem;
+    const unsigned k_lane_offset = (unsigned)(w4 * CPW * 1024 + lane * 16);
+    unsigned v_lane_offset[CPW];  // (the second copy's offset of 1024 counts for both places, and none may be below zero)
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) {
+        const int chunk = w4 * CPW + c;
+        v_lane_offset[c] = (unsigned)(v_piece(D, li, g) + v_piece(D, 32 * (chunk >> 1), 2 * (chunk & 1))) * 2u + 1024u * (CPW - 1 - c);
+    }
+    const unsigned copy_base = smem_base + (unsigned)(half * BLOCK_BYTES + w4 * CPW * 1024);
+    const int wrap = a.ring_blocks ? a.ring_blocks : 0x40000000;
+    unsigned slot_off = 0;  // where the tile's step 0 sits in the rings, in bytes
+    bool carried = false;   // the tile's first blocks came in behind the last of the one before
+    // What step i + 1 reads was copied in step i - 1 or before.
+    auto end_step = [&]() {
+        TT_WAIT_VMCNT(2 * CPW);
+        __syncthreads();
+    };
+
+    const int n_passes = (a.single_tiles || pair == a.n_tiles - 1 - pair) ? 1 : 2;
+    for (int pass = 0; pass < n_passes; ++pass) {
+        const int tile = item.longest_first ? a.n_tiles - 1 - pair : a.single_tiles ? pair : (pass == 0 ? a.n_tiles - 1 - pair : pair);
+        const int tok = tile * 32 + li;
+        const bool valid = tok < a.q_len;
+        const int lim = valid ? min(a.kv_valid, a.start + tok + 1) : 0;  // keys [lo, lim) are visible
+        const int lo = (a.window > 0 && a.start + tok + 1 > a.window) ? a.start + tok + 1 - a.window : 0;
+        const int tile_lo = (a.window > 0 && a.start + tile * 32 + 1 > a.window) ? a.start + tile * 32 + 1 - a.window : 0;
+        const int window_block = tile_lo >> 5;
+        const int last_lo_block = a.window > 0 ? (tile_lo + 31) >> 5 : -1;
+        const int end = min(a.kv_valid, a.start + min(a.q_len, tile * 32 + 32));
+        const int nb_tile = (end + 31) >> 5;                   // key blocks this tile needs
+        const int mask_from = (a.start + tile * 32 + 1) >> 5;  // first block in which some row is masked by causality
+        const int jb = window_block + (a.n_splits > 1 ? split * a.split_blocks : 0);
+        const int nb = (a.n_splits > 1 ? min(nb_tile, jb + a.split_blocks) : nb_tile) - jb;
+        if (nb <= 0) continue;  // nothing of this tile in the range (the same for every wave)
+        const int steps = (nb + 1) / 2, mine = (nb + 1 - half) / 2;  // blocks jb + 2 i + half, i < mine
+        const int first_masked = min(mask_from, end >> 5);
+
+        if (pass > 0) __syncthreads();  // every wave is done with the other tile's LDS
+        // The tile that follows takes its first blocks from the copies behind this one's last: from the block of the first key its first row sees.
+        int next_first = 0, next_nb = 0;
+        if (pass == 0 && n_passes == 2 && a.n_splits == 1) {
+            if (a.window > 0) next_first = max(a.start + pair * 32 + 1 - a.window, 0) >> 5;
+            next_nb = ((min(a.kv_valid, a.start + min(a.q_len, pair * 32 + 32)) + 31) >> 5) - next_first;
+        }
+        // Where the copies stand: sources of the next step's, its place, and how many steps run on in the page before that takes
+        // another look (a ring's end, the range's last block, and behind that each one).
+        const char *k_src, *v_src;
+        unsigned copy_off = slot_off;
+        int copy_step = carried ? kHalvesAhead : 0, run = 0, left = 0;
+        if (carried) copy_off = (copy_off + kHalvesAhead * SLOT_BYTES) & (RING_BYTES - 1);
+        auto look = [&]() {
+            copy_step += run;
+            const int phys = halves_block(copy_step, half, jb, nb, next_first, next_nb) % wrap;
+            run = copy_step < mine ? min(mine - copy_step, (wrap - phys + 1) / 2) : 1;
+            left = run;
+            const size_t at = (size_t)(unsigned)phys * BLOCK_BYTES;
+            k_src = reinterpret_cast<const char *>(kp) + at;
+            v_src = reinterpret_cast<const char *>(vp) + at - 1024 * (CPW - 1);
+        };
+        look();
+        auto copy_k = [&]() { copies_global_to_lds<CPW>(k_src, k_lane_offset, k_lane_offset, copy_base + copy_off); };
+        auto copy_v = [&]() {  // behind copy_k
+            copies_global_to_lds<CPW>(v_src, v_lane_offset[0], v_lane_offset[CPW - 1], copy_base + V_OFF + copy_off);
+            k_src += SLOT_BYTES;
+            v_src += SLOT_BYTES;
+            copy_off = (copy_off + SLOT_BYTES) & (RING_BYTES - 1);
+            if (--left == 0) look();
+        };
+        if (!carried) {
+#pragma unroll
+            for (int i = 0; i < kHalvesAhead - 1; ++i) {
+                copy_k();
+                copy_v();
+            }
+        }
+        unsigned k_read = slot_off, v_read = slot_off;  // where the step lies whose K, V are read next
+        // Blocks jb + 2 i + half with plain_from <= i < plain_from + plain need no mask.
+        const int plain_from = last_lo_block < jb + half ? 0 : (last_lo_block - jb - half) / 2 + 1;
+        const unsigned plain = (unsigned)max((first_masked - jb - half + 1) / 2 - plain_from, 0);
+        h8 qf[KS];
+        const _Float16 *qp = a.q + (long long)(valid ? tok : 0) * a.q_stride + (long long)head * D + 8 * g;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const h8 x = *reinterpret_cast<const h8 *>(qp + 16 * s);
+            qf[s] = valid ? x : (h8)(_Float16)0;
+        }
+        float m = kNegBig, l = 0.0f;
+        f16v o[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) o[mt] = (f16v)0.0f;
+        TT_WAIT_VMCNT(0);  // the first steps' blocks and the query rows
+        if (!carried) { copy_k(); copy_v(); }
+        __syncthreads();
+        h8 kf[KS], vf[2 * MT], pf[2];
+        f16v s1;
+        const char *const my_lds = smem + half * BLOCK_BYTES + lane * 16;
+#pragma unroll
+        for (int t = 0; t < KS; ++t) kf[t] = *reinterpret_cast<const h8 *>(my_lds + slot_off + t * 1024);
+
+        // Scores of the block whose K is in registers.
+        auto scores = [&]() {
+            s1 = (f16v)0.0f;
+#pragma unroll
+            for (int t = 0; t < KS; ++t) s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[t], qf[t], s1, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // Its probabilities; its V is read meanwhile.
+        auto weigh = [&](int i) {
+            __builtin_amdgcn_s_setprio(0);
+            const char *v_now = my_lds + V_OFF + v_read;
+            v_read = (v_read + SLOT_BYTES) & (RING_BYTES - 1);
+#pragma unroll
+            for (int t = 0; t < 2 * MT; ++t) vf[t] = *reinterpret_cast<const h8 *>(v_now + t * 1024);
+            __builtin_amdgcn_sched_barrier(0);
+            const float alpha = softmax_step(s1, (unsigned)(i - plain_from) >= plain, (jb + 2 * i + half) << 5, lo, lim, g, a.scale_log2e, m, l, pf);
+            if (__any(alpha != 1.0f)) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) rescale_tile(o[mt], alpha);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // ... and its values; the next block's K is read meanwhile, and the step's copies go out.
+        auto values = [&]() {
+            __builtin_amdgcn_s_setprio(1);
+            k_read = (k_read + SLOT_BYTES) & (RING_BYTES - 1);
+            const char *k_next = my_lds + k_read;
+#pragma unroll
+            for (int u = 0; u < 2 * MT; ++u) {
+                const int mt = u % MT, t = u / MT;
+                o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[2 * mt + t], pf[t], o[mt], 0, 0, 0);
+                kf[u] = *reinterpret_cast<const h8 *>(k_next + u * 1024);
+                if (u == 1) copy_k();
+                if (u == MT + 1) copy_v();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        static_assert(KS == 2 * MT, "a K fragment per value MFMA");
+        auto values_of_last = [&]() {
+#pragma unroll
+            for (int u = 0; u < 2 * MT; ++u) o[u % MT] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[2 * (u % MT) + u / MT], pf[u / MT], o[u % MT], 0, 0, 0);
+        };
+        if (half == 0) {
+            scores();
+#pragma nounroll
+            for (int i = 0; i < steps; ++i) {
+                weigh(i);
+                values();
+                scores();
+                end_step();
+            }
+        } else {
+            copy_k();
+            copy_v();
+            scores();
+            if (mine > 0) weigh(0);
+            end_step();
+#pragma nounroll
+            for (int i = 1; i < mine; ++i) {
+                values();
+                scores();
+                weigh(i);
+                end_step();
+            }
+            if (mine > 0) {
+                if (mine < steps) {  // (an odd number of blocks: the last step is the other half's)
+                    copy_k();
+                    copy_v();
+                    end_step();
+                }
+                values_of_last();
+            }
+        }
+        TT_WAIT_VMCNT(0);  // no copy of this tile is on its way when the next one's begin
+        // The halves' results.  Every wave has 8 KiB: X, and the places in the rings that the last step's copies would have taken (the
+        // next tile's first three steps are in the others).  What it hands over -- (reference max, sum), then the dims that the
+        // other wave writes out -- goes through its own 8 KiB, but the pair first through the OTHER's: whoever reads a place is the one who writes it next, so
+        // one barrier behind each is all the order there is.
+        const int mt0 = half * (MT / 2);  // the 32-dim tiles that this wave writes out: mt0 .. mt0 + MT / 2 - 1
+        const unsigned last_slot = (slot_off + (unsigned)(steps + RING - 1) * SLOT_BYTES) & (RING_BYTES - 1);
+        auto place_of = [&](int w) { return smem + lane * 16 + (w < 4 ? X_OFF + w * 8192 : (w < 6 ? (int)last_slot : V_OFF + (int)last_slot) + (w & 1) * 8192); };
+        char *const x_mine = place_of(wave), *const x_other = place_of(wave ^ 4);
+        l = sum_across_halves(l);
+        *reinterpret_cast<float2 *>(x_other) = float2{m, l};
+        __syncthreads();
+        // The rows' gate values are asked for now, by every lane (a row past the chunk's end reads row 0's): behind the exchange they
+        // would be a trip to memory of their own.
+        const bool gated = a.gate != nullptr && a.n_splits == 1;
+        h4 gate[MT / 2][4];
+        if (gated) {
+            const _Float16 *const gate_row = a.gate + (long long)(valid ? tok : 0) * a.g_stride + (long long)head * D + 32 * mt0 + 4 * g;
+#pragma unroll
+            for (int r = 0; r < MT / 2; ++r)
+#pragma unroll
+                for (int vq = 0; vq < 4; ++vq) gate[r][vq] = *reinterpret_cast<const h4 *>(gate_row + 32 * r + 8 * vq);
+        }
+        const float2 other = *reinterpret_cast<const float2 *>(x_mine);
+        const float top = fmaxf(m, other.x), scale_mine = fast_exp2(m - top), scale_other = fast_exp2(other.x - top);
+        l = l * scale_mine + other.y * scale_other;
+        m = top;
+        f16v result[MT / 2];
+#pragma unroll
+        for (int r = 0; r < MT / 2; ++r)
+#pragma unroll
+            for (int vq = 0; vq < 4; ++vq) {
+                f4 give;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {  // (half is uniform over the wave: selected register by register)
+                    give[v] = half == 0 ? o[MT / 2 + r][4 * vq + v] : o[r][4 * vq + v];
+                    result[r][4 * vq + v] = (half == 0 ? o[r][4 * vq + v] : o[MT / 2 + r][4 * vq + v]) * scale_mine;
+                }
+                *reinterpret_cast<f4 *>(x_mine + (4 * r + vq) * 1024) = give;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < MT / 2; ++r)
+#pragma unroll
+            for (int vq = 0; vq < 4; ++vq) {
+                const f4 x = *reinterpret_cast<const f4 *>(x_other + (4 * r + vq) * 1024);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) result[r][4 * vq + v] += x[v] * scale_other;
+            }
+        if (a.n_splits > 1) {
+            const size_t row = (((size_t)split * a.group * a.n_kv_heads + head) * a.n_tiles + tile) * 32 + li;
+            if (half == 0 && g == 0) {
+                a.part_ml[row * 2] = m;
+                a.part_ml[row * 2 + 1] = l;
+            }
+            float *po = a.part_o + row * D + 4 * g;
+#pragma unroll
+            for (int r = 0; r < MT / 2; ++r)
+#pragma unroll
+                for (int vq = 0; vq < 4; ++vq) {
+                    const f4 x = {result[r][4 * vq], result[r][4 * vq + 1], result[r][4 * vq + 2], result[r][4 * vq + 3]};
+                    *reinterpret_cast<f4 *>(po + 32 * (mt0 + r) + 8 * vq) = x;
+                }
+        } else {
+            char *const stage = x_other - lane * 16;  // (which this wave alone has read)
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            const int out_row = lane >> 2, out_piece = lane & 3;
+#pragma unroll
+            for (int r = 0; r < MT / 2; ++r) {
+#pragma unroll
+                for (int vq = 0; vq < 4; ++vq) {
+                    float r4[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) r4[i] = result[r][4 * vq + i] * inv;
+                    if (gated) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) r4[i] *= sigmoid((float)gate[r][vq][i]);
+                    }
+                    const h4 hv = {(_Float16)r4[0], (_Float16)r4[1], (_Float16)r4[2], (_Float16)r4[3]};
+                    *reinterpret_cast<h4 *>(stage + li * STAGE_PITCH + (8 * vq + 4 * g) * 2) = hv;
+                }
+#pragma unroll
+                for (int part = 0; part < 2; ++part) {
+                    const int row = 16 * part + out_row;
+                    const h8 x = *reinterpret_cast<const h8 *>(stage + row * STAGE_PITCH + out_piece * 16);
+                    const int t = tile * 32 + row;
+                    if (t < a.q_len)
+                        *reinterpret_cast<h8 *>(a.out + (long long)t * a.o_stride + (long long)head * D + 32 * (mt0 + r) + out_piece * 8) = x;
+                }
+            }
+        }
+        carried = next_nb > 0;
+        if (carried) slot_off = (slot_off + (unsigned)steps * SLOT_BYTES) & (RING_BYTES - 1);  // where its first step sits
     }
 }
 
@@ -545,28 +871,24 @@ bool prefill_kernel_serves(int n_q_heads, int n_kv_heads, int head_dim, bool ali
 }
 
 // the rings of K and V (128 KiB at D = 256, 112 at 128) + P^T hand-over (16, 32 KiB) + rescale factors and row sums + the output rows' staging (10 KiB)
-static constexpr int prefill_lds_bytes(int D, int NB) {
-    return (k_ring(NB) + v_ring(NB)) * NB * 32 * D * 2 + 2 * 4 * NB * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80;
-}
-static_assert(prefill_lds_bytes(256, 1) <= 160 * 1024 && prefill_lds_bytes(128, 2) <= 160 * 1024, "a CU's LDS");
+static constexpr int prefill_lds_bytes(int D) { return (k_ring(1) + v_ring(1)) * 32 * D * 2 + 2 * 4 * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80; }
 
-template <int D, int NB>
-static hipError_t configure_prefill() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_kernel<D, NB>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               prefill_lds_bytes(D, NB));
-}
+// ... the rings of the kernel over halves of the keys (128 KiB at D = 128) + the places that its wavefronts hand their results over in
+static constexpr int prefill_halves_lds_bytes(int D) { return 2 * kHalvesRing * 2 * 32 * D * 2 + 8 * 4096; }
+static_assert(prefill_lds_bytes(256) <= 160 * 1024 && prefill_halves_lds_bytes(128) <= 160 * 1024, "a CU's LDS");
+
 int configure_prefill_kernels(tt_hip_ctx *ctx) {
-    hipError_t e = configure_prefill<256, 1>();
-    if (e == hipSuccess) e = configure_prefill<128, 1>();
-    if (e == hipSuccess) e = configure_prefill<128, 2>();
-    if (e == hipSuccess) e = configure_prefill<64, 1>();
+    auto configure = [](const void *kernel, int lds) { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds); };
+    hipError_t e = configure(reinterpret_cast<const void *>(attn_prefill_kernel<256>), prefill_lds_bytes(256));
+    if (e == hipSuccess) e = configure(reinterpret_cast<const void *>(attn_prefill_kernel<128>), prefill_lds_bytes(128));
+    if (e == hipSuccess) e = configure(reinterpret_cast<const void *>(attn_prefill_kernel<64>), prefill_lds_bytes(64));
+    if (e == hipSuccess) e = configure(reinterpret_cast<const void *>(attn_prefill_halves_kernel<128>), prefill_halves_lds_bytes(128));
     return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "hipFuncSetAttribute(chunk kernel max dynamic LDS)");
 }
 
-template <int D, int NB>
-static int launch_prefill_d(tt_hip_ctx *ctx, const PrefillArgs &args, unsigned grid) {
-    constexpr int lds = prefill_lds_bytes(D, NB);
-    auto kernel = attn_prefill_kernel<D, NB>;  // (its LDS limit was raised when the first context on this device was created)
+// (the kernels' LDS limits were raised when the first context on this device was created)
+template <typename F>
+static int launch_chunk(tt_hip_ctx *ctx, F kernel, const PrefillArgs &args, unsigned grid, int lds) {
     launch_profiled(ctx, kernel, dim3(grid), dim3(512), (unsigned)lds, args);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "attn_prefill_kernel launch");
@@ -620,9 +942,11 @@ int launch_prefill(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot, int star
     const int walk = a.n_splits > 1 ? std::min(split_blocks, most_tile_blocks(start, q_len, kv_valid, window))
                                     : most_tile_blocks(start, q_len, kv_valid, window);
     switch (kv->head_dim) {
-        case 256: return launch_prefill_d<256, 1>(ctx, a, grid);
-        case 128: return step_blocks(128, walk) == 2 ? launch_prefill_d<128, 2>(ctx, a, grid) : launch_prefill_d<128, 1>(ctx, a, grid);
-        case 64: return launch_prefill_d<64, 1>(ctx, a, grid);
+        case 256: return launch_chunk(ctx, attn_prefill_kernel<256>, a, grid, prefill_lds_bytes(256));
+        case 128:
+            if (halves_of_keys(walk, (long long)grid, ctx->n_cus)) return launch_chunk(ctx, attn_prefill_halves_kernel<128>, a, grid, prefill_halves_lds_bytes(128));
+            return launch_chunk(ctx, attn_prefill_kernel<128>, a, grid, prefill_lds_bytes(128));
+        case 64: return launch_chunk(ctx, attn_prefill_kernel<64>, a, grid, prefill_lds_bytes(64));
         default: return TT_HIP_ERR_SHAPE;
     }
 }

@@ -29,19 +29,9 @@ inline int longest_tile_blocks(int start, int q_len, int kv_valid, int window) {
     return longest;
 }
 
-// ---- The chunk kernel's steps and the rings in LDS that its copies fill (attn_prefill.hip).
-
-// Key blocks of 32 that a step takes.  Heads of 128 take two: a step's MFMAs are then as many as at 256, its two score chains have no
-// link that waits for the one before it, and there is one barrier, one row maximum and one rescale test for 64 keys
-// (32/8 heads, 777 rows behind 5,003 keys 107.5 -> 95.4 us, 4096 behind 8,000 770 -> 710).  Two workgroups of one block a step on
-// a CU (rings of three, 128 registers) came to 721 where the chip is full and lost 5 % where it is not.  Not where a tile
-// walks so few that the steps in front of the first product and a half empty last step weigh more (one at a time / two, 64/8 heads,
-// 2,048 rows behind windows of 33 and 96 keys, three and five blocks: 46.0 / 49.1 us, 50.3 / 53.6; over three head counts and 256 to 4,096
-// rows seven blocks are 2 % slower in twos, six and eight 1 % faster).
-constexpr int step_blocks(int D, int walk) { return D == 128 && (walk == 6 || walk > 7) ? 2 : 1; }
-// How many steps' K and V the rings in LDS hold: with two blocks a step three of V, so that all of it stays within 160 KiB.
+// ---- The rings in LDS that the chunk kernels' copies fill (attn_prefill.hip): how many steps of K and V they hold.
 constexpr int k_ring(int) { return 4; }
-constexpr int v_ring(int step) { return step == 2 ? 3 : 4; }
+constexpr int v_ring(int) { return 4; }
 constexpr int in_ring(int ring, int j) { return (int)((unsigned)j % (unsigned)ring); }  // j >= 0
 // Step i, and in front of step 0 a turn for each i below it down to -copies_ahead, issues the copies of step i + copies_ahead.
 constexpr int copies_ahead(int ring, bool of_v) { return of_v ? ring - 2 : ring; }
@@ -54,6 +44,22 @@ constexpr int copied_block(int step, int ring, int j, int which, int first, int 
     return j < steps || carry == 0 ? first + (at < nb ? at : nb - 1) : (at < carry ? at : carry - 1);
 }
 
+
+// The kernel over halves of the keys takes two blocks a step, one for either half, and copies K and V `kHalvesAhead` steps ahead.  The last
+// step's copies are left out (where they would go the halves meet), so a tile leaves kHalvesAhead steps behind its own.
+constexpr int kHalvesRing = 4, kHalvesAhead = 3;
+// The block that step `step` of a range of `nb` blocks from `first` on holds for `half`.  Past the range's last the last again, or, when a second
+// tile follows, that tile's first ones.
+constexpr int halves_block(int step, int half, int first, int nb, int next_first, int next_nb) {
+    const int steps = (nb + 1) / 2, at = 2 * step + half, next = at - 2 * steps;
+    return step < steps || next_nb <= 0 ? first + (at < nb ? at : nb - 1) : next_first + (next < next_nb ? next : next_nb - 1);
+}
+// Whether a launch over heads of 128 goes by halves of the keys: not where a tile walks so few blocks (`walk`) that what the halves hand each
+// other outweighs them, which is sooner so in a launch of one round.  By halves / by roles, us: 64/8 heads, 2,048 rows behind windows of 33,
+// 64, 128 and 320 keys (3, 4, 6 and 12 blocks; four rounds) 44.5 / 43.8, 44.9 / 45.2, 47.5 / 50.0, 59.0 / 63.4; 8/2 heads, 4,096 rows (one
+// round) behind 128, 256 and 320 16.0 / 15.7, 17.7 / 17.7, 18.7 / 18.9.
+inline bool halves_of_keys(int walk, long long workgroups, int n_cus) { return walk >= (workgroups > n_cus ? 4 : 11); }
+
 // At most this many blocks a tile walks: of all keys up to its last row's, those that the windows of 32 rows can touch.
 inline int most_tile_blocks(int start, int q_len, int kv_valid, int window) {
     const int all = (int)((std::min<long long>(kv_valid, (long long)start + q_len) + 31) / 32);
@@ -64,7 +70,9 @@ inline int most_tile_blocks(int start, int q_len, int kv_valid, int window) {
 // 128 and 16 / 4 of 64, 512 to 4096 rows behind 0 to 9000 keys, whole and through windows of 1024 and 4096 keys.  `first_blocks`
 // and `last_blocks`: the key blocks its first and its last tile of 32 rows walk.
 
-// One key block of the chunk kernel's step, by how much of the chip takes part (at D = 256 the card's clock follows it; at 128 half a step of two).
+// One key block of the chunk kernel's step, by how much of the chip takes part (at D = 256 the card's clock follows it; at 128 the kernel
+// over halves of the keys is 10 % below, but the estimates of the other routes belong to this figure: with its own, 717 rows of 16/4 heads behind a
+// window of 4,096 keys went whole, 56 us, and not in ranges, 49).
 inline double chunk_step_us(int D, double fill) { return D == 256 ? 0.47 + 0.50 * fill : D == 128 ? 0.38 + 0.20 * fill : 0.45 + 0.05 * fill; }
 
 struct ChunkEstimate {
