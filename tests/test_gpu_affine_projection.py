@@ -312,6 +312,23 @@ def test_gemm_in_tiles_of_256_rows(gpu_ctx, bits, m, n, tokens, kw):
     assert np.array_equal(_project(gpu_ctx, bits, packed, scales, biases, x[perm], **kw), got[perm])
 
 
+@pytest.mark.parametrize("bits,m,n,tokens,kw", [
+    (4, 130, 17 * G, 520, {}), (4, 130, 18 * G, 520, {"weights_offset": 2}), (4, 130, 19 * G, 520, {}), (8, 130, 17 * G, 520, {}),
+    (8, 130, 19 * G, 520, {"weights_offset": 2}),                                                          # tiles of 64 tokens
+    (4, 2048, 18 * G, 1100, {}), (8, 2048, 21 * G, 1600, {}),                                              # of 96, and of 128 in two parts
+    (4, 2048, 2 * G, 2100, {}), (8, 2048, 3 * G, 2100, {}), (4, 2048, 7 * G, 2100, {"weights_offset": 2}),  # of 256 rows: one and two spans
+    (4, 2000, 37 * G, 5000, {}), (8, 2048, 35 * G, 5000, {"weights_offset": 2})])                          # two workgroups a CU: scales staged twice
+def test_gemm_over_every_remainder_of_a_span(gpu_ctx, bits, m, n, tokens, kw):
+    # Levels come a span (four groups of 4 bits, two of 8) ahead and x two groups ahead: fewer groups than either, and last spans of every length.
+    packed, scales, biases = _weights(m, n, bits, 125 + bits)
+    x = np.random.default_rng(126).standard_normal((tokens, n)).astype(np.float16)
+    got = _project(gpu_ctx, bits, packed, scales, biases, x, **kw)
+    pick = _sampled(tokens)
+    want = oracle.affine_projection(packed, scales, biases, x[pick].astype(np.float32), bits, half_weights=True)
+    _assert_parity(got[pick], want, _magnitude(packed, scales, biases, x[pick], bits), f"bits={bits} m={m} n={n} tokens={tokens} {kw}")
+    assert np.isfinite(got).all()
+
+
 def test_closed_forms(gpu_ctx):
     # constant rows are carried by the bias term alone (Int8AffineGEMVTests.swift:104-110); a one-hot x picks a column
     for bits in (4, 8):

@@ -22,6 +22,7 @@ namespace tt {
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 
@@ -383,7 +384,6 @@ void launch_tile(tt_hip_ctx *ctx, const ProjArgs &a) {
 // wavefronts through LDS in a fixed order.  256 workgroups at 2048 rows.
 // ---------------------------------------------------------------------------
 constexpr int kGemvWaves = 8, kGemvRows = 8, kGemvMaxTokens = 4;
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float dot8(h8 a, h8 b) {
     float d = 0.0f;
@@ -501,22 +501,27 @@ void launch_gemv(tt_hip_ctx *ctx, const ProjArgs &a) {
 //
 // A workgroup of 4 wavefronts owns 128 tokens x 128 weight rows; a wavefront 32 of the rows against all
 // 128 tokens, four 32x32 accumulators (no row's levels are widened twice).  Per group of 64 columns:
-// the x tile (128 x 64) goes global -> registers -> LDS (one copy per workgroup, double buffered, rows
-// padded to 144 B so that the fragment reads are conflict-free) and is read as A fragments; a lane
-// reads its own 16 / 32 bytes of levels of its weight row straight from global memory, widens and
-// scales them in registers into the B fragments of a group (no LDS, no shuffle), and 16 MFMAs per
+// the x tile (128 x 64) goes straight into LDS (one copy per workgroup, a ring of three, a group's copies issued two groups ahead) and is
+// read as A fragments; a wavefront's levels go there too, whole lines of its rows for four groups of 4 bits (two of 8) at a time, a span
+// ahead, and a lane reads its row's from there, widens and scales them in registers into the B fragments of a group, and 16 MFMAs per
 // group follow (4 contraction steps x 4 token tiles), each step's A fragments read while the step before it
-// multiplies; the rows' scales and biases come from a block in LDS, converted to fp16 once.  One barrier per
-// group, in its middle.  The output tile leaves through LDS, [token][row], as 16-byte stores.
+// multiplies (tiles of fewer tokens: two steps before); the rows' scales and biases come from a block in LDS, converted to fp16 once.  One barrier per
+// group.  The output tile leaves through LDS, [token][row], as 16-byte stores.
+// Before, x went through registers and a lane read its own 16 bytes of levels, 32 rows an instruction, with the MFMAs of a step in runs of three behind
+// one run of widening.  2048 x 4096 over 4 bits, 513 / 777 / 1,024 / 1,500 / 2,048 / 4,096 tokens 26.9 / 27.6 / 29.0 / 36.9 / 43.6 / 74.4 -> 23.7 / 25.3 /
+// 27.0 / 33.3 / 40.2 / 70.6 us (0.97 PFLOP/s), over 8 bits 29.3 / 29.7 / 30.9 / 39.2 / 46.5 / 76.7 -> 24.2 / 26.3 / 28.4 / 34.7 / 41.7 / 74.4.  What is left, from
+// builds without one thing (4,096 tokens; 1,024): MFMAs 21 us; 5, fragment reads 14; 3, widening 11; 5, copies 11; 3, the barrier 0; 0.
 // ---------------------------------------------------------------------------
 constexpr int kGemmTokens = 128, kGemmWaves = 4, kGemmRows = 32 * kGemmWaves;
-// From here on the chunk is a GEMM: 28-29 us up to 1024 tokens, 38 beyond and 43 at 2048, where its grid fills the chip, against
+// From here on the chunk is a GEMM: 24-27 us up to 1024 tokens, 33 beyond and 40 at 2048, where its grid fills the chip, against
 // 26 us at 512 tokens for the tiles above, whose time goes on growing by 25 us per 512 tokens.
 constexpr int kGemmMinTokens = 513;
 constexpr int kGemmThreads = kGemmWaves * 64;
-constexpr int kGemmPitch = kProjGroup + 8;                           // halves per token row of the x tile in LDS
-constexpr int kGemmParamGroups = 64;                                 // groups whose scales and biases sit in LDS at a time
-constexpr int gemm_tile_halves(int tokens) { return tokens * kGemmPitch; }
+constexpr int kGemmRing = 3;           // groups of x in LDS: read, landed, on their way
+constexpr int kGemmLevelBytes = 4096;  // a wavefront's levels in LDS: 32 rows x 128 bytes
+constexpr int gemm_tile_bytes(int tokens) { return tokens * 2 * kProjGroup; }
+// Groups whose scales and biases sit in LDS at a time: 64, over the parts that walk columns of their own; half as many where two workgroups share a CU.
+constexpr int gemm_param_groups(int ks, bool rs) { return rs ? 64 : ks == 1 ? 32 : 64 / ks; }
 // KS = parts the columns are split into inside a workgroup (1 or 2): KS x 4 wavefronts, part p's four take the
 // groups [p x part_groups, (p + 1) x part_groups) with x tiles and a block of scales and biases of their own, and
 // the parts' accumulators are added through LDS at the end, in a fixed order.  For chunks whose tiles number no
@@ -526,27 +531,61 @@ constexpr int gemm_tile_halves(int tokens) { return tokens * kGemmPitch; }
 // Its time goes with the tokens of its tile more than with its columns' parts (a third and fourth part of a tile of 64
 // tokens: 31.3 us against 29.1 at 777 tokens, its registers halved), so a chunk that leaves CUs without a workgroup takes
 // tiles of 64 or 96 (TOKENS).
-constexpr int gemm_lds_bytes(int ks, int tokens = kGemmTokens) {
-    return ks * 2 * gemm_tile_halves(tokens) * (int)sizeof(_Float16) + kGemmParamGroups * kGemmRows * 4;
+constexpr int gemm_lds_bytes(int ks, bool rs, int tokens) {
+    const int x = (rs ? 1 : ks) * kGemmRing * gemm_tile_bytes(tokens), rows = rs ? ks * kGemmRows : kGemmRows;
+    return x + ks * kGemmWaves * kGemmLevelBytes + (rs ? 1 : ks) * gemm_param_groups(ks, rs) * rows * 4;
 }
-constexpr int gemm_rs_lds_bytes() { return 2 * gemm_tile_halves(kGemmTokens) * (int)sizeof(_Float16) + kGemmParamGroups * 2 * kGemmRows * 4; }
+static_assert(gemm_lds_bytes(1, false, kGemmTokens) <= 80 * 1024, "two workgroups to a CU");
+
+// N copies of 16 bytes a lane, global -> LDS, the i-th to lds_addr + 1024 i + 16 lane.  (An instruction's offset counts for both places, so the
+// i-th source comes 1024 i below itself.)  In assembly: the compiler, seeing a copy into LDS, guards every later LDS read with a wait for
+// all of them.  m0 is the compiler's (naming it as a clobber is not honoured): saved and put back.
+template <int N>
+__device__ __forceinline__ void copies_to_lds(const char *const (&src)[N], unsigned lds_addr) {
+    static_assert(N >= 2 && N <= 4, "two to four copies");
+    lds_addr = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
+    unsigned saved_m0;
+    if constexpr (N == 2)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
+                     "s_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "s"(lds_addr), "v"(src[0]), "v"(src[1])
+                     : "memory");
+    else if constexpr (N == 3)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
+                     "global_load_lds_dwordx4 %4, off offset:2048\n\ts_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "s"(lds_addr), "v"(src[0]), "v"(src[1]), "v"(src[2])
+                     : "memory");
+    else
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
+                     "global_load_lds_dwordx4 %4, off offset:2048\n\tglobal_load_lds_dwordx4 %5, off offset:3072\n\ts_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "s"(lds_addr), "v"(src[0]), "v"(src[1]), "v"(src[2]), "v"(src[3])
+                     : "memory");
+}
+// vmcnt(n) only: leaves the LDS and export counters alone.
+#define TT_WAIT_COPIES(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
 template <int BITS, bool ALIGNED, int KS, bool RS = false, int TOKENS = kGemmTokens>
 __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const ProjArgs a) {
     // RS (with KS = 2): the two parts split the ROWS instead of the columns -- a tile of 128 tokens x 256 rows, one x
     // tile for all eight wavefronts.
-    constexpr int kThreads = kGemmThreads * KS, kPartParamGroups = RS ? kGemmParamGroups : kGemmParamGroups / KS;
+    constexpr int kThreads = kGemmThreads * KS, kPartParamGroups = gemm_param_groups(KS, RS);
     constexpr int kRows = RS ? kGemmRows * KS : kGemmRows;
-    constexpr int kStageThreads = RS ? kThreads : kGemmThreads, kStagePasses = TOKENS * 8 / kStageThreads;
+    constexpr int kStageThreads = RS ? kThreads : kGemmThreads, kCopies = TOKENS * 8 / kStageThreads;  // x copies of a wavefront per group
     constexpr int TT = TOKENS / 32;  // 32-token tiles: accumulators of a wavefront
-    static_assert(kGemmWaves * 64 * 16 * TT * (int)sizeof(float) <= gemm_lds_bytes(2, TOKENS), "the parts' accumulators meet in the store");
-    // per part two x tiles of TOKENS x kGemmPitch halves, then per part [kPartParamGroups][kGemmRows] (scale, bias) pairs as fp16
+    static_assert(kGemmWaves * 64 * 16 * TT * (int)sizeof(float) <= gemm_lds_bytes(2, false, TOKENS), "the parts' accumulators meet in the store");
+    // per part kGemmRing x tiles of TOKENS x 128 bytes, then per wavefront its levels, then per part [kPartParamGroups][kRows] (scale, bias)
+    // pairs as fp16.  A token's (a row's) 16-byte pieces are permuted by its number, so that the fragment reads hit every bank.
     extern __shared__ __attribute__((aligned(16))) _Float16 lds_store[];
     const int part = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kGemmThreads);
     const int tid = threadIdx.x % kGemmThreads, lane = tid & 63, wave = tid >> 6;  // tid, wave: inside the part
     const int stage_tid = RS ? (int)threadIdx.x : tid;
-    auto tile = [&](int which) { return lds_store + ((RS ? 0 : 2 * part) + which) * gemm_tile_halves(TOKENS); };
-    unsigned *const params = reinterpret_cast<unsigned *>(lds_store + (RS ? 1 : KS) * 2 * gemm_tile_halves(TOKENS)) + (RS ? 0 : part * kPartParamGroups * kRows);
+    constexpr int kXBytes = kGemmRing * gemm_tile_bytes(TOKENS), kXParts = RS ? 1 : KS;
+    char *const lds_bytes = reinterpret_cast<char *>(lds_store), *const x_tiles = lds_bytes + (RS ? 0 : part * kXBytes);
+    char *const level_tile = lds_bytes + kXParts * kXBytes + (kGemmWaves * part + wave) * kGemmLevelBytes;
+    unsigned *const params = reinterpret_cast<unsigned *>(lds_bytes + kXParts * kXBytes + KS * kGemmWaves * kGemmLevelBytes) + (RS ? 0 : part * kPartParamGroups * kRows);
     const int c = lane & 31, h = lane >> 5;
     // A wavefront owns 32 weight rows against all 128 tokens: every row's levels are widened by exactly one wavefront.
     // Workgroups are dealt to the 8 XCDs in turn, each with its own L2: the workgroups that share a token block
@@ -566,24 +605,46 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     const int part_groups = (groups + kColumnParts * kSpan - 1) / (kColumnParts * kSpan) * kSpan, first_group = RS ? 0 : part * part_groups;
     const size_t row_bytes = (size_t)a.columns * BITS / 8;
 
-    // x staging: thread -> 16 bytes (8 columns) of token tid / 8 (+ 32 per further pass): 8 threads read a row's 128 B
-    const _Float16 *x_src[kStagePasses];
-    int x_dst[kStagePasses];
+    // x: a copy of a wavefront is eight tokens' 128 bytes of a group.
+    const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) void *)lds_store;
+    const unsigned x_lds = lds_base + (unsigned)(x_tiles - lds_bytes) + (unsigned)((stage_tid >> 6) * kCopies * 1024);
+    const char *x_src[kCopies];
 #pragma unroll
-    for (int p = 0; p < kStagePasses; ++p) {
-        const int local = (stage_tid >> 3) + (kStageThreads / 8) * p;
-        x_src[p] = a.x + (long long)min(token0 + local, a.tokens - 1) * a.x_stride + 8 * (stage_tid & 7);
-        x_dst[p] = local * kGemmPitch + 8 * (stage_tid & 7);
+    for (int p = 0; p < kCopies; ++p) {
+        const int local = 8 * ((stage_tid >> 6) * kCopies + p) + (lane >> 3);
+        x_src[p] = reinterpret_cast<const char *>(a.x + (long long)min(token0 + local, a.tokens - 1) * a.x_stride) + 16 * ((lane & 7) ^ (lane >> 3)) - 1024 * p;
     }
+    auto copy_x = [&](int g, unsigned slot) {  // slot: the tile's offset in the ring
+        const int gc = min(first_group + g, groups - 1);  // past the end: the last group again, a valid address, unused
+        const char *src[kCopies];
+#pragma unroll
+        for (int p = 0; p < kCopies; ++p) src[p] = x_src[p] + 2 * kProjGroup * gc;
+        copies_to_lds<kCopies>(src, x_lds + slot);
+    };
     const int param_at = (RS ? kGemmRows * part : 0) + 32 * wave + c;  // this lane's weight row inside the workgroup's tile
-    const uint8_t *const w_src = a.weights + (size_t)min(row0 + param_at, a.rows - 1) * row_bytes;
-    // Scales and biases of this workgroup's rows for groups [first, first + kGemmParamGroups): a thread takes eight
+    // Levels: the 128 bytes of a span of the wavefront's 32 rows, a line each, in four copies of eight rows.  (Read by the lanes themselves, 16
+    // bytes of 32 rows an instruction, they were 32 lines for every KiB, and a CU's path to memory takes two cycles a line whatever is wanted of it:
+    // copies of 32, 64 and 128 bytes a row run at 34, 69 and 115 KB/us a CU.)
+    const unsigned level_lds = lds_base + (unsigned)(level_tile - lds_bytes);
+    const uint8_t *const w_row = a.weights + (size_t)min(row0 + param_at, a.rows - 1) * row_bytes;
+    const char *w_src[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = (RS ? kGemmRows * part : 0) + 32 * wave + 8 * i + (lane >> 3);
+        w_src[i] = reinterpret_cast<const char *>(a.weights + (size_t)min(row0 + row, a.rows - 1) * row_bytes) - 1024 * i;
+    }
+    auto copy_levels = [&](int first) {  // of groups [first, first + kSpan)
+        const size_t at = min((size_t)(first_group + first) * (8 * BITS) + 16 * ((lane & 7) ^ (lane >> 3)), row_bytes - 16);
+        const char *const src[4] = {w_src[0] + at, w_src[1] + at, w_src[2] + at, w_src[3] + at};
+        copies_to_lds<4>(src, level_lds);
+    };
+    // Scales and biases of this workgroup's rows for groups [first, first + kPartParamGroups): a thread takes eight
     // consecutive groups of a row, 16 bytes of scales and 16 of biases, and eight threads a row's 128 bytes, so the
     // rows are read as whole lines (one value per thread and load made 64 loads of 2 bytes per thread, every lane on
     // a line of its own: 16 us of a 107 us launch at 4096 tokens).  Converted to fp16 and stored [group][row], so that
     // the lanes of a wavefront -- consecutive rows -- read consecutive words.
     constexpr int kRowThreads = kPartParamGroups / 8, kPassRows = kStageThreads / kRowThreads;
-    static_assert(kGemmParamGroups == 64 && kGemmThreads == 256 && kRows % kPassRows == 0, "eight groups a thread");
+    static_assert(kPartParamGroups % 8 == 0 && kRows % kPassRows == 0, "eight groups a thread");
     const bool params_vector = (uintptr_t)a.scales % 16 == 0 && (uintptr_t)a.biases % 16 == 0 && groups % 8 == 0;
     auto stage_params = [&](int first) {
         const int k = 8 * (stage_tid % kRowThreads), g = first_group + first + k;
@@ -622,109 +683,143 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) acc[tt] = zero;
 
-    // x rows are loaded two groups ahead of their use: slot g % 2 of x_ring holds group g's rows until they go
-    // to LDS at the start of group g - 1 (the loop over a span is unrolled and spans are even, so the slot is a
-    // constant).
-    h8 x_ring[2][kStagePasses];
-    auto load_x = [&](h8 (&dst)[kStagePasses], int g) {
-        const int gc = min(first_group + g, groups - 1);  // past the end: the last group again, a valid address, unused
-#pragma unroll
-        for (int p = 0; p < kStagePasses; ++p) dst[p] = *reinterpret_cast<const h8 *>(x_src[p] + kProjGroup * gc);
-    };
-    auto store_x = [&](const h8 (&src)[kStagePasses], int g) {
-#pragma unroll
-        for (int p = 0; p < kStagePasses; ++p) *reinterpret_cast<h8 *>(tile(g & 1) + x_dst[p]) = src[p];
-    };
-    unsigned w_now[kSpan][BITS], w_next[kSpan][BITS];
+    unsigned w_now[kSpan][BITS], w_later[kSpan][BITS];  // (w_later: levels that are not aligned come by register, a span ahead)
     auto load_span = [&](unsigned (&w)[kSpan][BITS], int first) {
 #pragma unroll
         for (int k = 0; k < kSpan; ++k) {
             const int g = min(first_group + first + k, groups - 1);  // past the end: the last group again, a valid address, unused
-            load_levels<BITS, ALIGNED>(w[k], w_src + (size_t)g * (2 * kHalfGroupBytes) + h * kHalfGroupBytes);
+            load_levels<BITS, false>(w[k], w_row + (size_t)g * (2 * kHalfGroupBytes) + h * kHalfGroupBytes);
         }
     };
-    load_x(x_ring[0], 0);
-    load_x(x_ring[1], 1);
-    load_span(w_next, 0);
+    auto read_span = [&]() {
+#pragma unroll
+        for (int k = 0; k < kSpan; ++k)
+#pragma unroll
+            for (int i = 0; i < BITS / 4; ++i) {
+                const int piece = (BITS / 4) * (2 * k + h) + i;
+                const u4v v = *reinterpret_cast<const u4v *>(level_tile + c * 128 + ((piece ^ (c & 7)) << 4));
+                w_now[k][4 * i] = v[0];
+                w_now[k][4 * i + 1] = v[1];
+                w_now[k][4 * i + 2] = v[2];
+                w_now[k][4 * i + 3] = v[3];
+            }
+    };
+    if constexpr (ALIGNED) {
+        copy_levels(0);
+    } else {
+        load_span(w_now, 0);
+        load_span(w_later, kSpan);
+    }
+    copy_x(0, 0);
+    copy_x(1, gemm_tile_bytes(TOKENS));
     stage_params(0);
-    store_x(x_ring[0], 0);
-    load_x(x_ring[0], 2);
+    TT_WAIT_COPIES(0);
     __syncthreads();
+    if constexpr (ALIGNED) {
+        read_span();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (part_groups > kSpan) copy_levels(kSpan);
+    }
 
-    // B fragments of a group: its levels widened and scaled, bw[g % 2].  They are made one group ahead, in the
-    // shadow of the previous group's MFMAs: the matrix pipe takes 32 cycles per MFMA and the wavefront issues the
-    // next group's VALU work meanwhile, instead of widening first and multiplying after.
-    h8 bw[2][4];
-    auto widen_scale = [&](h8 &dst, const unsigned (&w)[BITS], int t, h8 scale, h8 bias) {
-        h8 levels;
-        if constexpr (BITS == 4) levels = levels_of_nibbles(w[t]);
-        else levels = levels_of_bytes(w[2 * t], w[2 * t + 1]);
-        dst = __builtin_elementwise_fma(levels, scale, bias);
+    // B fragments of a group: its levels widened and scaled, bw[g % 2], four registers of two halves each.  They are made one group ahead, a
+    // pair at a time behind the current group's MFMAs.
+    unsigned bw[2][4][4];
+    unsigned exponents = BITS == 4 ? 0x54006400u : 0x64646464u;  // (in a vector register: an instruction takes one scalar one)
+    asm volatile("" : "+v"(exponents));
+    auto widen_pair = [&](unsigned &dst, const unsigned (&w)[BITS], int t, int p, h2 scale, h2 bias) {  // columns 2 p, 2 p + 1 of a lane's eight
+        unsigned v;
+        h2 zero_level;
+        if constexpr (BITS == 4) {  // byte p twice: the low nibble under the exponent of 1024, the high one, four places up, under that of 64
+            v = (__builtin_amdgcn_perm(w[t], w[t], 0x0c000c00u + 0x00010001u * p) & 0x00f0000fu) | exponents;
+            zero_level = h2{1024, 64};
+        } else {
+            v = __builtin_amdgcn_perm(exponents, w[2 * t + p / 2], p % 2 ? 0x04030402u : 0x04010400u);
+            zero_level = h2{1024, 1024};
+        }
+        dst = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(h2, v) - zero_level, scale, bias));
     };
     // Past the matrix's last group the scale and the bias are zero: such a group's products add nothing, and the
     // loop over a span needs no exit in its middle.
     auto pair_of = [&](int g) { return first_group + g < groups ? params[(g % kPartParamGroups) * kRows + param_at] : 0u; };
-    auto scale_of = [&](unsigned pair) { return (h8)__builtin_bit_cast(_Float16, (uint16_t)(pair & 0xffffu)); };
-    auto bias_of = [&](unsigned pair) { return (h8)__builtin_bit_cast(_Float16, (uint16_t)(pair >> 16)); };
+    auto scale_of = [&](unsigned pair) { return (h2)__builtin_bit_cast(_Float16, (uint16_t)(pair & 0xffffu)); };
+    auto bias_of = [&](unsigned pair) { return (h2)__builtin_bit_cast(_Float16, (uint16_t)(pair >> 16)); };
     {
         const unsigned pair = pair_of(0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) widen_scale(bw[0][t], w_next[0], t, scale_of(pair), bias_of(pair));
-    }
-    // A fragments of contraction step t of a group: 32 tokens x 16 columns per token tile, af[t % 2]; a step's
-    // fragments are read from LDS while the step before it multiplies.
-    h8 af[2][TT];
-    auto read_fragments = [&](h8 (&dst)[TT], int g, int t) {
-        const _Float16 *xt = tile(g & 1);
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt) dst[tt] = *reinterpret_cast<const h8 *>(xt + (32 * tt + c) * kGemmPitch + 32 * h + 8 * t);
-    };
-    read_fragments(af[0], 0, 0);
+            for (int p = 0; p < 4; ++p) widen_pair(bw[0][t][p], w_now[0], t, p, scale_of(pair), bias_of(pair));
+    }
+    // A fragments of contraction step t of a group: 32 tokens x 16 columns per token tile, af[t]; a step's
+    // fragments are read from LDS kAhead steps before they multiply.
+    constexpr int kAhead = TT >= 4 ? 1 : 2;
+    h8 af[4][TT];
+    const int fragment_at = c * 128 + (((4 * h) ^ (c & 7)) << 4);
+    auto fragment = [&](unsigned slot, int t, int tt) { return *reinterpret_cast<const h8 *>(x_tiles + slot + (fragment_at ^ (t << 4)) + 4096 * tt); };
+    // The ring's places: of the group in hand, of the next (landed at the barrier) and of the one whose copies go out now.
+    unsigned here = 0, next = gemm_tile_bytes(TOKENS), ahead = 2 * gemm_tile_bytes(TOKENS);
+#pragma unroll
+    for (int t = 0; t < kAhead; ++t)
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) af[t][tt] = fragment(here, t, tt);
 
     for (int g0 = 0; g0 < part_groups; g0 += kSpan) {
-#pragma unroll
-        for (int k = 0; k < kSpan; ++k)
-#pragma unroll
-            for (int i = 0; i < BITS; ++i) w_now[k][i] = w_next[k][i];
-        load_span(w_next, g0 + kSpan);  // the next span's levels are in flight for the whole of this one
+        const bool more_spans = g0 + kSpan < part_groups, still_more = g0 + 2 * kSpan < part_groups;
 #pragma unroll
         for (int k = 0; k < kSpan; ++k) {
             const int g = g0 + k;
-            static_assert(kSpan % 2 == 0, "the ring slots of a group must not depend on the span");
-            // Group g + 1's rows go to the tile that group g - 1 was read from (every wavefront is past that
-            // group's barrier, behind which nobody reads it), and their registers take group g + 3's.
-            store_x(x_ring[(k + 1) & 1], g + 1);
-            load_x(x_ring[(k + 1) & 1], g + 3);
+            static_assert(kSpan % 2 == 0, "a group's fragments must not depend on the span");
             const unsigned pair_next = pair_of(g + 1);
-            const h8 scale_next = scale_of(pair_next), bias_next = bias_of(pair_next);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                __builtin_amdgcn_sched_barrier(0);
-                if (t == 3) {
-                    // Everybody's rows of group g + 1 are in LDS from here on, and nobody reads group g's any more.
-                    __syncthreads();
-                    read_fragments(af[0], g + 1, 0);
+            const h2 scale_next = scale_of(pair_next), bias_next = bias_of(pair_next);
+            // The copies of this group: x of group g + 2 into the place that group g - 1 was read from (every wavefront is past that group's barrier), and in
+            // a span's last group, when the next span's levels have gone to their registers, those of the span behind it.
+            const bool more_x = g + 2 < part_groups;
+            if (k == kSpan - 1 && more_spans) {
+                if constexpr (ALIGNED) {
+                    read_span();
                 } else {
-                    read_fragments(af[(t + 1) & 1], g, t + 1);
-                }
 #pragma unroll
-                for (int tt = 0; tt < TT; ++tt)
-                    acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t & 1][tt], bw[k & 1][t], acc[tt], 0, 0, 0);
-                // a quarter of the next group's fragments per MFMA step (after the last group: made and not used).
-                // The empty statements tie the quarter to this step: without them all four are made in one run
-                // before the group's first MFMA, and the matrix pipe idles meanwhile.
-                unsigned(&w_of_next)[BITS] = k + 1 < kSpan ? w_now[(k + 1) % kSpan] : w_next[0];
+                    for (int i = 0; i < kSpan; ++i)
 #pragma unroll
-                for (int i = 0; i < BITS / 4; ++i) asm volatile("" : "+v"(w_of_next[(BITS / 4) * t + i]));
-                widen_scale(bw[(k + 1) & 1][t], w_of_next, t, scale_next, bias_next);
-                asm volatile("" : "+v"(bw[(k + 1) & 1][t]));
-#pragma unroll
-                for (int i = 0; i < TT; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one fragment read
-                    __builtin_amdgcn_sched_group_barrier(0x002, 20 / TT, 0);  // a share of the widening
+                        for (int j = 0; j < BITS; ++j) w_now[i][j] = w_later[i][j];
                 }
             }
+            const unsigned(&w_of_next)[BITS] = w_now[(k + 1) % kSpan];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (t == 0 && more_x) copy_x(g + 2, ahead);
+                const bool levels_out = k == kSpan - 1 && still_more;
+                if (t == 1 && levels_out) {
+                    if constexpr (ALIGNED) {
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read_span's)
+                        copy_levels(g0 + 2 * kSpan);
+                    } else {
+                        load_span(w_later, g0 + 2 * kSpan);
+                    }
+                }
+                if (t == 4 - kAhead) {
+                    // Everybody's rows of group g + 1 are in LDS from here on: of the copies only this group's may still be on their way.
+                    if (ALIGNED && levels_out) TT_WAIT_COPIES(kCopies + 4);  // (a span behind the next: there is more x)
+                    else if (more_x) TT_WAIT_COPIES(kCopies);
+                    else TT_WAIT_COPIES(0);
+                    __syncthreads();
+                }
+                const h8 b = __builtin_bit_cast(h8, u4v{bw[k & 1][t][0], bw[k & 1][t][1], bw[k & 1][t][2], bw[k & 1][t][3]});
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt) {
+                    // One MFMA, one fragment read and a share of the next group's widening, in this order: the two wavefronts of a SIMD then have
+                    // something else to issue between any two MFMAs.
+                    acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t][tt], b, acc[tt], 0, 0, 0);
+                    af[(t + kAhead) % 4][tt] = fragment(t + kAhead < 4 ? here : next, (t + kAhead) % 4, tt);
+#pragma unroll
+                    for (int p = tt * 4 / TT; p < (tt + 1) * 4 / TT; ++p) widen_pair(bw[(k + 1) & 1][t][p], w_of_next, t, p, scale_next, bias_next);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            const unsigned done = here;
+            here = next;
+            next = ahead;
+            ahead = done;
             // The next block of scales and biases is first read one step before its first group is multiplied.
             if ((g + 2) % kPartParamGroups == 0 && g + 2 < part_groups) {  // the whole workgroup
                 __syncthreads();                                       // everyone has read this block
@@ -757,7 +852,7 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     }
     _Float16 *const out_tile = lds_store;
     constexpr int kOutPitch = kRows + 8;
-    static_assert(TOKENS * kOutPitch * (int)sizeof(_Float16) <= (RS ? gemm_rs_lds_bytes() : gemm_lds_bytes(KS, TOKENS)), "the output tile takes the store's space");
+    static_assert(TOKENS * kOutPitch * (int)sizeof(_Float16) <= gemm_lds_bytes(KS, RS, TOKENS), "the output tile takes the store's space");
     if (part == 0 || RS) {
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt)
@@ -786,11 +881,11 @@ __global__ __launch_bounds__(kGemmThreads * KS, 2) void affine_gemm_kernel(const
     }
 }
 
-// 68 KiB of LDS (104 KiB with two parts): above the 64 KiB a kernel gets without asking.
+// 80 to 160 KiB of LDS: above the 64 KiB a kernel gets without asking.
 template <int BITS, bool ALIGNED, int KS, bool RS = false, int TOKENS = kGemmTokens>
 int launch_gemm(tt_hip_ctx *ctx, const ProjArgs &a, dim3 grid) {
     auto kernel = affine_gemm_kernel<BITS, ALIGNED, KS, RS, TOKENS>;  // its LDS limit was raised when the context was created
-    launch_profiled(ctx, kernel, grid, dim3(kGemmThreads * KS), (unsigned)(RS ? gemm_rs_lds_bytes() : gemm_lds_bytes(KS, TOKENS)), a);
+    launch_profiled(ctx, kernel, grid, dim3(kGemmThreads * KS), (unsigned)gemm_lds_bytes(KS, RS, TOKENS), a);
     return TT_HIP_OK;
 }
 
@@ -801,26 +896,26 @@ int configure_affine_kernels(tt_hip_ctx *ctx) {
     hipError_t e = hipSuccess;
 #define TT_CFG(KERNEL, BYTES) \
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);
-    TT_CFG((affine_gemm_kernel<4, true, 1>), gemm_lds_bytes(1))
-    TT_CFG((affine_gemm_kernel<4, false, 1>), gemm_lds_bytes(1))
-    TT_CFG((affine_gemm_kernel<8, true, 1>), gemm_lds_bytes(1))
-    TT_CFG((affine_gemm_kernel<8, false, 1>), gemm_lds_bytes(1))
-    TT_CFG((affine_gemm_kernel<4, true, 2>), gemm_lds_bytes(2))
-    TT_CFG((affine_gemm_kernel<4, false, 2>), gemm_lds_bytes(2))
-    TT_CFG((affine_gemm_kernel<8, true, 2>), gemm_lds_bytes(2))
-    TT_CFG((affine_gemm_kernel<8, false, 2>), gemm_lds_bytes(2))
-    TT_CFG((affine_gemm_kernel<4, true, 2, false, 64>), gemm_lds_bytes(2, 64))
-    TT_CFG((affine_gemm_kernel<4, true, 2, false, 96>), gemm_lds_bytes(2, 96))
-    TT_CFG((affine_gemm_kernel<4, false, 2, false, 64>), gemm_lds_bytes(2, 64))
-    TT_CFG((affine_gemm_kernel<4, false, 2, false, 96>), gemm_lds_bytes(2, 96))
-    TT_CFG((affine_gemm_kernel<8, true, 2, false, 64>), gemm_lds_bytes(2, 64))
-    TT_CFG((affine_gemm_kernel<8, true, 2, false, 96>), gemm_lds_bytes(2, 96))
-    TT_CFG((affine_gemm_kernel<8, false, 2, false, 64>), gemm_lds_bytes(2, 64))
-    TT_CFG((affine_gemm_kernel<8, false, 2, false, 96>), gemm_lds_bytes(2, 96))
-    TT_CFG((affine_gemm_kernel<4, true, 2, true>), gemm_rs_lds_bytes())
-    TT_CFG((affine_gemm_kernel<4, false, 2, true>), gemm_rs_lds_bytes())
-    TT_CFG((affine_gemm_kernel<8, true, 2, true>), gemm_rs_lds_bytes())
-    TT_CFG((affine_gemm_kernel<8, false, 2, true>), gemm_rs_lds_bytes())
+    TT_CFG((affine_gemm_kernel<4, true, 1>), gemm_lds_bytes(1, false, 128))
+    TT_CFG((affine_gemm_kernel<4, false, 1>), gemm_lds_bytes(1, false, 128))
+    TT_CFG((affine_gemm_kernel<8, true, 1>), gemm_lds_bytes(1, false, 128))
+    TT_CFG((affine_gemm_kernel<8, false, 1>), gemm_lds_bytes(1, false, 128))
+    TT_CFG((affine_gemm_kernel<4, true, 2>), gemm_lds_bytes(2, false, 128))
+    TT_CFG((affine_gemm_kernel<4, false, 2>), gemm_lds_bytes(2, false, 128))
+    TT_CFG((affine_gemm_kernel<8, true, 2>), gemm_lds_bytes(2, false, 128))
+    TT_CFG((affine_gemm_kernel<8, false, 2>), gemm_lds_bytes(2, false, 128))
+    TT_CFG((affine_gemm_kernel<4, true, 2, false, 64>), gemm_lds_bytes(2, false, 64))
+    TT_CFG((affine_gemm_kernel<4, true, 2, false, 96>), gemm_lds_bytes(2, false, 96))
+    TT_CFG((affine_gemm_kernel<4, false, 2, false, 64>), gemm_lds_bytes(2, false, 64))
+    TT_CFG((affine_gemm_kernel<4, false, 2, false, 96>), gemm_lds_bytes(2, false, 96))
+    TT_CFG((affine_gemm_kernel<8, true, 2, false, 64>), gemm_lds_bytes(2, false, 64))
+    TT_CFG((affine_gemm_kernel<8, true, 2, false, 96>), gemm_lds_bytes(2, false, 96))
+    TT_CFG((affine_gemm_kernel<8, false, 2, false, 64>), gemm_lds_bytes(2, false, 64))
+    TT_CFG((affine_gemm_kernel<8, false, 2, false, 96>), gemm_lds_bytes(2, false, 96))
+    TT_CFG((affine_gemm_kernel<4, true, 2, true>), gemm_lds_bytes(2, true, 128))
+    TT_CFG((affine_gemm_kernel<4, false, 2, true>), gemm_lds_bytes(2, true, 128))
+    TT_CFG((affine_gemm_kernel<8, true, 2, true>), gemm_lds_bytes(2, true, 128))
+    TT_CFG((affine_gemm_kernel<8, false, 2, true>), gemm_lds_bytes(2, true, 128))
     TT_CFG((affine_tile_kernel<4, true, 1, 1, 4>), tile_lds_bytes(4, true, 1, 1, 4))
     TT_CFG((affine_tile_kernel<4, true, 1, 2, 4>), tile_lds_bytes(4, true, 1, 2, 4))
     TT_CFG((affine_tile_kernel<4, true, 2, 2, 4>), tile_lds_bytes(4, true, 2, 2, 4))
