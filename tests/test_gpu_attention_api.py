@@ -226,6 +226,24 @@ def test_prefill_padded_strides_and_offset_buffers(gpu_ctx, H, KH, D, start, chu
     c.close()
 
 
+# One split: the launch itself writes the gated rows, a thread's items with their gate values asked for together.  Tiles whose
+# valid rows end inside a round of items, fill one, or leave rounds without any.
+@pytest.mark.parametrize("H,KH,D", [(6, 2, 256), (5, 1, 128), (16, 2, 256), (12, 4, 64)])
+@pytest.mark.parametrize("chunk", [1, 2, 3, 7])
+def test_gated_rows_of_one_split(gpu_ctx, H, KH, D, chunk):
+    start, r = 90, np.random.default_rng(H * D + chunk)
+    q, g = (r.standard_normal((chunk, H * D)).astype(np.float16) for _ in range(2))
+    k, v = (r.standard_normal((start + chunk, KH, D)).astype(np.float16) for _ in range(2))
+    c = Cache(gpu_ctx, k, v)
+    scale = 1.0 / np.sqrt(D)
+    want = oracle.prefill_ref(q.astype(np.float32), c.k32, c.v32, H * D, KH * D, D, H, KH, start, chunk, start + chunk, 0, scale)
+    want = want.reshape(chunk, -1) / (1 + np.exp(-g.astype(np.float64)))
+    for pad, prefix in ((0, (0, 0, 0)), (5, (17, 19, 23))):
+        got = _prefill(gpu_ctx, c.kv, q, start, chunk, start + chunk, H, scale, o_stride=H * D + pad, gate=g, gate_stride=H * D + pad, prefix=prefix)
+        _check(got, want, f"{chunk} gated rows, strides + {pad}")
+    c.close()
+
+
 @pytest.mark.parametrize("start,chunk,gated", [(2100, 70, False), (4000, 130, True), (3000, 32, True),
                                                (8064, 128, True), (8500, 333, False), (9001, 130, True),
                                                (12000, 64, True)])

@@ -83,19 +83,13 @@ __device__ __forceinline__ TileInfo tile_info(const SplitKHot &a, const SplitKSe
 
 // The gate's four values of one output item, asked for ahead of the arithmetic they end up multiplying (a combine pass
 // that fetches them only when its sums are done waits for memory once more with nothing else to do), and kept as they come:
-// converted in the branch that loads them, they were waited for there, in front of the partial results' loads.
+// converted in the branch that loads them, they were waited for there, in front of the partial results' loads.  One load
+// whatever the row's alignment (see load_h8: of two branches, one for each, the compiler waits for a load in the first).
+typedef h4 h4_unaligned __attribute__((aligned(2)));
 template <typename Args>
-__device__ __forceinline__ h4 load_gate4(const Args &a, int seq, int tok, int head, int d, int D, bool aligned) {
+__device__ __forceinline__ h4 load_gate4(const Args &a, int seq, int tok, int head, int d, int D) {
     h4 g = (h4)(_Float16)0.0f;
-    if (a.gate) {
-        const global_halves gp = (global_halves)(a.gate + seq * a.g_seq_stride + tok * a.g_tok_stride + (long long)head * D + d);
-        if (aligned) {
-            g = *(const __attribute__((address_space(1))) h4 *)gp;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) g[i] = gp[i];
-        }
-    }
+    if (a.gate) g = *(const __attribute__((address_space(1))) h4_unaligned *)(global_halves)(a.gate + seq * a.g_seq_stride + tok * a.g_tok_stride + (long long)head * D + d);
     return g;
 }
 // Final value of one output element with the gate's values in hand: normalise, gate in fp32, round once.
@@ -114,33 +108,6 @@ __device__ __forceinline__ void store_out4_gated(const Args &a, int seq, int tok
     } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) op[i] = (_Float16)r[i];
-    }
-}
-
-// Final value of one output element: normalise, gate in fp32, round once.
-__device__ __forceinline__ void store_out4(const SplitKArgs &a, int seq, int tok, int head, int d, int D, f4 o,
-                                           float inv_l, bool aligned) {
-    f4 r = o * inv_l;
-    if (a.gate) {
-        const _Float16 *gp = a.gate + seq * a.g_seq_stride + tok * a.g_tok_stride + (long long)head * D + d;
-        float g0, g1, g2, g3;
-        if (aligned) {
-            h4 gv = *reinterpret_cast<const h4 *>(gp);
-            g0 = (float)gv[0]; g1 = (float)gv[1]; g2 = (float)gv[2]; g3 = (float)gv[3];
-        } else {
-            g0 = (float)gp[0]; g1 = (float)gp[1]; g2 = (float)gp[2]; g3 = (float)gp[3];
-        }
-        r[0] *= sigmoid(g0);
-        r[1] *= sigmoid(g1);
-        r[2] *= sigmoid(g2);
-        r[3] *= sigmoid(g3);
-    }
-    _Float16 *op = a.out + seq * a.o_seq_stride + tok * a.o_tok_stride + (long long)head * D + d;
-    if (aligned) {
-        h4 hv = {(_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3]};
-        *reinterpret_cast<h4 *>(op) = hv;
-    } else {
-        op[0] = (_Float16)r[0]; op[1] = (_Float16)r[1]; op[2] = (_Float16)r[2]; op[3] = (_Float16)r[3];
     }
 }
 
@@ -974,26 +941,13 @@ __device__ __forceinline__ void block_softmax_pv(RowState<D, NT> &st, Scores<D, 
 // KEEP = 4: the same, where few of a touched block's keys are listed (fp16 pages, tiles of 32): the plan lists groups of
 // four keys, and eight listed groups, wherever they lie, make a turn of the loop.
 // KEEP = 5: KEEP = 3 whose blocks' loads cover the listed keys only (lists_fetch_by_key).
-// The hot arguments and this workgroup's sequence entry, by three scalar loads issued together (the compiler
-// would fetch each field where it is first used: five or six dependent trips to the kernarg segment before
-// the first K/V load can go out, about 0.15 us each).
+// The hot arguments, this workgroup's sequence entry and where the rows go and their gate beside them, by five scalar loads issued
+// together (the compiler would fetch each field where it is first used: five or six dependent trips to the kernarg segment before
+// the first K/V load can go out, about 0.15 us each, and another ahead of the gate's loads).
 typedef int i16v __attribute__((ext_vector_type(16)));
 struct HotWords {
     i16v lo, hi;
 };
-__device__ __forceinline__ void load_hot(SplitKHot &hot, SplitKSeq &sq, int seq) {
-    const unsigned long long base = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();  // a scalar pair
-    const unsigned long long entry = base + (unsigned)seq * (unsigned)sizeof(SplitKSeq);
-    HotWords w;
-    i4 e;
-    asm volatile("s_load_dwordx16 %0, %3, 0x0\n\ts_load_dwordx16 %1, %3, 0x40\n\ts_load_dwordx4 %2, %4, 0x80\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&s"(w.lo), "=&s"(w.hi), "=&s"(e)
-                 : "s"(base), "s"(entry)
-                 : "memory");
-    hot = __builtin_bit_cast(SplitKHot, w);
-    sq = __builtin_bit_cast(SplitKSeq, e);
-}
-// ... and for a combine pass, whose first request is the gate's, where the rows go and their gate beside them.
 struct SplitKOut {
     const _Float16 *gate;
     _Float16 *out;
@@ -1001,8 +955,8 @@ struct SplitKOut {
 };
 static_assert(offsetof(SplitKArgs, gate) == 0x480 && offsetof(SplitKArgs, o_tok_stride) == 0x480 + offsetof(SplitKOut, o_tok_stride) &&
                   offsetof(SplitKArgs, out) == 0x480 + offsetof(SplitKOut, out) && sizeof(SplitKOut) == 48,
-              "load_combine's offsets");
-__device__ __forceinline__ void load_combine(SplitKHot &hot, SplitKSeq &sq, SplitKOut &out, int seq) {
+              "load_args' offsets");
+__device__ __forceinline__ void load_args(SplitKHot &hot, SplitKSeq &sq, SplitKOut &out, int seq) {
     typedef int i8v __attribute__((ext_vector_type(8)));
     struct OutWords {
         i8v lo;
@@ -1028,7 +982,7 @@ __device__ __forceinline__ seq_entries seq_table() {
     return (seq_entries)((__attribute__((address_space(4))) const char *)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(SplitKArgs, seq));
 }
 static_assert(kMaxSeqPerLaunch == 64 && offsetof(SplitKSeq, first_split) == 12, "a lane per sequence");
-static_assert(offsetof(SplitKArgs, hot) == 0 && offsetof(SplitKArgs, seq) == 0x80, "load_hot's offsets");
+static_assert(offsetof(SplitKArgs, hot) == 0 && offsetof(SplitKArgs, seq) == 0x80, "load_args' offsets");
 
 // STREAM: the launch reads every K/V byte once (see kStreamed); 2: and its V operands are paired (see v_tile_dim).
 // A row's 32 selection bytes of one key block, as 8 words in two loads (the row stride is a multiple of 4 bytes, which is
@@ -1060,7 +1014,8 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     int seq = blockIdx.z;
     SplitKHot a;
     SplitKSeq sq;
-    load_hot(a, sq, seq);
+    SplitKOut out;
+    load_args(a, sq, out, seq);
     int split = blockIdx.x, tile = blockIdx.y;
     if (a.flags & kHotPackedSplits) {
         // Sequences of unlike lengths, their splits one behind the other in x: the entries of all of them in one load (those
@@ -1473,6 +1428,24 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
         }
     }
 
+    // A launch of one split ends in the output rows: the gate's values of this thread's items, all asked for ahead of the staging and its
+    // barrier.  (Each asked for where it was stored, the items waited for memory one behind the other: a layer's three launches over 99 keys,
+    // 2 rows of 16/2 heads of 256, 15.3 us then and 13.9 now; 4 rows over 200 keys 17.1 / 15.7, 20 rows of a prompt 17.4 / 15.9.)
+    const int n_valid = ti.tile_rows * a.gh;
+    constexpr int D4 = D / 4, ITEMS = NT * D4 / (WAVES * 64), ROUND = WAVES * 64 / D4;
+    const bool last = a.n_splits_max == 1;
+    h4 gate[ITEMS];
+    if (last && out.gate) {
+        const global_halves rows = (global_halves)(out.gate + seq * out.g_seq_stride + ti.t0 * out.g_tok_stride + (long long)(ti.kvh * a.group + ti.hsub * a.gh) * D);
+        const int d = threadIdx.x % D4 * 4;
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (i * ROUND >= n_valid) break;
+            const int n = min(i * ROUND + (int)threadIdx.x / D4, n_valid - 1), tl = (n * a.gh_inv) >> 16;
+            gate[i] = *(const __attribute__((address_space(1))) h4_unaligned *)(rows + (tl * out.g_tok_stride + (n - tl * a.gh) * D + d));
+        }
+    }
+
     // Stage this wave's state in LDS.
     float l = st.l;
     l = (NT == 32) ? sum_across_halves(l) : sum_across_quarters(l);
@@ -1498,12 +1471,11 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     __syncthreads();
 
     // Merge the waves' states; every thread takes (row, 4 dims) items.
-    const int n_valid = ti.tile_rows * a.gh;
-    constexpr int D4 = D / 4;
     const size_t pbase = (((size_t)sq.first_split + split) * a.n_tiles + tile) * NT;
-    for (int item = threadIdx.x; item < n_valid * D4; item += WAVES * 64) {
-        const int n = item / D4;
-        const int d = (item - n * D4) * 4;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int n = i * ROUND + threadIdx.x / D4, d = threadIdx.x % D4 * 4;
+        if (n >= n_valid) break;
         float mw[WAVES];
         float ms = kNegBig;
 #pragma unroll
@@ -1519,10 +1491,10 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
             lsum += f * lds[w * REGION + NT * ROW + 2 * n + 1];
             acc += f * *reinterpret_cast<const f4 *>(lds + w * REGION + n * ROW + d);
         }
-        if (a.n_splits_max == 1) {
-            const int tl = n / a.gh;
+        if (last) {
+            const int tl = (n * a.gh_inv) >> 16;
             const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
-            store_out4(args, seq, ti.t0 + tl, hh, d, D, acc, lsum > 0.0f ? 1.0f / lsum : 0.0f, (a.flags & kHotAligned) != 0);
+            store_out4_gated(out, seq, ti.t0 + tl, hh, d, D, acc, lsum > 0.0f ? 1.0f / lsum : 0.0f, (a.flags & kHotAligned) != 0, gate[i]);
         } else {
             *reinterpret_cast<f4 *>(a.part_o + (pbase + n) * D + d) = acc;
             if (d == 0) {
@@ -1557,7 +1529,7 @@ __device__ __forceinline__ int splits_of(const TileInfo &ti, int split_len) {
 }
 
 template <int D, int NT>
-__global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] const SplitKArgs args) {  // (load_combine reads them)
+__global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] const SplitKArgs args) {  // (load_args reads them)
     constexpr int DCH = D / 64;
     __shared__ float sm[4][68];
     const int n = blockIdx.x / DCH, dchunk = blockIdx.x - n * DCH;
@@ -1565,7 +1537,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] cons
     SplitKHot a;
     SplitKSeq sq;
     SplitKOut out;
-    load_combine(a, sq, out, seq);
+    load_args(a, sq, out, seq);
     const TileInfo ti = tile_info(a, sq, tile);
     if (n >= ti.tile_rows * a.gh) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1581,7 +1553,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] cons
     const int tl = (n * a.gh_inv) >> 16;
     const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
     const bool aligned = (a.flags & kHotAligned) != 0;
-    const h4 gate4 = load_gate4(out, seq, ti.t0 + tl, hh, d, D, aligned);
+    const h4 gate4 = load_gate4(out, seq, ti.t0 + tl, hh, d, D);
     const int s0 = wave * 4 + (lane >> 4);
     f4 acc = (f4)0.0f;
     float l = 0.0f;
@@ -1653,14 +1625,14 @@ __global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] cons
 constexpr int kCombineRowsSplits = 16;
 
 template <int D, int NT>
-__global__ __launch_bounds__(256) void attn_combine_rows_kernel([[maybe_unused]] const SplitKArgs args) {  // (load_combine reads them)
+__global__ __launch_bounds__(256) void attn_combine_rows_kernel([[maybe_unused]] const SplitKArgs args) {  // (load_args reads them)
     constexpr int D4 = D / 4, ROWS = 4;
     static_assert(ROWS * D4 <= 256, "an item a thread");
     const int tile = blockIdx.y, seq = blockIdx.z;
     SplitKHot a;
     SplitKSeq sq;
     SplitKOut out;
-    load_combine(a, sq, out, seq);
+    load_args(a, sq, out, seq);
     const TileInfo ti = tile_info(a, sq, tile);
     const int n = blockIdx.x * ROWS + (int)threadIdx.x / D4, d = ((int)threadIdx.x % D4) * 4;
     if ((int)threadIdx.x >= ROWS * D4 || n >= ti.tile_rows * a.gh) return;
@@ -1672,7 +1644,7 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel([[maybe_unused]]
     const int tl = (n * a.gh_inv) >> 16;
     const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
     const bool aligned = (a.flags & kHotAligned) != 0;
-    const h4 gate4 = load_gate4(out, seq, ti.t0 + tl, hh, d, D, aligned);
+    const h4 gate4 = load_gate4(out, seq, ti.t0 + tl, hh, d, D);
     float mg = kNegBig, l = 0.0f;
     f4 acc = (f4)0.0f;
     auto turn = [&](auto splits, int first) {
