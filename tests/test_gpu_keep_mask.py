@@ -388,6 +388,47 @@ def test_prefill_chunk_over_index_lists_deep_in_a_long_context(gpu_ctx, bits, sp
         _check(by_list[t:t + 1], want, f"index lists at 128k keys, row {t}, bits {bits}, split {split_tokens}")
 
 
+# Both sides of the lines from which quantised pages are dequantised once for lists (tiles, tiles times keys, keys), by head dim and tokens of a
+# tile; and tiles in one range of keys dealt out XCD by XCD, in numbers that are no multiple of eight.  Against the mask form, which takes the pages as
+# they are, and the oracle.
+@pytest.mark.parametrize("H,KH,D,rows,T,bits", [
+    (16, 2, 256, 60, 6400, 8), (16, 2, 256, 61, 6400, 8), (16, 2, 256, 64, 6143, 4), (24, 2, 256, 33, 6401, 4),
+    (16, 2, 128, 124, 6400, 8), (16, 2, 128, 125, 6400, 4), (16, 4, 64, 128, 39968, 8), (16, 4, 64, 128, 40001, 8), (16, 4, 64, 121, 40000, 4),
+    (16, 2, 256, 519, 1300, 16), (8, 8, 128, 1060, 2100, 16), (32, 8, 128, 250, 700, 8)])
+def test_prefill_index_lists_on_both_sides_of_the_routes(gpu_ctx, H, KH, D, rows, T, bits):
+    import torch
+    from tinytitan_amd.engine import PrefillAttention, PrefillAttentionParams
+    start, r = T - rows, np.random.default_rng(H * D + T + bits)
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    q, gate = (r.standard_normal((rows, H * D)).astype(np.float16) for _ in range(2))
+    index_stride, cells = 2052, min(512, start // 4)
+    pick = np.argsort(r.random((rows, start // 4)), axis=1)[:, :cells]  # (in no order)
+    indices = np.zeros((rows, index_stride), np.uint32)
+    indices[:, :4 * cells] = (pick[:, :, None] * 4 + np.arange(4)).reshape(rows, -1)
+    indices[:, 4 * cells] = start + np.arange(rows)  # its own key
+    counts = np.full(rows, 4 * cells + 1, np.uint32)
+    stride = (T + 3) & ~3
+    keep = np.zeros((rows, stride), np.uint8)
+    np.put_along_axis(keep, indices[:, :4 * cells + 1].astype(np.int64), 1, axis=1)
+    kv = _cache(gpu_ctx, bits, KH, D, T)
+    _append(gpu_ctx, kv, 0, 0, 0, k, v)
+    scale = float(D) ** -0.5
+    qd, gd, keep_d, idx_d, cnt_d = _dev(q), _dev(gate), _dev(keep), _dev(indices.view(np.int32)), _dev(counts.view(np.int32))
+    by_mask, by_list = (torch.full(qd.shape, float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    att, params = PrefillAttention(gpu_ctx), PrefillAttentionParams(start, rows, T, H, scale, H * D, H * D, H * D)
+    att.encode_causal(kv, 0, 0, qd, by_mask, params, gate=gd, keep_mask=keep_d, keep_stride=stride)
+    att.encode_causal(kv, 0, 0, qd, by_list, params, gate=gd, keep_indices=idx_d, keep_index_stride=index_stride, keep_counts=cnt_d)
+    gpu_ctx.synchronize()
+    kv.close()
+    by_mask, by_list = by_mask.float().cpu().numpy(), by_list.float().cpu().numpy()
+    assert np.isfinite(by_list).all() and np.abs(by_list - by_mask).max() <= 2e-3  # (as the deep lists above)
+    ks, vs = (k, v) if bits == 16 else (_dequantised(k, bits), _dequantised(v, bits))
+    for t in (0, 31, rows // 2, rows - 1):
+        want = _oracle_rows_kept(q[t:t + 1], ks, vs, start + t, keep[t:t + 1, :T], H, KH, D, scale, gate=gate[t:t + 1])
+        _check(by_list[t:t + 1], want, f"index lists, {rows} rows behind {start} keys, row {t}, bits {bits}")
+
+
 def test_prefill_chunk_over_index_lists_goes_in_pieces_of_rows_when_its_plan_is_large(gpu_ctx):
     # One head per KV head: a tile is 32 tokens, and behind 262k keys a tile's plan has room for all 8,192 key blocks
     # times 33 words -- 124 tiles fill the 128 MiB a piece may take, so 4,100 rows go as two pieces.  Random lists of

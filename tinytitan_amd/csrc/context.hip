@@ -1077,13 +1077,20 @@ int tt_hip_attn_prefill_keep_indices(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, 
     const PageSource *pages = nullptr;
     // Quantised pages: a tile widens every block it walks, and blocks only, not groups of keys.  Where the tiles together walk
     // the context several times over and there are enough of them to matter, the visible blocks are dequantised once per
-    // call instead, as for a dense chunk, and the fp16 kernels walk those (8 bits, 16/2 heads of 256, rows with a selection
-    // each / all with one: 128 rows behind 32k keys 142.1 -> 92.4 us / 84.9 -> 63.0, 256 behind 100k 391.6 -> 234.3 / 147.4 ->
-    // 122.9, 512 behind 16k 260.6 -> 198.2; walked about once, 128 rows behind 250k, 268.4 against 323.7 the other way, and
-    // behind 4,000 keys 54.6 against 56.4: another launch).
+    // call instead, as for a dense chunk, and the fp16 kernels walk those.  us a sparse layer's step, pages as they are / dequantised, 8 bits
+    // (over 4 bits, which take longer to widen, the second way gains more), rows with a selection of 2,051 keys each / all with one:
+    //   heads of 256 from 32 tiles on: 16/2, 64 rows behind 12k keys 88 / 81, 86 / 75, 128 behind 60k 220 / 137, 148 / 121, 256 behind 150k
+    //     479 / 325, 269 / 244; 24/2, 100 behind 60k 259 / 151, 198 / 131; walked 1.3 times, 128 behind 200k, 294 / 281, 226 / 240: left alone
+    //   heads of 128, tiles of four tokens or fewer: 16/2, 128 rows behind 30k 129 / 96, 106 / 82; of more, whose selections touch most blocks
+    //     anyway: 32/8, 100 rows behind 60k (walked 3.6 times) 251 / 270, 165 / 194, behind 12k (17 times) 132 / 124, 125 / 117
+    //   heads of 64, whose tiles are the cheapest, over long contexts or many tiles: 16/4, 128 rows behind 12k 80 / 85, 79 / 85, behind
+    //     60k 150 / 119, 106 / 95, 400 behind 100k 406 / 237, 219 / 168; 64/8, 80 rows behind 30k 162 / 111, 128 / 95.
     const long long tok_tiles = (q_len + tt - 1) / tt, tiles = tok_tiles * (group / gh) * kv->n_kv_heads;
     const long long walked = tok_tiles * (entries < kv_valid ? entries : kv_valid);
-    if (kv->bits != 16 && !kv->ring && tiles * kv->head_dim >= 64 * 256 && kv_valid >= 6144 && walked >= 5ll * kv_valid) {
+    const bool worth = kv->head_dim == 256 ? tiles >= 32 && walked >= 3ll * kv_valid
+                       : kv->head_dim == 128 ? (tiles >= 128 && walked >= 5ll * kv_valid) || (tt <= 4 && tiles >= 64 && walked >= 3ll * kv_valid)
+                                             : (tiles >= 256 && walked >= 5ll * kv_valid) || (tiles * kv_valid >= 64 * 40000ll && walked >= 3ll * kv_valid);
+    if (kv->bits != 16 && !kv->ring && kv_valid >= 6144 && worth) {
         const int n_blocks = (kv_valid + 31) / 32;
         const size_t page = (size_t)n_blocks * 32 * kv->head_dim;
         if (ensure_stage(ctx, page * kv->n_kv_heads) == TT_HIP_OK) {  // (else, as inside a capture: the pages as they are)
