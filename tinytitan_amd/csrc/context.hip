@@ -454,8 +454,10 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             plan.n_splits_max = (max_keys + plan.split_len - 1) / plan.split_len;
             plan.workgroups = (long long)plan.n_splits_max * plan.n_tiles * n;
         }
-        // A chunk's token tiles over several key ranges: workgroups that share an XCD share the K/V blocks of a range.
-        plan.xcd_grid = ctx->xcd_grid && chunk_splits <= 1 && plan.tok_tiles > 1 && plan.n_splits_max > 1 && !ragged;
+        // A chunk's token tiles over several key ranges: workgroups that share an XCD share the K/V blocks of a range.  Over index lists also with
+        // one range: a KV head's tiles, one behind the other on the XCDs, were in all of their L2s (32/8 heads of 128, 256 rows behind 100k keys
+        // 644 -> 418 us a sparse layer's step, behind 60k 400 -> 328; 16/2 of 256, 500 rows 418 -> 301 and 291 -> 252).
+        plan.xcd_grid = ctx->xcd_grid && chunk_splits <= 1 && plan.tok_tiles > 1 && (plan.n_splits_max > 1 || lists) && !ragged;
         // Pages that the launch reads once -- one tile per KV head, as in a decode step or a verify pass of a few
         // rows -- are loaded non-temporal once there are enough of them that they would not survive in the
         // 256 MiB memory-side cache until the same layer's next step anyway (16 MiB a launch: sixteen layers of it).
