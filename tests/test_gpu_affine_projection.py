@@ -143,6 +143,13 @@ def test_tiles_of_every_form_at_their_edges(gpu_ctx, bits, m, n, tokens, offset)
     _case(gpu_ctx, bits, m, n, tokens, 2000 + m + n + tokens, x_stride=n + 8, y_stride=m + 3, weights_offset=offset)
 
 
+# 8 bits, two places in LDS: wavefronts of one span, of an odd last one, of none, in the three forms that have them (spans of two groups, of one).
+@pytest.mark.parametrize("m,tokens", [(33, 9), (2047, 40), (2040, 121)])
+@pytest.mark.parametrize("groups", [1, 9, 17, 65])
+def test_spans_on_their_way_beside_the_arithmetic(gpu_ctx, m, tokens, groups):
+    _case(gpu_ctx, 8, m, 64 * groups, tokens, 31 * m + groups)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("groups", [2, 6, 14, 16, 18, 30, 34, 1, 15, 20])  # by pairs: two groups a wavefront, four with an even count; not by pairs
 @pytest.mark.parametrize("shift", [0, 1, 2])  # scales and biases 2 and 4 bytes off a multiple of 8

@@ -126,17 +126,17 @@ typedef unsigned u2v __attribute__((ext_vector_type(2)));
 // The rest is bytes per CU, 16 MT x 8 KiB of x + 16 NR x 2.25 KiB of levels, at 35-40 KB/us.  us a launch, before (tiles of
 // 32 x 32, x through registers and private patches of LDS) -> now:
 //   2048 x 4096, 4 bits:   5 tokens 6.2 -> 4.7, 16: 9.7 -> 4.8, 32: 9.8 -> 5.0, 64: 9.9 -> 7.0, 128: 10.1 -> 8.7,
-//                          256: 18.1 -> 14.7, 512: 29.5 -> 25.9
-//   2048 x 4096, 8 bits:   32: 10.8 -> 5.9, 128: 10.9 -> 9.4, 512: 33.0 -> 27.5
+//                          256: 18.1 -> 14.7, 512: 29.5 -> 26.1
+//   2048 x 4096, 8 bits:   32: 10.8 -> 5.3, 128: 10.9 -> 9.3, 512: 33.0 -> 27.7
 //   2048 x 6144, 4 bits:   16: 13.7 -> 6.3, 128: 14.6 -> 11.0;  512 x 2048, 4 bits: 5: 4.8 -> 3.5, 128: 7.2 -> 3.8
 // ---------------------------------------------------------------------------
 constexpr int kTileWaves = 8;  // wavefronts that share a row's groups
 // A wavefront's part of LDS: x [token tile][group][16 tokens][128 B], then levels [16 NR rows][SPAN groups].
 constexpr int tile_x_bytes(int mt, int span) { return mt * span * 16 * 2 * kProjGroup; }
 constexpr int tile_w_bytes(int bits, bool aligned, int nr, int span) { return aligned ? nr * 16 * span * 8 * bits : 0; }
-constexpr int tile_lds_bytes(int bits, bool aligned, int mt, int nr, int span) {
+constexpr int tile_lds_bytes(int bits, bool aligned, int mt, int nr, int span, int ring) {
     const int sums = kTileWaves * 16 * mt * (16 * nr + 4) * 4;  // the partial tiles take the rows' place
-    const int staged = kTileWaves * (tile_x_bytes(mt, span) + tile_w_bytes(bits, aligned, nr, span));
+    const int staged = kTileWaves * ring * (tile_x_bytes(mt, span) + tile_w_bytes(bits, aligned, nr, span));
     return sums > staged ? sums : staged;
 }
 
@@ -159,8 +159,38 @@ __device__ __forceinline__ void transpose_quarters(unsigned (&v)[4]) {
     swap16(v[2], v[3]);
 }
 
-template <int BITS, bool ALIGNED, int MT, int NR, int SPAN>
+// N copies of 16 bytes a lane, global -> LDS, the i-th to lds_addr + 1024 i + 16 lane.  (An instruction's offset counts for both places, so the
+// i-th source comes 1024 i below itself.)  In assembly: the compiler, seeing a copy into LDS, guards every later LDS read with a wait for
+// all of them.  m0 is the compiler's (naming it as a clobber is not honoured): saved and put back.
+template <int N>
+__device__ __forceinline__ void copies_to_lds(const char *const (&src)[N], unsigned lds_addr) {
+    static_assert(N >= 2 && N <= 4, "two to four copies");
+    lds_addr = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
+    unsigned saved_m0;
+    if constexpr (N == 2)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
+                     "s_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "s"(lds_addr), "v"(src[0]), "v"(src[1])
+                     : "memory");
+    else if constexpr (N == 3)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
+                     "global_load_lds_dwordx4 %4, off offset:2048\n\ts_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "s"(lds_addr), "v"(src[0]), "v"(src[1]), "v"(src[2])
+                     : "memory");
+    else
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
+                     "global_load_lds_dwordx4 %4, off offset:2048\n\tglobal_load_lds_dwordx4 %5, off offset:3072\n\ts_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "s"(lds_addr), "v"(src[0]), "v"(src[1]), "v"(src[2]), "v"(src[3])
+                     : "memory");
+}
+
+// RING = 2: a wavefront's next span is on its way into a second place while this one is worked on.
+template <int BITS, bool ALIGNED, int MT, int NR, int SPAN, int RING>
 __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const ProjArgs a) {
+    static_assert(RING == 1 || ALIGNED, "levels that come through registers are waited for where they are asked for");
     constexpr int kTokens = 16 * MT, kRows = 16 * NR, kPitch = kRows + 4;
     constexpr int kXBytes = tile_x_bytes(MT, SPAN), kWaveBytes = kXBytes + tile_w_bytes(BITS, ALIGNED, NR, SPAN);
     constexpr int kRowPitch = SPAN * 8 * BITS, kRowPieces = kRowPitch / 16, kCopyRows = 64 / kRowPieces;  // of the levels in LDS
@@ -189,7 +219,8 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
 #pragma unroll
     for (int c = 0; c < 2 * MT; ++c)
         x_src[c] = a.x + (long long)min(token0 + 8 * c + (lane >> 3), a.tokens - 1) * a.x_stride + 8 * ((lane & 7) ^ (lane >> 3));
-    unsigned char *const x_lds = tile_lds + wave * kWaveBytes, *const w_lds = x_lds + kXBytes;
+    unsigned char *const wave_lds = tile_lds + wave * (RING * kWaveBytes);
+    const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)tile_lds, wave_lds_at = lds_base + wave * (RING * kWaveBytes);
     const uint8_t *w_src[NR];
     size_t p_at[NR];
 #pragma unroll
@@ -217,51 +248,107 @@ __global__ __launch_bounds__(kTileWaves * 64) void affine_tile_kernel(const Proj
     const h8 to_levels = {0x1p15f16, 0x1p15f16, 0x1p11f16, 0x1p11f16, 0x1p15f16, 0x1p15f16, 0x1p11f16, 0x1p11f16};
     constexpr float kBiasUnit = BITS == 4 ? 0x1p-9f : 1.0f, kSumUnit = BITS == 4 ? 0x1p9f : 1.0f;
 
+    // Tiles of 32 x 32 and two places: in assembly (4 bits, 2048 x 4096, 400 tokens 27.3 -> 25.8 us: not in front of every LDS read of the
+    // span a wait).  The others, where that wait costs nothing, by the builtin, which takes fewer instructions (16 tokens 5.10 against 5.18).
+    constexpr bool kAssembly = RING == 2 || (MT == 2 && NR == 2);
+    auto copies = [&](const auto &src, unsigned to) {  // the i-th to `to` + 1024 i + 16 lane
+        constexpr int N = sizeof(src) / sizeof(src[0]);
+        if constexpr (kAssembly) {
+            const char *below[N];
+#pragma unroll
+            for (int c = 0; c < N; ++c) below[c] = src[c] - 1024 * c;
+            copies_to_lds<N>(below, to);
+        } else {
+#pragma unroll
+            for (int c = 0; c < N; ++c)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src[c],
+                                                 (__attribute__((address_space(3))) void *)(tile_lds + (to - lds_base) + 1024 * c), 16, 0, 0);
+        }
+    };
+    auto copy_span = [&](int gs, int place) {  // groups gs .. gs + SPAN - 1
+        const unsigned x_at = wave_lds_at + place * kWaveBytes;
+#pragma unroll
+        for (int gi = 0; gi < SPAN; ++gi) {
+            if (gs + gi >= g_end) break;
+            const char *src[2 * MT];
+#pragma unroll
+            for (int c = 0; c < 2 * MT; ++c) src[c] = reinterpret_cast<const char *>(x_src[c] + kProjGroup * (gs + gi));
+            copies(src, x_at + gi * (2048 * MT));
+        }
+        if constexpr (ALIGNED) {
+            constexpr int kCopies = kRows / kCopyRows, kRun = kCopies < 4 ? kCopies : 4;
+#pragma unroll
+            for (int c0 = 0; c0 < kCopies; c0 += kRun) {
+                const char *src[kRun];
+#pragma unroll
+                for (int c = 0; c < kRun; ++c) {
+                    const int local = kCopyRows * (c0 + c) + lane / kRowPieces, row = min(row0 + local, a.rows - 1);
+                    const unsigned at = min((unsigned)gs * (8 * BITS) + 16 * ((lane % kRowPieces) ^ (local & kSwizzle)), (unsigned)row_bytes - 16);
+                    src[c] = reinterpret_cast<const char *>(a.weights + (size_t)row * row_bytes + at);
+                }
+                copies(src, x_at + kXBytes + 1024 * c0);
+            }
+        }
+    };
+    unsigned scales[NR][2], biases[NR][2], next_scales[NR][2], next_biases[NR][2];
+    auto ask_params = [&](unsigned (&sc)[NR][2], unsigned (&bi)[NR][2], int g0) {  // of groups g0 .. g0 + 3
+#pragma unroll
+        for (int nr = 0; nr < NR; ++nr) {
+            next_params(sc[nr], a.scales + p_at[nr], g0);
+            next_params(bi[nr], a.biases + p_at[nr], g0);
+        }
+    };
+    auto take_params = [&] {  // (touched here: waited for where they are used, they would be behind the next span's copies)
+#pragma unroll
+        for (int nr = 0; nr < NR; ++nr)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                asm volatile("" : "+v"(next_scales[nr][i]), "+v"(next_biases[nr][i]));
+                scales[nr][i] = next_scales[nr][i];
+                biases[nr][i] = next_biases[nr][i];
+            }
+    };
+    int place = 0;
+    if (RING == 2 && g_begin < g_end) {
+        ask_params(next_scales, next_biases, g_begin);
+        copy_span(g_begin, 0);
+    }
     for (int g0 = g_begin; g0 < g_end; g0 += 4) {
-        unsigned scales[NR][2], biases[NR][2];
 #pragma unroll
         for (int sub = 0; sub < 4; sub += SPAN) {
             if (g0 + sub >= g_end) break;
             const int gs = g0 + sub;
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last span's fragments have been read
-#pragma unroll
-            for (int gi = 0; gi < SPAN; ++gi) {
-                if (gs + gi >= g_end) break;
-#pragma unroll
-                for (int c = 0; c < 2 * MT; ++c)
-                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(x_src[c] + kProjGroup * (gs + gi)),
-                                                     (__attribute__((address_space(3))) void *)(x_lds + gi * (2048 * MT) + c * 1024), 16, 0, 0);
-            }
-            if constexpr (ALIGNED) {
-#pragma unroll
-                for (int c = 0; c < kRows / kCopyRows; ++c) {
-                    const int local = kCopyRows * c + lane / kRowPieces, row = min(row0 + local, a.rows - 1);
-                    const size_t at = min((size_t)gs * (8 * BITS) + 16 * ((lane % kRowPieces) ^ (local & kSwizzle)), row_bytes - 16);
-                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(a.weights + (size_t)row * row_bytes + at),
-                                                     (__attribute__((address_space(3))) void *)(w_lds + c * 1024), 16, 0, 0);
-                }
-            }
             unsigned w[NR][SPAN * BITS / 2];
-#pragma unroll
-            for (int nr = 0; nr < NR; ++nr) {
+            if constexpr (RING == 2) {
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this span is here, the last one's fragments have been read
+                if (sub == 0) take_params();
+                if (gs + SPAN < g_end) {
+                    if (sub + SPAN == 4) ask_params(next_scales, next_biases, g0 + 4);
+                    copy_span(gs + SPAN, place ^ 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last span's fragments have been read
+                copy_span(gs, 0);
+                if (sub == 0) ask_params(scales, biases, g0);
                 if constexpr (!ALIGNED) {
 #pragma unroll
-                    for (int j = 0; j < SPAN * BITS / 8; ++j) {
-                        unsigned v[4];
-                        if constexpr (BITS == 4) load_levels<4, false>(v, w_src[nr] + (size_t)min(gs + 2 * j + (kq >> 1), groups - 1) * 32 + 16 * (kq & 1));
-                        else load_levels<4, false>(v, w_src[nr] + (size_t)min(gs + j, groups - 1) * 64 + 16 * kq);
+                    for (int nr = 0; nr < NR; ++nr)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) w[nr][4 * j + i] = v[i];
-                    }
+                        for (int j = 0; j < SPAN * BITS / 8; ++j) {
+                            unsigned v[4];
+                            if constexpr (BITS == 4) load_levels<4, false>(v, w_src[nr] + (size_t)min(gs + 2 * j + (kq >> 1), groups - 1) * 32 + 16 * (kq & 1));
+                            else load_levels<4, false>(v, w_src[nr] + (size_t)min(gs + j, groups - 1) * 64 + 16 * kq);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) w[nr][4 * j + i] = v[i];
+                        }
                 }
-                if (sub == 0) {
-                    next_params(scales[nr], a.scales + p_at[nr], g0);
-                    next_params(biases[nr], a.biases + p_at[nr], g0);
-                }
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wavefront's own copies: no barrier
             }
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wavefront's own copies: no barrier
             __builtin_amdgcn_wave_barrier();
+            const unsigned char *const x_lds = wave_lds + place * kWaveBytes, *const w_lds = x_lds + kXBytes;
+            if constexpr (RING == 2) place ^= 1;
 #pragma unroll
             for (int nr = 0; nr < NR; ++nr)
 #pragma unroll
@@ -363,11 +450,16 @@ void launch_tile(tt_hip_ctx *ctx, const ProjArgs &a) {
         }
         launch_profiled(ctx, kernel, grid, dim3(kTileWaves * 64), (unsigned)lds, b);
     };
-    if (tiles(1, 1) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 1, 1, 4>, 1, 1, tile_lds_bytes(BITS, ALIGNED, 1, 1, 4));
-    else if (tiles(1, 2) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 1, 2, 4>, 1, 2, tile_lds_bytes(BITS, ALIGNED, 1, 2, 4));
-    else if (BITS == 4 && tiles(2, 2) <= ctx->n_cus) launch(affine_tile_kernel<4, ALIGNED, 2, 2, 4>, 2, 2, tile_lds_bytes(4, ALIGNED, 2, 2, 4));
-    else if (BITS == 4 || tiles(2, 2) <= ctx->n_cus) launch(affine_tile_kernel<BITS, ALIGNED, 2, 2, 2>, 2, 2, tile_lds_bytes(BITS, ALIGNED, 2, 2, 2));
-    else if constexpr (BITS == 8) launch(affine_tile_kernel<8, ALIGNED, 2, 4, 2>, 2, 4, tile_lds_bytes(8, ALIGNED, 2, 4, 2));
+    // 8 bits: two places in LDS, the next span on its way beside the arithmetic (5 / 32 / 64 / 128 tokens 5.62 / 6.15 / 9.1 / 10.2 -> 5.08 / 5.28 / 7.6 / 9.3
+    // us).  4 bits, half the bytes and twice the widening, are the arithmetic anyway: 16 / 64 / 128 tokens 5.1 / 7.25 / 9.0 in one place, 5.2 / 7.3 / 9.3 in two.
+    constexpr int kRing = ALIGNED && BITS == 8 ? 2 : 1, kSpan = kRing == 2 ? 2 : 4, kLarge = BITS == 4 ? 4 : ALIGNED ? 1 : 2;
+#define TT_TILE(mt, nr, span, ring) launch(affine_tile_kernel<BITS, ALIGNED, mt, nr, span, ring>, mt, nr, tile_lds_bytes(BITS, ALIGNED, mt, nr, span, ring))
+    if (tiles(1, 1) <= ctx->n_cus) TT_TILE(1, 1, kSpan, kRing);
+    else if (tiles(1, 2) <= ctx->n_cus) TT_TILE(1, 2, kSpan, kRing);
+    else if (tiles(2, 2) <= ctx->n_cus) TT_TILE(2, 2, kLarge, kRing);
+    else if constexpr (BITS == 4) TT_TILE(2, 2, 2, 1);
+    else TT_TILE(2, 4, 2, 1);
+#undef TT_TILE
 }
 
 // ---------------------------------------------------------------------------
@@ -537,33 +629,6 @@ constexpr int gemm_lds_bytes(int ks, bool rs, int tokens) {
 }
 static_assert(gemm_lds_bytes(1, false, kGemmTokens) <= 80 * 1024, "two workgroups to a CU");
 
-// N copies of 16 bytes a lane, global -> LDS, the i-th to lds_addr + 1024 i + 16 lane.  (An instruction's offset counts for both places, so the
-// i-th source comes 1024 i below itself.)  In assembly: the compiler, seeing a copy into LDS, guards every later LDS read with a wait for
-// all of them.  m0 is the compiler's (naming it as a clobber is not honoured): saved and put back.
-template <int N>
-__device__ __forceinline__ void copies_to_lds(const char *const (&src)[N], unsigned lds_addr) {
-    static_assert(N >= 2 && N <= 4, "two to four copies");
-    lds_addr = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
-    unsigned saved_m0;
-    if constexpr (N == 2)
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
-                     "s_mov_b32 m0, %0"
-                     : "=&s"(saved_m0)
-                     : "s"(lds_addr), "v"(src[0]), "v"(src[1])
-                     : "memory");
-    else if constexpr (N == 3)
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
-                     "global_load_lds_dwordx4 %4, off offset:2048\n\ts_mov_b32 m0, %0"
-                     : "=&s"(saved_m0)
-                     : "s"(lds_addr), "v"(src[0]), "v"(src[1]), "v"(src[2])
-                     : "memory");
-    else
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\tglobal_load_lds_dwordx4 %3, off offset:1024\n\t"
-                     "global_load_lds_dwordx4 %4, off offset:2048\n\tglobal_load_lds_dwordx4 %5, off offset:3072\n\ts_mov_b32 m0, %0"
-                     : "=&s"(saved_m0)
-                     : "s"(lds_addr), "v"(src[0]), "v"(src[1]), "v"(src[2]), "v"(src[3])
-                     : "memory");
-}
 // vmcnt(n) only: leaves the LDS and export counters alone.
 #define TT_WAIT_COPIES(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
@@ -916,22 +981,22 @@ int configure_affine_kernels(tt_hip_ctx *ctx) {
     TT_CFG((affine_gemm_kernel<4, false, 2, true>), gemm_lds_bytes(2, true, 128))
     TT_CFG((affine_gemm_kernel<8, true, 2, true>), gemm_lds_bytes(2, true, 128))
     TT_CFG((affine_gemm_kernel<8, false, 2, true>), gemm_lds_bytes(2, true, 128))
-    TT_CFG((affine_tile_kernel<4, true, 1, 1, 4>), tile_lds_bytes(4, true, 1, 1, 4))
-    TT_CFG((affine_tile_kernel<4, true, 1, 2, 4>), tile_lds_bytes(4, true, 1, 2, 4))
-    TT_CFG((affine_tile_kernel<4, true, 2, 2, 4>), tile_lds_bytes(4, true, 2, 2, 4))
-    TT_CFG((affine_tile_kernel<4, true, 2, 2, 2>), tile_lds_bytes(4, true, 2, 2, 2))
-    TT_CFG((affine_tile_kernel<4, false, 1, 1, 4>), tile_lds_bytes(4, false, 1, 1, 4))
-    TT_CFG((affine_tile_kernel<4, false, 1, 2, 4>), tile_lds_bytes(4, false, 1, 2, 4))
-    TT_CFG((affine_tile_kernel<4, false, 2, 2, 4>), tile_lds_bytes(4, false, 2, 2, 4))
-    TT_CFG((affine_tile_kernel<4, false, 2, 2, 2>), tile_lds_bytes(4, false, 2, 2, 2))
-    TT_CFG((affine_tile_kernel<8, true, 1, 1, 4>), tile_lds_bytes(8, true, 1, 1, 4))
-    TT_CFG((affine_tile_kernel<8, true, 1, 2, 4>), tile_lds_bytes(8, true, 1, 2, 4))
-    TT_CFG((affine_tile_kernel<8, true, 2, 4, 2>), tile_lds_bytes(8, true, 2, 4, 2))
-    TT_CFG((affine_tile_kernel<8, true, 2, 2, 2>), tile_lds_bytes(8, true, 2, 2, 2))
-    TT_CFG((affine_tile_kernel<8, false, 1, 1, 4>), tile_lds_bytes(8, false, 1, 1, 4))
-    TT_CFG((affine_tile_kernel<8, false, 1, 2, 4>), tile_lds_bytes(8, false, 1, 2, 4))
-    TT_CFG((affine_tile_kernel<8, false, 2, 4, 2>), tile_lds_bytes(8, false, 2, 4, 2))
-    TT_CFG((affine_tile_kernel<8, false, 2, 2, 2>), tile_lds_bytes(8, false, 2, 2, 2))
+    TT_CFG((affine_tile_kernel<4, true, 1, 1, 4, 1>), tile_lds_bytes(4, true, 1, 1, 4, 1))
+    TT_CFG((affine_tile_kernel<4, true, 1, 2, 4, 1>), tile_lds_bytes(4, true, 1, 2, 4, 1))
+    TT_CFG((affine_tile_kernel<4, true, 2, 2, 4, 1>), tile_lds_bytes(4, true, 2, 2, 4, 1))
+    TT_CFG((affine_tile_kernel<4, true, 2, 2, 2, 1>), tile_lds_bytes(4, true, 2, 2, 2, 1))
+    TT_CFG((affine_tile_kernel<4, false, 1, 1, 4, 1>), tile_lds_bytes(4, false, 1, 1, 4, 1))
+    TT_CFG((affine_tile_kernel<4, false, 1, 2, 4, 1>), tile_lds_bytes(4, false, 1, 2, 4, 1))
+    TT_CFG((affine_tile_kernel<4, false, 2, 2, 4, 1>), tile_lds_bytes(4, false, 2, 2, 4, 1))
+    TT_CFG((affine_tile_kernel<4, false, 2, 2, 2, 1>), tile_lds_bytes(4, false, 2, 2, 2, 1))
+    TT_CFG((affine_tile_kernel<8, true, 1, 1, 2, 2>), tile_lds_bytes(8, true, 1, 1, 2, 2))
+    TT_CFG((affine_tile_kernel<8, true, 1, 2, 2, 2>), tile_lds_bytes(8, true, 1, 2, 2, 2))
+    TT_CFG((affine_tile_kernel<8, true, 2, 2, 1, 2>), tile_lds_bytes(8, true, 2, 2, 1, 2))
+    TT_CFG((affine_tile_kernel<8, true, 2, 4, 2, 1>), tile_lds_bytes(8, true, 2, 4, 2, 1))
+    TT_CFG((affine_tile_kernel<8, false, 1, 1, 4, 1>), tile_lds_bytes(8, false, 1, 1, 4, 1))
+    TT_CFG((affine_tile_kernel<8, false, 1, 2, 4, 1>), tile_lds_bytes(8, false, 1, 2, 4, 1))
+    TT_CFG((affine_tile_kernel<8, false, 2, 2, 2, 1>), tile_lds_bytes(8, false, 2, 2, 2, 1))
+    TT_CFG((affine_tile_kernel<8, false, 2, 4, 2, 1>), tile_lds_bytes(8, false, 2, 4, 2, 1))
 #undef TT_CFG
     return e == hipSuccess ? TT_HIP_OK : hip_fail(ctx, e, "hipFuncSetAttribute(o_proj max dynamic LDS)");
 }
