@@ -429,6 +429,38 @@ def test_prefill_index_lists_on_both_sides_of_the_routes(gpu_ctx, H, KH, D, rows
         _check(by_list[t:t + 1], want, f"index lists, {rows} rows behind {start} keys, row {t}, bits {bits}")
 
 
+# The plan's threads share a row's list: runs that end short of, at and behind the entries a thread holds, rows that do not divide the threads, tokens of a
+# tile that do and do not divide a word's bits, and more blocks than one run of bits takes.
+@pytest.mark.parametrize("H,KH,rows", [(2, 2, 35), (3, 1, 21), (8, 1, 7), (10, 2, 13)])  # tiles of 32, 10, 4 and 6 tokens
+@pytest.mark.parametrize("index_stride,T", [(1, 300), (33, 1000), (576, 9000), (580, 40000), (1730, 20000)])
+def test_prefill_index_lists_of_any_width(gpu_ctx, H, KH, rows, index_stride, T):
+    import torch
+    from tinytitan_amd.engine import PrefillAttention, PrefillAttentionParams
+    D, start, r = 64, T - rows, np.random.default_rng(H * index_stride + T)
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    q = r.standard_normal((rows, H * D)).astype(np.float16)
+    indices = r.integers(0, T, size=(rows, index_stride), dtype=np.int64)  # (some twice, some that a row cannot see)
+    indices[:, 0] = start + np.arange(rows)
+    counts = r.integers(1, index_stride + 1, size=rows)
+    counts[rows // 2] = index_stride
+    keep = np.zeros((rows, (T + 3) & ~3), np.uint8)
+    for t in range(rows):
+        keep[t, indices[t, :counts[t]]] = 1
+    kv = _cache(gpu_ctx, 16, KH, D, T)
+    _append(gpu_ctx, kv, 0, 0, 0, k, v)
+    qd, idx_d, cnt_d = _dev(q), _dev(indices.astype(np.int32)), _dev(counts.astype(np.int32))
+    out = torch.full(qd.shape, float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    PrefillAttention(gpu_ctx).encode_causal(kv, 0, 0, qd, out, PrefillAttentionParams(start, rows, T, H, 0.125, H * D, H * D, H * D), keep_indices=idx_d,
+                                            keep_index_stride=index_stride, keep_counts=cnt_d)
+    gpu_ctx.synchronize()
+    kv.close()
+    got = out.float().cpu().numpy()
+    for t in {0, rows // 2, rows - 2, rows - 1}:
+        want = _oracle_rows_kept(q[t:t + 1], k, v, start + t, keep[t:t + 1, :T], H, KH, D, 0.125)
+        _check(got[t:t + 1], want, f"lists of {index_stride}, {rows} rows, {T} keys, row {t}")
+
+
 def test_prefill_chunk_over_index_lists_goes_in_pieces_of_rows_when_its_plan_is_large(gpu_ctx):
     # One head per KV head: a tile is 32 tokens, and behind 262k keys a tile's plan has room for all 8,192 key blocks
     # times 33 words -- 124 tiles fill the 128 MiB a piece may take, so 4,100 rows go as two pieces.  Random lists of

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void keep_rows_from_indices_kernel(uint8_t *ro
 // any order and repeat: a bit is set once.
 // GROUPS: the same with groups of four keys in the place of blocks: the ascending list of group ids, where the ranges start
 // in it, and per eight list positions and token one word, four bits a position.
-// LDS: bitmap[W], prefix[W], partial[kPlanThreads + 1], chunk[chunk_entries * tt] words, W = ceil(ceil(kv_valid / 32) / 32)
+// LDS: bitmap[W], prefix[W], partial[kPlanThreads + 1], chunk[chunk_entries * (tt | 1)] words, W = ceil(ceil(kv_valid / 32) / 32)
 // (GROUPS: ceil(ceil(kv_valid / 4) / 32), and an entry is eight positions).
 constexpr int kPlanThreads = 1024;  // sixteen wavefronts: the walks are chains of dependent scalar work that only other wavefronts hide
 constexpr int kPlanGroupKeys = 400000;  // keys whose groups' bitmap and prefix sums take 25 of the 64 KiB
@@ -137,48 +137,45 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
     const int ctx_blocks = (kv_valid + (1 << kShift) - 1) >> kShift, W = (ctx_blocks + 31) >> 5;
     unsigned *bitmap = plan_lds, *prefix = plan_lds + W, *partial = plan_lds + 2 * W;
     const int rows = min(tt, q_len - tile * tt);
-    // The tile's lists as one run of rows * index_stride places, every thread a run of `per` neighbouring ones (so
+    // Every row of the tile has as many threads as the others, every thread a run of `per` neighbouring entries of its row (so
     // that the lanes of a wavefront work on entries far apart, which seldom meet in one word of LDS: the entries of a
     // sorted list that 64 neighbouring lanes hold fall into a handful of words, and their atomics queue up).  A
-    // thread's first kHeld places are asked for at once, beside the rows' counts and ahead of everything else, and
-    // stay in registers for both walks over the lists: one trip to memory for a tile of the usual size.  Places
-    // beyond them are read again per walk, kBatch at a time.
-    constexpr unsigned kHeld = 16, kBatch = 8;
-    const uint32_t *lists = indices + (size_t)tile * tt * index_stride;
-    const unsigned places = (unsigned)rows * index_stride, per = (places + T - 1u) / T, mine = (unsigned)tid * per;
-    unsigned my_count = tid < rows ? min(counts[tile * tt + tid], index_stride) : 0u;
+    // thread's first kHeld entries are asked for at once, beside its row's count and ahead of everything else, and
+    // stay in registers for both walks over the lists: one trip to memory for a tile of the usual size.  Entries
+    // beyond them are read again per walk, kBatch at a time.  What a tile's workgroup spends its time on is instructions per entry and walk,
+    // sixteen wavefronts on four SIMDs: a thread that ran on from one row's list into the next had two dozen, with a place checked for
+    // every one it could hold.  128 rows of 16/2 heads with lists of 2,051 cells 11.5 -> 9.2 us, 100 rows of 32/8 17.2 -> 12.4, over 8 bits 12.2 -> 10.2.
+    constexpr unsigned kHeld = 18, kBatch = 8;  // (lists of 2,051 cells, tiles of four and of eight tokens: 9 and 17 entries a thread)
+    const unsigned row_threads = (unsigned)T / (unsigned)rows, row = min((unsigned)tid / row_threads, (unsigned)rows - 1u);  // (threads over: at the last row's end)
+    const unsigned per = (index_stride + row_threads - 1u) / row_threads, mine = ((unsigned)tid - row * row_threads) * per;
+    const uint32_t *list = indices + (size_t)(tile * tt + (int)row) * index_stride;
+    const unsigned count = min(counts[tile * tt + (int)row], index_stride), limit = (unsigned)min(kv_valid, start + tile * tt + (int)row + 1);
+    const unsigned end = min(mine + per, count);
     unsigned held[kHeld];
 #pragma unroll
-    for (unsigned j = 0; j < kHeld; ++j) held[j] = lists[min(mine + j, places - 1u)];
+    for (unsigned j = 0; j < kHeld; ++j)
+        if (j < per) held[j] = list[min(mine + j, index_stride - 1u)];  // (18 requests of 64 lanes' far apart words where 9 are wanted: 9.4 -> 11.1 us)
     for (int w = tid; w < W; w += T) bitmap[w] = 0u;
-    unsigned *row_counts = partial;  // (the scan's words: free until the bitmap is complete; tt <= 32)
-    if (tid < rows) row_counts[tid] = my_count;
     __syncthreads();
-    const unsigned row0 = min(mine, places - 1u) / index_stride;  // (the one division: a run's places are walked in order)
-    auto for_listed_keys = [&](auto &&use) {  // use(key, row): every listed key that its row can see, in list order
-        unsigned r = row0, i = mine - row0 * index_stride;  // the place in hand: entry i of the tile's row r
-        unsigned count = row_counts[min(r, (unsigned)rows - 1u)], limit = (unsigned)min(kv_valid, start + tile * tt + (int)r + 1);
+    auto for_listed_keys = [&](auto &&use) {  // use(key): every listed key of the thread's that its row can see
         auto place = [&](unsigned j, unsigned key) {
-            if (j < per && r < (unsigned)rows && i < count && key < limit) use(key, r);
-            if (++i == index_stride) {
-                i = 0u;
-                ++r;
-                count = row_counts[min(r, (unsigned)rows - 1u)];
-                limit = (unsigned)min(kv_valid, start + tile * tt + (int)r + 1);
-            }
+            if (mine + j < end && key < limit) use(key);
         };
 #pragma unroll
-        for (unsigned j = 0; j < kHeld; ++j) place(j, held[j]);
+        for (unsigned j = 0; j < kHeld; ++j) {
+            if (j >= per) break;
+            place(j, held[j]);
+        }
         for (unsigned base = kHeld; base < per; base += kBatch) {
             unsigned keys[kBatch];
 #pragma unroll
-            for (unsigned j = 0; j < kBatch; ++j) keys[j] = lists[min(mine + base + j, places - 1u)];
+            for (unsigned j = 0; j < kBatch; ++j) keys[j] = list[min(mine + base + j, index_stride - 1u)];
 #pragma unroll
             for (unsigned j = 0; j < kBatch; ++j) place(base + j, keys[j]);
         }
     };
-    for_listed_keys([&](unsigned key, unsigned) { atomicOr(&bitmap[key >> (kShift + 5)], 1u << ((key >> kShift) & 31u)); });
-    __syncthreads();  // (the scan takes the counts' words over: they are put back from my_count for the second walk)
+    for_listed_keys([&](unsigned key) { atomicOr(&bitmap[key >> (kShift + 5)], 1u << ((key >> kShift) & 31u)); });
+    __syncthreads();
     // exclusive prefix sums of the words' bit counts: a run of words per thread, a scan of the threads' runs inside
     // each wavefront by shuffles, the wavefronts' totals through LDS
     const int per_thread = (W + T - 1) / T, w_begin = tid * per_thread, w_end = min(W, w_begin + per_thread);
@@ -222,28 +219,27 @@ __global__ __launch_bounds__(kPlanThreads) void keep_plan_kernel(const uint32_t 
     // keys), then written out side by side.
     unsigned *my_bits = bits + (size_t)tile * (GROUPS ? cap >> 3 : cap) * tt;
     const int n_entries = GROUPS ? (n_touched + 7) >> 3 : n_touched;
-    unsigned *chunk = plan_lds + 2 * W + T + 1;  // chunk_entries * tt words
-    if (tid < rows) row_counts[tid] = my_count;
+    unsigned *chunk = plan_lds + 2 * W + T + 1;  // [chunk_entries][pitch]; an odd pitch: a row's entries in all banks
+    const int pitch = tt | 1;
+    const unsigned per_tt = ((1u << 19) + (unsigned)tt - 1u) / (unsigned)tt;  // i / tt == i * per_tt >> 19 for i < 16,384 and even tt <= 32
     for (int first = 0; first < n_entries; first += chunk_entries) {
         const int here = min(chunk_entries, n_entries - first);
-        __syncthreads();  // (the counts are back in their words; the previous run has been written out)
-        for (int i = tid; i < here * tt; i += T) chunk[i] = 0u;
+        __syncthreads();  // (the previous run has been written out)
+        for (int i = tid; i < here * pitch; i += T) chunk[i] = 0u;
         __syncthreads();
-        for_listed_keys([&](unsigned key, unsigned r) {
+        for_listed_keys([&](unsigned key) {
             const unsigned w = key >> (kShift + 5), bit = (key >> kShift) & 31u;
             const int rank = (int)(prefix[w] + __popc(bitmap[w] & ((1u << bit) - 1u)));
             const int entry = (GROUPS ? rank >> 3 : rank) - first;
             const unsigned at = GROUPS ? 4u * ((unsigned)rank & 7u) + (key & 3u) : key & 31u;
-            if (entry >= 0 && entry < here) atomicOr(&chunk[entry * tt + (int)r], 1u << at);
+            if (entry >= 0 && entry < here) atomicOr(&chunk[entry * pitch + (int)row], 1u << at);
         });
         __syncthreads();
-        for (int i = tid; i < here * tt; i += T) my_bits[(size_t)first * tt + i] = chunk[i];
+        for (int i = tid; i < here * tt; i += T) my_bits[(size_t)first * tt + i] = chunk[i + (int)((unsigned)i * per_tt >> 19) * (pitch - tt)];
         if (GROUPS || !any_keys) continue;
         for (int i = tid; i < here; i += T) {
             unsigned any = 0u;
-            // (each from a place of its own on: all from the first, 32 tokens' words are one bank's, and 30 rows of 8/8 heads of 128
-            // behind 48,000 keys took 177 us instead of 166)
-            for (int r = 0, at = i % tt; r < tt; ++r, at = at + 1 < tt ? at + 1 : 0) any |= chunk[i * tt + at];
+            for (int r = 0; r < tt; ++r) any |= chunk[i * pitch + r];
             my_blocks[2 * (first + i) + 1] = (int)any;
         }
     }
@@ -565,18 +561,17 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
             int *ranges = reinterpret_cast<int *>(ctx->keep_rows);
             int *blocks = ranges + list_ranges(plan.n_splits_max);
             unsigned *bits = reinterpret_cast<unsigned *>(blocks + n_blocks);
-            // LDS of the plan kernel: two words per 32 units of context and the run of bits it gathers at a time, 32 KiB
-            // of them or what the context's bitmap leaves of 64 KiB.
+            // LDS of the plan kernel: two words per 32 units of context and the run of bits it gathers at a time, what that leaves of
+            // 64 KiB: every run is another walk over the lists.
             const int words = (ctx_units + 31) / 32;
-            int chunk_words = (65536 / 4) - (2 * words + kPlanThreads + 1);
-            if (chunk_words > 8192) chunk_words = 8192;
-            const int chunk_entries = chunk_words / plan.tt;
+            const int chunk_words = (65536 / 4) - (2 * words + kPlanThreads + 1);
+            const int chunk_entries = chunk_words / (plan.tt | 1);
             if (chunk_entries < 1) return TT_HIP_ERR_CAPACITY;
             const bool by_key = !groups && launch_fetches_by_key(D, kv_bits, plan.n_tiles, (long long)plan.tt * (long long)lists->stride,
                                                                  totals[base], ctx->n_cus);
             const auto kernel = groups ? keep_plan_kernel<true> : keep_plan_kernel<false>;
             hipLaunchKernelGGL(kernel, dim3((unsigned)plan.tok_tiles), dim3(kPlanThreads),
-                               (size_t)(2 * words + kPlanThreads + 1 + chunk_entries * plan.tt) * sizeof(unsigned), ctx->stream, lists->indices,
+                               (size_t)(2 * words + kPlanThreads + 1 + chunk_entries * (plan.tt | 1)) * sizeof(unsigned), ctx->stream, lists->indices,
                                (unsigned)lists->stride, lists->counts, starts[base], rows, totals[base], plan.tt, plan.split_len / 32,
                                plan.n_splits_max, cap, chunk_entries, ranges, blocks, bits, by_key);
             e = hipGetLastError();
