@@ -199,6 +199,24 @@ def test_prefill_over_quantised_cache(gpu_ctx, bits, start, chunk):
     kv.close()
 
 
+# Chunks that the chunk kernel does not take: packed tiles where heads divide a tile's rows (with splits, and filling the chip without), tiles of one head
+# where they do not; over levels, and over fp16 pages for groups that are no multiple of four.
+@pytest.mark.parametrize("H,KH,D,start,chunk,bits", [(32, 8, 128, 600, 100, 8), (32, 8, 128, 900, 101, 4), (16, 2, 256, 0, 256, 8), (16, 4, 64, 700, 257, 4),
+                                                     (36, 4, 128, 300, 150, 8), (10, 2, 128, 40, 420, 16), (6, 2, 64, 900, 700, 8), (24, 2, 256, 100, 170, 4)])
+def test_chunks_in_packed_tiles_and_in_tiles_of_one_head(gpu_ctx, H, KH, D, start, chunk, bits):
+    kv_valid, scale = start + chunk, float(D) ** -0.5
+    k, v = _rows(kv_valid, KH, D, seed=H + start + bits, spread=False)
+    r = np.random.default_rng(H + chunk)
+    q, g = (r.standard_normal((chunk, H * D)).astype(np.float16) for _ in range(2))
+    kv = _cache(gpu_ctx, bits, KH, D, kv_valid)
+    _append(gpu_ctx, kv, 0, 0, 0, k, v)
+    got = _prefill(gpu_ctx, kv, q, start, chunk, kv_valid, H, scale, gate=g)
+    kv.close()
+    kq, vq = ((x.astype(np.float32) if bits == 16 else _dequantised(x, bits)).reshape(kv_valid, -1) for x in (k, v))
+    want = oracle.attention_batch(q.astype(np.float32), kq, vq, chunk, start, H, KH, D, scale, threads=4).reshape(chunk, -1)
+    _check(got, want / (1 + np.exp(-g.astype(np.float64))), f"{H}/{KH} heads of {D}, {chunk} rows at {start} over {bits} bits")
+
+
 @pytest.mark.parametrize("bits", [8, 4])
 def test_verify_rows_equal_decode_steps_and_batch(gpu_ctx, bits):
     import torch
@@ -314,6 +332,41 @@ def test_fused_epilogue_writes_the_same_rows(gpu_ctx, bits, H, KH, D, rot, n_seq
             assert not front_k.any() and not front_v.any()
     for cache in (plain, quant, want):
         cache.close()
+
+
+def test_a_chunk_captured_before_there_is_scratch_for_its_splits(gpu_ctx):
+    # the packed tiles' partial results would have to grow while capturing: tiles of one head, which leave none
+    import torch
+    from tinytitan_amd.engine import HIPContext, PrefillAttention, PrefillAttentionParams
+    H, KH, D, T, chunk = 32, 8, 128, 4100, 100
+    ctx = HIPContext(gpu_ctx.device)
+    k, v = _rows(T, KH, D, seed=78, spread=False)
+    kv = _cache(ctx, 8, KH, D, T)
+    _append(ctx, kv, 0, 0, 0, k, v)
+    q = _dev(np.random.default_rng(8).standard_normal((chunk, H * D)).astype(np.float16))
+    out = torch.zeros_like(q)
+    params, pre = PrefillAttentionParams(T - chunk, chunk, T, H, 0.0883883, H * D, H * D, H * D), PrefillAttention(ctx)
+    torch.cuda.synchronize()
+    ctx.graph_begin()
+    pre.encode_causal(kv, 0, 0, q, out, params)
+    graph = ctx.graph_end()
+    replays = []
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.launch()
+        ctx.synchronize()
+        replays.append(out.float().cpu().numpy())
+    graph.close()
+    out.zero_()
+    torch.cuda.synchronize()
+    pre.encode_causal(kv, 0, 0, q, out, params)
+    ctx.synchronize()
+    eager = out.float().cpu().numpy()
+    kv.close()
+    assert np.isfinite(eager).all() and np.abs(eager).max() > 0
+    for got in replays:
+        assert np.abs(got - eager).max() <= 2e-3
 
 
 def test_graph_replay_over_a_quantised_cache(gpu_ctx):

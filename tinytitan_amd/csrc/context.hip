@@ -1277,14 +1277,24 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
                              (long long)q_stride, gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride);
     }
     // What the chunk kernel does not serve (head groups that are no multiple of 4, unaligned rows, quantised pages
-    // that are not staged, a non-positive scale): the split-K kernel.  Tiles of 32 rows of ONE head, each walking
-    // all its keys, where they are plentiful and the context is short or they are very plentiful; otherwise --
-    // a few rows deep in a context -- GQA-packed tiles over key ranges, like a verify pass (one row at 32k keys over
-    // 8 bits took 460 us as 16 one-head tiles walking 32k keys each).
+    // that are not staged, a non-positive scale): the split-K kernel over GQA-packed tiles, like a verify pass -- or, where heads that do
+    // not divide a tile's 32 rows leave some of them empty, tiles of 32 rows of ONE head, each walking all its keys, as long as they are
+    // plentiful and the context is short or they are very plentiful (one row at 32k keys over 8 bits took 460 us as 16 one-head tiles
+    // walking 32k keys each).  us a layer over 8 bits, one-head tiles / packed ones, of groups of 4 (32/8 heads of 128): 100 rows behind
+    // 7,000 keys 86.1 / 58.8, 700 behind 2,000 91.8 / 80.1; of 8 (16/2 of 256): 256 rows behind 2,000 64.2 / 52.1, 700 of a prompt 76.6 / 67.5;
+    // of 9 (36/4 of 128): 1,500 rows behind 3,000 256 / 297; of 5 (40/8 of 128): 700 behind 7,000 253 / 262.
     const long long head_tiles = (long long)((q_len + 31) / 32) * n_q_heads;
-    const int kind = 2 * head_tiles >= ctx->n_cus && (kv_valid <= 8192 || head_tiles >= 2LL * ctx->n_cus) ? 1 : 0;
-    return run_attention(ctx, kv, kind, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride,
-                         gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride);
+    const bool rows_left_empty = 32 % packed_heads(n_q_heads / kv->n_kv_heads) != 0;
+    const bool plentiful = 2 * head_tiles >= ctx->n_cus && (kv_valid <= 8192 || head_tiles >= 2LL * ctx->n_cus);
+    auto in_tiles = [&](int kind) {
+        return run_attention(ctx, kv, kind, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride,
+                             gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride);
+    };
+    if (rows_left_empty && plentiful) return in_tiles(1);
+    st = in_tiles(0);
+    // (without memory for the splits' partial results, as inside a capture that would have to grow it: tiles of one head, which have none)
+    if (plentiful && (st == TT_HIP_ERR_BUSY || st == TT_HIP_ERR_OUT_OF_MEMORY)) st = in_tiles(1);
+    return st;
 }
 
 }  // extern "C"
