@@ -111,6 +111,71 @@ def test_decode_empty_sequence_and_gate(gpu_ctx):
     c.close()
 
 
+def _gate_factors(shape):
+    """Every finite fp16 gate, over and over, and its factor: the device's exp2 of the kernels' fp32 product, then numpy's division."""
+    import torch
+    gates = np.arange(65536, dtype=np.uint16).view(np.float16)
+    gates = np.resize(np.where(np.isfinite(gates), gates, np.float16(0)), shape)
+    x = torch.from_numpy(gates.astype(np.float32)).cuda()
+    e = torch.exp2(-x * torch.tensor(1.4426950408889634, dtype=torch.float32, device="cuda")).cpu().numpy()
+    return gates, np.float32(1) / (np.float32(1) + e)
+
+
+def _assert_gated(got, value, factor):
+    # (two infinities, a factor of zero times one of them: NaN on both sides)
+    with np.errstate(invalid="ignore"):
+        want = (value.astype(np.float32) * factor).astype(np.float16).astype(np.float32)
+    differ = (got != want) & ~(np.isnan(got) & np.isnan(want))
+    assert not differ.any(), f"{np.count_nonzero(differ)} of {differ.size} products"
+
+
+# A row all of whose weight is on one key gives that key's value exactly, so what is stored is fp16(value * factor), and the factor's fp32
+# bits show wherever a product lies next to a rounding boundary: with a reciprocal off in its last place some 80 of 2^20 do.
+
+@pytest.mark.parametrize("keys,split", [(1, 0), (300, 128)])
+def test_gate_factor_of_a_decode_step_is_the_divisions(gpu_ctx, keys, split):
+    import torch
+    from tinytitan_amd.engine import KVCacheManager
+    H, KH, D, n = 16, 2, 256, 64
+    gates, factor = _gate_factors((n, 1, H, D))
+    r = np.random.default_rng(41)
+    kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=n, max_context=keys, initial_capacity=keys)
+    k, v = (torch.zeros(keys, KH, D, dtype=torch.float16, device="cuda") for _ in range(2))
+    k[:-1] = -300.0  # the last key alone has any weight
+    results = []
+    for turn in range(4):
+        value = r.uniform(1, 2, (n, KH, D)).astype(np.float16)
+        if turn == 0:
+            value[:, 0, ::7] = np.inf
+        for slot in range(n):
+            v[-1] = torch.from_numpy(value[slot]).cuda()
+            torch.cuda.synchronize()
+            kv.append(0, slot, 0, k, v)
+            gpu_ctx.synchronize()
+        gpu_ctx.set_split_tokens(split)
+        got = _decode(gpu_ctx, kv, np.ones((n, 1, H, D), np.float16), [keys] * n, H, 1.0, gate=gates)[:, 0]
+        gpu_ctx.set_split_tokens(0)
+        results.append((got, np.repeat(value, H // KH, 1)))
+    kv.close()
+    for got, value in results:
+        _assert_gated(got, value, factor[:, 0])
+
+
+@pytest.mark.parametrize("D", [256, 128, 64])
+def test_gate_factor_of_a_chunk_is_the_divisions(gpu_ctx, D):
+    # Signs along every key that only its own row's query shares: the products of the others are some 500 below.
+    H, KH, rows = 16, 2, 1030
+    gates, factor = _gate_factors((rows, H * D))
+    r = np.random.default_rng(43)
+    k = (32 * r.choice([-1.0, 1.0], (rows, 1, D))).repeat(KH, 1).astype(np.float16)
+    q = (32 * np.sign(k[:, :1]).repeat(H, 1)).reshape(rows, H * D).astype(np.float16)
+    v = r.uniform(1, 2, (rows, KH, D)).astype(np.float16)
+    c = Cache(gpu_ctx, k, v)
+    got = _prefill(gpu_ctx, c.kv, q, 0, rows, rows, H, 1.0, gate=gates)
+    c.close()
+    _assert_gated(got.reshape(rows, H, D), np.repeat(v, H // KH, 1), factor.reshape(rows, H, D))
+
+
 # ---- batched decode == per-row decode ----------------------------------------------------------
 
 def test_batch_equals_per_row(gpu_ctx):
