@@ -514,7 +514,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
                 const float lt = *lsum_mine;
                 const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
                 // A tile's gate values are asked for one tile ahead, by every lane (a row past the chunk's end reads row 0's): under a
-                // condition of its own each load was waited for where it stood.  (With the gate's reciprocal: 16/2 heads of 256, position 0,
+                // condition of its own each load was waited for where it stood.  (Together with a cheaper division: 16/2 heads of 256, position 0,
                 // 4,096 rows 155 -> 149 us, 2,048 69 -> 64.5, 1,024 40 -> 36.5; 32/8 of 128, 4,096 rows 179 -> 172.)
                 const bool gated = a.gate != nullptr;
                 const _Float16 *const gate_row = a.gate + (long long)(valid ? tile * 32 + row_here : 0) * a.g_stride + (long long)head * D + 4 * g;

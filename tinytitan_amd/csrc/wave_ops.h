@@ -10,11 +10,14 @@ namespace tt {
 // The output gate's factor, 1 / (1 + e^-x), rounded as the fp32 division rounds it: the hardware's reciprocal (one unit in the last
 // place) and a Newton step, over a quarter of the denominator (exact) so that no reciprocal is subnormal; an infinite denominator
 // is the fixup's.  Every fp16 gate gives the division's bits (of the factors below 2^-126, which round any fp16 value to zero, all
-// but their last place): the bare reciprocal was off in 3,597 of them.  us a pass of 4,096 rows of 16/2 heads of 256 / of 777 rows of
-// 32/8 of 128: reciprocal 242.0 / 96.7, this 245.0 / 97.1, a full division 245.8 / 97.7 (a dozen instructions for every element of an output, 128 a lane in the chunk kernel).
+// but their last place): the bare reciprocal was off in 3,597 of them.  A pass of 4,096 rows of
+// 16/2 heads of 256 (245 us) and one of 777 rows of 32/8 of 128 (97.4 us) take 0.8 and 0.3 % more than with the bare reciprocal, with a full division
+// (a dozen instructions for every element of an output, 128 a lane in the chunk kernel) 1.6 and 1.0 %.
 __device__ __forceinline__ float sigmoid(float x) {
-    const float quarter = __builtin_fmaf(0.25f, __expf(-x), 0.25f), r = __builtin_amdgcn_rcpf(quarter);
-    return 0.25f * __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-quarter, r, 1.0f), r, r), quarter, 1.0f);
+    float scale = 0.25f;
+    asm("" : "+s"(scale));  // (kept in a vector register it was the one too many in the chunk kernel of heads of 256, which then spilled)
+    const float quarter = __builtin_fmaf(scale, __expf(-x), scale), r = __builtin_amdgcn_rcpf(quarter);
+    return scale * __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-quarter, r, 1.0f), r, r), quarter, 1.0f);
 }
 
 // v_permlane32_swap(x, x): first result = lanes 0-31 of x in both halves, second = lanes 32-63.
