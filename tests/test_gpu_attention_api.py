@@ -675,6 +675,37 @@ def test_combine_at_the_edges_of_its_batches(gpu_ctx, D, gated, splits):
     c.close()
 
 
+@pytest.mark.parametrize("D,rows", [(256, 1), (128, 1), (64, 3), (256, 8)])
+@pytest.mark.parametrize("splits", [2, 3, 5, 17, 33, 70, 130])
+def test_infinite_values_through_any_number_of_splits(gpu_ctx, D, rows, splits):
+    # An infinite value in any block that all rows see makes its dim infinite, and the other dims come out as they do without it: whatever a
+    # combine pass reads in the places of splits that are not there adds nothing, not even to an infinity.
+    import torch
+    from tinytitan_amd.engine import Attention
+    H, KH, T = 16, 2, 128 * splits - 5
+    r = np.random.default_rng(splits)
+    k, v = (r.standard_normal((T, KH, D)).astype(np.float16) for _ in range(2))
+    infinite = v.copy()
+    for block in range((T - rows + 1) // 32):
+        infinite[32 * block + block % 32, :, block % 48] = np.inf
+    dims = np.arange(D) < min(48, (T - rows + 1) // 32)
+    q = _dev((0.05 * r.standard_normal((1, rows, H, D))).astype(np.float16))
+    got = []
+    for values in (v, infinite):
+        c = Cache(gpu_ctx, k, values)
+        out = torch.full(q.shape, float("nan"), dtype=torch.float16, device="cuda")
+        torch.cuda.synchronize()
+        gpu_ctx.set_split_tokens(128)
+        Attention(gpu_ctx).encode_verify_rows(c.kv, 0, q, out, H, [T - rows], rows, D ** -0.5, [0])
+        gpu_ctx.synchronize()
+        gpu_ctx.set_split_tokens(0)
+        c.close()
+        got.append(out.float().cpu().numpy())
+    assert np.isfinite(got[0]).all()
+    assert (got[1][..., dims] == np.inf).all(), f"{np.isnan(got[1]).sum()} NaN"
+    assert np.array_equal(got[1][..., ~dims], got[0][..., ~dims])
+
+
 def test_graph_replay_matches_eager(gpu_ctx):
     import torch
     from tinytitan_amd import capi

@@ -163,7 +163,7 @@ def test_heads_of_128_in_steps_of_two_blocks(gpu_ctx, H, KH, rows, start, window
         _check(got[row:row + 1], want, f"row {row} of {rows} behind {start} keys, {H}q/{KH}kv/{D}, window {window}")
 
 
-@pytest.mark.parametrize("rows,kv_valid,first", [(128, 6200, 24), (128, 6300, 24), (160, 6400, 24), (160, 7300, 24), (545, 545, 0), (545, 577, 0)])
+@pytest.mark.parametrize("rows,kv_valid,first", [(128, 6200, 0), (128, 6300, 0), (160, 6400, 0), (160, 7300, 0), (545, 545, 0), (545, 577, 0)])
 def test_infinite_values_reach_the_output_as_they_are(gpu_ctx, rows, kv_valid, first):
     # Key ranges of 13, 11, 17 and 18 blocks, and a whole tile of one row and 18 or 19 blocks: an infinite value in a visible key's
     # dim makes that dim infinite, whichever block it lies in -- the step that has one block left must not add it again with
@@ -194,6 +194,37 @@ def test_infinite_values_reach_the_output_as_they_are(gpu_ctx, rows, kv_valid, f
     want = oracle.attention_batch(q.astype(np.float32), k.reshape(kv_valid, -1).astype(np.float32), v.reshape(kv_valid, -1).astype(np.float32),
                                   rows, start, H, KH, D, scale, threads=4).reshape(rows, H, D)[checked]
     _check(got[:, :, ~dims], want[:, :, ~dims], f"{rows} rows, {kv_valid} keys")
+
+
+@pytest.mark.parametrize("H,KH,D,rows,kv_valid", [
+    (24, 2, 256, 146, 2690), (24, 2, 256, 146, 2694),  # heads that leave rows of a tile empty, in front of the ranges' line and behind it: five
+    (24, 2, 256, 294, 2342), (24, 2, 256, 450, 2498), (24, 2, 256, 98, 4146), (24, 2, 256, 64, 6212),  # three, two, seven and thirteen
+    (64, 8, 256, 66, 4090), (64, 8, 256, 66, 4114), (64, 8, 256, 64, 4612),                             # split-K tiles, five ranges and seven
+    (64, 16, 128, 130, 4090), (64, 16, 128, 130, 4178), (64, 16, 128, 66, 5514)])                       # ... three and five
+def test_infinite_values_through_any_number_of_ranges(gpu_ctx, H, KH, D, rows, kv_valid):
+    # As above, over ranges that do not fill the places of a combine pass: every block that all rows see has an infinity, in one of the dims 0 .. 47
+    # each, and the other dims come out as they do without.
+    import torch
+    from tinytitan_amd.engine import KVCacheManager
+    start, scale = kv_valid - rows, float(D) ** -0.5
+    r = np.random.default_rng(kv_valid + rows)
+    k, v = (r.standard_normal((kv_valid, KH, D)).astype(np.float16) for _ in range(2))
+    q = (0.05 * r.standard_normal((rows, H * D))).astype(np.float16)
+    infinite = v.copy()
+    for block in range((start + 1) // 32):
+        infinite[32 * block + block % 32, :, block % 48] = np.inf
+    got = []
+    for values in (v, infinite):
+        kv = KVCacheManager(gpu_ctx, 1, KH, D, slots=1, max_context=kv_valid, initial_capacity=kv_valid)
+        kd, vd = _dev(k), _dev(values)
+        torch.cuda.synchronize()
+        kv.append(0, 0, 0, kd, vd)
+        gpu_ctx.synchronize()
+        got.append(_prefill(gpu_ctx, kv, q, start, rows, kv_valid, H, scale).reshape(rows, H, D))
+        kv.close()
+    assert np.isfinite(got[0]).all()
+    assert (got[1][:, :, :48] == np.inf).all(), f"{np.isnan(got[1]).sum()} NaN"
+    assert np.array_equal(got[1][:, :, 48:], got[0][:, :, 48:])
 
 
 @pytest.mark.parametrize("H,KH,rows,start,window,ring", [

@@ -1524,6 +1524,15 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(1))) f2 *global_pairs;  // part_ml: a partial row's (max, sum)
 typedef const __attribute__((address_space(1))) char *global_bytes;
 
+// What attn_combine_kernel reads in the place of a split that is not there: a partial row of zeros.  (Any other row's values would do but for
+// infinite ones, which a factor of zero makes NaN of; a select behind the load is instructions on every value, a branch around it a wait of its own.)
+static __device__ __align__(256) float no_split[256];
+__device__ __forceinline__ global_bytes no_row() {
+    global_bytes at = (global_bytes)no_split;
+    asm("" : "+s"(at));  // (an address like the others, not zeros the compiler knows of and branches to)
+    return at;
+}
+
 __device__ __forceinline__ int splits_of(const TileInfo &ti, int split_len) {
     return (int)((unsigned)(max(ti.tile_end - ti.k0, 1) + split_len - 1) / (unsigned)split_len);  // (an empty range has one, of zeros)
 }
@@ -1548,15 +1557,20 @@ __global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] cons
     const int d = dchunk * 64 + (lane & 15) * 4;
     const global_pairs ml = (global_pairs)a.part_ml + first_row;
     const global_bytes rows = (global_bytes)a.part_o + (first_row * D + d) * sizeof(float);
-    auto partial_row = [&](int s) { return *(const __attribute__((address_space(1))) f4 *)(rows + s * tstride * (D * sizeof(float))); };
-    // the gate's values of the item that threads 0-15 store at the end, first of all requests
+    const global_bytes zeros = no_row() + d * sizeof(float);
+    auto partial_row = [&](int s) {
+        return *(const __attribute__((address_space(1))) f4 *)(s < n_splits ? rows + s * tstride * (D * sizeof(float)) : zeros);
+    };
+    // the gate of the dim that a thread of the first wavefront stores at the end, first of all requests
     const int tl = (n * a.gh_inv) >> 16;
     const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
-    const bool aligned = (a.flags & kHotAligned) != 0;
-    const h4 gate4 = load_gate4(out, seq, ti.t0 + tl, hh, d, D);
+    const long long out_dim = (long long)hh * D + dchunk * 64 + lane;
+    const bool gated = wave == 0 && out.gate;
+    _Float16 gate = (_Float16)0.0f;
+    if (gated) gate = ((global_halves)out.gate)[seq * out.g_seq_stride + (ti.t0 + tl) * out.g_tok_stride + out_dim];
     const int s0 = wave * 4 + (lane >> 4);
     f4 acc = (f4)0.0f;
-    float l = 0.0f;
+    float l = 0.0f, factor = 1.0f;
     // This thread's first BATCH splits are requested BEFORE the global max is known: their
     // addresses do not depend on it, so the max's loads and these share one trip to memory.
     auto sum_splits = [&](auto batch) {
@@ -1568,11 +1582,15 @@ __global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] cons
         for (int i = 0; i < MAXIMA; ++i) maxima[i] = ml[min(lane + 64 * i, n_splits - 1) * tstride][0];
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) {
-            const int s = s0 + 16 * i < n_splits ? s0 + 16 * i : 0;
-            pml[i] = ml[s * tstride];
+            const int s = s0 + 16 * i;
+            pml[i] = ml[(s < n_splits ? s : 0) * tstride];
             po[i] = partial_row(s);
         }
         __builtin_amdgcn_sched_barrier(0);  // (the maximum's wait is not to come in front of the rest of the requests)
+        if (gated) {
+            factor = sigmoid((float)gate);
+            asm volatile("" : "+v"(factor));  // (here, while the rows are on their way, and not behind their sums)
+        }
         float mg = maxima[0];
 #pragma unroll
         for (int i = 1; i < MAXIMA; ++i) mg = fmaxf(mg, maxima[i]);
@@ -1604,15 +1622,17 @@ __global__ __launch_bounds__(256) void attn_combine_kernel([[maybe_unused]] cons
     if (lane < 16) *reinterpret_cast<f4 *>(&sm[wave][lane * 4]) = acc;
     if (lane == 0) sm[wave][64] = l;
     __syncthreads();
-    if (threadIdx.x < 16) {
-        f4 o = (f4)0.0f;
-        float lsum = 0.0f;
+    if (wave == 0) {
+        float o = 0.0f, lsum = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             lsum += sm[w][64];
-            o += *reinterpret_cast<const f4 *>(&sm[w][lane * 4]);
+            o += sm[w][lane];
         }
-        store_out4_gated(out, seq, ti.t0 + tl, hh, d, D, o, lsum > 0.0f ? 1.0f / lsum : 0.0f, aligned, gate4);
+        o *= lsum > 0.0f ? 1.0f / lsum : 0.0f;
+        if (gated) o *= factor;
+        typedef __attribute__((address_space(1))) _Float16 *global_out;
+        ((global_out)out.out)[seq * out.o_seq_stride + (ti.t0 + tl) * out.o_tok_stride + out_dim] = (_Float16)o;
     }
 }
 
@@ -1638,9 +1658,8 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel([[maybe_unused]]
     if ((int)threadIdx.x >= ROWS * D4 || n >= ti.tile_rows * a.gh) return;
     const int n_splits = splits_of(ti, a.split_len);
     const size_t tstride = (size_t)a.n_tiles * NT;
-    const size_t first_row = (size_t)sq.first_split * tstride + (size_t)tile * NT + n;
-    const global_pairs ml = (global_pairs)a.part_ml + first_row;
-    const global_bytes rows = (global_bytes)a.part_o + (first_row * D + d) * sizeof(float);
+    const size_t first_row = (size_t)sq.first_split * tstride + (size_t)tile * NT + blockIdx.x * ROWS;
+    const unsigned row_at = threadIdx.x * 16u, ml_at = threadIdx.x / D4 * 8u;  // this thread's in a split's four rows and pairs
     const int tl = (n * a.gh_inv) >> 16;
     const int hh = ti.kvh * a.group + ti.hsub * a.gh + (n - tl * a.gh);
     const bool aligned = (a.flags & kHotAligned) != 0;
@@ -1649,13 +1668,35 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel([[maybe_unused]]
     f4 acc = (f4)0.0f;
     auto turn = [&](auto splits, int first) {
         constexpr int SPLITS = decltype(splits)::value;
+        // Places past the row's last split read as zeros: the descriptors end behind it.  (Any other row's values times a factor of zero
+        // would do but for infinite ones, which become NaN; the host keeps 16 places of a launch within 4 GiB.)
+        const size_t base = first_row + first * tstride;
+        const unsigned there = min(n_splits - first, SPLITS) * (unsigned)tstride;
+        const __amdgpu_buffer_rsrc_t rows = make_rsrc(a.part_o + base * D, there * (unsigned)(D * sizeof(float)));
+        const __amdgpu_buffer_rsrc_t pairs = make_rsrc(a.part_ml + base * 2, there * (unsigned)(2 * sizeof(float)));
+        unsigned row_next = row_at, ml_next = ml_at, stride = (unsigned)tstride;
         f2 pml[SPLITS];
         f4 po[SPLITS];
+        // Requests in this order: six pairs and rows in turn, the other pairs, the other rows.  (16 ranges of 128 rows of 16/2 heads of 256, 33 MB: 7.4 us,
+        // all in turn 7.9, all rows in front 8.2, all pairs 7.85.)
+        constexpr int IN_TURN = SPLITS < 6 ? SPLITS : 6;
+        auto ask_row = [&](int i) {
+            po[i] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rows, row_next, 0, 0));
+            row_next += stride * (unsigned)(D * sizeof(float));
+        };
 #pragma unroll
         for (int i = 0; i < SPLITS; ++i) {
-            const int s = first + i < n_splits ? first + i : 0;
-            pml[i] = ml[s * tstride];
-            po[i] = *(const __attribute__((address_space(1))) f4 *)(rows + s * tstride * (D * sizeof(float)));
+            pml[i] = __builtin_bit_cast(f2, __builtin_amdgcn_raw_buffer_load_b64(pairs, ml_next, 0, 0));
+            asm volatile("" : "+s"(stride));  // (a place's offset is worked out here, not in front of all of them in a register of its own)
+            ml_next += stride * (unsigned)sizeof(f2);
+            if (i < IN_TURN) ask_row(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = IN_TURN; i < SPLITS; ++i) {
+            asm volatile("" : "+s"(stride));
+            ask_row(i);
+            __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_sched_barrier(0);  // (left alone, a request goes out when a row before it has come: fewer registers)
         float m_new = mg;
@@ -1791,7 +1832,9 @@ static int launch_combine_one(tt_hip_ctx *ctx, const LaunchPlan &plan, int n_seq
     // Many tiles with few splits each: from 64 of its workgroups on (8 sequences' decode rows, 4 sequences' verify
     // rows; a verify pass of 8 x 4 rows at 65k keys 174.5 -> 170.1 us a step, 8 sequences x 8 rows at 4k keys 36.9 ->
     // 30.0 us; with 32 workgroups -- 4 sequences' decode rows -- the other kernel is ahead, 13.1 against 14.3 us).
-    if (plan.n_splits_max <= 2 * kCombineRowsSplits && (long long)plan.n_tiles * n_seq * (NT / 4) >= 64) {
+    // (a turn's places are offsets of 32 bits)
+    const bool near = (unsigned long long)plan.n_tiles * NT * D * sizeof(float) * kCombineRowsSplits <= 0xffffffffull;
+    if (near && plan.n_splits_max <= 2 * kCombineRowsSplits && (long long)plan.n_tiles * n_seq * (NT / 4) >= 64) {
         dim3 cgrid((unsigned)(NT / 4), (unsigned)plan.n_tiles, (unsigned)n_seq);
         hipLaunchKernelGGL((attn_combine_rows_kernel<D, NT>), cgrid, dim3(256), 0, ctx->stream, args);
     } else {
