@@ -97,13 +97,10 @@ __device__ __forceinline__ void copy16_global_to_lds(const void *base, unsigned 
     const unsigned b_lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);  // (the builtin returns a signed int)
     base = (const void *)(((unsigned long long)b_hi << 32) | (unsigned long long)b_lo);
     lds_addr = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
-    // m0 carries the LDS address of the copy.  The compiler owns m0 (it is a reserved register: naming it as a
-    // clobber is not honoured), so the block saves it and puts it back; nothing else is touched.
-    unsigned saved_m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %2, %1\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved_m0)
-                 : "s"(base), "v"(lane_offset), "s"(lds_addr)
-                 : "memory");
+    // m0 carries the LDS address of the copy.  The compiler owns m0 (it is a reserved register: naming it as a clobber is not honoured), but has
+    // no use for it in the kernels that copy by this (tests/test_wait_states.py looks), so it is not put back.  Between a scalar write of m0 and a
+    // copy into LDS belongs one wait state, which is nobody's to add but the block's own.
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" : : "s"(base), "v"(lane_offset), "s"(lds_addr) : "memory");
 }
 
 // N pieces of 1 KiB that lie one behind the other in both places (an instruction's offset counts for both).
