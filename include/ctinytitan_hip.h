@@ -68,7 +68,11 @@ TT_HIP_API void tt_hip_ctx_destroy(tt_hip_ctx *ctx);
 
 /* Enqueue on a caller-owned hipStream_t instead of the context's own
  * (NULL restores the context's stream).  The reference's equivalent is the
- * MTLCommandBuffer argument of every encode call (Attention.swift:270-284). */
+ * MTLCommandBuffer argument of every encode call (Attention.swift:270-284).
+ * A change of stream is ordered: the new stream waits for what the old one holds
+ * at that moment, because a context's calls share its scratch.  Calls that are
+ * to overlap take a context each.  (No wait where either stream is being
+ * captured: launches of its graph are the caller's to order.) */
 TT_HIP_API int tt_hip_ctx_set_stream(tt_hip_ctx *ctx, void *hip_stream);
 /* Enqueue on HIP's legacy default (null) stream, whose handle is NULL and therefore cannot be
  * passed to tt_hip_ctx_set_stream.  A caller whose other work runs there (a framework's default

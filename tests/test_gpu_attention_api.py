@@ -850,6 +850,110 @@ def test_default_stream_orders_with_the_callers_work(gpu_ctx):
     c.close()
 
 
+def test_a_change_of_stream_is_ordered():
+    # The new stream starts behind what the old one holds: its first event cannot be over before the old stream's last.
+    import torch
+    from tinytitan_amd.engine import HIPContext
+    ctx = HIPContext(0)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    x = torch.randn(4096, 4096, device="cuda", dtype=torch.float16)
+    torch.cuda.synchronize()
+    for old, new in ((a, b), (b, torch.cuda.default_stream()), (torch.cuda.default_stream(), a)):
+        with torch.cuda.stream(old):
+            ctx.use_torch_stream()
+            for _ in range(60):
+                x @ x
+            last = torch.cuda.Event()
+            last.record()
+        with torch.cuda.stream(new):
+            ctx.use_torch_stream()
+            first = torch.cuda.Event()
+            first.record()
+        first.synchronize()
+        assert last.query()
+    torch.cuda.synchronize()
+    ctx.close()
+
+
+def test_calls_on_two_streams_in_turn_share_the_scratch():
+    # Chunks whose calls plan index lists, split their keys or dequantise pages, of unlike sizes, on one stream and the other without a word of
+    # synchronisation: the results of each call alone.
+    import torch
+    from tinytitan_amd.engine import HIPContext, KVCacheManager, PrefillAttention, PrefillAttentionParams
+    ctx = HIPContext(0)
+    r = np.random.default_rng(3)
+    calls = []
+    for H, KH, D, start, rows, bits, entries in ((16, 2, 256, 9000, 64, 16, 700), (16, 2, 256, 7000, 130, 8, 0), (16, 4, 64, 4000, 200, 16, 300),
+                                                 (32, 8, 128, 9000, 40, 16, 1000), (16, 2, 256, 30000, 1, 16, 0)):
+        total = start + rows
+        kv = KVCacheManager(ctx, 1, KH, D, slots=1, max_context=total, initial_capacity=total, precision_bits=bits)
+        k, v, q = (_dev(r.standard_normal((n, w)).astype(np.float16)) for n, w in ((total, KH * D), (total, KH * D), (rows, H * D)))
+        torch.cuda.synchronize()
+        kv.append(0, 0, 0, k, v)
+        lists = {}
+        if entries:
+            idx = np.stack([np.sort(r.permutation(start)[:entries]) for _ in range(rows)]).astype(np.int32)
+            lists = dict(keep_indices=_dev(idx), keep_index_stride=entries, keep_counts=_dev(np.full(rows, entries, np.int32)))
+        params = PrefillAttentionParams(start, rows, total, H, D ** -0.5, H * D, H * D, H * D)
+        calls.append((kv, q, params, lists))
+    pre = PrefillAttention(ctx)
+
+    def run(i, out):
+        kv, q, params, lists = calls[i]
+        pre.encode_causal(kv, 0, 0, q, out, params, **lists)
+
+    want = [torch.zeros_like(c[1]) for c in calls]
+    got = [[torch.zeros_like(c[1]) for c in calls] for _ in range(6)]
+    torch.cuda.synchronize()
+    for i, out in enumerate(want):
+        run(i, out)
+        ctx.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for turn, outs in enumerate(got):
+        for i, out in enumerate(outs):
+            with torch.cuda.stream(streams[(turn + i) % 2]):
+                ctx.use_torch_stream()
+                run(i, out)
+    torch.cuda.synchronize()
+    for kv, *_ in calls:
+        kv.close()
+    ctx.close()
+    assert all(w.abs().max() > 0 for w in want)
+    for outs in got:
+        for i, out in enumerate(outs):
+            assert torch.equal(out, want[i]), f"call {i}"
+
+
+def test_streams_that_are_being_captured_are_taken_as_they_are(gpu_ctx):
+    # A program's own capture, begun before the context is put on its stream and still open when it is taken off again: no wait goes into it.
+    import torch
+    from tinytitan_amd.engine import Attention
+    w = synthetic.decode_c2(context=900)
+    s = w.sequences[0]
+    c = Cache(gpu_ctx, s.k, s.v)
+    want = _decode(gpu_ctx, c.kv, s.q[None], [900], w.heads, w.scale, gate=s.gate[None])
+    qd, gd = _dev(s.q[None]), _dev(s.gate[None])
+    out = torch.zeros_like(qd)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph):
+            gpu_ctx.use_torch_stream()
+            Attention(gpu_ctx).encode_full(c.kv, 0, qd, out, w.heads, [900], w.scale, gate=gd)
+            gpu_ctx.set_stream(None)
+        got = []
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            got.append(out.float().cpu().numpy())
+    finally:
+        gpu_ctx.set_stream(None)
+    eager = _decode(gpu_ctx, c.kv, s.q[None], [900], w.heads, w.scale, gate=s.gate[None])
+    c.close()
+    assert np.array_equal(eager, want) and all(np.array_equal(g, want) for g in got)
+
+
 def test_profile_and_timer(gpu_ctx):
     import torch
     from tinytitan_amd.engine import Attention

@@ -1193,6 +1193,8 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     unsigned nxt_keys = ~0u;
     unsigned bits_cur = ~0u, bits_next = ~0u, bits_after = ~0u;
     const int bits_col = valid ? t_local : 0;
+    // A place in the tile's list as the plan gives it, inside the list's room whatever the words hold (nothing else bounds the reads below).
+    auto plan_place = [&](int word) { return (int)min((unsigned)__builtin_amdgcn_readfirstlane(word), (unsigned)args.plan_cap); };
     auto plan_entry = [&](int k) {  // the wavefront's k-th entry (a load; every lane the same words)
         const int e = e_at + k * WAVES;
         const int *at = plan_blocks_tile + 2 * (size_t)(e < e_hi ? e : 0);
@@ -1209,8 +1211,8 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     };
     if constexpr (LISTS) {
         const int *ranges = args.plan_ranges + (size_t)ti.tok_tile * (a.n_splits_max + 1) + split;
-        e_at = __builtin_amdgcn_readfirstlane(ranges[0]) + wave;
-        e_hi = __builtin_amdgcn_readfirstlane(ranges[1]);
+        e_at = plan_place(ranges[0]) + wave;
+        e_hi = plan_place(ranges[1]);
         plan_blocks_tile = args.plan_blocks + (size_t)ti.tok_tile * args.plan_cap * 2;
         plan_bits_tile = args.plan_bits + (size_t)ti.tok_tile * args.plan_cap * a.tt;
         const i2 e0 = plan_entry(0), e1 = plan_entry(1);
@@ -1245,8 +1247,8 @@ __global__ __launch_bounds__(WAVES * 64, (NT == 16 && KEEP < 2 ? 2 : 1)) void at
     };
     if constexpr (KEEP == 4) {
         const int *ranges = args.plan_ranges + (size_t)ti.tok_tile * (a.n_splits_max + 1) + split;
-        g_lo = __builtin_amdgcn_readfirstlane(ranges[0]);
-        g_hi = __builtin_amdgcn_readfirstlane(ranges[1]);
+        g_lo = plan_place(ranges[0]);
+        g_hi = plan_place(ranges[1]);
         run_end = g_hi > g_lo ? (g_hi + 7) >> 3 : 0;
         run = (g_lo >> 3) + wave;
         plan_blocks_tile = args.plan_blocks + (size_t)ti.tok_tile * args.plan_cap;

@@ -600,6 +600,30 @@ static int run_attention(tt_hip_ctx *ctx, tt_hip_kv *kv, int kind, int layer, in
 
 using namespace tt;
 
+// The calls that follow run on `next`, behind what the context has on its present stream: the stores it keeps for its calls -- partial results,
+// dequantised pages, the plans of index lists, the key selection's workspace -- are one set, and a call that overlapped another would work in
+// them while the other reads them (a list's plan holds places that the attention kernel reads at).  A stream that is being captured
+// has no part in that order: what it holds runs when its graph is launched, and its capture would not survive a wait for outside work.
+static int change_stream(tt_hip_ctx *ctx, hipStream_t next) {
+    if (next == ctx->stream) return TT_HIP_OK;
+    auto capturing = [](hipStream_t stream) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (stream && hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
+        return status != hipStreamCaptureStatusNone;
+    };
+    if (hipSetDevice(ctx->device) != hipSuccess) return TT_HIP_ERR_HIP;
+    if (!capturing(next) && !capturing(ctx->stream)) {
+        hipError_t e = hipEventRecord(ctx->ev_order, ctx->stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(next, ctx->ev_order, 0);
+        if (e != hipSuccess) {  // (a stream that its owner has destroyed meanwhile)
+            (void)hipGetLastError();
+            if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();
+        }
+    }
+    ctx->stream = next;
+    return TT_HIP_OK;
+}
+
 extern "C" {
 
 tt_hip_ctx *tt_hip_ctx_create(int device, int *out_err) {
@@ -621,7 +645,8 @@ tt_hip_ctx *tt_hip_ctx_create(int device, int *out_err) {
     ctx->device = device;
     ctx->n_cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
     if (hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&ctx->ev_begin) != hipSuccess || hipEventCreate(&ctx->ev_end) != hipSuccess) {
+        hipEventCreate(&ctx->ev_begin) != hipSuccess || hipEventCreate(&ctx->ev_end) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->ev_order, hipEventDisableTiming) != hipSuccess) {
         tt_hip_ctx_destroy(ctx);
         return fail(TT_HIP_ERR_HIP);
     }
@@ -667,6 +692,7 @@ void tt_hip_ctx_destroy(tt_hip_ctx *ctx) {
     for (hipEvent_t ev : ctx->prof_events) (void)hipEventDestroy(ev);
     if (ctx->ev_begin) (void)hipEventDestroy(ctx->ev_begin);
     if (ctx->ev_end) (void)hipEventDestroy(ctx->ev_end);
+    if (ctx->ev_order) (void)hipEventDestroy(ctx->ev_order);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
 }
@@ -675,16 +701,14 @@ int tt_hip_ctx_set_stream(tt_hip_ctx *ctx, void *hip_stream) {
     if (!ctx) return TT_HIP_ERR_INVALID_ARGUMENT;
     BusyGuard guard(ctx);
     if (!guard.ok || ctx->capturing) return TT_HIP_ERR_BUSY;
-    ctx->stream = hip_stream ? reinterpret_cast<hipStream_t>(hip_stream) : ctx->own_stream;
-    return TT_HIP_OK;
+    return change_stream(ctx, hip_stream ? reinterpret_cast<hipStream_t>(hip_stream) : ctx->own_stream);
 }
 
 int tt_hip_ctx_set_default_stream(tt_hip_ctx *ctx) {
     if (!ctx) return TT_HIP_ERR_INVALID_ARGUMENT;
     BusyGuard guard(ctx);
     if (!guard.ok || ctx->capturing) return TT_HIP_ERR_BUSY;
-    ctx->stream = nullptr;  // the legacy default stream
-    return TT_HIP_OK;
+    return change_stream(ctx, nullptr);  // the legacy default stream
 }
 
 void *tt_hip_ctx_stream(tt_hip_ctx *ctx) { return ctx ? reinterpret_cast<void *>(ctx->stream) : nullptr; }

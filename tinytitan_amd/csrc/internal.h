@@ -124,6 +124,7 @@ struct tt_hip_ctx {
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
+    hipEvent_t ev_order = nullptr;  // behind the work on a stream that the context leaves
     bool timer_open = false;
     float *part_o = nullptr;
     float *part_ml = nullptr;
