@@ -1249,29 +1249,33 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
     // rows at 4k 28.4 / 32.4, at 12k 47.7 / 42.8; 128 rows at 4k 32.0 / 35.0, at 8k 44.3 / 39.1; 192 rows at 4k 41.8 /
     // 38.6.  Over 8 bits: 64 rows at 4k 24.4 / 35.4, at 16k 50.1 / 49.2, at 32k 80.7 / 71.9; 128 rows at 4k 34.6 /
     // 40.2, at 8k 48.9 / 45.0.
-    // That is of 16 / 2 heads of 256, half a tile a row.  What the split-K way takes goes by its tiles, of which heads that leave a tile's rows empty
-    // have more: from 393,216 / (tiles x D / 256) keys on where that is earlier, and from 2,048 where rows stay empty.  us a layer, split-K / ranges:
-    // 24 / 2 heads of 256, 96 rows behind 7,000 keys 63.8 / 50.0, over 8 bits 81.0 / 55.7, 300 behind 3,000 109.2 / 74.9, 200 behind 1,600 53.0 / 56.0.
-    // (Later where there are fewer or narrower tiles would be faster, too -- 8 / 2 of 256, 128 rows behind 7,000 keys 38.1 / 35.6 the split-K way --, but
-    // the splits' combine pass gives NaN where it should give infinity, see the rows kernel, and the ranges do not there.)
+    // Heads that leave rows of a split-K tile empty make more tiles of the same rows, and what that way takes goes by its tiles: there from 393,216 /
+    // (tiles x D / 256) keys on where that is earlier, and from 2,048.  us a layer, split-K / ranges: 24 / 2 heads of 256, 96 rows behind 7,000 keys
+    // 63.8 / 50.0, over 8 bits 81.0 / 55.7, 300 behind 3,000 109.2 / 74.9, 200 behind 1,600 53.0 / 56.0.  Not for other heads, though the ranges would often
+    // be ahead (64 / 8 of 256, 130 rows behind 4,000 keys over 8 bits 173 / 119): not where the tiles share the chip out evenly (64 / 16 of 128, 64
+    // rows behind 7,900 keys 48.1 / 51.3, over 8 bits 58.6 / 77.9, 96 rows behind 5,100 67.8 / 75.8; 32 / 4 of 256, 64 rows 56.9 / 60.7).
     const bool rows_left_empty = 32 % packed_heads(n_q_heads / kv->n_kv_heads) != 0;
-    const long long tile_widths = splitk_tiles(n_q_heads, kv->n_kv_heads, q_len) * kv->head_dim;  // (at least 64)
-    const long long by_tiles = 393216ll * 256 / (tile_widths > 0 ? tile_widths : 1), by_rows = 786432 / (q_len > 0 ? q_len : 1);
-    const int all_floor = kv->bits == 16 ? 4096 : 2560, floor_keys = rows_left_empty ? 2048 : all_floor;
-    const long long line = std::min(by_tiles, by_rows);
-    int ranges_from = (int)std::min<long long>(std::max<long long>(line, floor_keys), 0x7fffffff);
-    if (ctx->capturing && serves && kv_valid >= ranges_from && kv_valid < std::max<long long>(by_rows, all_floor)) {
-        // inside a capture neither the partial results' store nor the staged pages grow: the split-K way, which has its own
-        const KeyRanges r = plan_key_ranges(ctx->n_cus, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, (kv_valid + 31) / 32);
-        const size_t part_rows = (size_t)r.n_splits * n_q_heads * ((q_len + 31) / 32) * 32;
-        const size_t staged_elems = kv->bits == 16 ? 0 : (size_t)((kv_valid + 31) / 32) * 32 * kv->head_dim * kv->n_kv_heads;
-        if (part_rows > ctx->part_rows || staged_elems > ctx->stage_elems) ranges_from = 0x7fffffff;
+    const long long by_rows = 786432 / (q_len > 0 ? q_len : 1), others_from = std::max<long long>(by_rows, kv->bits == 16 ? 4096 : 2560);
+    long long ranges_from = others_from;
+    if (rows_left_empty) {
+        const long long tile_widths = splitk_tiles(n_q_heads, kv->n_kv_heads, q_len) * kv->head_dim;
+        ranges_from = std::max<long long>(std::min(393216ll * 256 / (tile_widths > 0 ? tile_widths : 1), by_rows), 2048);
     }
     // ... and from this many rows on: 64; at fp16 32 rows deep in a context (32 rows at 32k keys 50 us against 54 us,
     // 48 rows 62 against 73).  Over quantised pages fewer rows stay with the split-K tiles, which widen a block once per
     // tile of 16 rows: dequantising the whole context for them costs more than that at any length measured (32 rows
     // at 64k keys over 8 bits 82 us against 107 us, 12 rows at 32k keys 30 us against 62 us).
     const int rows_from = kv->bits == 16 ? (kv_valid >= 32768 ? 32 : 64) : 64;
+    if (serves && !filled && (kv->bits == 16 || !kv->ring) && q_len >= rows_from && kv_valid >= ranges_from && kv_valid < others_from) {
+        // (no memory for the ranges' partial results or the dequantised pages, or a capture in which they would have to grow: the split-K way)
+        const int blocks = (kv_valid + 31) / 32;
+        const KeyRanges r = plan_key_ranges(ctx->n_cus, kv->head_dim, n_q_heads, kv->n_kv_heads, q_len, blocks);
+        if (hipSetDevice(ctx->device) != hipSuccess) return TT_HIP_ERR_HIP;
+        st = q_len >= 256 && whole.us < r.us ? TT_HIP_OK : ensure_partials(ctx, (size_t)r.n_splits * n_q_heads * ((q_len + 31) / 32) * 32, kv->head_dim);
+        if (st == TT_HIP_OK && kv->bits != 16) st = ensure_stage(ctx, (size_t)blocks * 32 * kv->head_dim * kv->n_kv_heads);
+        if (st == TT_HIP_ERR_BUSY || st == TT_HIP_ERR_OUT_OF_MEMORY) ranges_from = others_from;
+        else if (st != TT_HIP_OK) return st;
+    }
     if (kv->bits != 16 && !kv->ring && serves && q_len >= rows_from && (filled || kv_valid >= ranges_from)) {
         const int n_blocks = (kv_valid + 31) / 32;
         const size_t page = (size_t)n_blocks * 32 * kv->head_dim;
@@ -1328,7 +1332,8 @@ int tt_hip_attn_prefill_swa(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, int slot,
         return run_attention(ctx, kv, kind, layer, 1, &slot, &start_pos, &kv_valid, q_len, n_q_heads, q, 0, (long long)q_stride,
                              gate, 0, (long long)gate_stride, scale, out, 0, (long long)o_stride);
     };
-    // (and over fp16 pages, where a combine pass's NaN for an infinite value of split 0 would show)
+    // (over fp16 pages the two ways mostly take the same -- 116 of 120 chunks of groups of one and two within 5 %, 16/8 heads of 128, 300 rows behind 2,000 keys 37.5 /
+    // 38.6, 1,500 102.4 / 100.4, but 32/16 of 64, 100 rows behind 7,000, 52.9 / 37.8 --: one-head tiles, which need no partial results)
     if ((rows_left_empty || kv->bits == 16) && plentiful) return in_tiles(1);
     st = in_tiles(0);
     // (without memory for the splits' partial results, as inside a capture that would have to grow it: tiles of one head, which have none)
