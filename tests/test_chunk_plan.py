@@ -64,12 +64,12 @@ COPIES = r'''
 #include "chunk_plan.h"
 
 struct Ring {
-    int step, ring, ahead, which;
+    int ahead;
     std::map<int, int> landed;                 // slot -> block
     std::vector<std::vector<std::pair<int, int>>> flying;  // by turn: (slot, block)
     int slot_off = 0, bad = 0;
     void copy(int i, int first, int nb, int carry) {
-        const int j = i + ahead, slot = tt::in_ring(ring, j + slot_off), block = tt::copied_block(step, ring, j, which, first, nb, carry);
+        const int j = i + ahead, slot = tt::in_ring(j + slot_off), block = tt::copied_block(j, first, nb, carry);
         for (const auto &turn : flying)
             for (const auto &c : turn) bad += c.first == slot && c.second != block;
         flying.push_back({{slot, block}});
@@ -78,45 +78,42 @@ struct Ring {
         for (; flying.size() > turns; flying.erase(flying.begin()))
             for (const auto &c : flying.front()) landed[c.first] = c.second;
     }
-    void read(int j, int first, int nb) {  // step j's blocks, while this step's copies fly
-        const int slot = tt::in_ring(ring, j + slot_off), want = first + std::min(step * j + which, nb - 1);
+    void read(int j, int first, int nb) {  // step j's block, while this step's copies fly
+        const int slot = tt::in_ring(j + slot_off), want = first + std::min(j, nb - 1);
         bad += landed.count(slot) == 0 || landed[slot] != want;
         for (const auto &turn : flying)
             for (const auto &c : turn) bad += c.first == slot && c.second != want;
     }
 };
 
-static int run(int step, bool of_v, int which, int first, int nb, int carry) {
-    const int ring = of_v ? tt::v_ring(step) : tt::k_ring(step);
-    Ring r{step, ring, tt::copies_ahead(ring, of_v), which, {}, {}};
+static int run(bool of_v, int first, int nb, int carry) {
+    Ring r{tt::copies_ahead(of_v), {}, {}};
     for (int tile = 0; tile < (carry > 0 ? 2 : 1); ++tile) {
-        const int jb = tile ? 0 : first, n = tile ? carry : nb, next = tile ? 0 : carry, steps = (n + step - 1) / step;
+        const int jb = tile ? 0 : first, steps = tile ? carry : nb, next = tile ? 0 : carry;
         if (tile == 0)
-            for (int i = -r.ahead; i < 0; ++i) r.copy(i, jb, n, next);
+            for (int i = -r.ahead; i < 0; ++i) r.copy(i, jb, steps, next);
         r.wait(0);
-        if (!of_v) r.read(0, jb, n);
+        if (!of_v) r.read(0, jb, steps);
         for (int i = 0; i <= steps + 1; ++i) {
-            r.copy(i, jb, n, next);
-            if (!of_v && i + 1 < steps) r.read(i + 1, jb, n);
-            if (of_v && i >= 1 && i - 1 < steps) r.read(i - 1, jb, n);
-            r.wait(ring - 2);
+            r.copy(i, jb, steps, next);
+            if (!of_v && i + 1 < steps) r.read(i + 1, jb, steps);
+            if (of_v && i >= 1 && i - 1 < steps) r.read(i - 1, jb, steps);
+            r.wait(tt::kChunkRing - 2);
         }
         r.wait(0);
-        r.slot_off = tt::in_ring(ring, r.slot_off + steps);
+        r.slot_off = tt::in_ring(r.slot_off + steps);
     }
-    if (r.bad) std::printf("%d blocks a step, %s, block %d of a step, %d blocks, then %d: %d\n", step, of_v ? "V" : "K", which, nb, carry, r.bad);
+    if (r.bad) std::printf("%s, %d blocks, then %d: %d\n", of_v ? "V" : "K", nb, carry, r.bad);
     return r.bad != 0;
 }
 
 int main() {
     int bad = 0;
-    for (int step : {1, 2})
-        for (int of_v = 0; of_v < 2; ++of_v)
-            for (int which = 0; which < step; ++which)
-                for (int nb = 1; nb < 24; ++nb) {
-                    for (int carry = 0; carry < 24; ++carry) bad += run(step, of_v != 0, which, 0, nb, carry);
-                    bad += run(step, of_v != 0, which, 5, nb, 0);
-                }
+    for (int of_v = 0; of_v < 2; ++of_v)
+        for (int nb = 1; nb < 24; ++nb) {
+            for (int carry = 0; carry < 24; ++carry) bad += run(of_v != 0, 0, nb, carry);
+            bad += run(of_v != 0, 5, nb, 0);
+        }
     return bad != 0;
 }
 '''

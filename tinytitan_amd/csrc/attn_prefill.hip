@@ -25,7 +25,7 @@
 // Heads of 128 have half the matrix instructions for the same softmax, and a score wave is then most of a step: their two wavefronts a
 // SIMD share the KEYS instead (attn_prefill_halves_kernel).
 //
-// K/V blocks stream L2 -> LDS with direct-to-LDS 128-bit loads (no registers), three or four stages
+// K/V blocks stream L2 -> LDS with direct-to-LDS 128-bit loads (no registers), four stages
 // deep, issued one or two steps ahead of their first use; the K fragment layout in HBM is the MFMA
 // operand layout, V is permuted into it by the copy.
 //
@@ -230,12 +230,12 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     constexpr int KS = D / 16;  // k-steps of S^T
     constexpr int MT = D / 32;  // 32-dim tiles of O^T
     constexpr int BLOCK_BYTES = 32 * D * 2;
-    constexpr int KR = k_ring(1), VR = v_ring(1);
+    constexpr int RING = kChunkRing;
     constexpr int SLOT_BYTES = BLOCK_BYTES;
     constexpr int CHUNKS = BLOCK_BYTES / 1024;    // 1 KiB chunks per block (= KS = 2 MT)
     constexpr int CPW = CHUNKS / 4;               // copies one wave issues per step (K and V of a block over 8 waves)
-    constexpr int V_OFF = KR * SLOT_BYTES;             // K ring, then V ring
-    constexpr int P_OFF = (KR + VR) * SLOT_BYTES;      // P^T: [2 steps][4 heads][2 k-steps][64 lanes][16 B]
+    constexpr int V_OFF = RING * SLOT_BYTES;           // K ring, then V ring
+    constexpr int P_OFF = 2 * RING * SLOT_BYTES;       // P^T: [2 steps][4 heads][2 k-steps][64 lanes][16 B]
     constexpr int P_STEP = 4 * 2048;
     constexpr int ALPHA_OFF = P_OFF + 2 * P_STEP;      // rescale factors: [2 steps][4 heads][32 rows] floats
     constexpr int LSUM_OFF = ALPHA_OFF + 2 * 4 * 128;  // row sums: [4 heads][32 rows] floats
@@ -257,8 +257,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     const _Float16 *kp = a.k_slot + (size_t)kvh * a.page_elems;
     const _Float16 *vp = a.v_slot + (size_t)kvh * a.page_elems;
 
-    // Copies of step i: K of step i + KR and V of step i + VR - 2 (copies_ahead), of which this wave issues CPW one-KiB chunks.
-    // Step j's blocks live in slot j % KR (% VR) of their ring.  Past the end of the tile the
+    // Copies of step i: K of step i + RING and V of step i + RING - 2 (copies_ahead), of which this wave issues CPW one-KiB chunks.
+    // Step j's blocks live in slot j % RING of their ring.  Past the end of the tile the
     // last block is copied again (into a slot nobody reads any more), so that every step puts
     // the same number of copies in flight and one constant vmcnt tracks them.
     const unsigned smem_base = (unsigned)(size_t)(lds_ptr_t)smem;
@@ -271,11 +271,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     // without waiting for memory.  (A wave copies and reads K or V, so the offset is that of its own ring.)
     int slot_off = 0, carry_nb = 0;
     auto page_block = [&](int block) { return a.ring_blocks ? block % a.ring_blocks : block; };
-    auto role_ring = [&](int j) { return value_wave ? in_ring(VR, j) : in_ring(KR, j); };
     const int my_chunk = w4 * CPW;
-    auto source_block = [&](int j, int nb) {  // the block that step-relative index j stands for
-        return value_wave ? copied_block(1, VR, j, 0, jb, nb, carry_nb) : copied_block(1, KR, j, 0, jb, nb, carry_nb);
-    };
     // A step's copies: this wave's CPW one-KiB chunks of ONE block -- of K for the score waves (the LDS layout is the HBM
     // layout, fragment s is chunk s), of V for the value waves (gathered so that LDS holds fragment (mt, t) as [lane][8 halves]).  Where the block lies in the page and in the
     // ring is worked out ONCE per step (step_copies); a copy then costs two scalar adds on top of its load -- worked
@@ -293,10 +289,10 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
     }
     auto step_copies = [&](int i, int nb) {  // of step i; nb blocks in the range
         StepCopies sc;
-        const int j = i + (value_wave ? copies_ahead(VR, true) : copies_ahead(KR, false));
+        const int j = i + (value_wave ? copies_ahead(true) : copies_ahead(false));
         const _Float16 *page = value_wave ? vp : kp;
-        sc.src = reinterpret_cast<const char *>(page + (size_t)page_block(source_block(j, nb)) * (32 * D)) + (value_wave ? 0 : my_chunk * 1024);
-        sc.dst = smem_base + (unsigned)((value_wave ? V_OFF : 0) + role_ring(j + slot_off) * SLOT_BYTES + w4 * CPW * 1024);
+        sc.src = reinterpret_cast<const char *>(page + (size_t)page_block(copied_block(j, jb, nb, carry_nb)) * (32 * D)) + (value_wave ? 0 : my_chunk * 1024);
+        sc.dst = smem_base + (unsigned)((value_wave ? V_OFF : 0) + in_ring(j + slot_off) * SLOT_BYTES + w4 * CPW * 1024);
         return sc;
     };
     auto issue_copy = [&](const StepCopies &sc, int c) {  // copy c (0 .. CPW-1)
@@ -348,22 +344,19 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             carry_nb = max((end2 + 31) >> 5, 0);
         }
         if (!carried) {
-            // K of steps 0 .. KR - 1, V of steps 0 .. VR - 3, each to a place of its own: nothing orders two copies in flight.  (The value
-            // waves once took the score waves' KR turns: with a ring of three, two different blocks on their way to one place.)
+            // K of steps 0 .. RING - 1, V of steps 0 .. RING - 3, each to a place of its own: nothing orders two copies in flight.
 #pragma unroll
-            for (int i = -copies_ahead(KR, false); i < 0; ++i)
-                if (!value_wave || i >= -copies_ahead(VR, true)) issue_step(i, nb);
+            for (int i = -copies_ahead(false); i < 0; ++i)
+                if (!value_wave || i >= -copies_ahead(true)) issue_step(i, nb);
         }
 
-        // End of step i.  What the next step reads from LDS, K(i+2) and V(i), was copied in steps i + 2 - KR and i + 2 - VR
-        // and must have landed; the copies of the KR - 2 and VR - 2 steps since may still fly.  Then the
+        // End of step i.  What the next step reads from LDS, K(i+2) and V(i), was copied in step i + 2 - RING
+        // and must have landed; the copies of the RING - 2 steps since may still fly.  Then the
         // barrier that publishes them and this step's P^T.
-        auto end_step = [&](auto ring) {
-            TT_WAIT_VMCNT((decltype(ring)::value - 2) * CPW);
+        auto end_step = [&]() {
+            TT_WAIT_VMCNT((RING - 2) * CPW);
             __syncthreads();
         };
-        constexpr std::integral_constant<int, KR> k_landed{};
-        constexpr std::integral_constant<int, VR> v_landed{};
 
         // Step i (0 .. steps + 1): the score waves run the MFMAs of step i's blocks, the value waves those of
         // step i - 2's; both fetch the NEXT step's fragments from LDS into the registers the
@@ -389,7 +382,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             __syncthreads();  // every score wave holds K of step 0: step 0 may refill its slot
 #pragma nounroll
             for (int i = 0; i < nb; ++i) {
-                const char *next = smem + in_ring(KR, i + 1 + slot_off) * SLOT_BYTES + lane * 16;
+                const char *next = smem + in_ring(i + 1 + slot_off) * SLOT_BYTES + lane * 16;
                 const StepCopies sc = step_copies(i, nb);
                 f16v s = (f16v)0.0f;
 #pragma unroll
@@ -408,12 +401,12 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
 #pragma unroll
                 for (int t = 0; t < 2; ++t) *reinterpret_cast<h8 *>(pdst + t * 1024) = pf[t];
                 if (g == 0) alpha_mine[(i & 1) * 128] = alpha;
-                end_step(k_landed);
+                end_step();
             }
             issue_step(nb, nb);
-            end_step(k_landed);  // the value waves' last two steps
+            end_step();  // the value waves' last two steps
             issue_step(nb + 1, nb);
-            end_step(k_landed);
+            end_step();
             const float lt = sum_across_halves(l);
             if (g == 0) {
                 if (a.n_splits > 1) {  // partial: the row's reference max (log2 domain) and sum over this key range
@@ -437,7 +430,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
             // fetched from LDS into registers during step j + 1 and consumed in step j + 2, so
             // that the MFMAs of a step start right after its barrier.
             issue_step(0, nb);
-            end_step(v_landed);  // step 0: the score waves' first
+            end_step();  // step 0: the score waves' first
             issue_step(1, nb);
             h8 vf[2 * MT], pf[2];
 #pragma unroll
@@ -446,11 +439,11 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
 #pragma unroll
             for (int t = 0; t < 2; ++t) pf[t] = *reinterpret_cast<const h8 *>(p_mine + t * 1024);
             float alpha = alpha_mine[0];
-            end_step(v_landed);  // step 1
+            end_step();  // step 1
 #pragma nounroll
             for (int i = 2; i <= nb + 1; ++i) {
                 const int jn = i - 1;  // the step fetched in this one (past the last one: stale but harmless data)
-                const char *next = smem + V_OFF + in_ring(VR, jn + slot_off) * SLOT_BYTES + lane * 16;
+                const char *next = smem + V_OFF + in_ring(jn + slot_off) * SLOT_BYTES + lane * 16;
                 const char *psrc = p_mine + (jn & 1) * P_STEP;
                 const StepCopies sc = step_copies(i, nb);
                 if (__any(alpha != 1.0f)) {
@@ -484,7 +477,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
                         pf[t] = *reinterpret_cast<const h8 *>(psrc + t * 1024);
                     }
                 }
-                end_step(v_landed);
+                end_step();
             }
             TT_WAIT_VMCNT(0);
             __syncthreads();  // the row sums are in LDS
@@ -548,7 +541,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_prefill_kernel(cons
                 }
             }
         }
-        if (carry_nb > 0) slot_off = role_ring(slot_off + nb);  // where the next tile's first step sits
+        if (carry_nb > 0) slot_off = in_ring(slot_off + nb);  // where the next tile's first step sits
     }
 }
 
@@ -867,8 +860,8 @@ bool prefill_kernel_serves(int n_q_heads, int n_kv_heads, int head_dim, bool ali
     return aligned && group % 4 == 0 && (head_dim == 256 || head_dim == 128 || head_dim == 64);
 }
 
-// the rings of K and V (128 KiB at D = 256, 112 at 128) + P^T hand-over (16, 32 KiB) + rescale factors and row sums + the output rows' staging (10 KiB)
-static constexpr int prefill_lds_bytes(int D) { return (k_ring(1) + v_ring(1)) * 32 * D * 2 + 2 * 4 * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80; }
+// the rings of K and V (128, 64 and 32 KiB at D = 256, 128 and 64) + P^T hand-over (16 KiB) + rescale factors and row sums + the output rows' staging (10 KiB)
+static constexpr int prefill_lds_bytes(int D) { return 2 * kChunkRing * 32 * D * 2 + 2 * 4 * 2048 + 2 * 4 * 128 + 4 * 128 + 4 * 32 * 80; }
 
 // ... the rings of the kernel over halves of the keys (128 KiB at D = 128) + the places that its wavefronts hand their results over in
 static constexpr int prefill_halves_lds_bytes(int D) { return 2 * kHalvesRing * 2 * 32 * D * 2 + 8 * 4096; }

@@ -29,21 +29,18 @@ inline int longest_tile_blocks(int start, int q_len, int kv_valid, int window) {
     return longest;
 }
 
-// ---- The rings in LDS that the chunk kernels' copies fill (attn_prefill.hip): how many steps of K and V they hold.
-constexpr int k_ring(int) { return 4; }
-constexpr int v_ring(int) { return 4; }
-constexpr int in_ring(int ring, int j) { return (int)((unsigned)j % (unsigned)ring); }  // j >= 0
+// ---- The rings in LDS that the chunk kernels' copies fill (attn_prefill.hip): how many steps, a key block each, of K and of V they hold.
+constexpr int kChunkRing = 4;
+constexpr int in_ring(int j) { return (int)((unsigned)j % (unsigned)kChunkRing); }  // j >= 0
 // Step i, and in front of step 0 a turn for each i below it down to -copies_ahead, issues the copies of step i + copies_ahead.
-constexpr int copies_ahead(int ring, bool of_v) { return of_v ? ring - 2 : ring; }
-// What is copied for step j of a range of `nb` blocks from block `first` on: the `which`-th of the step's blocks.  Past the range's last the
-// last again, or, when a second tile follows (of `carry` blocks, from block 0), that tile's first, a ring of them; then
-// a slot's blocks again: the same bytes.
-constexpr int copied_block(int step, int ring, int j, int which, int first, int nb, int carry) {
-    const int steps = (nb + step - 1) / step;
-    const int at = j < steps || carry == 0 ? step * j + which : step * in_ring(ring, j - steps) + which;
-    return j < steps || carry == 0 ? first + (at < nb ? at : nb - 1) : (at < carry ? at : carry - 1);
+constexpr int copies_ahead(bool of_v) { return of_v ? kChunkRing - 2 : kChunkRing; }
+// The block copied for step j of a range of `nb` blocks from block `first` on.  Past the range's last the last again, or, when a second
+// tile follows (of `carry` blocks, from block 0), that tile's first, a ring of them; then a slot's blocks again: the same bytes.
+constexpr int copied_block(int j, int first, int nb, int carry) {
+    if (j < nb || carry == 0) return first + (j < nb ? j : nb - 1);
+    const int at = in_ring(j - nb);
+    return at < carry ? at : carry - 1;
 }
-
 
 // The kernel over halves of the keys takes two blocks a step, one for either half, and copies K and V `kHalvesAhead` steps ahead.  The last
 // step's copies are left out (where they would go the halves meet), so a tile leaves kHalvesAhead steps behind its own.
