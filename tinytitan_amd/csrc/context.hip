@@ -1106,6 +1106,8 @@ int tt_hip_attn_prefill_keep_indices(tt_hip_ctx *ctx, tt_hip_kv *kv, int layer, 
     //     anyway: 32/8, 100 rows behind 60k (walked 3.6 times) 251 / 270, 165 / 194, behind 12k (17 times) 132 / 124, 125 / 117
     //   heads of 64, whose tiles are the cheapest, over long contexts or many tiles: 16/4, 128 rows behind 12k 80 / 85, 79 / 85, behind
     //     60k 150 / 119, 106 / 95, 400 behind 100k 406 / 237, 219 / 168; 64/8, 80 rows behind 30k 162 / 111, 128 / 95.
+    // Distance from 64 bits: the 2-norm falls by a sixth or more, the largest single difference grows by a tenth to two fifths (every value of V is rounded
+    // to fp16 by itself, where a probability times a group's scale was, once for 64 dims).
     const long long tok_tiles = (q_len + tt - 1) / tt, tiles = tok_tiles * (group / gh) * kv->n_kv_heads;
     const long long walked = tok_tiles * (entries < kv_valid ? entries : kv_valid);
     const bool worth = kv->head_dim == 256 ? tiles >= 32 && walked >= 3ll * kv_valid
